@@ -164,8 +164,9 @@ struct EpiLane {
   int act;
 };
 
+// The lane's constants from the raw values of its four channels (1 / 1 / 0 where a constant is absent).
 template <class S>
-__device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev &e) {
+__device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, const EpiDev &e) {
   EpiLane L;
   L.use_rcp = S::rcp(e); L.use_div = S::truediv(e); L.use_bias = S::bias(e); L.use_res = S::resid(e);
   L.res_after = S::resid_after(e);
@@ -175,24 +176,28 @@ __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev
   // Reciprocal form with the power of two folded in:
   //   v = (f*2^e)/d  ==  q = f*(r*2^e); err = fma(-q, d*2^-e, f); fma(err, r*2^e, q)
   // (scaling by 2^e is exact, so every intermediate is the scaled image of the unfolded one)
-  L.div = v4f{1.f, 1.f, 1.f, 1.f}; L.rcp = v4f{1.f, 1.f, 1.f, 1.f}; L.bias = v4f{0.f, 0.f, 0.f, 0.f};
-  if (n_ok && (L.use_rcp || L.use_div)) L.div = *reinterpret_cast<const v4f *>(e.chan_div + n);
-  if (n_ok && L.use_rcp) {
-    L.rcp = *reinterpret_cast<const v4f *>(e.chan_rcp + n);
+  L.div = div; L.rcp = rcp; L.bias = bias;
+  if (L.use_rcp) {
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       L.rcp[t] = __builtin_ldexpf(L.rcp[t], e.exp2 + (S::kFoldScale ? e.q_neg_pos : 0));
       L.div[t] = __builtin_ldexpf(L.div[t], -e.exp2 - (S::kFoldScale ? e.q_neg_pos : 0));
     }
   }
-  if (n_ok && L.use_bias) {
-    L.bias = *reinterpret_cast<const v4f *>(e.bias + n);
-    if constexpr (S::kFoldScale) {
+  if constexpr (S::kFoldScale) {
 #pragma unroll
-      for (int t = 0; t < 4; ++t) L.bias[t] = __builtin_ldexpf(L.bias[t], e.q_neg_pos);
-    }
+    for (int t = 0; t < 4; ++t) L.bias[t] = __builtin_ldexpf(L.bias[t], e.q_neg_pos);
   }
   return L;
+}
+
+template <class S>
+__device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev &e) {
+  v4f div = {1.f, 1.f, 1.f, 1.f}, rcp = {1.f, 1.f, 1.f, 1.f}, bias = {0.f, 0.f, 0.f, 0.f};
+  if (n_ok && (S::rcp(e) || S::truediv(e))) div = *reinterpret_cast<const v4f *>(e.chan_div + n);
+  if (n_ok && S::rcp(e)) rcp = *reinterpret_cast<const v4f *>(e.chan_rcp + n);
+  if (n_ok && S::bias(e)) bias = *reinterpret_cast<const v4f *>(e.bias + n);
+  return epi_lane_finish<S>(div, rcp, bias, e);
 }
 
 // dequantization and bias of one integer sum: channel t of the lane's four

@@ -310,8 +310,15 @@ int gemm_nt_stream_i8(const void *a, const void *b, int64_t M, int64_t N, int64_
 int conv2d_stem_i8(const void *x, const void *w, int N, int H, int W, int Co, int kh, int kw, int sh, int sw, int dh,
                    int Ho, int Wo, const EpiDev &e, hipStream_t s);
 
+int contract_small_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                      int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
+
 int gemm_nt_mfma_i8(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e,
                     hipStream_t s) {
+  if (M < (1 << 20) && K < (1 << 20)) {  // few output tiles
+    const int st = contract_small_i8(a, b, (int)M, 1, 1, (int)K, (int)N, 1, 1, 0, 0, 1, 1, 1, 1, 1, 1, e, s);
+    if (st >= 0) return st;
+  }
   if (dma_enabled()) {  // short K, narrow N, many rows: the streaming kernel
     const int st = gemm_nt_stream_i8(a, b, M, N, K, e, s);
     if (st >= 0) return st;
@@ -355,6 +362,10 @@ int conv2d_mfma_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
   p.N = Co;
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo;
   p.kh = kh; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
+  if (Ci % 16 == 0) {  // few output tiles
+    const int st = contract_small_i8(x, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, e, s);
+    if (st >= 0) return st;
+  }
   if (Ci == 4 && ph == 0 && pw == 0 && dw == 1 && dma_enabled()) {  // framed few-channel image: streaming kernel
     const int st = conv2d_stem_i8(x, w, N, H, W, Co, kh, kw, sh, sw, dh, Ho, Wo, e, s);
     if (st >= 0) return st;

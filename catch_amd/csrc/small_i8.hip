@@ -1,0 +1,313 @@
+// int8 contractions of few output tiles: the K loop split over the waves of a block, no barrier inside it.
+//
+// What bounds such a launch (one image through a late layer, a few tokens through a linear): the tiled kernels give it
+// a handful of blocks, each a serial chain of K steps with a barrier and a memory latency per step -- 256 channels of a
+// 3x3 layer on one 14 x 14 image took 8.6 us on 8 blocks, 512 channels on 7 x 7 11.1 us on 16, where all of the
+// operands fit one microsecond of L2 traffic.  Here a block owns one tile of T x T outputs (T = 32 or 16: the smallest
+// that fills the device once) and its NW waves take a contiguous slice of K each: a wave's transfers (LDS-DMA, whole
+// 128-byte lines, two 128-byte K steps in flight per wave) go to a slice of LDS of its own, so it waits for nothing but
+// its own loads; the partial sums meet in LDS once, behind the loop, and every output is finished by the epilogue code
+// of the other kernels.  Residual and per-channel constants are requested before the first K step.
+#include <type_traits>
+
+#include "igemm_common.h"
+
+namespace catchq {
+
+typedef __attribute__((address_space(3))) void *lds_ptr_t;
+
+struct SmallParams {
+  int M, N, K;       // M < 2^20, K < 2^20
+  int H, W, Ci, Ho, Wo, kw, ph, pw, sh, sw, dh, dw;
+  unsigned img_stride, row_stride, pix_stride;  // elements
+  unsigned magic_wo, magic_ho, magic_ci, magic_kw, magic_t;  // ceil(2^32 / d); 0 for d = 1, whose mask is all ones
+  unsigned mask_wo, mask_ho, mask_ci, mask_kw, mask_t;
+  int tiles_m, tiles_n, nblocks;
+  int m_fastest;     // consecutive blocks walk the row tiles of one column tile first
+  int epi;           // epilogue variant (EPI_*), the same for every block
+  unsigned a_bytes, b_bytes;
+};
+
+#define CATCHQ_SMALL_VMCNT(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
+
+// n / d for n * d < 2^32 through magic = ceil(2^32 / d) (d = 1: magic 0, mask ~0)
+__device__ __forceinline__ unsigned div_magic(unsigned n, unsigned magic, unsigned mask) { return __umulhi(n, magic) + (n & mask); }
+
+__device__ __forceinline__ v4i small_ds_read(unsigned addr) {
+  v4i v;
+  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr));
+  return v;
+}
+// DENSE: a plain GEMM -- row m starts at m * K, no taps
+template <int T, int NW, bool DENSE>
+__global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restrict__ A, const int8_t *__restrict__ B,
+                                                          SmallParams p, EpiDev e) {
+  resolve_exp2(e);
+  constexpr int SLOTS = 2, BKB = 128;
+  constexpr int SLOT_BYTES = 2 * T * BKB, WAVE_BYTES = SLOTS * SLOT_BYTES;
+  constexpr int NA = T / 8, NI = 2 * NA;   // DMA instructions (8 rows of 128 bytes each) per K step
+  constexpr int SUB = T == 32 ? 4 : 2;     // matrix instructions per K step: 32 x 32 x 32 or 16 x 16 x 64
+  constexpr int PITCH = T + 4;             // ints per pixel of a partial tile
+  static_assert(T * PITCH * 4 <= WAVE_BYTES, "a partial tile fits the wave's slots");
+  extern __shared__ __attribute__((aligned(16))) int8_t lds[];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int logical = xcd_remap(blockIdx.x, p.nblocks);
+  const int outer = (int)div_magic((unsigned)logical, p.magic_t, p.mask_t);
+  const int inner = logical - outer * (p.m_fastest ? p.tiles_m : p.tiles_n);
+  const int tile_m = p.m_fastest ? inner : outer, tile_n = p.m_fastest ? outer : inner;
+  const int m0 = tile_m * T, n0 = tile_n * T;
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)p.a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)p.b_bytes, 0x00020000);
+  constexpr unsigned OOB = 0x80000000u;  // the hardware answers an offset beyond the buffer with zeros
+
+  // the epilogue's lanes: four channels of one pixel each, T * T / 4 of them (waves 0 ..)
+  constexpr int EPI_LANES = T * T / 4, CPR = T / 4;
+  const bool epi_wave = wave * 64 < EPI_LANES;
+  const bool vec = p.epi != EPI_SCALAR;
+  constexpr int ROUNDS = (EPI_LANES + 64 * NW - 1) / (64 * NW);
+  v4f c_div = {1.f, 1.f, 1.f, 1.f}, c_rcp = c_div, c_bias = {0.f, 0.f, 0.f, 0.f}, c_res[ROUNDS];
+  // 64 * NW is a multiple of CPR: a lane has the same four channels in every round.  (Plain loads: the transfers below
+  // and the statements that clobber memory keep them here, in front of the K loop.)
+  const int ec = n0 + (threadIdx.x % CPR) * 4;
+  if (epi_wave && vec) {
+    const int cc = min(ec, p.N - 4);
+    if (e.chan_div) c_div = *reinterpret_cast<const v4f *>(e.chan_div + cc);
+    if (e.chan_rcp) c_rcp = *reinterpret_cast<const v4f *>(e.chan_rcp + cc);
+    if (e.bias) c_bias = *reinterpret_cast<const v4f *>(e.bias + cc);
+#pragma unroll
+    for (int r = 0; r < ROUNDS; ++r) {
+      c_res[r] = v4f{0.f, 0.f, 0.f, 0.f};
+      const int em = min(m0 + (int)(threadIdx.x + r * 64 * NW) / CPR, p.M - 1);
+      if (e.resid) c_res[r] = *reinterpret_cast<const v4f *>(e.resid + (int64_t)em * p.N + cc);
+    }
+  }
+
+  // ---- loader ------------------------------------------------------------------------------------------------------
+  // A DMA instruction fills 8 rows of 128 bytes: lane l writes 16-byte piece l & 7 of row l >> 3.  It fetches the piece
+  // (l & 7) ^ ((row >> 1) & 7) of that row, so that the 16-byte fragment reads of 16 consecutive rows fall into 16
+  // different pieces of a 256-byte LDS line; row = 8 j + (l >> 3), so even and odd j differ in bit 2 of the piece.
+  const int lrow = lane >> 3;
+  const int chunk0 = (lane & 7) ^ (lane >> 4);
+  unsigned a_base[NA], b_base[NA];
+  int a_hi[NA], a_wi[NA];
+#pragma unroll
+  for (int j = 0; j < NA; ++j) {
+    const int m = m0 + j * 8 + lrow;
+    if constexpr (DENSE) {
+      a_hi[j] = a_wi[j] = 0;
+      a_base[j] = m < p.M ? (unsigned)m * (unsigned)p.K : OOB;
+    } else {
+      const unsigned t = div_magic((unsigned)m, p.magic_wo, p.mask_wo), wo = (unsigned)m - t * (unsigned)p.Wo;
+      const unsigned img = div_magic(t, p.magic_ho, p.mask_ho), ho = t - img * (unsigned)p.Ho;
+      a_hi[j] = m < p.M ? (int)ho * p.sh - p.ph : -(1 << 30);  // a row that does not exist is outside the image
+      a_wi[j] = (int)wo * p.sw - p.pw;
+      a_base[j] = img * p.img_stride + (unsigned)a_hi[j] * p.row_stride + (unsigned)a_wi[j] * p.pix_stride;  // mod 2^32
+    }
+    const int n = n0 + j * 8 + lrow;
+    b_base[j] = n < p.N ? (unsigned)n * (unsigned)p.K : OOB;
+  }
+  const int steps = (p.K + BKB - 1) / BKB;
+  const int per = steps / NW, rem = steps - per * NW;
+  const int first = wave * per + (wave < rem ? wave : rem);
+  const int mine = per + (wave < rem ? 1 : 0);
+  int8_t *const my = lds + wave * WAVE_BYTES;
+
+  auto issue = [&](int s) {  // step s of this wave's slice into its slot s & 1
+    const int slot = (s & 1) * SLOT_BYTES;
+    unsigned k[2], koff[2];
+    int dy[2], dx[2];
+    bool ok[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      k[h] = (unsigned)((first + s) * BKB + (chunk0 ^ (4 * h)) * 16);
+      ok[h] = (s < mine) & (k[h] < (unsigned)p.K);
+      koff[h] = k[h];
+      dy[h] = dx[h] = 0;
+      if constexpr (!DENSE) {
+        const unsigned tap = div_magic(k[h], p.magic_ci, p.mask_ci), ci = k[h] - tap * (unsigned)p.Ci;
+        const unsigned r = div_magic(tap, p.magic_kw, p.mask_kw), q = tap - r * (unsigned)p.kw;
+        dy[h] = (int)r * p.dh;
+        dx[h] = (int)q * p.dw;
+        koff[h] = (unsigned)dy[h] * p.row_stride + (unsigned)dx[h] * p.pix_stride + ci;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+      const int h = j & 1;
+      bool in = ok[h];
+      if constexpr (!DENSE)
+        in = in & ((unsigned)(a_hi[j] + dy[h]) < (unsigned)p.H) & ((unsigned)(a_wi[j] + dx[h]) < (unsigned)p.W);
+      unsigned voff = in ? a_base[j] + koff[h] : OOB;
+      asm volatile("" : "+v"(voff));  // one select and one load, not two loads under complementary masks
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
+    }
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+      const int h = j & 1;
+      unsigned voff = ok[h] ? b_base[j] + k[h] : OOB;
+      asm volatile("" : "+v"(voff));
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(my + slot + (NA + j) * 1024), 16, (int)voff, 0, 0, 0);
+    }
+  };
+
+  // ---- K loop: this wave's slice -------------------------------------------------------------------------------------
+  typedef typename std::conditional<T == 32, v16i, v4i>::type acc_t;
+  acc_t acc = {};
+  if (mine > 0) {
+    const int frow = lane & (T - 1), fk = lane / T;  // row of the fragment, 16-byte piece within a sub-step
+    const unsigned a_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t *)my + (unsigned)(frow * BKB);
+    const unsigned sw = (unsigned)((frow >> 1) & 7);
+    issue(0);
+    issue(1);  // (past the slice: nothing but zeros, so that the count of transfers in flight stays the same)
+    for (int s = 0; s < mine; ++s) {
+      CATCHQ_SMALL_VMCNT(NI);
+      const unsigned base = a_addr + (unsigned)((s & 1) * SLOT_BYTES);
+      v4i fa[SUB], fb[SUB];
+#pragma unroll
+      for (int u = 0; u < SUB; ++u) {
+        const unsigned piece = (((unsigned)(u * (64 / T) + fk)) ^ sw) * 16;
+        fa[u] = small_ds_read(base + piece);
+        fb[u] = small_ds_read(base + T * BKB + piece);
+      }
+#pragma unroll
+      for (int u = 0; u < SUB; ++u) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[u]), "+v"(fb[u])::"memory");
+      issue(s + 2);  // the slot has been read
+      // operands swapped (weights as A): a lane ends up with four consecutive channels of one pixel
+#pragma unroll
+      for (int u = 0; u < SUB; ++u) {
+        if constexpr (T == 32) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[u], fa[u], acc, 0, 0, 0);
+        else acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[u], fa[u], acc, 0, 0, 0);
+      }
+    }
+    CATCHQ_SMALL_VMCNT(0);  // the transfers past the slice have landed: the slots are free
+    int *part = reinterpret_cast<int *>(my) + frow * PITCH + fk * 4;
+    if constexpr (T == 32) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<v4i *>(part + 8 * g) = v4i{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+    } else {
+      *reinterpret_cast<v4i *>(part) = acc;
+    }
+  }
+  __syncthreads();
+  if (!epi_wave) return;
+
+  // ---- partial sums -> outputs ---------------------------------------------------------------------------------------
+  const int active = steps < NW ? steps : NW;
+#pragma unroll
+  for (int r = 0; r < ROUNDS; ++r) {
+    const int t = threadIdx.x + r * 64 * NW;
+    if (t >= EPI_LANES) break;
+    const int px = t / CPR, cg = t % CPR;
+    const int m = m0 + px;
+    const int *part = reinterpret_cast<const int *>(lds) + px * PITCH + cg * 4;
+    v4i a = *reinterpret_cast<const v4i *>(part);
+    for (int w = 1; w < active; ++w) a += *reinterpret_cast<const v4i *>(part + w * (WAVE_BYTES / 4));
+    if (m >= p.M || ec >= p.N) continue;
+    const int64_t idx = (int64_t)m * p.N + ec;
+    if (!vec) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        if (ec + u >= p.N) break;
+        if (e.acc_out) e.acc_out[idx + u] = a[u];
+        epi_store(epi_value((float)a[u], idx + u, ec + u, e), idx + u, e);
+      }
+      continue;
+    }
+    const v4f res = c_res[r];
+    auto run = [&](auto spec) {
+      typedef decltype(spec) S;
+      epi_vec4<S>(a, res, epi_lane_finish<S>(c_div, c_rcp, c_bias, e), idx, e);
+    };
+    switch (p.epi) {
+      case EPI_Q8_RELU: run(EpiOf<EPI_Q8_RELU>::type{}); break;
+      case EPI_RES_Y_Q8: run(EpiOf<EPI_RES_Y_Q8>::type{}); break;
+      case EPI_Y32: run(EpiOf<EPI_Y32>::type{}); break;
+      case EPI_RES_Q8: run(EpiOf<EPI_RES_Q8>::type{}); break;
+      case EPI_Q8_RELU6: run(EpiOf<EPI_Q8_RELU6>::type{}); break;
+      default: run(EpiGeneric{}); break;
+    }
+  }
+}
+
+static void magic(unsigned d, unsigned *m, unsigned *mask) {
+  *m = d <= 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d);
+  *mask = d <= 1 ? ~0u : 0u;
+}
+
+template <int T, int NW, bool DENSE>
+static int launch_small(const void *a, const void *b, SmallParams p, const EpiDev &e, hipStream_t s) {
+  constexpr int LDS_BYTES = NW * 2 * 2 * T * 128;
+  static_assert(LDS_BYTES <= 128 * 1024, "slots of all waves");
+  auto kern = small_i8_kernel<T, NW, DENSE>;
+  if (LDS_BYTES > 64 * 1024) {
+    static std::atomic<bool> raised[64];
+    if (raise_lds_limit((const void *)kern, LDS_BYTES, raised) != CATCHQ_OK) return CATCHQ_ERR_LAUNCH;
+  }
+  p.tiles_m = (p.M + T - 1) / T;
+  p.tiles_n = (p.N + T - 1) / T;
+  p.nblocks = p.tiles_m * p.tiles_n;
+  magic(p.m_fastest ? p.tiles_m : p.tiles_n, &p.magic_t, &p.mask_t);
+  kern<<<p.nblocks, 64 * NW, LDS_BYTES, s>>>((const int8_t *)a, (const int8_t *)b, p, e);
+  return launch_status();
+}
+
+// The shapes this kernel takes from the tiled ones.  kh = kw = 1, stride 1, no padding: a GEMM of M rows.  -1: not one.
+int contract_small_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                      int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
+  const int64_t M = (int64_t)N_img * Ho * Wo, K = (int64_t)kh * kw * Ci;
+  const int64_t a_bytes = (int64_t)N_img * H * W * Ci, b_bytes = (int64_t)Co * K;
+  if (Ci % 16 != 0 || M >= (1 << 20) || K >= (1 << 20) || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31)) return -1;
+  // the divisions through multiplication: dividend * divisor < 2^32
+  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+  if (!dense && (M * Wo >= (1ll << 32) || M * Ho >= (1ll << 32) || K * Ci >= (1ll << 32) || (int64_t)kh * kw * kw >= (1ll << 32) ||
+                 (int64_t)dh * kh >= (1 << 20) || (int64_t)dw * kw >= (1 << 20) || H >= (1 << 20) || W >= (1 << 20)))
+    return -1;
+  // Measured with the launch repeated in a graph (us, this kernel / the tiled ones; MI355X):
+  //   16 x 16 tiles while the device holds two per compute unit: 7x7 512->512 3x3 4.6 / 10.6, 14x14 256->256 3x3 4.0 / 7.7,
+  //     14x14/2 512->512 3x3 4.6 / 18.6, 1 x 3072 -> 768 3.4 / 7.0, 1 x 4096 -> 4096 3.8 / 8.5, 6x6x14 960->160 4.0 / 5.0
+  //   32 x 32 tiles up to one per unit: 784 x 256 x 512 3.4 / 3.7, 4 x 14x14 256->256 3x3 (200 tiles) 5.3 / 7.7
+  //     (K = 192 ties, K <= 128 loses: those launches are all set-up); to 1.75 per unit from K = 1024 on
+  //     (4 x 28x28 128->128 3x3, 392 tiles, 5.4 / 6.0; K = 512 loses, 4.3 / 3.7); more for the longest K
+  //     (197 x 4096 x 4096, 896 tiles, 13.8 / 16.8)
+  // Four waves share K (one wave's transfers and arithmetic run under another's wait; eight cost more set-up than they
+  // hide), eight where a step's tap arithmetic is long and the blocks do not fill the device.
+  const int64_t tiles32 = ((M + 31) / 32) * ((Co + 31) / 32), tiles16 = ((M + 15) / 16) * ((Co + 15) / 16);
+  const int steps = (int)((K + 127) / 128);
+  int T = 0, NW = 4;
+  if (tiles16 <= 2 * e.cus && K >= 64) {
+    T = 16;
+    if (!dense && steps >= 16 && tiles16 <= e.cus) NW = 8;
+  } else if ((tiles32 <= e.cus && K >= 256) || (tiles32 * 4 <= 7 * e.cus && K >= 1024) || (tiles32 * 2 <= 7 * e.cus && K >= 3072)) {
+    T = 32;
+    if (!dense && steps >= 32 && tiles32 <= e.cus) NW = 8;
+  }
+  if (const char *f = tuning_env("CATCHQ_SMALL")) {
+    const int v = std::atoi(f);  // 0: off; T * 100 + NW
+    T = v / 100;
+    NW = v % 100;
+  }
+  if (!T) return -1;
+  SmallParams p = {};
+  p.M = (int)M; p.N = Co; p.K = (int)K;
+  p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
+  p.img_stride = (unsigned)(H * W * Ci); p.row_stride = (unsigned)(W * Ci); p.pix_stride = (unsigned)Ci;
+  magic(Wo, &p.magic_wo, &p.mask_wo); magic(Ho, &p.magic_ho, &p.mask_ho);
+  magic(Ci, &p.magic_ci, &p.mask_ci); magic(kw, &p.magic_kw, &p.mask_kw);
+  p.m_fastest = b_bytes > a_bytes;
+  p.epi = pick_epilogue(Co, e);
+  p.a_bytes = (unsigned)a_bytes; p.b_bytes = (unsigned)b_bytes;
+#define CATCHQ_SMALL_CASE(T_, NW_) \
+  case T_ * 100 + NW_: return dense ? launch_small<T_, NW_, true>(x, w, p, e, s) : launch_small<T_, NW_, false>(x, w, p, e, s)
+  switch (T * 100 + NW) {
+    CATCHQ_SMALL_CASE(32, 4);
+    CATCHQ_SMALL_CASE(32, 8);
+    CATCHQ_SMALL_CASE(16, 4);
+    CATCHQ_SMALL_CASE(16, 8);
+    default: return -1;
+  }
+#undef CATCHQ_SMALL_CASE
+}
+
+}  // namespace catchq

@@ -252,6 +252,49 @@ def test_gemm_random_sweep(seed):
             assert same_bits(orc.quantize(y, q_bw, q_pos, q_scale), out["q"].cpu().numpy()), case
 
 
+# few output tiles: K split over the waves of a block.  Both tile sizes, four and eight waves, edges of the tiles and of the
+# 128-byte K steps (fewer steps than waves, K ending inside a step and inside a 16-byte piece of a tap), channels not a
+# multiple of four
+FEW_TILES_CASES = [
+    # n, h, w, ci, co, k, pad, stride, dil
+    (1, 1, 1, 64, 4, 1, 0, 1, 1), (15, 1, 1, 112, 33, 1, 0, 1, 1), (17, 1, 1, 144, 16, 1, 0, 1, 1),
+    (16, 1, 1, 4096, 1001, 1, 0, 1, 1), (33, 1, 1, 528, 1000, 1, 0, 1, 1), (197, 1, 1, 1040, 768, 1, 0, 1, 1),
+    (300, 1, 1, 3088, 1100, 1, 0, 1, 1), (1, 7, 7, 512, 512, 3, 1, 1, 1), (1, 14, 14, 512, 500, 3, 1, 2, 1),
+    (3, 9, 5, 16, 30, 3, 1, 1, 1), (2, 13, 11, 48, 66, 5, 2, 2, 1), (2, 12, 10, 80, 40, 3, 2, 1, 2),
+    (4, 14, 14, 256, 256, 3, 1, 1, 1), (4, 28, 28, 128, 128, 3, 1, 1, 1), (2, 14, 14, 512, 320, 3, 1, 1, 1),
+    (1, 14, 14, 96, 200, 1, 0, 2, 1), (2, 20, 20, 64, 48, 7, 0, 1, 1)]
+
+
+@pytest.mark.parametrize("case", FEW_TILES_CASES)
+def test_few_output_tiles(case):
+    n, h, w, ci, co, k, pad, stride, dil = case
+    note("few tiles", case)
+    r = rng(sum(case) * 11)
+    x, wt = _ints(r, (n, h, w, ci), 8), _ints(r, (co, k, k, ci), 8)
+    acc, ovf = orc.conv2d_nhwc(x, wt, (pad, pad), (stride, stride), (dil, dil), 1)
+    assert ovf == 0
+    div = r.uniform(0.6, 3.5, co).astype(np.float32)
+    bias = r.standard_normal(co).astype(np.float32)
+    res = (r.standard_normal(acc.shape) * 20).astype(np.float32)
+    args = dict(padding=(pad, pad), stride=(stride, stride), dilation=(dil, dil), exp2=-10)
+    xd, wd = cabi.dev(x), cabi.dev(wt)
+    dd, bd, rd, rcp = cabi.dev(div), cabi.dev(bias), cabi.dev(res), cabi.dev(np.float32(1) / div)
+    # (output, quantized output, activation, residual, accumulators): the specialised epilogues and the generic one
+    for y_dtype, q_bw, act, use_res, want_acc in ((torch.float32, 0, 0, False, True), (torch.float32, 0, 0, False, False),
+                                                  (None, 8, 1, False, False), (None, 8, 2, False, False),
+                                                  (torch.float32, 8, 1, True, False), (None, 8, 1, True, False),
+                                                  (torch.float16, 16, 0, True, False)):
+        out = cabi.conv2d_nhwc(xd, wd, chan_div=dd, chan_rcp=rcp, bias=bd, resid=rd if use_res else None, act=act,
+                               y_dtype=y_dtype, want_acc=want_acc, q_bw=q_bw, q_pos=-3, **args)
+        y = orc.epilogue(acc, -10, div, bias, res if use_res else None, act)
+        if want_acc:
+            assert same_bits(acc.astype(np.int32), out["acc"].cpu().numpy())
+        if y_dtype is not None:
+            assert same_bits(y.astype(np.float16) if y_dtype == torch.float16 else y, out["y"].cpu().numpy())
+        if q_bw:
+            assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
+
+
 def test_division_by_reciprocal_is_exact():
     """v/d evaluated as q=v*r, e=fma(-q,d,v), fma(e,r,q) with r = RN(1/d) must equal IEEE division bit
     for bit: adversarial divisor significands x a wide set of dividends x several exponents."""
