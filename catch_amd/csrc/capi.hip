@@ -24,6 +24,12 @@ int conv2d_mfma_a16w16(const void *x, const void *w, int N, int H, int W, int Ci
 int conv2d_dual_i8(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                    int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws, int Cs,
                    int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
+int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                           int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws,
+                           int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
+bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus);
+int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
+                         int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
 struct ChainLinkDev {  // igemm_i8_chain.hip
   const int8_t *x, *w;
   unsigned x_bytes, w_bytes;
@@ -266,7 +272,11 @@ CATCHQ_API int catchq_conv2d_shortcut_nhwc(const void *x, int x_bits, const void
     sd.chan_div = sc.chan_div;
     sd.chan_rcp = (sc.chan_div && sc.chan_rcp && sc.exp2 >= -64 && sc.exp2 <= 64) ? sc.chan_rcp : nullptr;
     sd.bias = sc.bias;
-    const int st2 = conv2d_dual_i8(x, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h, d.stride_w,
+    int st2 = contract_small_dual_i8(x, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h, d.stride_w,
+                                     d.dil_h, d.dil_w, ho, wo, sc.x, sc.w, sc.in_h, sc.in_w, sc.ci, sc.stride, e, sd,
+                                     as_stream(stream));
+    if (st2 >= 0) return st2;
+    st2 = conv2d_dual_i8(x, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h, d.stride_w,
                                    d.dil_h, d.dil_w, ho, wo, sc.x, sc.w, sc.in_h, sc.in_w, sc.ci, sc.stride, e, sd,
                                    as_stream(stream));
     if (st2 >= 0) return st2;
@@ -288,6 +298,51 @@ CATCHQ_API int catchq_conv2d_shortcut_nhwc(const void *x, int x_bits, const void
   catchq_epilogue_t em = *epilogue;
   em.resid = (const float *)workspace;
   return catchq_conv2d_nhwc(x, x_bits, w, w_bits, desc, &em, stream);
+}
+
+// shapes that quantize and contract in one launch (pointer alignment is checked at the call)
+static bool float_conv_fusable(const catchq_conv_desc_t *d, int ho, int wo, const catchq_epilogue_t *e) {
+  const bool dense = d->kh == 1 && d->kw == 1 && d->stride_h == 1 && d->stride_w == 1 && d->pad_h == 0 && d->pad_w == 0;
+  return d->groups == 1 && contract_small_float_ok((int64_t)d->n * ho * wo, d->co, (int64_t)d->kh * d->kw * d->ci, dense, d->ci,
+                                                   planned_cus(e->sharing));
+}
+
+CATCHQ_API int catchq_float_conv2d_workspace_size(int x_dtype, const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue,
+                                                  size_t *bytes) {
+  int ho, wo;
+  const int st = check_conv(desc, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  if (!bytes || !epilogue) return CATCHQ_ERR_ARG;
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  *bytes = float_conv_fusable(desc, ho, wo, epilogue) ? 0 : (size_t)desc->n * desc->h * desc->w * desc->ci;
+  return CATCHQ_OK;
+}
+
+CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_position, const void *w, const catchq_conv_desc_t *desc,
+                                        const catchq_epilogue_t *epilogue, void *workspace, size_t workspace_bytes,
+                                        catchq_stream_t stream) {
+  int ho, wo;
+  int st = check_conv(desc, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  st = check_epi(epilogue);
+  if (st != CATCHQ_OK) return st;
+  if (x_position < -126 || x_position > 126) return CATCHQ_ERR_ARG;
+  if (desc->n == 0) return CATCHQ_OK;
+  if (!x || !w) return CATCHQ_ERR_ARG;
+  const catchq_conv_desc_t &d = *desc;
+  if (float_conv_fusable(desc, ho, wo, epilogue) && aligned16(x) && aligned16(w)) {
+    const EpiDev e = make_epi(epilogue, (int64_t)d.n * ho * wo * d.co);
+    const int st2 = contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
+                                         d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
+    if (st2 >= 0) return st2;
+  }
+  // two launches: the quantized activations go through the workspace
+  const int64_t need = (int64_t)d.n * d.h * d.w * d.ci;
+  if (!workspace || workspace_bytes < (size_t)need || !aligned16(workspace)) return CATCHQ_ERR_ARG;
+  st = catchq_quantize(x, x_dtype, workspace, 8, need, x_position, 1.0f, stream);
+  if (st != CATCHQ_OK) return st;
+  return catchq_conv2d_nhwc(workspace, 8, w, 8, desc, epilogue, stream);
 }
 
 CATCHQ_API int catchq_conv1x1_chain_nhwc(const catchq_chain_link_t *links, int nlinks, int n, int ho, int wo, int co,

@@ -16,17 +16,31 @@ namespace catchq {
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
-struct SmallParams {
-  int M, N, K;       // M < 2^20, K < 2^20
-  int H, W, Ci, Ho, Wo, kw, ph, pw, sh, sw, dh, dw;
+// One contraction: activations [.., H, W, Ci] (int8, or floats that the loader quantizes) against filters [N][K]
+struct SmallSide {
+  const void *x;
+  const int8_t *w;
+  int K;             // kh * kw * Ci < 2^20
+  int H, W, Ci, kw, ph, pw, sh, sw, dh, dw;
   unsigned img_stride, row_stride, pix_stride;  // elements
-  unsigned magic_wo, magic_ho, magic_ci, magic_kw, magic_t;  // ceil(2^32 / d); 0 for d = 1, whose mask is all ones
-  unsigned mask_wo, mask_ho, mask_ci, mask_kw, mask_t;
-  int tiles_m, tiles_n, nblocks;
-  int m_fastest;     // consecutive blocks walk the row tiles of one column tile first
-  int epi;           // epilogue variant (EPI_*), the same for every block
+  unsigned magic_ci, magic_kw, mask_ci, mask_kw;  // ceil(2^32 / d), mask 0; for d = 1 magic 0, mask ~0
   unsigned a_bytes, b_bytes;
 };
+
+struct SmallParams {
+  SmallSide side[2];  // [1]: the projection shortcut of a two-branch launch
+  int M, N;           // M < 2^20
+  int Ho, Wo;
+  unsigned magic_wo, magic_ho, magic_t, mask_wo, mask_ho, mask_t;
+  int tiles_m, tiles_n, nblocks;
+  int m_fastest;      // consecutive blocks walk the row tiles of one column tile first
+  int epi;            // epilogue variant (EPI_*), the same for every block
+  int main_waves;     // two-branch launches: waves 0 .. main_waves - 1 run side 0, the others side 1
+  int x_neg_pos;      // floating activations: quantized at 2^-x_neg_pos
+  ShortcutDev sc;
+};
+
+enum { SMALL_I8 = 0, SMALL_F32 = 1, SMALL_F16 = 2 };
 
 #define CATCHQ_SMALL_VMCNT(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 
@@ -38,10 +52,39 @@ __device__ __forceinline__ v4i small_ds_read(unsigned addr) {
   asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr));
   return v;
 }
-// DENSE: a plain GEMM -- row m starts at m * K, no taps
-template <int T, int NW, bool DENSE>
-__global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restrict__ A, const int8_t *__restrict__ B,
-                                                          SmallParams p, EpiDev e) {
+__device__ __forceinline__ void small_ds_write(unsigned addr, v4i v) {
+  asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory");
+}
+
+// 16 floats (or halfs) -> 16 int8, the quantizer's own arithmetic with unit scale
+template <int IN>
+__device__ __forceinline__ v4i small_quantize(const v4i *raw, int neg_pos) {
+  v4i q;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    int b[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float v;
+      if constexpr (IN == SMALL_F32) v = __int_as_float(raw[d][t]);
+      else {
+        const int pair = raw[d >> 1][(d & 1) * 2 + (t >> 1)];
+        v = (float)__builtin_bit_cast(_Float16, (short)((t & 1) ? pair >> 16 : pair & 0xffff));
+      }
+      b[t] = quant1_unit<8>(v, neg_pos);
+    }
+    const unsigned lo = __builtin_amdgcn_perm((unsigned)b[1], (unsigned)b[0], 0x0c0c0400u);
+    const unsigned hi = __builtin_amdgcn_perm((unsigned)b[3], (unsigned)b[2], 0x04000c0cu);
+    q[d] = (int)(lo | hi);
+  }
+  return q;
+}
+
+// DENSE: a plain GEMM -- row m starts at m * K, no taps.  IN: type of the activations.  DUAL: a residual block's last
+// convolution and its projection shortcut over the same output tile; the block's waves are shared out between the two
+// in proportion to their K steps, and the shortcut's sums, dequantized with its own constants, are the residual.
+template <int T, int NW, bool DENSE, int IN, bool DUAL>
+__global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev e) {
   resolve_exp2(e);
   constexpr int SLOTS = 2, BKB = 128;
   constexpr int SLOT_BYTES = 2 * T * BKB, WAVE_BYTES = SLOTS * SLOT_BYTES;
@@ -57,8 +100,12 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
   const int inner = logical - outer * (p.m_fastest ? p.tiles_m : p.tiles_n);
   const int tile_m = p.m_fastest ? inner : outer, tile_n = p.m_fastest ? outer : inner;
   const int m0 = tile_m * T, n0 = tile_n * T;
-  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)p.a_bytes, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)p.b_bytes, 0x00020000);
+  const bool second = DUAL && wave >= p.main_waves;  // wave-uniform
+  const SmallSide &o = p.side[second ? 1 : 0];
+  const int group_wave = second ? wave - p.main_waves : wave;
+  const int group = DUAL ? (second ? NW - p.main_waves : p.main_waves) : NW;
+  const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)o.x, 0, (int)o.a_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)o.w, 0, (int)o.b_bytes, 0x00020000);
   constexpr unsigned OOB = 0x80000000u;  // the hardware answers an offset beyond the buffer with zeros
 
   // the epilogue's lanes: four channels of one pixel each, T * T / 4 of them (waves 0 ..)
@@ -67,6 +114,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
   const bool vec = p.epi != EPI_SCALAR;
   constexpr int ROUNDS = (EPI_LANES + 64 * NW - 1) / (64 * NW);
   v4f c_div = {1.f, 1.f, 1.f, 1.f}, c_rcp = c_div, c_bias = {0.f, 0.f, 0.f, 0.f}, c_res[ROUNDS];
+  v4f s_div = c_div, s_rcp = c_div, s_bias = c_bias;  // the shortcut's constants
   // 64 * NW is a multiple of CPR: a lane has the same four channels in every round.  (Plain loads: the transfers below
   // and the statements that clobber memory keep them here, in front of the K loop.)
   const int ec = n0 + (threadIdx.x % CPR) * 4;
@@ -75,11 +123,16 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
     if (e.chan_div) c_div = *reinterpret_cast<const v4f *>(e.chan_div + cc);
     if (e.chan_rcp) c_rcp = *reinterpret_cast<const v4f *>(e.chan_rcp + cc);
     if (e.bias) c_bias = *reinterpret_cast<const v4f *>(e.bias + cc);
+    if constexpr (DUAL) {
+      if (p.sc.chan_div) s_div = *reinterpret_cast<const v4f *>(p.sc.chan_div + cc);
+      if (p.sc.chan_rcp) s_rcp = *reinterpret_cast<const v4f *>(p.sc.chan_rcp + cc);
+      if (p.sc.bias) s_bias = *reinterpret_cast<const v4f *>(p.sc.bias + cc);
+    }
 #pragma unroll
     for (int r = 0; r < ROUNDS; ++r) {
       c_res[r] = v4f{0.f, 0.f, 0.f, 0.f};
       const int em = min(m0 + (int)(threadIdx.x + r * 64 * NW) / CPR, p.M - 1);
-      if (e.resid) c_res[r] = *reinterpret_cast<const v4f *>(e.resid + (int64_t)em * p.N + cc);
+      if (!DUAL && e.resid) c_res[r] = *reinterpret_cast<const v4f *>(e.resid + (int64_t)em * p.N + cc);
     }
   }
 
@@ -96,24 +149,28 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
     const int m = m0 + j * 8 + lrow;
     if constexpr (DENSE) {
       a_hi[j] = a_wi[j] = 0;
-      a_base[j] = m < p.M ? (unsigned)m * (unsigned)p.K : OOB;
+      a_base[j] = m < p.M ? (unsigned)m * (unsigned)o.K : OOB;
     } else {
       const unsigned t = div_magic((unsigned)m, p.magic_wo, p.mask_wo), wo = (unsigned)m - t * (unsigned)p.Wo;
       const unsigned img = div_magic(t, p.magic_ho, p.mask_ho), ho = t - img * (unsigned)p.Ho;
-      a_hi[j] = m < p.M ? (int)ho * p.sh - p.ph : -(1 << 30);  // a row that does not exist is outside the image
-      a_wi[j] = (int)wo * p.sw - p.pw;
-      a_base[j] = img * p.img_stride + (unsigned)a_hi[j] * p.row_stride + (unsigned)a_wi[j] * p.pix_stride;  // mod 2^32
+      a_hi[j] = m < p.M ? (int)ho * o.sh - o.ph : -(1 << 30);  // a row that does not exist is outside the image
+      a_wi[j] = (int)wo * o.sw - o.pw;
+      a_base[j] = img * o.img_stride + (unsigned)a_hi[j] * o.row_stride + (unsigned)a_wi[j] * o.pix_stride;  // mod 2^32
     }
     const int n = n0 + j * 8 + lrow;
-    b_base[j] = n < p.N ? (unsigned)n * (unsigned)p.K : OOB;
+    b_base[j] = n < p.N ? (unsigned)n * (unsigned)o.K : OOB;
   }
-  const int steps = (p.K + BKB - 1) / BKB;
-  const int per = steps / NW, rem = steps - per * NW;
-  const int first = wave * per + (wave < rem ? wave : rem);
-  const int mine = per + (wave < rem ? 1 : 0);
+  const int steps = (o.K + BKB - 1) / BKB;
+  const int per = steps / group, rem = steps - per * group;
+  const int first = group_wave * per + (group_wave < rem ? group_wave : rem);
+  const int mine = per + (group_wave < rem ? 1 : 0);
   int8_t *const my = lds + wave * WAVE_BYTES;
 
-  auto issue = [&](int s) {  // step s of this wave's slice into its slot s & 1
+  constexpr int ES = IN == SMALL_F32 ? 4 : (IN == SMALL_F16 ? 2 : 1);  // bytes per activation
+  constexpr int RAW = ES;  // 16-byte loads per 16 activations
+  v4i raw[NA][RAW];
+  (void)raw;
+  auto issue = [&](int s) {  // step s of this wave's slice into its slot s & 1 (floating activations: into raw)
     const int slot = (s & 1) * SLOT_BYTES;
     unsigned k[2], koff[2];
     int dy[2], dx[2];
@@ -121,33 +178,41 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       k[h] = (unsigned)((first + s) * BKB + (chunk0 ^ (4 * h)) * 16);
-      ok[h] = (s < mine) & (k[h] < (unsigned)p.K);
+      ok[h] = (s < mine) & (k[h] < (unsigned)o.K);
       koff[h] = k[h];
       dy[h] = dx[h] = 0;
       if constexpr (!DENSE) {
-        const unsigned tap = div_magic(k[h], p.magic_ci, p.mask_ci), ci = k[h] - tap * (unsigned)p.Ci;
-        const unsigned r = div_magic(tap, p.magic_kw, p.mask_kw), q = tap - r * (unsigned)p.kw;
-        dy[h] = (int)r * p.dh;
-        dx[h] = (int)q * p.dw;
-        koff[h] = (unsigned)dy[h] * p.row_stride + (unsigned)dx[h] * p.pix_stride + ci;
+        const unsigned tap = div_magic(k[h], o.magic_ci, o.mask_ci), ci = k[h] - tap * (unsigned)o.Ci;
+        const unsigned r = div_magic(tap, o.magic_kw, o.mask_kw), q = tap - r * (unsigned)o.kw;
+        dy[h] = (int)r * o.dh;
+        dx[h] = (int)q * o.dw;
+        koff[h] = (unsigned)dy[h] * o.row_stride + (unsigned)dx[h] * o.pix_stride + ci;
       }
+    }
+    // (the filters first: loads complete in order, so a wave that has its activations has its filters)
+#pragma unroll
+    for (int j = 0; j < NA; ++j) {
+      const int h = j & 1;
+      unsigned voff = ok[h] ? b_base[j] + k[h] : OOB;
+      asm volatile("" : "+v"(voff));  // one select and one load, not two loads under complementary masks
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(my + slot + (NA + j) * 1024), 16, (int)voff, 0, 0, 0);
     }
 #pragma unroll
     for (int j = 0; j < NA; ++j) {
       const int h = j & 1;
       bool in = ok[h];
       if constexpr (!DENSE)
-        in = in & ((unsigned)(a_hi[j] + dy[h]) < (unsigned)p.H) & ((unsigned)(a_wi[j] + dx[h]) < (unsigned)p.W);
-      unsigned voff = in ? a_base[j] + koff[h] : OOB;
-      asm volatile("" : "+v"(voff));  // one select and one load, not two loads under complementary masks
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
-    }
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      const int h = j & 1;
-      unsigned voff = ok[h] ? b_base[j] + k[h] : OOB;
+        in = in & ((unsigned)(a_hi[j] + dy[h]) < (unsigned)o.H) & ((unsigned)(a_wi[j] + dx[h]) < (unsigned)o.W);
+      if constexpr (DENSE) in = in & (a_base[j] != OOB);
+      unsigned voff = in ? (a_base[j] + koff[h]) * (unsigned)ES : OOB;
       asm volatile("" : "+v"(voff));
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(my + slot + (NA + j) * 1024), 16, (int)voff, 0, 0, 0);
+      if constexpr (IN == SMALL_I8) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
+      } else {
+#pragma unroll
+        for (int r = 0; r < RAW; ++r)
+          raw[j][r] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)voff + 16 * r, 0, 0));
+      }
     }
   };
 
@@ -156,12 +221,26 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
   acc_t acc = {};
   if (mine > 0) {
     const int frow = lane & (T - 1), fk = lane / T;  // row of the fragment, 16-byte piece within a sub-step
-    const unsigned a_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t *)my + (unsigned)(frow * BKB);
+    const unsigned my_addr = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t *)my;
+    const unsigned a_addr = my_addr + (unsigned)(frow * BKB);
     const unsigned sw = (unsigned)((frow >> 1) & 7);
     issue(0);
-    issue(1);  // (past the slice: nothing but zeros, so that the count of transfers in flight stays the same)
+    if constexpr (IN == SMALL_I8) issue(1);  // (past the slice: nothing but zeros, so that the number in flight stays the same)
     for (int s = 0; s < mine; ++s) {
-      CATCHQ_SMALL_VMCNT(NI);
+      if constexpr (IN == SMALL_I8) {
+        CATCHQ_SMALL_VMCNT(NI);
+      } else {
+        // the step's activations have arrived, and with them its filters: quantized into the slot, as a transfer
+        // would have left them; then the next step's loads
+        v4i q[NA];
+#pragma unroll
+        for (int j = 0; j < NA; ++j) q[j] = small_quantize<IN>(raw[j], p.x_neg_pos);
+#pragma unroll
+        for (int j = 0; j < NA; ++j)
+          small_ds_write(my_addr + (unsigned)((s & 1) * SLOT_BYTES + j * 1024 + lane * 16), q[j]);
+        issue(s + 1);
+        CATCHQ_SMALL_VMCNT(NA + NA * RAW);
+      }
       const unsigned base = a_addr + (unsigned)((s & 1) * SLOT_BYTES);
       v4i fa[SUB], fb[SUB];
 #pragma unroll
@@ -172,7 +251,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
       }
 #pragma unroll
       for (int u = 0; u < SUB; ++u) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[u]), "+v"(fb[u])::"memory");
-      issue(s + 2);  // the slot has been read
+      if constexpr (IN == SMALL_I8) issue(s + 2);  // the slot has been read
       // operands swapped (weights as A): a lane ends up with four consecutive channels of one pixel
 #pragma unroll
       for (int u = 0; u < SUB; ++u) {
@@ -194,7 +273,9 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
   if (!epi_wave) return;
 
   // ---- partial sums -> outputs ---------------------------------------------------------------------------------------
-  const int active = steps < NW ? steps : NW;
+  auto steps_of = [&](int K) { return (K + BKB - 1) / BKB; };
+  const int main_group = DUAL ? p.main_waves : NW;
+  const int main_active = min(steps_of(p.side[0].K), main_group);
 #pragma unroll
   for (int r = 0; r < ROUNDS; ++r) {
     const int t = threadIdx.x + r * 64 * NW;
@@ -203,7 +284,19 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
     const int m = m0 + px;
     const int *part = reinterpret_cast<const int *>(lds) + px * PITCH + cg * 4;
     v4i a = *reinterpret_cast<const v4i *>(part);
-    for (int w = 1; w < active; ++w) a += *reinterpret_cast<const v4i *>(part + w * (WAVE_BYTES / 4));
+    for (int w = 1; w < main_active; ++w) a += *reinterpret_cast<const v4i *>(part + w * (WAVE_BYTES / 4));
+    v4f res = c_res[r];
+    if constexpr (DUAL) {
+      const int active = min(steps_of(p.side[1].K), NW - main_group);
+      const int *part2 = part + main_group * (WAVE_BYTES / 4);
+      v4i a2 = *reinterpret_cast<const v4i *>(part2);
+      for (int w = 1; w < active; ++w) a2 += *reinterpret_cast<const v4i *>(part2 + w * (WAVE_BYTES / 4));
+      EpiDev es = {};
+      es.exp2 = p.sc.exp2; es.chan_div = p.sc.chan_div; es.chan_rcp = p.sc.chan_rcp; es.bias = p.sc.bias;
+      const EpiLane ls = epi_lane_finish<EpiGeneric>(s_div, s_rcp, s_bias, es);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) res[u] = epi_dequant1(a2[u], u, ls, es.exp2);
+    }
     if (m >= p.M || ec >= p.N) continue;
     const int64_t idx = (int64_t)m * p.N + ec;
     if (!vec) {
@@ -215,10 +308,14 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(const int8_t *__restr
       }
       continue;
     }
-    const v4f res = c_res[r];
     auto run = [&](auto spec) {
       typedef decltype(spec) S;
-      epi_vec4<S>(a, res, epi_lane_finish<S>(c_div, c_rcp, c_bias, e), idx, e);
+      EpiLane L = epi_lane_finish<S>(c_div, c_rcp, c_bias, e);
+      if constexpr (DUAL) {
+        L.use_res = true;
+        L.res_after = e.resid_after != 0;
+      }
+      epi_vec4<S>(a, res, L, idx, e);
     };
     switch (p.epi) {
       case EPI_Q8_RELU: run(EpiOf<EPI_Q8_RELU>::type{}); break;
@@ -236,11 +333,11 @@ static void magic(unsigned d, unsigned *m, unsigned *mask) {
   *mask = d <= 1 ? ~0u : 0u;
 }
 
-template <int T, int NW, bool DENSE>
-static int launch_small(const void *a, const void *b, SmallParams p, const EpiDev &e, hipStream_t s) {
+template <int T, int NW, bool DENSE, int IN, bool DUAL>
+static int launch_small(SmallParams p, const EpiDev &e, hipStream_t s) {
   constexpr int LDS_BYTES = NW * 2 * 2 * T * 128;
   static_assert(LDS_BYTES <= 128 * 1024, "slots of all waves");
-  auto kern = small_i8_kernel<T, NW, DENSE>;
+  auto kern = small_i8_kernel<T, NW, DENSE, IN, DUAL>;
   if (LDS_BYTES > 64 * 1024) {
     static std::atomic<bool> raised[64];
     if (raise_lds_limit((const void *)kern, LDS_BYTES, raised) != CATCHQ_OK) return CATCHQ_ERR_LAUNCH;
@@ -249,65 +346,128 @@ static int launch_small(const void *a, const void *b, SmallParams p, const EpiDe
   p.tiles_n = (p.N + T - 1) / T;
   p.nblocks = p.tiles_m * p.tiles_n;
   magic(p.m_fastest ? p.tiles_m : p.tiles_n, &p.magic_t, &p.mask_t);
-  kern<<<p.nblocks, 64 * NW, LDS_BYTES, s>>>((const int8_t *)a, (const int8_t *)b, p, e);
+  if (DUAL) {
+    const int s1 = (p.side[0].K + 127) / 128, s2 = (p.side[1].K + 127) / 128;
+    p.main_waves = (NW * s1 + (s1 + s2) / 2) / (s1 + s2);
+    p.main_waves = p.main_waves < 1 ? 1 : (p.main_waves > NW - 1 ? NW - 1 : p.main_waves);
+  }
+  kern<<<p.nblocks, 64 * NW, LDS_BYTES, s>>>(p, e);
   return launch_status();
+}
+
+// One side's constants; false where the kernel's 32-bit arithmetic does not cover the shape.
+static bool small_side(SmallSide *o, const void *x, int x_size, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
+                       int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense) {
+  const int64_t M = (int64_t)N_img * Ho * Wo, K = (int64_t)kh * kw * Ci;
+  const int64_t a_bytes = (int64_t)N_img * H * W * Ci * x_size, b_bytes = (int64_t)Co * K;
+  if (Ci % 16 != 0 || M >= (1 << 20) || K >= (1 << 20) || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31)) return false;
+  // the divisions through multiplication: dividend * divisor < 2^32
+  if (!dense && (M * Wo >= (1ll << 32) || M * Ho >= (1ll << 32) || K * Ci >= (1ll << 32) || (int64_t)kh * kw * kw >= (1ll << 32) ||
+                 (int64_t)dh * kh >= (1 << 20) || (int64_t)dw * kw >= (1 << 20) || H >= (1 << 20) || W >= (1 << 20)))
+    return false;
+  o->x = x; o->w = (const int8_t *)w;
+  o->K = (int)K;
+  o->H = H; o->W = W; o->Ci = Ci; o->kw = kw; o->ph = ph; o->pw = pw; o->sh = sh; o->sw = sw; o->dh = dh; o->dw = dw;
+  o->img_stride = (unsigned)((int64_t)H * W * Ci); o->row_stride = (unsigned)((int64_t)W * Ci); o->pix_stride = (unsigned)Ci;
+  magic(Ci, &o->magic_ci, &o->mask_ci);
+  magic(kw, &o->magic_kw, &o->mask_kw);
+  o->a_bytes = (unsigned)a_bytes; o->b_bytes = (unsigned)b_bytes;
+  return true;
+}
+
+// Tile and waves (T * 100 + NW) for M x N outputs over `steps` 128-byte K steps, 0: not this kernel's shape.
+//
+// Measured with the launch repeated in a graph (us, this kernel / the tiled ones; MI355X):
+//   16 x 16 tiles while the device holds two per compute unit: 7x7 512->512 3x3 4.6 / 10.6, 14x14 256->256 3x3 4.0 / 7.7,
+//     14x14/2 512->512 3x3 4.6 / 18.6, 1 x 3072 -> 768 3.4 / 7.0, 1 x 4096 -> 4096 3.8 / 8.5, 6x6x14 960->160 4.0 / 5.0
+//   32 x 32 tiles up to one per unit: 784 x 256 x 512 3.4 / 3.7, 4 x 14x14 256->256 3x3 (200 tiles) 5.3 / 7.7
+//     (K = 192 ties, K <= 128 loses: those launches are all set-up); to 1.75 per unit from K = 1024 on
+//     (4 x 28x28 128->128 3x3, 392 tiles, 5.4 / 6.0; K = 512 loses, 4.3 / 3.7); more for the longest K
+//     (197 x 4096 x 4096, 896 tiles, 13.8 / 16.8)
+// Four waves share K (one wave's transfers and arithmetic run under another's wait; eight cost more set-up than they
+// hide), eight where a step's tap arithmetic is long and the blocks do not fill the device.
+static int small_plan(int64_t M, int64_t N, int64_t K, bool dense, int cus) {
+  const int64_t tiles32 = ((M + 31) / 32) * ((N + 31) / 32), tiles16 = ((M + 15) / 16) * ((N + 15) / 16);
+  const int steps = (int)((K + 127) / 128);
+  int plan = 0;
+  if (tiles16 <= 2 * cus && K >= 64)
+    plan = (!dense && steps >= 16 && tiles16 <= cus) ? 1608 : 1604;
+  else if ((tiles32 <= cus && K >= 256) || (tiles32 * 4 <= 7 * cus && K >= 1024) || (tiles32 * 2 <= 7 * cus && K >= 3072))
+    plan = (!dense && steps >= 32 && tiles32 <= cus) ? 3208 : 3204;
+  if (const char *f = tuning_env("CATCHQ_SMALL")) plan = std::atoi(f);
+  return plan;
+}
+
+template <bool DENSE, int IN, bool DUAL>
+static int launch_small_plan(int plan, const SmallParams &p, const EpiDev &e, hipStream_t s) {
+  switch (plan) {
+    case 3204: return launch_small<32, 4, DENSE, IN, DUAL>(p, e, s);
+    case 3208: return launch_small<32, 8, DENSE, IN, DUAL>(p, e, s);
+    case 1604: return launch_small<16, 4, DENSE, IN, DUAL>(p, e, s);
+    case 1608: return launch_small<16, 8, DENSE, IN, DUAL>(p, e, s);
+    default: return -1;
+  }
+}
+
+static void small_common(SmallParams *p, int64_t M, int Co, int Ho, int Wo, const EpiDev &pick) {
+  p->M = (int)M; p->N = Co; p->Ho = Ho; p->Wo = Wo;
+  magic(Wo, &p->magic_wo, &p->mask_wo);
+  magic(Ho, &p->magic_ho, &p->mask_ho);
+  p->m_fastest = p->side[0].b_bytes > p->side[0].a_bytes;
+  p->epi = pick_epilogue(Co, pick);
 }
 
 // The shapes this kernel takes from the tiled ones.  kh = kw = 1, stride 1, no padding: a GEMM of M rows.  -1: not one.
 int contract_small_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                       int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
-  const int64_t M = (int64_t)N_img * Ho * Wo, K = (int64_t)kh * kw * Ci;
-  const int64_t a_bytes = (int64_t)N_img * H * W * Ci, b_bytes = (int64_t)Co * K;
-  if (Ci % 16 != 0 || M >= (1 << 20) || K >= (1 << 20) || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31)) return -1;
-  // the divisions through multiplication: dividend * divisor < 2^32
   const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-  if (!dense && (M * Wo >= (1ll << 32) || M * Ho >= (1ll << 32) || K * Ci >= (1ll << 32) || (int64_t)kh * kw * kw >= (1ll << 32) ||
-                 (int64_t)dh * kh >= (1 << 20) || (int64_t)dw * kw >= (1 << 20) || H >= (1 << 20) || W >= (1 << 20)))
-    return -1;
-  // Measured with the launch repeated in a graph (us, this kernel / the tiled ones; MI355X):
-  //   16 x 16 tiles while the device holds two per compute unit: 7x7 512->512 3x3 4.6 / 10.6, 14x14 256->256 3x3 4.0 / 7.7,
-  //     14x14/2 512->512 3x3 4.6 / 18.6, 1 x 3072 -> 768 3.4 / 7.0, 1 x 4096 -> 4096 3.8 / 8.5, 6x6x14 960->160 4.0 / 5.0
-  //   32 x 32 tiles up to one per unit: 784 x 256 x 512 3.4 / 3.7, 4 x 14x14 256->256 3x3 (200 tiles) 5.3 / 7.7
-  //     (K = 192 ties, K <= 128 loses: those launches are all set-up); to 1.75 per unit from K = 1024 on
-  //     (4 x 28x28 128->128 3x3, 392 tiles, 5.4 / 6.0; K = 512 loses, 4.3 / 3.7); more for the longest K
-  //     (197 x 4096 x 4096, 896 tiles, 13.8 / 16.8)
-  // Four waves share K (one wave's transfers and arithmetic run under another's wait; eight cost more set-up than they
-  // hide), eight where a step's tap arithmetic is long and the blocks do not fill the device.
-  const int64_t tiles32 = ((M + 31) / 32) * ((Co + 31) / 32), tiles16 = ((M + 15) / 16) * ((Co + 15) / 16);
-  const int steps = (int)((K + 127) / 128);
-  int T = 0, NW = 4;
-  if (tiles16 <= 2 * e.cus && K >= 64) {
-    T = 16;
-    if (!dense && steps >= 16 && tiles16 <= e.cus) NW = 8;
-  } else if ((tiles32 <= e.cus && K >= 256) || (tiles32 * 4 <= 7 * e.cus && K >= 1024) || (tiles32 * 2 <= 7 * e.cus && K >= 3072)) {
-    T = 32;
-    if (!dense && steps >= 32 && tiles32 <= e.cus) NW = 8;
-  }
-  if (const char *f = tuning_env("CATCHQ_SMALL")) {
-    const int v = std::atoi(f);  // 0: off; T * 100 + NW
-    T = v / 100;
-    NW = v % 100;
-  }
-  if (!T) return -1;
+  const int64_t M = (int64_t)N_img * Ho * Wo;
+  const int plan = small_plan(M, Co, (int64_t)kh * kw * Ci, dense, e.cus);
+  if (!plan) return -1;
   SmallParams p = {};
-  p.M = (int)M; p.N = Co; p.K = (int)K;
-  p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
-  p.img_stride = (unsigned)(H * W * Ci); p.row_stride = (unsigned)(W * Ci); p.pix_stride = (unsigned)Ci;
-  magic(Wo, &p.magic_wo, &p.mask_wo); magic(Ho, &p.magic_ho, &p.mask_ho);
-  magic(Ci, &p.magic_ci, &p.mask_ci); magic(kw, &p.magic_kw, &p.mask_kw);
-  p.m_fastest = b_bytes > a_bytes;
-  p.epi = pick_epilogue(Co, e);
-  p.a_bytes = (unsigned)a_bytes; p.b_bytes = (unsigned)b_bytes;
-#define CATCHQ_SMALL_CASE(T_, NW_) \
-  case T_ * 100 + NW_: return dense ? launch_small<T_, NW_, true>(x, w, p, e, s) : launch_small<T_, NW_, false>(x, w, p, e, s)
-  switch (T * 100 + NW) {
-    CATCHQ_SMALL_CASE(32, 4);
-    CATCHQ_SMALL_CASE(32, 8);
-    CATCHQ_SMALL_CASE(16, 4);
-    CATCHQ_SMALL_CASE(16, 8);
-    default: return -1;
-  }
-#undef CATCHQ_SMALL_CASE
+  if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense)) return -1;
+  small_common(&p, M, Co, Ho, Wo, e);
+  return dense ? launch_small_plan<true, SMALL_I8, false>(plan, p, e, s) : launch_small_plan<false, SMALL_I8, false>(plan, p, e, s);
+}
+
+// A residual block's last convolution with its 1x1 projection shortcut (arguments as conv2d_dual_i8).  -1: not one.
+int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                           int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws,
+                           int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s) {
+  if (e.exp2_a || e.exp2_b || e.resid || e.acc_out || !vec_epilogue_ok(Co, e) || !aligned16(sc.chan_div) ||
+      !aligned16(sc.chan_rcp) || !aligned16(sc.bias))
+    return -1;
+  const int64_t M = (int64_t)N_img * Ho * Wo;
+  const int plan = small_plan(M, Co, (int64_t)kh * kw * Ci + Cs, false, e.cus);
+  if (!plan) return -1;
+  SmallParams p = {};
+  if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false) ||
+      !small_side(&p.side[1], xs, 1, ws, N_img, Hs, Ws, Cs, Co, 1, 1, 0, 0, ss, ss, 1, 1, Ho, Wo, false))
+    return -1;
+  EpiDev probe = e;
+  probe.resid = reinterpret_cast<const float *>(e.y ? e.y : e.q);  // any 16-byte aligned non-null pointer
+  small_common(&p, M, Co, Ho, Wo, probe);
+  p.sc = sc;
+  return launch_small_plan<false, SMALL_I8, true>(plan, p, e, s);
+}
+
+// Activations still in floating point (NHWC), quantized at 2^position on their way into LDS: whether one launch serves
+// the shape, and that launch.
+bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus) {
+  return Ci % 16 == 0 && small_plan(M, Co, K, dense, cus) != 0;
+}
+int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
+                         int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
+  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+  const int64_t M = (int64_t)N_img * Ho * Wo;
+  const int plan = small_plan(M, Co, (int64_t)kh * kw * Ci, dense, e.cus);
+  if (!plan) return -1;
+  SmallParams p = {};
+  if (!small_side(&p.side[0], x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense)) return -1;
+  small_common(&p, M, Co, Ho, Wo, e);
+  p.x_neg_pos = -position;
+  if (half) return dense ? launch_small_plan<true, SMALL_F16, false>(plan, p, e, s) : launch_small_plan<false, SMALL_F16, false>(plan, p, e, s);
+  return dense ? launch_small_plan<true, SMALL_F32, false>(plan, p, e, s) : launch_small_plan<false, SMALL_F32, false>(plan, p, e, s);
 }
 
 }  // namespace catchq

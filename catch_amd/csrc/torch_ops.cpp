@@ -11,11 +11,13 @@
 // Device tensors only: there is deliberately no CPU implementation behind these ops (the
 // reference's own CPU fall-back for them returns its input, operators/op_methods.cpp:1019-1035).
 #include <ATen/ATen.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPEvent.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <torch/library.h>
 
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -58,6 +60,12 @@ int bits_of(const Tensor &t) {
     case at::kInt: return 32;
     default: TORCH_CHECK(false, "expected an int8/int16/int32 tensor, got ", t.scalar_type());
   }
+}
+
+// at::empty for the device without a trip through the dispatcher
+Tensor device_empty(at::IntArrayRef shape, at::ScalarType type, at::Device device,
+                    c10::optional<at::MemoryFormat> format = c10::nullopt) {
+  return Tensor(at::detail::empty_cuda(shape, type, device, format));
 }
 
 bool has_bias(const Tensor &b) { return b.defined() && b.numel() != 0 && b.dim() != 0; }
@@ -301,6 +309,7 @@ int64_t set_launch_sharing_op(int64_t launches) {
 Tensor as_f32_vec(const c10::optional<Tensor> &t, int64_t n, const char *name) {
   if (!t.has_value() || !t->defined()) return Tensor();
   TORCH_CHECK(t->numel() == n, name, ": expected ", n, " elements, got ", t->numel());
+  if (t->scalar_type() == at::kFloat && t->is_contiguous()) return *t;
   return t->to(at::kFloat).contiguous();
 }
 
@@ -318,6 +327,22 @@ struct RcpEntry {
 std::mutex g_rcp_mutex;
 std::unordered_map<const c10::TensorImpl *, RcpEntry> g_rcp_cache;
 
+Tensor reciprocals_of(const Tensor &div) {
+  Tensor host = div.to(at::kCPU).contiguous();
+  const float *d = host.data_ptr<float>();
+  const int64_t n = host.numel();
+  std::vector<float> r(n);
+  bool usable = n > 0;
+  for (int64_t i = 0; i < n; ++i) {
+    uint32_t bits;
+    std::memcpy(&bits, &d[i], 4);
+    if ((bits & 0x7fffffu) == 0x7fffffu || !(d[i] > 0.0f) || !std::isfinite(d[i])) usable = false;
+    r[i] = 1.0f / d[i];  // IEEE division: correctly rounded
+  }
+  if (!usable) return Tensor();
+  return at::from_blob(r.data(), {n}, at::TensorOptions().dtype(at::kFloat)).to(div.device());
+}
+
 Tensor reciprocals_for(const Tensor &div) {
   const c10::TensorImpl *key = div.unsafeGetTensorImpl();
   {
@@ -331,19 +356,7 @@ Tensor reciprocals_for(const Tensor &div) {
       g_rcp_cache.erase(it);
     }
   }
-  Tensor host = div.to(at::kCPU).contiguous();
-  const float *d = host.data_ptr<float>();
-  const int64_t n = host.numel();
-  std::vector<float> r(n);
-  bool usable = n > 0;
-  for (int64_t i = 0; i < n; ++i) {
-    uint32_t bits;
-    std::memcpy(&bits, &d[i], 4);
-    if ((bits & 0x7fffffu) == 0x7fffffu || !(d[i] > 0.0f) || !std::isfinite(d[i])) usable = false;
-    r[i] = 1.0f / d[i];  // IEEE division: correctly rounded
-  }
-  Tensor rcp;
-  if (usable) rcp = at::from_blob(r.data(), {n}, at::TensorOptions().dtype(at::kFloat)).to(div.device());
+  Tensor rcp = reciprocals_of(div);
   std::lock_guard<std::mutex> lock(g_rcp_mutex);
   if (g_rcp_cache.size() > 4096) g_rcp_cache.clear();
   g_rcp_cache.insert_or_assign(key, RcpEntry{c10::weak_intrusive_ptr<c10::TensorImpl>(div.getIntrusivePtr()),
@@ -827,7 +840,7 @@ Tensor quantize_to_nhwc(const Tensor &x, int bw, int pos, int64_t cpad, float sc
   TORCH_CHECK(x.dim() == 4, "a 4-d activation tensor is expected");
   const int64_t n = x.size(0), c = x.size(1), h = x.size(2), w = x.size(3);
   if (cpad < c) cpad = c;
-  Tensor q = at::empty({n, h, w, cpad}, x.options().dtype(int_type(bw)));
+  Tensor q = device_empty({n, h, w, cpad}, int_type(bw), x.device());
   if (cpad == c && x.is_contiguous(at::MemoryFormat::ChannelsLast)) {
     check_status(catchq_quantize(x.data_ptr(), dt, q.data_ptr(), bw, x.numel(), pos, scale, current_stream()),
                  "torch_mlu::quantize");
@@ -879,12 +892,21 @@ struct Prepared {
   bool per_channel = false;
   bool params_half = false;  // per-channel parameters derived with half tensor ops (half q_scale, int8)
   int variant = 0;   // caller's layout choice for qw (part of the cache key)
-  Tensor qw;         // conv: [Co,kh,kw,Ci/g]; linear: [N,K]
+  Tensor qw;         // conv: [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory; linear: [N,K]
   Tensor new_scale;  // device fp32 [Co] when per_channel
+  Tensor rcp;        // its correctly rounded reciprocals (undefined where the kernels have to divide)
+  // fp32 copy of the bias passed when the entry was made, if that one was not fp32 already: valid for the same tensor
+  // at the same version; another bias is converted at the call
+  c10::weak_intrusive_ptr<c10::TensorImpl> b_impl;
+  uint32_t b_ver = 0;
+  const void *b_ptr = nullptr;
+  Tensor bias32;
   // recorded on the stream that quantized the weight, behind those kernels: a later call on another stream
   // (another thread's, a side stream) waits for it before it reads qw / new_scale
   at::cuda::CUDAEvent ready;
-  Prepared() : w_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
+  std::atomic<bool> ready_seen{false};  // the event has been seen complete: no need to ask again
+  Prepared() : b_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
+               w_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
                s_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
                m_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)) {}
 };
@@ -912,6 +934,7 @@ bool still_valid(const Prepared &p, const Tensor &w, const Tensor &s, const Tens
   if (!(same(p.w_impl, w, p.w_ver) && same(p.s_impl, s, p.s_ver) && same(p.m_impl, m, p.m_ver) &&
         p.w_ptr == w.data_ptr() && p.s_ptr == s.data_ptr() && p.m_ptr == m.data_ptr()))
     return false;
+  if (!s.device().is_cpu() && !m.device().is_cpu()) return true;
   // Tensors without a version counter (inference tensors) and `.data =` swaps that keep the storage cannot be
   // told apart by identity.  q-params that live on the host are compared by content (a few bytes); for device
   // tensors the storage address above is what is checked -- reading them back would be the host synchronisation
@@ -930,7 +953,7 @@ c10::weak_intrusive_ptr<c10::TensorImpl> weak_of(const Tensor &t) {
 // Decode the two q-param encodings and quantize the weight (make_dense(weight, activation bit width)
 // returns it dense, dim 0 slowest, in the layout the caller's kernel wants).
 template <typename MakeDense>
-std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, const Tensor &q_scale,
+std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, const Tensor &bias, const Tensor &q_scale,
                                   const Tensor &q_mode) {
   auto p = std::make_shared<Prepared>();
   Tensor s_host = q_scale.to(at::kCPU).to(at::kFloat).contiguous();
@@ -988,11 +1011,16 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
   p->m_ptr = q_mode.data_ptr();
   p->s_host = q_scale.to(at::kCPU).contiguous().clone();
   p->m_host = q_mode.to(at::kCPU).contiguous().clone();
+  if (p->new_scale.defined()) p->rcp = reciprocals_of(p->new_scale);
+  if (has_bias(bias) && bias.device() == weight.device() && !(bias.scalar_type() == at::kFloat && bias.is_contiguous())) {
+    p->bias32 = bias.to(at::kFloat).contiguous();
+    p->b_impl = weak_of(bias); p->b_ver = version_of(bias); p->b_ptr = bias.data_ptr();
+  }
   return p;
 }
 
 template <typename MakeDense>
-std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_scale, const Tensor &q_mode,
+std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &bias, const Tensor &q_scale, const Tensor &q_mode,
                                        MakeDense make_dense, int variant = 0) {
   const bool use_cache = cache_enabled();
   const c10::TensorImpl *key = weight.unsafeGetTensorImpl();
@@ -1002,20 +1030,23 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_sca
     if (it != g_cache.end()) {
       if (it->second->variant == variant && still_valid(*it->second, weight, q_scale, q_mode)) {
         const auto cur = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
-        if (!it->second->ready.query())  // still in flight on the stream that prepared it
-          it->second->ready.block(cur);
+        if (!it->second->ready_seen.load(std::memory_order_acquire)) {
+          if (it->second->ready.query()) it->second->ready_seen.store(true, std::memory_order_release);
+          else it->second->ready.block(cur);  // still in flight on the stream that prepared it
+        }
         if (cur.id() != it->second->made_on) {
           // read on another stream than the one the caching allocator knows these blocks by: tell it, so that
           // an entry dropped while this stream's kernels still read it is not handed out again too early
           it->second->qw.record_stream(cur);
-          if (it->second->new_scale.defined()) it->second->new_scale.record_stream(cur);
+          for (const Tensor *t : {&it->second->new_scale, &it->second->rcp, &it->second->bias32})
+            if (t->defined()) t->record_stream(cur);
         }
         return it->second;
       }
       g_cache.erase(it);
     }
   }
-  auto p = prepare(make_dense, weight, q_scale, q_mode);
+  auto p = prepare(make_dense, weight, bias, q_scale, q_mode);
   p->variant = variant;
   const auto made_on = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
   p->made_on = made_on.id();
@@ -1045,19 +1076,74 @@ void clear_cache_op() {
   g_rcp_cache.clear();
 }
 
-// quantized activations [N,H,W,Ci] x prepared weight -> floating [N,Ho,Wo,Co]
-Tensor conv_prepared(const Tensor &qx, const Prepared &prep, const Tensor &bias, at::IntArrayRef padding,
-                     at::IntArrayRef stride, at::IntArrayRef dilation, int64_t groups, bool half) {
-  Tensor qw = prep.qw.permute({0, 2, 3, 1});  // view of the same memory as [Co,kh,kw,Ci/g], contiguous
-  EpiArgs a;
-  a.exp2 = prep.pos_x + prep.pos_w;
-  if (prep.per_channel) a.chan_div = prep.new_scale;
-  if (has_bias(bias)) a.bias = bias;
-  a.y_half = half;
+// The epilogue of the reference ops: dequantization with the entry's constants, bias, floating output into `y`.
+// `keep` holds a bias converted for this call.
+catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64_t co, const Tensor &y, Tensor *keep) {
+  catchq_epilogue_t e;
+  std::memset(&e, 0, sizeof(e));
+  e.exp2 = p.pos_x + p.pos_w;
+  TORCH_CHECK(e.exp2 >= -126 && e.exp2 <= 126, "position sum out of range");
+  if (p.per_channel) {
+    e.chan_div = p.new_scale.data_ptr<float>();
+    if (p.rcp.defined()) e.chan_rcp = p.rcp.data_ptr<float>();
+  }
+  if (has_bias(bias)) {
+    TORCH_CHECK(bias.numel() == co, "bias: expected ", co, " elements, got ", bias.numel());
+    if (bias.scalar_type() == at::kFloat && bias.is_contiguous()) {
+      e.bias = bias.data_ptr<float>();
+    } else if (p.bias32.defined() && p.b_impl._unsafe_get_target() == bias.unsafeGetTensorImpl() && !p.b_impl.expired() &&
+               p.b_ver == version_of(bias) && p.b_ptr == bias.data_ptr()) {
+      e.bias = p.bias32.data_ptr<float>();
+    } else {
+      *keep = bias.to(at::kFloat).contiguous();
+      e.bias = keep->data_ptr<float>();
+    }
+  }
+  const bool half = y.scalar_type() == at::kHalf;
+  e.y = y.data_ptr();
+  e.y_dtype = half ? CATCHQ_F16 : CATCHQ_F32;
   // per-channel branch on half tensors: the vendor convolution's half output, then `/ new_scale` and `+ bias` as
   // half tensor ops (quantify_conv_forward.cpp:123-129); where the q-params stayed fp32 (int16), so does this
-  a.half_steps = half && prep.per_channel && prep.params_half;
-  return qconv2d_impl(qx, qw, padding, stride, dilation, groups, a).y;
+  e.half_steps = half && p.per_channel && p.params_half;
+  e.sharing = t_launch_sharing;
+  return e;
+}
+
+// quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x) x prepared weight -> floating
+// output, logical [N,Co,Ho,Wo] over NHWC memory
+Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, const Prepared &prep, const Tensor &bias,
+                     at::IntArrayRef padding, at::IntArrayRef stride, at::IntArrayRef dilation, int64_t groups, bool half) {
+  TORCH_CHECK(padding.size() == 2 && stride.size() == 2 && dilation.size() == 2, "2-d conv parameters expected");
+  const Tensor &qw = prep.qw;  // [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory
+  TORCH_CHECK(groups > 0 && x_nhwc[3] == qw.size(1) * groups, "channel mismatch: input ", x_nhwc[3], ", weight ", qw.size(1),
+              " x groups ", groups);
+  catchq_conv_desc_t d = {(int)x_nhwc[0], (int)x_nhwc[1], (int)x_nhwc[2], (int)x_nhwc[3], (int)qw.size(0), (int)qw.size(2),
+                          (int)qw.size(3), (int)padding[0], (int)padding[1], (int)stride[0], (int)stride[1],
+                          (int)dilation[0], (int)dilation[1], (int)groups};
+  TORCH_CHECK(d.stride_h > 0 && d.stride_w > 0, "non-positive stride is not supported");
+  TORCH_CHECK(d.pad_h >= 0 && d.pad_w >= 0, "negative padding is not supported");
+  const int ho = catchq_conv_out_size(d.h, d.kh, d.pad_h, d.stride_h, d.dil_h);
+  const int wo = catchq_conv_out_size(d.w, d.kw, d.pad_w, d.stride_w, d.dil_w);
+  TORCH_CHECK(ho > 0 && wo > 0, "Calculated output size is too small");
+  Tensor y = device_empty({d.n, d.co, ho, wo}, half ? at::kHalf : at::kFloat, qw.device(), at::MemoryFormat::ChannelsLast);
+  if (d.n == 0 || d.co == 0) return y;  // nothing to compute: the empty output is the result
+  Tensor keep;
+  const catchq_epilogue_t e = prepared_epilogue(prep, bias, d.co, y, &keep);
+  if (qx.defined()) {
+    check_status(catchq_conv2d_nhwc(qx.data_ptr(), bits_of(qx), qw.data_ptr(), bits_of(qw), &d, &e, current_stream()),
+                 "torch_mlu::conv2d");
+    return y;
+  }
+  const int dt = half ? CATCHQ_F16 : CATCHQ_F32;
+  size_t ws_bytes = 0;
+  check_status(catchq_float_conv2d_workspace_size(dt, &d, &e, &ws_bytes), "torch_mlu::conv2d");
+  if (reinterpret_cast<uintptr_t>(x) & 15u) ws_bytes = (size_t)d.n * d.h * d.w * d.ci;  // one launch takes aligned tensors only
+  Tensor ws;
+  if (ws_bytes) ws = device_empty({(int64_t)ws_bytes}, at::kChar, qw.device());
+  check_status(catchq_float_conv2d_nhwc(x, dt, prep.pos_x, qw.data_ptr(), &d, &e, ws_bytes ? ws.data_ptr() : nullptr, ws_bytes,
+                                        current_stream()),
+               "torch_mlu::conv2d");
+  return y;
 }
 
 Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, at::IntArrayRef padding,
@@ -1082,7 +1168,7 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   };
   const int64_t kw_extra = (kw + 3) / 4 * 4 - kw;
   const bool can_frame = few && dilation.size() == 2 && dilation[1] == 1 && padding.size() == 2;
-  auto prep = prepared_for(weight, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
+  auto prep = prepared_for(weight, bias, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
     Tensor wd = w;
     const int64_t cpad = device_channels(bw_act) - ci;
     const int64_t taps = (few && bw_act == 8 && can_frame) ? kw_extra : 0;
@@ -1091,22 +1177,24 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
     return wd.contiguous(at::MemoryFormat::ChannelsLast);
   }, (few ? 1 : 0) | (can_frame ? 2 : 0));
   Tensor qx;
-  std::vector<int64_t> pad(padding.begin(), padding.end());
+  if (prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0 && input.is_contiguous(at::MemoryFormat::ChannelsLast))
+    return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), input.size(2), input.size(3), ci}, *prep, bias, padding, stride,
+                         dilation, groups, half);
   if (few && prep->bw_x == 8 && can_frame) {
     const Tensor xc = input.contiguous();
     const int64_t h = input.size(2), w_in = input.size(3);
-    qx = at::empty({input.size(0), h + 2 * pad[0], w_in + 2 * pad[1] + kw_extra, 4}, input.options().dtype(at::kChar));
+    qx = device_empty({input.size(0), h + 2 * padding[0], w_in + 2 * padding[1] + kw_extra, 4}, at::kChar, input.device());
     check_status(catchq_quantize_nchw_to_nhwc_frame(xc.data_ptr(), half ? CATCHQ_F16 : CATCHQ_F32, qx.data_ptr(), 8,
                                                     (int)input.size(0), (int)ci, (int)h, (int)w_in, 4, (int)qx.size(1),
-                                                    (int)qx.size(2), (int)pad[0], (int)pad[1], prep->pos_x, 1.0f,
+                                                    (int)qx.size(2), (int)padding[0], (int)padding[1], prep->pos_x, 1.0f,
                                                     current_stream()),
                  "torch_mlu::quantize");
-    pad = {0, 0};
+    return conv_prepared(qx, nullptr, qx.sizes(), *prep, bias, {0, 0}, stride, dilation, groups, half);
   } else {
     qx = quantize_to_nhwc(input, prep->bw_x, prep->pos_x, device_channels(prep->bw_x));
   }
-  Tensor y = conv_prepared(qx, *prep, bias, pad, stride, dilation, groups, half);
-  return y.permute({0, 3, 1, 2});  // logical NCHW over channels-last memory, like the reference
+  // logical NCHW over channels-last memory, like the reference
+  return conv_prepared(qx, nullptr, qx.sizes(), *prep, bias, padding, stride, dilation, groups, half);
 }
 
 // [N,C,L] x [Co,Ci/g,k]: a convolution over images of one row (the reference's module calls
@@ -1118,12 +1206,12 @@ Tensor conv1d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   TORCH_CHECK(padding.size() == 1 && stride.size() == 1 && dilation.size() == 1, "1-d conv parameters expected");
   const bool half = fp_dtype(input, "quantify only support input float/half") == CATCHQ_F16;
   c10::DeviceGuard guard(input.device());
-  auto prep = prepared_for(weight, q_scale, q_mode, [](const Tensor &w, int) {
+  auto prep = prepared_for(weight, bias, q_scale, q_mode, [](const Tensor &w, int) {
     return w.unsqueeze(2).contiguous(at::MemoryFormat::ChannelsLast);  // memory [Co][1][k][Ci/g]
   });
   Tensor qx = quantize_to_nhwc(input.unsqueeze(2), prep->bw_x, prep->pos_x, input.size(1));
-  Tensor y = conv_prepared(qx, *prep, bias, {0, padding[0]}, {1, stride[0]}, {1, dilation[0]}, groups, half);
-  return y.squeeze(1).permute({0, 2, 1});  // [N,Lo,Co] memory seen as [N,Co,Lo]
+  Tensor y = conv_prepared(qx, nullptr, qx.sizes(), *prep, bias, {0, padding[0]}, {1, stride[0]}, {1, dilation[0]}, groups, half);
+  return y.squeeze(2);  // [N,Lo,Co] memory seen as [N,Co,Lo]
 }
 
 // [N,C,D,H,W] x [Co,Ci/g,kd,kh,kw].  The depth taps are folded into the channel dimension of a 2-d
@@ -1146,7 +1234,7 @@ Tensor conv3d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
               weight.size(1), " x groups ", groups);
   const int64_t d_out = (dd_in + 2 * pd - dd * (kd - 1) - 1) / sd + 1;
   TORCH_CHECK(dd_in + 2 * pd >= dd * (kd - 1) + 1 && d_out > 0, "Calculated output size is too small");
-  auto prep = prepared_for(weight, q_scale, q_mode, [](const Tensor &wt, int) {
+  auto prep = prepared_for(weight, bias, q_scale, q_mode, [](const Tensor &wt, int) {
     // [Co, (Ci/g)*kd, kh, kw] with the depth tap fastest inside a channel, stored [Co][kh][kw][(Ci/g)*kd]
     return wt.reshape({wt.size(0), wt.size(1) * wt.size(2), wt.size(3), wt.size(4)})
         .contiguous(at::MemoryFormat::ChannelsLast);
@@ -1164,8 +1252,8 @@ Tensor conv3d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
       taps.push_back(q.slice(1, t * dd, t * dd + (d_out - 1) * sd + 1, sd));  // [N,Do,H,W,C]
     qx = at::stack(taps, 5).view({n * d_out, h, w, c * kd});
   }
-  Tensor y = conv_prepared(qx, *prep, bias, {padding[1], padding[2]}, {stride[1], stride[2]},
-                           {dilation[1], dilation[2]}, groups, half);
+  Tensor y = conv_prepared(qx, nullptr, qx.sizes(), *prep, bias, {padding[1], padding[2]}, {stride[1], stride[2]},
+                           {dilation[1], dilation[2]}, groups, half).permute({0, 2, 3, 1});  // [N*Do,Ho,Wo,Co]
   return y.view({n, d_out, y.size(1), y.size(2), y.size(3)}).permute({0, 4, 1, 2, 3});  // logical NCDHW
 }
 
@@ -1221,27 +1309,44 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   // K is padded with zeros on both operands to what the matrix-core routes take (16 int8 / 8 int16 values)
   const int64_t k = weight.size(1);
   auto device_k = [&](int bw_act) { return bw_act == 8 ? (k + 15) / 16 * 16 : (k + 7) / 8 * 8; };
-  auto prep = prepared_for(weight, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
+  auto prep = prepared_for(weight, bias, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
     const int64_t kpad = device_k(bw_act) - k;
     return kpad > 0 ? at::constant_pad_nd(w, {0, kpad}, 0).contiguous() : w.contiguous();
   });
-  Tensor x2 = input.contiguous().view({-1, k});
-  Tensor qx;
-  if (device_k(prep->bw_x) != k && x2.size(0) > 0)  // rows as pixels of a [M, K, 1, 1] image, zero channels appended
-    qx = quantize_to_nhwc(x2.view({x2.size(0), k, 1, 1}), prep->bw_x, prep->pos_x, device_k(prep->bw_x))
-             .view({x2.size(0), device_k(prep->bw_x)});
-  else if (device_k(prep->bw_x) != k)
-    qx = at::empty({0, device_k(prep->bw_x)}, x2.options().dtype(int_type(prep->bw_x)));
+  const Tensor xc = input.contiguous();
+  const int64_t n = weight.size(0), kd = device_k(prep->bw_x);
+  int64_t m = 1;
+  for (int64_t i = 0; i + 1 < input.dim(); ++i) m *= input.size(i);
+  c10::SmallVector<int64_t, 5> shape(input.sizes().begin(), input.sizes().end() - 1);
+  shape.push_back(n);
+  // output is fp32 whatever the input type (operators/cnnl/matmul.cpp:72-74)
+  Tensor y = device_empty(shape, at::kFloat, input.device());
+  if (m == 0 || n == 0) return y;  // nothing to compute
+  Tensor keep;
+  const catchq_epilogue_t e = prepared_epilogue(*prep, bias, n, y, &keep);
+  const int dt = input.scalar_type() == at::kHalf ? CATCHQ_F16 : CATCHQ_F32;
+  if (prep->bw_x == 8 && prep->bw_w == 8 && kd == k && m < (1ll << 31)) {
+    // rows as images of one pixel: small products quantize and multiply in one launch
+    const catchq_conv_desc_t d = {(int)m, 1, 1, (int)k, (int)n, 1, 1, 0, 0, 1, 1, 1, 1, 1};
+    size_t ws_bytes = 0;
+    check_status(catchq_float_conv2d_workspace_size(dt, &d, &e, &ws_bytes), "torch_mlu::linear");
+    if (ws_bytes == 0 && (reinterpret_cast<uintptr_t>(xc.data_ptr()) & 15u) == 0) {
+      check_status(catchq_float_conv2d_nhwc(xc.data_ptr(), dt, prep->pos_x, prep->qw.data_ptr(), &d, &e, nullptr, 0, current_stream()),
+                   "torch_mlu::linear");
+      return y;
+    }
+  }
+  Tensor qx = device_empty({m, kd}, int_type(prep->bw_x), input.device());
+  if (kd != k)  // rows as pixels of a [M, K, 1, 1] image, zero channels appended
+    check_status(catchq_quantize_nchw_to_nhwc(xc.data_ptr(), dt, qx.data_ptr(), prep->bw_x, (int)m, (int)k, 1, 1, (int)kd,
+                                              prep->pos_x, 1.0f, current_stream()),
+                 "torch_mlu::quantize");
   else
-    qx = quantize_op(x2, prep->bw_x, prep->pos_x, 1.0);
-  EpiArgs a;  // output is fp32 whatever the input type (operators/cnnl/matmul.cpp:72-74)
-  a.exp2 = prep->pos_x + prep->pos_w;
-  if (prep->per_channel) a.chan_div = prep->new_scale;
-  if (has_bias(bias)) a.bias = bias;
-  EpiOut o = qlinear_impl(qx, prep->qw, a);
-  std::vector<int64_t> shape(input.sizes().begin(), input.sizes().end() - 1);
-  shape.push_back(weight.size(0));
-  return o.y.view(shape);
+    check_status(catchq_quantize(xc.data_ptr(), dt, qx.data_ptr(), prep->bw_x, m * k, prep->pos_x, 1.0f, current_stream()),
+                 "torch_mlu::quantize");
+  check_status(catchq_gemm_nt(qx.data_ptr(), prep->bw_x, prep->qw.data_ptr(), prep->bw_w, m, n, kd, &e, current_stream()),
+               "torch_mlu::linear");
+  return y;
 }
 
 // x [N,H,W,C] contiguous int8 / int16 / fp32

@@ -237,6 +237,18 @@ int catchq_quantize_conv2d_nhwc(const void *x, int x_dtype, const int32_t *x_pos
                                 const catchq_conv_desc_t *desc, const float *bias, void *y, int y_dtype,
                                 void *workspace, size_t workspace_bytes, catchq_stream_t stream);
 
+/* Convolution of a floating activation tensor with filters that are already int8:
+ *   cnnl_quantify_offline_internal (quantify.cpp:69-101) followed by cnnl_quantify_convolution_internal
+ * x [n,h,w,ci] NHWC fp32/fp16, q = sat(rne(x * 2^-x_position)) at 8 bits, then as catchq_conv2d_nhwc (a linear is the
+ * convolution of n rows of 1 x 1 pixels).  Small contractions quantize on the way into the matrix cores and run as one
+ * launch; everything else goes through the workspace (the quantized activations) as two.  *_workspace_size returns 0
+ * where one launch serves the shape (for 16-byte aligned tensors). */
+int catchq_float_conv2d_workspace_size(int x_dtype, const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue,
+                                       size_t *bytes);
+int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_position, const void *w, const catchq_conv_desc_t *desc,
+                             const catchq_epilogue_t *epilogue, void *workspace, size_t workspace_bytes,
+                             catchq_stream_t stream);
+
 /* Last convolution of a residual block with the block's projection shortcut evaluated in the same launch.
  * In the reference a block with a projection ends in two torch_mlu::conv2d calls (cnnl_conv2d,
  * operators/cnnl/quantify_conv_forward.cpp:56-147: the 1x1 shortcut and the block's last convolution) and a

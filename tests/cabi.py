@@ -132,6 +132,20 @@ def conv2d_nhwc(x, w, padding=(0, 0), stride=(1, 1), dilation=(1, 1), groups=1, 
     return out
 
 
+def float_conv2d_nhwc(x, x_pos, w, padding=(0, 0), stride=(1, 1), dilation=(1, 1), exp2=0, chan_div=None, bias=None, act=0,
+                      y_dtype=torch.float32, q_bw=0, q_pos=0, chan_rcp=None):
+    """-> (outputs, workspace bytes the library asked for)"""
+    d = conv_desc(x.shape, w.shape, padding, stride, dilation, 1)
+    ho = lib().catchq_conv_out_size(d.h, d.kh, d.pad_h, d.stride_h, d.dil_h)
+    wo = lib().catchq_conv_out_size(d.w, d.kw, d.pad_w, d.stride_w, d.dil_w)
+    e, out = _epilogue((d.n, ho, wo, d.co), x.device, exp2, chan_div, bias, None, act, y_dtype, False, q_bw, q_pos, 1.0, chan_rcp)
+    sz = ctypes.c_size_t()
+    check(lib().catchq_float_conv2d_workspace_size(dt(x), ctypes.byref(d), ctypes.byref(e), ctypes.byref(sz)))
+    ws = torch.empty(max(sz.value, 16), dtype=torch.int8, device=x.device)
+    check(lib().catchq_float_conv2d_nhwc(ptr(x), dt(x), x_pos, ptr(w), ctypes.byref(d), ctypes.byref(e), ptr(ws), sz.value, stream()))
+    return out, sz.value
+
+
 def conv2d_shortcut_nhwc(x, w, sx, sw, sc_stride, sc_exp2, sc_chan_div=None, sc_bias=None, sc_chan_rcp=None, padding=(0, 0),
                          stride=(1, 1), dilation=(1, 1), exp2=0, chan_div=None, bias=None, act=0, y_dtype=torch.float32,
                          q_bw=0, q_pos=0, q_scale=1.0, chan_rcp=None, act_slope=0.0, resid_after_act=False):

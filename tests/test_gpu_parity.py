@@ -295,6 +295,30 @@ def test_few_output_tiles(case):
             assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("case", [FEW_TILES_CASES[i] for i in (0, 2, 3, 5, 6, 7, 9, 10, 11, 13, 15)] + [(70, 30, 30, 32, 40, 3, 1, 1, 1)])
+def test_floating_activations_quantized_on_the_way(case, dtype):
+    """one launch where the contraction is small, two through the workspace otherwise (last case); ties, NaN, values beyond
+    the range and infinities among the activations"""
+    n, h, w, ci, co, k, pad, stride, dil = case
+    note("floating activations", case, dtype)
+    r = rng(sum(case) * 13)
+    x = (r.standard_normal((n, h, w, ci)) * 2).astype(dtype)
+    flat = x.reshape(-1)
+    flat[:16] = [0.5, 1.5, -0.5, -1.5, 2.5, np.inf, -np.inf, np.nan, 1e4, -1e4, 0.03125, -0.03125, 0.046875, 0.0, -0.0, 4.0]
+    wt = _ints(r, (co, k, k, ci), 8)
+    div = r.uniform(0.6, 3.5, co).astype(np.float32)
+    bias = r.standard_normal(co).astype(np.float32)
+    acc, ovf = orc.conv2d_nhwc(orc.quantize(x, 8, -5), wt, (pad, pad), (stride, stride), (dil, dil), 1)
+    assert ovf == 0
+    out, ws = cabi.float_conv2d_nhwc(cabi.dev(x), -5, cabi.dev(wt), (pad, pad), (stride, stride), (dil, dil), exp2=-10,
+                                     chan_div=cabi.dev(div), chan_rcp=cabi.dev(np.float32(1) / div), bias=cabi.dev(bias), act=1,
+                                     y_dtype=torch.float32, q_bw=8, q_pos=-3)
+    assert (ws == 0) == (n != 70)
+    y = orc.epilogue(acc, -10, div, bias, None, 1)
+    assert same_bits(y, out["y"].cpu().numpy()) and same_bits(orc.quantize(y, 8, -3), out["q"].cpu().numpy())
+
+
 def test_division_by_reciprocal_is_exact():
     """v/d evaluated as q=v*r, e=fma(-q,d,v), fma(e,r,q) with r = RN(1/d) must equal IEEE division bit
     for bit: adversarial divisor significands x a wide set of dividends x several exponents."""
