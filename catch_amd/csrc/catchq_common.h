@@ -136,7 +136,8 @@ struct EpiDev {
   // the non-temporal hint so that it does not push the operands and the int8 output out of the caches
   int y_stream, resid_stream;
   int cus;  // compute units the launch plans its tiles for (planned_cus of the caller's hint)
-  int half_steps;  // fp16 output: round to binary16 after the scaling, the division and the bias (generic epilogues only)
+  int half_steps;  // fp16 output: round to binary16 after the scaling, the division and the bias
+  const float *half_rcp;  // half_steps: the divisors' reciprocals where the division may go through them
 };
 
 // The second operand pair of a two-branch launch: the projection shortcut of a residual block.  Its
@@ -179,6 +180,7 @@ inline EpiDev make_epi(const catchq_epilogue_t *e, int64_t out_elems = 0) {
   d.half_steps = (e->half_steps && e->y && e->y_dtype == CATCHQ_F16) ? 1 : 0;
   // (the reciprocal form folds the power of two into the division: not with a rounding between the two)
   d.chan_rcp = (e->chan_div && e->chan_rcp && !dev_exp && !d.half_steps && e->exp2 >= -64 && e->exp2 <= 64) ? e->chan_rcp : nullptr;
+  d.half_rcp = (d.half_steps && e->chan_div && !dev_exp) ? e->chan_rcp : nullptr;
   d.bias = e->bias;
   d.resid = e->resid;
   d.act = e->act;

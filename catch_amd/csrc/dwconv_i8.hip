@@ -232,6 +232,8 @@ static int dw3x3(const void *x, const void *w, int N, int H, int W, int C, int k
   switch (epi) {
     case EPI_Q8_RELU6: s2 ? dw3x3_launch<2, EPI_Q8_RELU6>(x, w, p, grid, e, s) : dw3x3_launch<1, EPI_Q8_RELU6>(x, w, p, grid, e, s); break;
     case EPI_Q8_RELU: s2 ? dw3x3_launch<2, EPI_Q8_RELU>(x, w, p, grid, e, s) : dw3x3_launch<1, EPI_Q8_RELU>(x, w, p, grid, e, s); break;
+    case EPI_Y32: s2 ? dw3x3_launch<2, EPI_Y32>(x, w, p, grid, e, s) : dw3x3_launch<1, EPI_Y32>(x, w, p, grid, e, s); break;
+    case EPI_Y16_STEPS: s2 ? dw3x3_launch<2, EPI_Y16_STEPS>(x, w, p, grid, e, s) : dw3x3_launch<1, EPI_Y16_STEPS>(x, w, p, grid, e, s); break;
     default: s2 ? dw3x3_launch<2, EPI_VECTOR>(x, w, p, grid, e, s) : dw3x3_launch<1, EPI_VECTOR>(x, w, p, grid, e, s); break;
   }
   return 0;

@@ -59,11 +59,13 @@ inline bool vec_epilogue_ok(int N, const EpiDev &e) {
 // What an epilogue instance knows at compile time.  A field of -1 is decided at run time from the
 // EpiDev (the generic instance); fixed fields let the compiler drop every untaken branch, which
 // matters because the epilogue is VALU-bound (about a dozen fp32 operations per output element).
-//   DIV  0 none, 1 reciprocal form, 2 true division      BIAS 0/1     RESID 0 none, 1 before, 2 after the activation
+//   DIV  0 none, 1 reciprocal form (the constants of a launch without divisors or bias are 1 and 0: nothing changes), 2 true
+//   division, 3 reciprocal form with every step rounded to binary16 (half_steps)      BIAS 0/1     RESID 0 none, 1 before, 2 after the activation
 //   ACT  CATCHQ_ACT_*       YM  0 none, 1 fp32, 2 fp16     QM  0 none, 8, 16     ACC 0/1
 template <int DIV, int BIAS, int RESID, int ACT, int YM, int QM, int ACC>
 struct EpiSpec {
   static constexpr bool kGeneric = DIV < 0;
+  static constexpr bool kSteps = DIV == 3;
   static constexpr int kAct = ACT;
   static constexpr int kQ = QM;
   // ReLU / ReLU6 feeding nothing but an int8 requantization: the activation folds into the clamp of the
@@ -112,7 +114,9 @@ enum {
   EPI_LK_Y_Q16 = 14,       // -> fp32 and int16
   EPI_LK_RESA_Q16 = 15,    // residual added after the activation -> int16
   EPI_LK_RESA_Y_Q16 = 16,  // residual added after the activation -> fp32 and int16
-  EPI_COUNT = 17
+  EPI_Y16 = 17,        // reciprocal-form dequant + bias -> fp16
+  EPI_Y16_STEPS = 18,  // ... with every step rounded to binary16, as half tensor ops would leave it
+  EPI_COUNT = 19
 };
 template <int EPI> struct EpiOf { typedef EpiGeneric type; };
 template <> struct EpiOf<EPI_Q8_RELU> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_RELU, 0, 8, 0> type; };
@@ -120,6 +124,8 @@ template <> struct EpiOf<EPI_RES_Y_Q8> { typedef EpiSpec<1, 1, 1, CATCHQ_ACT_REL
 template <> struct EpiOf<EPI_Y32> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_NONE, 1, 0, 0> type; };
 template <> struct EpiOf<EPI_RES_Y> { typedef EpiSpec<1, 1, 1, CATCHQ_ACT_RELU, 1, 0, 0> type; };
 template <> struct EpiOf<EPI_Y16_RELU> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_RELU, 2, 0, 0> type; };
+template <> struct EpiOf<EPI_Y16> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_NONE, 2, 0, 0> type; };
+template <> struct EpiOf<EPI_Y16_STEPS> { typedef EpiSpec<3, 1, 0, CATCHQ_ACT_NONE, 2, 0, 0> type; };
 template <> struct EpiOf<EPI_Q8_RELU6> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_RELU6, 0, 8, 0> type; };
 template <> struct EpiOf<EPI_RES_Q8> { typedef EpiSpec<1, 1, 1, CATCHQ_ACT_RELU, 0, 8, 0> type; };
 template <> struct EpiOf<EPI_LIN_Q8> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_NONE, 0, 8, 0> type; };
@@ -136,10 +142,13 @@ template <> struct EpiOf<EPI_LK_RESA_Y_Q16> { typedef EpiSpec<0, 1, 2, CATCHQ_AC
 // that has no instance of the variant returned uses the generic EPI_VECTOR
 inline int pick_epilogue(int N, const EpiDev &e) {
   if (!vec_epilogue_ok(N, e)) return EPI_SCALAR;
-  if (e.acc_out || (e.q && e.q_scale != 1.0f) || (e.chan_div && !e.chan_rcp) || e.half_steps) return EPI_VECTOR;
+  if (e.acc_out || (e.q && e.q_scale != 1.0f) || (e.chan_div && !e.chan_rcp && !e.half_rcp)) return EPI_VECTOR;
   // (the instances that fold the requantization's power of two into the per-channel constants keep those in range)
   if (e.q && (e.q_neg_pos < -40 || e.q_neg_pos > 40)) return EPI_VECTOR;
-  const int div = e.chan_rcp ? 1 : 0, bias = e.bias ? 1 : 0;
+  const int div = e.half_steps ? (e.half_rcp ? 3 : 2) : (e.chan_rcp ? 1 : 0), bias = e.bias ? 1 : 0;
+  // without divisors the reciprocal form runs on ones (x * 2^e exactly, the correction is zero), without a bias on zeros
+  // (x + 0 = x: an integer sum is never -0); the power of two has to stay in the range that form is stated for
+  const bool ones = div == 0 && !e.exp2_a && !e.exp2_b && e.exp2 >= -64 && e.exp2 <= 64;
   const int res = !e.resid ? 0 : (e.resid_after ? 2 : 1);
   const int ym = !e.y ? 0 : (e.y_f16 ? 2 : 1);
   const int qm = !e.q ? 0 : e.q_bw;
@@ -151,9 +160,10 @@ inline int pick_epilogue(int N, const EpiDev &e) {
       {EPI_LIN_Y_Q8, 1, 1, 0, CATCHQ_ACT_NONE, 1, 8},       {EPI_LIN_RES_Q8, 1, 1, 1, CATCHQ_ACT_NONE, 0, 8},
       {EPI_LIN_RES_Y_Q8, 1, 1, 1, CATCHQ_ACT_NONE, 1, 8},   {EPI_LK_Q16, 0, 1, 0, CATCHQ_ACT_LEAKY, 0, 16},
       {EPI_LK_Y_Q16, 0, 1, 0, CATCHQ_ACT_LEAKY, 1, 16},     {EPI_LK_RESA_Q16, 0, 1, 2, CATCHQ_ACT_LEAKY, 0, 16},
-      {EPI_LK_RESA_Y_Q16, 0, 1, 2, CATCHQ_ACT_LEAKY, 1, 16}};
+      {EPI_LK_RESA_Y_Q16, 0, 1, 2, CATCHQ_ACT_LEAKY, 1, 16}, {EPI_Y16, 1, 1, 0, CATCHQ_ACT_NONE, 2, 0},
+      {EPI_Y16_STEPS, 3, 1, 0, CATCHQ_ACT_NONE, 2, 0}};
   for (const auto &r : rows)
-    if (r.div == div && r.bias == bias && r.res == res && r.act == e.act && r.ym == ym && r.qm == qm) return r.epi;
+    if ((r.div == div || (r.div == 1 && ones)) && (r.bias == bias || bias == 0) && r.res == res && r.act == e.act && r.ym == ym && r.qm == qm) return r.epi;
   return EPI_VECTOR;
 }
 
@@ -161,6 +171,7 @@ inline int pick_epilogue(int N, const EpiDev &e) {
 struct EpiLane {
   v4f div, rcp, bias;
   bool use_rcp, use_div, use_bias, use_res, res_after, unit_q, half_steps;
+  bool steps_rcp = false;  // half_steps with the division in reciprocal form
   int act;
 };
 
@@ -172,7 +183,8 @@ __device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, c
   L.res_after = S::resid_after(e);
   L.act = S::act(e);
   L.unit_q = S::kGeneric ? (e.q_scale == 1.0f) : true;
-  L.half_steps = S::kGeneric ? (e.half_steps != 0) : false;
+  L.half_steps = S::kGeneric ? (e.half_steps != 0) : S::kSteps;
+  L.steps_rcp = S::kSteps;
   // Reciprocal form with the power of two folded in:
   //   v = (f*2^e)/d  ==  q = f*(r*2^e); err = fma(-q, d*2^-e, f); fma(err, r*2^e, q)
   // (scaling by 2^e is exact, so every intermediate is the scaled image of the unfolded one)
@@ -194,15 +206,26 @@ __device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, c
 template <class S>
 __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev &e) {
   v4f div = {1.f, 1.f, 1.f, 1.f}, rcp = {1.f, 1.f, 1.f, 1.f}, bias = {0.f, 0.f, 0.f, 0.f};
-  if (n_ok && (S::rcp(e) || S::truediv(e))) div = *reinterpret_cast<const v4f *>(e.chan_div + n);
-  if (n_ok && S::rcp(e)) rcp = *reinterpret_cast<const v4f *>(e.chan_rcp + n);
-  if (n_ok && S::bias(e)) bias = *reinterpret_cast<const v4f *>(e.bias + n);
+  const float *rcps = S::kSteps ? e.half_rcp : e.chan_rcp;
+  if (n_ok && (S::rcp(e) || S::truediv(e) || S::kSteps) && e.chan_div) div = *reinterpret_cast<const v4f *>(e.chan_div + n);
+  if (n_ok && (S::rcp(e) || S::kSteps) && rcps) rcp = *reinterpret_cast<const v4f *>(rcps + n);
+  if (n_ok && S::bias(e) && e.bias) bias = *reinterpret_cast<const v4f *>(e.bias + n);
   return epi_lane_finish<S>(div, rcp, bias, e);
 }
 
 // dequantization and bias of one integer sum: channel t of the lane's four
 __device__ __forceinline__ float epi_dequant1(int a, int t, const EpiLane &L, int exp2) {
   float x = (float)a;
+  if (L.steps_rcp) {
+    // fp32 operations on binary16 values rounded to binary16 are the binary16 operations.  The reciprocal form gives the
+    // correctly rounded fp32 quotient of the finite values; an infinite one (the scaled sum overflowed) stays infinite.
+    x = round_f16(__builtin_ldexpf(x, exp2));
+    const float q = x * L.rcp[t];
+    float v = __builtin_fmaf(__builtin_fmaf(-q, L.div[t], x), L.rcp[t], q);
+    v = __builtin_isinf(q) ? q : v;
+    asm volatile("" : "+v"(v));  // keeps the conversion below apart: fused into one operation it would round once
+    return round_f16(v) + L.bias[t];  // (rounded to binary16 by the conversion of the output)
+  }
   if (L.use_rcp) x = div_by_rcp(x, L.div[t], L.rcp[t]);
   else {
     x = __builtin_ldexpf(x, exp2);

@@ -131,6 +131,8 @@ static int pw_pick_epi(const void *a, const void *b, const IgemmParams &p, const
     case EPI_Q8_RELU: return pw_launch<KS, NF, EPI_Q8_RELU>(a, b, p, e, s);
     case EPI_LIN_Q8: return pw_launch<KS, NF, EPI_LIN_Q8>(a, b, p, e, s);
     case EPI_LIN_Y_Q8: return pw_launch<KS, NF, EPI_LIN_Y_Q8>(a, b, p, e, s);
+    case EPI_Y32: return pw_launch<KS, NF, EPI_Y32>(a, b, p, e, s);
+    case EPI_Y16_STEPS: return pw_launch<KS, NF, EPI_Y16_STEPS>(a, b, p, e, s);
     default: return pw_launch<KS, NF, EPI_VECTOR>(a, b, p, e, s);
   }
 }
@@ -261,6 +263,8 @@ static int stem_pick_epi(const void *x, const void *w, const IgemmParams &p, con
     case EPI_SCALAR: return -1;
     case EPI_Q8_RELU6: return stem_launch<KW4, STEPS, EPI_Q8_RELU6>(x, w, p, e, s);
     case EPI_Q8_RELU: return stem_launch<KW4, STEPS, EPI_Q8_RELU>(x, w, p, e, s);
+    case EPI_Y32: return stem_launch<KW4, STEPS, EPI_Y32>(x, w, p, e, s);
+    case EPI_Y16_STEPS: return stem_launch<KW4, STEPS, EPI_Y16_STEPS>(x, w, p, e, s);
     default: return stem_launch<KW4, STEPS, EPI_VECTOR>(x, w, p, e, s);
   }
 }

@@ -121,7 +121,8 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   if (epi_wave && vec) {
     const int cc = min(ec, p.N - 4);
     if (e.chan_div) c_div = *reinterpret_cast<const v4f *>(e.chan_div + cc);
-    if (e.chan_rcp) c_rcp = *reinterpret_cast<const v4f *>(e.chan_rcp + cc);
+    const float *rcps = e.chan_rcp ? e.chan_rcp : e.half_rcp;
+    if (rcps) c_rcp = *reinterpret_cast<const v4f *>(rcps + cc);
     if (e.bias) c_bias = *reinterpret_cast<const v4f *>(e.bias + cc);
     if constexpr (DUAL) {
       if (p.sc.chan_div) s_div = *reinterpret_cast<const v4f *>(p.sc.chan_div + cc);
@@ -323,6 +324,8 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       case EPI_Y32: run(EpiOf<EPI_Y32>::type{}); break;
       case EPI_RES_Q8: run(EpiOf<EPI_RES_Q8>::type{}); break;
       case EPI_Q8_RELU6: run(EpiOf<EPI_Q8_RELU6>::type{}); break;
+      case EPI_Y16: run(EpiOf<EPI_Y16>::type{}); break;
+      case EPI_Y16_STEPS: run(EpiOf<EPI_Y16_STEPS>::type{}); break;
       default: run(EpiGeneric{}); break;
     }
   }
