@@ -73,6 +73,7 @@ SIGNATURES = {
     "catchq_quantize_nchw_to_nhwc_frame": (_I, [_P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _F, _P]),
     "catchq_quantize_param_workspace_size": (_I, [_I64, ctypes.POINTER(_SZ)]),
     "catchq_quantize_param": (_I, [_P, _I, _I64, _I, _I, _P, _SZ, _P, _P, _P, _P, _P]),
+    "catchq_quantize_param_whole": (_I, [_P, _I, _I64, _I, _I, _P, _SZ, _P, _P, _P, _P, _P]),
     "catchq_quantize_param_noalloc": (_I, [_P, _I, _I64, _I, _I, _P, _P, _P, _P, _P]),
     "catchq_quantize_per_channel": (_I, [_P, _I, _P, _I, _I, _I64, _P, _P]),
     "catchq_quantize_per_channel_f16": (_I, [_P, _P, _I, _I, _I64, _P, _P]),

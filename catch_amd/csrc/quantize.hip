@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kThreads) void quantize_frame_f32_i8c4_kernel(const
   }
 }
 
-// General (any C) transpose-quantize through LDS: tile of 64 pixels x 64 channels.
+// General (any C) transpose-quantize through LDS: tile of 64 pixels x 64 channels, any alignment and pitch of the output.
 template <typename TIn, int BW>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_nhwc_tile_kernel(const TIn *__restrict__ x,
                                                                           typename QRange<BW>::type *__restrict__ q,
@@ -293,6 +293,80 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_nhwc_tile_kernel(const
   }
 }
 
+// The same where a pixel of the output is a whole number of aligned 16-byte pieces.  Bound by memory; the kernel above is
+// bound by its instructions (a load, a conversion, a byte store to LDS, one back and a byte store to memory per element:
+// 5 x 96 x 57 x 75 fp32 -> int8 took 10.4 us, this one 4.6).  A lane takes four consecutive pixels of four channels (four
+// 16-byte loads, a wave instruction covering 256 consecutive bytes of four planes), packs a pixel's four channels into a
+// dword (two for int16) in LDS -- the pitch of 16 DW + 1 dwords spreads a wave's stores over all banks -- and leaves with
+// 16-byte stores that cover whole 64-byte runs of a pixel.
+template <typename TIn> struct __attribute__((aligned(sizeof(TIn)))) px4 { TIn v[4]; };
+template <typename TIn, int BW>
+__global__ __launch_bounds__(kThreads) void quantize_nchw_nhwc_vec_kernel(const TIn *__restrict__ x,
+                                                                         typename QRange<BW>::type *__restrict__ q,
+                                                                         int c, int hw, int cpad, int pos, float scale) {
+  constexpr int DW = BW / 8;              // dwords of a pixel's four channels
+  constexpr int PITCH = 16 * DW + 1;
+  __shared__ int tile[64 * PITCH];
+  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
+  const int64_t img = blockIdx.z;
+  const int pg = threadIdx.x & 15, cq = threadIdx.x >> 4;
+  const int px = p0 + pg * 4, ch = c0 + cq * 4;
+  const TIn *src = x + (img * c + ch) * (int64_t)hw + px;
+  float v[4][4];  // [channel][pixel]
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (ch + j < c && px + 4 <= hw) {
+      const px4<TIn> t = *reinterpret_cast<const px4<TIn> *>(src + (int64_t)j * hw);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = ld_f(t.v, i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[j][i] = (ch + j < c && px + i < hw) ? ld_f(src + (int64_t)j * hw, i) : 0.0f;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int b[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) b[j] = quant1<BW>(v[j][i], scale, -pos);  // 0 -> 0: the padding channels
+    int *dst = tile + (pg * 4 + i) * PITCH + cq * DW;
+    if constexpr (BW == 8) {
+      dst[0] = (int)(__builtin_amdgcn_perm((unsigned)b[1], (unsigned)b[0], 0x0c0c0400u) |
+                     __builtin_amdgcn_perm((unsigned)b[3], (unsigned)b[2], 0x04000c0cu));
+    } else {
+      dst[0] = (b[0] & 0xffff) | (b[1] << 16);
+      dst[1] = (b[2] & 0xffff) | (b[3] << 16);
+    }
+  }
+  __syncthreads();
+  constexpr int PIECES = 4 * DW;  // 16-byte pieces of a pixel's 64 channels
+  const int piece = threadIdx.x % PIECES;
+  const bool c_ok = c0 * DW + piece * 16 < cpad * DW;
+#pragma unroll
+  for (int r = 0; r < DW; ++r) {
+    const int p = threadIdx.x / PIECES + r * (kThreads / PIECES);
+    const int *s = tile + p * PITCH + piece * 4;
+    if (c_ok && p0 + p < hw)
+      reinterpret_cast<v4i *>(q + (img * hw + p0 + p) * (int64_t)cpad + c0)[piece] = v4i{s[0], s[1], s[2], s[3]};
+  }
+}
+
+// Rows of c values -> rows of cpad (images of one pixel): four values per lane, zeros behind the row's end.
+template <typename TIn, int BW>
+__global__ __launch_bounds__(kThreads) void quantize_rows_kernel(const TIn *__restrict__ x, typename QRange<BW>::type *__restrict__ q,
+                                                                int64_t rows, int c, int cpad, int pos, float scale) {
+  typedef typename QRange<BW>::type TQ;
+  struct __attribute__((aligned(4 * sizeof(TQ)))) q4 { TQ v[4]; };
+  for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
+    for (int k = (blockIdx.x * kThreads + threadIdx.x) * 4; k < cpad; k += gridDim.x * kThreads * 4) {
+      q4 o;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) o.v[i] = (TQ)quant1<BW>(k + i < c ? ld_f(x, r * c + k + i) : 0.0f, scale, -pos);
+      *reinterpret_cast<q4 *>(q + r * cpad + k) = o;
+    }
+  }
+}
+
 template <typename TIn, int BW>
 static int launch_nchw_nhwc(const void *x, void *q, int n, int c, int h, int w, int cpad, int pos, float scale,
                             hipStream_t s) {
@@ -306,6 +380,15 @@ static int launch_nchw_nhwc(const void *x, void *q, int n, int c, int h, int w, 
   } else if (cpad == 8 && vec_ok && BW == 8) {
     quantize_nchw_nhwc_kernel<TIn, BW, 8><<<grid_for(total, kThreads), kThreads, 0, s>>>(
         (const TIn *)x, (TQ *)q, n, c, hw, pos, scale);
+  } else if (hw == 1 && cpad % 4 == 0 && aligned16(q)) {
+    // (a row as a pixel of its own left the tile kernel below one useful pixel in 64: 1379 x 1001 fp16 -> int8 x 1008
+    // took 104 us)
+    const unsigned gy = n < 65535 ? (unsigned)n : 65535u;
+    quantize_rows_kernel<TIn, BW><<<dim3((unsigned)((cpad + kThreads * 4 - 1) / (kThreads * 4)), gy), kThreads, 0, s>>>(
+        (const TIn *)x, (TQ *)q, n, c, cpad, pos, scale);
+  } else if (cpad * sizeof(TQ) % 16 == 0 && aligned16(q) && n < 65536 && cpad < 65536 * 64 && hw < (1ll << 31) - 64) {
+    quantize_nchw_nhwc_vec_kernel<TIn, BW><<<dim3((unsigned)((hw + 63) / 64), (unsigned)((cpad + 63) / 64), (unsigned)n), kThreads, 0, s>>>(
+        (const TIn *)x, (TQ *)q, c, (int)hw, cpad, pos, scale);
   } else {
     int64_t tiles = (int64_t)n * ((hw + 63) / 64) * ((cpad + 63) / 64);
     quantize_nchw_nhwc_tile_kernel<TIn, BW><<<grid_for(tiles, 1), kThreads, 0, s>>>(
@@ -483,79 +566,96 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+template <int NT>
+__device__ __forceinline__ float block_max(float m) {  // valid in thread 0
+  __shared__ float wm[NT / 64];
+  m = wave_max(m);
+  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int i = 1; i < NT / 64; ++i) m = fmaxf(m, wm[i]);
+  return m;
+}
+
+// largest absolute value of one lane's share: lane `first` of `stride`, nvec 16-byte vectors, then the rest one by one
+template <typename TIn, int UNROLL>
+__device__ __forceinline__ float absmax_slice(const TIn *__restrict__ x, int64_t n, int64_t first, int64_t stride, int64_t nvec) {
+  constexpr int VEC = 16 / sizeof(TIn);
+  float m = 0.0f;  // fmaxf ignores NaN operands, like the oracle's comparison
+  // UNROLL 16-byte loads (a stride apart) in flight per lane; the data is read once: non-temporal
+  for (int64_t i0 = first; i0 < nvec; i0 += stride * UNROLL) {
+    v4i raw[UNROLL];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      const int64_t i = i0 + u * stride;
+      raw[u] = v4i{0, 0, 0, 0};  // |+0| never wins
+      if (i < nvec) raw[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(x) + i);
+    }
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      if constexpr (sizeof(TIn) == 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) m = fmaxf(m, fabsf(__int_as_float(raw[u][j])));
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const __half2 h = as_half2(raw[u][j]);
+          m = fmaxf(m, fmaxf(fabsf(__low2float(h)), fabsf(__high2float(h))));
+        }
+      }
+    }
+  }
+  for (int64_t i = nvec * VEC + first; i < n; i += stride) m = fmaxf(m, fabsf(ld_f(x, i)));
+  return m;
+}
+
 template <typename TIn, int UNROLL = 4>
 __global__ __launch_bounds__(kThreads) void absmax_partial_kernel(const TIn *__restrict__ x, int64_t n,
                                                                  float *__restrict__ partial, int vec_ok) {
   constexpr int VEC = 16 / sizeof(TIn);
-  float m = 0.0f;  // fmaxf ignores NaN operands, like the oracle's comparison
-  const int64_t stride = (int64_t)gridDim.x * kThreads;
-  int64_t done = 0;
-  if (vec_ok) {
-    // UNROLL 16-byte loads (a grid stride apart) in flight per lane; the data is read once: non-temporal
-    const int64_t nvec = n / VEC;
-    for (int64_t i0 = (int64_t)blockIdx.x * kThreads + threadIdx.x; i0 < nvec; i0 += stride * UNROLL) {
-      v4i raw[UNROLL];
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        const int64_t i = i0 + u * stride;
-        raw[u] = v4i{0, 0, 0, 0};  // |+0| never wins
-        if (i < nvec) raw[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(x) + i);
-      }
-#pragma unroll
-      for (int u = 0; u < UNROLL; ++u) {
-        if constexpr (sizeof(TIn) == 4) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) m = fmaxf(m, fabsf(__int_as_float(raw[u][j])));
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const __half2 h = as_half2(raw[u][j]);
-            m = fmaxf(m, fmaxf(fabsf(__low2float(h)), fabsf(__high2float(h))));
-          }
-        }
-      }
-    }
-    done = nvec * VEC;
-  }
-  for (int64_t i = done + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
-    m = fmaxf(m, fabsf(ld_f(x, i)));
-  __shared__ float wm[kThreads / 64];
-  m = wave_max(m);
-  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float r = wm[0];
-    for (int i = 1; i < kThreads / 64; ++i) r = fmaxf(r, wm[i]);
-    partial[blockIdx.x] = r;
-  }
+  const float m = block_max<kThreads>(absmax_slice<TIn, UNROLL>(x, n, (int64_t)blockIdx.x * kThreads + threadIdx.x,
+                                                               (int64_t)gridDim.x * kThreads, vec_ok ? n / VEC : 0));
+  if (threadIdx.x == 0) partial[blockIdx.x] = m;
 }
 
-__global__ __launch_bounds__(kThreads) void absmax_finalize_kernel(const float *__restrict__ partial, int nparts,
-                                                                  int bw, float *absmax_out, int32_t *pos_out,
-                                                                  float *scale_out, float *offset_out) {
+// the parameters of a tensor whose largest absolute value is known; what a mode does not derive is left alone (null
+// pointers) or, with `whole`, set to the neutral value (scale 1, offset 0)
+struct ParamOut {
+  int bw, derive_scale;
+  float *absmax;
+  int32_t *pos;
+  float *scale, *offset;
+};
+__device__ __forceinline__ void write_params(float absmax, const ParamOut &o) {
+  const float qmax = (o.bw == 16) ? 32767.0f : 127.0f;
+  int pos = 0;
+  float scale = 1.0f;
+  if (absmax > 0.0f && absmax < __builtin_inff()) {
+    // floor(log2(absmax)) from the exponent: exact, no transcendental
+    pos = ilogbf(absmax) - (o.bw - 2);
+    // absmax * 2^-pos is exact (also for a denormal absmax), so the quotient is rounded once
+    scale = qmax / __builtin_ldexpf(absmax, -pos);
+  }
+  if (o.absmax) *o.absmax = absmax;
+  if (o.pos) *o.pos = pos;
+  if (o.scale) *o.scale = o.derive_scale ? scale : 1.0f;
+  if (o.offset) *o.offset = 0.0f;
+}
+
+__global__ __launch_bounds__(kThreads) void absmax_finalize_kernel(const float *__restrict__ partial, int nparts, ParamOut o) {
   float m = 0.0f;
   for (int i = threadIdx.x; i < nparts; i += kThreads) m = fmaxf(m, partial[i]);
-  __shared__ float wm[kThreads / 64];
-  m = wave_max(m);
-  if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float absmax = wm[0];
-    for (int i = 1; i < kThreads / 64; ++i) absmax = fmaxf(absmax, wm[i]);
-    const float qmax = (bw == 16) ? 32767.0f : 127.0f;
-    int pos = 0;
-    float scale = 1.0f;
-    if (absmax > 0.0f && absmax < __builtin_inff()) {
-      // floor(log2(absmax)) from the exponent: exact, no transcendental
-      pos = ilogbf(absmax) - (bw - 2);
-      // absmax * 2^-pos is exact (also for a denormal absmax), so the quotient is rounded once
-      scale = qmax / __builtin_ldexpf(absmax, -pos);
-    }
-    if (absmax_out) *absmax_out = absmax;
-    if (pos_out) *pos_out = pos;
-    if (scale_out) *scale_out = scale;
-    if (offset_out) *offset_out = 0.0f;
-  }
+  m = block_max<kThreads>(m);
+  if (threadIdx.x == 0) write_params(m, o);
+}
+
+// A tensor that one block reads in about the time of a launch: reduction and parameters in one launch.
+constexpr int kOneBlock = 1024;
+template <typename TIn>
+__global__ __launch_bounds__(kOneBlock) void absmax_one_block_kernel(const TIn *__restrict__ x, int n, ParamOut o) {
+  constexpr int VEC = 16 / sizeof(TIn);
+  const float m = block_max<kOneBlock>(absmax_slice<TIn, 4>(x, n, threadIdx.x, kOneBlock, n / VEC));
+  if (threadIdx.x == 0) write_params(m, o);
 }
 
 }  // namespace catchq
@@ -646,27 +746,49 @@ CATCHQ_API int catchq_quantize_param_workspace_size(int64_t n, size_t *bytes) {
   return CATCHQ_OK;
 }
 
-CATCHQ_API int catchq_quantize_param(const void *x, int x_dtype, int64_t n, int bitwidth, int mode,
-                                     void *workspace, size_t workspace_bytes, float *absmax_dev,
-                                     int32_t *position_dev, float *scale_dev, float *offset_dev,
-                                     catchq_stream_t stream) {
+// whole: every output is written in every mode
+static int quantize_param(const void *x, int x_dtype, int64_t n, int bitwidth, int mode, void *workspace, size_t workspace_bytes,
+                          float *absmax_dev, int32_t *position_dev, float *scale_dev, float *offset_dev, bool whole,
+                          hipStream_t s) {
   if (n < 0 || (n > 0 && !x) || !workspace) return CATCHQ_ERR_ARG;
   if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
   if (bitwidth != 8 && bitwidth != 16) return CATCHQ_ERR_BITWIDTH;
   if (mode < CATCHQ_QUANTIZE_POSITION || mode > CATCHQ_QUANTIZE_POSITION_SCALE_OFFSET) return CATCHQ_ERR_ARG;
   const int blocks = absmax_blocks(n);
   if (workspace_bytes < sizeof(float) * (size_t)blocks) return CATCHQ_ERR_ARG;
-  hipStream_t s = as_stream(stream);
+  const bool scale = mode >= CATCHQ_QUANTIZE_POSITION_SCALE, offset = mode >= CATCHQ_QUANTIZE_POSITION_SCALE_OFFSET;
+  const ParamOut o = {bitwidth, scale ? 1 : 0, absmax_dev, position_dev, scale || whole ? scale_dev : nullptr,
+                      offset || whole ? offset_dev : nullptr};
+  // up to 256 KiB one block's loads take what the second launch would
+  if (n * (x_dtype == CATCHQ_F32 ? 4 : 2) <= (256 << 10) && aligned16(x)) {
+    if (x_dtype == CATCHQ_F32) absmax_one_block_kernel<float><<<1, kOneBlock, 0, s>>>((const float *)x, (int)n, o);
+    else absmax_one_block_kernel<__half><<<1, kOneBlock, 0, s>>>((const __half *)x, (int)n, o);
+    return launch_status();
+  }
   float *partial = (float *)workspace;
   if (x_dtype == CATCHQ_F32)
     absmax_partial_kernel<float><<<blocks, kThreads, 0, s>>>((const float *)x, n, partial, aligned16(x) ? 1 : 0);
   else
     absmax_partial_kernel<__half><<<blocks, kThreads, 0, s>>>((const __half *)x, n, partial, aligned16(x) ? 1 : 0);
   if (launch_status() != CATCHQ_OK) return CATCHQ_ERR_LAUNCH;
-  absmax_finalize_kernel<<<1, kThreads, 0, s>>>(partial, blocks, bitwidth, absmax_dev, position_dev,
-                                               mode >= CATCHQ_QUANTIZE_POSITION_SCALE ? scale_dev : nullptr,
-                                               mode >= CATCHQ_QUANTIZE_POSITION_SCALE_OFFSET ? offset_dev : nullptr);
+  absmax_finalize_kernel<<<1, kThreads, 0, s>>>(partial, blocks, o);
   return launch_status();
+}
+
+CATCHQ_API int catchq_quantize_param(const void *x, int x_dtype, int64_t n, int bitwidth, int mode,
+                                     void *workspace, size_t workspace_bytes, float *absmax_dev,
+                                     int32_t *position_dev, float *scale_dev, float *offset_dev,
+                                     catchq_stream_t stream) {
+  return quantize_param(x, x_dtype, n, bitwidth, mode, workspace, workspace_bytes, absmax_dev, position_dev, scale_dev, offset_dev,
+                        false, as_stream(stream));
+}
+
+CATCHQ_API int catchq_quantize_param_whole(const void *x, int x_dtype, int64_t n, int bitwidth, int mode,
+                                           void *workspace, size_t workspace_bytes, float *absmax_dev,
+                                           int32_t *position_dev, float *scale_dev, float *offset_dev,
+                                           catchq_stream_t stream) {
+  return quantize_param(x, x_dtype, n, bitwidth, mode, workspace, workspace_bytes, absmax_dev, position_dev, scale_dev, offset_dev,
+                        true, as_stream(stream));
 }
 
 // ---- the same reduction for callers that cannot allocate ---------------------------------------------------

@@ -107,11 +107,11 @@ std::tuple<Tensor, Tensor, Tensor> quantize_param_op(const Tensor &x, int64_t bi
   Tensor xi = x.is_non_overlapping_and_dense() ? x : x.contiguous();
   size_t ws_bytes = 0;
   check_status(catchq_quantize_param_workspace_size(xi.numel(), &ws_bytes), "torch_mlu::quantize_param");
-  Tensor ws = at::empty({(int64_t)ws_bytes}, xi.options().dtype(at::kChar));
-  Tensor pos = at::empty({1}, xi.options().dtype(at::kInt));
-  Tensor scale = at::ones({1}, xi.options().dtype(at::kFloat));
-  Tensor offset = at::zeros({1}, xi.options().dtype(at::kFloat));
-  check_status(catchq_quantize_param(xi.data_ptr(), dt, xi.numel(), (int)bitwidth, (int)mode, ws.data_ptr(),
+  Tensor ws = device_empty({(int64_t)ws_bytes}, at::kChar, xi.device());
+  Tensor pos = device_empty({1}, at::kInt, xi.device());
+  Tensor scale = device_empty({1}, at::kFloat, xi.device());
+  Tensor offset = device_empty({1}, at::kFloat, xi.device());
+  check_status(catchq_quantize_param_whole(xi.data_ptr(), dt, xi.numel(), (int)bitwidth, (int)mode, ws.data_ptr(),
                                      ws_bytes, nullptr, pos.data_ptr<int32_t>(), scale.data_ptr<float>(),
                                      offset.data_ptr<float>(), current_stream()),
                "torch_mlu::quantize_param");

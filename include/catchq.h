@@ -110,6 +110,12 @@ int catchq_quantize_param(const void *x, int x_dtype, int64_t n, int bitwidth, i
                           size_t workspace_bytes, float *absmax_dev, int32_t *position_dev,
                           float *scale_dev, float *offset_dev, catchq_stream_t stream);
 
+/* The same, every output written in every mode (scale 1, offset 0 where the mode does not derive them): a caller that
+ * wants the reference's three tensors need not initialise them first. */
+int catchq_quantize_param_whole(const void *x, int x_dtype, int64_t n, int bitwidth, int mode, void *workspace,
+                                size_t workspace_bytes, float *absmax_dev, int32_t *position_dev, float *scale_dev,
+                                float *offset_dev, catchq_stream_t stream);
+
 /* catchq_quantize_param for callers that cannot allocate device memory or bring a workspace (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the
  * reference, whose wrapper allocates the vendor workspace on every call (operators/cnnl/internal/quantize_param.cpp:67-83).

@@ -97,6 +97,20 @@ def test_quantize_nchw_to_nhwc(shape, cpad, bw):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("bw", [8, 16])
+@pytest.mark.parametrize("shape,cpad", [((2, 96, 5, 7), 96), ((3, 70, 9, 9), 80), ((1, 16, 1, 63), 16), ((2, 130, 8, 8), 144),
+                                        ((2, 5, 13, 5), 16), ((5, 101, 1, 1), 112), ((300, 1030, 1, 1), 1040), ((2, 3, 1, 1), 4)])
+def test_quantize_transpose_and_row_padding(shape, cpad, bw, dtype):
+    """tiles of 64 pixels x 64 channels with ragged edges on both sides, channel padding, rows padded behind their end"""
+    note("quantize transpose", shape, cpad, bw, dtype)
+    x = (rng(sum(shape)).standard_normal(shape) * 3).astype(dtype)
+    x.reshape(-1)[::17] = [np.nan, np.inf, -np.inf, 1e4][sum(shape) % 4]
+    want = np.zeros((shape[0],) + shape[2:] + (cpad,), np.int8 if bw == 8 else np.int16)
+    want[..., :shape[1]] = orc.quantize(x, bw, -5).transpose(0, 2, 3, 1)
+    assert same_bits(want, cabi.quantize_nchw_to_nhwc(cabi.dev(x), bw, -5, cpad=cpad).cpu().numpy())
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("n", [1, 7, 100000, 4096 * 300 + 3, 4096 * 256 * 4 * 5 + 1029])
 def test_quantize_param(dtype, n):
     note("quantize_param", dtype.__name__, n)
