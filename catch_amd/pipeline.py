@@ -13,6 +13,7 @@ Every value is computed by the same arithmetic, in the same order, as the unfuse
 quantize -> integer conv -> dequant+bias -> add -> activation -> quantize, so all quantized
 tensors, int32 accumulators and fp32 outputs are identical to it bit for bit.
 """
+import copy
 import ctypes
 
 import numpy as np
@@ -187,6 +188,7 @@ class FusedNet(object):
         fuse_avgpool: a 1x1 convolution whose only reader is the global average pooling runs inside the pooling's launch
         (torch_mlu::qconv2d_avgpool) where the library's kernel serves the shape; its fp32 output is then never stored."""
         self.layers = list(layers)
+        self._fuse_shortcuts = fuse_shortcuts
         self.device = torch.device(device)
         self.outputs = outputs_of(self.layers)
         self.out_half = out_half
@@ -226,30 +228,12 @@ class FusedNet(object):
         # Projection shortcuts (1x1 convolution, no activation, consumed only as the residual of one
         # convolution): evaluated inside that convolution's launch, their fp32 output is never stored.
         # shortcut_of: main layer name -> shortcut layer; a traced pass runs them as launches of their own.
-        self.shortcut_of = {}
-        if fuse_shortcuts:
-            by_name = {l.name: l for l in self.layers}
-            for l in self.layers:
-                ds = by_name.get(l.add) if l.kind == "conv" and l.add else None
-                if ds is None or ds.kind != "conv" or l.groups != 1:
-                    continue
-                readers = [m for m in self.layers
-                           if m.src == ds.name or (isinstance(m.src, tuple) and ds.name in m.src) or m.add == ds.name]
-                lq, dq = self.q[l.name], self.q[ds.name]
-                if (ds.k == 1 and ds.pad == 0 and ds.groups == 1 and ds.act == "none" and not ds.add
-                        and readers == [l] and ds.name not in self.outputs and not self.q_demand[ds.name]
-                        and (lq.bw_x, lq.bw_w, dq.bw_x, dq.bw_w) == (8, 8, 8, 8)
-                        and not (self.stem and self.stem["name"] in (l.name, ds.name))):
-                    self.shortcut_of[l.name] = ds
+        self.shortcut_of = self._plan_shortcuts() if fuse_shortcuts else {}
         # Residual chains: chain_of[name] = [shortcut layer, last convolution of block 0, .., this layer]
         self.chain_of = {}
         if fuse_shortcuts and chain_links != 0:
             self._plan_chains(chain_links)
-        # a shortcut has no launch of its own when its one reader, the first block's last convolution, evaluates it
-        # itself (as a two-branch launch or as the head of a chain); later blocks' chains recompute it either way
-        self._fused_away = set(ds.name for ds in self.shortcut_of.values())
-        self._fused_away.update(links[0].name for links in self.chain_of.values()
-                                if links[1].name in self.chain_of or links[1].name in self.shortcut_of)
+        self._fused_away = self._layers_fused_away()
         # Heads: head_of[3x3 layer name] = the 1x1 layer in front of it.  Whether a pair runs as one launch also
         # depends on the image size (head_fuses), known when a batch arrives.
         self.head_of = {}
@@ -344,6 +328,55 @@ class FusedNet(object):
             self._block_inner[x.name] = pname
             self._block_inner[d.name] = pname
 
+        self._few = None  # the plan for few pixels (_few_plan), made when first needed
+
+    def _plan_shortcuts(self):
+        by_name = {l.name: l for l in self.layers}
+        shortcut_of = {}
+        for l in self.layers:
+            ds = by_name.get(l.add) if l.kind == "conv" and l.add else None
+            if ds is None or ds.kind != "conv" or l.groups != 1:
+                continue
+            readers = [m for m in self.layers
+                       if m.src == ds.name or (isinstance(m.src, tuple) and ds.name in m.src) or m.add == ds.name]
+            lq, dq = self.q[l.name], self.q[ds.name]
+            if (ds.k == 1 and ds.pad == 0 and ds.groups == 1 and ds.act == "none" and not ds.add
+                    and readers == [l] and ds.name not in self.outputs and not self.q_demand[ds.name]
+                    and (lq.bw_x, lq.bw_w, dq.bw_x, dq.bw_w) == (8, 8, 8, 8)
+                    and not (self.stem and self.stem["name"] in (l.name, ds.name))):
+                shortcut_of[l.name] = ds
+        return shortcut_of
+
+    def _layers_fused_away(self):
+        """shortcuts without a launch of their own: their one reader, the first block's last convolution, evaluates them
+        itself (as a two-branch launch or as the head of a chain); later blocks' chains recompute them either way"""
+        away = set(ds.name for ds in self.shortcut_of.values())
+        away.update(links[0].name for links in self.chain_of.values()
+                    if links[1].name in self.chain_of or links[1].name in self.shortcut_of)
+        return away
+
+    @staticmethod
+    def _few_pixels(n, h, w):
+        """Whether a batch is planned block by block (_few_plan): one two-branch launch per projection block and no residual
+        chain.  A chain recomputes a block's earlier branches to save fp32 traffic; up to two images of 224 x 224 there is
+        no traffic to speak of and its 64 x 128 tiles are a handful of blocks, where the two-branch launch has the
+        few-tiles kernel (ResNet-50, one stream: one image 234 -> 230 us, 2 x 224 x 224 ties, 4 x 128 x 128 233 -> 227 us;
+        6 x 224 x 224 loses, 336 -> 347 us)."""
+        return n * h * w <= 2 * 224 * 224
+
+    def _few_plan(self):
+        """the same network planned for few pixels"""
+        if self._few is None:
+            few = copy.copy(self)
+            few.chain_of = {}
+            few.head_of, few._head_names = {}, set()
+            few.shortcut_of = few._plan_shortcuts() if self._fuse_shortcuts else {}
+            few._fused_away = few._layers_fused_away()
+            few._plan_demands()
+            few._few = few
+            self._few = few
+        return self._few
+
     def block_fuses(self, proj, n, h, w):
         """whether the inverted-residual block that ends in the layer `proj` runs as one launch over n images whose
         block input is h x w.  The one-launch kernel is bound by the same vector arithmetic as the three launches and
@@ -375,8 +408,10 @@ class FusedNet(object):
         return bool(torch.ops.torch_mlu.conv1x1_avgpool_fuses(n, h * w, self.cdev[c.src], self.cdev[c.name]))
 
     def head_fuses(self, head, n, h, w):
-        """whether the 1x1 layer `head` and the 3x3 layer behind it run as one launch over n images of h x w"""
-        if head.name not in self._head_names:
+        """whether the 1x1 layer `head` and the 3x3 layer behind it run as one launch over n images of h x w.  Up to eight
+        images of 56 x 56 its bands of rows leave half of the device idle and two launches of the small-grid kernels are
+        faster (ResNet-50, one stream: 1 image 247 -> 234 us, 8 images 353 -> 348 us, 12 images 404 -> 406 us)."""
+        if head.name not in self._head_names or n * h * w <= 8 * 56 * 56:
             return False
         main = next(l for l in self.layers if self.head_of.get(l.name) is head)
         return bool(torch.ops.torch_mlu.conv1x1_conv3x3_fuses(n, h, w, self.cdev[head.src], self.cdev[head.name],
@@ -483,6 +518,8 @@ class FusedNet(object):
         timers: optional dict; every conv/fc launch is bracketed by a pair of events recorded on
         the current stream and the pair is appended to timers[layer name] (durations of the
         launches in their real sequence, caches as the previous layer left them)."""
+        if trace is None and self is not self._few and self._few_pixels(x.shape[0], x.shape[2], x.shape[3]):
+            return self._few_plan().forward(x, None, timers, keep)
         ops = torch.ops.torch_mlu
         env = {}
         tracing = trace is not None
@@ -701,11 +738,16 @@ class FusedNet(object):
         streams > 1 splits the batch into that many parts, each recorded on a stream of its own (all of
         default priority) between a fork and a join: the images are independent, so the results are the
         same tensors, and the launches of one part fill the compute units that the other part's launches
-        leave idle while they start up and drain."""
+        leave idle while they start up and drain.  A batch whose launches are too short for that is recorded as fewer
+        parts (_parts)."""
         static_in = example.clone()
-        parts = max(1, min(int(streams), static_in.shape[0]))
+        asked = max(1, min(int(streams), static_in.shape[0]))
+        parts = self._parts(asked, *static_in.shape)
         chunks = list(static_in.chunk(parts))
-        side = [torch.cuda.Stream() for _ in chunks]
+        # As many streams as asked for are drawn from the pool, used or not: its streams take turns on the four hardware
+        # queues, and a capture that advanced it by one left the branches of later graphs on one queue (Darknet-53 in two
+        # parts behind MobileNetV2 captures of one: 2.57 -> 3.0 ms)
+        side = [torch.cuda.Stream() for _ in range(asked)][:len(chunks)]
         # the launches recorded below will share the device: their tile shapes are chosen for a part of it (a hint
         # of this thread, handed to the kernel library with every call)
         before = torch.ops.torch_mlu.set_launch_sharing(len(chunks))
@@ -713,6 +755,37 @@ class FusedNet(object):
             return self._capture(static_in, chunks, side)
         finally:
             torch.ops.torch_mlu.set_launch_sharing(max(before, 1))
+
+    def _parts(self, parts, n, c, h, w):
+        """How many of the `parts` asked for pay.  A graph that is one chain of launches runs them back to back; one with
+        parallel branches is fed node by node, 4.0 to 4.3 us each (MobileNetV2 at 192 x 192, two parts: 426 us for 4 images
+        and 431 us for 27), so the batch has to keep the device busy for longer than that: its time as one chain -- 2.6 us
+        per launch + 0.65 us per million output elements + 1.76 us per billion int8 multiply-accumulates, fitted to
+        ResNet-50 and MobileNetV2 at batches of 64 and 128 -- less the 7 % that the overlap is worth.  Measured, one / two
+        parts: MobileNetV2 192 x 192, 27 images 277 / 431 us, 128 images 617 / 569; ResNet-50 224 x 224, 8 images
+        350 / 382 us, 16 447 / 451, 24 565 / 546, 64 1044 / 972; ResNet-18, 32 images 354 / 366, 64 571 / 548."""
+        if parts == 1:
+            return 1
+        size, launches, elems, macs = {"input": (h, w)}, 0, 0, 0
+        for l in self.layers:
+            hi, wi = size[l.src if isinstance(l.src, str) else l.src[0]]
+            if l.kind in ("conv", "maxpool"):
+                hi, wi = (hi + 2 * l.pad - l.k) // l.stride + 1, (wi + 2 * l.pad - l.k) // l.stride + 1
+            elif l.kind in ("gap", "fc"):
+                hi = wi = 1
+            elif l.kind == "upsample":
+                hi, wi = 2 * hi, 2 * wi
+            size[l.name] = hi, wi
+            if l.name in self._fused_away or l.name in self._pooled_names or (self.first_pool and l is self.first_pool):
+                continue
+            launches += 1
+            if l.kind in ("conv", "fc"):
+                elems += n * hi * wi * l.co
+                macs += n * hi * wi * l.co * (l.ci // (l.groups or 1)) * (l.k or 1) ** 2 * (2 if self.q[l.name].bw_x == 16 else 1)
+        chain_us = 2.6 * launches + 0.65e-6 * elems + 1.76e-9 * macs
+        while parts > 1 and 0.93 * chain_us < 4.2 * launches * parts:
+            parts -= 1
+        return parts
 
     def _capture(self, static_in, chunks, side):
         """Side streams only ever wait on the capturing stream (fork) and are only ever waited on by it (join).
