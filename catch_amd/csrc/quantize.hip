@@ -94,7 +94,8 @@ static int launch_quantize(const void *x, void *q, int64_t n, int pos, float sca
   typedef typename QRange<BW>::type TQ;
   constexpr int VEC = 16 / sizeof(TIn);
   if (aligned16(x) && aligned16(q)) {
-    quantize_vec_kernel<TIn, BW><<<grid_for(n / VEC, kThreads * 4), kThreads, 0, s>>>(
+    // one vector per lane until the device is full: a lane's loads follow each other
+    quantize_vec_kernel<TIn, BW><<<grid_for(n / VEC, kThreads), kThreads, 0, s>>>(
         (const TIn *)x, (TQ *)q, n, pos, scale, pos_dev, scale_dev);
   } else {
     quantize_scalar_kernel<TIn, BW><<<grid_for(n, kThreads * 4), kThreads, 0, s>>>(
