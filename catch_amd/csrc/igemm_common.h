@@ -213,9 +213,8 @@ __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev
   return epi_lane_finish<S>(div, rcp, bias, e);
 }
 
-// dequantization and bias of one integer sum: channel t of the lane's four
-__device__ __forceinline__ float epi_dequant1(int a, int t, const EpiLane &L, int exp2) {
-  float x = (float)a;
+// dequantization and bias of one integer sum (converted to fp32 once): channel t of the lane's four
+__device__ __forceinline__ float epi_dequant1(float x, int t, const EpiLane &L, int exp2) {
   if (L.steps_rcp) {
     // fp32 operations on binary16 values rounded to binary16 are the binary16 operations.  The reciprocal form gives the
     // correctly rounded fp32 quotient of the finite values; an infinite one (the scaled sum overflowed) stays infinite.
@@ -279,14 +278,17 @@ __device__ __forceinline__ T load_stream(const T *src, bool stream) {
   return v;
 }
 
-// four integer sums of one pixel (channels n..n+3 at `where`) -> all requested outputs
-template <class S, class At>
-__device__ __forceinline__ void epi_vec4(const v4i a, const v4f res, const EpiLane &L, const At where, const EpiDev &e) {
-  if (S::acc(e)) *reinterpret_cast<v4i *>(where.at(e.acc_out)) = a;
+// four integer sums of one pixel (channels n..n+3 at `where`) -> all requested outputs; sums too wide for an int32 come
+// converted to fp32 (v4f)
+template <class S, class At, class Sums>
+__device__ __forceinline__ void epi_vec4(const Sums a, const v4f res, const EpiLane &L, const At where, const EpiDev &e) {
+  if constexpr (std::is_same<Sums, v4i>::value) {
+    if (S::acc(e)) *reinterpret_cast<v4i *>(where.at(e.acc_out)) = a;
+  }
   float v[4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    float x = epi_dequant1(a[t], t, L, e.exp2);
+    float x = epi_dequant1((float)a[t], t, L, e.exp2);
     if (L.use_res && !L.res_after) x = x + res[t];
     if constexpr (!S::kFoldAct) {
       if (L.act == CATCHQ_ACT_LEAKY) x = (x > 0.0f) ? x : x * e.act_slope;
@@ -368,9 +370,9 @@ __device__ __forceinline__ void epi_vec4(const v4i a, const v4f res, const EpiLa
     *reinterpret_cast<v2i *>(where.at(reinterpret_cast<int16_t *>(e.q))) = pk;
   }
 }
-template <class S>
-__device__ __forceinline__ void epi_vec4(const v4i a, const v4f res, const EpiLane &L, int64_t idx, const EpiDev &e) {
-  epi_vec4<S, EpiAt64>(a, res, L, EpiAt64{idx}, e);
+template <class S, class Sums>
+__device__ __forceinline__ void epi_vec4(const Sums a, const v4f res, const EpiLane &L, int64_t idx, const EpiDev &e) {
+  epi_vec4<S, EpiAt64, Sums>(a, res, L, EpiAt64{idx}, e);
 }
 
 // this lane's four channels within a wave tile of TN*32 columns starting at n_w
@@ -491,7 +493,7 @@ __device__ __forceinline__ void igemm_epilogue_dual(v16i (&acc)[TM][TN], v16i (&
     for (int it = 0; it < 32 / RPI; ++it) {
       const v4i a = *reinterpret_cast<const v4i *>(stage + (it * RPI + rsub) * EPI_STRIDE + cg * 4);
 #pragma unroll
-      for (int t = 0; t < 4; ++t) resv[it][t] = epi_dequant1(a[t], t, L_sc, sc.exp2);
+      for (int t = 0; t < 4; ++t) resv[it][t] = epi_dequant1((float)a[t], t, L_sc, sc.exp2);
     }
     // the wave's LDS operations complete in order: these stores cannot overtake the reads above
 #pragma unroll

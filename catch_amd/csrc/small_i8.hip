@@ -296,7 +296,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       es.exp2 = p.sc.exp2; es.chan_div = p.sc.chan_div; es.chan_rcp = p.sc.chan_rcp; es.bias = p.sc.bias;
       const EpiLane ls = epi_lane_finish<EpiGeneric>(s_div, s_rcp, s_bias, es);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) res[u] = epi_dequant1(a2[u], u, ls, es.exp2);
+      for (int u = 0; u < 4; ++u) res[u] = epi_dequant1((float)a2[u], u, ls, es.exp2);
     }
     if (m >= p.M || ec >= p.N) continue;
     const int64_t idx = (int64_t)m * p.N + ec;

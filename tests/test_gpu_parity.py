@@ -309,6 +309,40 @@ def test_few_output_tiles(case):
             assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
 
 
+# int16 x int16 with K split over the waves: each tile size, dense and convolution, K ending inside a step, fewer steps
+# than waves, rows and columns beyond the last full tile, taps that end inside a transfer, output rows of any alignment
+WIDE_CASES = [
+    # n, h, w, ci, co, k, pad, stride, dil
+    (1, 1, 1, 8, 1, 1, 0, 1, 1), (33, 1, 1, 64, 45, 1, 0, 1, 1), (65, 1, 1, 1000, 36, 1, 0, 1, 1),
+    (700, 1, 1, 136, 1000, 1, 0, 1, 1), (1379, 1, 1, 200, 1001, 1, 0, 1, 1), (1901, 1, 1, 72, 1000, 1, 0, 1, 1),
+    (1900, 1, 1, 128, 1003, 1, 0, 1, 1), (5, 9, 7, 8, 30, 3, 1, 1, 1), (1, 14, 14, 24, 64, 5, 2, 2, 1),
+    (2, 12, 10, 80, 40, 3, 2, 1, 2), (40, 20, 20, 16, 44, 3, 1, 1, 1), (20, 30, 30, 24, 33, 3, 1, 1, 1), (34, 30, 30, 16, 40, 3, 1, 1, 1)]
+
+
+@pytest.mark.parametrize("case", WIDE_CASES)
+def test_int16_k_split(case):
+    n, h, w, ci, co, k, pad, stride, dil = case
+    note("int16 k split", case)
+    r = rng(sum(case) * 13)
+    x, wt = _ints(r, (n, h, w, ci), 16), _ints(r, (co, k, k, ci), 16)
+    ext = np.array([-32768, 32767, -1, 0, 128, -128, 255, 256], np.int16)
+    x.reshape(-1)[:8], wt.reshape(-1)[-8:] = ext, ext
+    acc, _ = orc.conv2d_nhwc(x, wt, (pad, pad), (stride, stride), (dil, dil), 1)
+    div = r.uniform(0.6, 3.5, co).astype(np.float32)
+    bias = r.standard_normal(co).astype(np.float32)
+    res = (r.standard_normal(acc.shape) * 20).astype(np.float32)
+    args = dict(padding=(pad, pad), stride=(stride, stride), dilation=(dil, dil), exp2=-26)
+    xd, wd = cabi.dev(x), cabi.dev(wt)
+    dd, bd, rd, rcp = cabi.dev(div), cabi.dev(bias), cabi.dev(res), cabi.dev(np.float32(1) / div)
+    for y_dtype, q_bw, act, use_res in ((torch.float32, 0, 0, False), (torch.float16, 0, 0, False), (torch.float32, 8, 1, True)):
+        out = cabi.conv2d_nhwc(xd, wd, chan_div=dd, chan_rcp=rcp, bias=bd, resid=rd if use_res else None, act=act,
+                               y_dtype=y_dtype, want_acc=False, q_bw=q_bw, q_pos=-3, **args)
+        y = orc.epilogue(acc, -26, div, bias, res if use_res else None, act)
+        assert same_bits(y.astype(np.float16) if y_dtype == torch.float16 else y, out["y"].cpu().numpy())
+        if q_bw:
+            assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
+
+
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("case", [FEW_TILES_CASES[i] for i in (0, 2, 3, 5, 6, 7, 9, 10, 11, 13, 15)] + [(70, 30, 30, 32, 40, 3, 1, 1, 1)])
 def test_floating_activations_quantized_on_the_way(case, dtype):
