@@ -13,15 +13,22 @@
 //
 // The split happens in registers, between the LDS fetch and the MFMA: activations stay plain
 // int16 NHWC in memory.  A-tile rows are 128 bytes (64 int16 of K) = eight 16-byte chunks, the
-// chunk index XOR-ed with row&7; weight rows keep the 64-byte layout of the int8 kernel.  (row&7
-// leaves a two-way bank conflict on the A fetches; the conflict-free (row>>1)&7 needs a second K
-// position per lane in the loader and measured 8 % slower end to end: the loop is bound by the
-// address arithmetic and issue of the loads, not by the LDS reads.)
+// chunk index XOR-ed with a swizzle of the row; weight rows keep the 64-byte layout of the int8 kernel.
+//
+// A wave's step is eight matrix instructions (64x128 tile) and, in the general loader, about a hundred
+// vector ones: tap bookkeeping per lane, the digit split, the weight sums.  The vector ones took longer.
+// UNIFORM, wherever a K step lies within one filter tap (channels, or K of a plain GEMM, a multiple of 64):
+// tap and position along K are the same for all lanes, so a load's offset is one register that changes only
+// with the tap plus a scalar that advances along K.  A lane's chunk is then a constant as well, and the
+// conflict-free swizzle (row>>1)&7 costs nothing (row&7, which the general loader needs to have one K
+// position per lane, leaves a two-way bank conflict on the A fetches).
+// Darknet-53 with 416x416 images, batch 16: 2473 -> 2296 us with the uniform loader and the weight sums
+// shared out between the two waves of a column.
 #include "igemm_i8_dma.inc"
 
 namespace catchq {
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD, int EPI>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD, bool UNIFORM, int EPI>
 __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(const int16_t *__restrict__ A,
                                                                             const int8_t *__restrict__ B,
                                                                             IgemmParams p, EpiDev e,
@@ -85,12 +92,30 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
         rowbase[j] = (unsigned)(mm * p.K * 2);
         vmask[j] = ok ? 1u : 0u;
       }
+      if constexpr (UNIFORM) rowbase[j] += (unsigned)(((lane & 7) ^ (lane >> 4) ^ ((slot & 1) * 4)) * 16);
     } else {
       const int n = n0 + (slot - NIA) * 16 + (lane >> 2);
       const bool ok = n < p.N;
       rowbase[j] = (unsigned)((int64_t)(ok ? n : 0) * p.K);
       vmask[j] = ok ? 1u : 0u;
+      if constexpr (UNIFORM) rowbase[j] += (unsigned)(((lane & 3) ^ ((lane >> 4) & 3)) * 16);
     }
+  }
+  // UNIFORM: offsets of the current tap (OOB: the row or the tap does not exist), rebuilt when the tap changes.
+  // Operands are smaller than 2 GiB, so an OOB offset stays out of range whatever the scalar adds.
+  unsigned voff[NI];
+  int u_k = 0, u_ci = 0, u_tap = 0, u_r = 0, u_q = 0;  // wave-uniform
+  auto enter_tap = [&]() {
+    const unsigned tapoff = (LOAD == LOAD_CONV) ? 2u * (unsigned)((u_r * p.dh * p.W + u_q * p.dw) * p.Ci) : 0u;
+    const unsigned bit = (LOAD == LOAD_CONV) ? (u_r < p.kh ? 1u << u_tap : 0u) : 1u;  // past the last tap: nothing
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+      if (wave * NI + j < NIA) voff[j] = select_u32((vmask[j] & bit) != 0, rowbase[j] + tapoff, OOB);
+  };
+  if constexpr (UNIFORM) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j) voff[j] = select_u32(vmask[j] != 0, rowbase[j], OOB);
+    enter_tap();
   }
   // this lane's position along K, in elements: as a loader of A (8-element chunks) and of B (16)
   int ka_lin = ((lane & 7) ^ (lane >> 3)) * 8;
@@ -105,9 +130,33 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
       tapbase = (unsigned)((kr * p.dh * p.W + kq * p.dw) * p.Ci);
     }
   };
-  if constexpr (LOAD == LOAD_CONV) normalise_tap();
+  if constexpr (LOAD == LOAD_CONV && !UNIFORM) normalise_tap();
 
   auto issue_stage = [&](int stage_off) {
+    if constexpr (UNIFORM) {
+      const int a_soff = 2 * ((LOAD == LOAD_CONV) ? u_ci : u_k);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) {
+        const int slot = wave * NI + j;
+        lds_ptr_t dst = (lds_ptr_t)(lds_dyn + stage_off + slot * 1024);
+        if (slot < NIA) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, (int)voff[j], a_soff, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, (int)voff[j], u_k, 0, 0);
+      }
+      // past the end of K the offsets stay where they are: a slot that is filled but never read
+      if (u_k + BK < p.K) {
+        u_k += BK;
+        if constexpr (LOAD == LOAD_CONV) {
+          u_ci += BK;
+          if (u_ci == p.Ci) {
+            u_ci = 0;
+            ++u_tap;
+            if (++u_q == p.kw) { u_q = 0; ++u_r; }
+            enter_tap();
+          }
+        }
+      }
+      return;
+    }
     const bool ka_ok = ka_lin < p.K, kb_ok = kb_lin < p.K;
     const unsigned a_koff = 2u * ((LOAD == LOAD_CONV) ? tapbase + (unsigned)kci : (unsigned)ka_lin);
     const unsigned a_bit = (LOAD == LOAD_CONV) ? (1u << tap) : 1u;
@@ -147,7 +196,8 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   const int frow = lane & 31, fhalf = lane >> 5;
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t *)lds_dyn;
   // A: elements [ks*32 + fhalf*16, +16) of the step = logical chunks ks*4 + fhalf*2 and the next one
-  const unsigned a_c0 = (unsigned)(((fhalf * 2) ^ (frow & 7)) * 16);
+  const int swa = UNIFORM ? ((frow >> 1) & 7) : (frow & 7);
+  const unsigned a_c0 = (unsigned)(((fhalf * 2) ^ swa) * 16);
   const unsigned a_row = lds_base + (unsigned)((wave_m * WM + frow) * (BK * 2));
   // B: as in the int8 kernel
   const int swb = (frow >> 2) & 3;
@@ -167,11 +217,15 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
     fb[0] = ds_read_b128<0>(b_addr);
     if constexpr (TN > 1) fb[1] = ds_read_b128<2048>(b_addr);
   };
-  auto multiply_half = [&](v4i (&fa)[TM][2], v4i (&fb)[TN]) {
+  // the waves of a column of the block hold the same weights: each sums one half of every K step
+  static_assert(WAVES_M == 2, "the weight sums are shared out between two waves");
+  auto multiply_half = [&](v4i (&fa)[TM][2], v4i (&fb)[TN], int half) {
+    if (wave_m == half) {  // wave-uniform
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+      for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int d = 0; d < 4; ++d) wsum[j] = __builtin_amdgcn_sdot4(fb[j][d], 0x01010101, wsum[j], false);
+        for (int d = 0; d < 4; ++d) wsum[j] = __builtin_amdgcn_sdot4(fb[j][d], 0x01010101, wsum[j], false);
+    }
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       v4i hi, lo;
@@ -186,21 +240,22 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   static_assert(TM <= 2 && TN <= 2, "wave tile larger than 64x64");
 
   // both halves are requested up front: the second half's fragments arrive while the first half is multiplied
-  auto compute = [&](unsigned stage_off) {
+  auto compute = [&](unsigned stage_off, int refill_off) {
     constexpr int NF = 2 * TM + TN;  // LDS reads per half
     v4i fa0[TM][2], fb0[TN], fa1[TM][2], fb1[TN];
     fetch_half(fa0, fb0, a_row + stage_off, a_c0, b_row + stage_off + b_k0);
     fetch_half(fa1, fb1, a_row + stage_off, a_c0 ^ 64u, b_row + stage_off + b_k1);
+    issue_stage(refill_off);
 #pragma unroll
     for (int i = 0; i < TM; ++i) { lgkm_wait<NF>(fa0[i][0]); lgkm_wait<NF>(fa0[i][1]); }
 #pragma unroll
     for (int j = 0; j < TN; ++j) lgkm_wait<NF>(fb0[j]);
-    multiply_half(fa0, fb0);
+    multiply_half(fa0, fb0, 0);
 #pragma unroll
     for (int i = 0; i < TM; ++i) { lgkm_wait<0>(fa1[i][0]); lgkm_wait<0>(fa1[i][1]); }
 #pragma unroll
     for (int j = 0; j < TN; ++j) lgkm_wait<0>(fb1[j]);
-    multiply_half(fa1, fb1);
+    multiply_half(fa1, fb1, 1);
   };
 
   // ---- pipeline (same schedule as the int8 kernel) ---------------------------------------------------
@@ -211,19 +266,27 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   for (int step = 0; step < nsteps; ++step) {
     CATCHQ_VMCNT(NI * (STAGES - 2));
     __builtin_amdgcn_s_barrier();
-    issue_stage(wr_off);
-    compute((unsigned)rd_off);
+    compute((unsigned)rd_off, wr_off);
     rd_off = (rd_off + STAGE_BYTES == PIPE_BYTES) ? 0 : rd_off + STAGE_BYTES;
     wr_off = (wr_off + STAGE_BYTES == PIPE_BYTES) ? 0 : wr_off + STAGE_BYTES;
   }
   CATCHQ_VMCNT(0);
   __syncthreads();
 
-  // the two K halves of a column's weight sum sit in lanes l and l^32; the accumulator layout has
-  // column = lane & 31, the same as the weight fragment's row
+  // a column's weight sum: two quarters of K sit in lanes l and l^32 of this wave, two in the other wave of the
+  // column (exchanged through LDS behind the epilogue's staging area); the accumulator layout has column = lane & 31,
+  // the same as the weight fragment's row
+  static_assert(NW * 32 * EPI_STRIDE * 4 + 2 * BN * 4 <= PIPE_BYTES, "weight sums fit behind the staging area");
+  int *const sums = reinterpret_cast<int *>(lds_dyn + PIPE_BYTES) - 2 * BN + wave_n * WN + frow;
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
-    const unsigned ws = (unsigned)(wsum[j] + __shfl_xor(wsum[j], 32, 64)) << 7;
+    wsum[j] += __shfl_xor(wsum[j], 32, 64);
+    if (fhalf == 0) sums[wave_m * BN + j * 32] = wsum[j];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    const unsigned ws = (unsigned)(wsum[j] + sums[(wave_m ^ 1) * BN + j * 32]) << 7;
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -236,7 +299,7 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   igemm_epilogue<TM, TN, EPI, EPI_PASSES>(acc_lo, stage, m0 + wave_m * WM, n0 + wave_n * WN, lane, p, e);
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD, int EPI>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD, bool UNIFORM, int EPI>
 static int launch_a16_epi(const void *a, const void *b, const IgemmParams &p, const EpiDev &e, int64_t a_bytes,
                           int64_t b_bytes, hipStream_t s) {
   constexpr int NW = WAVES_M * WAVES_N;
@@ -244,7 +307,7 @@ static int launch_a16_epi(const void *a, const void *b, const IgemmParams &p, co
   constexpr int EPI_BYTES = NW * 32 * (BN / WAVES_N + 8) * 4;
   constexpr int LDS_BYTES = PIPE_BYTES > EPI_BYTES ? PIPE_BYTES : EPI_BYTES;
   static_assert(LDS_BYTES <= 160 * 1024, "tile does not fit the LDS");
-  auto kern = igemm_a16_dma_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI>;
+  auto kern = igemm_a16_dma_kernel<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI>;
   if (LDS_BYTES > 64 * 1024) {
     static std::atomic<bool> raised[64];
     if (raise_lds_limit((const void *)kern, LDS_BYTES, raised) != CATCHQ_OK) return CATCHQ_ERR_LAUNCH;
@@ -254,7 +317,7 @@ static int launch_a16_epi(const void *a, const void *b, const IgemmParams &p, co
   return launch_status();
 }
 
-template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD>
+template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD, bool UNIFORM>
 static int launch_a16(const void *a, const void *b, IgemmParams p, const EpiDev &e, int64_t a_bytes, int64_t b_bytes,
                       hipStream_t s) {
   const int64_t tiles_m = (p.M + BM - 1) / BM;
@@ -264,20 +327,20 @@ static int launch_a16(const void *a, const void *b, IgemmParams p, const EpiDev 
   p.nblocks = (int)nb;
   const int epi = pick_epilogue(p.N, e);
   if (epi == EPI_SCALAR)
-    return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI_SCALAR>(a, b, p, e, a_bytes, b_bytes, s);
+    return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_SCALAR>(a, b, p, e, a_bytes, b_bytes, s);
   if constexpr (BM == 64) {  // the tiles of the detector layers: leaky ReLU, int16 requantization
     switch (epi) {
-      case EPI_LK_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI_LK_Q16>(a, b, p, e, a_bytes, b_bytes, s);
-      case EPI_LK_Y_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI_LK_Y_Q16>(a, b, p, e, a_bytes, b_bytes, s);
-      case EPI_LK_RESA_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI_LK_RESA_Q16>(a, b, p, e, a_bytes, b_bytes, s);
-      case EPI_LK_RESA_Y_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI_LK_RESA_Y_Q16>(a, b, p, e, a_bytes, b_bytes, s);
+      case EPI_LK_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_Q16>(a, b, p, e, a_bytes, b_bytes, s);
+      case EPI_LK_Y_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_Y_Q16>(a, b, p, e, a_bytes, b_bytes, s);
+      case EPI_LK_RESA_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_RESA_Q16>(a, b, p, e, a_bytes, b_bytes, s);
+      case EPI_LK_RESA_Y_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_RESA_Y_Q16>(a, b, p, e, a_bytes, b_bytes, s);
       default: break;
     }
   }
-  return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, EPI_VECTOR>(a, b, p, e, a_bytes, b_bytes, s);
+  return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_VECTOR>(a, b, p, e, a_bytes, b_bytes, s);
 }
 
-template <int LOAD>
+template <int LOAD, bool UNIFORM>
 static int pick_a16_tile(const void *a, const void *b, const IgemmParams &p, const EpiDev &e, int64_t a_bytes,
                          int64_t b_bytes, hipStream_t s) {
   auto blocks = [&](int bm, int bn) { return ((p.M + bm - 1) / bm) * ((p.N + bn - 1) / bn); };
@@ -301,10 +364,10 @@ static int pick_a16_tile(const void *a, const void *b, const IgemmParams &p, con
     }
   }
   switch (tile) {
-    case 128256: return launch_a16<128, 256, 2, 4, 4, LOAD>(a, b, p, e, a_bytes, b_bytes, s);
-    case 128128: return launch_a16<128, 128, 2, 2, 3, LOAD>(a, b, p, e, a_bytes, b_bytes, s);
-    case 64128: return launch_a16<64, 128, 2, 2, 3, LOAD>(a, b, p, e, a_bytes, b_bytes, s);
-    default: return launch_a16<64, 64, 2, 2, 3, LOAD>(a, b, p, e, a_bytes, b_bytes, s);
+    case 128256: return launch_a16<128, 256, 2, 4, 4, LOAD, UNIFORM>(a, b, p, e, a_bytes, b_bytes, s);
+    case 128128: return launch_a16<128, 128, 2, 2, 3, LOAD, UNIFORM>(a, b, p, e, a_bytes, b_bytes, s);
+    case 64128: return launch_a16<64, 128, 2, 2, 3, LOAD, UNIFORM>(a, b, p, e, a_bytes, b_bytes, s);
+    default: return launch_a16<64, 64, 2, 2, 3, LOAD, UNIFORM>(a, b, p, e, a_bytes, b_bytes, s);
   }
 }
 
@@ -312,8 +375,14 @@ static int pick_a16_tile(const void *a, const void *b, const IgemmParams &p, con
 int igemm_a16_launch(int load, const void *a, const void *b, IgemmParams p, const EpiDev &e, int64_t a_bytes,
                      int64_t b_bytes, hipStream_t s) {
   if (a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31) || a_bytes <= 0 || b_bytes <= 0) return -1;
-  if (load == LOAD_GEMM) return pick_a16_tile<LOAD_GEMM>(a, b, p, e, a_bytes, b_bytes, s);
-  if (load == LOAD_CONV) return pick_a16_tile<LOAD_CONV>(a, b, p, e, a_bytes, b_bytes, s);
+  // a K step of 64 never crosses a filter tap: the loader without per-lane bookkeeping (see the top of the file)
+  const bool uniform = (load == LOAD_CONV ? p.Ci : p.K) % BK == 0;
+  if (load == LOAD_GEMM)
+    return uniform ? pick_a16_tile<LOAD_GEMM, true>(a, b, p, e, a_bytes, b_bytes, s)
+                   : pick_a16_tile<LOAD_GEMM, false>(a, b, p, e, a_bytes, b_bytes, s);
+  if (load == LOAD_CONV)
+    return uniform ? pick_a16_tile<LOAD_CONV, true>(a, b, p, e, a_bytes, b_bytes, s)
+                   : pick_a16_tile<LOAD_CONV, false>(a, b, p, e, a_bytes, b_bytes, s);
   return -1;
 }
 

@@ -462,6 +462,30 @@ def test_gemm_a16_tiles(m, n, k):
     assert torch.equal(hi * 256 + lo + 128 * bsum[None, :], out["acc"])
 
 
+@pytest.mark.parametrize("n,h,w,ci,co,k,stride,dil", [
+    (1, 9, 11, 64, 64, 1, 1, 1),    # a single K step
+    (1, 7, 300, 64, 20, 1, 2, 1),   # strided 1x1: taps without padding
+    (2, 13, 10, 128, 132, 3, 2, 1),  # ragged in both directions, every tap's validity mask
+    (1, 21, 17, 64, 36, 3, 1, 2),   # dilated
+    (1, 15, 40, 192, 64, 5, 1, 1),  # 25 taps of three steps each
+    (1, 15, 40, 80, 64, 5, 1, 1),   # steps that cross taps: the general loader
+    (3, 8, 9, 40, 68, 3, 1, 1),
+])
+def test_conv_a16_loaders(n, h, w, ci, co, k, stride, dil):
+    """int16 x int8: K steps inside one filter tap (ci a multiple of 64) and across taps; the sums are integers, equal to
+    the oracle's"""
+    note("a16 loaders", n, h, w, ci, co, k, stride, dil)
+    r = rng(n * 100 + h + ci + co + k)
+    x, wt = (_ints(r, (n, h, w, ci), 16) // 64).astype(np.int16), _ints(r, (co, k, k, ci), 8)
+    x[0, 0, 0, :4] = (-32768, 32767, 255, -129)
+    x[-1, -1, -1, -4:] = (128, -1, 256, 32640)
+    pad = dil * (k // 2)
+    acc, ovf = orc.conv2d_nhwc(x, wt, (pad, pad), (stride, stride), (dil, dil), 1)
+    assert ovf == 0
+    out = cabi.conv2d_nhwc(cabi.dev(x), cabi.dev(wt), (pad, pad), (stride, stride), (dil, dil), y_dtype=None)
+    assert same_bits(acc.astype(np.int32), out["acc"].cpu().numpy())
+
+
 @pytest.mark.parametrize("m,n,k", [(4997, 2100, 512), (2500, 1100, 1024), (9001, 600, 256), (6000, 4100, 128)])
 def test_gemm_banded_tile_order(m, n, k):
     """grids that are large in both directions walk their tiles in bands of eight row tiles; ragged last band,
