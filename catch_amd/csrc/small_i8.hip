@@ -456,8 +456,20 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
 
 // Activations still in floating point (NHWC), quantized at 2^position on their way into LDS: whether one launch serves
 // the shape, and that launch.
+//
+// Every block converts its rows again for every filter tap and every column of tiles, which costs a wave more than the
+// step's multiplications; a quantizer's launch costs about 1 us in front of it on the device (and 2.5 us of the host).
+// So the one launch pays while a wave has few K steps.  Measured (one launch / two, us, half activations): 32 x 32 tiles,
+// two steps a wave 5.1 / 5.7 (512 x 768 x 512) and 6.6 / 7.2 (384 x 1024 x 768), three 6.1 / 6.3 (256 x 1280 x 768), five
+// 8.6 / 7.6 (4 x 14x14 256 -> 256 3x3), nine 37.7 / 19.0 (32 x 7x7 512 -> 512 3x3); 16 x 16 tiles, three steps 5.4 / 6.0
+// (14x14 256 -> 256 3x3), four 4.6 / 5.3 (8 x 2048 x 1000), six 5.5 / 5.3 (1 x 3072 x 768), eight 9.8 / 7.0
+// (32 x 4096 x 3072), thirteen 16.2 / 9.4 (2 x 14x14 256 -> 256 5x5).  Float activations lie within 1 us of these.
 bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus) {
-  return Ci % 16 == 0 && small_plan(M, Co, K, dense, cus) != 0;
+  const int plan = small_plan(M, Co, K, dense, cus);
+  if (Ci % 16 != 0 || !plan) return false;
+  const int waves = plan % 100;
+  const int64_t per_wave = ((K + 127) / 128 + waves - 1) / waves;
+  return per_wave <= (plan / 100 == 32 ? 3 : 6);
 }
 int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
                          int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
