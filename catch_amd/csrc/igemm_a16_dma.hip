@@ -328,12 +328,13 @@ static int launch_a16(const void *a, const void *b, IgemmParams p, const EpiDev 
   const int epi = pick_epilogue(p.N, e);
   if (epi == EPI_SCALAR)
     return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_SCALAR>(a, b, p, e, a_bytes, b_bytes, s);
-  if constexpr (BM == 64) {  // the tiles of the detector layers: leaky ReLU, int16 requantization
+  if constexpr (BM == 64) {  // the tiles of the detector layers: leaky ReLU, int16 requantization; half outputs of its heads
     switch (epi) {
       case EPI_LK_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_Q16>(a, b, p, e, a_bytes, b_bytes, s);
       case EPI_LK_Y_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_Y_Q16>(a, b, p, e, a_bytes, b_bytes, s);
       case EPI_LK_RESA_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_RESA_Q16>(a, b, p, e, a_bytes, b_bytes, s);
       case EPI_LK_RESA_Y_Q16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_LK_RESA_Y_Q16>(a, b, p, e, a_bytes, b_bytes, s);
+      case EPI_Y16: return launch_a16_epi<BM, BN, WAVES_M, WAVES_N, STAGES, LOAD, UNIFORM, EPI_Y16>(a, b, p, e, a_bytes, b_bytes, s);
       default: break;
     }
   }

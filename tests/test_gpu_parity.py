@@ -484,6 +484,10 @@ def test_conv_a16_loaders(n, h, w, ci, co, k, stride, dil):
     assert ovf == 0
     out = cabi.conv2d_nhwc(cabi.dev(x), cabi.dev(wt), (pad, pad), (stride, stride), (dil, dil), y_dtype=None)
     assert same_bits(acc.astype(np.int32), out["acc"].cpu().numpy())
+    bias = r.standard_normal(co).astype(np.float32)  # half outputs of a detector's heads: an epilogue instance of its own
+    out = cabi.conv2d_nhwc(cabi.dev(x), cabi.dev(wt), (pad, pad), (stride, stride), (dil, dil), exp2=-20, bias=cabi.dev(bias),
+                           y_dtype=torch.float16, want_acc=False)
+    assert same_bits(orc.epilogue(acc, -20, None, bias).astype(np.float16), out["y"].cpu().numpy())
 
 
 @pytest.mark.parametrize("m,n,k", [(4997, 2100, 512), (2500, 1100, 1024), (9001, 600, 256), (6000, 4100, 128)])
