@@ -27,6 +27,8 @@ int conv2d_dual_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
 int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                            int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws,
                            int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
+bool gemm_float_ok(int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
+int gemm_float(const void *x, bool half, int position, const void *w, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s);
 bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus);
 int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
                          int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
@@ -300,11 +302,15 @@ CATCHQ_API int catchq_conv2d_shortcut_nhwc(const void *x, int x_bits, const void
   return catchq_conv2d_nhwc(x, x_bits, w, w_bits, desc, &em, stream);
 }
 
-// shapes that quantize and contract in one launch (pointer alignment is checked at the call)
-static bool float_conv_fusable(const catchq_conv_desc_t *d, int ho, int wo, const catchq_epilogue_t *e) {
+// shapes that quantize and contract in one launch (pointer alignment is checked at the call): 1 few-tiles kernel, 2 GEMM of
+// few columns, 0 neither
+static int float_conv_fusable(const catchq_conv_desc_t *d, int x_dtype, int ho, int wo, const catchq_epilogue_t *e) {
   const bool dense = d->kh == 1 && d->kw == 1 && d->stride_h == 1 && d->stride_w == 1 && d->pad_h == 0 && d->pad_w == 0;
-  return d->groups == 1 && contract_small_float_ok((int64_t)d->n * ho * wo, d->co, (int64_t)d->kh * d->kw * d->ci, dense, d->ci,
-                                                   planned_cus(e->sharing));
+  const int64_t M = (int64_t)d->n * ho * wo;
+  const int cus = planned_cus(e->sharing);
+  if (d->groups != 1) return 0;
+  if (contract_small_float_ok(M, d->co, (int64_t)d->kh * d->kw * d->ci, dense, d->ci, cus)) return 1;
+  return dense && gemm_float_ok(M, d->co, d->ci, x_dtype == CATCHQ_F16 ? 2 : 4, cus) ? 2 : 0;
 }
 
 CATCHQ_API int catchq_float_conv2d_workspace_size(int x_dtype, const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue,
@@ -314,7 +320,7 @@ CATCHQ_API int catchq_float_conv2d_workspace_size(int x_dtype, const catchq_conv
   if (st != CATCHQ_OK) return st;
   if (!bytes || !epilogue) return CATCHQ_ERR_ARG;
   if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
-  *bytes = float_conv_fusable(desc, ho, wo, epilogue) ? 0 : (size_t)desc->n * desc->h * desc->w * desc->ci;
+  *bytes = float_conv_fusable(desc, x_dtype, ho, wo, epilogue) ? 0 : (size_t)desc->n * desc->h * desc->w * desc->ci;
   return CATCHQ_OK;
 }
 
@@ -331,8 +337,11 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
   if (desc->n == 0) return CATCHQ_OK;
   if (!x || !w) return CATCHQ_ERR_ARG;
   const catchq_conv_desc_t &d = *desc;
-  if (float_conv_fusable(desc, ho, wo, epilogue) && aligned16(x) && aligned16(w)) {
-    const EpiDev e = make_epi(epilogue, (int64_t)d.n * ho * wo * d.co);
+  const int fusable = float_conv_fusable(desc, x_dtype, ho, wo, epilogue);
+  if (fusable && aligned16(x) && aligned16(w)) {
+    const int64_t M = (int64_t)d.n * ho * wo;
+    const EpiDev e = make_epi(epilogue, M * d.co);
+    if (fusable == 2) return gemm_float(x, x_dtype == CATCHQ_F16, x_position, w, M, d.co, d.ci, e, as_stream(stream));
     const int st2 = contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
                                          d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
     if (st2 >= 0) return st2;

@@ -560,6 +560,33 @@ __device__ __forceinline__ void split_i16(const v4i c0, const v4i c1, v4i &hi, v
   lo[3] = (int)(__builtin_amdgcn_perm((unsigned)c1[3], (unsigned)c1[2], 0x06040200u) ^ 0x80808080u);
 }
 
+// type of the activations a contraction reads: int8, or floats that its loader quantizes
+enum { IN_I8 = 0, IN_F32 = 1, IN_F16 = 2 };
+
+// 16 floats (or halfs) -> 16 int8, the quantizer's own arithmetic with unit scale
+template <int IN>
+__device__ __forceinline__ v4i quantize16(const v4i *raw, int neg_pos) {
+  v4i q;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    int b[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      float v;
+      if constexpr (IN == IN_F32) v = __int_as_float(raw[d][t]);
+      else {
+        const int pair = raw[d >> 1][(d & 1) * 2 + (t >> 1)];
+        v = (float)__builtin_bit_cast(_Float16, (short)((t & 1) ? pair >> 16 : pair & 0xffff));
+      }
+      b[t] = quant1_unit<8>(v, neg_pos);
+    }
+    const unsigned lo = __builtin_amdgcn_perm((unsigned)b[1], (unsigned)b[0], 0x0c0c0400u);
+    const unsigned hi = __builtin_amdgcn_perm((unsigned)b[3], (unsigned)b[2], 0x04000c0cu);
+    q[d] = (int)(lo | hi);
+  }
+  return q;
+}
+
 // launchers of the LDS-DMA pipelined kernel (igemm_i8_dma.hip); return -1 when the shape is not
 // eligible (operand of 2 GiB or more, four-channel stem) and the caller takes the register-staged kernel
 int igemm_dma_launch(int load, const void *a, const void *b, IgemmParams p, const EpiDev &e, int64_t a_bytes,

@@ -40,8 +40,6 @@ struct SmallParams {
   ShortcutDev sc;
 };
 
-enum { SMALL_I8 = 0, SMALL_F32 = 1, SMALL_F16 = 2 };
-
 #define CATCHQ_SMALL_VMCNT(n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(n) : "memory")
 
 // n / d for n * d < 2^32 through magic = ceil(2^32 / d) (d = 1: magic 0, mask ~0)
@@ -54,30 +52,6 @@ __device__ __forceinline__ v4i small_ds_read(unsigned addr) {
 }
 __device__ __forceinline__ void small_ds_write(unsigned addr, v4i v) {
   asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory");
-}
-
-// 16 floats (or halfs) -> 16 int8, the quantizer's own arithmetic with unit scale
-template <int IN>
-__device__ __forceinline__ v4i small_quantize(const v4i *raw, int neg_pos) {
-  v4i q;
-#pragma unroll
-  for (int d = 0; d < 4; ++d) {
-    int b[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float v;
-      if constexpr (IN == SMALL_F32) v = __int_as_float(raw[d][t]);
-      else {
-        const int pair = raw[d >> 1][(d & 1) * 2 + (t >> 1)];
-        v = (float)__builtin_bit_cast(_Float16, (short)((t & 1) ? pair >> 16 : pair & 0xffff));
-      }
-      b[t] = quant1_unit<8>(v, neg_pos);
-    }
-    const unsigned lo = __builtin_amdgcn_perm((unsigned)b[1], (unsigned)b[0], 0x0c0c0400u);
-    const unsigned hi = __builtin_amdgcn_perm((unsigned)b[3], (unsigned)b[2], 0x04000c0cu);
-    q[d] = (int)(lo | hi);
-  }
-  return q;
 }
 
 // DENSE: a plain GEMM -- row m starts at m * K, no taps.  IN: type of the activations.  DUAL: a residual block's last
@@ -167,7 +141,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   const int mine = per + (group_wave < rem ? 1 : 0);
   int8_t *const my = lds + wave * WAVE_BYTES;
 
-  constexpr int ES = IN == SMALL_F32 ? 4 : (IN == SMALL_F16 ? 2 : 1);  // bytes per activation
+  constexpr int ES = IN == IN_F32 ? 4 : (IN == IN_F16 ? 2 : 1);  // bytes per activation
   constexpr int RAW = ES;  // 16-byte loads per 16 activations
   v4i raw[NA][RAW];
   (void)raw;
@@ -207,7 +181,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       if constexpr (DENSE) in = in & (a_base[j] != OOB);
       unsigned voff = in ? (a_base[j] + koff[h]) * (unsigned)ES : OOB;
       asm volatile("" : "+v"(voff));
-      if constexpr (IN == SMALL_I8) {
+      if constexpr (IN == IN_I8) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
       } else {
 #pragma unroll
@@ -226,16 +200,16 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     const unsigned a_addr = my_addr + (unsigned)(frow * BKB);
     const unsigned sw = (unsigned)((frow >> 1) & 7);
     issue(0);
-    if constexpr (IN == SMALL_I8) issue(1);  // (past the slice: nothing but zeros, so that the number in flight stays the same)
+    if constexpr (IN == IN_I8) issue(1);  // (past the slice: nothing but zeros, so that the number in flight stays the same)
     for (int s = 0; s < mine; ++s) {
-      if constexpr (IN == SMALL_I8) {
+      if constexpr (IN == IN_I8) {
         CATCHQ_SMALL_VMCNT(NI);
       } else {
         // the step's activations have arrived, and with them its filters: quantized into the slot, as a transfer
         // would have left them; then the next step's loads
         v4i q[NA];
 #pragma unroll
-        for (int j = 0; j < NA; ++j) q[j] = small_quantize<IN>(raw[j], p.x_neg_pos);
+        for (int j = 0; j < NA; ++j) q[j] = quantize16<IN>(raw[j], p.x_neg_pos);
 #pragma unroll
         for (int j = 0; j < NA; ++j)
           small_ds_write(my_addr + (unsigned)((s & 1) * SLOT_BYTES + j * 1024 + lane * 16), q[j]);
@@ -252,7 +226,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       }
 #pragma unroll
       for (int u = 0; u < SUB; ++u) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[u]), "+v"(fb[u])::"memory");
-      if constexpr (IN == SMALL_I8) issue(s + 2);  // the slot has been read
+      if constexpr (IN == IN_I8) issue(s + 2);  // the slot has been read
       // operands swapped (weights as A): a lane ends up with four consecutive channels of one pixel
 #pragma unroll
       for (int u = 0; u < SUB; ++u) {
@@ -430,7 +404,7 @@ int contract_small_i8(const void *x, const void *w, int N_img, int H, int W, int
   SmallParams p = {};
   if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense)) return -1;
   small_common(&p, M, Co, Ho, Wo, e);
-  return dense ? launch_small_plan<true, SMALL_I8, false>(plan, p, e, s) : launch_small_plan<false, SMALL_I8, false>(plan, p, e, s);
+  return dense ? launch_small_plan<true, IN_I8, false>(plan, p, e, s) : launch_small_plan<false, IN_I8, false>(plan, p, e, s);
 }
 
 // A residual block's last convolution with its 1x1 projection shortcut (arguments as conv2d_dual_i8).  -1: not one.
@@ -451,7 +425,7 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
   probe.resid = reinterpret_cast<const float *>(e.y ? e.y : e.q);  // any 16-byte aligned non-null pointer
   small_common(&p, M, Co, Ho, Wo, probe);
   p.sc = sc;
-  return launch_small_plan<false, SMALL_I8, true>(plan, p, e, s);
+  return launch_small_plan<false, IN_I8, true>(plan, p, e, s);
 }
 
 // Activations still in floating point (NHWC), quantized at 2^position on their way into LDS: whether one launch serves
@@ -481,8 +455,8 @@ int contract_small_float(const void *x, bool half, int position, const void *w, 
   if (!small_side(&p.side[0], x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense)) return -1;
   small_common(&p, M, Co, Ho, Wo, e);
   p.x_neg_pos = -position;
-  if (half) return dense ? launch_small_plan<true, SMALL_F16, false>(plan, p, e, s) : launch_small_plan<false, SMALL_F16, false>(plan, p, e, s);
-  return dense ? launch_small_plan<true, SMALL_F32, false>(plan, p, e, s) : launch_small_plan<false, SMALL_F32, false>(plan, p, e, s);
+  if (half) return dense ? launch_small_plan<true, IN_F16, false>(plan, p, e, s) : launch_small_plan<false, IN_F16, false>(plan, p, e, s);
+  return dense ? launch_small_plan<true, IN_F32, false>(plan, p, e, s) : launch_small_plan<false, IN_F32, false>(plan, p, e, s);
 }
 
 }  // namespace catchq

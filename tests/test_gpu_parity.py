@@ -367,6 +367,40 @@ def test_floating_activations_quantized_on_the_way(case, dtype):
     assert same_bits(y, out["y"].cpu().numpy()) and same_bits(orc.quantize(y, 8, -3), out["q"].cpu().numpy())
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("m,k,n", [
+    (4097, 64, 64),     # a single step, one row in the last tile
+    (4100, 16, 60),     # K shorter than a step
+    (8200, 80, 36),     # the second step a quarter full
+    (12225, 272, 64),   # five steps: odd, the last one short
+    (4200, 128, 61),    # epilogue without vectors
+    (12289, 512, 128),
+    (8300, 208, 100),   # ragged columns of the wide tile
+])
+def test_floating_activations_few_columns(m, k, n, dtype):
+    """pointwise convolutions of few output channels: quantization and product in one launch, bit-exact against quantize +
+    integer product + epilogue; ties, NaN, values beyond the range and infinities among the activations"""
+    note("floating activations, few columns", m, k, n, dtype)
+    r = rng(m + k + n)
+    x = (r.standard_normal((1, m, 1, k)) * 2).astype(dtype)
+    x.reshape(-1)[:16] = [0.5, 1.5, -0.5, -1.5, 2.5, np.inf, -np.inf, np.nan, 1e4, -1e4, 0.03125, -0.03125, 0.046875, 0.0, -0.0, 4.0]
+    x.reshape(-1)[-4:] = [1.0, -1.0, 0.015625, 3.0]
+    wt = _ints(r, (n, 1, 1, k), 8)
+    div, bias = r.uniform(0.6, 3.5, n).astype(np.float32), r.standard_normal(n).astype(np.float32)
+    acc, ovf = orc.conv2d_nhwc(orc.quantize(x, 8, -5), wt, (0, 0), (1, 1), (1, 1), 1)
+    assert ovf == 0
+    y = orc.epilogue(acc, -10, div, bias)
+    for y_dtype in (torch.float32, torch.float16):
+        out, ws = cabi.float_conv2d_nhwc(cabi.dev(x), -5, cabi.dev(wt), exp2=-10, chan_div=cabi.dev(div),
+                                         chan_rcp=cabi.dev(np.float32(1) / div), bias=cabi.dev(bias), y_dtype=y_dtype)
+        assert ws == 0
+        assert same_bits(y if y_dtype == torch.float32 else y.astype(np.float16), out["y"].cpu().numpy())
+    out, _ = cabi.float_conv2d_nhwc(cabi.dev(x), -5, cabi.dev(wt), exp2=-10, chan_div=cabi.dev(div), bias=cabi.dev(bias), act=1,
+                                    q_bw=8, q_pos=-3)
+    y = orc.epilogue(acc, -10, div, bias, None, 1)
+    assert same_bits(y, out["y"].cpu().numpy()) and same_bits(orc.quantize(y, 8, -3), out["q"].cpu().numpy())
+
+
 def test_division_by_reciprocal_is_exact():
     """v/d evaluated as q=v*r, e=fma(-q,d,v), fma(e,r,q) with r = RN(1/d) must equal IEEE division bit
     for bit: adversarial divisor significands x a wide set of dividends x several exponents."""
