@@ -27,8 +27,9 @@ int conv2d_dual_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
 int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                            int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws,
                            int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
-bool gemm_float_ok(int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
-int gemm_float(const void *x, bool half, int position, const void *w, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s);
+bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
+int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
+               int Wo, const EpiDev &e, hipStream_t s);
 bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus);
 int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
                          int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
@@ -310,7 +311,8 @@ static int float_conv_fusable(const catchq_conv_desc_t *d, int x_dtype, int ho, 
   const int cus = planned_cus(e->sharing);
   if (d->groups != 1) return 0;
   if (contract_small_float_ok(M, d->co, (int64_t)d->kh * d->kw * d->ci, dense, d->ci, cus)) return 1;
-  return dense && gemm_float_ok(M, d->co, d->ci, x_dtype == CATCHQ_F16 ? 2 : 4, cus) ? 2 : 0;
+  const bool pointwise = d->kh == 1 && d->kw == 1 && d->pad_h == 0 && d->pad_w == 0;
+  return pointwise && gemm_float_ok((int64_t)d->n * d->h * d->w, M, d->co, d->ci, x_dtype == CATCHQ_F16 ? 2 : 4, cus) ? 2 : 0;
 }
 
 CATCHQ_API int catchq_float_conv2d_workspace_size(int x_dtype, const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue,
@@ -341,7 +343,9 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
   if (fusable && aligned16(x) && aligned16(w)) {
     const int64_t M = (int64_t)d.n * ho * wo;
     const EpiDev e = make_epi(epilogue, M * d.co);
-    if (fusable == 2) return gemm_float(x, x_dtype == CATCHQ_F16, x_position, w, M, d.co, d.ci, e, as_stream(stream));
+    if (fusable == 2)
+      return gemm_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.stride_h, d.stride_w, ho, wo, e,
+                        as_stream(stream));
     const int st2 = contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
                                          d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
     if (st2 >= 0) return st2;

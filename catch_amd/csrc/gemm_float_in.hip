@@ -37,7 +37,13 @@ __global__ __launch_bounds__(256) void gemm_float_kernel(const void *__restrict_
   // ---- loader: activations, 16 of row threadIdx / 4 per lane; filters, rows of 64 bytes as in the int8 kernel ---------
   const int arow = threadIdx.x >> 2, achunk = threadIdx.x & 3;
   const bool a_ok = m0 + arow < p.M;
-  const unsigned a_row = a_ok ? (unsigned)((m0 + arow) * p.K) : 0u;  // elements
+  unsigned a_pix = a_ok ? (unsigned)(m0 + arow) : 0u;
+  if (p.sh * p.sw != 1) {  // strided: output pixel -> input pixel (fewer than 2^31 pixels: 32-bit divisions)
+    const unsigned t = a_pix / (unsigned)p.Wo, wo = a_pix - t * (unsigned)p.Wo;
+    const unsigned img = t / (unsigned)p.Ho, ho = t - img * (unsigned)p.Ho;
+    a_pix = (img * (unsigned)p.H + ho * (unsigned)p.sh) * (unsigned)p.W + wo * (unsigned)p.sw;
+  }
+  const unsigned a_row = a_pix * (unsigned)p.K;  // elements
   int ak = achunk * 16;
   unsigned b_off[NB];
   const int bchunk = (lane & 3) ^ ((lane >> 4) & 3);
@@ -154,19 +160,25 @@ static int launch_gemm_float(const void *a, const void *b, IgemmParams p, const 
 // More columns convert every activation more often: 6272 x 256 -> 1024 ties.  Few blocks are a serial chain of steps that
 // nothing covers: 1568 x 2048 -> 512 16.0 / 14.4, 2048 x 1024 -> 512 9.9 / 9.6 (11.7 / 9.8), 3136 x 512 -> 128 6.5 / 7.0
 // (7.4 / 7.1), 4096 x 3072 -> 128 22.3 / 21.1 (33.1 / 22.7).
-bool gemm_float_ok(int64_t M, int64_t N, int64_t K, int elem_bytes, int cus) {
-  if (K % 16 != 0 || M >= (1ll << 31) - 64 || M * K * elem_bytes >= (1ll << 31) || N * K >= (1ll << 31)) return false;
-  if (N > 512 || M < 1024 || K > 1024) return false;
+// A strided layer leaves most of the pixels unread that a quantizer converts, so it takes more columns: stride 2 on
+// 32 images, 56x56 256 -> 512 17.7 / 31.3 (21.4 / 39.1), 28x28 512 -> 1024 15.3 / 20.9 (19.2 / 26.4), 14x14 1024 -> 2048
+// 15.3 / 16.6 (17.0 / 19.1), 56x56 64 -> 128 5.1 / 10.1 (6.1 / 13.1).
+// in_pixels: pixels of the input, M of the output.
+bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus) {
+  if (K % 16 != 0 || M >= (1ll << 31) - 64 || in_pixels * K * elem_bytes >= (1ll << 31) || N * K >= (1ll << 31)) return false;
+  if (N > (in_pixels > M ? 2048 : 512) || M < 1024 || K > 1024) return false;
   const int64_t blocks = (M + 63) / 64 * (N <= 64 ? 1 : (N + 127) / 128);
   return blocks * 4 >= 3 * cus || K <= (elem_bytes == 2 ? 512 : 256);
 }
 
-int gemm_float(const void *x, bool half, int position, const void *w, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s) {
+int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
+               int Wo, const EpiDev &e, hipStream_t s) {
   IgemmParams p = {};
-  p.M = M;
-  p.N = (int)N;
-  p.K = (int)K;
-  const int64_t a_bytes = M * K * (half ? 2 : 4), b_bytes = N * K;
+  p.M = (int64_t)N_img * Ho * Wo;
+  p.N = Co;
+  p.K = Ci;
+  p.H = H; p.W = W; p.Ho = Ho; p.Wo = Wo; p.sh = sh; p.sw = sw;
+  const int64_t N = Co, a_bytes = (int64_t)N_img * H * W * Ci * (half ? 2 : 4), b_bytes = N * Ci;
   if (N <= 64) {
     return half ? launch_gemm_float<IN_F16, 64>(x, w, p, e, -position, a_bytes, b_bytes, s)
                 : launch_gemm_float<IN_F32, 64>(x, w, p, e, -position, a_bytes, b_bytes, s);

@@ -401,6 +401,21 @@ def test_floating_activations_few_columns(m, k, n, dtype):
     assert same_bits(y, out["y"].cpu().numpy()) and same_bits(orc.quantize(y, 8, -3), out["q"].cpu().numpy())
 
 
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("n,h,w,ci,co,stride", [(3, 41, 37, 64, 48, (2, 2)), (2, 60, 50, 80, 200, (2, 1)), (5, 64, 47, 32, 132, (1, 3))])
+def test_floating_activations_strided_pointwise(n, h, w, ci, co, stride, dtype):
+    """strided 1x1 convolutions read the pixels they use and nothing else: bit-exact against quantize + product + epilogue"""
+    note("floating activations, strided", n, h, w, ci, co, stride, dtype)
+    r = rng(n + h + w + ci + co)
+    x, wt = (r.standard_normal((n, h, w, ci)) * 2).astype(dtype), _ints(r, (co, 1, 1, ci), 8)
+    div, bias = r.uniform(0.6, 3.5, co).astype(np.float32), r.standard_normal(co).astype(np.float32)
+    acc, ovf = orc.conv2d_nhwc(orc.quantize(x, 8, -5), wt, (0, 0), stride, (1, 1), 1)
+    assert ovf == 0
+    out, ws = cabi.float_conv2d_nhwc(cabi.dev(x), -5, cabi.dev(wt), stride=stride, exp2=-10, chan_div=cabi.dev(div),
+                                     chan_rcp=cabi.dev(np.float32(1) / div), bias=cabi.dev(bias))
+    assert ws == 0 and same_bits(orc.epilogue(acc, -10, div, bias), out["y"].cpu().numpy())
+
+
 def test_division_by_reciprocal_is_exact():
     """v/d evaluated as q=v*r, e=fma(-q,d,v), fma(e,r,q) with r = RN(1/d) must equal IEEE division bit
     for bit: adversarial divisor significands x a wide set of dividends x several exponents."""
