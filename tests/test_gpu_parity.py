@@ -539,7 +539,8 @@ def test_conv_a16_loaders(n, h, w, ci, co, k, stride, dil):
     assert same_bits(orc.epilogue(acc, -20, None, bias).astype(np.float16), out["y"].cpu().numpy())
 
 
-@pytest.mark.parametrize("m,n,k", [(4997, 2100, 512), (2500, 1100, 1024), (9001, 600, 256), (6000, 4100, 128)])
+@pytest.mark.parametrize("m,n,k", [(4997, 2100, 512), (2500, 1100, 1024), (9001, 600, 256), (6000, 4100, 128),
+                                   (3497, 3996, 896), (4097, 4100, 768), (8190, 1030, 1024)])
 def test_gemm_banded_tile_order(m, n, k):
     """grids that are large in both directions walk their tiles in bands of eight row tiles; ragged last band,
     ragged last row and column tiles: rows sampled from every band against the oracle, and every row of C
