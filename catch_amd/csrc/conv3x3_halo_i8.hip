@@ -28,6 +28,13 @@ int conv2d_halo_i8(const void *x, const void *w, int N, int Hi, int Wi, int Ci, 
   }
 }
 
+// Whether a stride-1 layer runs here as a single round of blocks
+bool conv2d_halo_one_round(int N, int H, int W, int Ci, int Co, int cus) {
+  HaloParams hp;
+  int tn, lds_bytes, waves;
+  return halo_plan(N, H, W, Ci, Co, 1, hp, tn, lds_bytes, waves, 0, 1, cus) && hp.nblocks <= cus;
+}
+
 // The head's shapes: 1x1 convolution K1 -> 64 channels (+ ReLU, int8 requantization with unit scale) feeding a 3x3
 // layer 64 -> 64, stride 1, padding 1, whose tiles are bands of rows; K1 in {64, 256}.
 bool conv2d_head_halo_i8_ok(int N, int H, int W, int K1, int Cm, int Co) {

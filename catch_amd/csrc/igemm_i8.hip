@@ -306,6 +306,8 @@ static bool halo_enabled() {
 int conv2d_halo_i8(const void *x, const void *w, int N, int Hi, int Wi, int Ci, int Co, int stride, const EpiDev &e,
                    hipStream_t s);
 
+bool conv2d_halo_one_round(int N, int H, int W, int Ci, int Co, int cus);
+
 int gemm_nt_stream_i8(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s);
 int conv2d_stem_i8(const void *x, const void *w, int N, int H, int W, int Co, int kh, int kw, int sh, int sw, int dh,
                    int Ho, int Wo, const EpiDev &e, hipStream_t s);
@@ -362,7 +364,13 @@ int conv2d_mfma_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
   p.N = Co;
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo;
   p.kh = kh; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
-  if (Ci % 16 == 0) {  // few output tiles
+  // Beyond two 32x32 tiles per unit the patch-resident kernel is faster than the few-tiles one while it makes a single round
+  // of blocks: 7x7 512 -> 512 3x3, 24 images (592 tiles) 11.3 / 14.0 us, 32 images 11.7 / 16.3; 20 images (496 tiles)
+  // 11.3 / 9.6, 36 images (a second round) 20.9 / 16.5, stride 2 17.6 / 16.3
+  const bool halo_first = kh == 3 && kw == 3 && sh == 1 && sw == 1 && ph == 1 && pw == 1 && dh == 1 && dw == 1 &&
+                          dma_enabled() && halo_enabled() && ((p.M + 31) / 32) * ((Co + 31) / 32) > 2 * e.cus &&
+                          conv2d_halo_one_round(N, H, W, Ci, Co, e.cus);
+  if (Ci % 16 == 0 && !halo_first) {  // few output tiles
     const int st = contract_small_i8(x, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, e, s);
     if (st >= 0) return st;
   }

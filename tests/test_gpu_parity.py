@@ -276,7 +276,8 @@ FEW_TILES_CASES = [
     (300, 1, 1, 3088, 1100, 1, 0, 1, 1), (1, 7, 7, 512, 512, 3, 1, 1, 1), (1, 14, 14, 512, 500, 3, 1, 2, 1),
     (3, 9, 5, 16, 30, 3, 1, 1, 1), (2, 13, 11, 48, 66, 5, 2, 2, 1), (2, 12, 10, 80, 40, 3, 2, 1, 2),
     (4, 14, 14, 256, 256, 3, 1, 1, 1), (4, 28, 28, 128, 128, 3, 1, 1, 1), (2, 14, 14, 512, 320, 3, 1, 1, 1),
-    (1, 14, 14, 96, 200, 1, 0, 2, 1), (2, 20, 20, 64, 48, 7, 0, 1, 1)]
+    (1, 14, 14, 96, 200, 1, 0, 2, 1), (2, 20, 20, 64, 48, 7, 0, 1, 1),
+    (21, 7, 7, 512, 512, 3, 1, 1, 1)]  # the last: beyond two tiles per unit, where the patch-resident kernel is first
 
 
 @pytest.mark.parametrize("case", FEW_TILES_CASES)
