@@ -682,3 +682,23 @@ def test_half_q_scale_that_half_cannot_hold_is_refused():
     ref = oops.conv2d(x.cpu().numpy(), w2.float().cpu().numpy(), b.float().cpu().numpy(), (1, 1), (1, 1), (1, 1), 1,
                       s2.float().cpu().numpy(), [4])
     assert same_bits(ref["y"], got.cpu().numpy())
+
+
+@pytest.mark.parametrize("xs,ws,stride,groups", [((2, 64, 14, 14), (128, 16, 3, 3), 1, 4), ((1, 96, 9, 11), (96, 48, 1, 1), 1, 2),
+                                                 ((3, 64, 15, 8), (32, 32, 3, 3), 2, 2)])
+def test_grouped_half_per_channel_convolution(xs, ws, stride, groups):
+    """all-half per-channel convolution in groups: every group divides by its own channels' scales, as half tensor ops
+    leave it"""
+    note("grouped half per-channel", xs, ws, groups)
+    g = torch.Generator().manual_seed(sum(xs) + sum(ws))
+    x = torch.randn(xs, generator=g).half()
+    w = (torch.randn(ws, generator=g) * (0.05 + 0.4 * torch.rand(ws[0], 1, 1, 1, generator=g))).half()  # scales differ widely
+    b = torch.randn(ws[0], generator=g).half()
+    s_w = 127.0 / w.float().reshape(ws[0], -1).abs().amax(1)
+    scale = torch.cat([(127.0 / x.float().abs().max()).reshape(1), torch.zeros(1), s_w]).half()
+    mode = torch.tensor([3], dtype=torch.int32)
+    args = ([ws[-1] // 2] * 2, [stride] * 2, [1, 1], groups)
+    want = ref_order.conv2d_per_channel(x, w, b, *args, scale, mode.numpy())["y"]
+    xd = x.cuda().contiguous(memory_format=torch.channels_last)
+    got = torch.ops.torch_mlu.conv2d(xd, w.cuda(), b.cuda(), *args, scale.cuda(), mode.cuda())
+    assert same_bits(want.contiguous().numpy(), got.cpu().contiguous().numpy())
