@@ -154,7 +154,7 @@ CATCHQ_API int catchq_gemm_nt(const void *a, int a_bits, const void *b, int b_bi
                               int64_t k, const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
   if (m < 0 || n < 0 || k < 0) return CATCHQ_ERR_SHAPE;
   if ((a_bits != 8 && a_bits != 16) || (b_bits != 8 && b_bits != 16)) return CATCHQ_ERR_BITWIDTH;
-  int st = check_epi(epilogue);
+  int st = check_epi(epilogue, true);
   if (st != CATCHQ_OK) return st;
   if (m == 0 || n == 0) return CATCHQ_OK;
   if (k > 0 && (!a || !b)) return CATCHQ_ERR_ARG;
@@ -180,7 +180,7 @@ CATCHQ_API int catchq_conv2d_nhwc(const void *x, int x_bits, const void *w, int 
   int st = check_conv(desc, &ho, &wo);
   if (st != CATCHQ_OK) return st;
   if ((x_bits != 8 && x_bits != 16) || (w_bits != 8 && w_bits != 16)) return CATCHQ_ERR_BITWIDTH;
-  st = check_epi(epilogue);
+  st = check_epi(epilogue, true);
   if (st != CATCHQ_OK) return st;
   if (desc->n == 0) return CATCHQ_OK;
   if (!x || !w) return CATCHQ_ERR_ARG;
@@ -333,7 +333,7 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
   int st = check_conv(desc, &ho, &wo);
   if (st != CATCHQ_OK) return st;
   if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
-  st = check_epi(epilogue);
+  st = check_epi(epilogue, true);
   if (st != CATCHQ_OK) return st;
   if (x_position < -126 || x_position > 126) return CATCHQ_ERR_ARG;
   if (desc->n == 0) return CATCHQ_OK;
@@ -649,6 +649,7 @@ CATCHQ_API int catchq_first_layers_nchw(const float *x, int n, int c, int h, int
 static int check_conv_avgpool(int n, int hw, int ci, int co, const catchq_epilogue_t *e) {
   if (n < 0 || hw <= 0 || ci <= 0 || co <= 0) return CATCHQ_ERR_SHAPE;
   if (!e || e->y || e->q || e->acc_out || (e->resid && e->resid_after_act)) return CATCHQ_ERR_ARG;  // the output is not stored
+  if (e->bias && e->bias_dtype != CATCHQ_F32) return CATCHQ_ERR_DTYPE;
   if (e->act < CATCHQ_ACT_NONE || e->act > CATCHQ_ACT_LEAKY || e->exp2 < -126 || e->exp2 > 126 || e->sharing < 0)
     return CATCHQ_ERR_ARG;
   return CATCHQ_OK;

@@ -120,6 +120,7 @@ struct EpiDev {
   const float *chan_div;
   const float *chan_rcp;  // only set when the fused reciprocal form may be used
   const float *bias;
+  const __half *bias16;  // a bias in half precision: set instead of `bias`
   const float *resid;
   int act;
   void *y;
@@ -181,7 +182,8 @@ inline EpiDev make_epi(const catchq_epilogue_t *e, int64_t out_elems = 0) {
   // (the reciprocal form folds the power of two into the division: not with a rounding between the two)
   d.chan_rcp = (e->chan_div && e->chan_rcp && !dev_exp && !d.half_steps && e->exp2 >= -64 && e->exp2 <= 64) ? e->chan_rcp : nullptr;
   d.half_rcp = (d.half_steps && e->chan_div && !dev_exp) ? e->chan_rcp : nullptr;
-  d.bias = e->bias;
+  d.bias = e->bias_dtype == CATCHQ_F16 ? nullptr : e->bias;
+  d.bias16 = e->bias_dtype == CATCHQ_F16 ? reinterpret_cast<const __half *>(e->bias) : nullptr;
   d.resid = e->resid;
   d.act = e->act;
   d.y = e->y;
@@ -198,8 +200,10 @@ inline EpiDev make_epi(const catchq_epilogue_t *e, int64_t out_elems = 0) {
   return d;
 }
 
-inline int check_epi(const catchq_epilogue_t *e) {
+// half_bias: the caller's kernels read a bias in half precision
+inline int check_epi(const catchq_epilogue_t *e, bool half_bias = false) {
   if (!e) return CATCHQ_ERR_ARG;
+  if (e->bias && e->bias_dtype != CATCHQ_F32 && !(half_bias && e->bias_dtype == CATCHQ_F16)) return CATCHQ_ERR_DTYPE;
   if (!e->y && !e->acc_out && !e->q) return CATCHQ_ERR_ARG;
   if (e->y && e->y_dtype != CATCHQ_F32 && e->y_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
   if (e->q && e->q_bitwidth != 8 && e->q_bitwidth != 16) return CATCHQ_ERR_BITWIDTH;
@@ -231,8 +235,8 @@ __device__ __forceinline__ float epi_value(float facc, int64_t idx, int c, const
     v = v / e.chan_div[c];
     if (e.half_steps) v = round_f16(v);
   }
-  if (e.bias) {
-    v = v + e.bias[c];
+  if (e.bias || e.bias16) {
+    v = v + (e.bias ? e.bias[c] : __half2float(e.bias16[c]));
     if (e.half_steps) v = round_f16(v);
   }
   if (e.resid && !e.resid_after) v = v + e.resid[idx];

@@ -895,18 +895,11 @@ struct Prepared {
   Tensor qw;         // conv: [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory; linear: [N,K]
   Tensor new_scale;  // device fp32 [Co] when per_channel
   Tensor rcp;        // its correctly rounded reciprocals (undefined where the kernels have to divide)
-  // fp32 copy of the bias passed when the entry was made, if that one was not fp32 already: valid for the same tensor
-  // at the same version; another bias is converted at the call
-  c10::weak_intrusive_ptr<c10::TensorImpl> b_impl;
-  uint32_t b_ver = 0;
-  const void *b_ptr = nullptr;
-  Tensor bias32;
   // recorded on the stream that quantized the weight, behind those kernels: a later call on another stream
   // (another thread's, a side stream) waits for it before it reads qw / new_scale
   at::cuda::CUDAEvent ready;
   std::atomic<bool> ready_seen{false};  // the event has been seen complete: no need to ask again
-  Prepared() : b_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
-               w_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
+  Prepared() : w_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
                s_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
                m_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)) {}
 };
@@ -953,7 +946,7 @@ c10::weak_intrusive_ptr<c10::TensorImpl> weak_of(const Tensor &t) {
 // Decode the two q-param encodings and quantize the weight (make_dense(weight, activation bit width)
 // returns it dense, dim 0 slowest, in the layout the caller's kernel wants).
 template <typename MakeDense>
-std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, const Tensor &bias, const Tensor &q_scale,
+std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, const Tensor &q_scale,
                                   const Tensor &q_mode) {
   auto p = std::make_shared<Prepared>();
   Tensor s_host = q_scale.to(at::kCPU).to(at::kFloat).contiguous();
@@ -1012,15 +1005,11 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
   p->s_host = q_scale.to(at::kCPU).contiguous().clone();
   p->m_host = q_mode.to(at::kCPU).contiguous().clone();
   if (p->new_scale.defined()) p->rcp = reciprocals_of(p->new_scale);
-  if (has_bias(bias) && bias.device() == weight.device() && !(bias.scalar_type() == at::kFloat && bias.is_contiguous())) {
-    p->bias32 = bias.to(at::kFloat).contiguous();
-    p->b_impl = weak_of(bias); p->b_ver = version_of(bias); p->b_ptr = bias.data_ptr();
-  }
   return p;
 }
 
 template <typename MakeDense>
-std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &bias, const Tensor &q_scale, const Tensor &q_mode,
+std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_scale, const Tensor &q_mode,
                                        MakeDense make_dense, int variant = 0) {
   const bool use_cache = cache_enabled();
   const c10::TensorImpl *key = weight.unsafeGetTensorImpl();
@@ -1038,7 +1027,7 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &bias,
           // read on another stream than the one the caching allocator knows these blocks by: tell it, so that
           // an entry dropped while this stream's kernels still read it is not handed out again too early
           it->second->qw.record_stream(cur);
-          for (const Tensor *t : {&it->second->new_scale, &it->second->rcp, &it->second->bias32})
+          for (const Tensor *t : {&it->second->new_scale, &it->second->rcp})
             if (t->defined()) t->record_stream(cur);
         }
         return it->second;
@@ -1046,7 +1035,7 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &bias,
       g_cache.erase(it);
     }
   }
-  auto p = prepare(make_dense, weight, bias, q_scale, q_mode);
+  auto p = prepare(make_dense, weight, q_scale, q_mode);
   p->variant = variant;
   const auto made_on = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
   p->made_on = made_on.id();
@@ -1076,8 +1065,10 @@ void clear_cache_op() {
   g_rcp_cache.clear();
 }
 
-// The epilogue of the reference ops: dequantization with the entry's constants, bias, floating output into `y`.
-// `keep` holds a bias converted for this call.
+// The epilogue of the reference ops: dequantization with the entry's constants, bias, floating output into `y`.  The bias
+// is read where it lies, by this call's kernel: nothing of it is kept (a copy made earlier would miss writes that the
+// version counter does not show, and a captured graph would go on reading it).  `keep` holds one that the kernels cannot
+// read, converted for this call.
 catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64_t co, const Tensor &y, Tensor *keep) {
   catchq_epilogue_t e;
   std::memset(&e, 0, sizeof(e));
@@ -1091,9 +1082,9 @@ catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64
     TORCH_CHECK(bias.numel() == co, "bias: expected ", co, " elements, got ", bias.numel());
     if (bias.scalar_type() == at::kFloat && bias.is_contiguous()) {
       e.bias = bias.data_ptr<float>();
-    } else if (p.bias32.defined() && p.b_impl._unsafe_get_target() == bias.unsafeGetTensorImpl() && !p.b_impl.expired() &&
-               p.b_ver == version_of(bias) && p.b_ptr == bias.data_ptr()) {
-      e.bias = p.bias32.data_ptr<float>();
+    } else if (bias.scalar_type() == at::kHalf && bias.is_contiguous() && (reinterpret_cast<uintptr_t>(bias.data_ptr()) & 15u) == 0) {
+      e.bias = static_cast<const float *>(bias.data_ptr());  // (elsewhere the vectorised epilogues could not take it)
+      e.bias_dtype = CATCHQ_F16;
     } else {
       *keep = bias.to(at::kFloat).contiguous();
       e.bias = keep->data_ptr<float>();
@@ -1168,7 +1159,7 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   };
   const int64_t kw_extra = (kw + 3) / 4 * 4 - kw;
   const bool can_frame = few && dilation.size() == 2 && dilation[1] == 1 && padding.size() == 2;
-  auto prep = prepared_for(weight, bias, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
+  auto prep = prepared_for(weight, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
     Tensor wd = w;
     const int64_t cpad = device_channels(bw_act) - ci;
     const int64_t taps = (few && bw_act == 8 && can_frame) ? kw_extra : 0;
@@ -1206,7 +1197,7 @@ Tensor conv1d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   TORCH_CHECK(padding.size() == 1 && stride.size() == 1 && dilation.size() == 1, "1-d conv parameters expected");
   const bool half = fp_dtype(input, "quantify only support input float/half") == CATCHQ_F16;
   c10::DeviceGuard guard(input.device());
-  auto prep = prepared_for(weight, bias, q_scale, q_mode, [](const Tensor &w, int) {
+  auto prep = prepared_for(weight, q_scale, q_mode, [](const Tensor &w, int) {
     return w.unsqueeze(2).contiguous(at::MemoryFormat::ChannelsLast);  // memory [Co][1][k][Ci/g]
   });
   Tensor qx = quantize_to_nhwc(input.unsqueeze(2), prep->bw_x, prep->pos_x, input.size(1));
@@ -1234,7 +1225,7 @@ Tensor conv3d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
               weight.size(1), " x groups ", groups);
   const int64_t d_out = (dd_in + 2 * pd - dd * (kd - 1) - 1) / sd + 1;
   TORCH_CHECK(dd_in + 2 * pd >= dd * (kd - 1) + 1 && d_out > 0, "Calculated output size is too small");
-  auto prep = prepared_for(weight, bias, q_scale, q_mode, [](const Tensor &wt, int) {
+  auto prep = prepared_for(weight, q_scale, q_mode, [](const Tensor &wt, int) {
     // [Co, (Ci/g)*kd, kh, kw] with the depth tap fastest inside a channel, stored [Co][kh][kw][(Ci/g)*kd]
     return wt.reshape({wt.size(0), wt.size(1) * wt.size(2), wt.size(3), wt.size(4)})
         .contiguous(at::MemoryFormat::ChannelsLast);
@@ -1309,7 +1300,7 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   // K is padded with zeros on both operands to what the matrix-core routes take (16 int8 / 8 int16 values)
   const int64_t k = weight.size(1);
   auto device_k = [&](int bw_act) { return bw_act == 8 ? (k + 15) / 16 * 16 : (k + 7) / 8 * 8; };
-  auto prep = prepared_for(weight, bias, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
+  auto prep = prepared_for(weight, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
     const int64_t kpad = device_k(bw_act) - k;
     return kpad > 0 ? at::constant_pad_nd(w, {0, kpad}, 0).contiguous() : w.contiguous();
   });

@@ -171,9 +171,11 @@ typedef struct catchq_epilogue {
   int exp2;
   const float *chan_div; /* device [co] or NULL */
   const float *chan_rcp; /* device [co] or NULL: 1/chan_div[c] rounded to nearest (see below) */
-  const float *bias;     /* device [co] or NULL */
+  const float *bias;     /* device [co] or NULL; binary16 values behind the pointer with bias_dtype CATCHQ_F16 */
   const float *resid;    /* device [rows, co] fp32 or NULL */
   int act;               /* CATCHQ_ACT_* */
+  int bias_dtype;        /* CATCHQ_F32, or CATCHQ_F16 (converted as it is read, which is exact): catchq_gemm_nt,
+                            catchq_conv2d_nhwc and catchq_float_conv2d_nhwc only, CATCHQ_ERR_DTYPE elsewhere */
   void *y;               /* device [rows, co] or NULL */
   int y_dtype;           /* CATCHQ_F32 / CATCHQ_F16 */
   int32_t *acc_out;      /* device [rows, co] or NULL */

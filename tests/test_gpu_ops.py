@@ -702,3 +702,118 @@ def test_grouped_half_per_channel_convolution(xs, ws, stride, groups):
     xd = x.cuda().contiguous(memory_format=torch.channels_last)
     got = torch.ops.torch_mlu.conv2d(xd, w.cuda(), b.cuda(), *args, scale.cuda(), mode.cuda())
     assert same_bits(want.contiguous().numpy(), got.cpu().contiguous().numpy())
+
+
+def _qparams(x, w, mode, half_scale):
+    """q_scale / q_mode for max-abs ranges, as the modules hold them"""
+    qmax = 127.0 if mode in (1, 3) else 32767.0
+    s_x = qmax / x.float().abs().max().reshape(1)
+    wf = w.float().reshape(w.shape[0], -1).abs()
+    s = torch.cat([s_x, torch.zeros(1), qmax / wf.amax(1)]) if mode > 2 else torch.cat([s_x, qmax / wf.max().reshape(1)])
+    return s.half() if half_scale else s, torch.tensor([mode], dtype=torch.int32)
+
+
+HALF_BIAS_CASES = [
+    # input, weight, stride, groups, mode, half q_scale, channels-last input (None: linear)
+    ((1, 768), (3072, 768), 0, 0, 3, False, None),              # few tiles, activations quantized on the way
+    ((1, 768), (3072, 768), 0, 0, 1, True, None),
+    ((300, 4096), (1000, 4096), 0, 0, 3, False, None),          # few tiles behind a quantizer
+    ((4096, 256), (2048, 256), 0, 0, 3, False, None),           # tiled GEMM
+    ((700, 208), (61, 208), 0, 0, 3, False, None),              # channels not a multiple of four
+    ((12289, 512), (128, 512), 0, 0, 3, False, None),           # few columns, activations quantized on the way
+    ((201, 1000), (1001, 1000), 0, 0, 2, False, None),          # int16 x int16, both store forms
+    ((201, 1000), (1004, 1000), 0, 0, 4, False, None),
+    ((65, 37), (24, 37), 0, 0, 2, False, None),
+    ((1, 64, 14, 14), (64, 64, 3, 3), 1, 1, 3, True, True),     # few tiles: every step rounded to half / one rounding
+    ((1, 64, 14, 14), (64, 64, 3, 3), 1, 1, 3, False, True),
+    ((1, 64, 14, 14), (30, 64, 3, 3), 1, 1, 3, True, False),
+    ((24, 64, 56, 56), (64, 64, 3, 3), 1, 1, 3, True, False),   # patch-resident
+    ((16, 128, 28, 28), (256, 128, 3, 3), 2, 1, 3, False, False),
+    ((4, 96, 57, 75), (160, 96, 3, 3), 1, 1, 3, True, False),   # tiled convolution
+    ((8, 64, 56, 56), (64, 64, 1, 1), 1, 1, 3, True, True),     # few columns
+    ((8, 64, 56, 56), (128, 64, 1, 1), 2, 1, 3, False, True),
+    ((16, 96, 56, 56), (24, 96, 1, 1), 1, 1, 3, True, False),   # streaming pointwise kernel
+    ((16, 96, 56, 56), (144, 96, 1, 1), 1, 1, 3, False, False),
+    ((4, 32, 28, 28), (32, 1, 3, 3), 1, 32, 3, True, True),     # depthwise
+    ((4, 32, 28, 28), (32, 1, 3, 3), 2, 32, 3, False, True),
+    ((1, 36, 40, 40), (36, 1, 5, 5), 1, 36, 3, True, True),
+    ((2, 64, 14, 14), (128, 16, 3, 3), 1, 4, 3, True, True),    # grouped: channel slices of the bias
+    ((2, 6, 9, 11), (10, 3, 3, 3), 1, 2, 3, True, False),       # direct
+    ((4, 3, 96, 96), (64, 3, 7, 7), 2, 1, 3, True, False),      # first layers
+    ((2, 1, 20, 20), (24, 1, 5, 5), 1, 1, 1, False, False),
+    ((2, 64, 20, 20), (96, 64, 3, 3), 1, 1, 4, False, True),    # int16 x int16 convolution
+    ((2, 64, 26, 26), (128, 64, 3, 3), 1, 1, "16x8", False, True),  # int16 x int8
+]
+
+
+def _half_layer(case):
+    xs, ws, stride, groups, mode, half_scale, nhwc = case
+    g = torch.Generator().manual_seed(sum(xs) + sum(ws))
+    x, w = torch.randn(xs, generator=g).half(), (torch.randn(ws, generator=g) / math.sqrt(np.prod(ws[1:]))).half()
+    b1, b2 = torch.randn(ws[0], generator=g).half(), torch.randn(ws[0], generator=g).half()
+    if mode == "16x8":  # [bit widths], [positions]
+        scale, mode_t = torch.tensor([16.0, 8.0]), torch.tensor([-12, -8], dtype=torch.int32)
+    else:
+        scale, mode_t = _qparams(x, w, mode, half_scale)
+    x, w, b1, b2, scale, mode_t = (t.cuda() for t in (x, w, b1, b2, scale, mode_t))
+    if nhwc:
+        x = x.contiguous(memory_format=torch.channels_last)
+    k = ws[-1]
+
+    def layer(bias):
+        if nhwc is None:
+            return torch.ops.torch_mlu.linear(x, w, bias, scale, mode_t)
+        return torch.ops.torch_mlu.conv2d(x, w, bias, [k // 2, k // 2], [stride, stride], [1, 1], groups, scale, mode_t)
+    return layer, b1, b2
+
+
+@pytest.mark.parametrize("case", HALF_BIAS_CASES)
+def test_half_bias_is_read_at_every_call(case):
+    """A half bias gives the bits its fp32 copy gives (which is read where it lies), on every kernel family, and so after
+    a write that the version counter does not see (`.data`, an inference tensor), through views that start anywhere and
+    through strided ones"""
+    note("half bias", case)
+    layer, b, b2 = _half_layer(case)
+    torch.ops.torch_mlu.clear_weight_cache()
+    y1 = layer(b)
+    assert torch.equal(y1, layer(b.float()))
+    ver, where = b._version, b.data_ptr()
+    b.data.copy_(b2)
+    assert b._version == ver and b.data_ptr() == where
+    y2 = layer(b)
+    assert torch.equal(y2, layer(b2.float())) and not torch.equal(y1, y2)
+    with torch.inference_mode():
+        bi = b2.clone()
+        assert torch.equal(layer(bi), y2)
+        bi.mul_(2)
+        assert torch.equal(layer(bi), layer(b2.float() * 2))
+    n = b.numel()
+    wide = torch.zeros(2 * n + 1, dtype=torch.float16, device="cuda")
+    wide[1:n + 1] = b2
+    assert torch.equal(layer(wide[1:n + 1]), y2)
+    wide[:2 * n:2] = b2
+    assert torch.equal(layer(wide[:2 * n:2]), y2)
+
+
+@pytest.mark.parametrize("case", [HALF_BIAS_CASES[i] for i in (0, 3, 9, 10, 15)])
+def test_captured_half_layer_follows_its_bias(case):
+    """the bias changed in place between the replays of a captured eager layer, the program's own work in between"""
+    note("half bias, captured", case)
+    layer, b, b2 = _half_layer(case)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for _ in range(2):
+        with torch.cuda.stream(side):
+            layer(b)
+        torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = layer(b)
+    for i in range(4):
+        if i:
+            b.copy_(b2 * i)
+        graph.replay()
+        torch.cuda.synchronize()
+        got = out.clone()
+        assert torch.equal(got, layer(b.float())), "replay %d" % i
+        torch.cuda.synchronize()
