@@ -59,7 +59,7 @@ inline bool vec_epilogue_ok(int N, const EpiDev &e) {
 // What an epilogue instance knows at compile time.  A field of -1 is decided at run time from the
 // EpiDev (the generic instance); fixed fields let the compiler drop every untaken branch, which
 // matters because the epilogue is VALU-bound (about a dozen fp32 operations per output element).
-//   DIV  0 none, 1 reciprocal form (the constants of a launch without divisors or bias are 1 and 0: nothing changes), 2 true
+//   DIV  0 none, 1 reciprocal form (the constants of a launch without divisors or bias are 1 and -0: nothing changes), 2 true
 //   division, 3 reciprocal form with every step rounded to binary16 (half_steps)      BIAS 0 none, 1 yes, 2 half or none     RESID 0 none, 1 before, 2 after the activation
 //   ACT  CATCHQ_ACT_*       YM  0 none, 1 fp32, 2 fp16     QM  0 none, 8, 16     ACC 0/1
 template <int DIV, int BIAS, int RESID, int ACT, int YM, int QM, int ACC>
@@ -150,8 +150,9 @@ inline int pick_epilogue(int N, const EpiDev &e) {
   // (the instances that fold the requantization's power of two into the per-channel constants keep those in range)
   if (e.q && (e.q_neg_pos < -40 || e.q_neg_pos > 40)) return EPI_VECTOR;
   const int div = e.half_steps ? (e.half_rcp ? 3 : 2) : (e.chan_rcp ? 1 : 0), bias = (e.bias || e.bias16) ? 1 : 0;
-  // without divisors the reciprocal form runs on ones (x * 2^e exactly, the correction is zero), without a bias on zeros
-  // (x + 0 = x: an integer sum is never -0); the power of two has to stay in the range that form is stated for
+  // without divisors the reciprocal form runs on ones (x * 2^e exactly, the correction is zero), without a bias on -0
+  // (x + -0 = x for every x, -0 among them: a small negative sum rounded to binary16); the power of two has to stay in the
+  // range that form is stated for
   const bool ones = div == 0 && !e.exp2_a && !e.exp2_b && e.exp2 >= -64 && e.exp2 <= 64;
   const int res = !e.resid ? 0 : (e.resid_after ? 2 : 1);
   const int ym = !e.y ? 0 : (e.y_f16 ? 2 : 1);
@@ -184,6 +185,7 @@ struct EpiLane {
 
 // A bias of four consecutive channels (n a multiple of four) in two halves, the bits as they lie in memory and their
 // values: a conversion beside the load would wait for it there, in front of a K loop in one kernel.
+constexpr int kNoBias = (int)0x80000000u, kNoBias16 = (int)0x80008000u;  // one -0, two -0 in binary16
 __device__ __forceinline__ v4i load_bias4(const EpiDev &e, int n) {
   if (e.bias) return *reinterpret_cast<const v4i *>(e.bias + n);
   const v2i h = *reinterpret_cast<const v2i *>(e.bias16 + n);
@@ -198,7 +200,7 @@ __device__ __forceinline__ v4f bias4_values(const EpiDev &e, const v4i bits) {
   return e.bias16 ? wide : __builtin_bit_cast(v4f, bits);
 }
 
-// The lane's constants from the raw values of its four channels (1 / 1 / 0 where a constant is absent).
+// The lane's constants from the raw values of its four channels (1 / 1 / -0 where a constant is absent).
 template <class S>
 __device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, const EpiDev &e) {
   EpiLane L;
@@ -228,16 +230,16 @@ __device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, c
 
 template <class S>
 __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev &e) {
-  v4f div = {1.f, 1.f, 1.f, 1.f}, rcp = {1.f, 1.f, 1.f, 1.f}, bias = {0.f, 0.f, 0.f, 0.f};
+  v4f div = {1.f, 1.f, 1.f, 1.f}, rcp = {1.f, 1.f, 1.f, 1.f}, bias = {-0.f, -0.f, -0.f, -0.f};
   const float *rcps = S::kSteps ? e.half_rcp : e.chan_rcp;
   if (n_ok && (S::rcp(e) || S::truediv(e) || S::kSteps) && e.chan_div) div = *reinterpret_cast<const v4f *>(e.chan_div + n);
   if (n_ok && (S::rcp(e) || S::kSteps) && rcps) rcp = *reinterpret_cast<const v4f *>(rcps + n);
   if constexpr (S::kHalfBias) {
-    v2i h = {0, 0};
+    v2i h = {kNoBias16, kNoBias16};
     if (n_ok && e.bias16) h = *reinterpret_cast<const v2i *>(e.bias16 + n);
     bias = half4_values(h);
   } else if constexpr (S::kAnyBias) {
-    v4i bits = {0, 0, 0, 0};
+    v4i bits = {kNoBias, kNoBias, kNoBias, kNoBias};
     if (n_ok && S::bias(e) && (e.bias || e.bias16)) bits = load_bias4(e, n);
     bias = bias4_values(e, bits);
   } else {
@@ -250,11 +252,12 @@ __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev
 __device__ __forceinline__ float epi_dequant1(float x, int t, const EpiLane &L, int exp2) {
   if (L.steps_rcp) {
     // fp32 operations on binary16 values rounded to binary16 are the binary16 operations.  The reciprocal form gives the
-    // correctly rounded fp32 quotient of the finite values; an infinite one (the scaled sum overflowed) stays infinite.
+    // correctly rounded fp32 quotient of the finite values; an infinite one (the scaled sum overflowed) stays infinite, and
+    // a zero keeps its sign, which the correction step would make positive.
     x = round_f16(__builtin_ldexpf(x, exp2));
     const float q = x * L.rcp[t];
     float v = __builtin_fmaf(__builtin_fmaf(-q, L.div[t], x), L.rcp[t], q);
-    v = __builtin_isinf(q) ? q : v;
+    v = __builtin_amdgcn_classf(q, 0x264) ? q : v;  // -inf, -0, +0, +inf
     asm volatile("" : "+v"(v));  // keeps the conversion below apart: fused into one operation it would round once
     return round_f16(v) + L.bias[t];  // (rounded to binary16 by the conversion of the output)
   }

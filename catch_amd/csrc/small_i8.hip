@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   const bool vec = p.epi != EPI_SCALAR;
   constexpr int ROUNDS = (EPI_LANES + 64 * NW - 1) / (64 * NW);
   v4f c_div = {1.f, 1.f, 1.f, 1.f}, c_rcp = c_div, c_res[ROUNDS];
-  v4i c_bias = {0, 0, 0, 0};
+  v4i c_bias = {kNoBias, kNoBias, kNoBias, kNoBias};
   v4f s_div = c_div, s_rcp = c_div, s_bias = {0.f, 0.f, 0.f, 0.f};  // the shortcut's constants
   // 64 * NW is a multiple of CPR: a lane has the same four channels in every round.  (Plain loads: the transfers below
   // and the statements that clobber memory keep them here, in front of the K loop.)

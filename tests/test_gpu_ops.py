@@ -817,3 +817,38 @@ def test_captured_half_layer_follows_its_bias(case):
         got = out.clone()
         assert torch.equal(got, layer(b.float())), "replay %d" % i
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("bias", ["none", "+0", "-0", "normal"])
+@pytest.mark.parametrize("xs,ws,stride,groups,nhwc", [
+    ((1, 64, 14, 14), (64, 64, 3, 3), 1, 1, True),      # few tiles
+    ((4, 64, 56, 56), (64, 64, 3, 3), 1, 1, False),     # patch-resident
+    ((1, 96, 57, 75), (160, 96, 3, 3), 1, 1, False),    # tiled convolution
+    ((8, 64, 56, 56), (64, 64, 1, 1), 1, 1, True),      # few columns, activations quantized on the way
+    ((16, 96, 56, 56), (24, 96, 1, 1), 1, 1, False),    # streaming pointwise kernel
+    ((4, 32, 28, 28), (32, 1, 3, 3), 1, 32, True),      # depthwise
+    ((1, 64, 14, 14), (30, 64, 3, 3), 1, 1, True),      # channels not a multiple of four
+])
+def test_half_steps_keep_the_sign_of_zero(xs, ws, stride, groups, nhwc, bias):
+    """Sums so small that the scaled value rounds to a half zero: it keeps the sum's sign through `/ new_scale` and, with
+    no bias or one of -0, through the addition -- what half tensor ops leave"""
+    note("half steps, sign of zero", xs, ws, bias)
+    g = torch.Generator().manual_seed(sum(xs) + sum(ws))
+    # activations and weights of about 2^-9 (positions near -15): an integer sum below 32 lies under half the least half
+    x = (torch.randint(-2, 3, xs, generator=g).float() * 2.0 ** -14)
+    x.reshape(-1)[0] = 0.00196
+    w = (torch.rand(ws, generator=g) * 2 - 1) * 2.0 ** -13
+    w.reshape(ws[0], -1)[:, 0] = 0.00196 + 0.0005 * torch.rand(ws[0], generator=g)
+    x, w = x.half(), w.half()
+    scale, mode = _qparams(x, w, 3, True)
+    b = {"none": torch.full((ws[0],), -0.0), "+0": torch.zeros(ws[0]), "-0": torch.full((ws[0],), -0.0),
+         "normal": torch.randn(ws[0], generator=g) * 2.0 ** -22}[bias].half()
+    k = ws[-1]
+    args = ([k // 2, k // 2], [stride, stride], [1, 1], groups)
+    want = ref_order.conv2d_per_channel(x, w, b, args[0], args[1], args[2], groups, scale, mode.numpy())["y"]
+    if bias == "none":  # (x + -0 is x)
+        assert (want.view(torch.int16) == -32768).sum() > 20 and (want.view(torch.int16) == 0).sum() > 20
+    xd = x.cuda().contiguous(memory_format=torch.channels_last) if nhwc else x.cuda()
+    got = torch.ops.torch_mlu.conv2d(xd, w.cuda(), torch.empty(0).cuda() if bias == "none" else b.cuda(), *args, scale.cuda(),
+                                     mode.cuda())
+    assert same_bits(want.contiguous().numpy(), got.cpu().contiguous().numpy())
