@@ -30,7 +30,8 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
 bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
 int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
                int Wo, const EpiDev &e, hipStream_t s);
-bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus);
+bool contract_small_float_ok(bool half, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw,
+                             int dh, int dw, int Ho, int Wo, int cus);
 int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
                          int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
 struct ChainLinkDev {  // igemm_i8_chain.hip
@@ -306,11 +307,12 @@ CATCHQ_API int catchq_conv2d_shortcut_nhwc(const void *x, int x_bits, const void
 // shapes that quantize and contract in one launch (pointer alignment is checked at the call): 1 few-tiles kernel, 2 GEMM of
 // few columns, 0 neither
 static int float_conv_fusable(const catchq_conv_desc_t *d, int x_dtype, int ho, int wo, const catchq_epilogue_t *e) {
-  const bool dense = d->kh == 1 && d->kw == 1 && d->stride_h == 1 && d->stride_w == 1 && d->pad_h == 0 && d->pad_w == 0;
   const int64_t M = (int64_t)d->n * ho * wo;
   const int cus = planned_cus(e->sharing);
   if (d->groups != 1) return 0;
-  if (contract_small_float_ok(M, d->co, (int64_t)d->kh * d->kw * d->ci, dense, d->ci, cus)) return 1;
+  if (contract_small_float_ok(x_dtype == CATCHQ_F16, d->n, d->h, d->w, d->ci, d->co, d->kh, d->kw, d->pad_h, d->pad_w, d->stride_h,
+                              d->stride_w, d->dil_h, d->dil_w, ho, wo, cus))
+    return 1;
   const bool pointwise = d->kh == 1 && d->kw == 1 && d->pad_h == 0 && d->pad_w == 0;
   return pointwise && gemm_float_ok((int64_t)d->n * d->h * d->w, M, d->co, d->ci, x_dtype == CATCHQ_F16 ? 2 : 4, cus) ? 2 : 0;
 }
@@ -341,13 +343,12 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
   const catchq_conv_desc_t &d = *desc;
   const int fusable = float_conv_fusable(desc, x_dtype, ho, wo, epilogue);
   if (fusable && aligned16(x) && aligned16(w)) {
-    const int64_t M = (int64_t)d.n * ho * wo;
-    const EpiDev e = make_epi(epilogue, M * d.co);
-    if (fusable == 2)
-      return gemm_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.stride_h, d.stride_w, ho, wo, e,
-                        as_stream(stream));
-    const int st2 = contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
-                                         d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
+    const EpiDev e = make_epi(epilogue, (int64_t)d.n * ho * wo * d.co);
+    const int st2 =
+        fusable == 2 ? gemm_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.stride_h, d.stride_w, ho,
+                                  wo, e, as_stream(stream))
+                     : contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
+                                            d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
     if (st2 >= 0) return st2;
   }
   // two launches: the quantized activations go through the workspace

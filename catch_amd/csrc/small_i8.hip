@@ -439,22 +439,31 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
 // 8.6 / 7.6 (4 x 14x14 256 -> 256 3x3), nine 37.7 / 19.0 (32 x 7x7 512 -> 512 3x3); 16 x 16 tiles, three steps 5.4 / 6.0
 // (14x14 256 -> 256 3x3), four 4.6 / 5.3 (8 x 2048 x 1000), six 5.5 / 5.3 (1 x 3072 x 768), eight 9.8 / 7.0
 // (32 x 4096 x 3072), thirteen 16.2 / 9.4 (2 x 14x14 256 -> 256 5x5).  Float activations lie within 1 us of these.
-bool contract_small_float_ok(int64_t M, int64_t Co, int64_t K, bool dense, int Ci, int cus) {
-  const int plan = small_plan(M, Co, K, dense, cus);
-  if (Ci % 16 != 0 || !plan) return false;
+//
+// The plan (as small_plan) and the kernel's constants; 0: not the one launch.  The question and the launch ask it both.
+static int small_float_plan(SmallSide *o, const void *x, bool half, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
+                            int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense, int cus) {
+  const int64_t K = (int64_t)kh * kw * Ci;
+  const int plan = small_plan((int64_t)N_img * Ho * Wo, Co, K, dense, cus);
+  if (!plan) return 0;
   const int waves = plan % 100;
   const int64_t per_wave = ((K + 127) / 128 + waves - 1) / waves;
-  return per_wave <= (plan / 100 == 32 ? 3 : 6);
+  if (per_wave > (plan / 100 == 32 ? 3 : 6)) return 0;
+  return small_side(o, x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense) ? plan : 0;
+}
+bool contract_small_float_ok(bool half, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw,
+                             int dh, int dw, int Ho, int Wo, int cus) {
+  SmallSide o;
+  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+  return small_float_plan(&o, nullptr, half, nullptr, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, cus) != 0;
 }
 int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
                          int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
   const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-  const int64_t M = (int64_t)N_img * Ho * Wo;
-  const int plan = small_plan(M, Co, (int64_t)kh * kw * Ci, dense, e.cus);
-  if (!plan) return -1;
   SmallParams p = {};
-  if (!small_side(&p.side[0], x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense)) return -1;
-  small_common(&p, M, Co, Ho, Wo, e);
+  const int plan = small_float_plan(&p.side[0], x, half, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, e.cus);
+  if (!plan) return -1;
+  small_common(&p, (int64_t)N_img * Ho * Wo, Co, Ho, Wo, e);
   p.x_neg_pos = -position;
   if (half) return dense ? launch_small_plan<true, IN_F16, false>(plan, p, e, s) : launch_small_plan<false, IN_F16, false>(plan, p, e, s);
   return dense ? launch_small_plan<true, IN_F32, false>(plan, p, e, s) : launch_small_plan<false, IN_F32, false>(plan, p, e, s);

@@ -852,3 +852,19 @@ def test_half_steps_keep_the_sign_of_zero(xs, ws, stride, groups, nhwc, bias):
     got = torch.ops.torch_mlu.conv2d(xd, w.cuda(), torch.empty(0).cuda() if bias == "none" else b.cuda(), *args, scale.cuda(),
                                      mode.cuda())
     assert same_bits(want.contiguous().numpy(), got.cpu().contiguous().numpy())
+
+
+def test_strided_pointwise_layer_on_more_than_2_gib_of_activations():
+    """a stride that leaves few outputs of a huge floating input: served through a quantizer's launch"""
+    note("strided pointwise, 4 GiB input")
+    n, side, ci, co, stride = 1, 4096, 64, 16, 64
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn((n, side, side, ci), generator=g, device="cuda")
+    xs = x[:, ::stride, ::stride].contiguous().cpu().permute(0, 3, 1, 2)
+    w = torch.randn(co, ci, 1, 1, generator=torch.Generator().manual_seed(4)) * 0.1
+    b = torch.randn(co, generator=torch.Generator().manual_seed(5))
+    scale, mode = _qparams(xs, w, 3, False)
+    want = oops.conv2d(xs.contiguous().numpy(), w.numpy(), b.numpy(), (0, 0), (1, 1), (1, 1), 1, scale.numpy(), mode.numpy())["y"]
+    got = torch.ops.torch_mlu.conv2d(x.permute(0, 3, 1, 2), w.cuda(), b.cuda(), [0, 0], [stride, stride], [1, 1], 1, scale.cuda(),
+                                     mode.cuda())
+    assert same_bits(want, got.cpu().contiguous().numpy())

@@ -140,6 +140,25 @@ def test_routes(lib):
     assert lib.catchq_gemm_route(16, 16, 40, 30, 70000) == b"direct"  # K beyond what int32 digit sums hold
 
 
+def test_float_convolution_workspace_of_large_inputs(lib):
+    """one launch (no workspace) only where that launch can address its operands: never for 2 GiB of activations, nor for
+    the dilations, strides and sizes that its 32-bit arithmetic does not cover"""
+    from catch_amd._native import ConvDesc, Epilogue
+
+    def workspace(n, h, w, ci, co, k=1, stride=1, dil=1, pad=0, dtype=0):
+        d = ConvDesc(n, h, w, ci, co, k, k, pad, pad, stride, stride, dil, dil, 1)
+        size = ctypes.c_size_t(12345)
+        assert lib.catchq_float_conv2d_workspace_size(dtype, ctypes.byref(d), ctypes.byref(Epilogue()), ctypes.byref(size)) == 0
+        return size.value
+    for dtype, esize in ((0, 4), (1, 2)):
+        for side in (2048, 4096):
+            big = side * side * 64 * esize >= 1 << 31
+            assert workspace(1, side, side, 64, 16, stride=64, dtype=dtype) == (side * side * 64 if big else 0), (dtype, side)
+    assert workspace(1, 14, 14, 256, 256, k=3, pad=1) == 0
+    # taps 2^19 rows apart on a one-column image
+    assert workspace(1, (1 << 20) + 1, 1, 16, 16, k=3, pad=(1 << 19), dil=1 << 19, stride=1 << 18) == ((1 << 20) + 1) * 16
+
+
 # ------------------------------------------------------------------ the Python tool (A1/A2/A15)
 def _tool():
     import catch_amd  # noqa: F401
