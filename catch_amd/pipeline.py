@@ -172,10 +172,11 @@ class FusedNet(object):
         blocks' int8 tensors instead of being stored and read back in fp32: a block whose chain back to the
         stage's projection shortcut has at most this many links (the shortcut counts as one) evaluates the
         whole chain inside its last convolution's launch (torch_mlu::qconv2d_chain); None picks the default
-        rule (_default_chain_links), 0 switches the recomputation off.
+        rule (_default_chain_links, and no chains for few pixels: _few_pixels), 0 switches the recomputation off.
+        A given limit stands for every batch.
         fuse_heads: a 1x1 convolution + ReLU whose only reader is a 3x3 convolution (the first two layers of a
-        bottleneck block) runs inside that convolution's launch where the kernel library serves the shapes
-        (torch_mlu::qconv2d_head); its int8 output is then never stored.
+        bottleneck block) runs inside that convolution's launch where the kernel library serves the shapes and the images
+        are large enough for it to pay (torch_mlu::qconv2d_head, head_fuses); its int8 output is then never stored.
         fuse_blocks: an inverted-residual block (1x1 expansion, 3x3 depthwise, 1x1 linear projection, each hidden
         tensor read by the next layer only) runs as one launch (torch_mlu::qconv2d_irb) where the library's kernel
         serves the shape and the image is large enough for it to pay (block_fuses).  Off by default: the one-launch
@@ -189,6 +190,7 @@ class FusedNet(object):
         (torch_mlu::qconv2d_avgpool) where the library's kernel serves the shape; its fp32 output is then never stored."""
         self.layers = list(layers)
         self._fuse_shortcuts = fuse_shortcuts
+        self._chains_by_size = chain_links is None
         self.device = torch.device(device)
         self.outputs = outputs_of(self.layers)
         self.out_half = out_half
@@ -357,8 +359,8 @@ class FusedNet(object):
 
     @staticmethod
     def _few_pixels(n, h, w):
-        """Whether a batch is planned block by block (_few_plan): one two-branch launch per projection block and no residual
-        chain.  A chain recomputes a block's earlier branches to save fp32 traffic; up to two images of 224 x 224 there is
+        """Whether the default rule plans a batch block by block (_few_plan): one two-branch launch per projection block and no
+        residual chain.  A chain recomputes a block's earlier branches to save fp32 traffic; up to two images of 224 x 224 there is
         no traffic to speak of and its 64 x 128 tiles are a handful of blocks, where the two-branch launch has the
         few-tiles kernel (ResNet-50, one stream: one image 234 -> 230 us, 2 x 224 x 224 ties, 4 x 128 x 128 233 -> 227 us;
         6 x 224 x 224 loses, 336 -> 347 us)."""
@@ -369,13 +371,16 @@ class FusedNet(object):
         if self._few is None:
             few = copy.copy(self)
             few.chain_of = {}
-            few.head_of, few._head_names = {}, set()
             few.shortcut_of = few._plan_shortcuts() if self._fuse_shortcuts else {}
             few._fused_away = few._layers_fused_away()
             few._plan_demands()
             few._few = few
             self._few = few
         return self._few
+
+    def plan_for(self, n, h, w):
+        """the plan that an untraced pass over n images of h x w runs: this one, or its variant for few pixels"""
+        return self._few_plan() if self._chains_by_size and self._few_pixels(n, h, w) else self
 
     def block_fuses(self, proj, n, h, w):
         """whether the inverted-residual block that ends in the layer `proj` runs as one launch over n images whose
@@ -518,8 +523,10 @@ class FusedNet(object):
         timers: optional dict; every conv/fc launch is bracketed by a pair of events recorded on
         the current stream and the pair is appended to timers[layer name] (durations of the
         launches in their real sequence, caches as the previous layer left them)."""
-        if trace is None and self is not self._few and self._few_pixels(x.shape[0], x.shape[2], x.shape[3]):
-            return self._few_plan().forward(x, None, timers, keep)
+        if trace is None:
+            plan = self.plan_for(x.shape[0], x.shape[2], x.shape[3])
+            if plan is not self:
+                return plan.forward(x, None, timers, keep)
         ops = torch.ops.torch_mlu
         env = {}
         tracing = trace is not None

@@ -25,6 +25,20 @@ def note(*a):
     sys.stdout.flush()
 
 
+def count_calls(monkeypatch, *names):
+    """how often the plan launches each of these torch_mlu ops from here on"""
+    counts = dict.fromkeys(names, 0)
+
+    def counted(name, op):
+        def call(*args):
+            counts[name] += 1
+            return op(*args)
+        return call
+    for name in names:
+        monkeypatch.setattr(torch.ops.torch_mlu, name, counted(name, getattr(torch.ops.torch_mlu, name)))
+    return counts
+
+
 def np_sd(sd):
     return {k: v.detach().cpu().numpy() for k, v in sd.items()}
 
@@ -188,16 +202,19 @@ def test_projection_shortcuts_fused_into_block_end(depth, expect):
 
 
 @pytest.mark.parametrize("limit", [None, 0, 2, 3, 8])
-def test_resnet50_residual_chains(limit):
+def test_resnet50_residual_chains(limit, monkeypatch):
     """Blocks whose residual branch is recomputed from int8 tensors inside their last convolution's launch
     (chain_links): every tensor the plan still produces equals the block-by-block plan's, the logits equal the
     oracle's; with 8 links every block of every stage is a chain and no fp32 tensor is left between blocks."""
     note("residual chains, resnet50, limit", limit)
     layers = nets.resnet(50)
     net = nets.FloatNet(layers, seed=8).eval()
-    x = torch.randn(3, 3, 96, 96, generator=torch.Generator().manual_seed(9))
+    # the default rule makes no chains for few pixels, a limit that the caller gives stands for every size
+    side = 192 if limit is None else 96
+    x = torch.randn(3, 3, side, side, generator=torch.Generator().manual_seed(9))
     sd = pipeline.calibrate(net, x, "int8", True)
     fused = pipeline.FusedNet(layers, sd, chain_links=limit)
+    assert fused.plan_for(3, side, side) is fused
     plain = pipeline.FusedNet(layers, sd, chain_links=0, fuse_avgpool=False)
     lens = {n: len(c) for n, c in fused.chain_of.items()}
     if limit == 0:
@@ -212,12 +229,40 @@ def test_resnet50_residual_chains(limit):
     for name, c in fused.chain_of.items():
         assert c[-1].name == name and c[0].name.endswith(".ds") and [l.name[:2] for l in c] == [name[:2]] * len(c)
     ka, kb = {}, {}
+    counts = count_calls(monkeypatch, "qconv2d_chain", "qconv2d_shortcut")
     a = fused.forward(x.cuda(), keep=ka)
+    assert counts == {"qconv2d_chain": len(lens), "qconv2d_shortcut": 4 if limit == 0 else 0}
     b = plain.forward(x.cuda(), keep=kb)
+    assert counts == {"qconv2d_chain": len(lens), "qconv2d_shortcut": 8 if limit == 0 else 4}
     torch.cuda.synchronize()
     assert torch.equal(a, b)
     for key, t in ka.items():
         assert torch.equal(t, kb[key]), key
+    check_against_oracle(layers, sd, x, fused)
+
+
+def test_plan_of_few_pixels(monkeypatch):
+    """Up to two images of 224 x 224 the default plan has no residual chains: two-branch launches, the same tensors and
+    logits as the chained plan, which a batch beyond that and a caller's own chain limit get; a traced pass equals both"""
+    note("resnet50, plan of few pixels")
+    layers = nets.resnet(50)
+    net = nets.FloatNet(layers, seed=8).eval()
+    x = torch.randn(2, 3, 96, 128, generator=torch.Generator().manual_seed(9))
+    sd = pipeline.calibrate(net, x, "int8", True)
+    fused, chained = pipeline.FusedNet(layers, sd), pipeline.FusedNet(layers, sd, chain_links=3)
+    few = fused.plan_for(2, 96, 128)
+    assert few is not fused and not few.chain_of and few.plan_for(2, 96, 128) is few
+    assert fused.plan_for(2, 224, 224) is few and fused.plan_for(3, 224, 224) is fused and fused.plan_for(2, 224, 225) is fused
+    assert chained.plan_for(1, 32, 32) is chained and few.head_of == fused.head_of and fused.head_of
+    counts = count_calls(monkeypatch, "qconv2d_chain", "qconv2d_shortcut")
+    ka, kb = {}, {}
+    a = fused.forward(x.cuda(), keep=ka)
+    assert counts == {"qconv2d_chain": 0, "qconv2d_shortcut": 4}
+    b = chained.forward(x.cuda(), keep=kb)
+    assert counts["qconv2d_chain"] == len(chained.chain_of) > 0
+    assert torch.equal(a, b)
+    for key, t in kb.items():
+        assert torch.equal(t, ka[key]), key
     check_against_oracle(layers, sd, x, fused)
 
 
