@@ -582,7 +582,8 @@ def main():
     fused, xg, w_ = build_workload(args)
     net, x, sd, layers, batch, side, what, detector, t_cal = (w_[k] for k in ("net", "x", "sd", "layers", "batch", "side",
                                                                                "what", "detector", "t_cal"))
-    static_in, replay = fused.capture(xg, streams=args.streams)
+    static_in, replay = fused.capture(xg, parts=args.streams)
+    fused = fused.plan_for(batch // args.streams, side, side)  # the plan of the recorded passes
     static_in.copy_(xg)
     for _ in range(args.warmup):
         replay()
@@ -869,7 +870,7 @@ def other_networks(steps=20):
     for workload, key in (("mobilenet_v2", "mobilenet_v2_bs128"), ("darknet53_yolov3", "darknet53_yolov3_bs16")):
         a = _ap.Namespace(workload=workload, batch=0, calib_images=8, fractional_scale=False, streams=2, chain_links=-1)
         fused, xg, w_ = build_workload(a)
-        static_in, replay = fused.capture(xg, streams=a.streams)
+        static_in, replay = fused.capture(xg, parts=a.streams)
         static_in.copy_(xg)
         for _ in range(5):
             replay()

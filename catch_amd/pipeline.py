@@ -213,6 +213,7 @@ class FusedNet(object):
                   for l in self.layers if l.kind in ("conv", "fc")}
         self._plan_demands()
         self._graph = None
+        self.graph_parts = 0  # of the graph captured last
         # A few-channel int8 network input feeding one k x k convolution: quantize it into a zero frame
         # (the convolution's padding, materialised) and pad the filter rows to whole groups of 4 taps,
         # so the first layer fetches filter rows with plain 16-byte loads on the matrix-core route.
@@ -738,7 +739,7 @@ class FusedNet(object):
         return forms
 
     # ------------------------------------------------------------------------------------------
-    def capture(self, example, streams=1):
+    def capture(self, example, streams=1, parts=None):
         """Record one forward pass into a HIP graph; returns (static_input, replay) where replay()
         re-runs the whole network on whatever static_input holds and returns the static output(s).
 
@@ -746,11 +747,19 @@ class FusedNet(object):
         default priority) between a fork and a join: the images are independent, so the results are the
         same tensors, and the launches of one part fill the compute units that the other part's launches
         leave idle while they start up and drain.  A batch whose launches are too short for that is recorded as fewer
-        parts (_parts)."""
+        parts (_parts): `streams` is the most there may be.
+        parts: record exactly this many, whatever `streams` says and whether they pay or not.
+        graph_parts holds the number recorded."""
         static_in = example.clone()
-        asked = max(1, min(int(streams), static_in.shape[0]))
-        parts = self._parts(asked, *static_in.shape)
-        chunks = list(static_in.chunk(parts))
+        if parts is None:
+            asked = max(1, min(int(streams), static_in.shape[0]))
+            chunks = list(static_in.chunk(self._parts(asked, *static_in.shape)))
+        else:
+            asked = int(parts)
+            if not 1 <= asked <= static_in.shape[0]:
+                raise ValueError("capture: %d parts of a batch of %d" % (asked, static_in.shape[0]))
+            chunks = list(static_in.tensor_split(asked))
+        self.graph_parts = len(chunks)
         # As many streams as asked for are drawn from the pool, used or not: its streams take turns on the four hardware
         # queues, and a capture that advanced it by one left the branches of later graphs on one queue (Darknet-53 in two
         # parts behind MobileNetV2 captures of one: 2.57 -> 3.0 ms)

@@ -230,6 +230,7 @@ def test_resnet50_at_the_benchmark_shapes():
     assert np.array_equal(want, logits[pick].cpu().numpy())
     # the graph the benchmark replays (two halves on two streams) returns the same logits
     static_in, replay = fused.capture(x.cuda(), streams=2)
+    assert fused.graph_parts == 2
     assert torch.equal(replay(), logits)
 
 
@@ -362,6 +363,7 @@ def test_full_batch_graph_equals_its_images_alone(arch, batch, side):
         sd = pipeline.calibrate(net, x[:4], "int8", True)
     fused = pipeline.FusedNet(layers, sd, out_half=detector)
     static_in, replay = fused.capture(x.cuda(), streams=2)
+    assert fused.graph_parts == 2
     out = replay()
     outs = out if isinstance(out, tuple) else (out,)
     half = batch // 2

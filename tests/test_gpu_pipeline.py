@@ -148,8 +148,9 @@ def test_resnet50_small_batch_and_graph_replay():
 @pytest.mark.parametrize("arch,batch,streams", [("resnet50", 5, 2), ("resnet50", 4, 3), ("darknet53_yolov3", 3, 2),
                                                 ("resnet18", 2, 4)])
 def test_graph_with_the_batch_on_parallel_streams(arch, batch, streams):
-    """the batch split into parts that run on streams of their own inside one HIP graph (uneven parts, more
-    streams than images, several outputs): every replay equals the single eager pass, new inputs included"""
+    """the batch split into parts that run on streams of their own inside one HIP graph (uneven parts, more than two, one
+    image each, several outputs): every replay equals the single eager pass, new inputs included; asked for more streams
+    than such launches pay for, the plan records one part"""
     note("parallel streams", arch, batch, streams)
     layers = nets.NETS[arch]()
     det = arch.startswith("darknet")
@@ -160,7 +161,11 @@ def test_graph_with_the_batch_on_parallel_streams(arch, batch, streams):
     if det:
         sd = pipeline.to_position_encoding(sd, 16, 8)
     fused = pipeline.FusedNet(layers, sd, out_half=det)
-    static_in, replay = fused.capture(x.cuda(), streams=streams)
+    fused.capture(x.cuda(), streams=streams)
+    assert fused.graph_parts == 1  # (launches this short run back to back faster)
+    parts = min(batch, streams)
+    static_in, replay = fused.capture(x.cuda(), parts=parts)
+    assert fused.graph_parts == parts
     for i in range(4):
         xi = x.cuda() if i % 2 == 0 else (x.cuda() * 0.5 + 0.1)
         want = fused.forward(xi)
@@ -266,6 +271,30 @@ def test_plan_of_few_pixels(monkeypatch):
     check_against_oracle(layers, sd, x, fused)
 
 
+def test_parts_of_a_captured_batch():
+    """`streams` is the most parts a graph may have, fewer where the launches are too short to pay for the branches;
+    `parts` is the number recorded"""
+    note("resnet18, parts of a captured batch")
+    layers = nets.resnet(18)
+    net = nets.FloatNet(layers, seed=0).eval()
+    x = torch.randn(7, 3, 64, 64, generator=torch.Generator().manual_seed(1))
+    sd = pipeline.calibrate(net, x, "int8", True)
+    fused = pipeline.FusedNet(layers, sd)
+    assert fused._parts(2, 256, 3, 224, 224) == 2 and fused._parts(2, 2, 3, 224, 224) == 1
+    want = fused.forward(x.cuda())
+    for kwargs, parts in (({}, 1), (dict(streams=4), 1), (dict(parts=1), 1), (dict(parts=3), 3), (dict(streams=2, parts=5), 5),
+                          (dict(parts=7), 7)):
+        static_in, replay = fused.capture(x.cuda(), **kwargs)
+        assert fused.graph_parts == parts, kwargs
+        for i in range(2):
+            assert torch.equal(replay(), want), (kwargs, i)
+            _ = fused.forward(torch.randn(7, 3, 64, 64, device="cuda"))  # eager work between the replays
+            torch.cuda.synchronize()
+    for bad in (0, -1, 8):
+        with pytest.raises(ValueError, match="parts"):
+            fused.capture(x.cuda(), parts=bad)
+
+
 def test_mobilenet_v2_small():
     """MobileNetV2: depthwise stencil kernel, ReLU6, linear bottlenecks with residual adds, channel
     counts (24, 144) that the device layout pads to multiples of 16."""
@@ -363,7 +392,8 @@ def test_last_convolution_inside_the_average_pooling(arch):
     assert torch.equal(a, b)
     for key, t in ka.items():
         assert torch.equal(t, kb[key]), key
-    static_in, replay = fused.capture(x.cuda(), streams=2)
+    static_in, replay = fused.capture(x.cuda(), parts=2)
+    assert fused.graph_parts == 2
     for i in range(2):
         static_in.copy_(x.cuda())
         assert torch.equal(replay(), b), "replay %d" % i
