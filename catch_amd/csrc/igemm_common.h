@@ -53,7 +53,7 @@ __device__ __forceinline__ int xcd_remap(int bid, int nb) {
 inline bool vec_epilogue_ok(int N, const EpiDev &e) {
   // (N < 2^24: the per-lane part of an element index, at most 32 rows, fits 32 bits with room to spare)
   return N % 4 == 0 && N < (1 << 24) && aligned16(e.chan_div) && aligned16(e.chan_rcp) && aligned16(e.bias) && aligned16(e.resid) && aligned16(e.y) &&
-         aligned16(e.acc_out) && aligned16(e.q) && (reinterpret_cast<uintptr_t>(e.bias16) & 7u) == 0;
+         aligned16(e.acc_out) && aligned16(e.q);
 }
 
 // What an epilogue instance knows at compile time.  A field of -1 is decided at run time from the
@@ -84,7 +84,7 @@ struct EpiSpec {
   static __device__ __forceinline__ bool truediv(const EpiDev &e) {
     return DIV < 0 ? (e.chan_div != nullptr && e.chan_rcp == nullptr) : DIV == 2;
   }
-  static __device__ __forceinline__ bool bias(const EpiDev &e) { return BIAS < 0 ? e.bias || e.bias16 : BIAS >= 1; }
+  static __device__ __forceinline__ bool bias(const EpiDev &e) { return BIAS < 0 ? e.bias != nullptr : BIAS >= 1; }
   static __device__ __forceinline__ bool resid(const EpiDev &e) { return RESID < 0 ? e.resid != nullptr : RESID >= 1; }
   static __device__ __forceinline__ bool resid_after(const EpiDev &e) { return RESID < 0 ? e.resid_after != 0 : RESID == 2; }
   static __device__ __forceinline__ int act(const EpiDev &e) { return ACT < 0 ? e.act : ACT; }
@@ -146,10 +146,10 @@ template <> struct EpiOf<EPI_LK_RESA_Y_Q16> { typedef EpiSpec<0, 1, 2, CATCHQ_AC
 inline int pick_epilogue(int N, const EpiDev &e) {
   if (!vec_epilogue_ok(N, e)) return EPI_SCALAR;
   if (e.acc_out || (e.q && e.q_scale != 1.0f) || (e.chan_div && !e.chan_rcp && !e.half_rcp)) return EPI_VECTOR;
-  if (e.bias16 && (e.q || e.resid)) return EPI_VECTOR;  // (kAnyBias)
+  if (e.bias_f16 && (e.q || e.resid)) return EPI_VECTOR;  // (kAnyBias)
   // (the instances that fold the requantization's power of two into the per-channel constants keep those in range)
   if (e.q && (e.q_neg_pos < -40 || e.q_neg_pos > 40)) return EPI_VECTOR;
-  const int div = e.half_steps ? (e.half_rcp ? 3 : 2) : (e.chan_rcp ? 1 : 0), bias = (e.bias || e.bias16) ? 1 : 0;
+  const int div = e.half_steps ? (e.half_rcp ? 3 : 2) : (e.chan_rcp ? 1 : 0), bias = e.bias ? 1 : 0;
   // without divisors the reciprocal form runs on ones (x * 2^e exactly, the correction is zero), without a bias on -0
   // (x + -0 = x for every x, -0 among them: a small negative sum rounded to binary16); the power of two has to stay in the
   // range that form is stated for
@@ -169,7 +169,7 @@ inline int pick_epilogue(int N, const EpiDev &e) {
       {EPI_Y16_STEPS, 3, 1, 0, CATCHQ_ACT_NONE, 2, 0}};
   // The step-rounding instance takes a half bias, which is what a half layer has: in ResNet-50 at 32 images its one-launch
   // pointwise layers take 16.6 us so and 16.75 with a choice at run time, its 64 x 64 tiles 11.4 and 11.9.
-  if (div == 3 && e.bias) return EPI_VECTOR;
+  if (div == 3 && e.bias && !e.bias_f16) return EPI_VECTOR;
   for (const auto &r : rows)
     if ((r.div == div || (r.div == 1 && ones)) && (r.bias == bias || bias == 0) && r.res == res && r.act == e.act && r.ym == ym && r.qm == qm) return r.epi;
   return EPI_VECTOR;
@@ -183,22 +183,27 @@ struct EpiLane {
   int act;
 };
 
-// A bias of four consecutive channels (n a multiple of four) in two halves, the bits as they lie in memory and their
-// values: a conversion beside the load would wait for it there, in front of a K loop in one kernel.
-constexpr int kNoBias = (int)0x80000000u, kNoBias16 = (int)0x80008000u;  // one -0, two -0 in binary16
-__device__ __forceinline__ v4i load_bias4(const EpiDev &e, int n) {
-  if (e.bias) return *reinterpret_cast<const v4i *>(e.bias + n);
-  const v2i h = *reinterpret_cast<const v2i *>(e.bias16 + n);
-  return v4i{h[0], h[1], 0, 0};
-}
 __device__ __forceinline__ v4f half4_values(const v2i bits) {
   typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
   return __builtin_convertvector(__builtin_bit_cast(f16x4, bits), v4f);
 }
-__device__ __forceinline__ v4f bias4_values(const EpiDev &e, const v4i bits) {
-  const v4f wide = half4_values(v2i{bits[0], bits[1]});
-  return e.bias16 ? wide : __builtin_bit_cast(v4f, bits);
-}
+// A bias of four consecutive channels (n a multiple of four), of either precision: the bits as they lie in memory, and
+// their values later.  A conversion beside the load would wait for it there, in front of a K loop in one kernel.
+// (One load and a conditional one: a branch to either load measured the same or slower.)
+struct Bias4 {
+  v2i lo = {kNoBias, kNoBias}, hi = {kNoBias, kNoBias};  // halfs: all four in lo
+  static constexpr int kNoBias = (int)0x80000000u;       // -0: x + -0 = x
+  __device__ __forceinline__ void load(const EpiDev &e, int n) {
+    if (!e.bias) return;
+    const char *at = (const char *)e.bias + ((int64_t)n << (e.bias_f16 ? 1 : 2));
+    lo = *reinterpret_cast<const v2i *>(at);
+    if (!e.bias_f16) hi = *reinterpret_cast<const v2i *>(at + 8);
+  }
+  __device__ __forceinline__ v4f wide_values() const {
+    return __builtin_bit_cast(v4f, v4i{lo[0], lo[1], hi[0], hi[1]});
+  }
+  __device__ __forceinline__ v4f values(const EpiDev &e) const { return e.bias_f16 ? half4_values(lo) : wide_values(); }
+};
 
 // The lane's constants from the raw values of its four channels (1 / 1 / -0 where a constant is absent).
 template <class S>
@@ -235,13 +240,13 @@ __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev
   if (n_ok && (S::rcp(e) || S::truediv(e) || S::kSteps) && e.chan_div) div = *reinterpret_cast<const v4f *>(e.chan_div + n);
   if (n_ok && (S::rcp(e) || S::kSteps) && rcps) rcp = *reinterpret_cast<const v4f *>(rcps + n);
   if constexpr (S::kHalfBias) {
-    v2i h = {kNoBias16, kNoBias16};
-    if (n_ok && e.bias16) h = *reinterpret_cast<const v2i *>(e.bias16 + n);
+    v2i h = {(int)0x80008000u, (int)0x80008000u};
+    if (n_ok && e.bias) h = *reinterpret_cast<const v2i *>(reinterpret_cast<const __half *>(e.bias) + n);
     bias = half4_values(h);
   } else if constexpr (S::kAnyBias) {
-    v4i bits = {kNoBias, kNoBias, kNoBias, kNoBias};
-    if (n_ok && S::bias(e) && (e.bias || e.bias16)) bits = load_bias4(e, n);
-    bias = bias4_values(e, bits);
+    Bias4 b;
+    if (n_ok && S::bias(e)) b.load(e, n);
+    bias = b.values(e);
   } else {
     if (n_ok && S::bias(e) && e.bias) bias = *reinterpret_cast<const v4f *>(e.bias + n);
   }

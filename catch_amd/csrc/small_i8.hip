@@ -88,7 +88,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   const bool vec = p.epi != EPI_SCALAR;
   constexpr int ROUNDS = (EPI_LANES + 64 * NW - 1) / (64 * NW);
   v4f c_div = {1.f, 1.f, 1.f, 1.f}, c_rcp = c_div, c_res[ROUNDS];
-  v4i c_bias = {kNoBias, kNoBias, kNoBias, kNoBias};
+  Bias4 c_bias;
   v4f s_div = c_div, s_rcp = c_div, s_bias = {0.f, 0.f, 0.f, 0.f};  // the shortcut's constants
   // 64 * NW is a multiple of CPR: a lane has the same four channels in every round.  (Plain loads: the transfers below
   // and the statements that clobber memory keep them here, in front of the K loop.)
@@ -98,7 +98,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     if (e.chan_div) c_div = *reinterpret_cast<const v4f *>(e.chan_div + cc);
     const float *rcps = e.chan_rcp ? e.chan_rcp : e.half_rcp;
     if (rcps) c_rcp = *reinterpret_cast<const v4f *>(rcps + cc);
-    if (e.bias || e.bias16) c_bias = load_bias4(e, cc);  // (bits)
+    c_bias.load(e, cc);
     if constexpr (DUAL) {
       if (p.sc.chan_div) s_div = *reinterpret_cast<const v4f *>(p.sc.chan_div + cc);
       if (p.sc.chan_rcp) s_rcp = *reinterpret_cast<const v4f *>(p.sc.chan_rcp + cc);
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     }
     auto run = [&](auto spec) {
       typedef decltype(spec) S;
-      EpiLane L = epi_lane_finish<S>(c_div, c_rcp, bias4_values(e, c_bias), e);
+      EpiLane L = epi_lane_finish<S>(c_div, c_rcp, S::kAnyBias || S::kHalfBias ? c_bias.values(e) : c_bias.wide_values(), e);
       if constexpr (DUAL) {
         L.use_res = true;
         L.res_after = e.resid_after != 0;

@@ -281,8 +281,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
     if (n >= p.N) return;
     const bool plain = e.y && !e.q && !e.resid && e.act == CATCHQ_ACT_NONE && !e.half_steps;  // a floating output, nothing else
     const float c_div = e.chan_div ? e.chan_div[n] : 1.0f, c_rcp = e.chan_rcp ? e.chan_rcp[n] : 1.0f;
-    const bool biased = e.bias || e.bias16;
-    const float c_bias = e.bias ? e.bias[n] : (e.bias16 ? __half2float(e.bias16[n]) : 0.0f);
+    const float c_bias = e.bias ? bias_value(e, n) : 0.0f;
     for (int px = threadIdx.x / BN; px < BM; px += 64 * NW / BN) {
       const int m = m0 + px;
       if (m >= p.M) break;
@@ -293,7 +292,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
         float f = __builtin_ldexpf((float)v, e.exp2);
         if (e.chan_rcp) f = div_by_rcp(f, c_div, c_rcp);
         else if (e.chan_div) f = f / c_div;
-        if (biased) f = f + c_bias;
+        if (e.bias) f = f + c_bias;
         if (e.y_f16) {
           asm volatile("" : "+v"(f));  // the fp32 value exists: its conversion to fp16 is a rounding of its own
           reinterpret_cast<__half *>(e.y)[idx] = __float2half_rn(f);
