@@ -773,13 +773,19 @@ class FusedNet(object):
             torch.ops.torch_mlu.set_launch_sharing(max(before, 1))
 
     def _parts(self, parts, n, c, h, w):
-        """How many of the `parts` asked for pay.  A graph that is one chain of launches runs them back to back; one with
-        parallel branches is fed node by node, 4.0 to 4.3 us each (MobileNetV2 at 192 x 192, two parts: 426 us for 4 images
-        and 431 us for 27), so the batch has to keep the device busy for longer than that: its time as one chain -- 2.6 us
-        per launch + 0.65 us per million output elements + 1.76 us per billion int8 multiply-accumulates, fitted to
-        ResNet-50 and MobileNetV2 at batches of 64 and 128 -- less the 7 % that the overlap is worth.  Measured, one / two
-        parts: MobileNetV2 192 x 192, 27 images 277 / 431 us, 128 images 617 / 569; ResNet-50 224 x 224, 8 images
-        350 / 382 us, 16 447 / 451, 24 565 / 546, 64 1044 / 972; ResNet-18, 32 images 354 / 366, 64 571 / 548."""
+        """How many of the `parts` asked for pay.  A part's launches fill the compute units that the other part's leave idle,
+        but each does less work for the same start-up: few pixels per launch are faster as one chain.  The work that sets the
+        two apart -- 2.6 us per launch + 0.85 us per million output elements + 1.2 us per billion int8 multiply-accumulates
+        -- has to reach 3.7 us per launch of the graph; the weights are those that put the measured cases on the right side,
+        not a forecast of the time (which is 1 to 2 times as long).  Measured, one part / two (us), the smaller a batch that
+        is left as one, the larger one that is split:
+          MobileNetV2 224 x 224, 32 images 332 / 343, 48 436 / 419, 64 502 / 472; 192 x 192, 27 279 / 291, 64 430 / 413
+          ResNet-50 224 x 224, 8 images 346 / 407, 20 528 / 504, 64 1074 / 992; 112 x 112, 64 457 / 468
+          ResNet-18 224 x 224, 16 images 244 / 252, 40 472 / 422; 112 x 112, 64 264 / 272
+          Darknet-53 416 x 416, 3 images 1087 / 1142, 5 1318 / 1257; 320 x 320, 4 1056 / 1087, 8 1302 / 1237
+        Near the line it is off by up to 2 % (ResNet-18, 32 images, split: 345 / 349; MobileNetV2, 40, not: 397 / 390).  These
+        are with the branches on hardware queues of their own; where the streams that a process made before put both on one,
+        each node takes 4 us (MobileNetV2 192 x 192, 27 images, two parts: 431) and a long graph is up to a third slower."""
         if parts == 1:
             return 1
         size, launches, elems, macs = {"input": (h, w)}, 0, 0, 0
@@ -798,8 +804,8 @@ class FusedNet(object):
             if l.kind in ("conv", "fc"):
                 elems += n * hi * wi * l.co
                 macs += n * hi * wi * l.co * (l.ci // (l.groups or 1)) * (l.k or 1) ** 2 * (2 if self.q[l.name].bw_x == 16 else 1)
-        chain_us = 2.6 * launches + 0.65e-6 * elems + 1.76e-9 * macs
-        while parts > 1 and 0.93 * chain_us < 4.2 * launches * parts:
+        work_us = 2.6 * launches + 0.85e-6 * elems + 1.2e-9 * macs
+        while parts > 1 and work_us < 3.7 * launches * parts:
             parts -= 1
         return parts
 
