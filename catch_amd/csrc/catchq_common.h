@@ -251,6 +251,33 @@ __device__ __forceinline__ float epi_value(float facc, int64_t idx, int c, const
   return v;
 }
 
+// The same for a lane that finishes many rows of one channel: the channel's constants are read once, the division goes
+// through the reciprocal where there is one (the same bits).
+struct EpiColumn { float div, rcp, bias; };
+__device__ __forceinline__ EpiColumn epi_column(const EpiDev &e, int c) {
+  return {e.chan_div ? e.chan_div[c] : 1.0f, e.chan_rcp ? e.chan_rcp[c] : 1.0f, e.bias ? bias_value(e, c) : 0.0f};
+}
+__device__ __forceinline__ float epi_value(float facc, int64_t idx, const EpiColumn &k, const EpiDev &e) {
+  float v = __builtin_ldexpf(facc, e.exp2);
+  if (e.half_steps) v = round_f16(v);
+  if (e.chan_rcp) v = div_by_rcp(v, k.div, k.rcp);
+  else if (e.chan_div) {
+    v = v / k.div;
+    if (e.half_steps) v = round_f16(v);
+  }
+  if (e.bias) {
+    v = v + k.bias;
+    if (e.half_steps) v = round_f16(v);
+  }
+  if (e.resid && !e.resid_after) v = v + e.resid[idx];
+  if (e.act == CATCHQ_ACT_LEAKY) v = (v > 0.0f) ? v : v * e.act_slope;
+  else if (e.act >= CATCHQ_ACT_RELU) v = (v > 0.0f) ? v : 0.0f;
+  if (e.act == CATCHQ_ACT_RELU6) v = (v < 6.0f) ? v : 6.0f;
+  if (e.resid && e.resid_after) v = v + e.resid[idx];
+  asm volatile("" : "+v"(v));  // the fp32 value exists: its conversion to fp16 is a rounding of its own
+  return v;
+}
+
 __device__ __forceinline__ void epi_store(float v, int64_t idx, const EpiDev &e) {
   if (e.y) {
     if (e.y_f16) reinterpret_cast<__half *>(e.y)[idx] = __float2half_rn(v);

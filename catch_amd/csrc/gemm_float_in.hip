@@ -122,7 +122,8 @@ __global__ __launch_bounds__(256) void gemm_float_kernel(const void *__restrict_
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // the slots are dead: staging area
   int *stage = reinterpret_cast<int *>(lds_dyn) + wave * 32 * EPI_STRIDE;
-  igemm_epilogue<1, TN, EPI>(acc, stage, m0 + wave_m * 32, n0 + wave_n * WN, lane, p, e);
+  if constexpr (EPI == EPI_SCALAR) igemm_epilogue_columns<1, TN>(acc, stage, m0 + wave_m * 32, n0 + wave_n * WN, lane, p, e);
+  else igemm_epilogue<1, TN, EPI>(acc, stage, m0 + wave_m * 32, n0 + wave_n * WN, lane, p, e);
 }
 
 template <int IN, int BN>

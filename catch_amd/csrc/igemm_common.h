@@ -589,6 +589,42 @@ __device__ __forceinline__ void igemm_epilogue(v16i (&acc)[TM][TN], int *stage, 
   }
 }
 
+// Epilogue of one wave for rows of any length and alignment, through the wave's staging area (32 * (TN*32 + 8) ints): a lane
+// keeps its columns, so their constants are read once and a store is a run of a row.  The loop is rolled: straight-line code
+// for every accumulator, as EPI_SCALAR has it above, is 30 KB of divisions and branches that a short launch waits for
+// (1089 x 16 -> 126 in one launch 16.0 us with it).
+template <int TM, int TN>
+__device__ __forceinline__ void igemm_epilogue_columns(v16i (&acc)[TM][TN], int *stage, int64_t m_w, int n_w, int lane,
+                                                       const IgemmParams &p, const EpiDev &e) {
+  constexpr int WN = TN * 32, EPI_STRIDE = WN + 8;
+  constexpr int LC = WN < 64 ? WN : 64, RPI = 64 / LC;  // lanes along a row, rows a wave handles at once
+  const int frow = lane & 31, fhalf = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    // wave-private staging: stores then loads of the same wave, ordered by the LDS counter
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        stage[(8 * (r >> 2) + 4 * fhalf + (r & 3)) * EPI_STRIDE + j * 32 + frow] = acc[i][j][r];
+    const int64_t left = p.M - (m_w + i * 32);
+    const int rows = left < 0 ? 0 : (left > 32 ? 32 : (int)left);
+#pragma unroll 1
+    for (int c = lane % LC; c < WN; c += LC) {
+      const int n = n_w + c;
+      if (n >= p.N) break;
+      const EpiColumn k = epi_column(e, n);
+#pragma unroll 2
+      for (int row = lane / LC; row < rows; row += RPI) {
+        const int a = stage[row * EPI_STRIDE + c];
+        const int64_t idx = (m_w + i * 32 + row) * out_ld(p) + n;
+        if (e.acc_out) e.acc_out[idx] = a;
+        epi_store(epi_value((float)a, idx, k, e), idx, e);
+      }
+    }
+  }
+}
+
 // 16 consecutive int16 (two 16-byte chunks) -> their high bytes and their biased low bytes
 __device__ __forceinline__ void split_i16(const v4i c0, const v4i c1, v4i &hi, v4i &lo) {
   hi[0] = (int)__builtin_amdgcn_perm((unsigned)c0[1], (unsigned)c0[0], 0x07050301u);
