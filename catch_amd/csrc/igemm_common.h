@@ -233,6 +233,20 @@ __device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, c
   return L;
 }
 
+// the same from vectors of any alignment and length N (channels beyond it: the last one's constants)
+template <class S>
+__device__ __forceinline__ EpiLane epi_lane_setup_ragged(int n, int N, const EpiDev &e) {
+  v4f div, rcp, bias;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int c = min(n + t, N - 1);
+    div[t] = e.chan_div ? e.chan_div[c] : 1.0f;
+    rcp[t] = e.chan_rcp ? e.chan_rcp[c] : 1.0f;
+    bias[t] = e.bias ? bias_value(e, c) : -0.0f;
+  }
+  return epi_lane_finish<S>(div, rcp, bias, e);
+}
+
 template <class S>
 __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev &e) {
   v4f div = {1.f, 1.f, 1.f, 1.f}, rcp = {1.f, 1.f, 1.f, 1.f}, bias = {-0.f, -0.f, -0.f, -0.f};
@@ -294,6 +308,25 @@ struct EpiAtSplit {
   template <class T> __device__ __forceinline__ T *at(T *base) const { return (base + uni) + off; }
 };
 
+// Rows of any length and alignment: four channels of which the first `left` exist (floating outputs only).
+struct EpiAtRagged {
+  int64_t idx;
+  int left;
+  template <class T> __device__ __forceinline__ T *at(T *base) const { return base + idx; }
+};
+// four elements at once (global memory takes any element's alignment), one by one at the end of a row
+template <class T, class V>
+__device__ __forceinline__ void store_ragged(T *dst, const V v, int left) {
+  typedef T vec_t __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+  if (left >= 4) {
+    *reinterpret_cast<vec_t *>(dst) = __builtin_bit_cast(vec_t, v);
+  } else {
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+      if (t < left) dst[t] = v[t];
+  }
+}
+
 // A store / load with or without the non-temporal hint, chosen by a wave-uniform flag.  The empty volatile
 // statements keep the two branches apart: merged into one access, they would lose the hint.
 template <class T>
@@ -345,10 +378,16 @@ __device__ __forceinline__ void epi_vec4(const Sums a, const v4f res, const EpiL
     typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
     const f16x2 h01 = __builtin_convertvector(f32x2{v[0], v[1]}, f16x2), h23 = __builtin_convertvector(f32x2{v[2], v[3]}, f16x2);
     const v2i packed = {__builtin_bit_cast(int, h01), __builtin_bit_cast(int, h23)};
-    store_stream(reinterpret_cast<v2i *>(where.at(reinterpret_cast<__half *>(e.y))), packed, e.y_stream != 0);
+    if constexpr (std::is_same<At, EpiAtRagged>::value) {
+      typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+      store_ragged(where.at(reinterpret_cast<_Float16 *>(e.y)), __builtin_bit_cast(f16x4, packed), where.left);
+    } else
+      store_stream(reinterpret_cast<v2i *>(where.at(reinterpret_cast<__half *>(e.y))), packed, e.y_stream != 0);
   } else if (S::y32(e)) {
     v4f o = {v[0], v[1], v[2], v[3]};
-    store_stream(reinterpret_cast<v4f *>(where.at(reinterpret_cast<float *>(e.y))), o, e.y_stream != 0);
+    if constexpr (std::is_same<At, EpiAtRagged>::value) store_ragged(where.at(reinterpret_cast<float *>(e.y)), o, where.left);
+    else
+      store_stream(reinterpret_cast<v4f *>(where.at(reinterpret_cast<float *>(e.y))), o, e.y_stream != 0);
   }
   if constexpr (S::kFoldScale) {
     // v is already in units of the output's step: clamp to 0 .. min(127, 6 / step) (the median maps a NaN to 0, as
