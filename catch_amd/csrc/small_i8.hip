@@ -361,7 +361,9 @@ static bool small_side(SmallSide *o, const void *x, int x_size, const void *w, i
 //   32 x 32 tiles up to one per unit: 784 x 256 x 512 3.4 / 3.7, 4 x 14x14 256->256 3x3 (200 tiles) 5.3 / 7.7
 //     (K = 192 ties, K <= 128 loses: those launches are all set-up); to 1.75 per unit from K = 1024 on
 //     (4 x 28x28 128->128 3x3, 392 tiles, 5.4 / 6.0; K = 512 loses, 4.3 / 3.7); more for the longest K
-//     (197 x 4096 x 4096, 896 tiles, 13.8 / 16.8)
+//     (197 x 4096 x 4096, 896 tiles, 13.8 / 16.8), up to three per unit where there are more rows (with a quantizer in
+//     front: 2048 x 3072 x 384, 768 tiles, 18.4 / 19.4, but 784 x 3072 x 1120, 875 tiles, 18.7 / 17.8 and
+//     2048 x 3072 x 416, 832 tiles, 20.5 / 19.7)
 // Four waves share K (one wave's transfers and arithmetic run under another's wait; eight cost more set-up than they
 // hide), eight where a step's tap arithmetic is long and the blocks do not fill the device.
 static int small_plan(int64_t M, int64_t N, int64_t K, bool dense, int cus) {
@@ -370,7 +372,7 @@ static int small_plan(int64_t M, int64_t N, int64_t K, bool dense, int cus) {
   int plan = 0;
   if (tiles16 <= 2 * cus && K >= 64)
     plan = (!dense && steps >= 16 && tiles16 <= cus) ? 1608 : 1604;
-  else if ((tiles32 <= cus && K >= 256) || (tiles32 * 4 <= 7 * cus && K >= 1024) || (tiles32 * 2 <= 7 * cus && K >= 3072))
+  else if ((tiles32 <= cus && K >= 256) || (tiles32 * 4 <= 7 * cus && K >= 1024) || (tiles32 * 2 <= (M <= 512 ? 7 : 6) * cus && K >= 3072))
     plan = (!dense && steps >= 32 && tiles32 <= cus) ? 3208 : 3204;
   if (const char *f = tuning_env("CATCHQ_SMALL")) plan = std::atoi(f);
   return plan;
