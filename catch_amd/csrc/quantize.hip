@@ -94,7 +94,8 @@ static int launch_quantize(const void *x, void *q, int64_t n, int pos, float sca
   typedef typename QRange<BW>::type TQ;
   constexpr int VEC = 16 / sizeof(TIn);
   if (aligned16(x) && aligned16(q)) {
-    // one vector per lane until the device is full: a lane's loads follow each other
+    // one vector per lane up to the grid's limit (4.2 M fp32 values), whose lanes walk on from there: a lane's loads follow
+    // each other
     quantize_vec_kernel<TIn, BW><<<grid_for(n / VEC, kThreads), kThreads, 0, s>>>(
         (const TIn *)x, (TQ *)q, n, pos, scale, pos_dev, scale_dev);
   } else {
