@@ -1,6 +1,7 @@
 """GPU parity: every HIP kernel, called through the C ABI, against the CPU oracle on the same
 seeded inputs.  Bit-exact for integer outputs; floating outputs are compared bit-exactly too
 where the oracle fixes the operation order, and within 1e-3 of the output range otherwise."""
+import ctypes
 import sys
 
 import numpy as np
@@ -400,6 +401,53 @@ def test_floating_activations_few_columns(m, k, n, dtype):
                                     q_bw=8, q_pos=-3)
     y = orc.epilogue(acc, -10, div, bias, None, 1)
     assert same_bits(y, out["y"].cpu().numpy()) and same_bits(orc.quantize(y, 8, -3), out["q"].cpu().numpy())
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("m,k,n", [(1089, 16, 126), (4097, 64, 65), (4160, 144, 129), (12225, 272, 255), (1030, 80, 510)])
+def test_floating_activations_ragged_columns(m, k, n, dtype):
+    """one launch with output channels not a multiple of four, columns in the second half of a wave's tile and in a second
+    tile: floating outputs with a true and a reciprocal-form division, without divisors, requantized outputs"""
+    note("floating activations, ragged columns", m, k, n, dtype)
+    r = rng(m + k + n)
+    x, wt = (r.standard_normal((1, m, 1, k)) * 2).astype(dtype), _ints(r, (n, 1, 1, k), 8)
+    div, bias = r.uniform(0.6, 3.5, n).astype(np.float32), r.standard_normal(n).astype(np.float32)
+    acc, ovf = orc.conv2d_nhwc(orc.quantize(x, 8, -5), wt, (0, 0), (1, 1), (1, 1), 1)
+    assert ovf == 0
+    for use_div, use_rcp, use_bias, act, y_dtype, q_bw in ((True, True, True, 0, torch.float32, 0), (True, False, True, 0, torch.float16, 0),
+                                                           (False, False, False, 2, torch.float32, 8), (True, True, False, 1, torch.float16, 16)):
+        y = orc.epilogue(acc, -10, div if use_div else None, bias if use_bias else None, None, act)
+        out, ws = cabi.float_conv2d_nhwc(cabi.dev(x), -5, cabi.dev(wt), exp2=-10, chan_div=cabi.dev(div) if use_div else None,
+                                         chan_rcp=cabi.dev(np.float32(1) / div) if use_rcp else None,
+                                         bias=cabi.dev(bias) if use_bias else None, act=act, y_dtype=y_dtype, q_bw=q_bw, q_pos=-3)
+        assert ws == 0 and same_bits(y if y_dtype == torch.float32 else y.astype(np.float16), out["y"].cpu().numpy())
+        if q_bw:
+            assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
+
+
+@pytest.mark.parametrize("y_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("m,k,n", [(1, 64, 1), (33, 72, 2), (65, 200, 3), (130, 64, 5), (31, 1000, 63), (200, 136, 66), (97, 320, 127),
+                                   (4100, 64, 146), (12000, 40, 131)])
+def test_int16_rows_of_any_length(m, k, n, y_dtype):
+    """int16 x int16 with output channels not a multiple of four (and rows of aligned length at an unaligned address): four
+    channels finished together, the end of a row one by one, nothing written behind the last row"""
+    note("int16, rows of any length", m, k, n, y_dtype)
+    r = rng(m + k + n)
+    a, b = _ints(r, (m, k), 16), _ints(r, (n, k), 16)
+    div, bias = r.uniform(0.6, 3.5, n).astype(np.float32), r.standard_normal(n).astype(np.float32)
+    acc, _ = orc.gemm_nt(a, b)
+    for use_div, use_rcp, use_bias in ((True, True, True), (True, False, True), (False, False, False), (True, True, False)):
+        e, _ = cabi._epilogue((m, n), "cuda", -26, None, None, None, 0, None, False, 0, 0, 1.0)
+        keep = cabi.dev(div), cabi.dev(np.float32(1) / div), cabi.dev(bias)  # (alive until the launch has run)
+        e.chan_div, e.chan_rcp, e.bias = (cabi.ptr(t) if u else None for t, u in zip(keep, (use_div, use_rcp, use_bias)))
+        whole = torch.full((m * n + 8,), 7.0, dtype=y_dtype, device="cuda")
+        e.y, e.y_dtype = cabi.ptr(whole[1:]), int(y_dtype == torch.float16)
+        da, db = cabi.dev(a), cabi.dev(b)
+        cabi.check(cabi.lib().catchq_gemm_nt(cabi.ptr(da), 16, cabi.ptr(db), 16, m, n, k, ctypes.byref(e), cabi.stream()))
+        y = orc.epilogue(acc, -26, div if use_div else None, bias if use_bias else None)
+        got = whole.cpu().numpy()
+        assert same_bits(y if y_dtype == torch.float32 else y.astype(np.float16), got[1:m * n + 1].reshape(m, n))
+        assert got[0] == 7 and (got[m * n + 1:] == 7).all()
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
