@@ -187,9 +187,8 @@ __device__ __forceinline__ v4f half4_values(const v2i bits) {
   typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
   return __builtin_convertvector(__builtin_bit_cast(f16x4, bits), v4f);
 }
-// A bias of four consecutive channels (n a multiple of four), of either precision: the bits as they lie in memory, and
-// their values later.  A conversion beside the load would wait for it there, in front of a K loop in one kernel.
-// (One load and a conditional one: a branch to either load measured the same or slower.)
+// A bias of four consecutive channels (n a multiple of four), of either precision.  (One load and a conditional one: a branch
+// to either load measured the same or slower.)
 struct Bias4 {
   v2i lo = {kNoBias, kNoBias}, hi = {kNoBias, kNoBias};  // halfs: all four in lo
   static constexpr int kNoBias = (int)0x80000000u;       // -0: x + -0 = x
@@ -199,10 +198,9 @@ struct Bias4 {
     lo = *reinterpret_cast<const v2i *>(at);
     if (!e.bias_f16) hi = *reinterpret_cast<const v2i *>(at + 8);
   }
-  __device__ __forceinline__ v4f wide_values() const {
-    return __builtin_bit_cast(v4f, v4i{lo[0], lo[1], hi[0], hi[1]});
+  __device__ __forceinline__ v4f values(const EpiDev &e) const {
+    return e.bias_f16 ? half4_values(lo) : __builtin_bit_cast(v4f, v4i{lo[0], lo[1], hi[0], hi[1]});
   }
-  __device__ __forceinline__ v4f values(const EpiDev &e) const { return e.bias_f16 ? half4_values(lo) : wide_values(); }
 };
 
 // The lane's constants from the raw values of its four channels (1 / 1 / -0 where a constant is absent).

@@ -57,7 +57,8 @@ __device__ __forceinline__ void small_ds_write(unsigned addr, v4i v) {
 // DENSE: a plain GEMM -- row m starts at m * K, no taps.  IN: type of the activations.  DUAL: a residual block's last
 // convolution and its projection shortcut over the same output tile; the block's waves are shared out between the two
 // in proportion to their K steps, and the shortcut's sums, dequantized with its own constants, are the residual.
-template <int T, int NW, bool DENSE, int IN, bool DUAL>
+// HALF_BIAS: there is a bias, in half precision (a choice at run time costs every launch 0.05 us).
+template <int T, int NW, bool DENSE, int IN, bool DUAL, bool HALF_BIAS>
 __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev e) {
   resolve_exp2(e);
   constexpr int SLOTS = 2, BKB = 128;
@@ -88,7 +89,8 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   const bool vec = p.epi != EPI_SCALAR;
   constexpr int ROUNDS = (EPI_LANES + 64 * NW - 1) / (64 * NW);
   v4f c_div = {1.f, 1.f, 1.f, 1.f}, c_rcp = c_div, c_res[ROUNDS];
-  Bias4 c_bias;
+  v4f c_bias = {-0.f, -0.f, -0.f, -0.f};
+  v2i c_bias16 = {0, 0};  // (converted behind the K loop: here the conversion would wait for the load)
   v4f s_div = c_div, s_rcp = c_div, s_bias = {0.f, 0.f, 0.f, 0.f};  // the shortcut's constants
   // 64 * NW is a multiple of CPR: a lane has the same four channels in every round.  (Plain loads: the transfers below
   // and the statements that clobber memory keep them here, in front of the K loop.)
@@ -98,7 +100,8 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     if (e.chan_div) c_div = *reinterpret_cast<const v4f *>(e.chan_div + cc);
     const float *rcps = e.chan_rcp ? e.chan_rcp : e.half_rcp;
     if (rcps) c_rcp = *reinterpret_cast<const v4f *>(rcps + cc);
-    c_bias.load(e, cc);
+    if constexpr (HALF_BIAS) c_bias16 = *reinterpret_cast<const v2i *>(reinterpret_cast<const __half *>(e.bias) + cc);
+    else if (e.bias) c_bias = *reinterpret_cast<const v4f *>(e.bias + cc);
     if constexpr (DUAL) {
       if (p.sc.chan_div) s_div = *reinterpret_cast<const v4f *>(p.sc.chan_div + cc);
       if (p.sc.chan_rcp) s_rcp = *reinterpret_cast<const v4f *>(p.sc.chan_rcp + cc);
@@ -286,7 +289,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     }
     auto run = [&](auto spec) {
       typedef decltype(spec) S;
-      EpiLane L = epi_lane_finish<S>(c_div, c_rcp, S::kAnyBias || S::kHalfBias ? c_bias.values(e) : c_bias.wide_values(), e);
+      EpiLane L = epi_lane_finish<S>(c_div, c_rcp, HALF_BIAS ? half4_values(c_bias16) : c_bias, e);
       if constexpr (DUAL) {
         L.use_res = true;
         L.res_after = e.resid_after != 0;
@@ -311,11 +314,11 @@ static void magic(unsigned d, unsigned *m, unsigned *mask) {
   *mask = d <= 1 ? ~0u : 0u;
 }
 
-template <int T, int NW, bool DENSE, int IN, bool DUAL>
+template <int T, int NW, bool DENSE, int IN, bool DUAL, bool HALF_BIAS>
 static int launch_small(SmallParams p, const EpiDev &e, hipStream_t s) {
   constexpr int LDS_BYTES = NW * 2 * 2 * T * 128;
   static_assert(LDS_BYTES <= 128 * 1024, "slots of all waves");
-  auto kern = small_i8_kernel<T, NW, DENSE, IN, DUAL>;
+  auto kern = small_i8_kernel<T, NW, DENSE, IN, DUAL, HALF_BIAS>;
   if (LDS_BYTES > 64 * 1024) {
     static std::atomic<bool> raised[64];
     if (raise_lds_limit((const void *)kern, LDS_BYTES, raised) != CATCHQ_OK) return CATCHQ_ERR_LAUNCH;
@@ -378,15 +381,23 @@ static int small_plan(int64_t M, int64_t N, int64_t K, bool dense, int cus) {
   return plan;
 }
 
-template <bool DENSE, int IN, bool DUAL>
-static int launch_small_plan(int plan, const SmallParams &p, const EpiDev &e, hipStream_t s) {
+template <bool DENSE, int IN, bool DUAL, bool HALF_BIAS>
+static int launch_small_bias(int plan, const SmallParams &p, const EpiDev &e, hipStream_t s) {
   switch (plan) {
-    case 3204: return launch_small<32, 4, DENSE, IN, DUAL>(p, e, s);
-    case 3208: return launch_small<32, 8, DENSE, IN, DUAL>(p, e, s);
-    case 1604: return launch_small<16, 4, DENSE, IN, DUAL>(p, e, s);
-    case 1608: return launch_small<16, 8, DENSE, IN, DUAL>(p, e, s);
+    case 3204: return launch_small<32, 4, DENSE, IN, DUAL, HALF_BIAS>(p, e, s);
+    case 3208: return launch_small<32, 8, DENSE, IN, DUAL, HALF_BIAS>(p, e, s);
+    case 1604: return launch_small<16, 4, DENSE, IN, DUAL, HALF_BIAS>(p, e, s);
+    case 1608: return launch_small<16, 8, DENSE, IN, DUAL, HALF_BIAS>(p, e, s);
     default: return -1;
   }
+}
+
+template <bool DENSE, int IN, bool DUAL>
+static int launch_small_plan(int plan, const SmallParams &p, const EpiDev &e, hipStream_t s) {
+  if constexpr (!DUAL) {
+    if (e.bias_f16) return launch_small_bias<DENSE, IN, DUAL, true>(plan, p, e, s);
+  }
+  return launch_small_bias<DENSE, IN, DUAL, false>(plan, p, e, s);
 }
 
 static void small_common(SmallParams *p, int64_t M, int Co, int Ho, int Wo, const EpiDev &pick) {
