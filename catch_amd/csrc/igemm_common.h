@@ -60,7 +60,7 @@ inline bool vec_epilogue_ok(int N, const EpiDev &e) {
 // EpiDev (the generic instance); fixed fields let the compiler drop every untaken branch, which
 // matters because the epilogue is VALU-bound (about a dozen fp32 operations per output element).
 //   DIV  0 none, 1 reciprocal form (the constants of a launch without divisors or bias are 1 and -0: nothing changes), 2 true
-//   division, 3 reciprocal form with every step rounded to binary16 (half_steps)      BIAS 0 none, 1 yes, 2 half or none     RESID 0 none, 1 before, 2 after the activation
+//   division, 3 reciprocal form with every step rounded to binary16 (half_steps)      BIAS 0/1     RESID 0 none, 1 before, 2 after the activation
 //   ACT  CATCHQ_ACT_*       YM  0 none, 1 fp32, 2 fp16     QM  0 none, 8, 16     ACC 0/1
 template <int DIV, int BIAS, int RESID, int ACT, int YM, int QM, int ACC>
 struct EpiSpec {
@@ -68,9 +68,8 @@ struct EpiSpec {
   static constexpr bool kSteps = DIV == 3;
   static constexpr int kAct = ACT;
   static constexpr int kQ = QM;
-  // the other instances of layers with a floating output and nothing else read a bias of either precision
-  static constexpr bool kHalfBias = BIAS == 2;
-  static constexpr bool kAnyBias = DIV < 0 || (BIAS == 1 && QM == 0 && RESID == 0);
+  // the instances of layers with a floating output and nothing else read a bias of either precision
+  static constexpr bool kAnyBias = DIV < 0 || (QM == 0 && RESID == 0);
   // ReLU / ReLU6 feeding nothing but an int8 requantization: the activation folds into the clamp of the
   // quantizer, 0 <= x <= min(6, 127 * 2^pos)
   static constexpr bool kFoldAct = DIV >= 0 && QM == 8 && YM == 0 && ACC == 0 && RESID != 2 &&
@@ -84,7 +83,7 @@ struct EpiSpec {
   static __device__ __forceinline__ bool truediv(const EpiDev &e) {
     return DIV < 0 ? (e.chan_div != nullptr && e.chan_rcp == nullptr) : DIV == 2;
   }
-  static __device__ __forceinline__ bool bias(const EpiDev &e) { return BIAS < 0 ? e.bias != nullptr : BIAS >= 1; }
+  static __device__ __forceinline__ bool bias(const EpiDev &e) { return BIAS < 0 ? e.bias != nullptr : BIAS == 1; }
   static __device__ __forceinline__ bool resid(const EpiDev &e) { return RESID < 0 ? e.resid != nullptr : RESID >= 1; }
   static __device__ __forceinline__ bool resid_after(const EpiDev &e) { return RESID < 0 ? e.resid_after != 0 : RESID == 2; }
   static __device__ __forceinline__ int act(const EpiDev &e) { return ACT < 0 ? e.act : ACT; }
@@ -128,7 +127,7 @@ template <> struct EpiOf<EPI_Y32> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_NONE, 1,
 template <> struct EpiOf<EPI_RES_Y> { typedef EpiSpec<1, 1, 1, CATCHQ_ACT_RELU, 1, 0, 0> type; };
 template <> struct EpiOf<EPI_Y16_RELU> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_RELU, 2, 0, 0> type; };
 template <> struct EpiOf<EPI_Y16> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_NONE, 2, 0, 0> type; };
-template <> struct EpiOf<EPI_Y16_STEPS> { typedef EpiSpec<3, 2, 0, CATCHQ_ACT_NONE, 2, 0, 0> type; };
+template <> struct EpiOf<EPI_Y16_STEPS> { typedef EpiSpec<3, 1, 0, CATCHQ_ACT_NONE, 2, 0, 0> type; };
 template <> struct EpiOf<EPI_Q8_RELU6> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_RELU6, 0, 8, 0> type; };
 template <> struct EpiOf<EPI_RES_Q8> { typedef EpiSpec<1, 1, 1, CATCHQ_ACT_RELU, 0, 8, 0> type; };
 template <> struct EpiOf<EPI_LIN_Q8> { typedef EpiSpec<1, 1, 0, CATCHQ_ACT_NONE, 0, 8, 0> type; };
@@ -167,9 +166,6 @@ inline int pick_epilogue(int N, const EpiDev &e) {
       {EPI_LK_Y_Q16, 0, 1, 0, CATCHQ_ACT_LEAKY, 1, 16},     {EPI_LK_RESA_Q16, 0, 1, 2, CATCHQ_ACT_LEAKY, 0, 16},
       {EPI_LK_RESA_Y_Q16, 0, 1, 2, CATCHQ_ACT_LEAKY, 1, 16}, {EPI_Y16, 1, 1, 0, CATCHQ_ACT_NONE, 2, 0},
       {EPI_Y16_STEPS, 3, 1, 0, CATCHQ_ACT_NONE, 2, 0}};
-  // The step-rounding instance takes a half bias, which is what a half layer has: in ResNet-50 at 32 images its one-launch
-  // pointwise layers take 16.6 us so and 16.75 with a choice at run time, its 64 x 64 tiles 11.4 and 11.9.
-  if (div == 3 && e.bias && !e.bias_f16) return EPI_VECTOR;
   for (const auto &r : rows)
     if ((r.div == div || (r.div == 1 && ones)) && (r.bias == bias || bias == 0) && r.res == res && r.act == e.act && r.ym == ym && r.qm == qm) return r.epi;
   return EPI_VECTOR;
@@ -251,11 +247,7 @@ __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev
   const float *rcps = S::kSteps ? e.half_rcp : e.chan_rcp;
   if (n_ok && (S::rcp(e) || S::truediv(e) || S::kSteps) && e.chan_div) div = *reinterpret_cast<const v4f *>(e.chan_div + n);
   if (n_ok && (S::rcp(e) || S::kSteps) && rcps) rcp = *reinterpret_cast<const v4f *>(rcps + n);
-  if constexpr (S::kHalfBias) {
-    v2i h = {(int)0x80008000u, (int)0x80008000u};
-    if (n_ok && e.bias) h = *reinterpret_cast<const v2i *>(reinterpret_cast<const __half *>(e.bias) + n);
-    bias = half4_values(h);
-  } else if constexpr (S::kAnyBias) {
+  if constexpr (S::kAnyBias) {
     Bias4 b;
     if (n_ok && S::bias(e)) b.load(e, n);
     bias = b.values(e);
@@ -269,12 +261,12 @@ __device__ __forceinline__ EpiLane epi_lane_setup(int n, bool n_ok, const EpiDev
 __device__ __forceinline__ float epi_dequant1(float x, int t, const EpiLane &L, int exp2) {
   if (L.steps_rcp) {
     // fp32 operations on binary16 values rounded to binary16 are the binary16 operations.  The reciprocal form gives the
-    // correctly rounded fp32 quotient of the finite values; an infinite one (the scaled sum overflowed) stays infinite, and
-    // a zero keeps its sign, which the correction step would make positive.
+    // correctly rounded fp32 quotient of the finite values; an infinite one (the scaled sum overflowed) stays infinite.  The
+    // residual is taken as q d - x and subtracted: a zero quotient then keeps its sign (x - q d would be +0 and make -0 positive).
     x = round_f16(__builtin_ldexpf(x, exp2));
     const float q = x * L.rcp[t];
-    float v = __builtin_fmaf(__builtin_fmaf(-q, L.div[t], x), L.rcp[t], q);
-    v = __builtin_amdgcn_classf(q, 0x264) ? q : v;  // -inf, -0, +0, +inf
+    float v = __builtin_fmaf(-__builtin_fmaf(q, L.div[t], -x), L.rcp[t], q);
+    v = __builtin_isinf(q) ? q : v;
     asm volatile("" : "+v"(v));  // keeps the conversion below apart: fused into one operation it would round once
     return round_f16(v) + L.bias[t];  // (rounded to binary16 by the conversion of the output)
   }
