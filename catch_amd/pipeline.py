@@ -212,7 +212,6 @@ class FusedNet(object):
         self.q = {l.name: _decode(l, state_dict, self.device, self.cdev[l.src], self.cdev[l.name], fractional_scale)
                   for l in self.layers if l.kind in ("conv", "fc")}
         self._plan_demands()
-        self._graph = None
         self.graph_parts = 0  # of the graph captured last
         # A few-channel int8 network input feeding one k x k convolution: quantize it into a zero frame
         # (the convolution's padding, materialised) and pad the filter rows to whole groups of 4 taps,
@@ -749,7 +748,9 @@ class FusedNet(object):
         leave idle while they start up and drain.  A batch whose launches are too short for that is recorded as fewer
         parts (_parts): `streams` is the most there may be.
         parts: record exactly this many, whatever `streams` says and whether they pay or not.
-        graph_parts holds the number recorded."""
+        graph_parts holds the number recorded.
+        replay owns the graph and its memory: dropping it gives both back (the plan keeps no graph, so recording another
+        one destroys none)."""
         static_in = example.clone()
         if parts is None:
             asked = max(1, min(int(streams), static_in.shape[0]))
@@ -848,7 +849,6 @@ class FusedNet(object):
                 for st in side:
                     cur.wait_stream(st)
                 static_out = tuple(whole) if isinstance(sample, tuple) else whole[0]
-        self._graph = graph
         # the first replays of a new graph are slower (the executable graph is uploaded on first use): take them here
         for _ in range(8):
             graph.replay()
