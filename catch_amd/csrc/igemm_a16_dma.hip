@@ -24,9 +24,22 @@
 // position per lane, leaves a two-way bank conflict on the A fetches).
 // Darknet-53 with 416x416 images, batch 16: 2473 -> 2296 us with the uniform loader and the weight sums
 // shared out between the two waves of a column.
+//
+// What a launch of few blocks per unit is bound by is a step's chain (barrier, LDS reads, digit split, matrix
+// instructions) and the set-up in front of the first transfer.  Without branches between a step's transfers, with the
+// barrier in the middle of a step's multiplications (the next fragments arrive under them) and with the validity of a
+// tap decided when the tap is entered instead of up front: 800 -> 570 clocks a step, 6500 -> 2500 clocks of set-up;
+// 3 x 3 layers, us: 8 x 13 x 13, 512 -> 1024 channels 33.9 -> 30.2, 8 x 26 x 26, 256 -> 512 29.8 -> 27.5, 8 x 52 x 52,
+// 128 -> 256 30.5 -> 28.8, 1 x 26 x 26 18.2 -> 13.2.
 #include "igemm_i8_dma.inc"
 
 namespace catchq {
+
+// one 1 KiB transfer of a wave; base, bytes, dst and soff are wave-uniform
+__device__ __forceinline__ void dma_to_lds(void *base, int bytes, int8_t *dst, unsigned voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(__builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000), (lds_ptr_t)dst, 16,
+                                           (int)voff, soff, 0, 0);
+}
 
 template <int BM, int BN, int WAVES_M, int WAVES_N, int STAGES, int LOAD, bool UNIFORM, int EPI>
 __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(const int16_t *__restrict__ A,
@@ -66,9 +79,11 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   // B instruction: 16 tile rows x 4 chunks (lane -> row lane/4, physical chunk lane%4).
   unsigned rowbase[NI];  // byte offset of the row's K origin
   unsigned vmask[NI];    // A: bit t = filter tap t inside the image; B / plain GEMM: bit 0 = row exists
+  int hi0[NI], wi0[NI];  // UNIFORM convolution: image position of tap 0 (vmask: the row exists)
 #pragma unroll
   for (int j = 0; j < NI; ++j) {
     const int slot = wave * NI + j;
+    hi0[j] = wi0[j] = 0;
     if (slot < NIA) {
       const int64_t m = m0 + slot * 8 + (lane >> 3);
       const bool ok = m < p.M;
@@ -80,14 +95,10 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
         const int wo = (int)(mu - t * (unsigned)p.Wo);
         const unsigned img = t / (unsigned)p.Ho;
         const int ho = (int)(t - img * (unsigned)p.Ho);
-        const int hi0 = ho * p.sh - p.ph, wi0 = wo * p.sw - p.pw;
-        rowbase[j] = 2u * ((unsigned)((int64_t)img * p.H * p.W * p.Ci) + (unsigned)((hi0 * p.W + wi0) * p.Ci));  // mod 2^32
-        unsigned mask = 0;
-        for (int r = 0; r < p.kh; ++r)
-          for (int q = 0; q < p.kw; ++q)
-            if ((unsigned)(hi0 + r * p.dh) < (unsigned)p.H && (unsigned)(wi0 + q * p.dw) < (unsigned)p.W)
-              mask |= 1u << (r * p.kw + q);
-        vmask[j] = ok ? mask : 0u;
+        hi0[j] = ho * p.sh - p.ph;
+        wi0[j] = wo * p.sw - p.pw;
+        rowbase[j] = 2u * ((unsigned)((int64_t)img * p.H * p.W * p.Ci) + (unsigned)((hi0[j] * p.W + wi0[j]) * p.Ci));  // mod 2^32
+        vmask[j] = !ok ? 0u : (UNIFORM ? 1u : tap_mask(hi0[j], wi0[j], p));
       } else {
         rowbase[j] = (unsigned)(mm * p.K * 2);
         vmask[j] = ok ? 1u : 0u;
@@ -103,19 +114,35 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   }
   // UNIFORM: offsets of the current tap (OOB: the row or the tap does not exist), rebuilt when the tap changes.
   // Operands are smaller than 2 GiB, so an OOB offset stays out of range whatever the scalar adds.
+  // Which operand a transfer serves is the same in every step: its resource and the pace of its scalar offset are chosen
+  // here, once (a choice inside the loop is two taken branches per transfer, ten of them a step).
   unsigned voff[NI];
-  int u_k = 0, u_ci = 0, u_tap = 0, u_r = 0, u_q = 0;  // wave-uniform
+  void *base[NI];                             // wave-uniform, as the rest
+  int bytes[NI], soff[NI], pace[NI], last[NI];
+  int u_k = 0, u_ci = 0, u_r = 0, u_q = 0;
   auto enter_tap = [&]() {
-    const unsigned tapoff = (LOAD == LOAD_CONV) ? 2u * (unsigned)((u_r * p.dh * p.W + u_q * p.dw) * p.Ci) : 0u;
-    const unsigned bit = (LOAD == LOAD_CONV) ? (u_r < p.kh ? 1u << u_tap : 0u) : 1u;  // past the last tap: nothing
+    const int dy = u_r * p.dh, dx = u_q * p.dw;
+    const unsigned tapoff = 2u * (unsigned)((dy * p.W + dx) * p.Ci);
 #pragma unroll
     for (int j = 0; j < NI; ++j)
-      if (wave * NI + j < NIA) voff[j] = select_u32((vmask[j] & bit) != 0, rowbase[j] + tapoff, OOB);
+      if (wave * NI + j < NIA) {
+        const bool in = (vmask[j] != 0) & ((unsigned)(hi0[j] + dy) < (unsigned)p.H) & ((unsigned)(wi0[j] + dx) < (unsigned)p.W);
+        voff[j] = select_u32(in, rowbase[j] + tapoff, OOB);
+        soff[j] = 0;
+      }
   };
   if constexpr (UNIFORM) {
 #pragma unroll
-    for (int j = 0; j < NI; ++j) voff[j] = select_u32(vmask[j] != 0, rowbase[j], OOB);
-    enter_tap();
+    for (int j = 0; j < NI; ++j) {
+      const bool is_a = wave * NI + j < NIA;
+      base[j] = is_a ? (void *)A : (void *)B;
+      bytes[j] = (int)(is_a ? a_bytes : b_bytes);
+      pace[j] = is_a ? 2 * BK : BK;
+      last[j] = is_a ? 2 * (p.Ci - BK) : p.K - BK;
+      soff[j] = 0;
+      voff[j] = select_u32(vmask[j] != 0, rowbase[j], OOB);
+    }
+    if constexpr (LOAD == LOAD_CONV) enter_tap();
   }
   // this lane's position along K, in elements: as a loader of A (8-element chunks) and of B (16)
   int ka_lin = ((lane & 7) ^ (lane >> 3)) * 8;
@@ -134,25 +161,25 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
 
   auto issue_stage = [&](int stage_off) {
     if constexpr (UNIFORM) {
-      const int a_soff = 2 * ((LOAD == LOAD_CONV) ? u_ci : u_k);
 #pragma unroll
-      for (int j = 0; j < NI; ++j) {
-        const int slot = wave * NI + j;
-        lds_ptr_t dst = (lds_ptr_t)(lds_dyn + stage_off + slot * 1024);
-        if (slot < NIA) __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, (int)voff[j], a_soff, 0, 0);
-        else __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, dst, 16, (int)voff[j], u_k, 0, 0);
-      }
-      // past the end of K the offsets stay where they are: a slot that is filled but never read
-      if (u_k + BK < p.K) {
-        u_k += BK;
-        if constexpr (LOAD == LOAD_CONV) {
-          u_ci += BK;
-          if (u_ci == p.Ci) {
-            u_ci = 0;
-            ++u_tap;
-            if (++u_q == p.kw) { u_q = 0; ++u_r; }
-            enter_tap();
-          }
+      for (int j = 0; j < NI; ++j)
+        dma_to_lds(base[j], bytes[j], lds_dyn + stage_off + (wave * NI + j) * 1024, voff[j], soff[j]);
+      // Past the end of K a slot is filled from inside the operand and never read.  (A branch that leaves the offsets where
+      // they are: 0.3 us less on the short loops of 1 x 1 layers; a minimum: 1.3 us of 23 less on 72 steps.)
+      if constexpr (LOAD == LOAD_GEMM) {
+        if (u_k + BK < p.K) {
+          u_k += BK;
+#pragma unroll
+          for (int j = 0; j < NI; ++j) soff[j] += pace[j];
+        }
+      } else {
+#pragma unroll
+        for (int j = 0; j < NI; ++j) soff[j] = min(soff[j] + pace[j], last[j]);
+        u_ci += BK;
+        if (u_ci == p.Ci) {
+          u_ci = 0;
+          if (++u_q == p.kw) { u_q = 0; ++u_r; }
+          enter_tap();
         }
       }
       return;
@@ -239,37 +266,40 @@ __global__ __launch_bounds__(64 * WAVES_M *WAVES_N) void igemm_a16_dma_kernel(co
   };
   static_assert(TM <= 2 && TN <= 2, "wave tile larger than 64x64");
 
-  // both halves are requested up front: the second half's fragments arrive while the first half is multiplied
-  auto compute = [&](unsigned stage_off, int refill_off) {
-    constexpr int NF = 2 * TM + TN;  // LDS reads per half
-    v4i fa0[TM][2], fb0[TN], fa1[TM][2], fb1[TN];
-    fetch_half(fa0, fb0, a_row + stage_off, a_c0, b_row + stage_off + b_k0);
-    fetch_half(fa1, fb1, a_row + stage_off, a_c0 ^ 64u, b_row + stage_off + b_k1);
-    issue_stage(refill_off);
+  auto arrived = [&](v4i (&fa)[TM][2], v4i (&fb)[TN], auto behind_c) {  // but for the reads issued behind them
+    constexpr int BEHIND = decltype(behind_c)::value;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) { lgkm_wait<NF>(fa0[i][0]); lgkm_wait<NF>(fa0[i][1]); }
+    for (int i = 0; i < TM; ++i) lgkm_wait<BEHIND>(fa[i][0], fa[i][1]);
 #pragma unroll
-    for (int j = 0; j < TN; ++j) lgkm_wait<NF>(fb0[j]);
-    multiply_half(fa0, fb0, 0);
-#pragma unroll
-    for (int i = 0; i < TM; ++i) { lgkm_wait<0>(fa1[i][0]); lgkm_wait<0>(fa1[i][1]); }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) lgkm_wait<0>(fb1[j]);
-    multiply_half(fa1, fb1, 1);
+    for (int j = 0; j < TN; ++j) lgkm_wait<BEHIND>(fb[j]);
   };
 
-  // ---- pipeline (same schedule as the int8 kernel) ---------------------------------------------------
+  // ---- pipeline -----------------------------------------------------------------------------------------
+  // The barrier sits in the middle of a step's multiplications: behind it the first half of the next step is requested,
+  // which arrives under the second half of this one, and this step's slot, which every wave has read, is refilled.
+  constexpr int NF = 2 * TM + TN;  // LDS reads per half
   const int nsteps = (p.K + BK - 1) / BK;
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s) issue_stage(s * STAGE_BYTES);
-  int rd_off = 0, wr_off = (STAGES - 1) * STAGE_BYTES;
+  for (int s = 0; s < STAGES; ++s) issue_stage(s * STAGE_BYTES);
+  CATCHQ_VMCNT(NI * (STAGES - 1));
+  __builtin_amdgcn_s_barrier();
+  v4i fa0[TM][2], fb0[TN], fa1[TM][2], fb1[TN];
+  fetch_half(fa0, fb0, a_row, a_c0, b_row + b_k0);
+  int rd_off = 0;
   for (int step = 0; step < nsteps; ++step) {
-    CATCHQ_VMCNT(NI * (STAGES - 2));
-    __builtin_amdgcn_s_barrier();
-    compute((unsigned)rd_off, wr_off);
+    fetch_half(fa1, fb1, a_row + (unsigned)rd_off, a_c0 ^ 64u, b_row + (unsigned)rd_off + b_k1);
+    arrived(fa0, fb0, std::integral_constant<int, NF>{});
+    multiply_half(fa0, fb0, 0);
+    arrived(fa1, fb1, std::integral_constant<int, 0>{});
+    CATCHQ_VMCNT(NI * (STAGES - 2));  // this wave's part of the next stage has landed ...
+    __builtin_amdgcn_s_barrier();     // ... and everyone else's; the stage in hand is no longer read
+    const int wr_off = rd_off;
     rd_off = (rd_off + STAGE_BYTES == PIPE_BYTES) ? 0 : rd_off + STAGE_BYTES;
-    wr_off = (wr_off + STAGE_BYTES == PIPE_BYTES) ? 0 : wr_off + STAGE_BYTES;
+    fetch_half(fa0, fb0, a_row + (unsigned)rd_off, a_c0, b_row + (unsigned)rd_off + b_k0);  // (past the end: not used)
+    issue_stage(wr_off);
+    multiply_half(fa1, fb1, 1);
   }
+  arrived(fa0, fb0, std::integral_constant<int, 0>{});
   CATCHQ_VMCNT(0);
   __syncthreads();
 
