@@ -417,7 +417,14 @@ int igemm_a16_launch(int load, const void *a, const void *b, IgemmParams p, cons
   return -1;
 }
 
+int contract_ksplit(const void *x, bool a16, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                    int sh, int sw, int dh, int dw, int Ho, int Wo, bool patch, const EpiDev &e, hipStream_t s);
+
 int gemm_nt_mfma_a16(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s) {
+  if (M < (1 << 20) && K < (1 << 20)) {  // a few blocks per unit, long K
+    const int st = contract_ksplit(a, true, b, (int)M, 1, 1, (int)K, (int)N, 1, 1, 0, 0, 1, 1, 1, 1, 1, 1, false, e, s);
+    if (st >= 0) return st;
+  }
   IgemmParams p = {};
   p.M = M;
   p.N = (int)N;
@@ -540,6 +547,10 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo;
   p.kh = kh; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
   p.K = kh * kw * Ci;
+  if (Ci % 16 == 0) {  // a few blocks per unit, long K
+    const int st = contract_ksplit(x, true, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false, e, s);
+    if (st >= 0) return st;
+  }
   if (p.M >= (1ll << 31)) return -1;  // the loaders split a pixel index with 32-bit divisions
   if (Ci == 8 && ph == 0 && pw == 0 && dw == 1) {  // framed few-channel image: streaming kernel
     const int st = conv2d_stem_a16(x, w, N, H, W, Co, kh, kw, sh, sw, dh, Ho, Wo, e, s);

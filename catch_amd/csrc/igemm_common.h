@@ -181,6 +181,18 @@ inline int pick_epilogue(int N, const EpiDev &e) {
   return EPI_VECTOR;
 }
 
+// For rows whose length or alignment the vectorised epilogues do not take, a floating output and nothing else: the epilogue
+// (EPI_Y32 or EPI_Y16) that serves them with stores that need no alignment (EpiAtRagged); EPI_SCALAR: neither does.
+inline int ragged_epilogue(int N, const EpiDev &e) {
+  if (N >= (1 << 24)) return EPI_SCALAR;
+  EpiDev aligned = e;
+  auto stand_in = [](const auto *q) { return reinterpret_cast<decltype(q)>(q ? (uintptr_t)16 : 0); };  // (presence only)
+  aligned.chan_div = stand_in(e.chan_div); aligned.chan_rcp = stand_in(e.chan_rcp); aligned.bias = stand_in(e.bias);
+  aligned.y = const_cast<void *>((const void *)stand_in((const char *)e.y));
+  const int epi = pick_epilogue((N + 3) / 4 * 4, aligned);
+  return epi == EPI_Y32 || epi == EPI_Y16 ? epi : EPI_SCALAR;
+}
+
 // per-channel constants of one lane's four consecutive channels
 struct EpiLane {
   v4f div, rcp, bias;

@@ -315,10 +315,15 @@ int conv2d_stem_i8(const void *x, const void *w, int N, int H, int W, int Co, in
 int contract_small_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                       int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
 
+int contract_ksplit(const void *x, bool a16, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                    int sh, int sw, int dh, int dw, int Ho, int Wo, bool patch, const EpiDev &e, hipStream_t s);
+
 int gemm_nt_mfma_i8(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e,
                     hipStream_t s) {
-  if (M < (1 << 20) && K < (1 << 20)) {  // few output tiles
-    const int st = contract_small_i8(a, b, (int)M, 1, 1, (int)K, (int)N, 1, 1, 0, 0, 1, 1, 1, 1, 1, 1, e, s);
+  if (M < (1 << 20) && K < (1 << 20)) {  // a few blocks per unit; few output tiles
+    int st = contract_ksplit(a, false, b, (int)M, 1, 1, (int)K, (int)N, 1, 1, 0, 0, 1, 1, 1, 1, 1, 1, false, e, s);
+    if (st >= 0) return st;
+    st = contract_small_i8(a, b, (int)M, 1, 1, (int)K, (int)N, 1, 1, 0, 0, 1, 1, 1, 1, 1, 1, e, s);
     if (st >= 0) return st;
   }
   if (dma_enabled()) {  // short K, narrow N, many rows: the streaming kernel
@@ -370,6 +375,10 @@ int conv2d_mfma_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
   const bool halo_first = kh == 3 && kw == 3 && sh == 1 && sw == 1 && ph == 1 && pw == 1 && dh == 1 && dw == 1 &&
                           dma_enabled() && halo_enabled() && ((p.M + 31) / 32) * ((Co + 31) / 32) > 2 * e.cus &&
                           conv2d_halo_one_round(N, H, W, Ci, Co, e.cus);
+  if (Ci % 16 == 0) {  // a few blocks per unit
+    const int st = contract_ksplit(x, false, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, halo_first, e, s);
+    if (st >= 0) return st;
+  }
   if (Ci % 16 == 0 && !halo_first) {  // few output tiles
     const int st = contract_small_i8(x, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, e, s);
     if (st >= 0) return st;

@@ -384,15 +384,10 @@ int conv2d_mfma_a16w16(const void *x, const void *w, int N, int H, int W, int Ci
   magic(kw, &p.magic_kw, &p.mask_kw);
   p.m_fastest = b_bytes > a_bytes;
   p.epi = pick_epilogue(Co, e);
-  if (p.epi == EPI_SCALAR && Co < (1 << 24)) {
-    // A floating output and nothing else: the epilogue of aligned rows of the same outputs, with stores that need no alignment
-    // (33759 x 192 -> 146 62.8 us with one element at a time, 47.5 so, 148 channels 46.3).
-    EpiDev aligned = e;
-    auto stand_in = [](const auto *q) { return reinterpret_cast<decltype(q)>(q ? (uintptr_t)16 : 0); };  // (presence only)
-    aligned.chan_div = stand_in(e.chan_div); aligned.chan_rcp = stand_in(e.chan_rcp); aligned.bias = stand_in(e.bias);
-    aligned.y = const_cast<void *>((const void *)stand_in((const char *)e.y));
-    const int epi = pick_epilogue((Co + 3) / 4 * 4, aligned);
-    if (epi == EPI_Y32 || epi == EPI_Y16) { p.epi = epi; p.ragged = 1; }
+  if (p.epi == EPI_SCALAR) {
+    // (33759 x 192 -> 146 62.8 us with one element at a time, 47.5 so, 148 channels 46.3)
+    const int epi = ragged_epilogue(Co, e);
+    if (epi != EPI_SCALAR) { p.epi = epi; p.ragged = 1; }
   }
   p.a_bytes = (unsigned)a_bytes; p.b_bytes = (unsigned)b_bytes;
   return dense ? pick_wide<true>(p, e, s) : pick_wide<false>(p, e, s);

@@ -311,6 +311,59 @@ def test_few_output_tiles(case):
             assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
 
 
+# A few blocks per unit: K split over waves with tiles of their own.  Every plan of the kernel, at the edges of its tiles: rows
+# and columns beyond the last full one, as many steps as waves, K ending inside a step, filter taps of whole steps and of
+# 16-byte pieces, strides, dilation, padding, rows of any alignment
+K_SPLIT_CASES = [
+    # bits, n, h, w, ci, co, k, pad, stride, dil
+    (8, 500, 1, 1, 272, 500, 1, 0, 1, 1), (8, 783, 1, 1, 1040, 261, 1, 0, 1, 1), (8, 395, 1, 1, 256, 512, 1, 0, 1, 1),  # 32 x 32
+    (8, 1000, 1, 1, 2064, 500, 1, 0, 1, 1),                                                                           # 64 x 64
+    (8, 4, 28, 28, 128, 100, 3, 1, 1, 1), (8, 3, 25, 23, 48, 256, 3, 1, 1, 1), (8, 2, 29, 20, 64, 200, 5, 4, 1, 2),  # 32 x 32
+    (8, 4, 14, 14, 256, 256, 3, 1, 1, 1), (8, 2, 21, 22, 240, 130, 3, 1, 1, 1),                                      # ... eight waves
+    (8, 5, 28, 28, 128, 128, 3, 1, 1, 1), (8, 1, 90, 90, 48, 128, 3, 1, 1, 1), (8, 2, 40, 40, 96, 132, 3, 0, 1, 1),  # 32 x 64
+    (8, 8, 7, 7, 512, 500, 3, 1, 1, 1), (8, 12, 14, 14, 512, 512, 3, 1, 2, 1), (8, 16, 7, 7, 480, 512, 3, 1, 1, 1),  # long K
+    (8, 12, 20, 20, 256, 130, 5, 2, 1, 1), (8, 5, 40, 40, 96, 96, 5, 2, 1, 1), (8, 40, 7, 7, 512, 512, 3, 1, 1, 1),   # 64 x 64
+    (16, 1, 1, 1, 256, 4, 1, 0, 1, 1), (16, 169, 1, 1, 272, 512, 1, 0, 1, 1), (16, 1350, 1, 1, 1024, 508, 1, 0, 1, 1),
+    (16, 1, 13, 13, 512, 1020, 3, 1, 1, 1), (16, 2, 13, 13, 512, 1024, 3, 1, 1, 1), (16, 1, 15, 17, 64, 36, 3, 2, 2, 2),
+    (16, 6, 13, 13, 512, 1024, 3, 1, 1, 1), (16, 4, 26, 26, 64, 512, 3, 1, 1, 1), (16, 1, 52, 52, 128, 256, 3, 1, 1, 1)]
+
+
+@pytest.mark.parametrize("case", K_SPLIT_CASES)
+def test_k_split_over_waves_with_tiles(case):
+    bits, n, h, w, ci, co, k, pad, stride, dil = case
+    note("k split, tiles per wave", case)
+    r = rng(sum(case) * 17)
+    x, wt = _ints(r, (n, h, w, ci), bits), _ints(r, (co, k, k, ci), 8)
+    if bits == 16:
+        x = (x // 64).astype(np.int16)  # (the sums fit an int32)
+        x[0, 0, 0, :4] = (-32768, 32767, 255, -129)
+    acc, ovf = orc.conv2d_nhwc(x, wt, (pad, pad), (stride, stride), (dil, dil), 1)
+    assert ovf == 0
+    div = r.uniform(0.6, 3.5, co).astype(np.float32)
+    bias = r.standard_normal(co).astype(np.float32)
+    res = (r.standard_normal(acc.shape) * 20).astype(np.float32)
+    xd, wd, dd, bd, rd = (cabi.dev(t) for t in (x, wt, div, bias, res))
+    rcp = cabi.dev(np.float32(1) / div)
+    args = dict(padding=(pad, pad), stride=(stride, stride), dilation=(dil, dil))
+    assert same_bits(acc.astype(np.int32), cabi.conv2d_nhwc(xd, wd, y_dtype=None, **args)["acc"].cpu().numpy())
+    # (divisors, output, quantized output, activation, residual, residual behind the activation)
+    layers = ((True, torch.float32, 0, 0, False, False), (True, torch.float16, 0, 0, False, False),
+              (True, None, 8, 1, False, False), (True, None, 8, 2, False, False), (True, torch.float32, 8, 1, True, False),
+              (True, None, 8, 0, True, False)) if bits == 8 else \
+             ((True, torch.float16, 0, 0, False, False), (False, None, 16, 3, False, False),
+              (False, None, 16, 3, True, True), (False, torch.float32, 16, 3, True, True))
+    e = -10 if bits == 8 else -20
+    for use_div, y_dtype, q_bw, act, use_res, after in layers:
+        out = cabi.conv2d_nhwc(xd, wd, exp2=e, chan_div=dd if use_div else None, chan_rcp=rcp if use_div else None, bias=bd,
+                               resid=rd if use_res else None, act=act, act_slope=0.1, resid_after_act=after, y_dtype=y_dtype,
+                               want_acc=False, q_bw=q_bw, q_pos=-3, **args)
+        y = orc.epilogue(acc, e, div if use_div else None, bias, res if use_res else None, act, act_slope=0.1, resid_after_act=after)
+        if y_dtype is not None:
+            assert same_bits(y.astype(np.float16) if y_dtype == torch.float16 else y, out["y"].cpu().numpy())
+        if q_bw:
+            assert same_bits(orc.quantize(y, q_bw, -3), out["q"].cpu().numpy())
+
+
 # int16 x int16 with K split over the waves: each tile size, dense and convolution, K ending inside a step, fewer steps
 # than waves, rows and columns beyond the last full tile, taps that end inside a transfer, output rows of any alignment
 WIDE_CASES = [
