@@ -1297,9 +1297,17 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   TORCH_CHECK(input.dim() >= 1 && input.size(-1) == weight.size(1), "size mismatch: input ", input.sizes(),
               ", weight ", weight.sizes());
   c10::DeviceGuard guard(input.device());
-  // K is padded with zeros on both operands to what the matrix-core routes take (16 int8 / 8 int16 values)
+  // K is padded with zeros on both operands: at least to what the matrix-core routes take (16 int8 / 8 int16 values), and where
+  // padding costs nothing that is not paid anyway -- int8 rows that need it in any case, int16 rows, which are never quantized
+  // inside the product -- to whole K steps of 64, so that the kernels' 64- and 128-byte pieces of a row do not straddle cache
+  // lines: int8 4000 x 1000 -> 1000 21.9 -> 17.9 us, 6000 x 2500 -> 700 49.6 -> 37.8, 8000 x 97 -> 120 9.3 -> 6.6, int16
+  // 1379 x 1000 -> 1001 22.4 -> 20.5.  (Shorter rows keep the streaming kernel, which takes up to 96 values; the matrix-core
+  // routes of int16 end at 65536 values of K and 2^30 of an operand.)
   const int64_t k = weight.size(1);
-  auto device_k = [&](int bw_act) { return bw_act == 8 ? (k + 15) / 16 * 16 : (k + 7) / 8 * 8; };
+  auto device_k = [&](int bw_act) {
+    const int64_t least = bw_act == 8 ? (k + 15) / 16 * 16 : (k + 7) / 8 * 8, whole = (k + 63) / 64 * 64;
+    return k > 96 && whole < 65536 && weight.size(0) * whole < (1ll << 30) && (bw_act != 8 || least != k) ? whole : least;
+  };
   auto prep = prepared_for(weight, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
     const int64_t kpad = device_k(bw_act) - k;
     return kpad > 0 ? at::constant_pad_nd(w, {0, kpad}, 0).contiguous() : w.contiguous();
@@ -1327,16 +1335,25 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
       return y;
     }
   }
-  Tensor qx = device_empty({m, kd}, int_type(prep->bw_x), input.device());
-  if (kd != k)  // rows as pixels of a [M, K, 1, 1] image, zero channels appended
-    check_status(catchq_quantize_nchw_to_nhwc(xc.data_ptr(), dt, qx.data_ptr(), prep->bw_x, (int)m, (int)k, 1, 1, (int)kd,
-                                              prep->pos_x, 1.0f, current_stream()),
-                 "torch_mlu::quantize");
-  else
-    check_status(catchq_quantize(xc.data_ptr(), dt, qx.data_ptr(), prep->bw_x, m * k, prep->pos_x, 1.0f, current_stream()),
-                 "torch_mlu::quantize");
-  check_status(catchq_gemm_nt(qx.data_ptr(), prep->bw_x, prep->qw.data_ptr(), prep->bw_w, m, n, kd, &e, current_stream()),
-               "torch_mlu::linear");
+  // (as many rows at a time as an int16 operand may have values: padding makes no product a slower route's)
+  int64_t rows = m;
+  if (prep->bw_x == 16 && m * kd >= (1ll << 30)) rows = std::max<int64_t>(((1ll << 30) - 1) / kd, 1);
+  Tensor qx = device_empty({rows, kd}, int_type(prep->bw_x), input.device());
+  for (int64_t r = 0; r < m; r += rows) {
+    const int64_t count = std::min(rows, m - r);
+    const char *x = static_cast<const char *>(xc.data_ptr()) + r * k * xc.element_size();
+    if (kd != k)  // rows as pixels of a [M, K, 1, 1] image, zero channels appended
+      check_status(catchq_quantize_nchw_to_nhwc(x, dt, qx.data_ptr(), prep->bw_x, (int)count, (int)k, 1, 1, (int)kd, prep->pos_x,
+                                                1.0f, current_stream()),
+                   "torch_mlu::quantize");
+    else
+      check_status(catchq_quantize(x, dt, qx.data_ptr(), prep->bw_x, count * k, prep->pos_x, 1.0f, current_stream()),
+                   "torch_mlu::quantize");
+    catchq_epilogue_t er = e;
+    er.y = static_cast<float *>(e.y) + r * n;
+    check_status(catchq_gemm_nt(qx.data_ptr(), prep->bw_x, prep->qw.data_ptr(), prep->bw_w, count, n, kd, &er, current_stream()),
+                 "torch_mlu::linear");
+  }
   return y;
 }
 

@@ -140,6 +140,21 @@ def test_linear_leading_dims_and_no_bias_tensor():
         torch.ops.torch_mlu.linear(x.cuda(), w.cuda()[None], zero_dim_bias.cuda(), q_scale.cuda(), q_mode.cuda())
 
 
+@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("m,k,n", [(1, 97, 5), (130, 104, 33), (70, 129, 65), (65, 191, 130), (300, 1000, 70)])
+def test_linear_rows_padded_to_whole_steps(m, k, n, mode):
+    """K behind the last 64-value step, on both sides of the streaming kernel's rows; same integers whatever the padding"""
+    note("linear padded rows", m, k, n, mode)
+    torch.manual_seed(m + k + n)
+    w, x, b = torch.randn(n, k) * 0.1, torch.randn(m, k), torch.randn(n)
+    top = 127.0 if mode == 1 else 32767.0
+    q_scale = torch.tensor([top / x.abs().max().item(), top / w.abs().max().item()])
+    q_mode = torch.tensor([mode], dtype=torch.int32)
+    got = torch.ops.torch_mlu.linear(x.cuda(), w.cuda(), b.cuda(), q_scale.cuda(), q_mode.cuda())
+    ref = oops.linear(x.numpy(), w.numpy(), b.numpy(), q_scale.numpy(), q_mode.numpy())
+    assert same_bits(ref["y"], got.cpu().numpy())
+
+
 def test_conv2d_cnnl_encoding_int16_act_int8_weight():
     """q_scale = [bitwidth_in, bitwidth_w], q_mode = [pos_in, pos_w] (quantify_conv_forward.cpp:132-145)"""
     note("conv2d encoding B")

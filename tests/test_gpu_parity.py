@@ -112,6 +112,18 @@ def test_quantize_transpose_and_row_padding(shape, cpad, bw, dtype):
 
 
 @pytest.mark.parametrize("dtype", [np.float32, np.float16])
+@pytest.mark.parametrize("bw", [8, 16])
+@pytest.mark.parametrize("c,cpad", [(12, 12), (13, 20), (9, 16), (63, 64), (97, 128), (100, 108)])
+def test_quantize_padded_rows(c, cpad, bw, dtype):
+    """rows of eights and of fours, starting at every alignment, ending anywhere in a lane's run"""
+    note("quantize rows", c, cpad, bw, dtype)
+    x = (rng(c).standard_normal((37, c, 1, 1)) * 40).astype(dtype)
+    want = np.zeros((37, 1, 1, cpad), np.int8 if bw == 8 else np.int16)
+    want[..., :c] = orc.quantize(x, bw, -1).transpose(0, 2, 3, 1)
+    assert same_bits(want, cabi.quantize_nchw_to_nhwc(cabi.dev(x), bw, -1, cpad=cpad).cpu().numpy())
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float16])
 @pytest.mark.parametrize("n", [1, 7, 100000, 4096 * 300 + 3, 4096 * 256 * 4 * 5 + 1029])
 def test_quantize_param(dtype, n):
     note("quantize_param", dtype.__name__, n)
