@@ -27,6 +27,9 @@ int conv2d_dual_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
 int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                            int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws,
                            int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
+int float_rows(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, const EpiDev &e,
+               hipStream_t s);
+int pack_filters(const void *w, void *packed, int64_t N, int64_t K, hipStream_t s);
 bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
 int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
                int Wo, const EpiDev &e, hipStream_t s);
@@ -357,6 +360,38 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
   st = catchq_quantize(x, x_dtype, workspace, 8, need, x_position, 1.0f, stream);
   if (st != CATCHQ_OK) return st;
   return catchq_conv2d_nhwc(workspace, 8, w, 8, desc, epilogue, stream);
+}
+
+CATCHQ_API int catchq_packed_filters_size(int64_t n, int64_t k, size_t *bytes) {
+  if (!bytes || n <= 0 || k <= 0) return CATCHQ_ERR_ARG;
+  if (k % 16 != 0 || n >= (1ll << 31) || k >= (1ll << 31) || n * k >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  *bytes = (size_t)((n + 31) / 32 * ((k + 31) / 32)) * 1024;
+  return CATCHQ_OK;
+}
+
+CATCHQ_API int catchq_pack_filters(const void *w, int64_t n, int64_t k, void *packed, catchq_stream_t stream) {
+  size_t bytes;
+  const int st = catchq_packed_filters_size(n, k, &bytes);
+  if (st != CATCHQ_OK) return st;
+  if (!w || !packed || !aligned16(w) || !aligned16(packed)) return CATCHQ_ERR_ARG;
+  return pack_filters(w, packed, n, k, as_stream(stream));
+}
+
+CATCHQ_API int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n,
+                                          int64_t k, const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  const int st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  size_t bytes;
+  if (m < 0 || x_position < -126 || x_position > 126) return CATCHQ_ERR_ARG;
+  if (m >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  const int sized = catchq_packed_filters_size(n, k, &bytes);
+  if (sized != CATCHQ_OK) return sized;
+  if (m == 0) return CATCHQ_OK;
+  if (!x || !packed) return CATCHQ_ERR_ARG;
+  if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;
+  const int done = float_rows(x, x_dtype == CATCHQ_F16, x_position, packed, m, n, k, make_epi(epilogue, m * n), as_stream(stream));
+  return done < 0 ? CATCHQ_ERR_UNSUPPORTED : done;
 }
 
 CATCHQ_API int catchq_conv1x1_chain_nhwc(const catchq_chain_link_t *links, int nlinks, int n, int ho, int wo, int co,

@@ -893,6 +893,7 @@ struct Prepared {
   bool params_half = false;  // per-channel parameters derived with half tensor ops (half q_scale, int8)
   int variant = 0;   // caller's layout choice for qw (part of the cache key)
   Tensor qw;         // conv: [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory; linear: [N,K]
+  Tensor packed;     // int8 linears and pointwise convolutions of many rows: qw in the order of the matrix instruction
   Tensor new_scale;  // device fp32 [Co] when per_channel
   Tensor rcp;        // its correctly rounded reciprocals (undefined where the kernels have to divide)
   // recorded on the stream that quantized the weight, behind those kernels: a later call on another stream
@@ -1008,6 +1009,29 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
   return p;
 }
 
+// Filters of the shapes that catchq_float_linear_packed may take (its columns and row lengths), laid out for it: once per weight,
+// so only where the entry is kept.
+void pack_filters(Prepared &p) {
+  const Tensor &w = p.qw;
+  if (p.bw_x != 8 || p.bw_w != 8 || w.dim() < 2) return;
+  const int64_t n = w.size(0), k = w.size(1);
+  if (n <= 256 || k < 64 || k > 1312 || k % 16 != 0 || w.numel() != n * k) return;
+  size_t bytes = 0;
+  if (catchq_packed_filters_size(n, k, &bytes) != CATCHQ_OK) return;
+  p.packed = device_empty({(int64_t)bytes}, at::kChar, w.device());
+  check_status(catchq_pack_filters(w.data_ptr(), n, k, p.packed.data_ptr(), current_stream()), "torch_mlu::quantize");
+}
+
+// The product of floating rows with packed filters; false: another route serves it.
+bool linear_packed(const void *x, int dt, const Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
+                   const char *what) {
+  if (!prep.packed.defined() || m < 1024) return false;
+  const int st = catchq_float_linear_packed(x, dt, prep.pos_x, prep.packed.data_ptr(), m, n, k, &e, current_stream());
+  if (st == CATCHQ_ERR_UNSUPPORTED) return false;
+  check_status(st, what);
+  return true;
+}
+
 template <typename MakeDense>
 std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_scale, const Tensor &q_mode,
                                        MakeDense make_dense, int variant = 0) {
@@ -1027,7 +1051,7 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_sca
           // read on another stream than the one the caching allocator knows these blocks by: tell it, so that
           // an entry dropped while this stream's kernels still read it is not handed out again too early
           it->second->qw.record_stream(cur);
-          for (const Tensor *t : {&it->second->new_scale, &it->second->rcp})
+          for (const Tensor *t : {&it->second->packed, &it->second->new_scale, &it->second->rcp})
             if (t->defined()) t->record_stream(cur);
         }
         return it->second;
@@ -1036,6 +1060,7 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_sca
     }
   }
   auto p = prepare(make_dense, weight, q_scale, q_mode);
+  if (use_cache) pack_filters(*p);
   p->variant = variant;
   const auto made_on = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
   p->made_on = made_on.id();
@@ -1126,6 +1151,9 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, co
     return y;
   }
   const int dt = half ? CATCHQ_F16 : CATCHQ_F32;
+  if (d.kh == 1 && d.kw == 1 && d.stride_h == 1 && d.stride_w == 1 && d.pad_h == 0 && d.pad_w == 0 && d.groups == 1 &&
+      linear_packed(x, dt, prep, (int64_t)d.n * d.h * d.w, d.co, d.ci, e, "torch_mlu::conv2d"))
+    return y;
   size_t ws_bytes = 0;
   check_status(catchq_float_conv2d_workspace_size(dt, &d, &e, &ws_bytes), "torch_mlu::conv2d");
   if (reinterpret_cast<uintptr_t>(x) & 15u) ws_bytes = (size_t)d.n * d.h * d.w * d.ci;  // one launch takes aligned tensors only
@@ -1325,6 +1353,7 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   const catchq_epilogue_t e = prepared_epilogue(*prep, bias, n, y, &keep);
   const int dt = input.scalar_type() == at::kHalf ? CATCHQ_F16 : CATCHQ_F32;
   if (prep->bw_x == 8 && prep->bw_w == 8 && kd == k && m < (1ll << 31)) {
+    if (linear_packed(xc.data_ptr(), dt, *prep, m, n, k, e, "torch_mlu::linear")) return y;
     // rows as images of one pixel: small products quantize and multiply in one launch
     const catchq_conv_desc_t d = {(int)m, 1, 1, (int)k, (int)n, 1, 1, 0, 0, 1, 1, 1, 1, 1};
     size_t ws_bytes = 0;

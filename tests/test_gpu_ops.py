@@ -155,6 +155,50 @@ def test_linear_rows_padded_to_whole_steps(m, k, n, mode):
     assert same_bits(ref["y"], got.cpu().numpy())
 
 
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m,k,n,mode", [(1024, 64, 1224, 3), (1090, 80, 1152, 1), (1025, 448, 1220, 3), (1087, 464, 1284, 3),
+                                        (1061, 1312, 1280, 3), (1500, 752, 900, 1), (16500, 496, 260, 3)])
+def test_linear_on_packed_filters(m, k, n, mode, half):
+    """rows converted once per block: both block sizes, K ending inside a sub-step and inside a turn of the ring, ragged rows
+    and columns, special values; every row as the general path has it (which takes calls of fewer rows) and the first against
+    the oracle"""
+    note("linear packed", m, k, n, mode, half)
+    torch.manual_seed(m + k + n)
+    w, x, b = torch.randn(n, k) * 0.1, torch.randn(m, k) * 3, torch.randn(n)
+    q_scale = [127 / 4.0, 127 / 0.4] if mode == 1 else [127 / 4.0, 0.0] + (127 / w.abs().amax(1)).tolist()
+    x[5, :4] = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0])
+    x[m - 1] = 1e4
+    x = x.half() if half else x
+    q_scale, q_mode = torch.tensor(q_scale), torch.tensor([mode], dtype=torch.int32)
+    xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
+    got = torch.ops.torch_mlu.linear(xd, wd, bd, q_scale, q_mode)
+    parts = torch.cat([torch.ops.torch_mlu.linear(xd[i:i + 600], wd, bd, q_scale, q_mode) for i in range(0, m, 600)])
+    assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
+    rows = torch.tensor([0, 5, m - 1])
+    ref = oops.linear(x[rows].float().numpy(), w.numpy(), b.numpy(), q_scale.numpy(), q_mode.numpy())
+    assert same_bits(ref["y"], got[rows.cuda()].cpu().numpy())
+
+
+@pytest.mark.parametrize("params_half", [False, True])
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n,ci,side,co", [(4, 80, 25, 644), (3, 256, 24, 1024), (5, 960, 15, 1160)])
+def test_conv1x1_on_packed_filters(n, ci, side, co, half, params_half):
+    """pointwise layers of unit stride, fp32 and half outputs, half steps: as the general path has each image"""
+    note("conv packed", n, ci, side, co, half, params_half)
+    torch.manual_seed(n + ci + co)
+    w, b = torch.randn(co, ci, 1, 1) * 0.1, torch.randn(co)
+    x = torch.randn(n, ci, side, side).to(memory_format=torch.channels_last).cuda()
+    q_scale = torch.tensor([127 / 4.0, 0.0] + (127 / w.abs().amax((1, 2, 3))).tolist())
+    q_mode = torch.tensor([3], dtype=torch.int32)
+    if params_half:
+        w, b, q_scale = w.half(), b.half(), q_scale.half()
+    x = x.half() if half else x
+    args = (w.cuda(), b.cuda(), [0, 0], [1, 1], [1, 1], 1, q_scale, q_mode)
+    got = torch.ops.torch_mlu.conv2d(x, *args)
+    parts = torch.cat([torch.ops.torch_mlu.conv2d(x[i:i + 1], *args) for i in range(n)])
+    assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
+
+
 def test_conv2d_cnnl_encoding_int16_act_int8_weight():
     """q_scale = [bitwidth_in, bitwidth_w], q_mode = [pos_in, pos_w] (quantify_conv_forward.cpp:132-145)"""
     note("conv2d encoding B")
