@@ -87,6 +87,10 @@ SIGNATURES = {
     "catchq_global_avgpool_quantize_nhwc": (_I, [_P, _P, _I, _I, _I, _I, _I, _F, _P]),
     "catchq_quantize_conv2d_workspace_size": (_I, [ctypes.POINTER(ConvDesc), _I, _I, ctypes.POINTER(_SZ)]),
     "catchq_quantize_conv2d_nhwc": (_I, [_P, _I, _P, _I, _P, _I, _P, _I, ctypes.POINTER(ConvDesc), _P, _P, _I, _P, _SZ, _P]),
+    "catchq_packed_digits_size": (_I, [_I64, _I64, ctypes.POINTER(_SZ)]),
+    "catchq_pack_digits": (_I, [_P, _I64, _I64, _I64, _P, _P]),
+    "catchq_float_linear_digits_workspace_size": (_I, [_I64, _I64, _I64, ctypes.POINTER(Epilogue), ctypes.POINTER(_SZ)]),
+    "catchq_float_linear_digits": (_I, [_P, _I, _I, _P, _I64, _I64, _I64, ctypes.POINTER(Epilogue), _P, _SZ, _P]),
     "catchq_packed_filters_size": (_I, [_I64, _I64, ctypes.POINTER(_SZ)]),
     "catchq_pack_filters": (_I, [_P, _I64, _I64, _P, _P]),
     "catchq_float_linear_packed": (_I, [_P, _I, _I, _P, _I64, _I64, _I64, ctypes.POINTER(Epilogue), _P]),

@@ -29,6 +29,11 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
                            int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
 int float_rows(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, const EpiDev &e,
                hipStream_t s);
+int64_t packed_digits_bytes(int64_t N, int64_t K);
+int pack_digits(const void *w, int64_t N, int64_t K, int64_t ld, void *packed, hipStream_t s);
+int64_t gemm_digits_bytes(int64_t M, int64_t N, int64_t K, const EpiDev &e);
+int gemm_digits(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, void *digits,
+                const EpiDev &e, hipStream_t s);
 int pack_filters(const void *w, void *packed, int64_t N, int64_t K, hipStream_t s);
 bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
 int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
@@ -392,6 +397,44 @@ CATCHQ_API int catchq_float_linear_packed(const void *x, int x_dtype, int x_posi
   if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;
   const int done = float_rows(x, x_dtype == CATCHQ_F16, x_position, packed, m, n, k, make_epi(epilogue, m * n), as_stream(stream));
   return done < 0 ? CATCHQ_ERR_UNSUPPORTED : done;
+}
+
+CATCHQ_API int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes) {
+  if (!bytes || n <= 0 || k <= 0) return CATCHQ_ERR_ARG;
+  if (k > 8192 || n >= (1ll << 31) || packed_digits_bytes(n, k) >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  *bytes = (size_t)packed_digits_bytes(n, k);
+  return CATCHQ_OK;
+}
+
+CATCHQ_API int catchq_pack_digits(const void *w, int64_t n, int64_t k, int64_t ld, void *packed, catchq_stream_t stream) {
+  size_t bytes;
+  const int st = catchq_packed_digits_size(n, k, &bytes);
+  if (st != CATCHQ_OK) return st;
+  if (!w || !packed || ld < k || !aligned16(packed)) return CATCHQ_ERR_ARG;
+  return pack_digits(w, n, k, ld, packed, as_stream(stream));
+}
+
+CATCHQ_API int catchq_float_linear_digits_workspace_size(int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue,
+                                                         size_t *bytes) {
+  if (!bytes || m < 0) return CATCHQ_ERR_ARG;
+  const int sized = catchq_packed_digits_size(n, k, bytes);
+  if (sized != CATCHQ_OK) return sized;
+  const int st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  *bytes = m < (1ll << 31) ? (size_t)gemm_digits_bytes(m, n, k, make_epi(epilogue, m * n)) : 0;
+  return *bytes ? CATCHQ_OK : CATCHQ_ERR_UNSUPPORTED;
+}
+
+CATCHQ_API int catchq_float_linear_digits(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n,
+                                          int64_t k, const catchq_epilogue_t *epilogue, void *workspace, size_t workspace_bytes,
+                                          catchq_stream_t stream) {
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  if (x_position < -126 || x_position > 126) return CATCHQ_ERR_ARG;
+  size_t bytes;
+  const int st = catchq_float_linear_digits_workspace_size(m, n, k, epilogue, &bytes);
+  if (st != CATCHQ_OK) return st;
+  if (!x || !packed || !aligned16(packed) || !workspace || !aligned16(workspace) || workspace_bytes < bytes) return CATCHQ_ERR_ARG;
+  return gemm_digits(x, x_dtype == CATCHQ_F16, x_position, packed, m, n, k, workspace, make_epi(epilogue, m * n), as_stream(stream));
 }
 
 CATCHQ_API int catchq_conv1x1_chain_nhwc(const catchq_chain_link_t *links, int nlinks, int n, int ho, int wo, int co,

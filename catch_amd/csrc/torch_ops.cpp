@@ -893,7 +893,7 @@ struct Prepared {
   bool params_half = false;  // per-channel parameters derived with half tensor ops (half q_scale, int8)
   int variant = 0;   // caller's layout choice for qw (part of the cache key)
   Tensor qw;         // conv: [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory; linear: [N,K]
-  Tensor packed;     // int8 linears and pointwise convolutions of many rows: qw in the order of the matrix instruction
+  Tensor packed;     // qw in the order of the matrix instruction: int8 linears and pointwise convolutions, int16 linears (digits)
   Tensor new_scale;  // device fp32 [Co] when per_channel
   Tensor rcp;        // its correctly rounded reciprocals (undefined where the kernels have to divide)
   // recorded on the stream that quantized the weight, behind those kernels: a later call on another stream
@@ -1009,12 +1009,19 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
   return p;
 }
 
-// Filters of the shapes that catchq_float_linear_packed may take (its columns and row lengths), laid out for it: once per weight,
-// so only where the entry is kept.
+// Weights of the shapes that catchq_float_linear_packed (8 bits) and catchq_float_linear_digits (16) may take, laid out for
+// them: once per weight, so only where the entry is kept.
 void pack_filters(Prepared &p) {
   const Tensor &w = p.qw;
-  if (p.bw_x != 8 || p.bw_w != 8 || w.dim() < 2) return;
+  if (p.bw_x != p.bw_w || w.dim() < 2) return;
   const int64_t n = w.size(0), k = w.size(1);
+  if (p.bw_w == 16) {
+    size_t bytes = 0;
+    if (w.dim() != 2 || n == 0 || k < 32 || catchq_packed_digits_size(n, k, &bytes) != CATCHQ_OK) return;
+    p.packed = device_empty({(int64_t)bytes}, at::kChar, w.device());
+    check_status(catchq_pack_digits(w.data_ptr(), n, k, k, p.packed.data_ptr(), current_stream()), "torch_mlu::quantize");
+    return;
+  }
   if (n <= 256 || k < 64 || k > 1312 || k % 16 != 0 || w.numel() != n * k) return;
   size_t bytes = 0;
   if (catchq_packed_filters_size(n, k, &bytes) != CATCHQ_OK) return;
@@ -1363,6 +1370,18 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
                    "torch_mlu::linear");
       return y;
     }
+  }
+  if (prep->bw_x == 16 && prep->packed.defined() && k >= 32) {  // (rows of the packed weights end in zeros where kd > k)
+    size_t ws_bytes = 0;
+    const int st = catchq_float_linear_digits_workspace_size(m, n, k, &e, &ws_bytes);
+    if (st == CATCHQ_OK) {
+      Tensor digits = device_empty({(int64_t)ws_bytes}, at::kChar, input.device());
+      check_status(catchq_float_linear_digits(xc.data_ptr(), dt, prep->pos_x, prep->packed.data_ptr(), m, n, k, &e,
+                                              digits.data_ptr(), ws_bytes, current_stream()),
+                   "torch_mlu::linear");
+      return y;
+    }
+    if (st != CATCHQ_ERR_UNSUPPORTED) check_status(st, "torch_mlu::linear");
   }
   // (as many rows at a time as an int16 operand may have values: padding makes no product a slower route's)
   int64_t rows = m;

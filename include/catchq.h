@@ -266,6 +266,17 @@ int catchq_pack_filters(const void *w, int64_t n, int64_t k, void *packed, catch
 int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n, int64_t k,
                                const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 
+/* A linear on floating activations with int16 weights, both split into the bytes that the matrix cores multiply:
+ *   cnnl_quantify_offline_internal (quantify.cpp:69-101) followed by linear.cpp:92-110, 16 bits on either side
+ * catchq_pack_digits lays the weights out once (w [n,ld] int16, k values of a row used, k <= 8192); the call quantizes x [m,k]
+ * into the workspace and multiplies.  *_workspace_size returns CATCHQ_ERR_UNSUPPORTED where quantizing and catchq_gemm_nt serve
+ * the call better, or alone (too few tiles of 64 x 128 outputs for the device, an output other than fp32 y). */
+int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes);
+int catchq_pack_digits(const void *w, int64_t n, int64_t k, int64_t ld, void *packed, catchq_stream_t stream);
+int catchq_float_linear_digits_workspace_size(int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue, size_t *bytes);
+int catchq_float_linear_digits(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n, int64_t k,
+                               const catchq_epilogue_t *epilogue, void *workspace, size_t workspace_bytes, catchq_stream_t stream);
+
 /* Last convolution of a residual block with the block's projection shortcut evaluated in the same launch.
  * In the reference a block with a projection ends in two torch_mlu::conv2d calls (cnnl_conv2d,
  * operators/cnnl/quantify_conv_forward.cpp:56-147: the 1x1 shortcut and the block's last convolution) and a

@@ -179,6 +179,32 @@ def test_linear_on_packed_filters(m, k, n, mode, half):
     assert same_bits(ref["y"], got[rows.cuda()].cpu().numpy())
 
 
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m,k,n,mode", [(10240, 32, 65, 4), (5121, 33, 250, 2), (2600, 130, 500, 4), (1300, 257, 1000, 4),
+                                        (1379, 1000, 1001, 2), (640, 2050, 2048, 4), (5190, 700, 131, 4)])
+def test_linear_on_packed_digits(m, k, n, mode, half):
+    """int16: rows of any alignment, one slab of K and several, ending in its first and second half, ragged rows and columns,
+    special and extreme values; every row as the general path has it (which takes calls of fewer rows) and some against the
+    oracle"""
+    note("linear digits", m, k, n, mode, half)
+    torch.manual_seed(m + k + n)
+    w, x, b = torch.randn(n, k) * 0.1, torch.randn(m, k) * 3, torch.randn(n)
+    w[0] = w[0].abs().max() * torch.where(torch.arange(k) % 2 == 0, 1.0, -1.0)  # sums of the largest products
+    q_scale = [32767 / 4.0, 32767 / 0.4] if mode == 2 else [32767 / 4.0, 0.0] + (32767 / w.abs().amax(1)).tolist()
+    x[5, :4] = torch.tensor([float("nan"), float("inf"), -float("inf"), -0.0])
+    x[m - 1] = 1e4
+    x[m - 2] = -1e4 * w[0].sign()
+    x = x.half() if half else x
+    q_scale, q_mode = torch.tensor(q_scale), torch.tensor([mode], dtype=torch.int32)
+    xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
+    got = torch.ops.torch_mlu.linear(xd, wd, bd, q_scale, q_mode)
+    parts = torch.cat([torch.ops.torch_mlu.linear(xd[i:i + 300], wd, bd, q_scale, q_mode) for i in range(0, m, 300)])
+    assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
+    rows = torch.tensor([0, 5, m - 2, m - 1])
+    ref = oops.linear(x[rows].float().numpy(), w.numpy(), b.numpy(), q_scale.numpy(), q_mode.numpy())
+    assert same_bits(ref["y"], got[rows.cuda()].cpu().numpy())
+
+
 @pytest.mark.parametrize("params_half", [False, True])
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("n,ci,side,co", [(4, 80, 25, 644), (3, 256, 24, 1024), (5, 960, 15, 1160)])
