@@ -401,7 +401,9 @@ static int launch_ksplit(KsplitParams p, const EpiDev &e, hipStream_t s) {
 // int8.  Where 16 x 16 tiles (small_i8.hip) leave no unit more than two they are ahead.  Beyond, 32 x 32 tiles while no unit
 //   has more than 1.75: 784 x 1024 -> 512 (t 400) 4.2 / 5.1 (4.4 / 5.3), 196 x 256 -> 1024 (224) 3.1 / 3.3, 300 x 2048 -> 900 5.2 /
 //   6.0, 3 x 3 on 4 x 28 x 28, 128 channels (392) 4.5 / 5.7 (5.0 / 5.8), on 4 x 14 x 14, 256 (200) 4.4 on eight waves / 5.6
-//   (4.9 / 5.5).  A GEMM of more than 40 steps (512 x 3072 -> 768, t 384, 7.5 / 7.3) stays as it was.
+//   (4.9 / 5.5).  A GEMM of more than 40 steps (512 x 3072 -> 768, t 384, 7.5 / 7.3) stays as it was, and
+//   beyond 24 one whose rows do not start on cache lines (with the quantizer: 1794 x 1936 -> 84 10.4 / 9.8, 716 x 1904 -> 364
+//   10.7 / 10.2, 1099 x 1712 -> 120 9.2 / 8.7, but 1993 x 2048 -> 136 11.4 / 12.0).
 //   Convolutions: 32 x 64 tiles up to one per unit -- 5 x 28 x 28, 128 channels (t2 246) 5.0 / 6.3 (5.5 / 6.3) -- and up to two for
 //   short K, 5 x 56 x 56, 64 channels (490, nine steps) 4.9 / 5.7 (5.3 / 5.7).  64 x 64 tiles up to one per unit -- 5 x 5, 256 ->
 //   128 on 8 x 28 x 28 (t4 196) 15.1 / 24.0 (15.6 / 24.7), 40 x 7 x 7, 512 (248) 12.5 / 20.8, 12 x 28 x 28 / 2, 256 (148) 7.5 / 9.6
@@ -410,8 +412,9 @@ static int launch_ksplit(KsplitParams p, const EpiDev &e, hipStream_t s) {
 //   9.1), 16 x 7 x 7 (t2 200) 8.7 / 9.2 (9.5 / 9.7); the few-tiles kernel is ahead for 20 x 7 x 7 (t 496, t2 248) 9.3 / 9.6, and the
 //   patch-resident one, where it makes one round, for 6 x 17 x 17, 512 -> 448 (t4 196) 10.9 / 12.1, not for 24 x 7 x 7 (152)
 //   11.3 / 10.2 (11.9 / 11.2).
-//   GEMMs: 64 x 64 tiles up to 0.9 per unit from K = 2048 on, 900 x 4096 -> 900 (t4 225) 13.3 / 15.8, 1024 x 2048 -> 768 (192)
-//   7.3 / 7.6; 700 x 3008 -> 1500 (264) 14.0 / 13.4, 1024 x 1024 -> 1024 (256) 6.0 / 5.6.
+//   GEMMs: 64 x 64 tiles up to 0.9 per unit from K = 4096 on, 900 x 4096 -> 900 (t4 225) 13.3 / 15.8; 700 x 3008 -> 1500 (264)
+//   14.0 / 13.4, 1024 x 1024 -> 1024 (256) 6.0 / 5.6, with the quantizer 981 x 3200 -> 492 (128) 16.1 / 15.1, 2219 x 2128 -> 384
+//   (210) 16.9 / 16.0.
 // int16, 3 x 3: one 13 x 13 image, 512 -> 1024 (t 192) 7.7 on eight waves / 29.9 (8.3 / 30.4), two (t2 176) 10.7 / 30.4, six
 //   (t4 256) 18.0 / 31.0, eight (t2 688, two waves) 26.7 / 34.0; 26 x 26, 256 -> 512: one image (t2 176) 7.1 / 18.0, two (t 688)
 //   11.1 / 18.8, four (t2 680, two waves) 15.8 / 21.3; 52 x 52, 128 -> 256: one (t 680) 7.6 / 12.4, two (t2 676, two waves) 11.1 /
@@ -431,8 +434,9 @@ static int ksplit_plan(int64_t M, int64_t N, int64_t K, bool dense, bool a16, bo
     return 0;
   }
   if (tiles(16, 16) <= 2 * cus) return 0;
-  if (t * 4 <= 7 * cus && steps <= 40) return !dense && steps >= 32 && t <= cus ? 1182 : 1142;
-  if (dense) return t * 4 > 7 * cus && t4 * 10 <= 9 * cus && K >= 2048 ? 2242 : 0;
+  if (t * 4 <= 7 * cus && (dense ? steps <= 24 || (steps <= 40 && K % 128 == 0) : steps <= 40))
+    return !dense && steps >= 32 && t <= cus ? 1182 : 1142;
+  if (dense) return t * 4 > 7 * cus && t4 * 10 <= 9 * cus && K >= 4096 ? 2242 : 0;
   if (steps > 64) {
     if (t <= cus) return 1182;
     if (t * 4 <= 5 * cus) return 1142;

@@ -329,7 +329,7 @@ def test_few_output_tiles(case):
 K_SPLIT_CASES = [
     # bits, n, h, w, ci, co, k, pad, stride, dil
     (8, 500, 1, 1, 272, 500, 1, 0, 1, 1), (8, 783, 1, 1, 1040, 261, 1, 0, 1, 1), (8, 395, 1, 1, 256, 512, 1, 0, 1, 1),  # 32 x 32
-    (8, 1000, 1, 1, 2064, 500, 1, 0, 1, 1),                                                                           # 64 x 64
+    (8, 1000, 1, 1, 2064, 500, 1, 0, 1, 1), (8, 961, 1, 1, 4112, 484, 1, 0, 1, 1), (8, 300, 1, 1, 2048, 900, 1, 0, 1, 1),  # 64 x 64
     (8, 4, 28, 28, 128, 100, 3, 1, 1, 1), (8, 3, 25, 23, 48, 256, 3, 1, 1, 1), (8, 2, 29, 20, 64, 200, 5, 4, 1, 2),  # 32 x 32
     (8, 4, 14, 14, 256, 256, 3, 1, 1, 1), (8, 2, 21, 22, 240, 130, 3, 1, 1, 1),                                      # ... eight waves
     (8, 5, 28, 28, 128, 128, 3, 1, 1, 1), (8, 1, 90, 90, 48, 128, 3, 1, 1, 1), (8, 2, 40, 40, 96, 132, 3, 0, 1, 1),  # 32 x 64
