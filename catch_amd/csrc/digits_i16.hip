@@ -3,8 +3,8 @@
 // With  x = 256 xh + xl + 128  and  w = 256 wh + wl + 128  (high byte signed, low byte biased into int8)
 //   sum x w = 65536 S_hh + 256 (S_hl + S_lh) + S_ll + 128 (X + sum w),   X = sum (256 xh + xl)
 // over the K positions walked; positions beyond K and rows beyond M and N hold the value 0.  The four sums are int8 products
-// (|S| <= K 2^14, K <= 2^13), the combination is done in integers, and its one rounding to fp32 is the
-// int64 sum's.
+// (|S| <= K 2^14, K <= 2^13), the combination is done in fp64, which holds every value of it, and its one
+// conversion to fp32 is the int64 sum's.
 //
 // The kernel for int16 operands as they lie splits every fragment in every wave that reads it: 20 vector operations a fragment
 // beside the matrix instructions, and sums of both operands' digits.  Here the quantizer writes the activations' digits and the
@@ -14,8 +14,8 @@
 // wave's weights come straight into its registers, four K sub-steps of 32 ahead.  64 x 32 outputs a wave are eight matrix
 // instructions for two kilobytes of weights and four LDS reads.  What bounds it: the transfers from the Infinity Cache through
 // L2 (25 B a clock and unit, a slab of 96 KB in 3700 clocks where its multiplications take 2800), the first slab (4100 clocks)
-// and the epilogue (4800).  Tried without gain: floats converted by the blocks themselves (every run of columns converts them
-// again: 67 us), K shared between two groups of waves, unrolled fp64 sums at the end.
+// and the epilogue (4000).  Tried without gain: floats converted by the blocks themselves (every run of columns converts them
+// again: 67 us), K shared between two groups of waves.
 //
 // Measured: see gemm_digits_bytes below.
 #include <type_traits>
@@ -154,10 +154,9 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
   }
 
   // ---- outputs -----------------------------------------------------------------------------------------------------------------
-  // value = 65536 hh + 256 mid + ll + 128 (row's digit sum + sum w) = 65536 H + L with H = hh + (s >> 9), L = ll + 128 (s & 511)
-  // for s = 2 mid + row's + column's sum, all of it in 32 bits (K <= 8192).  The sums go through LDS as they are, and the
-  // arithmetic is a rolled loop: unrolled over a wave's 32 sums per lane it is ten kilobytes of code that every block waits
-  // for (6400 clocks of 26000 at 1379 x 1000 -> 1001).
+  // value = 65536 hh + 128 (2 mid + row's digit sum + sum w) + ll, in fp64.  The sums go through LDS as they are, and the
+  // arithmetic is a rolled loop: in the registers' order, with its carries in 32-bit integers and its eight turns unrolled it
+  // took 0.5 us of 19 more at 1379 x 1000 -> 1001 and 2 us of 52 at 4096 x 768 -> 3072.
   __syncthreads();  // the slabs are dead: the waves' shares of the rows' digit sums, then [row tile's sums][32][STAGE] of a wave
   int *rows = reinterpret_cast<int *>(lds_dyn);  // [NW][64]
   const int frow = lane & 31, fhalf = lane >> 5;
@@ -169,6 +168,9 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
   int *const stage = rows + NW * BM + wave * 3 * 32 * STAGE;
   __syncthreads();
   if (t >= n32) return;
+  int my_row = 0;  // the digit sum of row `lane`
+#pragma unroll
+  for (int w = 0; w < NW; ++w) my_row += rows[w * BM + lane];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -184,17 +186,12 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
       const int *at = stage + row * STAGE + cg * 4;
       const v4i h16 = *reinterpret_cast<const v4i *>(at), m16 = *reinterpret_cast<const v4i *>(at + 32 * STAGE);
       const v4i l16 = *reinterpret_cast<const v4i *>(at + 2 * 32 * STAGE);
-      int row_sum = 0;
-#pragma unroll
-      for (int w = 0; w < NW; ++w) row_sum += rows[w * BM + i * 32 + row];
+      const int row_sum = __shfl(my_row, i * 32 + row, 64);
       v4f sums;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int both = 2 * m16[k] + row_sum + col_sum[k];
-        const int h = h16[k] + (both >> 9), l = l16[k] + ((both & 511) << 7);
-        // 65536 h + l = 2^23 top + low, both exact in fp32 (|value| < 2^47): one rounding
-        const int carried = h + (l >> 16), top = carried >> 7, low = ((carried & 127) << 16) | (l & 0xffff);
-        sums[k] = __builtin_fmaf((float)top, 8388608.0f, (float)low);
+        const int both = 2 * m16[k] + row_sum + col_sum[k];  // (K <= 8192)
+        sums[k] = (float)__builtin_fma((double)h16[k], 65536.0, __builtin_fma((double)both, 128.0, (double)l16[k]));
       }
       const int64_t m = m0 + i * 32 + row;
       if (m < p.M && n < p.N) {
@@ -277,6 +274,13 @@ int pack_digits(const void *w, int64_t N, int64_t K, int64_t ld, void *packed, h
   return launch_status();
 }
 
+// EPI_Y32 or EPI_Y16, with or without aligned rows; 0: an epilogue this kernel does not have
+static int digit_epilogue(int N, const EpiDev &e) {
+  int epi = pick_epilogue(N, e);
+  if (epi != EPI_Y32 && epi != EPI_Y16) epi = ragged_epilogue(N, e);
+  return epi == EPI_Y32 || epi == EPI_Y16 ? epi : 0;
+}
+
 // Bytes of the activations' digits where this route serves the product; 0: another one does.
 //
 // With the quantizer, before (the quantizer of int16 and the kernel for operands as they lie) and now, us (half activations
@@ -289,7 +293,7 @@ int64_t gemm_digits_bytes(int64_t M, int64_t N, int64_t K, const EpiDev &e) {
   if (K < 32 || K > 8192 || M >= (1ll << 31) - 64 || N >= (1 << 24)) return 0;
   const int64_t blocks = (M + 63) / 64 * ((N + 127) / 128), bytes = digit_bytes(M, K);
   if (blocks * 8 < 5 * (int64_t)e.cus || blocks >= (1 << 27) || bytes >= (1ll << 31) || digit_bytes(N, K) >= (1ll << 31)) return 0;
-  return pick_epilogue((int)N, e) == EPI_Y32 || ragged_epilogue((int)N, e) == EPI_Y32 ? bytes : 0;
+  return digit_epilogue((int)N, e) ? bytes : 0;
 }
 
 // x [M, K] floats (halfs) -> its digits in `digits` -> the product with the packed weights of N rows
@@ -322,8 +326,10 @@ int gemm_digits(const void *x, bool half, int position, const void *packed, int6
     if (best < 0 || cost < best) best = cost, p.die_cols = cols, p.rect_m = (int)rm, p.rect_n = (int)rn;
   }
   const unsigned blocks = (unsigned)(8 * p.rect_m * p.rect_n);
-  if (pick_epilogue((int)N, e) != EPI_Y32) gemm_digits_kernel<EPI_Y32, true><<<blocks, 256, LDS_BYTES, s>>>(a, b, sums, p, e);
-  else gemm_digits_kernel<EPI_Y32, false><<<blocks, 256, LDS_BYTES, s>>>(a, b, sums, p, e);
+  const bool whole = pick_epilogue((int)N, e) == EPI_Y32 || pick_epilogue((int)N, e) == EPI_Y16;
+  auto kern = digit_epilogue((int)N, e) == EPI_Y32 ? (whole ? gemm_digits_kernel<EPI_Y32, false> : gemm_digits_kernel<EPI_Y32, true>)
+                                                   : (whole ? gemm_digits_kernel<EPI_Y16, false> : gemm_digits_kernel<EPI_Y16, true>);
+  kern<<<blocks, 256, LDS_BYTES, s>>>(a, b, sums, p, e);
   return launch_status();
 }
 

@@ -1017,7 +1017,7 @@ void pack_filters(Prepared &p) {
   const int64_t n = w.size(0), k = w.size(1);
   if (p.bw_w == 16) {
     size_t bytes = 0;
-    if (w.dim() != 2 || n == 0 || k < 32 || catchq_packed_digits_size(n, k, &bytes) != CATCHQ_OK) return;
+    if (w.numel() != n * k || n == 0 || k < 32 || catchq_packed_digits_size(n, k, &bytes) != CATCHQ_OK) return;
     p.packed = device_empty({(int64_t)bytes}, at::kChar, w.device());
     check_status(catchq_pack_digits(w.data_ptr(), n, k, k, p.packed.data_ptr(), current_stream()), "torch_mlu::quantize");
     return;
@@ -1034,6 +1034,21 @@ bool linear_packed(const void *x, int dt, const Prepared &prep, int64_t m, int64
                    const char *what) {
   if (!prep.packed.defined() || m < 1024) return false;
   const int st = catchq_float_linear_packed(x, dt, prep.pos_x, prep.packed.data_ptr(), m, n, k, &e, current_stream());
+  if (st == CATCHQ_ERR_UNSUPPORTED) return false;
+  check_status(st, what);
+  return true;
+}
+
+// The same at 16 bits, through the activations' digits.
+bool linear_digits(const void *x, int dt, const Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
+                   const c10::Device &device, const char *what) {
+  if (prep.bw_x != 16 || !prep.packed.defined() || k < 32) return false;
+  size_t bytes = 0;
+  int st = catchq_float_linear_digits_workspace_size(m, n, k, &e, &bytes);
+  if (st == CATCHQ_OK) {
+    Tensor digits = device_empty({(int64_t)bytes}, at::kChar, device);
+    st = catchq_float_linear_digits(x, dt, prep.pos_x, prep.packed.data_ptr(), m, n, k, &e, digits.data_ptr(), bytes, current_stream());
+  }
   if (st == CATCHQ_ERR_UNSUPPORTED) return false;
   check_status(st, what);
   return true;
@@ -1158,9 +1173,19 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, co
     return y;
   }
   const int dt = half ? CATCHQ_F16 : CATCHQ_F32;
-  if (d.kh == 1 && d.kw == 1 && d.stride_h == 1 && d.stride_w == 1 && d.pad_h == 0 && d.pad_w == 0 && d.groups == 1 &&
-      linear_packed(x, dt, prep, (int64_t)d.n * d.h * d.w, d.co, d.ci, e, "torch_mlu::conv2d"))
+  if (d.kh == 1 && d.kw == 1 && d.stride_h == 1 && d.stride_w == 1 && d.pad_h == 0 && d.pad_w == 0 && d.groups == 1) {
+    const int64_t m = (int64_t)d.n * d.h * d.w;
+    if (prep.bw_x == 16 ? linear_digits(x, dt, prep, m, d.co, d.ci, e, qw.device(), "torch_mlu::conv2d")
+                        : linear_packed(x, dt, prep, m, d.co, d.ci, e, "torch_mlu::conv2d"))
+      return y;
+  }
+  if (prep.bw_x == 16) {  // no single launch takes these: the quantized activations of all channels
+    Tensor qn = device_empty({d.n, d.h, d.w, d.ci}, int_type(16), qw.device());
+    check_status(catchq_quantize(x, dt, qn.data_ptr(), 16, (int64_t)d.n * d.h * d.w * d.ci, prep.pos_x, 1.0f, current_stream()),
+                 "torch_mlu::quantize");
+    check_status(catchq_conv2d_nhwc(qn.data_ptr(), 16, qw.data_ptr(), bits_of(qw), &d, &e, current_stream()), "torch_mlu::conv2d");
     return y;
+  }
   size_t ws_bytes = 0;
   check_status(catchq_float_conv2d_workspace_size(dt, &d, &e, &ws_bytes), "torch_mlu::conv2d");
   if (reinterpret_cast<uintptr_t>(x) & 15u) ws_bytes = (size_t)d.n * d.h * d.w * d.ci;  // one launch takes aligned tensors only
@@ -1203,7 +1228,9 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
     return wd.contiguous(at::MemoryFormat::ChannelsLast);
   }, (few ? 1 : 0) | (can_frame ? 2 : 0));
   Tensor qx;
-  if (prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0 && input.is_contiguous(at::MemoryFormat::ChannelsLast))
+  if (input.is_contiguous(at::MemoryFormat::ChannelsLast) &&
+      ((prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0) ||
+       (prep->bw_x == 16 && prep->bw_w == 16 && ci % 8 == 0 && dense && kw == 1 && weight.size(2) == 1 && prep->packed.defined())))
     return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), input.size(2), input.size(3), ci}, *prep, bias, padding, stride,
                          dilation, groups, half);
   if (few && prep->bw_x == 8 && can_frame) {
@@ -1371,18 +1398,8 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
       return y;
     }
   }
-  if (prep->bw_x == 16 && prep->packed.defined() && k >= 32) {  // (rows of the packed weights end in zeros where kd > k)
-    size_t ws_bytes = 0;
-    const int st = catchq_float_linear_digits_workspace_size(m, n, k, &e, &ws_bytes);
-    if (st == CATCHQ_OK) {
-      Tensor digits = device_empty({(int64_t)ws_bytes}, at::kChar, input.device());
-      check_status(catchq_float_linear_digits(xc.data_ptr(), dt, prep->pos_x, prep->packed.data_ptr(), m, n, k, &e,
-                                              digits.data_ptr(), ws_bytes, current_stream()),
-                   "torch_mlu::linear");
-      return y;
-    }
-    if (st != CATCHQ_ERR_UNSUPPORTED) check_status(st, "torch_mlu::linear");
-  }
+  // (rows of the packed weights end in zeros where kd > k)
+  if (linear_digits(xc.data_ptr(), dt, *prep, m, n, k, e, input.device(), "torch_mlu::linear")) return y;
   // (as many rows at a time as an int16 operand may have values: padding makes no product a slower route's)
   int64_t rows = m;
   if (prep->bw_x == 16 && m * kd >= (1ll << 30)) rows = std::max<int64_t>(((1ll << 30) - 1) / kd, 1);

@@ -270,7 +270,7 @@ int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const
  *   cnnl_quantify_offline_internal (quantify.cpp:69-101) followed by linear.cpp:92-110, 16 bits on either side
  * catchq_pack_digits lays the weights out once (w [n,ld] int16, k values of a row used, k <= 8192); the call quantizes x [m,k]
  * into the workspace and multiplies.  *_workspace_size returns CATCHQ_ERR_UNSUPPORTED where quantizing and catchq_gemm_nt serve
- * the call better, or alone (too few tiles of 64 x 128 outputs for the device, an output other than fp32 y). */
+ * the call better, or alone (too few tiles of 64 x 128 outputs for the device, an output other than y). */
 int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes);
 int catchq_pack_digits(const void *w, int64_t n, int64_t k, int64_t ld, void *packed, catchq_stream_t stream);
 int catchq_float_linear_digits_workspace_size(int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue, size_t *bytes);

@@ -205,6 +205,25 @@ def test_linear_on_packed_digits(m, k, n, mode, half):
     assert same_bits(ref["y"], got[rows.cuda()].cpu().numpy())
 
 
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("n,ci,side,co,stride,pad", [(12, 40, 33, 131, 1, 0), (9, 256, 24, 300, 1, 0), (9, 64, 24, 300, 1, 1),
+                                                     (20, 64, 24, 132, 2, 0)])
+def test_conv1x1_on_packed_digits(n, ci, side, co, stride, pad, half):
+    """int16 pointwise layers: as the general path has each image; padded and strided ones stay on it"""
+    note("conv digits", n, ci, side, co, stride, pad, half)
+    torch.manual_seed(n + ci + co)
+    w, b = torch.randn(co, ci, 1, 1) * 0.1, torch.randn(co)
+    x = torch.randn(n, ci, side, side).to(memory_format=torch.channels_last).cuda()
+    q_scale = torch.tensor([32767 / 4.0, 0.0] + (32767 / w.abs().amax((1, 2, 3))).tolist())
+    x = x.half() if half else x
+    args = (w.cuda(), b.cuda(), [pad, pad], [stride, stride], [1, 1], 1, q_scale, torch.tensor([4], dtype=torch.int32))
+    got = torch.ops.torch_mlu.conv2d(x, *args)
+    parts = torch.cat([torch.ops.torch_mlu.conv2d(x[i:i + 1], *args) for i in range(n)])
+    assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
+    nchw = torch.ops.torch_mlu.conv2d(x.contiguous(), *args)
+    assert same_bits(nchw.cpu().numpy(), got.cpu().numpy())
+
+
 @pytest.mark.parametrize("params_half", [False, True])
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("n,ci,side,co", [(4, 80, 25, 644), (3, 256, 24, 1024), (5, 960, 15, 1160)])
