@@ -1029,20 +1029,22 @@ void pack_filters(Prepared &p) {
   check_status(catchq_pack_filters(w.data_ptr(), n, k, p.packed.data_ptr(), current_stream()), "torch_mlu::quantize");
 }
 
-// The product of floating rows with packed filters; false: another route serves it.
+// The product of floating rows with packed filters; false: another route serves it.  (The route's lower bounds are asked here
+// too: a call of a few microseconds does not pay for the entry point's answer.)
 bool linear_packed(const void *x, int dt, const Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
                    const char *what) {
-  if (!prep.packed.defined() || m < 1024) return false;
+  if (!prep.packed.defined() || m < 1024 || m * n < 1250000) return false;
   const int st = catchq_float_linear_packed(x, dt, prep.pos_x, prep.packed.data_ptr(), m, n, k, &e, current_stream());
   if (st == CATCHQ_ERR_UNSUPPORTED) return false;
   check_status(st, what);
   return true;
 }
 
-// The same at 16 bits, through the activations' digits.
+// The same at 16 bits, through the activations' digits.  (Five eighths of a tile of 64 x 128 per unit are the least that the
+// route takes: 20 on an eighth of a device.)
 bool linear_digits(const void *x, int dt, const Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
                    const c10::Device &device, const char *what) {
-  if (prep.bw_x != 16 || !prep.packed.defined() || k < 32) return false;
+  if (prep.bw_x != 16 || !prep.packed.defined() || k < 32 || (m + 63) / 64 * ((n + 127) / 128) < 20) return false;
   size_t bytes = 0;
   int st = catchq_float_linear_digits_workspace_size(m, n, k, &e, &bytes);
   if (st == CATCHQ_OK) {
