@@ -47,7 +47,7 @@ def parse():
     ap.add_argument("--fractional-scale", action="store_true",
                     help="quantize with position and fractional scale (steps of absmax/qmax) instead of power-of-two steps")
     ap.add_argument("--streams", type=int, default=2,
-                    help="parts the batch is split into inside the HIP graph, each on a stream of its own (1: one launch sequence)")
+                    help="parts the batch is split into, each a HIP graph replayed on a stream of its own (1: one launch sequence)")
     ap.add_argument("--chain-links", type=int, default=-1,
                     help="longest residual chain recomputed inside a block's last launch (0: none, -1: the plan's own rule)")
     ap.add_argument("--fuse-blocks", action="store_true",
@@ -601,8 +601,8 @@ def main():
         assert torch.isfinite(o.float()).all()
 
     launches = plan_launches(fused, batch // args.streams, side, side)
-    config = {"workload": "%s %s, fused requant pipeline replayed from a HIP graph%s" % (
-        args.workload, what, "" if args.streams <= 1 else " (the batch in %d parts on parallel streams)" % args.streams),
+    config = {"workload": "%s %s, fused requant pipeline replayed from %s" % (
+        args.workload, what, "a HIP graph" if args.streams <= 1 else "HIP graphs (the batch in %d parts on parallel streams)" % args.streams),
               "global_batch": batch, "calibration_images": args.calib_images, "graph_streams": args.streams,
               "gop_per_step": round(2 * nets.conv_macs(layers, batch, side, side) / 1e9, 1),
               # blocks whose residual branch is recomputed from int8 tensors inside their last launch: links per launch
@@ -861,7 +861,7 @@ def extras():
 
 
 def other_networks(steps=20):
-    """the other two network configurations, each as its own fused plan replayed from a HIP graph (two parts of the
+    """the other two network configurations, each as its own fused plan replayed from HIP graphs (two parts of the
     batch on parallel streams): throughput, algorithmic bytes and integer operations of one step, fractions of the roofs"""
     import argparse as _ap
     import torch

@@ -742,15 +742,15 @@ class FusedNet(object):
         """Record one forward pass into a HIP graph; returns (static_input, replay) where replay()
         re-runs the whole network on whatever static_input holds and returns the static output(s).
 
-        streams > 1 splits the batch into that many parts, each recorded on a stream of its own (all of
-        default priority) between a fork and a join: the images are independent, so the results are the
-        same tensors, and the launches of one part fill the compute units that the other part's launches
-        leave idle while they start up and drain.  A batch whose launches are too short for that is recorded as fewer
-        parts (_parts): `streams` is the most there may be.
+        streams > 1 splits the batch into that many parts, each recorded as a graph of its own and replayed on a
+        stream of its own (all of default priority; the first on the caller's): the images are independent, so the
+        results are the same tensors, and the launches of one part fill the compute units that the other part's
+        launches leave idle while they start up and drain.  A batch whose launches are too short for that is recorded
+        as fewer parts (_parts): `streams` is the most there may be.
         parts: record exactly this many, whatever `streams` says and whether they pay or not.
         graph_parts holds the number recorded.
-        replay owns the graph and its memory: dropping it gives both back (the plan keeps no graph, so recording another
-        one destroys none)."""
+        replay owns the graphs and their memory: dropping it gives both back (the plan keeps no graph, so recording
+        another one destroys none)."""
         static_in = example.clone()
         if parts is None:
             asked = max(1, min(int(streams), static_in.shape[0]))
@@ -761,15 +761,11 @@ class FusedNet(object):
                 raise ValueError("capture: %d parts of a batch of %d" % (asked, static_in.shape[0]))
             chunks = list(static_in.tensor_split(asked))
         self.graph_parts = len(chunks)
-        # As many streams as asked for are drawn from the pool, used or not: its streams take turns on the four hardware
-        # queues, and a capture that advanced it by one left the branches of later graphs on one queue (Darknet-53 in two
-        # parts behind MobileNetV2 captures of one: 2.57 -> 3.0 ms)
-        side = [torch.cuda.Stream() for _ in range(asked)][:len(chunks)]
         # the launches recorded below will share the device: their tile shapes are chosen for a part of it (a hint
         # of this thread, handed to the kernel library with every call)
         before = torch.ops.torch_mlu.set_launch_sharing(len(chunks))
         try:
-            return self._capture(static_in, chunks, side)
+            return self._capture(static_in, chunks)
         finally:
             torch.ops.torch_mlu.set_launch_sharing(max(before, 1))
 
@@ -780,13 +776,12 @@ class FusedNet(object):
         -- has to reach 3.7 us per launch of the graph; the weights are those that put the measured cases on the right side,
         not a forecast of the time (which is 1 to 2 times as long).  Measured, one part / two (us), the smaller a batch that
         is left as one, the larger one that is split:
-          MobileNetV2 224 x 224, 32 images 332 / 343, 48 436 / 419, 64 502 / 472; 192 x 192, 27 279 / 291, 64 430 / 413
-          ResNet-50 224 x 224, 8 images 346 / 407, 20 528 / 504, 64 1074 / 992; 112 x 112, 64 457 / 468
-          ResNet-18 224 x 224, 16 images 244 / 252, 40 472 / 422; 112 x 112, 64 264 / 272
-          Darknet-53 416 x 416, 3 images 1087 / 1142, 5 1318 / 1257; 320 x 320, 4 1056 / 1087, 8 1302 / 1237
-        Near the line it is off by up to 2 % (ResNet-18, 32 images, split: 345 / 349; MobileNetV2, 40, not: 397 / 390).  These
-        are with the branches on hardware queues of their own; where the streams that a process made before put both on one,
-        each node takes 4 us (MobileNetV2 192 x 192, 27 images, two parts: 431) and a long graph is up to a third slower."""
+          MobileNetV2 224 x 224, 32 images 348 / 353, 48 441 / 426, 64 511 / 490; 192 x 192, 27 277 / 293, 64 434 / 423
+          ResNet-50 224 x 224, 8 images 343 / 365, 20 530 / 528, 64 1066 / 999; 112 x 112, 64 477 / 464 (not split)
+          ResNet-18 224 x 224, 16 images 238 / 250, 40 473 / 433; 112 x 112, 64 248 / 261
+          Darknet-53 416 x 416, 3 images 841 / 929, 5 1136 / 1106; 320 x 320, 4 806 / 813, 8 1117 / 1061
+        Near the line it is off by up to 4 % (ResNet-18, 32 images, split: 351 / 365; ResNet-50, 112 x 112, as above).  These are
+        with the parts on hardware queues of their own (_streams_beside)."""
         if parts == 1:
             return 1
         size, launches, elems, macs = {"input": (h, w)}, 0, 0, 0
@@ -810,55 +805,109 @@ class FusedNet(object):
             parts -= 1
         return parts
 
-    def _capture(self, static_in, chunks, side):
-        """Side streams only ever wait on the capturing stream (fork) and are only ever waited on by it (join).
-        Waits between two side streams in both directions inside one capture ended a capture with a segmentation
-        fault inside the runtime's end-of-capture call; nothing here may introduce such a wait."""
-        cur0 = torch.cuda.current_stream()
-        if len(set(s.cuda_stream for s in side)) != len(side) or any(s.cuda_stream == cur0.cuda_stream for s in side):
-            raise ValueError("capture: every part needs a side stream of its own, distinct from the capturing stream")
+    def _capture(self, static_in, chunks):
+        """Every part is a graph of its own, a chain of launches without branches.  The fork and the join are events between
+        the streams at each replay, outside of the graphs, so neither what a capture holds nor what a graph's launch has to
+        do depends on the streams: recorded as branches of one graph, a part whose stream was the one that the capture ran
+        on became serial, and the graph's launch cost the host 330 us where two chains cost 125 (ResNet-50, 64 images; one
+        step alone 1125 -> 1045 us, steps behind one another 983 / 985; Darknet-53, 16 images, 2470 -> 2290 and 2277 /
+        2275; MobileNetV2, 64 images, 646 -> 530 and 489 / 487)."""
+        caller = torch.cuda.current_stream()
+        recorded_on = [torch.cuda.Stream() for _ in chunks]
         sample = None
-        for st, c in zip(side, chunks):  # warm-up outside the capture, on the streams the graph will use
-            st.wait_stream(torch.cuda.current_stream())
+        for st, c in zip(recorded_on, chunks):  # warm-up outside the capture
+            st.wait_stream(caller)
             with torch.cuda.stream(st):
                 for _ in range(2):
                     sample = self.forward(c)
-        for st in side:
-            torch.cuda.current_stream().wait_stream(st)
+        for st in recorded_on:
+            caller.wait_stream(st)
         torch.cuda.synchronize()
-        # the whole batch's outputs, allocated outside the graph; every part fills its rows
-        sample_outs = sample if isinstance(sample, tuple) else (sample,)
-        whole = [torch.empty((static_in.shape[0],) + tuple(o.shape[1:]), dtype=o.dtype, device=o.device,
-                             memory_format=torch.channels_last if o.dim() == 4 else torch.contiguous_format)
-                 for o in sample_outs]  # feature maps stay NHWC in memory, like the parts' own outputs
-        graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(graph):
-            if len(chunks) == 1:
+        graphs = []
+        if len(chunks) == 1:
+            graphs.append(torch.cuda.CUDAGraph())
+            with torch.cuda.graph(graphs[0], stream=recorded_on[0]):
                 static_out = self.forward(static_in)
-            else:
-                # every part copies its outputs into its rows of the whole batch's outputs on its own stream
-                cur = torch.cuda.current_stream()
-                row = 0
-                for st, c in zip(side, chunks):
-                    st.wait_stream(cur)
-                    with torch.cuda.stream(st):
-                        out = self.forward(c)
-                        for w_, o in zip(whole, out if isinstance(out, tuple) else (out,)):
-                            w_[row:row + c.shape[0]].copy_(o)
-                    row += c.shape[0]
-                for st in side:
-                    cur.wait_stream(st)
-                static_out = tuple(whole) if isinstance(sample, tuple) else whole[0]
-        # the first replays of a new graph are slower (the executable graph is uploaded on first use): take them here
-        for _ in range(8):
-            graph.replay()
-        torch.cuda.synchronize()
+        else:
+            # the whole batch's outputs, allocated outside the graphs; every part copies its own into its rows
+            sample_outs = sample if isinstance(sample, tuple) else (sample,)
+            whole = [torch.empty((static_in.shape[0],) + tuple(o.shape[1:]), dtype=o.dtype, device=o.device,
+                                 memory_format=torch.channels_last if o.dim() == 4 else torch.contiguous_format)
+                     for o in sample_outs]  # feature maps stay NHWC in memory, like the parts' own outputs
+            static_out = tuple(whole) if isinstance(sample, tuple) else whole[0]
+            row = 0
+            for st, c in zip(recorded_on, chunks):
+                graphs.append(torch.cuda.CUDAGraph())
+                with torch.cuda.graph(graphs[-1], stream=st):
+                    out = self.forward(c)
+                    for w_, o in zip(whole, out if isinstance(out, tuple) else (out,)):
+                        w_[row:row + c.shape[0]].copy_(o)
+                row += c.shape[0]
+        side = _streams_beside(caller, len(chunks) - 1, graphs[0].replay, static_in.device)
+        fork, done = torch.cuda.Event(), [torch.cuda.Event() for _ in graphs[1:]]
 
         def replay():
-            graph.replay()
+            if not done:
+                graphs[0].replay()
+                return static_out
+            cur = torch.cuda.current_stream()
+            fork.record(cur)
+            graphs[0].replay()
+            # (one stream more than there are parts beside the caller's: the caller may be on one of them)
+            for st, graph, end in zip((s for s in side if s.cuda_stream != cur.cuda_stream), graphs[1:], done):
+                st.wait_event(fork)
+                with torch.cuda.stream(st):
+                    graph.replay()
+                    end.record(st)
+            for end in done:
+                cur.wait_event(end)
             return static_out
 
+        # the first replays of a new graph are slower (the executable graph is uploaded on first use): take them here
+        for _ in range(8):
+            replay()
+        torch.cuda.synchronize()
         return static_in, replay
+
+
+def _streams_beside(caller, count, work, device):
+    """count + 1 streams, the first `count` of them, as far as there are any, on hardware queues other than the caller's and
+    each other's (none for count 0).
+
+    A process has four hardware queues, and the pool's streams take turns on them: which queue a stream shares depends on
+    all that were drawn before.  On one queue two parts run one after the other (ResNet-50, 64 images: 1429 us a step, 977
+    on two), so the queues are looked at: a kernel behind `work` (some hundred microseconds) on a stream comes back before
+    it only if it went through another queue."""
+    if count == 0:
+        return []
+    mark = torch.zeros(1, device=device)
+    work()  # (the first one is slower)
+    torch.cuda.synchronize()
+
+    def beside(stream, other):
+        with torch.cuda.stream(other):
+            work()
+            end = other.record_event()
+        with torch.cuda.stream(stream):
+            mark.zero_()
+            back = stream.record_event()
+        back.synchronize()
+        free = not end.query()
+        end.synchronize()
+        return free
+
+    found, rest = [], []
+    for turn in range(max(2 * count, 8)):
+        st = torch.cuda.Stream()
+        if any(st.cuda_stream == s.cuda_stream for s in [caller] + found + rest):
+            continue
+        (found if turn < 8 and len(found) < count and all(beside(st, s) for s in [caller] + found) else rest).append(st)
+        if (turn >= 7 or len(found) == count) and rest and len(found) + len(rest) > count:
+            break
+    streams = (found + rest)[:count + 1]
+    if len(streams) <= count:
+        raise ValueError("capture: every part needs a side stream of its own")
+    return streams
 
 
 def calibrate(float_net, x_cpu, dtype="int8", per_channel=True):

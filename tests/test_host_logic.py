@@ -321,3 +321,114 @@ def test_per_channel_params_in_half_follow_the_tensor_ops(lib):
     out = np.empty(1, np.uint16)
     p = ctypes.c_int()
     assert lib.catchq_per_channel_params_f16(16, bad.ctypes.data, 1, ctypes.byref(p), out.ctypes.data, out.ctypes.data) == 1
+
+
+class FakeDevice(object):
+    """Streams on four queues, graphs and events as far as FusedNet.capture uses them; nothing runs.  A graph's replay keeps
+    its queue busy until somebody waits for an event behind it."""
+
+    def __init__(self, monkeypatch, drawn=0, caller=None):
+        import contextlib
+        dev = self
+
+        class Stream(object):
+            def __init__(self, number=None):
+                if number is None:
+                    number, dev.drawn = 1 + dev.drawn % 32, dev.drawn + 1
+                self.cuda_stream, self.queue = number, number % 4
+
+            def wait_stream(self, other):
+                dev.note("wait", self.cuda_stream, other.cuda_stream)
+
+            def wait_event(self, event):
+                dev.note("wait", self.cuda_stream, event.on.cuda_stream)
+
+            def record_event(self):
+                event = Event()
+                event.record(self)
+                return event
+
+        class Event(object):
+            def record(self, stream=None):
+                self.on = stream or dev.current
+                dev.note("record", self.on.cuda_stream)
+
+            def query(self):
+                return self.on.queue not in dev.busy
+
+            def synchronize(self):
+                dev.busy.discard(self.on.queue)
+
+        class Graph(object):
+            def replay(self):
+                dev.busy.add(dev.current.queue)
+                dev.launched.append((self, dev.current))
+
+        @contextlib.contextmanager
+        def stream(st):
+            before, dev.current = dev.current, st
+            yield
+            dev.current = before
+
+        @contextlib.contextmanager
+        def graph(g, stream=None):
+            dev.recording = g
+            before, dev.current = dev.current, stream or Stream(5)
+            yield
+            dev.current, dev.recording = before, None
+
+        self.drawn, self.recording, self.busy, self.launched, self.notes, self.recorded = drawn, None, set(), [], [], []
+        self.Stream = Stream
+        self.current = Stream(caller or 0)
+        for name, fake in dict(Stream=Stream, Event=Event, CUDAGraph=Graph, stream=stream, graph=graph,
+                               current_stream=lambda: self.current, synchronize=self.busy.clear).items():
+            monkeypatch.setattr(torch.cuda, name, fake)
+
+    def note(self, *what):
+        assert self.recording is None, "%s while a graph is recorded" % (what,)
+        self.notes.append(what)
+
+    def plan(self):
+        from catch_amd import pipeline
+        net = object.__new__(pipeline.FusedNet)
+
+        def forward(x):
+            if self.recording is not None:
+                self.recorded.append((self.recording, x.shape[0]))
+            return x * 2
+        net.forward = forward
+        return net
+
+
+@pytest.mark.parametrize("caller", [0, 3, 9])
+@pytest.mark.parametrize("drawn", range(9))
+@pytest.mark.parametrize("parts", [1, 2, 3, 4, 7])
+def test_parts_of_a_graph_side_by_side(monkeypatch, parts, drawn, caller):
+    """Whatever streams a process has drawn before and whichever the caller is on: nothing crosses streams while a part is
+    recorded, a part is a graph, the parts of a replay run on streams and (as far as there are any) queues of their own,
+    between an event of the caller's stream and events that it waits for"""
+    dev = FakeDevice(monkeypatch, drawn, caller)
+    net = dev.plan()
+    static_in, replay = net.capture(torch.ones(9, 2), parts=parts)
+    assert net.graph_parts == parts and [n for _, n in dev.recorded] == [len(c) for c in torch.arange(9).tensor_split(parts)]
+    graphs = [g for g, _ in dev.recorded]
+    assert len(set(map(id, graphs))) == parts
+    here = dev.current
+    sides = [st for _, st in dev.launched[-parts:]][1:]
+    for cur in [here] + sides + [dev.Stream(40)]:
+        dev.current, dev.launched, dev.notes = cur, [], []
+        out = replay()
+        assert tuple(out.shape) == (9, 2) and [g for g, _ in dev.launched] == graphs
+        used = [st for _, st in dev.launched]
+        assert used[0] is cur and len(set(st.cuda_stream for st in used)) == parts
+        if cur is here:
+            assert len(set(st.queue for st in used)) == min(parts, 4)
+        for st in used[1:]:
+            assert ("wait", st.cuda_stream, cur.cuda_stream) in dev.notes and ("wait", cur.cuda_stream, st.cuda_stream) in dev.notes
+
+
+def test_more_parts_than_streams_are_refused(monkeypatch):
+    dev = FakeDevice(monkeypatch)
+    with pytest.raises(ValueError, match="stream of its own"):
+        dev.plan().capture(torch.ones(40, 2), parts=33)
+    dev.plan().capture(torch.ones(40, 2), parts=32)
