@@ -749,8 +749,8 @@ class FusedNet(object):
         as fewer parts (_parts): `streams` is the most there may be.
         parts: record exactly this many, whatever `streams` says and whether they pay or not.
         graph_parts holds the number recorded.
-        replay owns the graphs and their memory: dropping it gives both back (the plan keeps no graph, so recording
-        another one destroys none)."""
+        replay owns the graphs, their memory and static_input: dropping it gives them back (the plan keeps no graph, so
+        recording another one destroys none)."""
         static_in = example.clone()
         if parts is None:
             asked = max(1, min(int(streams), static_in.shape[0]))
@@ -845,11 +845,12 @@ class FusedNet(object):
                 row += c.shape[0]
         side = _streams_beside(caller, len(chunks) - 1, graphs[0].replay, static_in.device)
         fork, done = torch.cuda.Event(), [torch.cuda.Event() for _ in graphs[1:]]
+        held = static_in, static_out  # the graphs read and write them: they live as long
 
         def replay():
             if not done:
                 graphs[0].replay()
-                return static_out
+                return held[1]
             cur = torch.cuda.current_stream()
             fork.record(cur)
             graphs[0].replay()
@@ -861,7 +862,7 @@ class FusedNet(object):
                     end.record(st)
             for end in done:
                 cur.wait_event(end)
-            return static_out
+            return held[1]
 
         # the first replays of a new graph are slower (the executable graph is uploaded on first use): take them here
         for _ in range(8):

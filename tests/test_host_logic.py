@@ -432,3 +432,21 @@ def test_more_parts_than_streams_are_refused(monkeypatch):
     with pytest.raises(ValueError, match="stream of its own"):
         dev.plan().capture(torch.ones(40, 2), parts=33)
     dev.plan().capture(torch.ones(40, 2), parts=32)
+
+
+def test_replay_owns_its_graphs_and_their_input(monkeypatch):
+    """the recorded launches read static_input: it lives as long as replay does, and both go with it"""
+    import gc
+    import weakref
+    dev = FakeDevice(monkeypatch)
+    static_in, replay = dev.plan().capture(torch.ones(4, 2), parts=2)
+    kept, graph = weakref.ref(static_in), weakref.ref(dev.recorded[0][0])
+    dev.launched, dev.recorded = [], []
+    gc.disable()
+    try:
+        del static_in
+        assert kept() is not None and graph() is not None
+        del replay
+        assert kept() is None and graph() is None
+    finally:
+        gc.enable()
