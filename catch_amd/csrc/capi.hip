@@ -27,6 +27,7 @@ int conv2d_dual_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
 int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                            int sh, int sw, int dh, int dw, int Ho, int Wo, const void *xs, const void *ws, int Hs, int Ws,
                            int Cs, int ss, const EpiDev &e, const ShortcutDev &sc, hipStream_t s);
+bool float_rows_takes(bool half, int64_t M, int64_t N, int64_t K, const EpiDev &e);
 int float_rows(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, const EpiDev &e,
                hipStream_t s);
 int64_t packed_digits_bytes(int64_t N, int64_t K);
@@ -382,6 +383,18 @@ CATCHQ_API int catchq_pack_filters(const void *w, int64_t n, int64_t k, void *pa
   return pack_filters(w, packed, n, k, as_stream(stream));
 }
 
+CATCHQ_API int catchq_float_linear_packed_takes(int x_dtype, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue) {
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  const int st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  size_t bytes;
+  if (m < 0) return CATCHQ_ERR_ARG;
+  if (m >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  const int sized = catchq_packed_filters_size(n, k, &bytes);
+  if (sized != CATCHQ_OK) return sized;
+  return m == 0 || float_rows_takes(x_dtype == CATCHQ_F16, m, n, k, make_epi(epilogue, m * n)) ? CATCHQ_OK : CATCHQ_ERR_UNSUPPORTED;
+}
+
 CATCHQ_API int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n,
                                           int64_t k, const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
   if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
@@ -401,7 +414,7 @@ CATCHQ_API int catchq_float_linear_packed(const void *x, int x_dtype, int x_posi
 
 CATCHQ_API int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes) {
   if (!bytes || n <= 0 || k <= 0) return CATCHQ_ERR_ARG;
-  if (k > 8192 || n >= (1ll << 31) || packed_digits_bytes(n, k) >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  if (k > kDigitsMaxK || n >= (1ll << 31) || packed_digits_bytes(n, k) >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
   *bytes = (size_t)packed_digits_bytes(n, k);
   return CATCHQ_OK;
 }

@@ -8,6 +8,7 @@
 #include <cstdlib>
 
 #include "catchq.h"
+#include "packed_rules.h"
 
 #define CATCHQ_API extern "C" __attribute__((visibility("default")))
 
@@ -21,13 +22,6 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 inline hipStream_t as_stream(catchq_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? CATCHQ_OK : CATCHQ_ERR_LAUNCH; }
-
-// compute units one launch should plan its tile shapes for: the device's 256, divided by the number of
-// launches the caller says share the device (catchq_epilogue_t::sharing)
-inline int planned_cus(int sharing) {
-  const int cus = 256 / (sharing < 1 ? 1 : sharing);
-  return cus < 1 ? 1 : cus;
-}
 
 // Allow `kern` more than the default 64 KiB of dynamic LDS: needed once per kernel and device.  `raised` is the
 // call site's own flag array (one per kernel instance); setting the attribute twice is harmless, so relaxed

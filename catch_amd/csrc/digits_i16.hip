@@ -11,7 +11,7 @@
 // preparation of a weight writes its, both in the order of the matrix instruction's lanes -- [row / 32][k / 32][high, low
 // digits], a kilobyte each --, so that every transfer is a run of memory and every LDS read is conflict-free as it lies.  A
 // block of NW waves owns 64 rows x 32 NW columns: the rows go to LDS, 256 values of K at a time and the next ones under way; a
-// wave's weights come straight into its registers, four K sub-steps of 32 ahead.  64 x 32 outputs a wave are eight matrix
+// wave's weights come straight into its registers, eight K sub-steps of 32 ahead.  64 x 32 outputs a wave are eight matrix
 // instructions for two kilobytes of weights and four LDS reads.  What bounds it: the transfers from the Infinity Cache through
 // L2 (25 B a clock and unit, a slab of 96 KB in 3700 clocks where its multiplications take 2800), the first slab (4100 clocks)
 // and the epilogue (4000).  Tried without gain: floats converted by the blocks themselves (every run of columns converts them
@@ -312,9 +312,9 @@ static int digit_epilogue(int N, const EpiDev &e) {
 // them leave units idle: 339 x 203 -> 2765 half (132 blocks) 10.3 / 11.8, 908 x 875 -> 737 half (90) 14.9 / 16.7,
 // 1202 x 2480 -> 253 (38) 19.6 / 27.4, 116 x 1514 -> 627 half (10) 10.5 / 19.0.
 int64_t gemm_digits_bytes(int64_t M, int64_t N, int64_t K, const EpiDev &e) {
-  if (K < 32 || K > 8192 || M >= (1ll << 31) - 64 || N >= (1 << 24)) return 0;
+  if (M >= (1ll << 31) - 64 || N >= (1 << 24) || !digits_sizes(M, N, K, e.cus)) return 0;
   const int64_t blocks = (M + 63) / 64 * ((N + 127) / 128), bytes = digit_bytes(M, K);
-  if (blocks * 8 < 5 * (int64_t)e.cus || blocks >= (1 << 27) || bytes >= (1ll << 31) || digit_bytes(N, K) >= (1ll << 31)) return 0;
+  if (blocks >= (1 << 27) || bytes >= (1ll << 31) || digit_bytes(N, K) >= (1ll << 31)) return 0;
   return digit_epilogue((int)N, e) ? bytes : 0;
 }
 

@@ -240,14 +240,20 @@ static int launch_float_rows(const void *a, const void *b, IgemmParams p, const 
 // round of blocks (20853 x 560 -> 572 half 25.4 / 31.4).  Else eight waves, one block a unit, and the fewest blocks that give
 // one round: every run of columns converts the rows again (14938 x 1200 -> 512 half 23.5 on all columns, 29.6 on half of
 // them; 3689 x 912 -> 2160 half 19.9 on 12 tiles, 23.0 on nine, which leave waves without a second tile).
+bool float_rows_takes(bool half, int64_t M, int64_t N, int64_t K, const EpiDev &e) {
+  if (!float_rows_sizes(M, N, K, e.y_f16 != 0)) return false;
+  if (M * K * (half ? 2 : 4) >= (1ll << 31) || (N + 31) / 32 * ((K + 31) / 32) * 1024 >= (1ll << 31) ||
+      (M + 63) / 64 * ((N + 63) / 64) >= (1ll << 31))
+    return false;
+  const int epi = pick_epilogue((int)N, e);
+  return epi == EPI_Y32 || epi == EPI_Y16 || epi == EPI_Y16_STEPS;
+}
+
 int float_rows(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, const EpiDev &e,
                hipStream_t s) {
+  if (!float_rows_takes(half, M, N, K, e)) return -1;
   const int64_t row_tiles = (M + 63) / 64, tiles = (N + 63) / 64;
-  if (K % 16 != 0 || K < 64 || K > 1312 || M < 1024 || N <= (e.y_f16 ? 512 : 256) || M * N < 1250000) return -1;
-  if (M * K * (half ? 2 : 4) >= (1ll << 31) || (N + 31) / 32 * ((K + 31) / 32) * 1024 >= (1ll << 31) || row_tiles * tiles >= (1ll << 31))
-    return -1;
   const int epi = pick_epilogue((int)N, e);
-  if (epi != EPI_Y32 && epi != EPI_Y16 && epi != EPI_Y16_STEPS) return -1;
   const int64_t rows_lds = 64 * ((K + 31) / 32 * 2 + 1) * 16;
   auto lds = [&](int nw) { return (int)(rows_lds + nw * kStageBytes); };
   const bool four = K <= 448 || (row_tiles > e.cus && 2 * lds(4) <= kLdsBytes);

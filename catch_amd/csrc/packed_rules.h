@@ -1,0 +1,26 @@
+// Which products the routes on packed weights take, by their sizes: asked by their launchers (float_rows.hip, digits_i16.hip,
+// where both sides of every bound are measured) and by the operators, which lay a weight out only for calls that will read it.
+#pragma once
+#include <cstdint>
+
+namespace catchq {
+
+// compute units one launch should plan its tile shapes for: the device's 256, divided by the number of
+// launches the caller says share the device (catchq_epilogue_t::sharing)
+inline int planned_cus(int sharing) {
+  const int cus = 256 / (sharing < 1 ? 1 : sharing);
+  return cus < 1 ? 1 : cus;
+}
+
+// int8, float_rows
+inline bool float_rows_sizes(int64_t m, int64_t n, int64_t k, bool half_out) {
+  return m >= 1024 && n > (half_out ? 512 : 256) && m * n >= 1250000 && k >= 64 && k <= 1312 && k % 16 == 0;
+}
+
+// int16, gemm_digits: five eighths of a tile of 64 x 128 outputs per unit; the digits' sums fit 32 bits up to kDigitsMaxK
+constexpr int64_t kDigitsMaxK = 8192;
+inline bool digits_sizes(int64_t m, int64_t n, int64_t k, int cus) {
+  return k >= 32 && k <= kDigitsMaxK && (m + 63) / 64 * ((n + 127) / 128) * 8 >= 5 * (int64_t)cus;
+}
+
+}  // namespace catchq

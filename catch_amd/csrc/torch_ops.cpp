@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "catchq.h"
+#include "packed_rules.h"
 
 namespace {
 
@@ -893,13 +894,20 @@ struct Prepared {
   bool params_half = false;  // per-channel parameters derived with half tensor ops (half q_scale, int8)
   int variant = 0;   // caller's layout choice for qw (part of the cache key)
   Tensor qw;         // conv: [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory; linear: [N,K]
-  Tensor packed;     // qw in the order of the matrix instruction: int8 linears and pointwise convolutions, int16 linears (digits)
   Tensor new_scale;  // device fp32 [Co] when per_channel
   Tensor rcp;        // its correctly rounded reciprocals (undefined where the kernels have to divide)
   // recorded on the stream that quantized the weight, behind those kernels: a later call on another stream
   // (another thread's, a side stream) waits for it before it reads qw / new_scale
   at::cuda::CUDAEvent ready;
   std::atomic<bool> ready_seen{false};  // the event has been seen complete: no need to ask again
+  // qw in the order of the matrix instruction (packed_weight), with a stream and an event of its own
+  std::mutex packing;
+  bool packed_asked = false;
+  Tensor packed;     // (kept as long as the entry)
+  std::atomic<const void *> packed_data{nullptr};  // set last, when it can be read on packed_on
+  c10::StreamId packed_on = 0;
+  at::cuda::CUDAEvent packed_ready;
+  bool packed_seen = false;
   Prepared() : w_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
                s_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)),
                m_impl(c10::weak_intrusive_ptr<c10::TensorImpl>::reclaim(nullptr)) {}
@@ -1009,47 +1017,95 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
   return p;
 }
 
-// Weights of the shapes that catchq_float_linear_packed (8 bits) and catchq_float_linear_digits (16) may take, laid out for
-// them: once per weight, so only where the entry is kept.
-void pack_filters(Prepared &p) {
-  const Tensor &w = p.qw;
-  if (p.bw_x != p.bw_w || w.dim() < 2) return;
-  const int64_t n = w.size(0), k = w.size(1);
-  if (p.bw_w == 16) {
-    size_t bytes = 0;
-    if (w.numel() != n * k || n == 0 || k < 32 || catchq_packed_digits_size(n, k, &bytes) != CATCHQ_OK) return;
-    p.packed = device_empty({(int64_t)bytes}, at::kChar, w.device());
-    check_status(catchq_pack_digits(w.data_ptr(), n, k, k, p.packed.data_ptr(), current_stream()), "torch_mlu::quantize");
-    return;
-  }
-  if (n <= 256 || k < 64 || k > 1312 || k % 16 != 0 || w.numel() != n * k) return;
-  size_t bytes = 0;
-  if (catchq_packed_filters_size(n, k, &bytes) != CATCHQ_OK) return;
-  p.packed = device_empty({(int64_t)bytes}, at::kChar, w.device());
-  check_status(catchq_pack_filters(w.data_ptr(), n, k, p.packed.data_ptr(), current_stream()), "torch_mlu::quantize");
+bool capturing(const c10::hip::HIPStreamMasqueradingAsCUDA &stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream.stream(), &status) == hipSuccess) return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
 }
 
-// The product of floating rows with packed filters; false: another route serves it.  (The route's lower bounds are asked here
-// too: a call of a few microseconds does not pay for the entry point's answer.)
-bool linear_packed(const void *x, int dt, const Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
+// While it lives, a capture of this thread lets calls pass that only ask.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+// The entry's weight as catchq_float_linear_packed (8 bits) and catchq_float_linear_digits (16) read it; null: the call goes
+// without.  The weight is laid out at the second call that the route takes.  A caller that rewrites its weight between calls, or
+// uses it once, does not pay for that (6 us of kernel, a launch and an allocation: first pass of 1 x 768 -> 3072 on a new
+// weight 226 us with it, 218 without), and a weight whose calls do not take the route is not held twice.
+template <typename Takes>
+const void *packed_weight(Prepared &p, Takes takes) {
+  const auto cur = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
+  const void *data = p.packed_data.load(std::memory_order_acquire);
+  if (data && cur.id() == p.packed_on) return data;
+  std::lock_guard<std::mutex> lock(p.packing);
+  if (!p.packed.defined()) {
+    if (!takes()) return nullptr;
+    const bool first = !p.packed_asked;
+    p.packed_asked = true;
+    if (first || capturing(cur)) return nullptr;  // (what a capture lays out is not there before its graph is replayed)
+    const int64_t n = p.qw.size(0), k = p.qw.numel() / n;
+    size_t bytes = 0;
+    const bool digits = p.bw_w == 16;
+    if ((digits ? catchq_packed_digits_size(n, k, &bytes) : catchq_packed_filters_size(n, k, &bytes)) != CATCHQ_OK) return nullptr;
+    Tensor packed;
+    try {
+      packed = device_empty({(int64_t)bytes}, at::kChar, p.qw.device());
+    } catch (const c10::OutOfMemoryError &) {
+      return nullptr;  // (the other routes need no second copy)
+    }
+    check_status(digits ? catchq_pack_digits(p.qw.data_ptr(), n, k, k, packed.data_ptr(), current_stream())
+                        : catchq_pack_filters(p.qw.data_ptr(), n, k, packed.data_ptr(), current_stream()),
+                 "torch_mlu::quantize");
+    p.packed_on = cur.id();
+    p.packed_ready.record(cur);
+    p.packed = packed;
+    p.packed_data.store(packed.data_ptr(), std::memory_order_release);
+    return packed.data_ptr();
+  }
+  if (cur.id() != p.packed_on) {  // as in prepared_for
+    if (!p.packed_seen) {
+      {
+        RelaxedCapture asking;
+        p.packed_seen = p.packed_ready.query();
+      }
+      if (!p.packed_seen) {
+        if (capturing(cur)) return nullptr;  // (a capture cannot wait for what was recorded outside of it)
+        p.packed_ready.block(cur);
+      }
+    }
+    p.packed.record_stream(cur);
+  }
+  return p.packed.data_ptr();
+}
+
+// The product of floating rows with packed filters; false: another route serves it.
+bool linear_packed(const void *x, int dt, Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
                    const char *what) {
-  if (!prep.packed.defined() || m < 1024 || m * n < 1250000) return false;
-  const int st = catchq_float_linear_packed(x, dt, prep.pos_x, prep.packed.data_ptr(), m, n, k, &e, current_stream());
+  if (!catchq::float_rows_sizes(m, n, k, e.y_dtype == CATCHQ_F16) || prep.bw_x != 8 || prep.bw_w != 8 ||
+      (reinterpret_cast<uintptr_t>(x) & 15u) != 0)
+    return false;
+  const void *packed = packed_weight(prep, [&] { return catchq_float_linear_packed_takes(dt, m, n, k, &e) == CATCHQ_OK; });
+  if (!packed) return false;
+  const int st = catchq_float_linear_packed(x, dt, prep.pos_x, packed, m, n, k, &e, current_stream());
   if (st == CATCHQ_ERR_UNSUPPORTED) return false;
   check_status(st, what);
   return true;
 }
 
-// The same at 16 bits, through the activations' digits.  (Five eighths of a tile of 64 x 128 per unit are the least that the
-// route takes: 20 on an eighth of a device.)
-bool linear_digits(const void *x, int dt, const Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
+// The same at 16 bits, through the activations' digits.
+bool linear_digits(const void *x, int dt, Prepared &prep, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t &e,
                    const c10::Device &device, const char *what) {
-  if (prep.bw_x != 16 || !prep.packed.defined() || k < 32 || (m + 63) / 64 * ((n + 127) / 128) < 20) return false;
+  if (!catchq::digits_sizes(m, n, k, catchq::planned_cus(e.sharing)) || prep.bw_x != 16 || prep.bw_w != 16) return false;
   size_t bytes = 0;
   int st = catchq_float_linear_digits_workspace_size(m, n, k, &e, &bytes);
   if (st == CATCHQ_OK) {
+    const void *packed = packed_weight(prep, [] { return true; });
+    if (!packed) return false;
     Tensor digits = device_empty({(int64_t)bytes}, at::kChar, device);
-    st = catchq_float_linear_digits(x, dt, prep.pos_x, prep.packed.data_ptr(), m, n, k, &e, digits.data_ptr(), bytes, current_stream());
+    st = catchq_float_linear_digits(x, dt, prep.pos_x, packed, m, n, k, &e, digits.data_ptr(), bytes, current_stream());
   }
   if (st == CATCHQ_ERR_UNSUPPORTED) return false;
   check_status(st, what);
@@ -1075,7 +1131,7 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_sca
           // read on another stream than the one the caching allocator knows these blocks by: tell it, so that
           // an entry dropped while this stream's kernels still read it is not handed out again too early
           it->second->qw.record_stream(cur);
-          for (const Tensor *t : {&it->second->packed, &it->second->new_scale, &it->second->rcp})
+          for (const Tensor *t : {&it->second->new_scale, &it->second->rcp})
             if (t->defined()) t->record_stream(cur);
         }
         return it->second;
@@ -1084,7 +1140,6 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_sca
     }
   }
   auto p = prepare(make_dense, weight, q_scale, q_mode);
-  if (use_cache) pack_filters(*p);
   p->variant = variant;
   const auto made_on = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
   p->made_on = made_on.id();
@@ -1151,7 +1206,7 @@ catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64
 
 // quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x) x prepared weight -> floating
 // output, logical [N,Co,Ho,Wo] over NHWC memory
-Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, const Prepared &prep, const Tensor &bias,
+Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Prepared &prep, const Tensor &bias,
                      at::IntArrayRef padding, at::IntArrayRef stride, at::IntArrayRef dilation, int64_t groups, bool half) {
   TORCH_CHECK(padding.size() == 2 && stride.size() == 2 && dilation.size() == 2, "2-d conv parameters expected");
   const Tensor &qw = prep.qw;  // [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory
@@ -1232,7 +1287,7 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   Tensor qx;
   if (input.is_contiguous(at::MemoryFormat::ChannelsLast) &&
       ((prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0) ||
-       (prep->bw_x == 16 && prep->bw_w == 16 && ci % 8 == 0 && dense && kw == 1 && weight.size(2) == 1 && prep->packed.defined())))
+       (prep->bw_x == 16 && prep->bw_w == 16 && ci % 8 == 0 && dense && kw == 1 && weight.size(2) == 1)))
     return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), input.size(2), input.size(3), ci}, *prep, bias, padding, stride,
                          dilation, groups, half);
   if (few && prep->bw_x == 8 && can_frame) {

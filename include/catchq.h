@@ -260,9 +260,11 @@ int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_position, const v
 /* The same for a linear (a pointwise convolution of unit stride: m pixels) whose int8 filters were laid out once in the order
  * of the matrix instruction: catchq_pack_filters writes catchq_packed_filters_size bytes from w [n,k], k a multiple of 16.
  * x [m,k] fp32/fp16, y [m,n].  CATCHQ_ERR_UNSUPPORTED: catchq_float_conv2d_nhwc on the filters as they are serves the call
- * better, or alone (few rows or columns, long rows, an output other than y). */
+ * better, or alone (few rows or columns, long rows, an output other than y); *_takes answers so without a launch, for a
+ * caller that has not laid the filters out yet. */
 int catchq_packed_filters_size(int64_t n, int64_t k, size_t *bytes);
 int catchq_pack_filters(const void *w, int64_t n, int64_t k, void *packed, catchq_stream_t stream);
+int catchq_float_linear_packed_takes(int x_dtype, int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue);
 int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n, int64_t k,
                                const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 

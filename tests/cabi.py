@@ -89,6 +89,7 @@ def _epilogue(shape, device, exp2, chan_div, bias, resid, act, y_dtype, want_acc
     e.exp2 = exp2
     e.chan_div, e.chan_rcp, e.bias, e.resid = ptr(chan_div), ptr(chan_rcp), ptr(bias), ptr(resid)
     e.act = act
+    e.bias_dtype = F16 if bias is not None and bias.dtype == torch.float16 else F32
     if y_dtype is not None:
         out["y"] = torch.empty(shape, dtype=y_dtype, device=device)
         e.y, e.y_dtype = ptr(out["y"]), (F16 if y_dtype == torch.float16 else F32)
@@ -144,6 +145,43 @@ def float_conv2d_nhwc(x, x_pos, w, padding=(0, 0), stride=(1, 1), dilation=(1, 1
     ws = torch.empty(max(sz.value, 16), dtype=torch.int8, device=x.device)
     check(lib().catchq_float_conv2d_nhwc(ptr(x), dt(x), x_pos, ptr(w), ctypes.byref(d), ctypes.byref(e), ptr(ws), sz.value, stream()))
     return out, sz.value
+
+
+def pack_filters(w):
+    n, k = w.shape
+    sz = ctypes.c_size_t()
+    check(lib().catchq_packed_filters_size(n, k, ctypes.byref(sz)))
+    packed = torch.empty(sz.value, dtype=torch.int8, device=w.device)
+    check(lib().catchq_pack_filters(ptr(w), n, k, ptr(packed), stream()))
+    return packed
+
+
+def float_linear_packed(x, x_pos, packed, n, exp2=0, chan_div=None, bias=None, y_dtype=torch.float32, chan_rcp=None, q_bw=0):
+    """-> (status of the query, status of the call, outputs)"""
+    m, k = x.shape
+    e, out = _epilogue((m, n), x.device, exp2, chan_div, bias, None, 0, y_dtype, False, q_bw, 0, 1.0, chan_rcp)
+    takes = lib().catchq_float_linear_packed_takes(dt(x), m, n, k, ctypes.byref(e))
+    return takes, lib().catchq_float_linear_packed(ptr(x), dt(x), x_pos, ptr(packed), m, n, k, ctypes.byref(e), stream()), out
+
+
+def pack_digits(w, k):
+    n, ld = w.shape
+    sz = ctypes.c_size_t()
+    check(lib().catchq_packed_digits_size(n, k, ctypes.byref(sz)))
+    packed = torch.empty(sz.value, dtype=torch.int8, device=w.device)
+    check(lib().catchq_pack_digits(ptr(w), n, k, ld, ptr(packed), stream()))
+    return packed
+
+
+def float_linear_digits(x, x_pos, packed, n, exp2=0, chan_div=None, bias=None, y_dtype=torch.float32, chan_rcp=None, short=0, q_bw=0):
+    """-> (status of the query, status of the call with `short` bytes of workspace less than asked for, outputs)"""
+    m, k = x.shape
+    e, out = _epilogue((m, n), x.device, exp2, chan_div, bias, None, 0, y_dtype, False, q_bw, 0, 1.0, chan_rcp)
+    sz = ctypes.c_size_t()
+    asked = lib().catchq_float_linear_digits_workspace_size(m, n, k, ctypes.byref(e), ctypes.byref(sz))
+    ws = torch.empty(max(sz.value, 16), dtype=torch.int8, device=x.device)
+    return asked, lib().catchq_float_linear_digits(ptr(x), dt(x), x_pos, ptr(packed), m, n, k, ctypes.byref(e), ptr(ws),
+                                                   max(sz.value - short, 0), stream()), out
 
 
 def conv2d_shortcut_nhwc(x, w, sx, sw, sc_stride, sc_exp2, sc_chan_div=None, sc_bias=None, sc_chan_rcp=None, padding=(0, 0),

@@ -41,6 +41,25 @@ def same_bits(a, b):
     return a.shape == b.shape and a.dtype == b.dtype and np.array_equal(a.view(np.uint8), b.view(np.uint8))
 
 
+def held():
+    """bytes asked of the allocator and not given back"""
+    return torch.cuda.memory_stats()["requested_bytes.all.current"]
+
+
+def on_packed_weight(op, x, w, *args):
+    """the op on its packed weight: laid out at the second call that reads it, which holds that much more memory then"""
+    first, before = op(x, w, *args), held()
+    got = op(x, w, *args)
+    size = got.numel() * got.element_size()
+    assert held() - before >= size + w.numel(), "the weight was not packed"
+    before = held()
+    again = op(x, w, *args)
+    assert held() - before == size
+    for y in (first, again):
+        assert same_bits(y.cpu().numpy(), got.cpu().numpy())
+    return got
+
+
 def calibrate(model, x, bw, per_channel):
     qconfig = {"use_avg": False, "data_scale": 1.0, "per_channel": per_channel, "firstconv": False}
     calib = quantize_dynamic_mlu(model, qconfig, dtype=bw, gen_quant=True)
@@ -171,7 +190,7 @@ def test_linear_on_packed_filters(m, k, n, mode, half):
     x = x.half() if half else x
     q_scale, q_mode = torch.tensor(q_scale), torch.tensor([mode], dtype=torch.int32)
     xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
-    got = torch.ops.torch_mlu.linear(xd, wd, bd, q_scale, q_mode)
+    got = on_packed_weight(torch.ops.torch_mlu.linear, xd, wd, bd, q_scale, q_mode)
     parts = torch.cat([torch.ops.torch_mlu.linear(xd[i:i + 600], wd, bd, q_scale, q_mode) for i in range(0, m, 600)])
     assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
     rows = torch.tensor([0, 5, m - 1])
@@ -197,19 +216,23 @@ def test_linear_on_packed_digits(m, k, n, mode, half):
     x = x.half() if half else x
     q_scale, q_mode = torch.tensor(q_scale), torch.tensor([mode], dtype=torch.int32)
     xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
-    got = torch.ops.torch_mlu.linear(xd, wd, bd, q_scale, q_mode)
+    got = on_packed_weight(torch.ops.torch_mlu.linear, xd, wd, bd, q_scale, q_mode)
     parts = torch.cat([torch.ops.torch_mlu.linear(xd[i:i + 300], wd, bd, q_scale, q_mode) for i in range(0, m, 300)])
     assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
     rows = torch.tensor([0, 5, m - 2, m - 1])
     ref = oops.linear(x[rows].float().numpy(), w.numpy(), b.numpy(), q_scale.numpy(), q_mode.numpy())
     assert same_bits(ref["y"], got[rows.cuda()].cpu().numpy())
+    bh = bd.half()
+    assert same_bits(torch.ops.torch_mlu.linear(xd, wd, bh.float(), q_scale, q_mode).cpu().numpy(),
+                     torch.ops.torch_mlu.linear(xd, wd, bh, q_scale, q_mode).cpu().numpy())
 
 
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("n,ci,side,co,stride,pad", [(12, 40, 33, 131, 1, 0), (9, 256, 24, 300, 1, 0), (9, 64, 24, 300, 1, 1),
                                                      (20, 64, 24, 132, 2, 0)])
 def test_conv1x1_on_packed_digits(n, ci, side, co, stride, pad, half):
-    """int16 pointwise layers: as the general path has each image; padded and strided ones stay on it"""
+    """int16 pointwise layers: as the general path has each image and the oracle some pixels; padded and strided ones stay on
+    the general path, their weight is not packed"""
     note("conv digits", n, ci, side, co, stride, pad, half)
     torch.manual_seed(n + ci + co)
     w, b = torch.randn(co, ci, 1, 1) * 0.1, torch.randn(co)
@@ -217,7 +240,16 @@ def test_conv1x1_on_packed_digits(n, ci, side, co, stride, pad, half):
     q_scale = torch.tensor([32767 / 4.0, 0.0] + (32767 / w.abs().amax((1, 2, 3))).tolist())
     x = x.half() if half else x
     args = (w.cuda(), b.cuda(), [pad, pad], [stride, stride], [1, 1], 1, q_scale, torch.tensor([4], dtype=torch.int32))
-    got = torch.ops.torch_mlu.conv2d(x, *args)
+    if pad == 0 and stride == 1:
+        got = on_packed_weight(torch.ops.torch_mlu.conv2d, x, *args)
+        bh = b.cuda().half()
+        assert same_bits(torch.ops.torch_mlu.conv2d(x, args[0], bh.float(), *args[2:]).cpu().numpy(),
+                         torch.ops.torch_mlu.conv2d(x, args[0], bh, *args[2:]).cpu().numpy())
+    else:
+        got = torch.ops.torch_mlu.conv2d(x, *args)
+    corner = x[:1, :, :4, :4].cpu().contiguous()
+    ref = oops.conv2d(corner.numpy(), w.numpy(), b.numpy(), (pad, pad), (stride, stride), (1, 1), 1, q_scale.numpy(), [4])["y"]
+    assert same_bits(ref[:, :, :2, :2], got[:1, :, :2, :2].cpu().numpy())
     parts = torch.cat([torch.ops.torch_mlu.conv2d(x[i:i + 1], *args) for i in range(n)])
     assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
     nchw = torch.ops.torch_mlu.conv2d(x.contiguous(), *args)
@@ -228,7 +260,8 @@ def test_conv1x1_on_packed_digits(n, ci, side, co, stride, pad, half):
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("n,ci,side,co", [(4, 80, 25, 644), (3, 256, 24, 1024), (5, 960, 15, 1160)])
 def test_conv1x1_on_packed_filters(n, ci, side, co, half, params_half):
-    """pointwise layers of unit stride, fp32 and half outputs, half steps: as the general path has each image"""
+    """pointwise layers of unit stride, fp32 and half outputs, half steps: as the general path has each image and the oracle
+    some pixels"""
     note("conv packed", n, ci, side, co, half, params_half)
     torch.manual_seed(n + ci + co)
     w, b = torch.randn(co, ci, 1, 1) * 0.1, torch.randn(co)
@@ -239,9 +272,173 @@ def test_conv1x1_on_packed_filters(n, ci, side, co, half, params_half):
         w, b, q_scale = w.half(), b.half(), q_scale.half()
     x = x.half() if half else x
     args = (w.cuda(), b.cuda(), [0, 0], [1, 1], [1, 1], 1, q_scale, q_mode)
-    got = torch.ops.torch_mlu.conv2d(x, *args)
+    got = on_packed_weight(torch.ops.torch_mlu.conv2d, x, *args)
     parts = torch.cat([torch.ops.torch_mlu.conv2d(x[i:i + 1], *args) for i in range(n)])
     assert same_bits(parts.cpu().numpy(), got.cpu().numpy())
+    corner = x[:1, :, :2, :2].cpu().contiguous()
+    if half and params_half:
+        want = ref_order.conv2d_per_channel(corner, w, b, [0, 0], [1, 1], [1, 1], 1, q_scale, q_mode.numpy())["y"].contiguous().numpy()
+    elif not params_half:
+        want = oops.conv2d(corner.numpy(), w.numpy(), b.numpy(), (0, 0), (1, 1), (1, 1), 1, q_scale.numpy(), q_mode.numpy())["y"]
+    else:
+        return  # (fp32 activations with half parameters: derived in half, applied in fp32)
+    assert same_bits(want, got[:1, :, :2, :2].cpu().numpy())
+
+
+def _packed_case(bits, m=1300, k=768, n=1024, seed=5):
+    """a linear that takes the packed route at either width"""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.1
+    x, b = torch.randn(m, k, generator=g, device="cuda"), torch.randn(n, generator=g, device="cuda")
+    top = 127.0 if bits == 8 else 32767.0
+    args = (b, torch.tensor([top / 4.0, top / 0.5]), torch.tensor([1 if bits == 8 else 2], dtype=torch.int32))
+    return x, w, args
+
+
+def _rows(x, w, args, step=100):
+    """the same product a few rows at a time, which the packed routes do not take"""
+    return torch.cat([torch.ops.torch_mlu.linear(x[i:i + step], w, *args) for i in range(0, len(x), step)])
+
+
+@pytest.mark.parametrize("name,op", [
+    ("few rows", lambda: (torch.ops.torch_mlu.linear,) + _flat(_packed_case(8, m=64))),
+    ("few rows, int16", lambda: (torch.ops.torch_mlu.linear,) + _flat(_packed_case(16, m=64))),
+    ("padded K", lambda: (torch.ops.torch_mlu.linear,) + _flat(_packed_case(8, m=2000, k=1000))),
+    ("columns not a multiple of four", lambda: (torch.ops.torch_mlu.linear,) + _flat(_packed_case(8, m=2000, n=1001))),
+    ("rows that do not start on 16 bytes", lambda: (torch.ops.torch_mlu.linear,) + _flat(_packed_case(8), shift=True)),
+    ("strided", lambda: _conv_case([0, 0], [2, 2], 1, True)), ("padded", lambda: _conv_case([1, 1], [1, 1], 1, True)),
+    ("grouped", lambda: _conv_case([0, 0], [1, 1], 2, True)), ("NCHW", lambda: _conv_case([0, 0], [1, 1], 1, False)),
+])
+def test_weights_that_no_packed_route_reads_are_not_packed(name, op):
+    note("not packed", name)
+    fn, *args = op()
+    torch.ops.torch_mlu.clear_weight_cache()
+    before = held()
+    fn(*args)
+    once = held()
+    assert once - before < args[1].numel() * (3 if "int16" in name else 1.5)  # the quantized weight
+    for _ in range(3):
+        fn(*args)
+    assert held() == once
+
+
+def _flat(case, shift=False):
+    x, w, args = case
+    if shift:
+        wide = torch.empty(x.numel() + 1, device="cuda")
+        wide[1:] = x.reshape(-1)
+        x = wide[1:].view(x.shape)
+    return (x, w) + args
+
+
+def _conv_case(pad, stride, groups, nhwc):
+    g = torch.Generator(device="cuda").manual_seed(3)
+    x = torch.randn(4, 256, 48, 48, generator=g, device="cuda")
+    w = torch.randn(1024, 256 // groups, 1, 1, generator=g, device="cuda") * 0.1
+    b = torch.randn(1024, generator=g, device="cuda")
+    x = x.contiguous(memory_format=torch.channels_last) if nhwc else x
+    return (torch.ops.torch_mlu.conv2d, x, w, b, pad, stride, [1, 1], groups, torch.tensor([127 / 4.0, 127 / 0.5]),
+            torch.tensor([1], dtype=torch.int32))
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+def test_packed_weight_follows_the_weight(bits):
+    """written in place, quantized with other parameters, dropped from the cache: the packed weight goes with the quantized one"""
+    note("packed weight, updates", bits)
+    x, w, args = _packed_case(bits)
+    linear = torch.ops.torch_mlu.linear
+    for turn in range(3):
+        want = _rows(x, w, args)
+        for call in range(3):
+            assert torch.equal(linear(x, w, *args), want), (turn, call)
+        w.mul_(-0.5)
+    other = (args[0], args[1] * 2, args[2])
+    want = _rows(x, w, other)
+    for call in range(3):
+        assert torch.equal(linear(x, w, *other), want), call
+    torch.ops.torch_mlu.clear_weight_cache()
+    for call in range(3):
+        assert torch.equal(linear(x, w, *other), want), call
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+def test_packed_weight_on_several_streams(bits):
+    """quantized on one stream, packed on the next, read on a third, nothing waited for in between; then dropped and its memory
+    used again while the last one still reads it"""
+    note("packed weight, streams", bits)
+    linear = torch.ops.torch_mlu.linear
+    for rep in range(4):
+        x, w, args = _packed_case(bits, seed=rep)
+        want = _rows(x, w, args)
+        torch.ops.torch_mlu.clear_weight_cache()
+        torch.cuda.synchronize()
+        outs = []
+        for _ in range(4):
+            with torch.cuda.stream(torch.cuda.Stream()):
+                outs.append(linear(x, w, *args))
+        torch.ops.torch_mlu.clear_weight_cache()
+        noise = [torch.full((1 << 20,), 3, dtype=torch.int8, device="cuda") for _ in range(8)]
+        torch.cuda.synchronize()
+        for i, y in enumerate(outs):
+            assert torch.equal(y, want), (rep, i)
+        del noise
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+def test_packed_weight_from_several_threads(bits):
+    import threading
+    note("packed weight, threads", bits)
+    linear = torch.ops.torch_mlu.linear
+    for rep in range(3):
+        x, w, args = _packed_case(bits, seed=rep)
+        want = _rows(x, w, args)
+        torch.ops.torch_mlu.clear_weight_cache()
+        torch.cuda.synchronize()
+        errors, gate = [], threading.Barrier(4)
+
+        def work(t):
+            try:
+                with torch.cuda.stream(torch.cuda.Stream()):
+                    gate.wait()
+                    for i in range(6):
+                        y = linear(x, w, *args)
+                        torch.cuda.current_stream().synchronize()
+                        if not torch.equal(y, want):
+                            errors.append((t, i))
+                    torch.cuda.current_stream().synchronize()
+            except Exception as exc:  # noqa: BLE001
+                errors.append(repr(exc))
+        threads = [threading.Thread(target=work, args=(t,)) for t in range(4)]
+        for th in threads:
+            th.start()
+        for th in threads:
+            th.join()
+        assert not errors, errors
+
+
+@pytest.mark.parametrize("calls", [1, 2, 3])
+@pytest.mark.parametrize("bits", [8, 16])
+def test_captured_layer_and_its_packed_weight(bits, calls):
+    """captured after one call (nothing is laid out inside the capture: the graph takes the general route) and after more (it
+    reads the packed weight); eager calls in between pack what is not packed"""
+    note("packed weight, captured", bits, calls)
+    x, w, args = _packed_case(bits)
+    linear = torch.ops.torch_mlu.linear
+    want = _rows(x, w, args)
+    torch.ops.torch_mlu.clear_weight_cache()
+    for _ in range(calls):
+        assert torch.equal(linear(x, w, *args), want)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = linear(x, w, *args)
+    for i in range(4):
+        assert torch.equal(linear(x, w, *args), want), "eager %d" % i
+        torch.cuda.synchronize()
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), "replay %d" % i
 
 
 def test_conv2d_cnnl_encoding_int16_act_int8_weight():

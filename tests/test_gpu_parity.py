@@ -1688,3 +1688,70 @@ def test_conv_input_beyond_32_bit_offsets():
         assert same_bits(want[:, first:last], got), (img, h0)
     del x, out
     torch.cuda.empty_cache()
+
+
+OK, ERR_ARG, UNSUPPORTED = 0, 1, 6  # catchq_status_t
+
+
+@pytest.mark.parametrize("x_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("y_dtype", [torch.float32, torch.float16])
+def test_packed_filters_entry_points(x_dtype, y_dtype):
+    """a call inside the route's sizes runs on it, one just outside is answered without a launch"""
+    note("packed filters, C ABI", x_dtype, y_dtype)
+    r = rng(7)
+    m, n, k = 1100, 1160, 80
+    x = (r.standard_normal((m, k)) * 3).astype(np.float16)
+    w = _ints(r, (n, k), 8)
+    div, bias = r.uniform(0.6, 3.5, n).astype(np.float32), r.standard_normal(n).astype(np.float32)
+    xd, wd = cabi.dev(x).to(x_dtype), cabi.dev(w)
+    packed = cabi.pack_filters(wd)
+    args = dict(chan_div=cabi.dev(div), bias=cabi.dev(bias), chan_rcp=cabi.dev(np.float32(1) / div), y_dtype=y_dtype)
+    takes, st, out = cabi.float_linear_packed(xd, -4, packed, n, exp2=-10, **args)
+    assert (takes, st) == (OK, OK)
+    acc, _ = orc.gemm_nt(orc.quantize(x, 8, -4), w)
+    y = orc.epilogue(acc, -10, div, bias)
+    assert same_bits(y.astype(np.float16) if y_dtype == torch.float16 else y, out["y"].cpu().numpy())
+    assert cabi.float_linear_packed(xd[:1023], -4, packed, n, **args)[:2] == (UNSUPPORTED, UNSUPPORTED)  # rows
+    for odd in (n - 1, 256):  # columns not a multiple of four, too few
+        assert cabi.float_linear_packed(xd, -4, packed, odd, y_dtype=y_dtype)[:2] == (UNSUPPORTED, UNSUPPORTED)
+    assert cabi.float_linear_packed(xd, -4, packed, n, y_dtype=None, q_bw=8)[:2] == (UNSUPPORTED, UNSUPPORTED)  # another output
+    wide = torch.zeros(m * k + 1, dtype=x_dtype, device="cuda")
+    assert cabi.float_linear_packed(wide[1:].view(m, k), -4, packed, n, **args)[:2] == (OK, UNSUPPORTED)  # not on 16 bytes
+    sz = ctypes.c_size_t()
+    lib = cabi.lib()
+    assert lib.catchq_packed_filters_size(64, 72, ctypes.byref(sz)) == UNSUPPORTED
+    assert lib.catchq_packed_filters_size(0, 64, ctypes.byref(sz)) == ERR_ARG
+    assert lib.catchq_pack_filters(ctypes.c_void_p(wd.data_ptr() + 1), n, k, cabi.ptr(packed), cabi.stream()) == ERR_ARG
+
+
+@pytest.mark.parametrize("half_bias", [False, True])
+@pytest.mark.parametrize("y_dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("n", [1160, 1001])
+def test_packed_digits_entry_points(n, y_dtype, half_bias):
+    """weights inside longer rows, halfs and floats, biases of either precision; a workspace that is too small, weights and
+    workspaces off 16 bytes and calls outside the route's sizes are answered without a launch"""
+    note("packed digits, C ABI", n, y_dtype, half_bias)
+    r = rng(n)
+    m, k, ld = 1290, 203, 217
+    x = (r.standard_normal((m, k)) * 3).astype(np.float16)
+    wide = _ints(r, (n, ld), 16)
+    w = np.ascontiguousarray(wide[:, :k])
+    div, bias = r.uniform(0.6, 3.5, n).astype(np.float32), r.standard_normal(n).astype(np.float16)
+    packed = cabi.pack_digits(cabi.dev(wide), k)
+    assert torch.equal(packed, cabi.pack_digits(cabi.dev(w), k))
+    acc, _ = orc.gemm_nt(orc.quantize(x, 16, -12), w)
+    y = orc.epilogue(acc, -26, div, bias.astype(np.float32))
+    args = dict(exp2=-26, chan_div=cabi.dev(div), chan_rcp=cabi.dev(np.float32(1) / div), y_dtype=y_dtype,
+                bias=cabi.dev(bias) if half_bias else cabi.dev(bias.astype(np.float32)))
+    for xd in (cabi.dev(x), cabi.dev(x).float()):
+        asked, st, out = cabi.float_linear_digits(xd, -12, packed, n, **args)
+        assert (asked, st) == (OK, OK)
+        assert same_bits(y.astype(np.float16) if y_dtype == torch.float16 else y, out["y"].cpu().numpy())
+    assert cabi.float_linear_digits(xd, -12, packed, n, short=1, **args)[:2] == (OK, ERR_ARG)
+    assert cabi.float_linear_digits(xd, -12, packed[1:], n, **args)[:2] == (OK, ERR_ARG)
+    assert cabi.float_linear_digits(xd[:64], -12, packed, n, **args)[:2] == (UNSUPPORTED, UNSUPPORTED)
+    assert cabi.float_linear_digits(xd, -12, packed, n, y_dtype=None, q_bw=16)[:2] == (UNSUPPORTED, UNSUPPORTED)
+    lib, sz = cabi.lib(), ctypes.c_size_t()
+    assert lib.catchq_packed_digits_size(64, 8193, ctypes.byref(sz)) == UNSUPPORTED
+    assert lib.catchq_pack_digits(cabi.ptr(packed), n, k, k - 1, cabi.ptr(packed), cabi.stream()) == ERR_ARG
+    assert lib.catchq_pack_digits(cabi.ptr(packed), n, k, k, ctypes.c_void_p(packed.data_ptr() + 2), cabi.stream()) == ERR_ARG
