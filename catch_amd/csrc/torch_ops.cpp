@@ -952,10 +952,16 @@ c10::weak_intrusive_ptr<c10::TensorImpl> weak_of(const Tensor &t) {
   return c10::weak_intrusive_ptr<c10::TensorImpl>(t.getIntrusivePtr());
 }
 
+// a weight that is used as make_dense returns it
+struct AsItIs {
+  int64_t operator()(int) const { return 0; }
+};
+
 // Decode the two q-param encodings and quantize the weight (make_dense(weight, activation bit width)
-// returns it dense, dim 0 slowest, in the layout the caller's kernel wants).
-template <typename MakeDense>
-std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, const Tensor &q_scale,
+// returns it dense, dim 0 slowest, in the layout the caller's kernel wants).  row_length(activation bit width): values in a
+// row of the quantized weight, zeros behind those of a [N,K] weight's row; 0: as many as it has.
+template <typename MakeDense, typename RowLength>
+std::shared_ptr<Prepared> prepare(MakeDense make_dense, RowLength row_length, const Tensor &weight, const Tensor &q_scale,
                                   const Tensor &q_mode) {
   auto p = std::make_shared<Prepared>();
   Tensor s_host = q_scale.to(at::kCPU).to(at::kFloat).contiguous();
@@ -971,6 +977,17 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
     bw_act = (int)s[0];
   }
   const Tensor w_dense = make_dense(weight, bw_act);
+  const int64_t row = row_length(bw_act), pad = row > 0 && w_dense.numel() > 0 ? row - w_dense.size(-1) : 0;
+  // (padded while it is quantized: as a float copy of its own, made first, it was 20 us of the first pass on a new weight)
+  auto quantized = [&](int bw, int pos) {
+    if (pad <= 0) return quantize_op(w_dense, bw, pos, 1.0);
+    Tensor q = device_empty({w_dense.size(0), row}, int_type(bw), w_dense.device());
+    check_status(catchq_quantize_nchw_to_nhwc(w_dense.data_ptr(), fp_dtype(w_dense, "quantify only support input float/half"),
+                                              q.data_ptr(), bw, (int)w_dense.size(0), (int)w_dense.size(1), 1, 1, (int)row, pos,
+                                              1.0f, current_stream()),
+                 "torch_mlu::quantize");
+    return q;
+  };
   if (m_host.numel() == 1) {
     // CNML-compatible encoding: q_mode in {1:int8, 2:int16, 3:int8 per-channel, 4:int16 per-channel},
     // q_scale = [s_in, s_w | 0, s_c0 ...]   (quantify_conv_forward.cpp:77-131; linear.cpp:81-144)
@@ -983,7 +1000,7 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
     check_status(catchq_pos_from_scale(bw, s[0], &p->pos_x), "input position");
     if (!p->per_channel) {
       check_status(catchq_pos_from_scale(bw, s[1], &p->pos_w), "weight position");
-      p->qw = quantize_op(w_dense, bw, p->pos_w, 1.0);
+      p->qw = quantized(bw, p->pos_w);
     } else {
       const int64_t co = w_dense.size(0);
       TORCH_CHECK(s_host.numel() == 2 + co, "per-channel q_scale must hold 2 + ", co, " values, got ", s_host.numel());
@@ -994,6 +1011,7 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
       p->pos_w = pc.new_pos;
       p->new_scale = pc.new_scale;
       p->qw = quantize_weight_per_channel(w_dense, pc, bw);
+      if (pad > 0) p->qw = at::constant_pad_nd(p->qw, {0, pad}, 0);
     }
   } else {
     // CNNL encoding: q_scale = [bitwidth_in, bitwidth_w], q_mode = [pos_in, pos_w]
@@ -1004,7 +1022,7 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, const Tensor &weight, co
     TORCH_CHECK((p->bw_x == 8 || p->bw_x == 16) && (p->bw_w == 8 || p->bw_w == 16), "bitwidth not support");
     p->pos_x = m[0];
     p->pos_w = m[1];
-    p->qw = quantize_op(w_dense, p->bw_w, p->pos_w, 1.0);
+    p->qw = quantized(p->bw_w, p->pos_w);
   }
   p->w_impl = weak_of(weight); p->s_impl = weak_of(q_scale); p->m_impl = weak_of(q_mode);
   p->w_ver = version_of(weight); p->s_ver = version_of(q_scale); p->m_ver = version_of(q_mode);
@@ -1112,9 +1130,9 @@ bool linear_digits(const void *x, int dt, Prepared &prep, int64_t m, int64_t n, 
   return true;
 }
 
-template <typename MakeDense>
+template <typename MakeDense, typename RowLength = AsItIs>
 std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_scale, const Tensor &q_mode,
-                                       MakeDense make_dense, int variant = 0) {
+                                       MakeDense make_dense, int variant = 0, RowLength row_length = RowLength()) {
   const bool use_cache = cache_enabled();
   const c10::TensorImpl *key = weight.unsafeGetTensorImpl();
   if (use_cache) {
@@ -1139,7 +1157,7 @@ std::shared_ptr<Prepared> prepared_for(const Tensor &weight, const Tensor &q_sca
       g_cache.erase(it);
     }
   }
-  auto p = prepare(make_dense, weight, q_scale, q_mode);
+  auto p = prepare(make_dense, row_length, weight, q_scale, q_mode);
   p->variant = variant;
   const auto made_on = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();
   p->made_on = made_on.id();
@@ -1427,10 +1445,7 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
     const int64_t least = bw_act == 8 ? (k + 15) / 16 * 16 : (k + 7) / 8 * 8, whole = (k + 63) / 64 * 64;
     return k > 96 && whole < 65536 && weight.size(0) * whole < (1ll << 30) && (bw_act != 8 || least != k) ? whole : least;
   };
-  auto prep = prepared_for(weight, q_scale, q_mode, [&](const Tensor &w, int bw_act) {
-    const int64_t kpad = device_k(bw_act) - k;
-    return kpad > 0 ? at::constant_pad_nd(w, {0, kpad}, 0).contiguous() : w.contiguous();
-  });
+  auto prep = prepared_for(weight, q_scale, q_mode, [](const Tensor &w, int) { return w.contiguous(); }, 0, device_k);
   const Tensor xc = input.contiguous();
   const int64_t n = weight.size(0), kd = device_k(prep->bw_x);
   int64_t m = 1;

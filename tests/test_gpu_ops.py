@@ -159,18 +159,43 @@ def test_linear_leading_dims_and_no_bias_tensor():
         torch.ops.torch_mlu.linear(x.cuda(), w.cuda()[None], zero_dim_bias.cuda(), q_scale.cuda(), q_mode.cuda())
 
 
-@pytest.mark.parametrize("mode", [1, 2])
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
 @pytest.mark.parametrize("m,k,n", [(1, 97, 5), (130, 104, 33), (70, 129, 65), (65, 191, 130), (300, 1000, 70)])
 def test_linear_rows_padded_to_whole_steps(m, k, n, mode):
     """K behind the last 64-value step, on both sides of the streaming kernel's rows; same integers whatever the padding"""
     note("linear padded rows", m, k, n, mode)
     torch.manual_seed(m + k + n)
     w, x, b = torch.randn(n, k) * 0.1, torch.randn(m, k), torch.randn(n)
-    top = 127.0 if mode == 1 else 32767.0
-    q_scale = torch.tensor([top / x.abs().max().item(), top / w.abs().max().item()])
+    top = 127.0 if mode in (1, 3) else 32767.0
+    q_scale = torch.tensor([top / x.abs().max().item()] +
+                           ([top / w.abs().max().item()] if mode < 3 else [0.0] + (top / w.abs().amax(1)).tolist()))
     q_mode = torch.tensor([mode], dtype=torch.int32)
     got = torch.ops.torch_mlu.linear(x.cuda(), w.cuda(), b.cuda(), q_scale.cuda(), q_mode.cuda())
     ref = oops.linear(x.numpy(), w.numpy(), b.numpy(), q_scale.numpy(), q_mode.numpy())
+    assert same_bits(ref["y"], got.cpu().numpy())
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
+def test_first_use_of_a_weight_with_padded_rows(mode, half):
+    """no padded copy of the floating weight is made: the first call asks for the quantized weight (twice where each channel
+    has a scale of its own) and little else"""
+    note("first use, padded rows", mode, half)
+    g = torch.Generator().manual_seed(mode)
+    w, x, b = torch.randn(2000, 1000, generator=g) * 0.1, torch.randn(2, 1000, generator=g), torch.randn(2000, generator=g)
+    w, x = (w.half(), x.half()) if half else (w, x)
+    top = 127.0 if mode in (1, 3) else 32767.0
+    q_scale = torch.tensor([top / 4.0] + ([top / 0.5] if mode < 3 else [0.0] + (top / w.float().abs().amax(1)).tolist()))
+    q_mode = torch.tensor([mode], dtype=torch.int32)
+    xd, wd, bd = x.cuda(), w.cuda(), b.cuda()
+    torch.ops.torch_mlu.linear(xd, wd[:5].clone(), bd[:5], q_scale if mode < 3 else q_scale[:7], q_mode)
+    torch.ops.torch_mlu.clear_weight_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = held()
+    got = torch.ops.torch_mlu.linear(xd, wd, bd, q_scale, q_mode)
+    quantized = 2000 * 1024 * (1 if mode in (1, 3) else 2)
+    assert torch.cuda.memory_stats()["requested_bytes.all.peak"] - before < quantized * (1 if mode < 3 else 2) + 200000
+    ref = oops.linear(x.float().numpy(), w.float().numpy(), b.numpy(), q_scale.numpy(), q_mode.numpy())
     assert same_bits(ref["y"], got.cpu().numpy())
 
 
