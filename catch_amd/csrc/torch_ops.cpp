@@ -1439,7 +1439,7 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   // inside the product -- to whole K steps of 64, so that the kernels' 64- and 128-byte pieces of a row do not straddle cache
   // lines: int8 4000 x 1000 -> 1000 21.9 -> 17.9 us, 6000 x 2500 -> 700 49.6 -> 37.8, 8000 x 97 -> 120 9.3 -> 6.6, int16
   // 1379 x 1000 -> 1001 22.4 -> 20.5.  (Shorter rows keep the streaming kernel, which takes up to 96 values; the matrix-core
-  // routes of int16 end at 65536 values of K and 2^30 of an operand.)
+  // routes end at 2^31 bytes of an operand, those of int16 at 65536 values of K.)
   const int64_t k = weight.size(1);
   auto device_k = [&](int bw_act) {
     const int64_t least = bw_act == 8 ? (k + 15) / 16 * 16 : (k + 7) / 8 * 8, whole = (k + 63) / 64 * 64;
@@ -1472,9 +1472,10 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   }
   // (rows of the packed weights end in zeros where kd > k)
   if (linear_digits(xc.data_ptr(), dt, *prep, m, n, k, e, input.device(), "torch_mlu::linear")) return y;
-  // (as many rows at a time as an int16 operand may have values: padding makes no product a slower route's)
-  int64_t rows = m;
-  if (prep->bw_x == 16 && m * kd >= (1ll << 30)) rows = std::max<int64_t>(((1ll << 30) - 1) / kd, 1);
+  // (as many rows at a time as an operand of the matrix-core routes may have, 2^31 bytes: padding makes no product a slower
+  // route's)
+  const int64_t row_bytes = std::max<int64_t>(kd, 1) * (prep->bw_x / 8);
+  const int64_t rows = std::min(m, std::max<int64_t>(((1ll << 31) - 1) / row_bytes, 1));
   Tensor qx = device_empty({rows, kd}, int_type(prep->bw_x), input.device());
   for (int64_t r = 0; r < m; r += rows) {
     const int64_t count = std::min(rows, m - r);

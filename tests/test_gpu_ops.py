@@ -175,6 +175,31 @@ def test_linear_rows_padded_to_whole_steps(m, k, n, mode):
     assert same_bits(ref["y"], got.cpu().numpy())
 
 
+@pytest.mark.parametrize("mode,m,k,n", [(1, 17000000, 100, 4), (2, 1080000, 1000, 5), (2, 130500, 8200, 6)])
+def test_linear_whose_padded_rows_pass_an_operands_limit(mode, m, k, n):
+    """worked on in runs of rows whose quantized operand stays below 2^31 bytes: rows on both sides of a run's end as a call
+    of few rows has them, and the oracle"""
+    note("linear, runs of rows", mode, m, k, n)
+    kd, size = (k + 63) // 64 * 64, 1 if mode == 1 else 2
+    assert m * kd * size >= 1 << 31
+    g = torch.Generator(device="cuda").manual_seed(k)
+    w, b = torch.randn(n, k, generator=g, device="cuda") * 0.1, torch.randn(n, generator=g, device="cuda")
+    x = torch.empty(m, k, dtype=torch.float16, device="cuda").normal_(generator=g)
+    top = 127.0 if mode == 1 else 32767.0
+    q_scale, q_mode = torch.tensor([top / 4.0, top / 0.5]), torch.tensor([mode], dtype=torch.int32)
+    end = ((1 << 31) - 1) // (kd * size)
+    near = torch.ops.torch_mlu.linear(x[end - 50:end + 50], w, b, q_scale, q_mode)
+    last = torch.ops.torch_mlu.linear(x[-40:], w, b, q_scale, q_mode)
+    torch.cuda.reset_peak_memory_stats()
+    before = held()
+    got = torch.ops.torch_mlu.linear(x, w, b, q_scale, q_mode)
+    assert torch.cuda.memory_stats()["requested_bytes.all.peak"] - before < (1 << 31) + got.numel() * 4 + (1 << 20)
+    assert torch.equal(got[end - 50:end + 50], near) and torch.equal(got[-40:], last)
+    rows = torch.tensor([0, end - 1, end, m - 1])
+    ref = oops.linear(x[rows.cuda()].float().cpu().numpy(), w.cpu().numpy(), b.cpu().numpy(), q_scale.numpy(), q_mode.numpy())
+    assert same_bits(ref["y"], got[rows.cuda()].cpu().numpy())
+
+
 @pytest.mark.parametrize("half", [False, True])
 @pytest.mark.parametrize("mode", [1, 2, 3, 4])
 def test_first_use_of_a_weight_with_padded_rows(mode, half):
