@@ -314,6 +314,27 @@ def test_plan_of_few_pixels(monkeypatch):
     check_against_oracle(layers, sd, x, fused)
 
 
+def test_parts_that_pay_and_parts_that_are_refused():
+    """`streams` is the most parts a batch is recorded in: fewer where the launches are too short to pay for more; a batch has
+    no parts without images"""
+    note("resnet18, parts that pay")
+    layers = nets.resnet(18)
+    net = nets.FloatNet(layers, seed=0).eval()
+    x = torch.randn(7, 3, 64, 64, generator=torch.Generator().manual_seed(1))
+    fused = pipeline.FusedNet(layers, pipeline.calibrate(net, x, "int8", True))
+    assert fused._parts(2, 256, 3, 224, 224) == 2 and fused._parts(2, 2, 3, 224, 224) == 1
+    for bad in (0, -1, 8):
+        with pytest.raises(ValueError, match="parts"):
+            fused.capture(x.cuda(), parts=bad)
+    want = fused.forward(x.cuda())
+    _, replay = fused.capture(x.cuda(), streams=4)
+    assert fused.graph_parts == 1
+    for i in range(3):
+        assert torch.equal(replay(), want), i
+        _ = fused.forward(torch.randn(7, 3, 64, 64, device="cuda"))  # eager work between the replays
+        torch.cuda.synchronize()
+
+
 @recorded_again_in_parts
 def test_parts_of_a_captured_batch():
     """`streams` is the most parts a graph may have, fewer where the launches are too short to pay for the branches;
