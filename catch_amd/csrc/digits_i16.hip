@@ -243,10 +243,10 @@ __global__ __launch_bounds__(256) void quantize_digits_kernel(const TIn *__restr
   store_digits(out, run, ks, nk, lane, q);
 }
 
-// w [N, ld] int16, K values of a row used -> digits, zeros beyond N and K, and the rows' sums (once per weight, in front of its
-// first product).  A block takes 32 rows, its waves every sixteenth sub-step: bound by the latency of the steps that a wave
-// takes one after the other.  1001 x 1000: 5.7 us; the first pass on a new weight (1379 rows, half) 191 us with one wave for a
-// block's rows, 137 with sixteen.
+// w [N, ld] int16, K values of a row used -> digits, zeros beyond N and K, and the rows' sums (once per weight that is
+// read packed).  A block takes 32 rows, its waves every sixteenth sub-step: bound by the latency of the steps that a wave
+// takes one after the other.  1001 x 1000: 5.7 us; a pass that packs (1379 rows, half, on a new weight) 191 us with one wave for
+// a block's rows, 137 with sixteen.
 constexpr int kPackWaves = 16;
 __global__ __launch_bounds__(64 * kPackWaves) void pack_digits_kernel(const int16_t *__restrict__ w, int8_t *__restrict__ out,
                                                                       int *__restrict__ sums, int N, int K, int64_t ld, int nk) {

@@ -978,7 +978,8 @@ std::shared_ptr<Prepared> prepare(MakeDense make_dense, RowLength row_length, co
   }
   const Tensor w_dense = make_dense(weight, bw_act);
   const int64_t row = row_length(bw_act), pad = row > 0 && w_dense.numel() > 0 ? row - w_dense.size(-1) : 0;
-  // (padded while it is quantized: as a float copy of its own, made first, it was 20 us of the first pass on a new weight)
+  // (padded while it is quantized: the first pass on a new weight, 1379 x 1000 -> 1001 half at 16 bits, 137 us with a padded float
+  // copy made first, 129 so)
   auto quantized = [&](int bw, int pos) {
     if (pad <= 0) return quantize_op(w_dense, bw, pos, 1.0);
     Tensor q = device_empty({w_dense.size(0), row}, int_type(bw), w_dense.device());
