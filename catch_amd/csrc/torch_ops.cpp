@@ -1497,6 +1497,32 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
 }
 
 // x [N,H,W,C] contiguous int8 / int16 / fp32
+// Channel concatenation of quantized tensors (catchq_concat_nhwc): kinds[i] says in which form source i is given.
+Tensor concat_nhwc_op(at::TensorList xs, at::IntArrayRef kinds, int64_t bitwidth, int64_t position, double scale) {
+  TORCH_CHECK(!xs.empty() && xs.size() == kinds.size(), "concat_nhwc: one kind for every source");
+  TORCH_CHECK(bitwidth == 8 || bitwidth == 16, "bitwidth not support");
+  c10::DeviceGuard guard(xs[0].device());
+  std::vector<catchq_concat_source_t> s(xs.size());
+  int64_t n = -1, h = 0, w = 0, channels = 0;
+  for (size_t i = 0; i < xs.size(); ++i) {
+    const Tensor &x = xs[i];
+    const bool is_float = kinds[i] == CATCHQ_CONCAT_FLOAT;
+    const int64_t up = kinds[i] == CATCHQ_CONCAT_UP2 ? 2 : 1;
+    TORCH_CHECK(x.dim() == 4 && x.is_contiguous() && x.device() == xs[0].device(), "concat_nhwc expects contiguous [N,H,W,C] tensors");
+    TORCH_CHECK(x.scalar_type() == (is_float ? at::kFloat : int_type(bitwidth)), "concat_nhwc: source ", (int64_t)i, " has another type");
+    if (n < 0) { n = x.size(0); h = up * x.size(1); w = up * x.size(2); }
+    TORCH_CHECK(x.size(0) == n && up * x.size(1) == h && up * x.size(2) == w, "concat_nhwc: source ", (int64_t)i, " has another size");
+    channels += x.size(3);
+    s[i] = {x.data_ptr(), (int)x.size(3), (int)kinds[i]};
+  }
+  Tensor out = at::empty({n, h, w, channels}, xs[0].options().dtype(int_type(bitwidth)));
+  if (out.numel() == 0) return out;
+  check_status(catchq_concat_nhwc(s.data(), (int)s.size(), (int)bitwidth, (int)position, (float)scale, (int)n, (int)h, (int)w,
+                                  out.data_ptr(), current_stream()),
+               "torch_mlu::concat_nhwc");
+  return out;
+}
+
 Tensor maxpool_nhwc_op(const Tensor &x, int64_t k, int64_t stride, int64_t pad) {
   TORCH_CHECK(x.dim() == 4 && x.is_contiguous(), "maxpool_nhwc expects a contiguous [N,H,W,C] tensor");
   int bits = 0;
@@ -1593,6 +1619,7 @@ TORCH_LIBRARY(torch_mlu, m) {
         "float q_scale=1.0) -> (Tensor, Tensor, Tensor)");
   m.def("quantize_conv2d(Tensor input, Tensor input_position, Tensor weight, Tensor weight_position, Tensor bias, "
         "int[] padding, int[] stride, int[] dilation, int groups, int input_bitwidth=8, int weight_bitwidth=8) -> Tensor");
+  m.def("concat_nhwc(Tensor[] xs, int[] kinds, int bitwidth, int position, float scale=1.0) -> Tensor");
   m.def("maxpool_nhwc(Tensor x, int k, int stride, int pad) -> Tensor");
   m.def("global_avgpool_nhwc(Tensor x, int q_bitwidth=0, int q_position=0, float q_scale=1.0) -> Tensor");
   m.def("set_launch_sharing(int launches) -> int", &set_launch_sharing_op);
@@ -1629,6 +1656,7 @@ TORCH_LIBRARY_IMPL(torch_mlu, CUDA, m) {  // ROCm tensors dispatch on the CUDA k
   m.impl("qconv2d_avgpool", &qconv2d_avgpool_op);
   m.impl("qconv2d_chain", &qconv2d_chain_op);
   m.impl("qlinear", &qlinear_op);
+  m.impl("concat_nhwc", &concat_nhwc_op);
   m.impl("maxpool_nhwc", &maxpool_nhwc_op);
   m.impl("global_avgpool_nhwc", &global_avgpool_nhwc_op);
 }

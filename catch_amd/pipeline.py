@@ -24,6 +24,7 @@ from .nets import LEAKY_SLOPE, outputs_of
 
 _ACT_CODE = {"none": 0, "relu": 1, "relu6": 2, "leaky": 3}
 _PASS = ("maxpool", "upsample", "concat")
+_CONCAT_COPY, _CONCAT_UP2, _CONCAT_FLOAT = range(3)  # CATCHQ_CONCAT_*
 
 
 def _key(name):
@@ -512,6 +513,50 @@ class FusedNet(object):
         for l in self.layers:
             if l.kind in ("conv", "fc") and len(self.q_demand[l.name]) > 1:
                 self.f_demand[l.name] = True
+        self._plan_concats()
+
+    def _plan_concats(self):
+        """concat_kinds[(concat layer, form)]: in which form torch_mlu::concat_nhwc takes the layer's sources.  An upsampled tensor
+        that only such launches read is never stored, nor is a form of a convolution's output beyond the first
+        (at_concat: (layer,) + form of those)."""
+        by_name = {l.name: l for l in self.layers}
+
+        def form_readers(name, form):
+            for m in self.layers:
+                if name == m.src or (isinstance(m.src, tuple) and name in m.src):
+                    mq = self.q.get(m.name)
+                    if mq is not None and (mq.bw_x, mq.pos_x, mq.scale_x) == form or m.kind in _PASS and form in self.q_demand[m.name]:
+                        yield m
+                    elif m.kind == "gap":
+                        yield m  # (pooled from fp32; counted all the same)
+
+        takes = set((l.name, d) for l in self.layers if l.kind == "concat" and len(l.src) <= 4 for d in self.q_demand[l.name]
+                    if all(self.cdev[s] % (128 // d[0]) == 0 for s in l.src))
+        self.concat_kinds, self.at_concat = {}, set()
+        for name, form in sorted(takes):
+            kinds = []
+            for s in by_name[name].src:
+                sl = by_name.get(s)
+                alone = all((m.name, form) in takes for m in form_readers(s, form))
+                if sl is not None and alone and sl.kind == "upsample" and form in self.q_demand[sl.src]:
+                    kinds.append(_CONCAT_UP2)
+                elif (sl is not None and alone and sl.kind == "conv" and form in self.q_demand[s][1:] and self.f_demand[s]
+                      and not (self.out_half and s in self.outputs)):
+                    kinds.append(_CONCAT_FLOAT)
+                else:
+                    kinds.append(_CONCAT_COPY)
+                    continue
+                self.at_concat.add((s,) + form)
+            self.concat_kinds[(name, form)] = kinds
+
+    def _concat(self, l, form, env):
+        kinds = self.concat_kinds.get((l.name, form))
+        if kinds is None:
+            return torch.cat([env[(s,) + form] for s in l.src], 3)
+        by_name = {m.name: m for m in self.layers}
+        xs = [env[(by_name[s].src,) + form] if k == _CONCAT_UP2 else env[(s, "f")] if k == _CONCAT_FLOAT else env[(s,) + form]
+              for s, k in zip(l.src, kinds)]
+        return torch.ops.torch_mlu.concat_nhwc(xs, kinds, form[0], form[1], form[2])
 
     # ------------------------------------------------------------------------------------------
     def forward(self, x, trace=None, timers=None, keep=None):
@@ -598,7 +643,7 @@ class FusedNet(object):
                     env[(name, "f")] = y
                 if qd:
                     env[(name,) + qd] = q
-                for dd in self.q_demand[name][1:]:
+                for dd in self._further_forms(name):
                     env[(name,) + dd] = ops.quantize(y, dd[0], dd[1], dd[2])
                 continue
             if l.kind == "conv" and not tracing and name in self._fused_away:
@@ -623,7 +668,7 @@ class FusedNet(object):
                     env[(name, "f")] = y
                 if qd:
                     env[(name,) + qd] = q
-                for d in self.q_demand[name][1:]:
+                for d in self._further_forms(name):
                     env[(name,) + d] = ops.quantize(y, d[0], d[1], d[2])
                 continue
             if l.kind == "conv":
@@ -662,7 +707,7 @@ class FusedNet(object):
                     env[(name, "f")] = y
                 if qd:
                     env[(name,) + qd] = q
-                for d in self.q_demand[name][1:]:
+                for d in self._further_forms(name):
                     env[(name,) + d] = ops.quantize(y, d[0], d[1], d[2])
                 if tracing:
                     trace[name] = dict(qx=qx, acc=acc, y=y)
@@ -712,11 +757,13 @@ class FusedNet(object):
                         env[(name,) + d] = g.reshape(g.shape[0], 1, 1, g.shape[1])
             elif l.kind == "upsample":
                 for form in self._forms(name):
+                    if (name,) + form in self.at_concat:
+                        continue
                     t = env[(l.src,) + form]
                     env[(name,) + form] = t.repeat_interleave(2, 1).repeat_interleave(2, 2)
             elif l.kind == "concat":
                 for form in self._forms(name):
-                    env[(name,) + form] = torch.cat([env[(s,) + form] for s in l.src], 3)
+                    env[(name,) + form] = self._concat(l, form, env)
             else:
                 raise ValueError(l.kind)
         if keep is not None:
@@ -730,6 +777,10 @@ class FusedNet(object):
         return outs[0] if len(outs) == 1 else tuple(outs)
 
     __call__ = forward
+
+    def _further_forms(self, name):
+        """quantized forms of a convolution's output that are made from its fp32 copy (the epilogue writes the first)"""
+        return [d for d in self.q_demand[name][1:] if (name,) + d not in self.at_concat]
 
     def _forms(self, name):
         forms = [tuple(d) for d in self.q_demand[name]]

@@ -460,6 +460,25 @@ int catchq_conv1x1_chain_nhwc(const catchq_chain_link_t *links, int nlinks, int 
 int catchq_maxpool_nhwc(const void *x, void *y, int elem_bits, int n, int h, int w, int c, int k, int stride,
                         int pad, catchq_stream_t stream);
 
+/* Channel concatenation of quantized tensors in one launch: out [n, h, w, sum of channels] int8 / int16 (bitwidth 8 / 16).
+ * In the reference a detector's route is torch.cat (cnnl_cat, operators/cnnl/cat.cpp) behind a nearest upsampling
+ * (operators/cnnl/upsample.cpp), all in float, and the quantizer of the layer behind it.  Copying and repeating commute with
+ * quantization, so here every source is given in the form that it already has:
+ *   CATCHQ_CONCAT_COPY   integers [n, h, w, channels]
+ *   CATCHQ_CONCAT_UP2    integers [n, h / 2, w / 2, channels], every pixel repeated twice in both directions (h, w even)
+ *   CATCHQ_CONCAT_FLOAT  fp32 [n, h, w, channels], q = sat(rne(x * scale * 2^-position))
+ * CATCHQ_ERR_UNSUPPORTED: more than CATCHQ_CONCAT_MAX sources, channels that do not fill 16-byte pieces, unaligned pointers,
+ * 2^31 pieces or more. */
+#define CATCHQ_CONCAT_MAX 4
+enum { CATCHQ_CONCAT_COPY = 0, CATCHQ_CONCAT_UP2 = 1, CATCHQ_CONCAT_FLOAT = 2 };
+typedef struct catchq_concat_source {
+  const void *x;
+  int channels;
+  int kind;
+} catchq_concat_source_t;
+int catchq_concat_nhwc(const catchq_concat_source_t *sources, int nsources, int bitwidth, int position, float scale, int n,
+                       int h, int w, void *out, catchq_stream_t stream);
+
 /* Global average pooling of an fp32 NHWC tensor [n, hw, c] -> [n, c]: sequential fp32 sum over the
  * pixels in storage order, then one division by hw (adaptive_avg_pool2d((1,1)) in the reference's
  * models, operators/cnnl/pooling.cpp). */
