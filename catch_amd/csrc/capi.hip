@@ -36,6 +36,9 @@ int64_t gemm_digits_bytes(int64_t M, int64_t N, int64_t K, const EpiDev &e);
 int gemm_digits(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, void *digits,
                 const EpiDev &e, hipStream_t s);
 int pack_filters(const void *w, void *packed, int64_t N, int64_t K, hipStream_t s);
+int64_t packed3x3_bytes(int64_t Co, int64_t Ci);
+int pack3x3(const void *w, void *packed, int64_t Co, int64_t Ci, hipStream_t s);
+int conv3x3_a16_packed(const void *x, const void *packed, int N, int H, int W, int Ci, int Co, const EpiDev &e, hipStream_t s);
 bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
 int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
                int Wo, const EpiDev &e, hipStream_t s);
@@ -410,6 +413,37 @@ CATCHQ_API int catchq_float_linear_packed(const void *x, int x_dtype, int x_posi
   if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;
   const int done = float_rows(x, x_dtype == CATCHQ_F16, x_position, packed, m, n, k, make_epi(epilogue, m * n), as_stream(stream));
   return done < 0 ? CATCHQ_ERR_UNSUPPORTED : done;
+}
+
+CATCHQ_API int catchq_packed_conv3x3_size(int64_t co, int64_t ci, size_t *bytes) {
+  if (!bytes || co <= 0 || ci <= 0) return CATCHQ_ERR_ARG;
+  if (ci % 64 != 0 || co >= (1 << 24) || ci >= (1 << 24) || packed3x3_bytes(co, ci) >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  *bytes = (size_t)packed3x3_bytes(co, ci);
+  return CATCHQ_OK;
+}
+
+CATCHQ_API int catchq_pack_conv3x3(const void *w, int64_t co, int64_t ci, void *packed, catchq_stream_t stream) {
+  size_t bytes;
+  const int st = catchq_packed_conv3x3_size(co, ci, &bytes);
+  if (st != CATCHQ_OK) return st;
+  if (!w || !packed || !aligned16(w) || !aligned16(packed)) return CATCHQ_ERR_ARG;
+  return pack3x3(w, packed, co, ci, as_stream(stream));
+}
+
+CATCHQ_API int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                                     const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  int st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  if (n < 0 || h <= 0 || w <= 0) return CATCHQ_ERR_ARG;
+  size_t bytes;
+  st = catchq_packed_conv3x3_size(co, ci, &bytes);
+  if (st != CATCHQ_OK) return st;
+  if (n == 0) return CATCHQ_OK;
+  if (!x || !packed) return CATCHQ_ERR_ARG;
+  if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;
+  if ((int64_t)h * w >= (1ll << 31) || (int64_t)n * h * w >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  st = conv3x3_a16_packed(x, packed, n, h, w, ci, co, make_epi(epilogue, (int64_t)n * h * w * co), as_stream(stream));
+  return st < 0 ? CATCHQ_ERR_UNSUPPORTED : st;
 }
 
 CATCHQ_API int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes) {

@@ -411,8 +411,9 @@ EpiOut prepare_epilogue(const EpiArgs &a, at::IntArrayRef out_shape, int64_t co,
 }
 
 // qx [N,H,W,Ci] int8/int16 contiguous, qw [Co,kh,kw,Ci/g] contiguous -> outputs [N,Ho,Wo,Co]
+// packed: pack_conv3x3(qw), read instead of qw where the kernel on packed filters serves the call
 EpiOut qconv2d_impl(const Tensor &qx, const Tensor &qw, at::IntArrayRef padding, at::IntArrayRef stride,
-                    at::IntArrayRef dilation, int64_t groups, const EpiArgs &a) {
+                    at::IntArrayRef dilation, int64_t groups, const EpiArgs &a, const c10::optional<Tensor> &packed = c10::nullopt) {
   TORCH_CHECK(qx.dim() == 4 && qw.dim() == 4 && qx.is_contiguous() && qw.is_contiguous(),
               "qconv2d expects contiguous NHWC activations and [Co,kh,kw,Ci/g] weights");
   TORCH_CHECK(padding.size() == 2 && stride.size() == 2 && dilation.size() == 2, "2-d conv parameters expected");
@@ -434,6 +435,21 @@ EpiOut qconv2d_impl(const Tensor &qx, const Tensor &qw, at::IntArrayRef padding,
   std::vector<Tensor> keep;
   EpiOut o = prepare_epilogue(a, {d.n, ho, wo, d.co}, d.co, qx.options(), &e, &keep);
   if (d.n == 0 || d.co == 0) return o;  // nothing to compute: the empty outputs are the result
+  if (packed.has_value() && packed->defined()) {
+    size_t bytes = 0;
+    TORCH_CHECK(qw.scalar_type() == at::kChar && d.kh == 3 && d.kw == 3 && d.groups == 1 &&
+                    catchq_packed_conv3x3_size(d.co, d.ci, &bytes) == CATCHQ_OK && packed->scalar_type() == at::kChar &&
+                    packed->is_contiguous() && packed->numel() == (int64_t)bytes && packed->device() == qx.device(),
+                "qconv2d: the packed filters are not those of the weight");
+    if (qx.scalar_type() == at::kShort && d.pad_h == 1 && d.pad_w == 1 && d.stride_h == 1 && d.stride_w == 1 && d.dil_h == 1 &&
+        d.dil_w == 1) {
+      const int st = catchq_conv3x3_packed(qx.data_ptr(), packed->data_ptr(), d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
+      if (st != CATCHQ_ERR_UNSUPPORTED) {
+        check_status(st, "torch_mlu::conv2d");
+        return o;
+      }
+    }
+  }
   check_status(catchq_conv2d_nhwc(qx.data_ptr(), bits_of(qx), qw.data_ptr(), bits_of(qw), &d, &e, current_stream()),
                "torch_mlu::conv2d");
   return o;
@@ -527,11 +543,23 @@ std::tuple<Tensor, Tensor, Tensor> qconv2d_op(const Tensor &qx, const Tensor &qw
                                               at::IntArrayRef stride, at::IntArrayRef dilation, int64_t groups,
                                               int64_t act, bool want_y, bool y_half, bool want_acc,
                                               int64_t q_bitwidth, int64_t q_position, double q_scale,
-                                              double act_slope, bool resid_after_act) {
+                                              double act_slope, bool resid_after_act, const c10::optional<Tensor> &packed) {
   c10::DeviceGuard guard(qx.device());
   return tup(qconv2d_impl(qx, qw, padding, stride, dilation, groups,
                           make_args(exp2, chan_div, bias, resid, act, want_y, y_half, want_acc, q_bitwidth,
-                                    q_position, q_scale, act_slope, resid_after_act)));
+                                    q_position, q_scale, act_slope, resid_after_act), packed));
+}
+
+// qw [Co,3,3,Ci] int8 in the order that catchq_conv3x3_packed reads
+Tensor pack_conv3x3_op(const Tensor &qw) {
+  TORCH_CHECK(qw.dim() == 4 && qw.is_contiguous() && qw.scalar_type() == at::kChar && qw.size(1) == 3 && qw.size(2) == 3,
+              "pack_conv3x3 expects contiguous int8 [Co,3,3,Ci] filters");
+  c10::DeviceGuard guard(qw.device());
+  size_t bytes = 0;
+  check_status(catchq_packed_conv3x3_size(qw.size(0), qw.size(3), &bytes), "torch_mlu::pack_conv3x3");
+  Tensor packed = at::empty({(int64_t)bytes}, qw.options());
+  check_status(catchq_pack_conv3x3(qw.data_ptr(), qw.size(0), qw.size(3), packed.data_ptr(), current_stream()), "torch_mlu::pack_conv3x3");
+  return packed;
 }
 
 std::tuple<Tensor, Tensor> qconv2d_shortcut_op(const Tensor &qx, const Tensor &qw, int64_t exp2,
@@ -1595,7 +1623,8 @@ TORCH_LIBRARY(torch_mlu, m) {
   m.def("qconv2d(Tensor qx, Tensor qw, int exp2, Tensor? chan_div, Tensor? bias, Tensor? resid, "
         "int[] padding, int[] stride, int[] dilation, int groups, int act=0, bool want_y=True, "
         "bool y_half=False, bool want_acc=False, int q_bitwidth=0, int q_position=0, float q_scale=1.0, "
-        "float act_slope=0.0, bool resid_after_act=False) -> (Tensor, Tensor, Tensor)");
+        "float act_slope=0.0, bool resid_after_act=False, Tensor? packed=None) -> (Tensor, Tensor, Tensor)");
+  m.def("pack_conv3x3(Tensor qw) -> Tensor");
   m.def("qconv2d_shortcut(Tensor qx, Tensor qw, int exp2, Tensor? chan_div, Tensor? bias, Tensor sx, Tensor sw, "
         "int s_stride, int s_exp2, Tensor? s_chan_div, Tensor? s_bias, int[] padding, int[] stride, int[] dilation, "
         "int act=0, bool want_y=True, bool y_half=False, int q_bitwidth=0, int q_position=0, float q_scale=1.0, "
@@ -1649,6 +1678,7 @@ TORCH_LIBRARY_IMPL(torch_mlu, CUDA, m) {  // ROCm tensors dispatch on the CUDA k
   m.impl("mm_q", &mm_q_op);
   m.impl("quantize_conv2d", &quantize_conv2d_op);
   m.impl("qconv2d", &qconv2d_op);
+  m.impl("pack_conv3x3", &pack_conv3x3_op);
   m.impl("qconv2d_shortcut", &qconv2d_shortcut_op);
   m.impl("qconv2d_head", &qconv2d_head_op);
   m.impl("qconv2d_irb", &qconv2d_irb_op);

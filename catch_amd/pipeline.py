@@ -49,7 +49,7 @@ def quant_params(bw, scale):
 
 class _LayerQ(object):
     """decoded q-params and the quantized weight of one conv / fc layer"""
-    __slots__ = ("bw_x", "bw_w", "pos_x", "scale_x", "pos_w", "qw", "chan_div", "bias", "exp2", "cpad", "groups")
+    __slots__ = ("bw_x", "bw_w", "pos_x", "scale_x", "pos_w", "qw", "chan_div", "bias", "exp2", "cpad", "groups", "packed")
 
 
 def _pad16(c, bw=8):
@@ -159,6 +159,9 @@ def _decode(layer, sd, device, ci_dev, co_dev, fractional=False):
         if q.chan_div is not None:
             q.chan_div = pad(q.chan_div, (0, co_dev - co), value=1.0)
     q.qw = qw.contiguous()
+    q.packed = None
+    if (layer.kind, layer.k, layer.stride, layer.pad, q.groups, q.bw_x, q.bw_w) == ("conv", 3, 1, 1, 1, 16, 8) and ci_dev % 64 == 0:
+        q.packed = torch.ops.torch_mlu.pack_conv3x3(q.qw)  # (read by the launches that the kernel on packed filters serves)
     return q
 
 
@@ -701,7 +704,7 @@ class FusedNet(object):
                                             [l.stride, l.stride], [1, 1], lq.groups, _ACT_CODE[l.act], want_y,
                                             self.out_half and name in self.outputs, tracing,
                                             qd[0] if qd else 0, qd[1] if qd else 0, qd[2] if qd else 1.0, LEAKY_SLOPE,
-                                            bool(l.add_after))
+                                            bool(l.add_after), lq.packed)
                 tick(name)
                 if want_y:
                     env[(name, "f")] = y

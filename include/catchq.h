@@ -268,6 +268,15 @@ int catchq_float_linear_packed_takes(int x_dtype, int64_t m, int64_t n, int64_t 
 int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n, int64_t k,
                                const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 
+/* A 3 x 3 convolution (stride 1, padding 1) of int16 activations with int8 filters laid out once in the order of the matrix
+ * instruction: catchq_pack_conv3x3 writes catchq_packed_conv3x3_size bytes from w [co,3,3,ci], ci a multiple of 64.  x [n,h,w,ci],
+ * outputs as catchq_conv2d_nhwc's.  CATCHQ_ERR_UNSUPPORTED: catchq_conv2d_nhwc on the filters as they are serves the call better,
+ * or alone (few output channels or blocks, wide images, rows that the vector epilogues do not take). */
+int catchq_packed_conv3x3_size(int64_t co, int64_t ci, size_t *bytes);
+int catchq_pack_conv3x3(const void *w, int64_t co, int64_t ci, void *packed, catchq_stream_t stream);
+int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                          const catchq_epilogue_t *epilogue, catchq_stream_t stream);
+
 /* A linear on floating activations with int16 weights, both split into the bytes that the matrix cores multiply:
  *   cnnl_quantify_offline_internal (quantify.cpp:69-101) followed by linear.cpp:92-110, 16 bits on either side
  * catchq_pack_digits lays the weights out once (w [n,ld] int16, k values of a row used, k <= 8192); the call quantizes x [m,k]

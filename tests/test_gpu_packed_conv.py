@@ -1,0 +1,92 @@
+"""torch_mlu::qconv2d on filters laid out by pack_conv3x3: the same bits as on the filters as they are, and which calls read them."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(n, h, w, ci, co, seed=0, lim=30000):
+    gen = torch.Generator().manual_seed(seed + 7 * h + w)
+    x = torch.randint(-lim, lim + 1, (n, h, w, ci), generator=gen).short()
+    x.view(-1)[:4] = torch.tensor([-32768, 32767, -1, 0])
+    # (the true sums fit 32 bits: 9 * ci * |w| * 2^15 < 2^31)
+    top = max(1, min(127, (1 << 16) // (9 * ci) - 1))
+    qw = torch.randint(-top, top + 1, (co, 3, 3, ci), generator=gen).to(torch.int8)
+    return x, qw
+
+
+def _outputs(out):
+    return [t for t in out if t is not None and t.numel()]
+
+
+# sharing makes the rules plan for 256 / sharing units: small layers take the blocks of 32 and of 64 pixels.  Widths: either side of
+# what one more pass over the patch takes; 96 is beyond the last.
+@pytest.mark.parametrize("n,h,w,ci,co,sharing,taken", [
+    (1, 1, 1, 64, 256, 256, True), (2, 1, 31, 64, 192, 256, True), (1, 9, 32, 64, 256, 256, True),
+    (3, 5, 63, 128, 256, 256, True), (1, 3, 64, 64, 252, 256, True), (1, 4, 95, 64, 448, 256, True),
+    (1, 4, 96, 64, 256, 256, False), (5, 13, 13, 192, 512, 256, True), (2, 8, 1, 64, 256, 256, True),
+    # blocks of 32 pixels
+    (1, 10, 15, 64, 256, 40, True), (1, 10, 16, 128, 256, 40, True), (1, 4, 47, 64, 256, 36, True),
+    (2, 2, 48, 64, 256, 36, True), (1, 2, 79, 192, 256, 42, True), (1, 2, 80, 64, 260, 42, False),
+    (1, 2, 95, 64, 256, 36, True), (7, 5, 5, 64, 256, 42, True),
+    # too few blocks, channels or multiples
+    (1, 13, 13, 128, 256, 1, False), (4, 13, 13, 64, 128, 256, False), (4, 13, 13, 64, 320, 256, False),
+])
+def test_packed_conv3x3(n, h, w, ci, co, sharing, taken):
+    ops = torch.ops.torch_mlu
+    x, qw = _case(n, h, w, ci, co)
+    gen = torch.Generator().manual_seed(11)
+    other = qw[torch.randperm(co, generator=gen)].contiguous()  # which of the two were read shows in the outputs
+    x, qw, other = x.cuda(), qw.cuda(), other.cuda()
+    bias = torch.randn(co, generator=gen).cuda()
+    resid = torch.randn(n, h, w, co, generator=gen).cuda()
+    div = (torch.rand(co, generator=gen) + 0.5).cuda()
+    geometry = ([1, 1], [1, 1], [1, 1], 1)
+    calls = [  # chan_div, resid, act, want_y, y_half, want_acc, q_bitwidth, q_position, q_scale, slope, resid_after
+        (None, None, 3, False, False, False, 16, -8, 1.0, 0.1, False), (None, resid, 3, True, False, False, 16, -8, 1.0, 0.1, True),
+        (None, resid, 3, False, False, False, 16, -8, 1.0, 0.1, True), (None, None, 3, True, False, False, 16, -8, 1.0, 0.1, False),
+        (None, None, 0, True, True, True, 0, 0, 1.0, 0.0, False), (div, resid, 1, True, False, True, 8, -2, 1.3, 0.0, False)]
+    packed, read = ops.pack_conv3x3(other), other if taken else qw
+    ops.set_launch_sharing(sharing)
+    try:
+        for d, r, act, *rest in calls:
+            got = ops.qconv2d(x, qw, -12, d, bias, r, *geometry, act, *rest, packed)
+            want = ops.qconv2d(x, read, -12, d, bias, r, *geometry, act, *rest)
+            assert len(_outputs(got)) == len(_outputs(want)) > 0
+            for a, b in zip(_outputs(got), _outputs(want)):
+                assert torch.equal(a, b)
+    finally:
+        ops.set_launch_sharing(1)
+    acc = ops.qconv2d(x, read, 0, None, None, None, *geometry, 0, False, False, True)[2]
+    want = torch.nn.functional.conv2d(x.cpu().double().permute(0, 3, 1, 2), read.cpu().double().permute(0, 3, 1, 2), padding=1)
+    assert torch.equal(acc.cpu().double(), want.permute(0, 2, 3, 1))  # integers below 2^53: exact
+
+
+def test_packed_conv3x3_large_grid():
+    """more than one round of blocks in either order of the grid"""
+    ops = torch.ops.torch_mlu
+    for n, h, w, ci, co in [(9, 26, 26, 256, 512), (7, 13, 13, 512, 1024), (8, 52, 52, 128, 256)]:
+        x, qw = _case(n, h, w, ci, co)
+        x, qw = x.cuda(), qw.cuda()
+        args = (-12, None, None, None, [1, 1], [1, 1], [1, 1], 1, 0, False, False, True)
+        want = ops.qconv2d(x, qw, *args)[2]
+        got = ops.qconv2d(x, qw, *args, 0, 0, 1.0, 0.0, False, ops.pack_conv3x3(qw))[2]
+        assert torch.equal(got, want)
+
+
+def test_packed_conv3x3_other_calls():
+    ops = torch.ops.torch_mlu
+    x, qw = _case(4, 16, 16, 64, 256)
+    x, qw = x.cuda(), qw.cuda()
+    packed = ops.pack_conv3x3(qw)
+    for pad, stride, dil in [([0, 0], [1, 1], [1, 1]), ([1, 1], [2, 2], [1, 1]), ([2, 2], [1, 1], [2, 2]), ([1, 1], [1, 2], [1, 1])]:
+        args = (-12, None, None, None, pad, stride, dil, 1, 0, False, False, True)
+        a = ops.qconv2d(x, qw, *args, 0, 0, 1.0, 0.0, False, packed)[2]
+        assert torch.equal(a, ops.qconv2d(x, qw, *args)[2])
+    x8 = (x // 256).to(torch.int8)
+    args = (-12, None, None, None, [1, 1], [1, 1], [1, 1], 1, 0, False, False, True)
+    assert torch.equal(ops.qconv2d(x8, qw, *args, 0, 0, 1.0, 0.0, False, packed)[2], ops.qconv2d(x8, qw, *args)[2])
+    with pytest.raises(RuntimeError):  # other sizes' filters
+        ops.qconv2d(x, qw, *args, 0, 0, 1.0, 0.0, False, packed[:-16].contiguous())
+    with pytest.raises(RuntimeError):  # channels that are no multiple of 64
+        ops.pack_conv3x3(qw[..., :48].contiguous())
