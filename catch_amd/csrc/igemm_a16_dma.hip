@@ -417,6 +417,8 @@ int igemm_a16_launch(int load, const void *a, const void *b, IgemmParams p, cons
   return -1;
 }
 
+int conv3x3_a16_c32(const void *x, const void *w, int N, int H, int W, int Co, int stride, int Ho, int Wo, const EpiDev &e,
+                    hipStream_t s);
 int contract_ksplit(const void *x, bool a16, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                     int sh, int sw, int dh, int dw, int Ho, int Wo, bool patch, const EpiDev &e, hipStream_t s);
 
@@ -554,6 +556,10 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   if (p.M >= (1ll << 31)) return -1;  // the loaders split a pixel index with 32-bit divisions
   if (Ci == 8 && ph == 0 && pw == 0 && dw == 1) {  // framed few-channel image: streaming kernel
     const int st = conv2d_stem_a16(x, w, N, H, W, Co, kh, kw, sh, sw, dh, Ho, Wo, e, s);
+    if (st >= 0) return st;
+  }
+  if (Ci == 32 && kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1) {  // walks over tiles
+    const int st = conv3x3_a16_c32(x, w, N, H, W, Co, sh, Ho, Wo, e, s);
     if (st >= 0) return st;
   }
   // a pointwise convolution is a plain GEMM over the pixels: row address = index x K, no pixel split and no

@@ -1,0 +1,44 @@
+"""3 x 3 convolutions of 32 int16 channels (the kernel that walks over tiles of 16 x 4 outputs) against 64-bit sums and the epilogue's
+operations in fp32."""
+import pytest
+import torch
+
+import catch_amd  # noqa: F401  (registers torch_mlu::*)
+
+pytestmark = pytest.mark.gpu
+
+
+# edges of tiles either way, images smaller than one, more tiles than blocks, channels that end inside a wave's or are one wave's less
+@pytest.mark.parametrize("n,h,w,co,stride", [
+    (1, 1, 1, 64, 1), (1, 1, 1, 64, 2), (2, 4, 16, 64, 1), (1, 5, 17, 36, 1), (3, 7, 33, 64, 2), (1, 8, 32, 60, 2), (2, 9, 15, 48, 2),
+    (1, 3, 50, 64, 1), (4, 66, 130, 64, 1), (5, 129, 131, 64, 2),
+    (1, 6, 6, 32, 1), (1, 6, 6, 68, 1),  # not this kernel's
+])
+def test_conv_c32(n, h, w, co, stride):
+    gen = torch.Generator().manual_seed(h * w + co)
+    x = torch.randint(-32768, 32768, (n, h, w, 32), generator=gen).short()
+    x.view(-1)[:2] = torch.tensor([-32768, 32767])
+    qw = torch.randint(-128, 128, (co, 3, 3, 32), generator=gen).to(torch.int8)
+    bias = torch.randn(co, generator=gen)
+    acc = torch.nn.functional.conv2d(x.double().permute(0, 3, 1, 2), qw.double().permute(0, 3, 1, 2), stride=stride, padding=1)
+    acc = acc.permute(0, 2, 3, 1).contiguous()  # exact: below 9 * 32 * 2^22
+    resid = torch.randn(acc.shape, generator=gen)
+    xd, qd, bd, rd = x.cuda(), qw.cuda(), bias.cuda(), resid.cuda()
+    op = torch.ops.torch_mlu.qconv2d
+
+    def run(r, act, *rest):
+        return op(xd, qd, -20, None, bd, r, [1, 1], [stride, stride], [1, 1], 1, act, *rest)
+
+    y, _, got = run(None, 0, True, False, True)
+    v = acc.float() * 2.0 ** -20 + bias
+    assert torch.equal(got.cpu().double(), acc) and torch.equal(y.cpu(), v)
+    leaky = torch.where(v > 0, v, v * torch.tensor(0.1))
+    for r, want_y in [(None, False), (None, True), (rd, False), (rd, True)]:
+        want = leaky if r is None else leaky + resid
+        y, q, _ = run(r, 3, want_y, False, False, 16, -7, 1.0, 0.1, True)
+        assert torch.equal(q.cpu().int(), torch.clamp(torch.round(want * 128), -32768, 32767).int())
+        assert not want_y or torch.equal(y.cpu(), want)
+    y, q, _ = run(rd, 1, True, True, False, 8, -2, 1.3, 0.0, False)
+    want = torch.relu(v + resid)
+    assert torch.equal(y.cpu(), want.half())
+    assert torch.equal(q.cpu().int(), torch.clamp(torch.round(want * torch.tensor(1.3) * 4), -128, 127).int())

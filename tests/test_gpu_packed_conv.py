@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+import catch_amd  # noqa: F401  (registers torch_mlu::*)
+
 pytestmark = pytest.mark.gpu
 
 
