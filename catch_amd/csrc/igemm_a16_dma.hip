@@ -417,8 +417,8 @@ int igemm_a16_launch(int load, const void *a, const void *b, IgemmParams p, cons
   return -1;
 }
 
-int conv3x3_a16_c32(const void *x, const void *w, int N, int H, int W, int Co, int stride, int Ho, int Wo, const EpiDev &e,
-                    hipStream_t s);
+int conv3x3_a16_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
+                     hipStream_t s);
 int contract_ksplit(const void *x, bool a16, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                     int sh, int sw, int dh, int dw, int Ho, int Wo, bool patch, const EpiDev &e, hipStream_t s);
 
@@ -549,6 +549,10 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo;
   p.kh = kh; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
   p.K = kh * kw * Ci;
+  if ((Ci == 32 || Ci == 64) && kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1) {  // walks over tiles
+    const int st = conv3x3_a16_walk(x, w, N, H, W, Ci, Co, sh, Ho, Wo, e, s);
+    if (st >= 0) return st;
+  }
   if (Ci % 16 == 0) {  // a few blocks per unit, long K
     const int st = contract_ksplit(x, true, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false, e, s);
     if (st >= 0) return st;
@@ -556,10 +560,6 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   if (p.M >= (1ll << 31)) return -1;  // the loaders split a pixel index with 32-bit divisions
   if (Ci == 8 && ph == 0 && pw == 0 && dw == 1) {  // framed few-channel image: streaming kernel
     const int st = conv2d_stem_a16(x, w, N, H, W, Co, kh, kw, sh, sw, dh, Ho, Wo, e, s);
-    if (st >= 0) return st;
-  }
-  if (Ci == 32 && kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1) {  // walks over tiles
-    const int st = conv3x3_a16_c32(x, w, N, H, W, Co, sh, Ho, Wo, e, s);
     if (st >= 0) return st;
   }
   // a pointwise convolution is a plain GEMM over the pixels: row address = index x K, no pixel split and no

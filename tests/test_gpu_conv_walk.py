@@ -1,5 +1,5 @@
-"""3 x 3 convolutions of 32 int16 channels (the kernel that walks over tiles of 16 x 4 outputs) against 64-bit sums and the epilogue's
-operations in fp32."""
+"""3 x 3 convolutions of 32 and 64 int16 channels (the kernel that walks over small tiles of the outputs) against
+64-bit sums and the epilogue's operations in fp32."""
 import pytest
 import torch
 
@@ -9,19 +9,22 @@ pytestmark = pytest.mark.gpu
 
 
 # edges of tiles either way, images smaller than one, more tiles than blocks, channels that end inside a wave's or are one wave's less
-@pytest.mark.parametrize("n,h,w,co,stride", [
-    (1, 1, 1, 64, 1), (1, 1, 1, 64, 2), (2, 4, 16, 64, 1), (1, 5, 17, 36, 1), (3, 7, 33, 64, 2), (1, 8, 32, 60, 2), (2, 9, 15, 48, 2),
-    (1, 3, 50, 64, 1), (4, 66, 130, 64, 1), (5, 129, 131, 64, 2),
-    (1, 6, 6, 32, 1), (1, 6, 6, 68, 1),  # not this kernel's
+@pytest.mark.parametrize("n,h,w,ci,co,stride", [
+    (1, 1, 1, 32, 64, 1), (1, 1, 1, 32, 64, 2), (2, 4, 16, 32, 64, 1), (1, 5, 17, 32, 36, 1), (3, 7, 33, 32, 64, 2), (1, 8, 32, 32, 60, 2),
+    (2, 9, 15, 32, 48, 2), (1, 3, 50, 32, 64, 1), (4, 66, 130, 32, 64, 1), (5, 129, 131, 32, 64, 2),
+    (3, 33, 60, 64, 128, 1), (13, 7, 62, 64, 68, 1), (2, 67, 130, 64, 128, 2), (3, 129, 66, 64, 100, 2),
+    (200, 3, 3, 64, 96, 1), (200, 4, 8, 64, 128, 2),
+    (1, 6, 6, 32, 32, 1), (1, 6, 6, 32, 68, 1),  # not this kernel's
 ])
-def test_conv_c32(n, h, w, co, stride):
+def test_conv_walk(n, h, w, ci, co, stride):
     gen = torch.Generator().manual_seed(h * w + co)
-    x = torch.randint(-32768, 32768, (n, h, w, 32), generator=gen).short()
+    x = torch.randint(-32768, 32768, (n, h, w, ci), generator=gen).short()
     x.view(-1)[:2] = torch.tensor([-32768, 32767])
-    qw = torch.randint(-128, 128, (co, 3, 3, 32), generator=gen).to(torch.int8)
+    top = 4096 // ci - 1  # (the true sums fit 32 bits)
+    qw = torch.randint(-top - 1, top + 1, (co, 3, 3, ci), generator=gen).to(torch.int8)
     bias = torch.randn(co, generator=gen)
     acc = torch.nn.functional.conv2d(x.double().permute(0, 3, 1, 2), qw.double().permute(0, 3, 1, 2), stride=stride, padding=1)
-    acc = acc.permute(0, 2, 3, 1).contiguous()  # exact: below 9 * 32 * 2^22
+    acc = acc.permute(0, 2, 3, 1).contiguous()  # exact: below 9 * 2^27
     resid = torch.randn(acc.shape, generator=gen)
     xd, qd, bd, rd = x.cuda(), qw.cuda(), bias.cuda(), resid.cuda()
     op = torch.ops.torch_mlu.qconv2d
