@@ -45,3 +45,34 @@ def test_conv_walk(n, h, w, ci, co, stride):
     want = torch.relu(v + resid)
     assert torch.equal(y.cpu(), want.half())
     assert torch.equal(q.cpu().int(), torch.clamp(torch.round(want * torch.tensor(1.3) * 4), -128, 127).int())
+
+
+# int8: more tiles than the rule asks for (sharing makes it plan for 256 / sharing units), edges of tiles either way, fewer than one wave's
+# channels, all eight waves
+@pytest.mark.parametrize("n,h,w,ci,co,stride,sharing", [
+    (1, 4, 8, 16, 16, 1, 256), (1, 9, 33, 16, 36, 1, 64), (3, 13, 17, 32, 256, 1, 64), (2, 10, 16, 32, 4, 1, 64), (5, 129, 131, 16, 20, 1, 1),
+    (2, 17, 30, 16, 128, 2, 64), (3, 16, 31, 32, 100, 2, 64), (40, 66, 50, 32, 256, 2, 1), (2, 60, 60, 32, 64, 2, 64),
+    (1, 9, 33, 32, 260, 1, 64), (4, 33, 33, 48, 64, 1, 64), (4, 60, 60, 32, 32, 2, 1),  # not this kernel's
+])
+def test_conv_walk_int8(n, h, w, ci, co, stride, sharing):
+    gen = torch.Generator().manual_seed(h * w + co)
+    x = torch.randint(-128, 128, (n, h, w, ci), generator=gen).to(torch.int8)
+    qw = torch.randint(-128, 128, (co, 3, 3, ci), generator=gen).to(torch.int8)
+    bias = torch.randn(co, generator=gen)
+    div = (torch.rand(co, generator=gen) + 0.5)
+    acc = torch.nn.functional.conv2d(x.float().permute(0, 3, 1, 2), qw.float().permute(0, 3, 1, 2), stride=stride, padding=1)
+    acc = acc.permute(0, 2, 3, 1).contiguous()  # exact: below 9 * 32 * 2^14 < 2^24
+    resid = torch.randn(acc.shape, generator=gen)
+    xd, qd, bd, dd, rd = x.cuda(), qw.cuda(), bias.cuda(), div.cuda(), resid.cuda()
+    v = acc * 2.0 ** -12 / div + bias
+    torch.ops.torch_mlu.set_launch_sharing(sharing)
+    try:
+        def run(r, act, *rest):
+            return torch.ops.torch_mlu.qconv2d(xd, qd, -12, dd, bd, r, [1, 1], [stride, stride], [1, 1], 1, act, *rest)
+        assert torch.equal(run(None, 0, True)[0].cpu(), v)
+        y, _, got = run(rd, 1, True, True, True)
+        assert torch.equal(got.cpu().float(), acc) and torch.equal(y.cpu(), torch.relu(v + resid).half())
+        q = run(None, 1, False, False, False, 8, -4)[1]
+        assert torch.equal(q.cpu().int(), torch.clamp(torch.round(torch.relu(v) * 16), -128, 127).int())
+    finally:
+        torch.ops.torch_mlu.set_launch_sharing(1)
