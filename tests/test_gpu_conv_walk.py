@@ -76,3 +76,32 @@ def test_conv_walk_int8(n, h, w, ci, co, stride, sharing):
         assert torch.equal(q.cpu().int(), torch.clamp(torch.round(torch.relu(v) * 16), -128, 127).int())
     finally:
         torch.ops.torch_mlu.set_launch_sharing(1)
+
+
+# rows that end inside a block's, columns that end inside a wave's, every count of waves side by side
+@pytest.mark.parametrize("n,h,w,ci,co", [
+    (1, 1, 1, 64, 4), (1, 3, 43, 64, 32), (2, 8, 8, 64, 36), (1, 5, 13, 64, 64), (3, 11, 3, 64, 100), (1, 8, 16, 64, 128), (3, 61, 67, 64, 96),
+    (1, 1, 1, 128, 32), (1, 7, 9, 128, 28), (1, 8, 8, 128, 64), (5, 13, 5, 128, 68), (2, 31, 33, 128, 128), (2, 9, 9, 64, 132), (2, 9, 9, 192, 64),
+])
+def test_pointwise_int16(n, h, w, ci, co):
+    gen = torch.Generator().manual_seed(h * w + co)
+    x = torch.randint(-32768, 32768, (n, h, w, ci), generator=gen).short()
+    x.view(-1)[:2] = torch.tensor([-32768, 32767])
+    qw = torch.randint(-128, 128, (co, 1, 1, ci), generator=gen).to(torch.int8)
+    bias = torch.randn(co, generator=gen)
+    acc = (x.double().reshape(-1, ci) @ qw.double().reshape(co, ci).t()).reshape(n, h, w, co)  # exact: below 192 * 2^22
+    resid = torch.randn(acc.shape, generator=gen)
+    xd, qd, bd, rd = x.cuda(), qw.cuda(), bias.cuda(), resid.cuda()
+
+    def run(r, act, *rest):
+        return torch.ops.torch_mlu.qconv2d(xd, qd, -20, None, bd, r, [0, 0], [1, 1], [1, 1], 1, act, *rest)
+
+    v = acc.float() * 2.0 ** -20 + bias
+    y, _, got = run(None, 0, True, False, True)
+    assert torch.equal(got.cpu().double(), acc) and torch.equal(y.cpu(), v)
+    leaky = torch.where(v > 0, v, v * torch.tensor(0.1))
+    q = run(None, 3, False, False, False, 16, -7, 1.0, 0.1)[1]
+    assert torch.equal(q.cpu().int(), torch.clamp(torch.round(leaky * 128), -32768, 32767).int())
+    y, q, _ = run(rd, 3, True, True, False, 16, -7, 1.0, 0.1, True)
+    assert torch.equal(y.cpu(), (leaky + resid).half())
+    assert torch.equal(q.cpu().int(), torch.clamp(torch.round((leaky + resid) * 128), -32768, 32767).int())
