@@ -322,7 +322,7 @@ def plan_launches(fused, n, h, w):
             b += ((2 if y_half else 4) * n_out if want_y else 0) + (n_out * qd[0] // 8 if qd else 0)
             rows.append(dict(name=l.name, kind="conv", ops=2 * macs, bytes=b, m=n * ho * wo, n=fused.cdev[l.name],
                              k=lq.qw.numel() // lq.qw.shape[0] + k_extra))
-            for d in fused.q_demand[l.name][1:]:
+            for d in fused._further_forms(l.name):
                 rows.append(dict(name=l.name, kind="quantize", ops=0, bytes=n_out * 4 + n_out * d[0] // 8))
         elif l.kind == "fc":
             lq = fused.q[l.name]
@@ -355,6 +355,8 @@ def plan_launches(fused, n, h, w):
             hi, wi = shape[l.src]
             shape[l.name] = (hi * 2, wi * 2)
             for form in fused._forms(l.name):  # torch's repeat_interleave, twice: rows doubled, then columns
+                if (l.name,) + form in fused.at_concat:
+                    continue  # inside the concatenation's launch
                 e = 4 if form == ("f",) else form[0] // 8
                 rows.append(dict(name=l.name, kind="upsample", ops=0, bytes=n * fused.cdev[l.src] * e * hi * wi * 3))
                 rows.append(dict(name=l.name, kind="upsample", ops=0, bytes=n * fused.cdev[l.src] * e * hi * wi * 6))
@@ -363,7 +365,9 @@ def plan_launches(fused, n, h, w):
             hi, wi = shape[l.name]
             for form in fused._forms(l.name):
                 e = 4 if form == ("f",) else form[0] // 8
-                rows.append(dict(name=l.name, kind="concat", ops=0, bytes=2 * n * fused.cdev[l.name] * e * hi * wi))
+                kinds = fused.concat_kinds.get((l.name, form), [0] * len(l.src))  # copied, upsampled, quantized from fp32
+                read = sum(fused.cdev[s] * hi * wi * (e, e / 4, 4)[k] for s, k in zip(l.src, kinds))
+                rows.append(dict(name=l.name, kind="concat", ops=0, bytes=n * int(read) + n * fused.cdev[l.name] * e * hi * wi))
     return rows
 
 
@@ -698,7 +702,7 @@ def main():
         print("sum of conv/fc launches (%d parts of %d images): %.1f us repeated back to back, %.1f us in sequence; graph step: %.1f us" % (
             n_parts, parts[0].shape[0], t_all * 1e6, n_parts * sum(r["t_seq"] for r in rows) * 1e6, ms_per_step * 1e3), file=sys.stderr)
     roofline = {"bound": "hbm", "kernel": "%s (all %d launches of one step: %d layers x %d parts of the batch)" % (
-                    "igemm_a16_dma_kernel" if detector else "igemm_i8_dma_kernel + conv3x3_halo_kernel + igemm_i8_chain_kernel",
+                    "igemm_a16_dma_kernel + conv3x3_a16_packed_kernel + conv3x3_a16_walk_kernel + pw_a16_short_kernel" if detector else "igemm_i8_dma_kernel + conv3x3_halo_kernel + igemm_i8_chain_kernel",
                     n_parts * len(conv_rows), len(conv_rows), n_parts),
                 "achieved": round(b_conv / t_conv / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(b_conv / t_conv / 1e9 / HBM_PEAK_GBS, 4),

@@ -516,6 +516,11 @@ class FusedNet(object):
         for l in self.layers:
             if l.kind in ("conv", "fc") and len(self.q_demand[l.name]) > 1:
                 self.f_demand[l.name] = True
+                # forms that a layer multiplies come first: a concatenation can make its own from the fp32 copy (Darknet-53 with
+                # YOLOv3 heads, 16 images of 416 x 416: 18 us of two quantizers for 6 us more in the concatenations)
+                read = set((self.q[m.name].bw_x, self.q[m.name].pos_x, self.q[m.name].scale_x) for m in self.layers
+                           if m.kind in ("conv", "fc") and m.src == l.name)
+                self.q_demand[l.name].sort(key=lambda d: d not in read)
         self._plan_concats()
 
     def _plan_concats(self):

@@ -66,6 +66,11 @@ def test_detector_routes_are_one_launch_each():
     keep = {}
     out = fused.forward(x.cuda(), keep=keep)
     assert ("up26",) + fused.q_demand["up26"][0] not in keep and fused.at_concat
+    for route, cat in (("c26", "cat52"), ("c43", "cat26")):  # what the next layer multiplies is written by the epilogue
+        forms = fused.q_demand[route]
+        nxt = fused.q["c%d" % (int(route[1:]) + 1)]
+        assert forms[0] == (nxt.bw_x, nxt.pos_x, nxt.scale_x)
+        assert len(forms) == 1 or (forms[1] == fused.q_demand[cat][0] and fused._further_forms(route) == [])
     plain = pipeline.FusedNet(layers, sd)
     for p in (plain, plain._few_plan()):
         p.concat_kinds, p.at_concat = {}, set()
