@@ -1078,8 +1078,8 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// The entry's weight as catchq_float_linear_packed (8 bits) and catchq_float_linear_digits (16) read it; null: the call goes
-// without.  The weight is laid out at the second call that the route takes.  A caller that rewrites its weight between calls, or
+// The entry's weight as catchq_float_linear_packed and catchq_conv3x3_i8_packed (8 bits) and catchq_float_linear_digits (16) read
+// it; null: the call goes without.  The weight is laid out at the second call that the route takes.  A caller that rewrites its weight between calls, or
 // uses it once, does not pay for that (6 us of kernel, a launch and an allocation: first pass of 1 x 768 -> 3072 on a new
 // weight 226 us with it, 218 without), and a weight whose calls do not take the route is not held twice.
 template <typename Takes>
@@ -1251,6 +1251,15 @@ catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64
   return e;
 }
 
+// The filters of a 3 x 3 layer that catchq_conv3x3_i8_packed takes; null: another route serves it.
+const void *conv3x3_packed(Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e) {
+  if (prep.bw_x != 8 || prep.bw_w != 8 || d.kh != 3 || d.kw != 3 || d.groups != 1 || d.pad_h != 1 || d.pad_w != 1 || d.stride_h != 1 ||
+      d.stride_w != 1 || d.dil_h != 1 || d.dil_w != 1 || d.ci % 32 != 0)
+    return nullptr;
+  if (catchq_conv3x3_i8_packed_takes(d.n, d.h, d.w, d.ci, d.co, &e) != CATCHQ_OK) return nullptr;
+  return packed_weight(prep, [] { return true; });
+}
+
 // quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x) x prepared weight -> floating
 // output, logical [N,Co,Ho,Wo] over NHWC memory
 Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Prepared &prep, const Tensor &bias,
@@ -1271,7 +1280,15 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Pr
   if (d.n == 0 || d.co == 0) return y;  // nothing to compute: the empty output is the result
   Tensor keep;
   const catchq_epilogue_t e = prepared_epilogue(prep, bias, d.co, y, &keep);
+  const void *packed = conv3x3_packed(prep, d, e);
   if (qx.defined()) {
+    if (packed) {
+      const int st = catchq_conv3x3_i8_packed(qx.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
+      if (st != CATCHQ_ERR_UNSUPPORTED) {
+        check_status(st, "torch_mlu::conv2d");
+        return y;
+      }
+    }
     check_status(catchq_conv2d_nhwc(qx.data_ptr(), bits_of(qx), qw.data_ptr(), bits_of(qw), &d, &e, current_stream()),
                  "torch_mlu::conv2d");
     return y;
@@ -1292,6 +1309,17 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Pr
   }
   size_t ws_bytes = 0;
   check_status(catchq_float_conv2d_workspace_size(dt, &d, &e, &ws_bytes), "torch_mlu::conv2d");
+  if (packed && ws_bytes) {  // (two launches either way)
+    const int64_t elems = (int64_t)d.n * d.h * d.w * d.ci;
+    Tensor qn = device_empty({elems}, at::kChar, qw.device());
+    check_status(catchq_quantize(x, dt, qn.data_ptr(), 8, elems, prep.pos_x, 1.0f, current_stream()), "torch_mlu::quantize");
+    const int st = catchq_conv3x3_i8_packed(qn.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
+    if (st == CATCHQ_ERR_UNSUPPORTED)
+      check_status(catchq_conv2d_nhwc(qn.data_ptr(), 8, qw.data_ptr(), 8, &d, &e, current_stream()), "torch_mlu::conv2d");
+    else
+      check_status(st, "torch_mlu::conv2d");
+    return y;
+  }
   if (reinterpret_cast<uintptr_t>(x) & 15u) ws_bytes = (size_t)d.n * d.h * d.w * d.ci;  // one launch takes aligned tensors only
   Tensor ws;
   if (ws_bytes) ws = device_empty({(int64_t)ws_bytes}, at::kChar, qw.device());

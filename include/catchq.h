@@ -277,6 +277,12 @@ int catchq_pack_conv3x3(const void *w, int64_t co, int64_t ci, void *packed, cat
 int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
                           const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 
+/* The same for int8 activations, ci a multiple of 32, and filters that catchq_pack_filters laid out from w [co, 9 * ci] (taps first).
+ * *_takes answers CATCHQ_ERR_UNSUPPORTED without a launch where catchq_conv2d_nhwc serves the call better, or alone. */
+int catchq_conv3x3_i8_packed_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue);
+int catchq_conv3x3_i8_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                             const catchq_epilogue_t *epilogue, catchq_stream_t stream);
+
 /* A linear on floating activations with int16 weights, both split into the bytes that the matrix cores multiply:
  *   cnnl_quantify_offline_internal (quantify.cpp:69-101) followed by linear.cpp:92-110, 16 bits on either side
  * catchq_pack_digits lays the weights out once (w [n,ld] int16, k values of a row used, k <= 8192); the call quantizes x [m,k]

@@ -92,3 +92,39 @@ def test_packed_conv3x3_other_calls():
         ops.qconv2d(x, qw, *args, 0, 0, 1.0, 0.0, False, packed[:-16].contiguous())
     with pytest.raises(RuntimeError):  # channels that are no multiple of 64
         ops.pack_conv3x3(qw[..., :48].contiguous())
+
+
+# edges of blocks of 32 and of 64 pixels and of images, one wave to eight and two blocks of them side by side; sharing makes the rule plan
+# for 256 / sharing units
+@pytest.mark.parametrize("n,ci,h,w,co,mode,dtype,nhwc,sharing", [
+    (1, 96, 1, 1, 4, 1, torch.float32, False, 256), (1, 96, 5, 13, 36, 3, torch.float32, False, 256), (3, 160, 7, 9, 100, 3, torch.float16, True, 256),
+    (1, 96, 3, 33, 256, 3, torch.float32, True, 64), (2, 192, 1, 50, 260, 3, torch.float32, False, 64), (5, 224, 6, 7, 512, 1, torch.float32, True, 64),
+    (2, 320, 9, 1, 64, 3, torch.float16, False, 256), (1, 96, 2, 300, 32, 3, torch.float32, False, 64), (2, 96, 57, 75, 160, 3, torch.float32, False, 1),
+    (1, 96, 9, 9, 30, 3, torch.float32, False, 256), (1, 128, 9, 9, 64, 3, torch.float32, False, 256), (1, 96, 9, 9, 64, 3, torch.float32, False, 1),
+])
+def test_packed_conv3x3_int8(n, ci, h, w, co, mode, dtype, nhwc, sharing):
+    """the first call of a weight goes without packed filters, later ones read them: the same bits, equal to the oracle's"""
+    from oracle import ops as oops
+    gen = torch.Generator().manual_seed(ci + h * w)
+    x = torch.randn(n, ci, h, w, generator=gen).to(dtype)
+    wt = (torch.randn(co, ci, 3, 3, generator=gen) * 0.05).to(dtype)
+    b = torch.randn(co, generator=gen).to(dtype)
+    top = wt.float().reshape(co, -1).abs()
+    scale = torch.cat([torch.tensor([127.0 / x.float().abs().max()]), torch.tensor([0.0]), 127.0 / top.amax(1)]) if mode == 3 else \
+        torch.tensor([127.0 / x.float().abs().max(), 127.0 / top.max()])
+    mode = torch.tensor([mode], dtype=torch.int32)
+    xd = x.cuda().contiguous(memory_format=torch.channels_last) if nhwc else x.cuda()
+    args = (xd, wt.cuda(), b.cuda(), [1, 1], [1, 1], [1, 1], 1, scale.cuda(), mode.cuda())
+    torch.ops.torch_mlu.set_launch_sharing(sharing)
+    try:
+        first, second, third = [torch.ops.torch_mlu.conv2d(*args) for _ in range(3)]
+        xd.mul_(0.5)  # other inputs through the same filters
+        other = torch.ops.torch_mlu.conv2d(*args)
+    finally:
+        torch.ops.torch_mlu.set_launch_sharing(1)
+    assert torch.equal(first, second) and torch.equal(second, third)
+    if dtype == torch.float32:
+        ref = oops.conv2d(x.numpy(), wt.numpy(), b.numpy(), (1, 1), (1, 1), (1, 1), 1, scale.numpy(), mode.numpy())
+        assert torch.equal(torch.from_numpy(ref["y"]), second.cpu().contiguous())
+        ref = oops.conv2d(xd.cpu().contiguous().numpy(), wt.numpy(), b.numpy(), (1, 1), (1, 1), (1, 1), 1, scale.numpy(), mode.numpy())
+        assert torch.equal(torch.from_numpy(ref["y"]), other.cpu().contiguous())
