@@ -59,6 +59,11 @@ class ChainLink(ctypes.Structure):
                 ("chan_rcp", ctypes.c_void_p), ("bias", ctypes.c_void_p)]
 
 
+class ConcatSource(ctypes.Structure):
+    """struct catchq_concat_source"""
+    _fields_ = [("x", ctypes.c_void_p), ("channels", ctypes.c_int), ("kind", ctypes.c_int)]
+
+
 # name -> (restype, argtypes); every symbol include/catchq.h declares
 _I, _I64, _F, _P, _SZ = ctypes.c_int, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p, ctypes.c_size_t
 SIGNATURES = {
@@ -87,6 +92,12 @@ SIGNATURES = {
     "catchq_global_avgpool_quantize_nhwc": (_I, [_P, _P, _I, _I, _I, _I, _I, _F, _P]),
     "catchq_quantize_conv2d_workspace_size": (_I, [ctypes.POINTER(ConvDesc), _I, _I, ctypes.POINTER(_SZ)]),
     "catchq_quantize_conv2d_nhwc": (_I, [_P, _I, _P, _I, _P, _I, _P, _I, ctypes.POINTER(ConvDesc), _P, _P, _I, _P, _SZ, _P]),
+    "catchq_packed_conv3x3_size": (_I, [_I64, _I64, ctypes.POINTER(_SZ)]),
+    "catchq_pack_conv3x3": (_I, [_P, _I64, _I64, _P, _P]),
+    "catchq_conv3x3_packed": (_I, [_P, _P, _I, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P]),
+    "catchq_conv3x3_i8_packed_takes": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(Epilogue)]),
+    "catchq_conv3x3_i8_packed": (_I, [_P, _P, _I, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P]),
+    "catchq_concat_nhwc": (_I, [ctypes.POINTER(ConcatSource), _I, _I, _I, _F, _I, _I, _I, _P, _P]),
     "catchq_packed_digits_size": (_I, [_I64, _I64, ctypes.POINTER(_SZ)]),
     "catchq_pack_digits": (_I, [_P, _I64, _I64, _I64, _P, _P]),
     "catchq_float_linear_digits_workspace_size": (_I, [_I64, _I64, _I64, ctypes.POINTER(Epilogue), ctypes.POINTER(_SZ)]),

@@ -450,3 +450,26 @@ def test_replay_owns_its_graphs_and_their_input(monkeypatch):
         assert kept() is None and graph() is None
     finally:
         gc.enable()
+
+
+def test_packed_conv3x3_refusals(lib):
+    """what the 3 x 3 routes on packed filters answer before anything is launched: sizes, and which calls are served elsewhere"""
+    import ctypes
+    from catch_amd import _native
+    OK, ARG, UNSUPPORTED = 0, 1, 6
+    sz = ctypes.c_size_t()
+    assert lib.catchq_packed_conv3x3_size(256, 64, ctypes.byref(sz)) == OK and sz.value >= 256 * 9 * 64 + 4 * 256
+    assert lib.catchq_packed_conv3x3_size(256, 96, ctypes.byref(sz)) == UNSUPPORTED
+    assert lib.catchq_packed_conv3x3_size(0, 64, ctypes.byref(sz)) == ARG
+    assert lib.catchq_packed_conv3x3_size(1 << 20, 1 << 14, ctypes.byref(sz)) == UNSUPPORTED
+    e = _native.Epilogue()
+    assert lib.catchq_conv3x3_i8_packed_takes(5, 57, 75, 96, 160, ctypes.byref(e)) == ARG  # an epilogue without an output
+    e.y = 16
+    takes = lambda *a: lib.catchq_conv3x3_i8_packed_takes(*a, ctypes.byref(e))  # noqa: E731
+    assert takes(5, 57, 75, 96, 160) == OK and takes(0, 57, 75, 96, 160) == OK
+    for n, h, w, ci, co in [(5, 57, 75, 64, 160), (5, 57, 75, 128, 160), (5, 57, 75, 112, 160), (1, 28, 28, 192, 192), (5, 57, 75, 96, 162),
+                            (1, 57, 600, 96, 160), (1, 1 << 20, 8, 96, 160), (64, 1000, 400, 96, 32), (1 << 20, 64, 64, 96, 32)]:
+        assert takes(n, h, w, ci, co) == UNSUPPORTED, (n, h, w, ci, co)
+    assert takes(5, 0, 75, 96, 160) == ARG
+    e.sharing = 4  # a quarter of the units: fewer blocks will do
+    assert takes(1, 28, 28, 192, 192) == UNSUPPORTED and takes(2, 28, 28, 192, 192) == OK
