@@ -217,7 +217,7 @@ def layer_profile(fused, x, iters=20, only=None):
                                    [l.stride, l.stride], [1, 1], lq.groups,
                                    {"none": 0, "relu": 1, "relu6": 2, "leaky": 3}[l.act],
                                    want_y, y_half, False, qd[0] if qd else 0, qd[1] if qd else 0, 1.0, 0.1,
-                                   bool(l.add_after))
+                                   bool(l.add_after), getattr(lq, "packed", None))
             route = ops.conv2d_route(lq.bw_x, lq.bw_w, list(qx.shape), list(lq.qw.shape[:3]) + [lq.qw.shape[3]],
                                      fused.padding(l), [l.stride, l.stride], [1, 1], lq.groups)
         else:

@@ -131,12 +131,10 @@ static int launch_packed_i8(const void *x, const void *w, const PackedI8Params &
 // The rows of 32 pixels a wave takes, 0: not this kernel's shape
 static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e) {
   const int64_t M = N * H * W, groups = ((int64_t)Co + 31) / 32;
-  if (Ci % 32 != 0 || Ci > 1024 || W > 512 || H >= (1 << 20) || M * Ci >= (1ll << 31) || groups * Ci * 288 >= (1ll << 31)) return 0;
+  // (the patch-resident kernels: 32 x 28 x 28, 128 channels, 16.4 / 16.8 us with this one, 32 x 14 x 14, 256 14.0 / 15.0)
+  if (!conv3x3_i8_packed_channels(Ci) || W > 512 || H >= (1 << 20) || M * Ci >= (1ll << 31) || groups * Ci * 288 >= (1ll << 31)) return 0;
   const int epi = pick_epilogue(Co, e);
   if (epi != EPI_Y32 && epi != EPI_Y16 && epi != EPI_Y16_STEPS && epi != EPI_VECTOR) return 0;
-  // the patch-resident kernels (conv3x3_halo_i8.hip) are ahead on the channels they have instances for (32 x 28 x 28, 128: 16.4 / 16.8,
-  // 32 x 14 x 14, 256: 14.0 / 15.0), the kernel that walks over tiles (conv3x3_i8_walk.hip) on 32
-  if (Ci < 96 || Ci == 128 || Ci == 256 || Ci == 512) return 0;
   // Half a block of 32 pixels for a unit (us, tiled / this: 1 x 57 x 75, 96 -> 160, 134 blocks, 9.7 / 9.0, 10 x 14 x 14, 160 -> 512, 124,
   // 11.2 / 11.3, 3 x 30 x 33, 448 -> 224, 93, 14.9 / 16.0, 1 x 28 x 28, 192, 25, 7.9 / 9.8); blocks of 64, which read half the
   // filters, from as many of those on (8 x 25 x 25, 160 -> 320, 158, 13.3 / 12.6 with 64; 8 x 28 x 28, 192, 98, 11.5 / 13.4).

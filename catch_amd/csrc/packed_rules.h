@@ -23,4 +23,10 @@ inline bool digits_sizes(int64_t m, int64_t n, int64_t k, int cus) {
   return k >= 32 && k <= kDigitsMaxK && (m + 63) / 64 * ((n + 127) / 128) * 8 >= 5 * (int64_t)cus;
 }
 
+// int8, conv3x3_i8_packed: the patch-resident kernels (conv3x3_halo_i8.hip) are ahead on the channels they have instances for, the one
+// that walks over tiles (conv3x3_i8_walk.hip) on 32
+inline bool conv3x3_i8_packed_channels(int64_t ci) {
+  return ci >= 96 && ci <= 1024 && ci % 32 == 0 && ci != 128 && ci != 256 && ci != 512;
+}
+
 }  // namespace catchq
