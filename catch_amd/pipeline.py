@@ -160,7 +160,8 @@ def _decode(layer, sd, device, ci_dev, co_dev, fractional=False):
             q.chan_div = pad(q.chan_div, (0, co_dev - co), value=1.0)
     q.qw = qw.contiguous()
     q.packed = None
-    if (layer.kind, layer.k, layer.stride, layer.pad, q.groups, q.bw_x, q.bw_w) == ("conv", 3, 1, 1, 1, 16, 8) and ci_dev % 64 == 0:
+    if ((layer.kind, layer.k, layer.stride, layer.pad, q.groups, q.bw_x, q.bw_w) == ("conv", 3, 1, 1, 1, 16, 8)
+            and ci_dev % 64 == 0 and q.qw.numel() < 1 << 30):  # (larger filters have no packed form)
         q.packed = torch.ops.torch_mlu.pack_conv3x3(q.qw)  # (read by the launches that the kernel on packed filters serves)
     return q
 
