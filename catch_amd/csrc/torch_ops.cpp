@@ -1552,7 +1552,6 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   return y;
 }
 
-// x [N,H,W,C] contiguous int8 / int16 / fp32
 // Channel concatenation of quantized tensors (catchq_concat_nhwc): kinds[i] says in which form source i is given.
 Tensor concat_nhwc_op(at::TensorList xs, at::IntArrayRef kinds, int64_t bitwidth, int64_t position, double scale) {
   TORCH_CHECK(!xs.empty() && xs.size() == kinds.size(), "concat_nhwc: one kind for every source");
@@ -1579,6 +1578,7 @@ Tensor concat_nhwc_op(at::TensorList xs, at::IntArrayRef kinds, int64_t bitwidth
   return out;
 }
 
+// x [N,H,W,C] contiguous int8 / int16 / fp32
 Tensor maxpool_nhwc_op(const Tensor &x, int64_t k, int64_t stride, int64_t pad) {
   TORCH_CHECK(x.dim() == 4 && x.is_contiguous(), "maxpool_nhwc expects a contiguous [N,H,W,C] tensor");
   int bits = 0;
