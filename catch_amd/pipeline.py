@@ -25,6 +25,7 @@ from .nets import LEAKY_SLOPE, outputs_of
 _ACT_CODE = {"none": 0, "relu": 1, "relu6": 2, "leaky": 3}
 _PASS = ("maxpool", "upsample", "concat")
 _CONCAT_COPY, _CONCAT_UP2, _CONCAT_FLOAT = range(3)  # CATCHQ_CONCAT_*
+_CONCAT_PIECES = 1 << 31  # of 16 bytes: catchq_concat_nhwc counts them in 31 bits (and the pixels, which are no more)
 
 
 def _key(name):
@@ -565,7 +566,13 @@ class FusedNet(object):
         by_name = {m.name: m for m in self.layers}
         xs = [env[(by_name[s].src,) + form] if k == _CONCAT_UP2 else env[(s, "f")] if k == _CONCAT_FLOAT else env[(s,) + form]
               for s, k in zip(l.src, kinds)]
-        return torch.ops.torch_mlu.concat_nhwc(xs, kinds, form[0], form[1], form[2])
+        pixels = xs[0].shape[0] * xs[0].shape[1] * xs[0].shape[2] * (4 if kinds[0] == _CONCAT_UP2 else 1)
+        if pixels * sum(x.shape[3] for x in xs) * form[0] // 128 < _CONCAT_PIECES:
+            return torch.ops.torch_mlu.concat_nhwc(xs, kinds, form[0], form[1], form[2])
+        # more than one launch takes: the sources as they would be stored
+        return torch.cat([x.repeat_interleave(2, 1).repeat_interleave(2, 2) if k == _CONCAT_UP2 else
+                          torch.ops.torch_mlu.quantize(x, form[0], form[1], form[2]) if k == _CONCAT_FLOAT else x
+                          for x, k in zip(xs, kinds)], 3)
 
     # ------------------------------------------------------------------------------------------
     def forward(self, x, trace=None, timers=None, keep=None):

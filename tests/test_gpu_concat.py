@@ -81,3 +81,24 @@ def test_detector_routes_are_one_launch_each():
     for key, t in keep.items():
         assert torch.equal(t, kept[key]), key
     assert len(kept) > len(keep)
+
+
+def test_routes_too_large_for_one_launch(monkeypatch):
+    """the same bits where a concatenation's sources are repeated, quantized and concatenated apart"""
+    layers = nets.darknet53_yolov3()
+    net = nets.FloatNet(layers, seed=3, weight_std="he").eval()
+    x = torch.rand(2, 3, 64, 96, generator=torch.Generator().manual_seed(5))
+    fused = pipeline.FusedNet(layers, pipeline.to_position_encoding(pipeline.calibrate(net, x, "int16", False), 16, 8))
+    want = fused(x.cuda())
+    monkeypatch.setattr(pipeline, "_CONCAT_PIECES", 1)
+    for a, b in zip(fused(x.cuda()), want):
+        assert torch.equal(a, b)
+    # a form that is quantized on the way
+    plan = pipeline.FusedNet.__new__(pipeline.FusedNet)
+    cat = nets.Layer("concat", "cat", ("a", "b"))
+    plan.layers, form = [cat], (16, -11, 1.37)
+    plan.concat_kinds = {("cat", form): [FLOAT, COPY]}
+    env = {("a", "f"): torch.randn(2, 5, 7, 16, device="cuda"), ("b",) + form: torch.full((2, 5, 7, 8), 7, dtype=torch.int16, device="cuda")}
+    apart = plan._concat(cat, form, env)
+    monkeypatch.undo()
+    assert apart.dtype == torch.int16 and torch.equal(apart, plan._concat(cat, form, env))

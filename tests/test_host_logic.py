@@ -473,3 +473,18 @@ def test_packed_conv3x3_refusals(lib):
     assert takes(5, 0, 75, 96, 160) == ARG
     e.sharing = 4  # a quarter of the units: fewer blocks will do
     assert takes(1, 28, 28, 192, 192) == UNSUPPORTED and takes(2, 28, 28, 192, 192) == OK
+
+
+def test_concatenations_beyond_one_launch():
+    """2^31 pieces of 16 bytes are more than the concatenating launch counts: repeated and concatenated apart, as before there was one"""
+    from catch_amd import nets, pipeline
+    plan = pipeline.FusedNet.__new__(pipeline.FusedNet)
+    up, cat = nets.Layer("upsample", "up", "a"), nets.Layer("concat", "cat", ("up", "b"))
+    form = (8, -5, 1.0)
+    plan.layers, plan.concat_kinds = [up, cat], {("cat", form): [pipeline._CONCAT_UP2, pipeline._CONCAT_COPY]}
+    meta = lambda *shape: torch.empty(shape, dtype=torch.int8, device="meta")  # noqa: E731
+    env = {("a",) + form: meta(64, 2048, 2048, 16), ("b",) + form: meta(64, 4096, 4096, 16)}
+    assert plan._concat(cat, form, env).shape == (64, 4096, 4096, 32)
+    env = {("a",) + form: meta(63, 2048, 2048, 16), ("b",) + form: meta(63, 4096, 4096, 16)}
+    with pytest.raises(NotImplementedError):  # one launch, which tensors without memory do not have
+        plan._concat(cat, form, env)
