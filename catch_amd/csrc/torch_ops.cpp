@@ -1280,9 +1280,8 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Pr
   if (d.n == 0 || d.co == 0) return y;  // nothing to compute: the empty output is the result
   Tensor keep;
   const catchq_epilogue_t e = prepared_epilogue(prep, bias, d.co, y, &keep);
-  const void *packed = conv3x3_packed(prep, d, e);
   if (qx.defined()) {
-    if (packed) {
+    if (const void *packed = conv3x3_packed(prep, d, e)) {
       const int st = catchq_conv3x3_i8_packed(qx.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
       if (st != CATCHQ_ERR_UNSUPPORTED) {
         check_status(st, "torch_mlu::conv2d");
@@ -1309,7 +1308,8 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Pr
   }
   size_t ws_bytes = 0;
   check_status(catchq_float_conv2d_workspace_size(dt, &d, &e, &ws_bytes), "torch_mlu::conv2d");
-  if (packed && ws_bytes) {  // (two launches either way)
+  const void *packed = ws_bytes ? conv3x3_packed(prep, d, e) : nullptr;  // (of one launch, the filters as they are)
+  if (packed) {
     const int64_t elems = (int64_t)d.n * d.h * d.w * d.ci;
     Tensor qn = device_empty({elems}, at::kChar, qw.device());
     check_status(catchq_quantize(x, dt, qn.data_ptr(), 8, elems, prep.pos_x, 1.0f, current_stream()), "torch_mlu::quantize");

@@ -128,3 +128,21 @@ def test_packed_conv3x3_int8(n, ci, h, w, co, mode, dtype, nhwc, sharing):
         assert torch.equal(torch.from_numpy(ref["y"]), second.cpu().contiguous())
         ref = oops.conv2d(xd.cpu().contiguous().numpy(), wt.numpy(), b.numpy(), (1, 1), (1, 1), (1, 1), 1, scale.numpy(), mode.numpy())
         assert torch.equal(torch.from_numpy(ref["y"]), other.cpu().contiguous())
+
+
+@pytest.mark.parametrize("n,ci,h,w,co,packs", [(1, 160, 57, 75, 96, False), (2, 96, 57, 75, 160, True)])
+def test_filters_are_held_twice_where_they_are_read(n, ci, h, w, co, packs):
+    """the first is one launch on floating activations and filters as they are, the second a quantizer and the packed filters"""
+    import gc
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn(n, ci, h, w, generator=gen, device="cuda").contiguous(memory_format=torch.channels_last)
+    wt, b = torch.randn(co, ci, 3, 3, generator=gen, device="cuda"), torch.randn(co, generator=gen, device="cuda")
+    scale, mode = torch.tensor([127 / 5.0, 127 / 5.0], device="cuda"), torch.tensor([1], dtype=torch.int32, device="cuda")
+    call = lambda: torch.ops.torch_mlu.conv2d(x, wt, b, [1, 1], [1, 1], [1, 1], 1, scale, mode)  # noqa: E731
+    gc.collect()
+    held = []
+    for _ in range(3):
+        call()
+        torch.cuda.synchronize()
+        held.append(torch.cuda.memory_allocated())
+    assert held[2] == held[1] and (held[1] - held[0] >= co * ci * 9) == packs and (held[1] == held[0]) == (not packs)
