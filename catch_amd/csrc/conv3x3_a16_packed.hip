@@ -218,12 +218,12 @@ static int launch_packed(const void *x, const void *w, const PackedConvParams &p
 
 // Where the blocks of 32 pixels leave most units without one, the waves that split K (ksplit.hip) are ahead: 5 x 13 x 13, 512 ->
 // 1024 (108 blocks for 256 units; the whole network 1000 / 1045 us), 2 x 13 x 13 (44) 9.8 / 16.9, 2 x 26 x 26 (86) 10.8 / 10.6;
-// 4 x 26 x 26 (170) 15.5 / 11.3.  Columns that do not exist cost as much as others: up to a quarter of them.
+// 4 x 26 x 26 (170) 15.5 / 11.3.
 bool conv3x3_a16_packed_takes(int N, int H, int W, int Ci, int Co, const EpiDev &e) {
   const int64_t M = (int64_t)N * H * W, columns = ((int64_t)Co + 255) / 256 * 256;
-  if (Ci % 64 != 0 || M * Ci * 2 >= (1ll << 31) || columns / 32 * Ci * 288 >= (1ll << 31) - (1 << 20)) return false;
+  if (!conv3x3_a16_packed_filters(Co, Ci) || M * Ci * 2 >= (1ll << 31) || columns / 32 * Ci * 288 >= (1ll << 31) - (1 << 20)) return false;
   if (W > 95 || H >= (1 << 20) || pick_epilogue(Co, e) == EPI_SCALAR) return false;
-  return Co * 4ll >= columns * 3 && (M + 31) / 32 * (columns / 256) * 8 >= 5 * (int64_t)e.cus;
+  return (M + 31) / 32 * (columns / 256) * 8 >= 5 * (int64_t)e.cus;
 }
 
 int64_t packed3x3_filter_bytes(int64_t Co, int64_t Ci) { return (Co + 31) / 32 * Ci * 288; }

@@ -29,4 +29,10 @@ inline bool conv3x3_i8_packed_channels(int64_t ci) {
   return ci >= 96 && ci <= 1024 && ci % 32 == 0 && ci != 128 && ci != 256 && ci != 512;
 }
 
+// int16 x int8, conv3x3_a16_packed: what its rule asks of the filters alone.  Blocks have 256 columns; those that do not exist cost as
+// much as others, up to a quarter of them pays.
+inline bool conv3x3_a16_packed_filters(int64_t co, int64_t ci) {
+  return ci % 64 == 0 && co % 4 == 0 && co * 4 >= (co + 255) / 256 * 256 * 3;
+}
+
 }  // namespace catchq

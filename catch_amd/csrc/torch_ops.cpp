@@ -550,6 +550,12 @@ std::tuple<Tensor, Tensor, Tensor> qconv2d_op(const Tensor &qx, const Tensor &qw
                                     q_position, q_scale, act_slope, resid_after_act), packed));
 }
 
+// Whether catchq_conv3x3_packed serves any call of such filters (by their channels: the rest of its rule is the image's)
+bool conv3x3_packed_serves_op(int64_t co, int64_t ci) {
+  size_t bytes = 0;
+  return catchq_packed_conv3x3_size(co, ci, &bytes) == CATCHQ_OK && catchq::conv3x3_a16_packed_filters(co, ci);
+}
+
 // qw [Co,3,3,Ci] int8 in the order that catchq_conv3x3_packed reads
 Tensor pack_conv3x3_op(const Tensor &qw) {
   TORCH_CHECK(qw.dim() == 4 && qw.is_contiguous() && qw.scalar_type() == at::kChar && qw.size(1) == 3 && qw.size(2) == 3,
@@ -1684,6 +1690,7 @@ TORCH_LIBRARY(torch_mlu, m) {
   m.def("inverted_residual_fuses(int n, int h, int w, int ci, int hid, int co, int stride) -> bool", &irb_fuses_op);
   m.def("first_layers_fuse(int n, int c, int h, int w, int co, int k, int stride, int pad, int pool_k, int pool_stride, "
         "int pool_pad) -> bool", &first_layers_fuse_op);
+  m.def("conv3x3_packed_serves(int co, int ci) -> bool", &conv3x3_packed_serves_op);
   m.def("conv1x1_avgpool_fuses(int n, int hw, int ci, int co) -> bool", &conv_avgpool_fuses_op);
   m.def("clear_weight_cache() -> ()", &clear_cache_op);
   m.def("weight_cache_size() -> int", &cache_size_op);

@@ -162,8 +162,8 @@ def _decode(layer, sd, device, ci_dev, co_dev, fractional=False):
     q.qw = qw.contiguous()
     q.packed = None
     if ((layer.kind, layer.k, layer.stride, layer.pad, q.groups, q.bw_x, q.bw_w) == ("conv", 3, 1, 1, 1, 16, 8)
-            and ci_dev % 64 == 0 and q.qw.numel() < 1 << 30):  # (larger filters have no packed form)
-        q.packed = torch.ops.torch_mlu.pack_conv3x3(q.qw)  # (read by the launches that the kernel on packed filters serves)
+            and torch.ops.torch_mlu.conv3x3_packed_serves(q.qw.shape[0], ci_dev)):
+        q.packed = torch.ops.torch_mlu.pack_conv3x3(q.qw)  # (the calls of a few blocks, or wide images, read the filters as they are)
     return q
 
 

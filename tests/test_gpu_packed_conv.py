@@ -146,3 +146,14 @@ def test_filters_are_held_twice_where_they_are_read(n, ci, h, w, co, packs):
         torch.cuda.synchronize()
         held.append(torch.cuda.memory_allocated())
     assert held[2] == held[1] and (held[1] - held[0] >= co * ci * 9) == packs and (held[1] == held[0]) == (not packs)
+
+
+def test_plans_hold_packed_filters_that_are_read():
+    """a detector's 3 x 3 layers of 128 output channels, which the walking kernel serves at every size, are not held twice"""
+    from catch_amd import nets, pipeline
+    layers = nets.darknet53_yolov3()
+    net = nets.FloatNet(layers, seed=3, weight_std="he").eval()
+    sd = pipeline.calibrate(net, torch.rand(1, 3, 64, 64, generator=torch.Generator().manual_seed(5)), "int16", False)
+    fused = pipeline.FusedNet(layers, pipeline.to_position_encoding(sd, 16, 8))
+    packed = set((l.ci, l.co) for l in layers if l.kind == "conv" and fused.q[l.name].packed is not None)
+    assert packed == {(128, 256), (256, 512), (512, 1024)}

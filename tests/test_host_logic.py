@@ -488,3 +488,12 @@ def test_concatenations_beyond_one_launch():
     env = {("a",) + form: meta(63, 2048, 2048, 16), ("b",) + form: meta(63, 4096, 4096, 16)}
     with pytest.raises(NotImplementedError):  # one launch, which tensors without memory do not have
         plan._concat(cat, form, env)
+
+
+def test_plans_pack_filters_that_a_launch_can_read():
+    """by the channels alone: a multiple of 64 in, a multiple of 4 out that fills three quarters of whole blocks of 256; below 2 GiB
+    packed, which few output channels (rounded up to 32) reach before the filters themselves do"""
+    serves = torch.ops.torch_mlu.conv3x3_packed_serves
+    assert [co for co in (4, 64, 128, 188, 192, 194, 256, 320, 380, 384, 512, 572, 576, 1024) if serves(co, 64)] == [192, 256, 384, 512, 576, 1024]
+    assert not serves(256, 96) and not serves(256, 0) and not serves(0, 64)
+    assert serves(256, 64 * 14500) and not serves(256, 64 * 14600) and not serves(8, 1 << 23)
