@@ -140,11 +140,19 @@ static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, const EpiDev 
   // filters, from as many of those on (8 x 25 x 25, 160 -> 320, 158, 13.3 / 12.6 with 64; 8 x 28 x 28, 192, 98, 11.5 / 13.4).
   // 96 and 128 pixels a block gain nothing more.
   const int64_t columns = (groups + 7) / 8;
-  auto fits = [&](int tm) { return (int64_t)(tm * 32 + 2 * W + 2) * (Ci + 16) + Ci <= 80 * 1024; };  // two blocks a unit
+  auto patch = [&](int tm) { return (int64_t)(tm * 32 + 2 * W + 2) * (Ci + 16) + Ci; };
+  auto fits = [&](int tm) { return patch(tm) <= 80 * 1024; };  // two blocks a unit
   auto blocks = [&](int tm) { return (M + tm * 32 - 1) / (tm * 32) * columns; };
+  // Up to 64 channels leave a block one wave or two: more than a round of blocks, and four (three) of them to a unit, have to hide
+  // what it waits for (with the quantizer: 6 x 28 x 28, 384 -> 16, 74 blocks, 9.1 / 13.4, 64 x 14 x 14, 192 -> 32, 196, 9.4 / 12.2, 64
+  // 11.2 / 12.3; 32 x 28 x 28, 96 -> 32, 392, 11.8 / 10.9, 64 12.5 / 11.8; but 60 x 60, 384 -> 16, 562 of 75 KB, a quarter slower).
+  if (groups <= 2) return blocks(2) * 8 >= 9 * (int64_t)e.cus && patch(2) <= (groups == 1 ? 40 : 52) * 1024 ? 2 : 0;
   if (blocks(1) * 2 < e.cus) return 0;
-  if (blocks(2) * 2 >= e.cus && fits(2)) return 2;
-  return fits(1) ? 1 : 0;
+  if (blocks(2) * 2 < e.cus) return fits(1) ? 1 : 0;
+  if (fits(2)) return 2;
+  // where only blocks of 32 fit, the wider tiles of many columns are ahead (with the quantizer: 5 x 57 x 75, 384 -> 192 46.7 / 39.8,
+  // 512 65.4 / 80.0; 8 x 56 x 56, 480 -> 192 62.3 / 55.0, 256 66.9 / 68.7, 512 84.9 / 109.8)
+  return fits(1) && groups < 8 ? 1 : 0;
 }
 
 bool conv3x3_i8_packed_takes(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e) { return packed_i8_plan(N, H, W, Ci, Co, e) != 0; }

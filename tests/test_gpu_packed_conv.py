@@ -1,8 +1,11 @@
 """torch_mlu::qconv2d on filters laid out by pack_conv3x3: the same bits as on the filters as they are, and which calls read them."""
+import ctypes
+
 import pytest
 import torch
 
 import catch_amd  # noqa: F401  (registers torch_mlu::*)
+from catch_amd import _native
 
 pytestmark = pytest.mark.gpu
 
@@ -96,13 +99,19 @@ def test_packed_conv3x3_other_calls():
 
 # edges of blocks of 32 and of 64 pixels and of images, one wave to eight and two blocks of them side by side; sharing makes the rule plan
 # for 256 / sharing units
-@pytest.mark.parametrize("n,ci,h,w,co,mode,dtype,nhwc,sharing", [
-    (1, 96, 1, 1, 4, 1, torch.float32, False, 256), (1, 96, 5, 13, 36, 3, torch.float32, False, 256), (3, 160, 7, 9, 100, 3, torch.float16, True, 256),
-    (1, 96, 3, 33, 256, 3, torch.float32, True, 64), (2, 192, 1, 50, 260, 3, torch.float32, False, 64), (5, 224, 6, 7, 512, 1, torch.float32, True, 64),
-    (2, 320, 9, 1, 64, 3, torch.float16, False, 256), (1, 96, 2, 300, 32, 3, torch.float32, False, 64), (2, 96, 57, 75, 160, 3, torch.float32, False, 1),
-    (1, 96, 9, 9, 30, 3, torch.float32, False, 256), (1, 128, 9, 9, 64, 3, torch.float32, False, 256), (1, 96, 9, 9, 64, 3, torch.float32, False, 1),
+@pytest.mark.parametrize("n,ci,h,w,co,mode,dtype,nhwc,sharing,taken", [
+    (1, 96, 1, 1, 4, 1, torch.float32, False, 256, False), (1, 96, 5, 13, 36, 3, torch.float32, False, 256, True),
+    (3, 160, 7, 9, 100, 3, torch.float16, True, 256, True), (1, 96, 3, 33, 256, 3, torch.float32, True, 64, True),
+    (2, 192, 1, 50, 260, 3, torch.float32, False, 64, True), (5, 224, 6, 7, 512, 1, torch.float32, True, 64, True),
+    (2, 320, 9, 1, 64, 3, torch.float16, False, 256, False), (1, 96, 2, 300, 32, 3, torch.float32, False, 64, False),
+    (2, 96, 57, 75, 160, 3, torch.float32, False, 1, True), (1, 96, 9, 9, 30, 3, torch.float32, False, 256, False),
+    (1, 128, 9, 9, 64, 3, torch.float32, False, 256, False), (1, 96, 9, 9, 64, 3, torch.float32, False, 1, False),
+    (1, 96, 9, 8, 4, 1, torch.float32, False, 256, True), (2, 320, 37, 1, 64, 3, torch.float16, False, 256, True),
+    (1, 96, 2, 140, 32, 3, torch.float32, False, 64, True), (1, 160, 1, 1, 68, 1, torch.float32, False, 256, True),
+    (2, 96, 5, 33, 196, 3, torch.float16, False, 256, True), (1, 480, 3, 60, 164, 3, torch.float32, False, 256, True),
+    (1, 480, 3, 60, 228, 3, torch.float32, False, 256, False),
 ])
-def test_packed_conv3x3_int8(n, ci, h, w, co, mode, dtype, nhwc, sharing):
+def test_packed_conv3x3_int8(n, ci, h, w, co, mode, dtype, nhwc, sharing, taken):
     """the first call of a weight goes without packed filters, later ones read them: the same bits, equal to the oracle's"""
     from oracle import ops as oops
     gen = torch.Generator().manual_seed(ci + h * w)
@@ -115,6 +124,8 @@ def test_packed_conv3x3_int8(n, ci, h, w, co, mode, dtype, nhwc, sharing):
     mode = torch.tensor([mode], dtype=torch.int32)
     xd = x.cuda().contiguous(memory_format=torch.channels_last) if nhwc else x.cuda()
     args = (xd, wt.cuda(), b.cuda(), [1, 1], [1, 1], [1, 1], 1, scale.cuda(), mode.cuda())
+    e = _native.Epilogue(y=16, sharing=sharing)
+    assert (_native.kernel_lib().catchq_conv3x3_i8_packed_takes(n, h, w, ci, co, ctypes.byref(e)) == 0) == taken
     torch.ops.torch_mlu.set_launch_sharing(sharing)
     try:
         first, second, third = [torch.ops.torch_mlu.conv2d(*args) for _ in range(3)]

@@ -471,6 +471,13 @@ def test_packed_conv3x3_refusals(lib):
                             (1, 57, 600, 96, 160), (1, 1 << 20, 8, 96, 160), (64, 1000, 400, 96, 32), (1 << 20, 64, 64, 96, 32)]:
         assert takes(n, h, w, ci, co) == UNSUPPORTED, (n, h, w, ci, co)
     assert takes(5, 0, 75, 96, 160) == ARG
+    # a wave or two a block: more than a round of blocks, small patches
+    for n, h, w, ci, co, want in [(6, 28, 28, 384, 16, False), (64, 14, 14, 192, 64, False), (64, 14, 14, 192, 68, True), (32, 28, 28, 96, 32, True),
+                                  (32, 28, 28, 96, 64, True), (10, 60, 60, 384, 64, False), (40, 23, 23, 320, 32, True), (40, 23, 23, 480, 32, False),
+                                  (40, 23, 23, 352, 64, True),
+                                  # only blocks of 32 pixels fit twice into a unit
+                                  (8, 56, 56, 480, 192, True), (8, 56, 56, 480, 224, True), (8, 56, 56, 480, 228, False), (8, 56, 56, 480, 512, False)]:
+        assert (takes(n, h, w, ci, co) == OK) == want, (n, h, w, ci, co)
     e.sharing = 4  # a quarter of the units: fewer blocks will do
     assert takes(1, 28, 28, 192, 192) == UNSUPPORTED and takes(2, 28, 28, 192, 192) == OK
 
