@@ -211,6 +211,7 @@ static int launch_packed(const void *x, const void *w, const PackedConvParams &p
     case EPI_LK_Y_Q16: return launch_packed_epi<TM, NIT, EPI_LK_Y_Q16>(x, w, p, e, s);
     case EPI_LK_RESA_Q16: return launch_packed_epi<TM, NIT, EPI_LK_RESA_Q16>(x, w, p, e, s);
     case EPI_LK_RESA_Y_Q16: return launch_packed_epi<TM, NIT, EPI_LK_RESA_Y_Q16>(x, w, p, e, s);
+    case EPI_Y16: return launch_packed_epi<TM, NIT, EPI_Y16>(x, w, p, e, s);
     case EPI_SCALAR: return -1;
     default: return launch_packed_epi<TM, NIT, EPI_VECTOR>(x, w, p, e, s);
   }
@@ -219,11 +220,20 @@ static int launch_packed(const void *x, const void *w, const PackedConvParams &p
 // Where the blocks of 32 pixels leave most units without one, the waves that split K (ksplit.hip) are ahead: 5 x 13 x 13, 512 ->
 // 1024 (108 blocks for 256 units; the whole network 1000 / 1045 us), 2 x 13 x 13 (44) 9.8 / 16.9, 2 x 26 x 26 (86) 10.8 / 10.6;
 // 4 x 26 x 26 (170) 15.5 / 11.3.
+// Columns that do not exist cost as much as others.  Beyond an eighth of them, epilogues without an instance of their own are behind
+// (us, that kernel / this, to int16 behind a ReLU: 8 x 52 x 52, 128 -> 192 24.7 / 28.3, 16 x 26 x 26, 256 -> 384 37.9 / 39.7; of 224
+// columns 2 x 52 x 52, 64 10.7 / 11.5), and so are the others' single rounds of blocks with long K (2 x 52 x 52, 512 -> 192, 169
+// blocks of 32, 18.0 / 19.7; 4 x 52 x 52, 338, 34.1 / 32.8) and wide images (4 x 80 x 80, 192 -> 384 50.2 / 52.0).
 bool conv3x3_a16_packed_takes(int N, int H, int W, int Ci, int Co, const EpiDev &e) {
   const int64_t M = (int64_t)N * H * W, columns = ((int64_t)Co + 255) / 256 * 256;
   if (!conv3x3_a16_packed_filters(Co, Ci) || M * Ci * 2 >= (1ll << 31) || columns / 32 * Ci * 288 >= (1ll << 31) - (1 << 20)) return false;
-  if (W > 95 || H >= (1 << 20) || pick_epilogue(Co, e) == EPI_SCALAR) return false;
-  return (M + 31) / 32 * (columns / 256) * 8 >= 5 * (int64_t)e.cus;
+  const int epi = pick_epilogue(Co, e);
+  if (W > 95 || H >= (1 << 20) || epi == EPI_SCALAR) return false;
+  const int64_t blocks = (M + 31) / 32 * (columns / 256);
+  if (blocks * 8 < 5 * (int64_t)e.cus) return false;
+  const bool own = epi == EPI_LK_Q16 || epi == EPI_LK_Y_Q16 || epi == EPI_LK_RESA_Q16 || epi == EPI_LK_RESA_Y_Q16 || epi == EPI_Y16;
+  if (!own) return Co * 16ll >= columns * 15;
+  return Co * 8ll >= columns * 7 || ((Ci < 256 || blocks * 4 >= 5 * (int64_t)e.cus) && (W <= 63 || Co < 256));
 }
 
 int64_t packed3x3_filter_bytes(int64_t Co, int64_t Ci) { return (Co + 31) / 32 * Ci * 288; }

@@ -25,15 +25,22 @@ def _outputs(out):
 
 
 # sharing makes the rules plan for 256 / sharing units: small layers take the blocks of 32 and of 64 pixels.  Widths: either side of
-# what one more pass over the patch takes; 96 is beyond the last.
+# what one more pass over the patch takes; 96 is beyond the last.  OWN: where more than a sixteenth of a block's columns do not exist,
+# only the epilogues with an instance of their own.
+OWN = "own"
+
+
 @pytest.mark.parametrize("n,h,w,ci,co,sharing,taken", [
-    (1, 1, 1, 64, 256, 256, True), (2, 1, 31, 64, 192, 256, True), (1, 9, 32, 64, 256, 256, True),
-    (3, 5, 63, 128, 256, 256, True), (1, 3, 64, 64, 252, 256, True), (1, 4, 95, 64, 448, 256, True),
+    (1, 1, 1, 64, 256, 256, True), (2, 1, 31, 64, 192, 256, OWN), (1, 9, 32, 64, 256, 256, True),
+    (3, 5, 63, 128, 256, 256, True), (1, 3, 64, 64, 252, 256, True), (1, 4, 95, 64, 448, 256, OWN),
     (1, 4, 96, 64, 256, 256, False), (5, 13, 13, 192, 512, 256, True), (2, 8, 1, 64, 256, 256, True),
     # blocks of 32 pixels
     (1, 10, 15, 64, 256, 40, True), (1, 10, 16, 128, 256, 40, True), (1, 4, 47, 64, 256, 36, True),
     (2, 2, 48, 64, 256, 36, True), (1, 2, 79, 192, 256, 42, True), (1, 2, 80, 64, 260, 42, False),
     (1, 2, 95, 64, 256, 36, True), (7, 5, 5, 64, 256, 42, True),
+    # a quarter of the columns missing: a round of blocks with long K, wide images of several columns
+    (1, 3, 31, 192, 192, 64, OWN), (1, 3, 31, 256, 192, 64, False), (1, 4, 31, 256, 192, 85, OWN), (1, 2, 63, 64, 384, 256, OWN),
+    (1, 2, 64, 64, 384, 256, False), (1, 2, 64, 64, 192, 256, OWN), (1, 4, 15, 64, 240, 256, True), (1, 4, 15, 64, 236, 256, OWN),
     # too few blocks, channels or multiples
     (1, 13, 13, 128, 256, 1, False), (4, 13, 13, 64, 128, 256, False), (4, 13, 13, 64, 320, 256, False),
 ])
@@ -47,14 +54,17 @@ def test_packed_conv3x3(n, h, w, ci, co, sharing, taken):
     resid = torch.randn(n, h, w, co, generator=gen).cuda()
     div = (torch.rand(co, generator=gen) + 0.5).cuda()
     geometry = ([1, 1], [1, 1], [1, 1], 1)
+    # the first five have an instance of their own
     calls = [  # chan_div, resid, act, want_y, y_half, want_acc, q_bitwidth, q_position, q_scale, slope, resid_after
         (None, None, 3, False, False, False, 16, -8, 1.0, 0.1, False), (None, resid, 3, True, False, False, 16, -8, 1.0, 0.1, True),
         (None, resid, 3, False, False, False, 16, -8, 1.0, 0.1, True), (None, None, 3, True, False, False, 16, -8, 1.0, 0.1, False),
+        (None, None, 0, True, True, False, 0, 0, 1.0, 0.0, False),
         (None, None, 0, True, True, True, 0, 0, 1.0, 0.0, False), (div, resid, 1, True, False, True, 8, -2, 1.3, 0.0, False)]
-    packed, read = ops.pack_conv3x3(other), other if taken else qw
+    packed = ops.pack_conv3x3(other)
     ops.set_launch_sharing(sharing)
     try:
-        for d, r, act, *rest in calls:
+        for i, (d, r, act, *rest) in enumerate(calls):
+            read = other if taken is True or taken == OWN and i < 5 else qw
             got = ops.qconv2d(x, qw, -12, d, bias, r, *geometry, act, *rest, packed)
             want = ops.qconv2d(x, read, -12, d, bias, r, *geometry, act, *rest)
             assert len(_outputs(got)) == len(_outputs(want)) > 0
