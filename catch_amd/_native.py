@@ -130,6 +130,7 @@ SIGNATURES = {
     "catchq_conv1x1_avgpool_nhwc": (_I, [_P, _P, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P, _P, _I, _I, ctypes.c_float,
                                          _P, _SZ, _P]),
     "catchq_conv2d_route": (ctypes.c_char_p, [_I, _I, ctypes.POINTER(ConvDesc)]),
+    "catchq_conv2d_kernel": (ctypes.c_char_p, [_I, _I, ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue)]),
     "catchq_gemm_route": (ctypes.c_char_p, [_I, _I, _I64, _I64, _I64]),
     "catchq_diag_mfma_i8_loop": (_I, [_P, _I, _I, _P, _P]),
 }

@@ -19,6 +19,9 @@ typedef int v2i __attribute__((ext_vector_type(2)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
+// kernels that serve some convolutions ahead of their family's general ones (catchq_conv2d_kernel)
+enum ConvKernel { kConvGeneral, kConvWalk };
+
 inline hipStream_t as_stream(catchq_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 
 inline int launch_status() { return hipGetLastError() == hipSuccess ? CATCHQ_OK : CATCHQ_ERR_LAUNCH; }

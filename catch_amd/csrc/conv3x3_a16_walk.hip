@@ -2,17 +2,21 @@
 // the layers in front of a detector, where images are large and channels few.
 //
 // What bounds them is HBM -- 32 channels of 16 images of 416 x 416 to 64 at stride 2, with fp32 and int16 outputs, are 443 MB for
-// 51 TOP -- and the kernel of the other layers (igemm_a16_dma.hip) is far from it: five K steps of a 64 x 64 tile leave each
+// 51 GOP -- and the kernel of the other layers (igemm_a16_dma.hip) is far from it: five K steps of a 64 x 64 tile leave each
 // block a chain of one start-up, five operand deliveries and one epilogue.  Here a wave keeps its filters in registers (9 taps x
 // 32 columns: 36 of them, 72 with 64 channels) and a block walks over tiles of 64 (32) output pixels: the next tile's patch is on
 // its way while this one's is multiplied.  What fills HBM is the number of tiles on their way at once, so everything is small: one
 // set of accumulators (the high digits' sums are shifted up before the low digits are added), 128 registers and 27 KB for four
-// blocks a unit of 32 channels at stride 1, three otherwise.  The digits and the constant are those of igemm_a16_dma.hip; a patch
-// is split into digits once, on its way into LDS, and pixels outside the image arrive as zeros.
+// blocks a unit of 32 channels at stride 1, three otherwise, two of 64 channels at stride 2 behind a generic epilogue (182 registers;
+// as many blocks are started as fit: with three started for places of two 2 x 208 x 208, 64 -> 128 took 17.1, now 14.2, 15.0 before
+// this kernel).  Stride 2 of 32 channels would fit four (128 registers, 40 KB; not tried).  The digits and the constant are those of
+// igemm_a16_dma.hip; a patch is split into digits once, on its way into LDS, and pixels outside the image arrive as zeros.
 // us, before / now / at 6 TB/s, 16 images: 32 channels, 416 x 416 at stride 2 126 / 83 / 74, 208 x 208 with a residual 123 / 58 / 52;
 // 64 channels, 208 x 208 at stride 2 58 / 44 / 37, 104 x 104 with a residual and fp32 output 71 / 48 / 41, to int16 only 55 / 37 / 11.
-// One image: 13.2 / 10.6, 11.7 / 9.1, 9.9 / 9.9, 10.1 / 9.7.  With tiles of 16 x 8, 64 columns a wave and both digits' sums at once
-// (two blocks a unit) the first two were 91 and 113.
+// One image: 13.2 / 10.6, 11.7 / 9.1, 9.9 / 9.9, 10.1 / 9.7.  To halfs only, which the tiled kernel has an instance for as well:
+// 2 x 208 x 208, 64 -> 128 35.4 / 22.3, at stride 2 12.3 / 12.7, 6 x 190 x 190 at stride 2 24.2 / 20.0; with the generic epilogue 28.6,
+// 16.9 and 29.9.  With tiles of 16 x 8, 64 columns a wave and both digits' sums at once (two blocks a unit) the first two of 16
+// images were 91 and 113.
 #include "conv3x3_halo.h"
 
 namespace catchq {
@@ -23,9 +27,14 @@ struct WalkParams {
   unsigned x_bytes;
 };
 
+// Blocks of a unit: what an instance's registers are bounded for and what its launch starts
 template <int CI, int S, int EPI>
-__global__ __launch_bounds__(256, CI == 32 && S == 1 && EPI != EPI_VECTOR ? 4 : (CI == 64 && S == 2 && EPI == EPI_VECTOR ? 2 : 3)) void conv3x3_a16_walk_kernel(const int16_t *__restrict__ X, const int8_t *__restrict__ B,
-                                                                 WalkParams p, EpiDev e) {
+constexpr int walk_blocks() { return CI == 32 && S == 1 ? 4 : (CI == 64 && S == 2 && EPI == EPI_VECTOR ? 2 : 3); }
+
+template <int CI, int S, int EPI>
+__global__ __launch_bounds__(256, (walk_blocks<CI, S, EPI>())) void conv3x3_a16_walk_kernel(const int16_t *__restrict__ X,
+                                                                                          const int8_t *__restrict__ B,
+                                                                                          WalkParams p, EpiDev e) {
   resolve_exp2(e);
   typedef typename EpiOf<EPI>::type Spec;
   constexpr int CG = CI == 32 ? 2 : 4;  // waves side by side on a tile, 32 columns each; 4 / CG runs of 32 pixels
@@ -161,44 +170,56 @@ __global__ __launch_bounds__(256, CI == 32 && S == 1 && EPI != EPI_VECTOR ? 4 : 
 
 template <int CI, int S>
 static int launch_walk(const void *x, const void *w, const WalkParams &p, const EpiDev &e, hipStream_t s) {
-  const int most = 256 * (CI == 32 && S == 1 ? 4 : 3), blocks = p.ntiles < most ? p.ntiles : most;
 #define CATCHQ_WALK(EPI_)                                                                                             \
-  case EPI_:                                                                                                          \
+  case EPI_: {                                                                                                        \
+    const int most = 256 * walk_blocks<CI, S, EPI_>(), blocks = p.ntiles < most ? p.ntiles : most;                    \
     conv3x3_a16_walk_kernel<CI, S, EPI_><<<blocks, 256, 0, s>>>((const int16_t *)x, (const int8_t *)w, p, e);         \
-    return launch_status()
-  switch (pick_epilogue(p.g.N, e)) {
-    CATCHQ_WALK(EPI_LK_Q16);
-    CATCHQ_WALK(EPI_LK_Y_Q16);
-    case EPI_SCALAR: return -1;
-    default: break;
+    return launch_status();                                                                                           \
   }
+  const int epi = pick_epilogue(p.g.N, e);
   if constexpr (S == 1) {  // (a residual branch has its block's size)
-    switch (pick_epilogue(p.g.N, e)) {
-      CATCHQ_WALK(EPI_LK_RESA_Q16);
-      CATCHQ_WALK(EPI_LK_RESA_Y_Q16);
+    switch (epi) {
+      CATCHQ_WALK(EPI_LK_RESA_Q16)
+      CATCHQ_WALK(EPI_LK_RESA_Y_Q16)
       default: break;
     }
   }
-  conv3x3_a16_walk_kernel<CI, S, EPI_VECTOR><<<blocks, 256, 0, s>>>((const int16_t *)x, (const int8_t *)w, p, e);
-  return launch_status();
+  switch (epi) {
+    CATCHQ_WALK(EPI_LK_Q16)
+    CATCHQ_WALK(EPI_LK_Y_Q16)
+    CATCHQ_WALK(EPI_Y32)
+    CATCHQ_WALK(EPI_Y16)
+    default:
+    CATCHQ_WALK(EPI_VECTOR)
+  }
 #undef CATCHQ_WALK
 }
 
-// x [N, H, W, Ci] int16, w [Co, 3, 3, Ci], Ci 32 or 64; -1: not this kernel's shape
-int conv3x3_a16_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
-                     hipStream_t s) {
-  const int tw = Ci == 32 ? 16 : 8;
+static int walk_tile_columns(int Ci) { return Ci == 32 ? 16 : 8; }
+
+// 3 x 3, padding 1
+bool conv3x3_a16_walk_takes(int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e) {
+  const int tw = walk_tile_columns(Ci);
   const int64_t tiles_x = (Wo + tw - 1) / tw, tiles_y = (Ho + 3) / 4, tiles = N * tiles_x * tiles_y;
-  if ((Ci != 32 && Ci != 64) || Co <= Ci || Co > 2 * Ci || (stride != 1 && stride != 2)) return -1;
+  if ((Ci != 32 && Ci != 64) || Co <= Ci || Co > 2 * Ci || (stride != 1 && stride != 2)) return false;
   if ((int64_t)N * H * W * Ci * 2 >= (1ll << 31) || tiles >= (1 << 30) || (int64_t)Wo * Co >= (1 << 28) || (int64_t)N * Ho * Wo >= (1ll << 31))
-    return -1;
+    return false;
   // 64 channels on a few tiles: what reads the filters as it needs them is ahead (us, this / that: 26 x 26, 28 tiles, 6.1 / 5.0,
   // 64 x 64, 128 tiles, 6.0 / 5.9; 2 x 64 x 64, 256, 6.0 / 8.6); 32 channels are ahead from one tile on (4 x 7 x 7 4.6 / 7.6)
-  if (Ci == 64 && tiles * 4 < 3 * (int64_t)e.cus) return -1;
+  // At stride 2 more columns ask for more of them (128 columns, two outputs: 208 x 208, 338 tiles, 9.7 / 10.0, 2 x 208 x 208, 676, 14.0 /
+  // 13.5; 96 columns, 338 tiles, 9.6 / 9.3).
+  if (Ci == 64 && (tiles * 4 < 3 * (int64_t)e.cus || (stride == 2 && Co > 96 && tiles < 2 * (int64_t)e.cus))) return false;
+  return pick_epilogue(Co, e) != EPI_SCALAR;
+}
+
+// x [N, H, W, Ci] int16, w [Co, 3, 3, Ci], a call that conv3x3_a16_walk_takes
+int conv3x3_a16_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
+                     hipStream_t s) {
+  const int tw = walk_tile_columns(Ci), tiles_x = (Wo + tw - 1) / tw, tiles_y = (Ho + 3) / 4;
   WalkParams p = {};
   p.g.M = (int64_t)N * Ho * Wo;
   p.g.N = Co; p.g.K = 9 * Ci; p.g.H = H; p.g.W = W; p.g.Ci = Ci; p.g.Ho = Ho; p.g.Wo = Wo;
-  p.tiles_x = (int)tiles_x; p.tiles_y = (int)tiles_y; p.ntiles = (int)tiles;
+  p.tiles_x = tiles_x; p.tiles_y = tiles_y; p.ntiles = N * tiles_x * tiles_y;
   p.x_bytes = (unsigned)((int64_t)N * H * W * Ci * 2);
   if (Ci == 32) return stride == 1 ? launch_walk<32, 1>(x, w, p, e, s) : launch_walk<32, 2>(x, w, p, e, s);
   return stride == 1 ? launch_walk<64, 1>(x, w, p, e, s) : launch_walk<64, 2>(x, w, p, e, s);

@@ -417,6 +417,7 @@ int igemm_a16_launch(int load, const void *a, const void *b, IgemmParams p, cons
   return -1;
 }
 
+bool conv3x3_a16_walk_takes(int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e);
 int conv3x3_a16_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
                      hipStream_t s);
 int pw_a16_short(const void *x, const void *w, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s);
@@ -542,6 +543,13 @@ static int conv2d_stem_a16(const void *x, const void *w, int N, int H, int W, in
   return launch_status();
 }
 
+ConvKernel conv2d_a16_kernel(int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho,
+                             int Wo, const EpiDev &e) {
+  if (kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1 && conv3x3_a16_walk_takes(N, H, W, Ci, Co, sh, Ho, Wo, e))
+    return kConvWalk;
+  return kConvGeneral;
+}
+
 int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                     int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
   IgemmParams p = {};
@@ -550,10 +558,8 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo;
   p.kh = kh; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
   p.K = kh * kw * Ci;
-  if ((Ci == 32 || Ci == 64) && kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1) {  // walks over tiles
-    const int st = conv3x3_a16_walk(x, w, N, H, W, Ci, Co, sh, Ho, Wo, e, s);
-    if (st >= 0) return st;
-  }
+  const ConvKernel kernel = conv2d_a16_kernel(N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, e);
+  if (kernel == kConvWalk) return conv3x3_a16_walk(x, w, N, H, W, Ci, Co, sh, Ho, Wo, e, s);
   if (Ci % 16 == 0) {  // a few blocks per unit, long K
     const int st = contract_ksplit(x, true, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false, e, s);
     if (st >= 0) return st;

@@ -1,22 +1,32 @@
 """3 x 3 convolutions of 32 and 64 int16 channels (the kernel that walks over small tiles of the outputs) against
 64-bit sums and the epilogue's operations in fp32."""
+import ctypes
+
 import pytest
 import torch
 
 import catch_amd  # noqa: F401  (registers torch_mlu::*)
+from catch_amd import _native
 
 pytestmark = pytest.mark.gpu
 
 
+def _kernel(bits, n, h, w, ci, co, ksize, stride, sharing=1):
+    """which kernel serves the calls of a layer that these tests make"""
+    d = _native.ConvDesc(n, h, w, ci, co, ksize, ksize, ksize // 2, ksize // 2, stride, stride, 1, 1, 1)
+    e = _native.Epilogue(y=16, sharing=sharing)
+    return _native.kernel_lib().catchq_conv2d_kernel(bits, 8, ctypes.byref(d), ctypes.byref(e)).decode()
+
+
 # edges of tiles either way, images smaller than one, more tiles than blocks, channels that end inside a wave's or are one wave's less
-@pytest.mark.parametrize("n,h,w,ci,co,stride", [
+@pytest.mark.parametrize("n,h,w,ci,co,stride,kernel", [row + ("walk",) for row in [
     (1, 1, 1, 32, 64, 1), (1, 1, 1, 32, 64, 2), (2, 4, 16, 32, 64, 1), (1, 5, 17, 32, 36, 1), (3, 7, 33, 32, 64, 2), (1, 8, 32, 32, 60, 2),
     (2, 9, 15, 32, 48, 2), (1, 3, 50, 32, 64, 1), (4, 66, 130, 32, 64, 1), (5, 129, 131, 32, 64, 2),
-    (3, 33, 60, 64, 128, 1), (13, 7, 62, 64, 68, 1), (2, 67, 130, 64, 128, 2), (3, 129, 66, 64, 100, 2),
-    (200, 3, 3, 64, 96, 1), (200, 4, 8, 64, 128, 2),
-    (1, 6, 6, 32, 32, 1), (1, 6, 6, 32, 68, 1),  # not this kernel's
-])
-def test_conv_walk(n, h, w, ci, co, stride):
+    (3, 33, 60, 64, 128, 1), (13, 7, 62, 64, 68, 1), (200, 3, 3, 64, 96, 1),
+    (3, 129, 66, 64, 96, 2), (4, 130, 131, 64, 128, 2), (520, 4, 8, 64, 128, 2), (520, 5, 7, 64, 100, 2)]] + [row + ("general",) for row in [
+    (2, 67, 130, 64, 128, 2), (3, 129, 66, 64, 100, 2), (200, 4, 8, 64, 128, 2), (1, 6, 6, 32, 32, 1), (1, 6, 6, 32, 68, 1)]])
+def test_conv_walk(n, h, w, ci, co, stride, kernel):
+    assert _kernel(16, n, h, w, ci, co, 3, stride) == kernel
     gen = torch.Generator().manual_seed(h * w + co)
     x = torch.randint(-32768, 32768, (n, h, w, ci), generator=gen).short()
     x.view(-1)[:2] = torch.tensor([-32768, 32767])
@@ -41,6 +51,7 @@ def test_conv_walk(n, h, w, ci, co, stride):
         y, q, _ = run(r, 3, want_y, False, False, 16, -7, 1.0, 0.1, True)
         assert torch.equal(q.cpu().int(), torch.clamp(torch.round(want * 128), -32768, 32767).int())
         assert not want_y or torch.equal(y.cpu(), want)
+    assert torch.equal(run(None, 0, True)[0].cpu(), v) and torch.equal(run(None, 0, True, True)[0].cpu(), v.half())
     y, q, _ = run(rd, 1, True, True, False, 8, -2, 1.3, 0.0, False)
     want = torch.relu(v + resid)
     assert torch.equal(y.cpu(), want.half())

@@ -133,6 +133,7 @@ def test_routes(lib):
     assert route(8, 32, 3, 1, (16, 8)) == "mfma_a16"
     assert route(4, 32, 3, 1, (16, 8)) == "direct"
     assert route(64, 64, 30, 1) == "invalid"  # kernel larger than the image
+    assert lib.catchq_conv2d_kernel(16, 8, ctypes.byref(ConvDesc(1, 16, 16, 32, 64, 3, 3, 1, 1, 1, 1, 1, 1, 1)), None) == b"invalid"
     assert lib.catchq_gemm_route(8, 8, 4096, 3072, 768) == b"mfma"
     assert lib.catchq_gemm_route(8, 8, 10, 25, 10) == b"direct"
     assert lib.catchq_gemm_route(16, 8, 4096, 3072, 768) == b"mfma_a16"
@@ -504,3 +505,15 @@ def test_plans_pack_filters_that_a_launch_can_read():
     assert [co for co in (4, 64, 128, 188, 192, 194, 256, 320, 380, 384, 512, 572, 576, 1024) if serves(co, 64)] == [192, 256, 384, 512, 576, 1024]
     assert not serves(256, 96) and not serves(256, 0) and not serves(0, 64)
     assert serves(256, 64 * 14500) and not serves(256, 64 * 14600) and not serves(8, 1 << 23)
+
+
+def test_int16_layers_of_64_channels_at_stride_2(lib):
+    """128 columns ask for two tiles of 8 x 4 outputs a unit; up to 96, and stride 1, for three quarters of one"""
+    from catch_amd import _native
+
+    def kernel(n, side, co, stride, **k):
+        d = _native.ConvDesc(n, side, side, 64, co, 3, 3, 1, 1, stride, stride, 1, 1, 1)
+        return lib.catchq_conv2d_kernel(16, 8, ctypes.byref(d), ctypes.byref(_native.Epilogue(y=16, **k))).decode()
+    assert kernel(1, 208, 128, 2) == kernel(1, 208, 100, 2) == "general"
+    assert kernel(1, 208, 96, 2) == kernel(2, 208, 128, 2) == kernel(1, 208, 128, 2, sharing=2) == kernel(1, 104, 128, 1) == "walk"
+    assert kernel(1, 48, 128, 1) == kernel(2, 208, 130, 2) == "general"  # few tiles, rows of no whole groups of four
