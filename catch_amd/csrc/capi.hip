@@ -19,6 +19,8 @@ int gemm_nt_mfma_a16(const void *a, const void *b, int64_t M, int64_t N, int64_t
 int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                     int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
 int gemm_nt_mfma_a16w16(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s);
+ConvKernel conv2d_i8_kernel(int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho,
+                            int Wo, const EpiDev &e);
 ConvKernel conv2d_a16_kernel(int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho,
                              int Wo, const EpiDev &e);
 int conv2d_mfma_a16w16(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
@@ -172,9 +174,10 @@ CATCHQ_API const char *catchq_conv2d_kernel(int x_bits, int w_bits, const catchq
   if (check_conv(desc, &ho, &wo) != CATCHQ_OK || check_epi(epilogue, true) != CATCHQ_OK) return route_name(kBad);
   const catchq_conv_desc_t &d = *desc;
   const Route route = conv_route(x_bits, w_bits, desc, nullptr, nullptr);
-  if (route != kMfmaA16) return "general";
+  if (route != kMfma && route != kMfmaA16) return "general";
   const EpiDev e = make_epi(epilogue, (int64_t)d.n * ho * wo * d.co);
-  switch (conv2d_a16_kernel(d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e)) {
+  switch ((route == kMfma ? conv2d_i8_kernel : conv2d_a16_kernel)(d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h,
+                                                                  d.stride_w, d.dil_h, d.dil_w, ho, wo, e)) {
     case kConvWalk: return "walk";
     default: return "general";
   }

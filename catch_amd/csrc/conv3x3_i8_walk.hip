@@ -126,7 +126,6 @@ template <int S>
 static int launch_walk_i8(const void *x, const void *w, const WalkI8Params &p, const EpiDev &e, hipStream_t s) {
   typedef WalkI8<S> G;
   const int waves = (p.g.N + 31) / 32, threads = 64 * waves, lds = G::PATCH + waves * 32 * 40 * 4;
-  if (G::PW * G::PH * G::PIECES > kWalkPasses * threads) return -1;
   const int most = 256 * (16 / waves), blocks = p.ntiles < most ? p.ntiles : most;
 #define CATCHQ_WALK(EPI_)                                                                                              \
   case EPI_:                                                                                                           \
@@ -137,28 +136,40 @@ static int launch_walk_i8(const void *x, const void *w, const WalkI8Params &p, c
     CATCHQ_WALK(EPI_Y16_STEPS);
     CATCHQ_WALK(EPI_Q8_RELU);
     CATCHQ_WALK(EPI_VECTOR);
-    case EPI_SCALAR: return -1;
-    default: break;
+    default: return -1;
   }
-  return -1;
 #undef CATCHQ_WALK
 }
 
-// x [N, H, W, Ci] int8, w [Co, 3, 3, Ci], Ci a multiple of 16; -1: not this kernel's shape
-int conv3x3_i8_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
-                    hipStream_t s) {
+template <int S>
+static bool walk_i8_patch_fits(int Co) { return WalkI8<S>::PW * WalkI8<S>::PH * WalkI8<S>::PIECES <= kWalkPasses * 64 * ((Co + 31) / 32); }
+
+// 3 x 3, padding 1
+bool conv3x3_i8_walk_takes(int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e) {
   const int64_t tiles_x = (Wo + 7) / 8, tiles_y = (Ho + 3) / 4, tiles = N * tiles_x * tiles_y;
-  if ((Ci != 16 && Ci != 32) || Co > 256 || (stride != 1 && stride != 2)) return -1;
+  if ((Ci != 16 && Ci != 32) || Co > 256 || (stride != 1 && stride != 2)) return false;
   if ((int64_t)N * H * W * Ci >= (1ll << 31) || tiles >= (1 << 30) || (int64_t)Wo * Co >= (1 << 28) || (int64_t)N * Ho * Wo >= (1ll << 31))
-    return -1;
+    return false;
   // Four tiles a unit pay for a block's filters (us, tiled kernels / this, 1568 tiles: 16 -> 256 channels 18.7 / 16.9, 32 -> 64 9.0 /
   // 8.9, 32 -> 32 7.8 / 5.8; 392 tiles: 32 -> 64 4.6 / 5.0, 16 -> 256 8.6 / 9.1); of 16 channels one and a half (392 tiles: 16 -> 16
   // 5.2 / 4.0, 16 -> 128 6.5 / 5.8; 112 tiles: 16 -> 16 3.2 / 3.8).
-  if (tiles < 4 * (int64_t)e.cus && !(Ci == 16 && Co <= 128 && tiles * 2 >= 3 * (int64_t)e.cus)) return -1;
+  if (tiles < 4 * (int64_t)e.cus && !(Ci == 16 && Co <= 128 && tiles * 2 >= 3 * (int64_t)e.cus)) return false;
+  if (!(stride == 1 ? walk_i8_patch_fits<1>(Co) : walk_i8_patch_fits<2>(Co))) return false;
+  const int epi = pick_epilogue(Co, e);
+  // The generic epilogue holds up what the walk overlaps (to int8 behind a leaky ReLU: 8 x 112 x 112, 16 -> 192 35.0 / 44.1, 4 x 112 x
+  // 112, 1568 tiles, 32 -> 64 10.8 / 11.8, 128 equal; 8 x 112 x 112, 3136 tiles, 64 6 % ahead, 96 a fifth, 32 a quarter).
+  if (epi == EPI_VECTOR && Co > 32) return Co <= 128 && tiles >= (Co <= 64 ? 8 : 4) * (int64_t)e.cus;
+  return epi == EPI_Y32 || epi == EPI_Y16_STEPS || epi == EPI_Q8_RELU || epi == EPI_VECTOR;
+}
+
+// x [N, H, W, Ci] int8, w [Co, 3, 3, Ci], a call that conv3x3_i8_walk_takes
+int conv3x3_i8_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
+                    hipStream_t s) {
+  const int tiles_x = (Wo + 7) / 8, tiles_y = (Ho + 3) / 4;
   WalkI8Params p = {};
   p.g.M = (int64_t)N * Ho * Wo;
   p.g.N = Co; p.g.K = 9 * Ci; p.g.H = H; p.g.W = W; p.g.Ci = Ci; p.g.Ho = Ho; p.g.Wo = Wo;
-  p.tiles_x = (int)tiles_x; p.tiles_y = (int)tiles_y; p.ntiles = (int)tiles;
+  p.tiles_x = tiles_x; p.tiles_y = tiles_y; p.ntiles = N * tiles_x * tiles_y;
   p.x_bytes = (unsigned)((int64_t)N * H * W * Ci);
   return stride == 1 ? launch_walk_i8<1>(x, w, p, e, s) : launch_walk_i8<2>(x, w, p, e, s);
 }

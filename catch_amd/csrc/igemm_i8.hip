@@ -362,8 +362,16 @@ int conv2d_mfma_i8_grouped(const void *x, const void *w, int N, int H, int W, in
   return igemm_dma_launch(LOAD_CONV, x, w, p, e, (int64_t)N * H * W * Ci, (int64_t)Co * p.K, s);
 }
 
+bool conv3x3_i8_walk_takes(int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e);
 int conv3x3_i8_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
                     hipStream_t s);
+
+ConvKernel conv2d_i8_kernel(int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho,
+                            int Wo, const EpiDev &e) {
+  if (kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1 && conv3x3_i8_walk_takes(N, H, W, Ci, Co, sh, Ho, Wo, e))
+    return kConvWalk;
+  return kConvGeneral;
+}
 
 int conv2d_mfma_i8(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph,
                    int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
@@ -372,10 +380,8 @@ int conv2d_mfma_i8(const void *x, const void *w, int N, int H, int W, int Ci, in
   p.N = Co;
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo;
   p.kh = kh; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
-  if (kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1) {
-    const int st = conv3x3_i8_walk(x, w, N, H, W, Ci, Co, sh, Ho, Wo, e, s);
-    if (st >= 0) return st;
-  }
+  if (conv2d_i8_kernel(N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, e) == kConvWalk)
+    return conv3x3_i8_walk(x, w, N, H, W, Ci, Co, sh, Ho, Wo, e, s);
   // Beyond two 32x32 tiles per unit the patch-resident kernel is faster than the few-tiles one while it makes a single round
   // of blocks: 7x7 512 -> 512 3x3, 24 images (592 tiles) 11.3 / 14.0 us, 32 images 11.7 / 16.3; 20 images (496 tiles)
   // 11.3 / 9.6, 36 images (a second round) 20.9 / 16.5, stride 2 17.6 / 16.3

@@ -11,10 +11,10 @@ from catch_amd import _native
 pytestmark = pytest.mark.gpu
 
 
-def _kernel(bits, n, h, w, ci, co, ksize, stride, sharing=1):
-    """which kernel serves the calls of a layer that these tests make"""
+def _kernel(bits, n, h, w, ci, co, ksize, stride, sharing=1, **epilogue):
+    """which kernel serves a layer with a floating output and what else the epilogue has"""
     d = _native.ConvDesc(n, h, w, ci, co, ksize, ksize, ksize // 2, ksize // 2, stride, stride, 1, 1, 1)
-    e = _native.Epilogue(y=16, sharing=sharing)
+    e = _native.Epilogue(y=16, sharing=sharing, **epilogue)
     return _native.kernel_lib().catchq_conv2d_kernel(bits, 8, ctypes.byref(d), ctypes.byref(e)).decode()
 
 
@@ -59,13 +59,20 @@ def test_conv_walk(n, h, w, ci, co, stride, kernel):
 
 
 # int8: more tiles than the rule asks for (sharing makes it plan for 256 / sharing units), edges of tiles either way, fewer than one wave's
-# channels, all eight waves
-@pytest.mark.parametrize("n,h,w,ci,co,stride,sharing", [
-    (1, 4, 8, 16, 16, 1, 256), (1, 9, 33, 16, 36, 1, 64), (3, 13, 17, 32, 256, 1, 64), (2, 10, 16, 32, 4, 1, 64), (5, 129, 131, 16, 20, 1, 1),
-    (2, 17, 30, 16, 128, 2, 64), (3, 16, 31, 32, 100, 2, 64), (40, 66, 50, 32, 256, 2, 1), (2, 60, 60, 32, 64, 2, 64),
-    (1, 9, 33, 32, 260, 1, 64), (4, 33, 33, 48, 64, 1, 64), (4, 60, 60, 32, 32, 2, 1),  # not this kernel's
+# channels, all eight waves.  kernels: of an epilogue with an instance of its own, and of the generic one
+BOTH, OWN, NONE = ("walk", "walk"), ("walk", "general"), ("general", "general")
+
+
+@pytest.mark.parametrize("n,h,w,ci,co,stride,sharing,kernels", [
+    (1, 4, 16, 16, 16, 1, 256, BOTH), (1, 9, 33, 16, 36, 1, 64, OWN), (3, 13, 17, 32, 256, 1, 64, OWN), (2, 10, 17, 32, 4, 1, 64, BOTH),
+    (5, 129, 131, 16, 20, 1, 1, BOTH), (2, 17, 30, 16, 128, 2, 64, OWN), (3, 17, 33, 32, 100, 2, 64, BOTH), (40, 66, 50, 32, 256, 2, 1, OWN),
+    (2, 60, 60, 32, 64, 2, 64, BOTH), (1, 16, 32, 32, 64, 1, 64, OWN), (1, 17, 60, 32, 64, 1, 64, BOTH), (1, 17, 60, 32, 128, 1, 64, BOTH),
+    (1, 17, 60, 32, 132, 1, 64, OWN), (1, 9, 33, 16, 32, 1, 64, BOTH),
+    (1, 4, 8, 16, 16, 1, 256, NONE), (2, 10, 16, 32, 4, 1, 64, NONE), (3, 16, 31, 32, 100, 2, 64, NONE),
+    (1, 9, 33, 32, 260, 1, 64, NONE), (4, 33, 33, 48, 64, 1, 64, NONE), (4, 60, 60, 32, 32, 2, 1, NONE),
 ])
-def test_conv_walk_int8(n, h, w, ci, co, stride, sharing):
+def test_conv_walk_int8(n, h, w, ci, co, stride, sharing, kernels):
+    assert (_kernel(8, n, h, w, ci, co, 3, stride, sharing), _kernel(8, n, h, w, ci, co, 3, stride, sharing, acc_out=16)) == kernels
     gen = torch.Generator().manual_seed(h * w + co)
     x = torch.randint(-128, 128, (n, h, w, ci), generator=gen).to(torch.int8)
     qw = torch.randint(-128, 128, (co, 3, 3, ci), generator=gen).to(torch.int8)

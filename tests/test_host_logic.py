@@ -517,3 +517,16 @@ def test_int16_layers_of_64_channels_at_stride_2(lib):
     assert kernel(1, 208, 128, 2) == kernel(1, 208, 100, 2) == "general"
     assert kernel(1, 208, 96, 2) == kernel(2, 208, 128, 2) == kernel(1, 208, 128, 2, sharing=2) == kernel(1, 104, 128, 1) == "walk"
     assert kernel(1, 48, 128, 1) == kernel(2, 208, 130, 2) == "general"  # few tiles, rows of no whole groups of four
+
+
+def test_int8_layers_of_few_channels_with_a_generic_epilogue(lib):
+    """... walk up to 128 columns: from four tiles of 8 x 4 outputs a unit on beyond 64 of them, from eight beyond 32"""
+    from catch_amd import _native
+
+    def kernel(n, side, ci, co, **k):
+        d = _native.ConvDesc(n, side, side, ci, co, 3, 3, 1, 1, 1, 1, 1, 1, 1)
+        return lib.catchq_conv2d_kernel(8, 8, ctypes.byref(d), ctypes.byref(_native.Epilogue(y=16, **k))).decode()
+    for n, ci, co, want in [(8, 16, 192, "general"), (8, 32, 132, "general"), (4, 32, 64, "general"), (8, 32, 64, "walk"), (4, 32, 96, "walk"),
+                            (4, 16, 128, "walk"), (1, 16, 96, "general"), (1, 16, 32, "walk"), (4, 32, 32, "walk")]:
+        assert kernel(n, 112, ci, co, acc_out=16) == want, (n, ci, co)
+        assert kernel(n, 112, ci, co) == "walk"  # fp32 alone: an instance of its own
