@@ -179,6 +179,7 @@ CATCHQ_API const char *catchq_conv2d_kernel(int x_bits, int w_bits, const catchq
   switch ((route == kMfma ? conv2d_i8_kernel : conv2d_a16_kernel)(d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h,
                                                                   d.stride_w, d.dil_h, d.dil_w, ho, wo, e)) {
     case kConvWalk: return "walk";
+    case kConvShort: return "short";
     default: return "general";
   }
 }

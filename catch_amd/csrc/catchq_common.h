@@ -20,7 +20,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 
 // kernels that serve some convolutions ahead of their family's general ones (catchq_conv2d_kernel)
-enum ConvKernel { kConvGeneral, kConvWalk };
+enum ConvKernel { kConvGeneral, kConvWalk, kConvShort };
 
 inline hipStream_t as_stream(catchq_stream_t s) { return reinterpret_cast<hipStream_t>(s); }
 

@@ -420,6 +420,7 @@ int igemm_a16_launch(int load, const void *a, const void *b, IgemmParams p, cons
 bool conv3x3_a16_walk_takes(int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e);
 int conv3x3_a16_walk(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int stride, int Ho, int Wo, const EpiDev &e,
                      hipStream_t s);
+bool pw_a16_short_takes(int64_t M, int64_t N, int64_t K, const EpiDev &e);
 int pw_a16_short(const void *x, const void *w, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s);
 int contract_ksplit(const void *x, bool a16, const void *w, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
                     int sh, int sw, int dh, int dw, int Ho, int Wo, bool patch, const EpiDev &e, hipStream_t s);
@@ -547,6 +548,7 @@ ConvKernel conv2d_a16_kernel(int N, int H, int W, int Ci, int Co, int kh, int kw
                              int Wo, const EpiDev &e) {
   if (kh == 3 && kw == 3 && ph == 1 && pw == 1 && sh == sw && dh == 1 && dw == 1 && conv3x3_a16_walk_takes(N, H, W, Ci, Co, sh, Ho, Wo, e))
     return kConvWalk;
+  if (kh == 1 && kw == 1 && ph == 0 && pw == 0 && sh == 1 && sw == 1 && pw_a16_short_takes((int64_t)N * Ho * Wo, Co, Ci, e)) return kConvShort;
   return kConvGeneral;
 }
 
@@ -560,6 +562,7 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   p.K = kh * kw * Ci;
   const ConvKernel kernel = conv2d_a16_kernel(N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, e);
   if (kernel == kConvWalk) return conv3x3_a16_walk(x, w, N, H, W, Ci, Co, sh, Ho, Wo, e, s);
+  if (kernel == kConvShort) return pw_a16_short(x, w, p.M, Co, Ci, e, s);
   if (Ci % 16 == 0) {  // a few blocks per unit, long K
     const int st = contract_ksplit(x, true, w, N, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false, e, s);
     if (st >= 0) return st;
@@ -571,10 +574,6 @@ int conv2d_mfma_a16(const void *x, const void *w, int N, int H, int W, int Ci, i
   }
   // a pointwise convolution is a plain GEMM over the pixels: row address = index x K, no pixel split and no
   // tap masks in front of the first load
-  if (kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0) {
-    const int st = pw_a16_short(x, w, p.M, Co, Ci, e, s);
-    if (st >= 0) return st;
-  }
   const char *as_gemm = tuning_env("CATCHQ_PW_AS_GEMM");
   if (kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && !(as_gemm && atoi(as_gemm) == 0)) {
     const int st = igemm_a16_launch(LOAD_GEMM, x, w, p, e, p.M * Ci * 2, (int64_t)Co * Ci, s);

@@ -12,7 +12,7 @@
 namespace catchq {
 
 struct PwA16Params {
-  IgemmParams g;   // M, N, K, tiles_n, nblocks
+  IgemmParams g;   // M, N, K, nblocks
   unsigned x_bytes;
   int col_groups;  // waves side by side, 32 columns each (a power of two); the others take further rows
 };
@@ -31,10 +31,8 @@ __global__ __launch_bounds__(256, 4) void pw_a16_short_kernel(const int16_t *__r
   const int frow = lane & 31, fhalf = lane >> 5;
   const int cg = wave & (p.col_groups - 1), pg = wave / p.col_groups;
   const int rows = 128 / p.col_groups;  // of the block
-  const int logical = xcd_remap(blockIdx.x, p.g.nblocks);
-  const int tile_m = logical / p.g.tiles_n, tile_n = logical - tile_m * p.g.tiles_n;
-  const int64_t m0 = (int64_t)tile_m * rows;
-  const int n0 = (tile_n * p.col_groups + cg) * 32;
+  const int64_t m0 = (int64_t)xcd_remap(blockIdx.x, p.g.nblocks) * rows;
+  const int n0 = cg * 32;
   const __amdgpu_buffer_rsrc_t rsrc_x = __builtin_amdgcn_make_buffer_rsrc((void *)X, 0, (int)p.x_bytes, 0x00020000);
 
   // rows -> digits in LDS: 16 values a piece
@@ -89,31 +87,32 @@ __global__ __launch_bounds__(256, 4) void pw_a16_short_kernel(const int16_t *__r
 
 template <int KK>
 static int launch_pw_a16(const void *x, const void *w, const PwA16Params &p, const EpiDev &e, hipStream_t s) {
-#define CATCHQ_PW(EPI_)                                                                                              \
-  case EPI_:                                                                                                         \
-    pw_a16_short_kernel<KK, EPI_><<<p.g.nblocks, 256, 0, s>>>((const int16_t *)x, (const int8_t *)w, p, e);          \
-    return launch_status()
-  switch (pick_epilogue(p.g.N, e)) {
-    CATCHQ_PW(EPI_LK_Q16);
-    CATCHQ_PW(EPI_VECTOR);
-    default: return -1;
-  }
-#undef CATCHQ_PW
+  if (pick_epilogue(p.g.N, e) == EPI_LK_Q16)
+    pw_a16_short_kernel<KK, EPI_LK_Q16><<<p.g.nblocks, 256, 0, s>>>((const int16_t *)x, (const int8_t *)w, p, e);
+  else
+    pw_a16_short_kernel<KK, EPI_VECTOR><<<p.g.nblocks, 256, 0, s>>>((const int16_t *)x, (const int8_t *)w, p, e);
+  return launch_status();
 }
 
-// x [M, K] int16, w [N, K]; -1: not this kernel's shape
+// A few columns of 64 channels on less than half a block for a unit stay with the tiled kernel (us to int16 behind a ReLU, tiled / this:
+// 52 x 52, 64 -> 4 6.9 / 7.7, 8 7.0 / 7.5, 12 ahead by 8 %; 4 x 104 x 104, 338 blocks, 4 a fifth ahead).
+bool pw_a16_short_takes(int64_t M, int64_t N, int64_t K, const EpiDev &e) {
+  if ((K != 64 && K != 128) || N > 128 || M * K * 2 >= (1ll << 31)) return false;
+  if (K == 64 && N <= 8 && (M + 127) / 128 * 2 < e.cus) return false;
+  const int epi = pick_epilogue((int)N, e);
+  return epi == EPI_LK_Q16 || epi == EPI_VECTOR;
+}
+
+// x [M, K] int16, w [N, K], a call that pw_a16_short_takes
 int pw_a16_short(const void *x, const void *w, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s) {
-  if ((K != 64 && K != 128) || N > 128 || M * K * 2 >= (1ll << 31)) return -1;
-  const int64_t groups = (N + 31) / 32;
+  const int groups = (int)((N + 31) / 32);
   PwA16Params p = {};
   p.g.M = M; p.g.N = (int)N; p.g.K = (int)K;
   p.x_bytes = (unsigned)(M * K * 2);
-  p.col_groups = groups > 2 ? 4 : (int)groups;
+  p.col_groups = groups > 2 ? 4 : groups;
   if (K == 128 && p.col_groups == 1) p.col_groups = 2;  // (128 rows of 128 channels: twice the room)
   const int rows = 128 / p.col_groups;
-  p.g.tiles_n = (int)((groups + p.col_groups - 1) / p.col_groups);
-  const int64_t nb = (M + rows - 1) / rows * p.g.tiles_n;
-  p.g.nblocks = (int)nb;  // (fewer than 2^24 rows)
+  p.g.nblocks = (int)((M + rows - 1) / rows);  // (fewer than 2^24 rows)
   return K == 64 ? launch_pw_a16<2>(x, w, p, e, s) : launch_pw_a16<4>(x, w, p, e, s);
 }
 

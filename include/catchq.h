@@ -511,7 +511,7 @@ int catchq_global_avgpool_quantize_nhwc(const float *x, void *q, int bitwidth, i
 const char *catchq_conv2d_route(int x_bits, int w_bits, const catchq_conv_desc_t *desc);
 const char *catchq_gemm_route(int a_bits, int b_bits, int64_t m, int64_t n, int64_t k);
 /* ... and whether a kernel of its own goes ahead of that family's general ones, with operands on 16-byte boundaries: "walk" (3 x 3
- * layers of few channels), "general". */
+ * layers of few channels), "short" (pointwise int16 layers of few), "general". */
 const char *catchq_conv2d_kernel(int x_bits, int w_bits, const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue);
 
 /* ------------------------------------------------------------------ diagnostics */

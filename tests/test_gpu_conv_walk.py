@@ -97,11 +97,12 @@ def test_conv_walk_int8(n, h, w, ci, co, stride, sharing, kernels):
 
 
 # rows that end inside a block's, columns that end inside a wave's, every count of waves side by side
-@pytest.mark.parametrize("n,h,w,ci,co", [
-    (1, 1, 1, 64, 4), (1, 3, 43, 64, 32), (2, 8, 8, 64, 36), (1, 5, 13, 64, 64), (3, 11, 3, 64, 100), (1, 8, 16, 64, 128), (3, 61, 67, 64, 96),
-    (1, 1, 1, 128, 32), (1, 7, 9, 128, 28), (1, 8, 8, 128, 64), (5, 13, 5, 128, 68), (2, 31, 33, 128, 128), (2, 9, 9, 64, 132), (2, 9, 9, 192, 64),
-])
-def test_pointwise_int16(n, h, w, ci, co):
+@pytest.mark.parametrize("n,h,w,ci,co,kernel", [row + ("short",) for row in [
+    (1, 1, 1, 64, 12), (1, 3, 43, 64, 32), (2, 8, 8, 64, 36), (1, 5, 13, 64, 64), (3, 11, 3, 64, 100), (1, 8, 16, 64, 128), (3, 61, 67, 64, 96),
+    (1, 1, 1, 128, 32), (1, 7, 9, 128, 28), (1, 8, 8, 128, 64), (5, 13, 5, 128, 68), (2, 31, 33, 128, 128), (1, 1, 1, 128, 4),
+    (1, 129, 128, 64, 8)]] + [row + ("general",) for row in [(1, 1, 1, 64, 4), (1, 127, 127, 64, 8), (2, 9, 9, 64, 132), (2, 9, 9, 192, 64)]])
+def test_pointwise_int16(n, h, w, ci, co, kernel):
+    assert _kernel(16, n, h, w, ci, co, 1, 1, acc_out=16) == _kernel(16, n, h, w, ci, co, 1, 1, acc_out=16, resid=16) == kernel
     gen = torch.Generator().manual_seed(h * w + co)
     x = torch.randint(-32768, 32768, (n, h, w, ci), generator=gen).short()
     x.view(-1)[:2] = torch.tensor([-32768, 32767])

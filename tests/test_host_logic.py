@@ -530,3 +530,14 @@ def test_int8_layers_of_few_channels_with_a_generic_epilogue(lib):
                             (4, 16, 128, "walk"), (1, 16, 96, "general"), (1, 16, 32, "walk"), (4, 32, 32, "walk")]:
         assert kernel(n, 112, ci, co, acc_out=16) == want, (n, ci, co)
         assert kernel(n, 112, ci, co) == "walk"  # fp32 alone: an instance of its own
+
+
+def test_int16_pointwise_layers_of_a_few_columns(lib):
+    """... of 64 channels stay with the tiled kernel on less than half a block of 128 rows for a unit"""
+    from catch_amd import _native
+
+    def kernel(side, ci, co):
+        d = _native.ConvDesc(1, side, side, ci, co, 1, 1, 0, 0, 1, 1, 1, 1, 1)
+        return lib.catchq_conv2d_kernel(16, 8, ctypes.byref(d), ctypes.byref(_native.Epilogue(y=16, acc_out=16))).decode()
+    assert kernel(52, 64, 4) == kernel(126, 64, 8) == kernel(52, 64, 132) == kernel(52, 192, 64) == "general"
+    assert kernel(52, 64, 12) == kernel(128, 64, 4) == kernel(52, 128, 4) == "short"
