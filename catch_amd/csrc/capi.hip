@@ -467,20 +467,24 @@ CATCHQ_API int catchq_conv3x3_packed(const void *x, const void *packed, int n, i
   return st < 0 ? CATCHQ_ERR_UNSUPPORTED : st;
 }
 
-CATCHQ_API int catchq_conv3x3_i8_packed_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {
-  int st = check_epi(epilogue, true);
+static int check_conv3x3_i8_packed(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {
+  const int st = check_epi(epilogue, true);
   if (st != CATCHQ_OK) return st;
   if (n < 0 || h <= 0 || w <= 0 || ci <= 0 || co <= 0) return CATCHQ_ERR_ARG;
-  size_t bytes;
-  st = catchq_packed_filters_size(co, 9 * (int64_t)ci, &bytes);
-  if (st != CATCHQ_OK) return st;
   if ((int64_t)h * w >= (1ll << 31) || (int64_t)n * h * w >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  size_t bytes;
+  return catchq_packed_filters_size(co, 9 * (int64_t)ci, &bytes);
+}
+
+CATCHQ_API int catchq_conv3x3_i8_packed_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {
+  const int st = check_conv3x3_i8_packed(n, h, w, ci, co, epilogue);
+  if (st != CATCHQ_OK) return st;
   return n == 0 || conv3x3_i8_packed_takes(n, h, w, ci, co, make_epi(epilogue, (int64_t)n * h * w * co)) ? CATCHQ_OK : CATCHQ_ERR_UNSUPPORTED;
 }
 
 CATCHQ_API int catchq_conv3x3_i8_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
                                         const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
-  const int st = catchq_conv3x3_i8_packed_takes(n, h, w, ci, co, epilogue);
+  const int st = check_conv3x3_i8_packed(n, h, w, ci, co, epilogue);
   if (st != CATCHQ_OK || n == 0) return st;
   if (!x || !packed) return CATCHQ_ERR_ARG;
   if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;

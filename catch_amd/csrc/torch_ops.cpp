@@ -1257,13 +1257,13 @@ catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64
   return e;
 }
 
-// The filters of a 3 x 3 layer that catchq_conv3x3_i8_packed takes; null: another route serves it.
+// The filters of a 3 x 3 layer for catchq_conv3x3_i8_packed; null: another route serves it.  Packed ones are handed out without a
+// question: that call answers it.
 const void *conv3x3_packed(Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e) {
   if (prep.bw_x != 8 || prep.bw_w != 8 || d.kh != 3 || d.kw != 3 || d.groups != 1 || d.pad_h != 1 || d.pad_w != 1 || d.stride_h != 1 ||
       d.stride_w != 1 || d.dil_h != 1 || d.dil_w != 1 || !catchq::conv3x3_i8_packed_channels(d.ci))
     return nullptr;
-  if (catchq_conv3x3_i8_packed_takes(d.n, d.h, d.w, d.ci, d.co, &e) != CATCHQ_OK) return nullptr;
-  return packed_weight(prep, [] { return true; });
+  return packed_weight(prep, [&] { return catchq_conv3x3_i8_packed_takes(d.n, d.h, d.w, d.ci, d.co, &e) == CATCHQ_OK; });
 }
 
 // quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x) x prepared weight -> floating

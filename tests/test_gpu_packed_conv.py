@@ -178,3 +178,19 @@ def test_plans_hold_packed_filters_that_are_read():
     fused = pipeline.FusedNet(layers, pipeline.to_position_encoding(sd, 16, 8))
     packed = set((l.ci, l.co) for l in layers if l.kind == "conv" and fused.q[l.name].packed is not None)
     assert packed == {(128, 256), (256, 512), (512, 1024)}
+
+
+def test_packed_filters_and_calls_that_other_routes_serve():
+    """a batch that the packed filters serve, one that they do not (a block of 32 pixels for less than half the units), and back: the
+    same bits as on a weight that was never packed, NCHW and NHWC"""
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    wt, b = torch.randn(192, 96, 3, 3, generator=gen, device="cuda"), torch.randn(192, generator=gen, device="cuda")
+    scale, mode = torch.tensor([127 / 5.0, 127 / 5.0], device="cuda"), torch.tensor([1], dtype=torch.int32, device="cuda")
+    call = lambda x, w: torch.ops.torch_mlu.conv2d(x, w, b, [1, 1], [1, 1], [1, 1], 1, scale, mode)  # noqa: E731
+    e = _native.Epilogue(y=16)
+    takes = lambda n, h: _native.kernel_lib().catchq_conv3x3_i8_packed_takes(n, h, h, 96, 192, ctypes.byref(e)) == 0  # noqa: E731
+    assert takes(8, 28) and not takes(1, 60)
+    for n, h in [(8, 28), (8, 28), (1, 60), (8, 28), (1, 60), (0, 28)]:
+        x = torch.randn(n, 96, h, h, generator=gen, device="cuda")
+        want = call(x, wt.clone())
+        assert torch.equal(call(x, wt), want) and torch.equal(call(x.contiguous(memory_format=torch.channels_last), wt), want)
