@@ -7,15 +7,18 @@
 // - a block's activations come once per 64 channels, not once per tap: nine taps of 64 consecutive output pixels (stride 1, same
 //   size) read one run of 64 + 2 W + 2 consecutive input pixels.  They are split into digits on their way into LDS; taps outside
 //   the image read a pixel of zeros instead (per lane and tap);
-// - filters go from L2 to registers (each wave has 64 columns of its own), one half step ahead, and never through LDS;
+// - filters go from L2 to registers (each wave has 64 columns of its own), two half steps ahead (five with 32 rows a wave), and
+//   never through LDS;
 // - a wave has 64 (or 32) x 64 outputs: 16 matrix instructions of 32 clocks a step for 8 KB out of LDS and 4 KB out of L2.
-// Barriers: one per 64 channels.  Two waves a SIMD: one's address arithmetic and loads run under the other's matrix
+// Barriers: one per 64 channels.  Two waves a SIMD (246 to 253 registers with 64 rows a wave, 169 to 187 with 32, where 168 would be
+// three; a shorter ring of filters there is not tried): one's address arithmetic and loads run under the other's matrix
 // instructions.  What bounds it now: the matrix pipes while a block has its unit to itself (46 clocks an instruction at 2.4 GHz,
 // whatever the depth of the filter ring), the last round of blocks, and an epilogue that all blocks reach together.
 // us, before / now (16 images unless said): 13 x 13, 512 -> 1024 46 / 33, 26 x 26, 256 -> 512 37 / 30, 52 x 52, 128 -> 256 42 / 31,
-// with the residual and fp32 output 51 / 42; 8 images 26 / 18, 25 / 18, 22 / 19.
-// Tried: 96 and 128 rows a wave on one wave a SIMD (30 and 36 us on 16 x 26 x 26, 37 and 45 on 52 x 52), filters nine half
-// steps ahead (equal), 128 x 128 blocks for 64 -> 128 channels on 104 x 104 (51 / 52: its outputs bound it).
+// with the residual and fp32 output 51 / 42; 8 images 26 / 18, 25 / 18, 22 / 19 (launches in their sequence; repeated in a graph, 16
+// images, 47 / 33, 38 / 32, 43 / 33, 52 / 45).
+// Tried: 96 and 128 rows a wave on one wave a SIMD (30 and 36 us on 16 x 26 x 26, 37 and 45 on 52 x 52), filters five or
+// eight half steps ahead (equal), 128 x 128 blocks for 64 -> 128 channels on 104 x 104 (51 / 52: its outputs bound it).
 #include "conv3x3_halo.h"
 
 namespace catchq {

@@ -6,8 +6,9 @@
 // overlaps.  Here a block requests the whole run of input pixels that its outputs read (TM * 32 + 2 W + 2 of them: same size,
 // stride 1) at once and meets one barrier; filters go from L2 to registers, nine fragments ahead.  Taps outside the image read a
 // pixel of zeros, per lane and tap.  A wave has TM * 32 pixels x 32 channels, a block up to eight waves side by side.
-// us with the quantizer in front, tiled / this: 5 x 57 x 75, 96 -> 160 on NCHW floats 18.7 / 15.9, on NHWC halfs 16.7 / 14.1;
-// 8 x 28 x 28, 192 14.5 / 11.5, 16 x 14 x 14, 384 20.2 / 15.0, 20 x 57 x 75, 96 -> 160 53.1 / 42.5.
+// us with the quantizer in front, repeated in a graph on the same inputs, tiled / this: 5 x 57 x 75, 96 -> 160 on NCHW floats 18.7 /
+// 16.0 (17.6 / 15.5 on changing inputs), on NHWC halfs 16.8 / 14.1; on NCHW floats 8 x 28 x 28, 192 14.3 / 11.4, 16 x 14 x 14, 384
+// 19.9 / 14.6, 20 x 57 x 75, 96 -> 160 51.6 / 41.9.
 #include "conv3x3_halo.h"
 
 namespace catchq {

@@ -1085,9 +1085,9 @@ struct RelaxedCapture {
 };
 
 // The entry's weight as catchq_float_linear_packed and catchq_conv3x3_i8_packed (8 bits) and catchq_float_linear_digits (16) read
-// it; null: the call goes without.  The weight is laid out at the second call that the route takes.  A caller that rewrites its weight between calls, or
-// uses it once, does not pay for that (6 us of kernel, a launch and an allocation: first pass of 1 x 768 -> 3072 on a new
-// weight 226 us with it, 218 without), and a weight whose calls do not take the route is not held twice.
+// it; null: the call goes without.  The weight is laid out at the second call that the route takes.  A caller that rewrites its
+// weight between calls, or uses it once, does not pay for that (6 us of kernel, a launch and an allocation: first pass of 1 x 768 ->
+// 3072 on a new weight 226 us with it, 218 without), and a weight whose calls do not take the route is not held twice.
 template <typename Takes>
 const void *packed_weight(Prepared &p, Takes takes) {
   const auto cur = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA();

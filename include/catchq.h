@@ -271,7 +271,8 @@ int catchq_float_linear_packed(const void *x, int x_dtype, int x_position, const
 /* A 3 x 3 convolution (stride 1, padding 1) of int16 activations with int8 filters laid out once in the order of the matrix
  * instruction: catchq_pack_conv3x3 writes catchq_packed_conv3x3_size bytes from w [co,3,3,ci], ci a multiple of 64.  x [n,h,w,ci],
  * outputs as catchq_conv2d_nhwc's.  CATCHQ_ERR_UNSUPPORTED: catchq_conv2d_nhwc on the filters as they are serves the call better,
- * or alone (few output channels or blocks, wide images, rows that the vector epilogues do not take). */
+ * or alone (output channels that leave much of the last 256 empty, few blocks, wide images, rows that the vector epilogues do not
+ * take). */
 int catchq_packed_conv3x3_size(int64_t co, int64_t ci, size_t *bytes);
 int catchq_pack_conv3x3(const void *w, int64_t co, int64_t ci, void *packed, catchq_stream_t stream);
 int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
