@@ -147,13 +147,24 @@ static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, const EpiDev 
   // Up to 64 channels leave a block one wave or two: more than a round of blocks, and four (three) of them to a unit, have to hide
   // what it waits for (with the quantizer: 6 x 28 x 28, 384 -> 16, 74 blocks, 9.1 / 13.4, 64 x 14 x 14, 192 -> 32, 196, 9.4 / 12.2, 64
   // 11.2 / 12.3; 32 x 28 x 28, 96 -> 32, 392, 11.8 / 10.9, 64 12.5 / 11.8; but 60 x 60, 384 -> 16, 562 of 75 KB, a quarter slower).
-  if (groups <= 2) return blocks(2) * 8 >= 9 * (int64_t)e.cus && patch(2) <= (groups == 1 ? 40 : 52) * 1024 ? 2 : 0;
+  // Wide images ask for two rounds of them (5 x 57 x 75, 160 -> 16, 334 blocks, 14.3 / 15.4).
+  if (groups <= 2) {
+    if (blocks(2) * 8 >= 9 * (int64_t)e.cus && patch(2) <= (groups == 1 ? 40 : 52) * 1024 && (W <= 48 || blocks(2) >= 2 * (int64_t)e.cus)) return 2;
+    // Channels that are no multiple of 64 make the tiled kernel's steps cross filter taps, and fewer blocks or larger patches will do
+    // (40 x 28 x 28, 608 -> 64, 490 of 75 KB, a tenth ahead; of 32 pixels 10 x 28 x 28, 480 -> 64, 245 blocks, a seventh, 64 x 14 x 14,
+    // 992 -> 64 a sixth, 6 x 28 x 28, 147, 800 -> 64 an eighth, 224 -> 64 equal; not up to 44 channels or on wide images: 227 of 160 -> 36
+    // on rows of 55 8 % behind)
+    if (Ci % 64 == 0 || Co < 48 || W > 48) return 0;
+    if (blocks(2) * 2 >= 3 * (int64_t)e.cus && fits(2)) return 2;
+    return fits(1) && (blocks(1) * 8 >= 7 * (int64_t)e.cus || (Ci >= 480 && blocks(1) * 2 >= e.cus)) ? 1 : 0;
+  }
   if (blocks(1) * 2 < e.cus) return 0;
   if (blocks(2) * 2 < e.cus) return fits(1) ? 1 : 0;
   if (fits(2)) return 2;
-  // where only blocks of 32 fit, the wider tiles of many columns are ahead (with the quantizer: 5 x 57 x 75, 384 -> 192 46.7 / 39.8,
-  // 512 65.4 / 80.0; 8 x 56 x 56, 480 -> 192 62.3 / 55.0, 256 66.9 / 68.7, 512 84.9 / 109.8)
-  return fits(1) && groups < 8 ? 1 : 0;
+  // Where only blocks of 32 fit, the wider tiles of many columns are ahead on many rows (with the quantizer: 5 x 57 x 75, 384 -> 192
+  // 46.7 / 39.8, 320 60.0 / 55.3, 512, 1336 blocks, 65.4 / 80.0; 8 x 56 x 56, 480 -> 192 62.3 / 55.0, 512, 1568, 84.9 / 109.8; but
+  // 10 x 28 x 28, 768 -> 320, 490, 50.6 / 36.8, 64 x 14 x 14, 992 -> 384, 784, 118 / 87).
+  return fits(1) && (groups <= 10 || blocks(1) * 4 <= 13 * (int64_t)e.cus) ? 1 : 0;
 }
 
 bool conv3x3_i8_packed_takes(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e) { return packed_i8_plan(N, H, W, Ci, Co, e) != 0; }

@@ -117,9 +117,10 @@ def test_packed_conv3x3_other_calls():
     (2, 96, 57, 75, 160, 3, torch.float32, False, 1, True), (1, 96, 9, 9, 30, 3, torch.float32, False, 256, False),
     (1, 128, 9, 9, 64, 3, torch.float32, False, 256, False), (1, 96, 9, 9, 64, 3, torch.float32, False, 1, False),
     (1, 96, 9, 8, 4, 1, torch.float32, False, 256, True), (2, 320, 37, 1, 64, 3, torch.float16, False, 256, True),
-    (1, 96, 2, 140, 32, 3, torch.float32, False, 64, True), (1, 160, 1, 1, 68, 1, torch.float32, False, 256, True),
+    (1, 96, 2, 140, 32, 3, torch.float32, False, 64, False), (1, 96, 7, 40, 32, 3, torch.float32, False, 64, True), (1, 160, 1, 1, 68, 1, torch.float32, False, 256, True),
     (2, 96, 5, 33, 196, 3, torch.float16, False, 256, True), (1, 480, 3, 60, 164, 3, torch.float32, False, 256, True),
-    (1, 480, 3, 60, 228, 3, torch.float32, False, 256, False),
+    (1, 480, 3, 60, 320, 3, torch.float32, False, 256, True),
+    (1, 480, 3, 60, 324, 3, torch.float32, False, 256, False), (1, 96, 3, 20, 64, 3, torch.float32, True, 256, True),
 ])
 def test_packed_conv3x3_int8(n, ci, h, w, co, mode, dtype, nhwc, sharing, taken):
     """the first call of a weight goes without packed filters, later ones read them: the same bits, equal to the oracle's"""

@@ -476,8 +476,14 @@ def test_packed_conv3x3_refusals(lib):
     for n, h, w, ci, co, want in [(6, 28, 28, 384, 16, False), (64, 14, 14, 192, 64, False), (64, 14, 14, 192, 68, True), (32, 28, 28, 96, 32, True),
                                   (32, 28, 28, 96, 64, True), (10, 60, 60, 384, 64, False), (40, 23, 23, 320, 32, True), (40, 23, 23, 480, 32, False),
                                   (40, 23, 23, 352, 64, True),
+                                  # blocks of 32 pixels of channels that are no multiple of 64
+                                  (10, 28, 28, 480, 64, True), (10, 28, 28, 480, 44, False), (10, 28, 28, 448, 64, False),
+                                  (9, 28, 28, 480, 64, True), (9, 28, 28, 416, 64, False), (5, 28, 28, 480, 64, False),
+                                  (64, 14, 14, 992, 64, True), (5, 57, 75, 160, 16, False), (10, 57, 75, 160, 16, True), (3, 49, 49, 160, 64, False), (3, 49, 48, 160, 64, False),
+                                  (4, 44, 44, 160, 64, True), (4, 44, 49, 160, 64, False),
                                   # only blocks of 32 pixels fit twice into a unit
-                                  (8, 56, 56, 480, 192, True), (8, 56, 56, 480, 224, True), (8, 56, 56, 480, 228, False), (8, 56, 56, 480, 512, False)]:
+                                  (8, 56, 56, 480, 192, True), (8, 56, 56, 480, 224, True), (8, 56, 56, 480, 320, True), (8, 56, 56, 480, 324, False),
+                                  (8, 56, 56, 480, 512, False), (10, 28, 28, 768, 320, True), (64, 14, 14, 992, 384, True), (5, 57, 75, 384, 512, False)]:
         assert (takes(n, h, w, ci, co) == OK) == want, (n, h, w, ci, co)
     e.sharing = 4  # a quarter of the units: fewer blocks will do
     assert takes(1, 28, 28, 192, 192) == UNSUPPORTED and takes(2, 28, 28, 192, 192) == OK
