@@ -106,6 +106,7 @@ SIGNATURES = {
     "catchq_pack_filters": (_I, [_P, _I64, _I64, _P, _P]),
     "catchq_float_linear_packed_takes": (_I, [_I, _I64, _I64, _I64, ctypes.POINTER(Epilogue)]),
     "catchq_float_linear_packed": (_I, [_P, _I, _I, _P, _I64, _I64, _I64, ctypes.POINTER(Epilogue), _P]),
+    "catchq_float_conv2d_small": (_I, [_P, _I, _I, _I, _I, _P, _I, ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue), _P]),
     "catchq_float_conv2d_workspace_size": (_I, [_I, ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue), ctypes.POINTER(_SZ)]),
     "catchq_float_conv2d_nhwc": (_I, [_P, _I, _I, _P, ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue), _P, _SZ, _P]),
     "catchq_conv2d_shortcut_workspace_size": (_I, [_I, _I, ctypes.POINTER(ConvDesc), ctypes.POINTER(Shortcut),

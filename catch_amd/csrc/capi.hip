@@ -50,8 +50,11 @@ int gemm_float(const void *x, bool half, int position, const void *w, int N_img,
                int Wo, const EpiDev &e, hipStream_t s);
 bool contract_small_float_ok(bool half, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw,
                              int dh, int dw, int Ho, int Wo, int cus);
-int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
-                         int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
+int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int x_ci, bool apart, int Ci,
+                         int Co, int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e,
+                         hipStream_t s);
+int contract_wide_float(const void *x, bool half, int position, const void *w, int N, int H, int W, int x_ci, bool apart, int Ci, int Co,
+                        int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s);
 struct ChainLinkDev {  // igemm_i8_chain.hip
   const int8_t *x, *w;
   unsigned x_bytes, w_bytes;
@@ -380,8 +383,8 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
     const int st2 =
         fusable == 2 ? gemm_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.stride_h, d.stride_w, ho,
                                   wo, e, as_stream(stream))
-                     : contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
-                                            d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
+                     : contract_small_float(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, d.ci, false, d.ci, d.co, d.kh, d.kw,
+                                            d.pad_h, d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
     if (st2 >= 0) return st2;
   }
   // two launches: the quantized activations go through the workspace
@@ -390,6 +393,27 @@ CATCHQ_API int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_positi
   st = catchq_quantize(x, x_dtype, workspace, 8, need, x_position, 1.0f, stream);
   if (st != CATCHQ_OK) return st;
   return catchq_conv2d_nhwc(workspace, 8, w, 8, desc, epilogue, stream);
+}
+
+CATCHQ_API int catchq_float_conv2d_small(const void *x, int x_dtype, int x_position, int x_ci, int x_nchw, const void *w, int w_bits,
+                                         const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  int ho, wo;
+  int st = check_conv(desc, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  if (w_bits != 8 && w_bits != 16) return CATCHQ_ERR_BITWIDTH;
+  st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  if (x_position < -126 || x_position > 126 || x_ci <= 0 || x_ci > desc->ci) return CATCHQ_ERR_ARG;
+  if (desc->n == 0) return CATCHQ_OK;
+  if (!x || !w) return CATCHQ_ERR_ARG;
+  if (desc->groups != 1 || (reinterpret_cast<uintptr_t>(x) & 3u) || !aligned16(w)) return CATCHQ_ERR_UNSUPPORTED;
+  const catchq_conv_desc_t &d = *desc;
+  const EpiDev e = make_epi(epilogue, (int64_t)d.n * ho * wo * d.co);
+  st = (w_bits == 8 ? contract_small_float : contract_wide_float)(x, x_dtype == CATCHQ_F16, x_position, w, d.n, d.h, d.w, x_ci, x_nchw != 0,
+                                                                  d.ci, d.co, d.kh, d.kw, d.pad_h, d.pad_w, d.stride_h, d.stride_w,
+                                                                  d.dil_h, d.dil_w, ho, wo, e, as_stream(stream));
+  return st < 0 ? CATCHQ_ERR_UNSUPPORTED : st;
 }
 
 CATCHQ_API int catchq_packed_filters_size(int64_t n, int64_t k, size_t *bytes) {

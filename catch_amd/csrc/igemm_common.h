@@ -715,6 +715,81 @@ __device__ __forceinline__ v4i quantize16(const v4i *raw, int neg_pos) {
   return q;
 }
 
+// What the kernels of few output tiles (small_i8.hip, wide_i16.hip) read beyond that: halfs whose rows start on any element, and
+// floats or halfs whose channels lie `chan_bytes` apart (NCHW).
+enum { IN_F16_ANY = 3, IN_F32_APART = 4, IN_F16_APART = 5 };
+constexpr bool in_apart(int in) { return in == IN_F32_APART || in == IN_F16_APART; }
+constexpr int in_bytes(int in) { return in == IN_I8 ? 1 : (in == IN_F32 || in == IN_F32_APART ? 4 : 2); }
+// loads per V values, and the dwords that hold them
+constexpr int in_loads(int in, int v) { return in_apart(in) ? v : in == IN_F16_ANY ? v / 8 + 1 : v * in_bytes(in) / 16; }
+constexpr int in_dwords(int in, int v) { return in_apart(in) ? v : in == IN_F16_ANY ? v / 2 + 1 : v * in_bytes(in) / 4; }
+
+// V values from byte `off` of a buffer on; an offset past its end gives zeros.
+template <int IN, int V>
+struct FloatPiece {
+  int d[in_dwords(IN, V)];
+  unsigned shift;  // IN_F16_ANY: bits in front of the first value
+  __device__ __forceinline__ void load(const __amdgpu_buffer_rsrc_t rsrc, unsigned off, unsigned chan_bytes) {
+    if constexpr (in_apart(IN)) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const int at = (int)(off + (unsigned)i * chan_bytes);
+        if constexpr (IN == IN_F32_APART) d[i] = (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, at, 0, 0);
+        else d[i] = (int)__builtin_amdgcn_raw_buffer_load_b16(rsrc, at, 0, 0);
+      }
+    } else {
+      constexpr int WIDE = in_dwords(IN, V) / 4;
+      if constexpr (IN == IN_F16_ANY) {  // whole dwords around the values
+        shift = (off & 2u) * 8u;
+        off &= ~3u;
+        d[4 * WIDE] = (int)__builtin_amdgcn_raw_buffer_load_b32(rsrc, (int)off + 16 * WIDE, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < WIDE; ++r) {
+        const v4i t = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)off + 16 * r, 0, 0));
+#pragma unroll
+        for (int u = 0; u < 4; ++u) d[4 * r + u] = t[u];
+      }
+    }
+  }
+  __device__ __forceinline__ float value(int i) const {
+    if constexpr (IN == IN_F32 || IN == IN_F32_APART) return __int_as_float(d[i]);
+    else if constexpr (IN == IN_F16_APART) return (float)__builtin_bit_cast(_Float16, (short)d[i]);
+    else {
+      int pair = d[i / 2];
+      if constexpr (IN == IN_F16_ANY) pair = (int)__builtin_amdgcn_alignbit((unsigned)d[i / 2 + 1], (unsigned)d[i / 2], shift);
+      return (float)__builtin_bit_cast(_Float16, (short)((i & 1) ? pair >> 16 : pair & 0xffff));
+    }
+  }
+};
+
+// 16 values -> 16 int8, 8 values -> 8 int16: the quantizer's own arithmetic with unit scale
+template <int IN>
+__device__ __forceinline__ v4i quantize_piece(const FloatPiece<IN, 16> &p, int neg_pos) {
+  v4i q;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    int b[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) b[t] = quant1_unit<8>(p.value(4 * d + t), neg_pos);
+    const unsigned lo = __builtin_amdgcn_perm((unsigned)b[1], (unsigned)b[0], 0x0c0c0400u);
+    const unsigned hi = __builtin_amdgcn_perm((unsigned)b[3], (unsigned)b[2], 0x04000c0cu);
+    q[d] = (int)(lo | hi);
+  }
+  return q;
+}
+template <int IN>
+__device__ __forceinline__ v4i quantize_piece(const FloatPiece<IN, 8> &p, int neg_pos) {
+  v4i q;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    const int a = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(p.value(2 * d), neg_pos)));
+    const int b = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(p.value(2 * d + 1), neg_pos)));
+    q[d] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pk_i16(a, b));  // (saturates)
+  }
+  return q;
+}
+
 // launchers of the LDS-DMA pipelined kernel (igemm_i8_dma.hip); return -1 when the shape is not
 // eligible (operand of 2 GiB or more, four-channel stem) and the caller takes the register-staged kernel
 int igemm_dma_launch(int load, const void *a, const void *b, IgemmParams p, const EpiDev &e, int64_t a_bytes,

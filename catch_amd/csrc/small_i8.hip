@@ -21,8 +21,9 @@ struct SmallSide {
   const void *x;
   const int8_t *w;
   int K;             // kh * kw * Ci < 2^20
-  int H, W, Ci, kw, ph, pw, sh, sw, dh, dw;
-  unsigned img_stride, row_stride, pix_stride;  // elements
+  int H, W, Ci, kw, ph, pw, sh, sw, dh, dw;  // Ci: channels of the filters; where the activations have fewer, those beyond read
+                                             // whatever lies there, against zeros
+  unsigned img_stride, row_stride, pix_stride, chan_stride;  // elements
   unsigned magic_ci, magic_kw, mask_ci, mask_kw;  // ceil(2^32 / d), mask 0; for d = 1 magic 0, mask ~0
   unsigned a_bytes, b_bytes;
 };
@@ -128,7 +129,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     const int m = m0 + j * 8 + lrow;
     if constexpr (DENSE) {
       a_hi[j] = a_wi[j] = 0;
-      a_base[j] = m < p.M ? (unsigned)m * (unsigned)o.K : OOB;
+      a_base[j] = m < p.M ? (unsigned)m * o.pix_stride : OOB;
     } else {
       const unsigned t = div_magic((unsigned)m, p.magic_wo, p.mask_wo), wo = (unsigned)m - t * (unsigned)p.Wo;
       const unsigned img = div_magic(t, p.magic_ho, p.mask_ho), ho = t - img * (unsigned)p.Ho;
@@ -145,10 +146,11 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   const int mine = per + (group_wave < rem ? 1 : 0);
   int8_t *const my = lds + wave * WAVE_BYTES;
 
-  constexpr int ES = IN == IN_F32 ? 4 : (IN == IN_F16 ? 2 : 1);  // bytes per activation
-  constexpr int RAW = ES;  // 16-byte loads per 16 activations
-  v4i raw[NA][RAW];
+  constexpr int ES = in_bytes(IN);          // bytes per activation
+  constexpr int RAW = in_loads(IN, 16);     // loads per 16 activations
+  FloatPiece<IN, 16> raw[NA];
   (void)raw;
+  const unsigned chan_bytes = in_apart(IN) ? o.chan_stride * (unsigned)ES : 0u;
   auto issue = [&](int s) {  // step s of this wave's slice into its slot s & 1 (floating activations: into raw)
     const int slot = (s & 1) * SLOT_BYTES;
     unsigned k[2], koff[2];
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
         const unsigned r = div_magic(tap, o.magic_kw, o.mask_kw), q = tap - r * (unsigned)o.kw;
         dy[h] = (int)r * o.dh;
         dx[h] = (int)q * o.dw;
-        koff[h] = (unsigned)dy[h] * o.row_stride + (unsigned)dx[h] * o.pix_stride + ci;
+        koff[h] = (unsigned)dy[h] * o.row_stride + (unsigned)dx[h] * o.pix_stride + (in_apart(IN) ? ci * o.chan_stride : ci);
       }
     }
     // (the filters first: loads complete in order, so a wave that has its activations has its filters)
@@ -188,9 +190,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       if constexpr (IN == IN_I8) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
       } else {
-#pragma unroll
-        for (int r = 0; r < RAW; ++r)
-          raw[j][r] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rsrc_a, (int)voff + 16 * r, 0, 0));
+        raw[j].load(rsrc_a, voff, chan_bytes);
       }
     }
   };
@@ -213,12 +213,12 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
         // would have left them; then the next step's loads
         v4i q[NA];
 #pragma unroll
-        for (int j = 0; j < NA; ++j) q[j] = quantize16<IN>(raw[j], p.x_neg_pos);
+        for (int j = 0; j < NA; ++j) q[j] = quantize_piece<IN>(raw[j], p.x_neg_pos);
 #pragma unroll
         for (int j = 0; j < NA; ++j)
           small_ds_write(my_addr + (unsigned)((s & 1) * SLOT_BYTES + j * 1024 + lane * 16), q[j]);
         issue(s + 1);
-        CATCHQ_SMALL_VMCNT(NA + NA * RAW);
+        CATCHQ_SMALL_VMCNT(NA + NA * RAW < 63 ? NA + NA * RAW : 63);  // (what the counter holds)
       }
       const unsigned base = a_addr + (unsigned)((s & 1) * SLOT_BYTES);
       v4i fa[SUB], fb[SUB];
@@ -336,12 +336,15 @@ static int launch_small(SmallParams p, const EpiDev &e, hipStream_t s) {
   return launch_status();
 }
 
-// One side's constants; false where the kernel's 32-bit arithmetic does not cover the shape.
+// One side's constants; false where the kernel's 32-bit arithmetic does not cover the shape.  x_ci: channels of the activations
+// (Ci and more of them make no sense), apart: their order is [N, channel, H, W].
 static bool small_side(SmallSide *o, const void *x, int x_size, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
-                       int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense) {
+                       int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense, int x_ci, bool apart) {
   const int64_t M = (int64_t)N_img * Ho * Wo, K = (int64_t)kh * kw * Ci;
-  const int64_t a_bytes = (int64_t)N_img * H * W * Ci * x_size, b_bytes = (int64_t)Co * K;
-  if (Ci % 16 != 0 || M >= (1 << 20) || K >= (1 << 20) || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31)) return false;
+  const int64_t a_bytes = ((int64_t)N_img * H * W * x_ci * x_size + 3) / 4 * 4, b_bytes = (int64_t)Co * K;  // (whole dwords)
+  // (no offset wraps: one past the last channel stays below 2^32, one of 2^31 and a piece's channels behind it too)
+  if (apart && (int64_t)H * W * x_size * (Ci - x_ci + 16) >= (1ll << 30)) return false;
+  if (Ci % 16 != 0 || x_ci > Ci || M >= (1 << 20) || K >= (1 << 20) || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31)) return false;
   // the divisions through multiplication: dividend * divisor < 2^32
   if (!dense && (M * Wo >= (1ll << 32) || M * Ho >= (1ll << 32) || K * Ci >= (1ll << 32) || (int64_t)kh * kw * kw >= (1ll << 32) ||
                  (int64_t)dh * kh >= (1 << 20) || (int64_t)dw * kw >= (1 << 20) || H >= (1 << 20) || W >= (1 << 20)))
@@ -349,7 +352,10 @@ static bool small_side(SmallSide *o, const void *x, int x_size, const void *w, i
   o->x = x; o->w = (const int8_t *)w;
   o->K = (int)K;
   o->H = H; o->W = W; o->Ci = Ci; o->kw = kw; o->ph = ph; o->pw = pw; o->sh = sh; o->sw = sw; o->dh = dh; o->dw = dw;
-  o->img_stride = (unsigned)((int64_t)H * W * Ci); o->row_stride = (unsigned)((int64_t)W * Ci); o->pix_stride = (unsigned)Ci;
+  o->img_stride = (unsigned)((int64_t)H * W * x_ci);
+  o->row_stride = (unsigned)(apart ? W : (int64_t)W * x_ci);
+  o->pix_stride = apart ? 1u : (unsigned)x_ci;
+  o->chan_stride = apart ? (unsigned)((int64_t)H * W) : 1u;
   magic(Ci, &o->magic_ci, &o->mask_ci);
   magic(kw, &o->magic_kw, &o->mask_kw);
   o->a_bytes = (unsigned)a_bytes; o->b_bytes = (unsigned)b_bytes;
@@ -416,7 +422,7 @@ int contract_small_i8(const void *x, const void *w, int N_img, int H, int W, int
   const int plan = small_plan(M, Co, (int64_t)kh * kw * Ci, dense, e.cus);
   if (!plan) return -1;
   SmallParams p = {};
-  if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense)) return -1;
+  if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, Ci, false)) return -1;
   small_common(&p, M, Co, Ho, Wo, e);
   return dense ? launch_small_plan<true, IN_I8, false>(plan, p, e, s) : launch_small_plan<false, IN_I8, false>(plan, p, e, s);
 }
@@ -432,8 +438,8 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
   const int plan = small_plan(M, Co, (int64_t)kh * kw * Ci + Cs, false, e.cus);
   if (!plan) return -1;
   SmallParams p = {};
-  if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false) ||
-      !small_side(&p.side[1], xs, 1, ws, N_img, Hs, Ws, Cs, Co, 1, 1, 0, 0, ss, ss, 1, 1, Ho, Wo, false))
+  if (!small_side(&p.side[0], x, 1, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, false, Ci, false) ||
+      !small_side(&p.side[1], xs, 1, ws, N_img, Hs, Ws, Cs, Co, 1, 1, 0, 0, ss, ss, 1, 1, Ho, Wo, false, Cs, false))
     return -1;
   EpiDev probe = e;
   probe.resid = reinterpret_cast<const float *>(e.y ? e.y : e.q);  // any 16-byte aligned non-null pointer
@@ -453,31 +459,53 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
 // (14x14 256 -> 256 3x3), four 4.6 / 5.3 (8 x 2048 x 1000), six 5.5 / 5.3 (1 x 3072 x 768), eight 9.8 / 7.0
 // (32 x 4096 x 3072), thirteen 16.2 / 9.4 (2 x 14x14 256 -> 256 5x5).  Float activations lie within 1 us of these.
 //
+// Activations whose channels lie apart ([N, channel, H, W]) cost a load a value, against a quantizer that transposes (a call's time, us,
+// two launches / one, 3 x 3 and 1 x 1 layers of 16 to 512 channels): 16 x 16 tiles on four waves, one step a wave 10.5 / 7.0, two 10.6 /
+// 7.1, three and four 10.6 / 7.8 to 10.0 with up to a tile per unit and 11 / 13 to 17 with two; on eight waves two 11.9 / 10.3, three
+// 11 / 12; 32 x 32 tiles one 10.5 / 6.8, two 11.8 / 9.1 up to a tile per unit, three 10.6 / 13.9.  Rows of any length in halfs, read in
+// whole dwords, lie within 1 us of aligned ones: linears of an unaligned K 9.2 / 5.6, pixels of padded channels 10 / 7.
+//
 // The plan (as small_plan) and the kernel's constants; 0: not the one launch.  The question and the launch ask it both.
 static int small_float_plan(SmallSide *o, const void *x, bool half, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
-                            int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense, int cus) {
+                            int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense, int x_ci, bool apart,
+                            int cus) {
   const int64_t K = (int64_t)kh * kw * Ci;
   const int plan = small_plan((int64_t)N_img * Ho * Wo, Co, K, dense, cus);
   if (!plan) return 0;
   const int waves = plan % 100;
   const int64_t per_wave = ((K + 127) / 128 + waves - 1) / waves;
-  if (per_wave > (plan / 100 == 32 ? 3 : 6)) return 0;
-  return small_side(o, x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense) ? plan : 0;
+  int most = plan / 100 == 32 ? 3 : 6;
+  if (apart) {
+    const int64_t M = (int64_t)N_img * Ho * Wo;
+    if (plan / 100 == 32) most = waves == 4 ? (((M + 31) / 32) * ((Co + 31) / 32) <= cus ? 2 : 1) : 0;
+    else most = waves == 4 && ((M + 15) / 16) * ((Co + 15) / 16) <= cus ? 4 : 2;
+  }
+  if (per_wave > most) return 0;
+  return small_side(o, x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, x_ci, apart) ? plan : 0;
 }
 bool contract_small_float_ok(bool half, int N_img, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw, int sh, int sw,
                              int dh, int dw, int Ho, int Wo, int cus) {
   SmallSide o;
   const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-  return small_float_plan(&o, nullptr, half, nullptr, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, cus) != 0;
+  return small_float_plan(&o, nullptr, half, nullptr, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, Ci, false,
+                          cus) != 0;
 }
-int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
-                         int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
-  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+// x_ci channels in the activations, Ci in the filters (a multiple of 16, zeros where the activations have none); apart: [N, channel,
+// H, W] activations.  Halfs of rows that start on any element are read in whole dwords and shifted.
+int contract_small_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int x_ci, bool apart, int Ci,
+                         int Co, int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e,
+                         hipStream_t s) {
+  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && !apart;
   SmallParams p = {};
-  const int plan = small_float_plan(&p.side[0], x, half, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, e.cus);
+  const int plan = small_float_plan(&p.side[0], x, half, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, x_ci,
+                                    apart, e.cus);
   if (!plan) return -1;
   small_common(&p, (int64_t)N_img * Ho * Wo, Co, Ho, Wo, e);
   p.x_neg_pos = -position;
+  if (apart)
+    return half ? launch_small_plan<false, IN_F16_APART, false>(plan, p, e, s) : launch_small_plan<false, IN_F32_APART, false>(plan, p, e, s);
+  if (half && x_ci % 2 != 0)
+    return dense ? launch_small_plan<true, IN_F16_ANY, false>(plan, p, e, s) : launch_small_plan<false, IN_F16_ANY, false>(plan, p, e, s);
   if (half) return dense ? launch_small_plan<true, IN_F16, false>(plan, p, e, s) : launch_small_plan<false, IN_F16, false>(plan, p, e, s);
   return dense ? launch_small_plan<true, IN_F32, false>(plan, p, e, s) : launch_small_plan<false, IN_F32, false>(plan, p, e, s);
 }

@@ -1272,10 +1272,24 @@ const void *conv3x3_packed(Prepared &prep, const catchq_conv_desc_t &d, const ca
   return packed_weight(prep, [&] { return catchq_conv3x3_i8_packed_takes(d.n, d.h, d.w, d.ci, d.co, &e) == CATCHQ_OK; });
 }
 
-// quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x) x prepared weight -> floating
-// output, logical [N,Co,Ho,Wo] over NHWC memory
-Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Prepared &prep, const Tensor &bias,
-                     at::IntArrayRef padding, at::IntArrayRef stride, at::IntArrayRef dilation, int64_t groups, bool half) {
+// The layer on floating activations in one launch, channels-last or contiguous, the channels that only the filters have left out;
+// false: another route serves it.
+bool conv_small(const Tensor &x, const Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e) {
+  if (prep.bw_x != prep.bw_w || d.groups != 1) return false;
+  const bool rows = x.is_contiguous(at::MemoryFormat::ChannelsLast);
+  if (!rows && !x.is_contiguous()) return false;
+  const int dt = x.scalar_type() == at::kHalf ? CATCHQ_F16 : CATCHQ_F32;
+  const int st = catchq_float_conv2d_small(x.data_ptr(), dt, prep.pos_x, (int)x.size(1), rows ? 0 : 1, prep.qw.data_ptr(), prep.bw_w, &d,
+                                           &e, current_stream());
+  if (st == CATCHQ_ERR_UNSUPPORTED) return false;
+  check_status(st, "torch_mlu::conv2d");
+  return true;
+}
+
+// quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x, or those of `input`, whose order and
+// channel count may differ) x prepared weight -> floating output, logical [N,Co,Ho,Wo] over NHWC memory
+Tensor conv_prepared(Tensor qx, const void *x, at::IntArrayRef x_nhwc, Prepared &prep, const Tensor &bias, at::IntArrayRef padding,
+                     at::IntArrayRef stride, at::IntArrayRef dilation, int64_t groups, bool half, const Tensor *input = nullptr) {
   TORCH_CHECK(padding.size() == 2 && stride.size() == 2 && dilation.size() == 2, "2-d conv parameters expected");
   const Tensor &qw = prep.qw;  // [Co,Ci/g,kh,kw] over [Co][kh][kw][Ci/g] memory
   TORCH_CHECK(groups > 0 && x_nhwc[3] == qw.size(1) * groups, "channel mismatch: input ", x_nhwc[3], ", weight ", qw.size(1),
@@ -1292,6 +1306,10 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Pr
   if (d.n == 0 || d.co == 0) return y;  // nothing to compute: the empty output is the result
   Tensor keep;
   const catchq_epilogue_t e = prepared_epilogue(prep, bias, d.co, y, &keep);
+  if (input && !x) {
+    if (conv_small(*input, prep, d, e)) return y;
+    qx = quantize_to_nhwc(*input, prep.bw_x, prep.pos_x, d.ci);
+  }
   if (qx.defined()) {
     if (const void *packed = conv3x3_packed(prep, d, e)) {
       const int st = catchq_conv3x3_i8_packed(qx.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
@@ -1311,7 +1329,8 @@ Tensor conv_prepared(const Tensor &qx, const void *x, at::IntArrayRef x_nhwc, Pr
                         : linear_packed(x, dt, prep, m, d.co, d.ci, e, "torch_mlu::conv2d"))
       return y;
   }
-  if (prep.bw_x == 16) {  // no single launch takes these: the quantized activations of all channels
+  if (prep.bw_x == 16) {
+    if (input && conv_small(*input, prep, d, e)) return y;
     Tensor qn = device_empty({d.n, d.h, d.w, d.ci}, int_type(16), qw.device());
     check_status(catchq_quantize(x, dt, qn.data_ptr(), 16, (int64_t)d.n * d.h * d.w * d.ci, prep.pos_x, 1.0f, current_stream()),
                  "torch_mlu::quantize");
@@ -1371,27 +1390,27 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
     // the memory of a channels-last [Co,Ci/g,kh,kw] tensor is [Co][kh][kw][Ci/g]
     return wd.contiguous(at::MemoryFormat::ChannelsLast);
   }, (few ? 1 : 0) | (can_frame ? 2 : 0));
-  Tensor qx;
-  if (input.is_contiguous(at::MemoryFormat::ChannelsLast) &&
-      ((prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0) ||
-       (prep->bw_x == 16 && prep->bw_w == 16 && ci % 8 == 0 && dense && kw == 1 && weight.size(2) == 1)))
-    return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), input.size(2), input.size(3), ci}, *prep, bias, padding, stride,
-                         dilation, groups, half);
+  const int64_t h = input.size(2), w_in = input.size(3), cdev = device_channels(prep->bw_x);
+  if (input.is_contiguous(at::MemoryFormat::ChannelsLast)) {
+    const bool one_by_one = kw == 1 && weight.size(2) == 1;
+    if (prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0)
+      return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), h, w_in, ci}, *prep, bias, padding, stride, dilation, groups, half);
+    if (prep->bw_x == 16 && prep->bw_w == 16 && ci % 8 == 0 && dense && one_by_one)
+      return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), h, w_in, ci}, *prep, bias, padding, stride, dilation, groups, half,
+                           &input);
+  }
   if (few && prep->bw_x == 8 && can_frame) {
     const Tensor xc = input.contiguous();
-    const int64_t h = input.size(2), w_in = input.size(3);
-    qx = device_empty({input.size(0), h + 2 * padding[0], w_in + 2 * padding[1] + kw_extra, 4}, at::kChar, input.device());
+    Tensor qx = device_empty({input.size(0), h + 2 * padding[0], w_in + 2 * padding[1] + kw_extra, 4}, at::kChar, input.device());
     check_status(catchq_quantize_nchw_to_nhwc_frame(xc.data_ptr(), half ? CATCHQ_F16 : CATCHQ_F32, qx.data_ptr(), 8,
                                                     (int)input.size(0), (int)ci, (int)h, (int)w_in, 4, (int)qx.size(1),
                                                     (int)qx.size(2), (int)padding[0], (int)padding[1], prep->pos_x, 1.0f,
                                                     current_stream()),
                  "torch_mlu::quantize");
     return conv_prepared(qx, nullptr, qx.sizes(), *prep, bias, {0, 0}, stride, dilation, groups, half);
-  } else {
-    qx = quantize_to_nhwc(input, prep->bw_x, prep->pos_x, device_channels(prep->bw_x));
   }
   // logical NCHW over channels-last memory, like the reference
-  return conv_prepared(qx, nullptr, qx.sizes(), *prep, bias, padding, stride, dilation, groups, half);
+  return conv_prepared(Tensor(), nullptr, {input.size(0), h, w_in, cdev}, *prep, bias, padding, stride, dilation, groups, half, &input);
 }
 
 // [N,C,L] x [Co,Ci/g,k]: a convolution over images of one row (the reference's module calls
@@ -1541,6 +1560,16 @@ Tensor linear_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   }
   // (rows of the packed weights end in zeros where kd > k)
   if (linear_digits(xc.data_ptr(), dt, *prep, m, n, k, e, input.device(), "torch_mlu::linear")) return y;
+  // few rows or columns: quantized on the way into the product, rows of any length and alignment of their elements
+  if (prep->bw_x == prep->bw_w && (kd != k || prep->bw_x == 16) && k > 0 && m < (1ll << 31) && n < (1ll << 31)) {
+    const catchq_conv_desc_t d = {(int)m, 1, 1, (int)kd, (int)n, 1, 1, 0, 0, 1, 1, 1, 1, 1};
+    const int st = catchq_float_conv2d_small(xc.data_ptr(), dt, prep->pos_x, (int)k, 0, prep->qw.data_ptr(), prep->bw_w, &d, &e,
+                                             current_stream());
+    if (st != CATCHQ_ERR_UNSUPPORTED) {
+      check_status(st, "torch_mlu::linear");
+      return y;
+    }
+  }
   // (as many rows at a time as an operand of the matrix-core routes may have, 2^31 bytes: padding makes no product a slower
   // route's)
   const int64_t row_bytes = std::max<int64_t>(kd, 1) * (prep->bw_x / 8);

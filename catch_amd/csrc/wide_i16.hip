@@ -32,10 +32,12 @@ typedef __attribute__((address_space(3))) void *lds_ptr_t;
 typedef double v2d __attribute__((ext_vector_type(2)));
 
 struct WideParams {
-  const int16_t *x, *w;
+  const void *x;  // int16, or floats that the loader quantizes
+  const int16_t *w;
   int M, N, K;  // K < 2^16
   int H, W, Ci, Ho, Wo, kw, ph, pw, sh, sw, dh, dw;
-  unsigned img_stride, row_stride, pix_stride;  // elements
+  unsigned img_stride, row_stride, pix_stride, chan_stride;  // elements
+  int x_neg_pos;      // floating activations: quantized at 2^-x_neg_pos
   unsigned magic_ci, magic_kw, mask_ci, mask_kw;  // ceil(2^32 / d), mask 0; for d = 1 magic 0, mask ~0
   int tiles_m, tiles_n, nblocks;
   int m_fastest;  // consecutive blocks walk the row tiles of one column tile first
@@ -54,7 +56,7 @@ __device__ __forceinline__ v4i wide_ds_read(unsigned addr) {
   return v;
 }
 
-template <int TM, int TN, int NW, bool DENSE>
+template <int TM, int TN, int NW, bool DENSE, int IN>
 __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev e) {
   resolve_exp2(e);
   constexpr int BM = TM * 32, BN = TN * 32;
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
     if constexpr (DENSE) {
       a_hi[j] = m < p.M ? 0 : -1;
       a_wi[j] = 0;
-      a_base[j] = (unsigned)m * (unsigned)p.K;
+      a_base[j] = (unsigned)m * p.pix_stride;
     } else {
       const unsigned t = (unsigned)m / (unsigned)p.Wo, wo = (unsigned)m - t * (unsigned)p.Wo;
       const unsigned img = t / (unsigned)p.Ho, ho = t - img * (unsigned)p.Ho;
@@ -114,10 +116,16 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
 #pragma unroll
   for (int j = 0; j < NB; ++j) b_off[j] = b_base[j] != OOB ? 2u * (b_base[j] + (unsigned)((chunk0 ^ (4 * (j & 1))) * 8)) : OOB;
 
+  constexpr int ES = IN == IN_I8 ? 2 : in_bytes(IN);  // bytes per activation (IN_I8: integers as they are, of 16 bits)
+  FloatPiece<IN, 8> raw[NA];
+  (void)raw;
+  const unsigned chan_bytes = in_apart(IN) ? p.chan_stride * (unsigned)ES : 0u;
+  (void)chan_bytes;
+
   auto issue = [&](int s) {
     const int slot = (s & 1) * SLOT_BYTES;
     const bool full = (first + s + 1) * KS <= p.K;
-    if (DENSE && full) {
+    if (DENSE && IN == IN_I8 && full) {
       const int step = (first + s) * (KS * 2);
 #pragma unroll
       for (int j = 0; j < NA; ++j)
@@ -141,27 +149,34 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
         const unsigned r = wide_div(tap, p.magic_kw, p.mask_kw), q = tap - r * (unsigned)p.kw;
         dy[h] = (int)r * p.dh;
         dx[h] = (int)q * p.dw;
-        koff[h] = (unsigned)dy[h] * p.row_stride + (unsigned)dx[h] * p.pix_stride + ci;
+        koff[h] = (unsigned)dy[h] * p.row_stride + (unsigned)dx[h] * p.pix_stride + (in_apart(IN) ? ci * p.chan_stride : ci);
       }
     }
+    const int step = (first + s) * (KS * 2);
+    auto filters = [&] {
+#pragma unroll
+      for (int j = 0; j < NB; ++j) {
+        unsigned voff = ok[j & 1] ? b_off[j] + (unsigned)step : OOB;
+        voff = b_off[j] == OOB ? OOB : voff;
+        asm volatile("" : "+v"(voff));
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(my + slot + (NA + j) * 1024), 16, (int)voff, 0, 0, 0);
+      }
+    };
+    // (in front of floating activations: loads complete in order, so a wave that has those has its filters)
+    if constexpr (IN != IN_I8) filters();
 #pragma unroll
     for (int j = 0; j < NA; ++j) {
       const int h = j & 1;
       bool in = ok[h];
       if constexpr (DENSE) in = in & (a_hi[j] == 0);
       else in = in & ((unsigned)(a_hi[j] + dy[h]) < (unsigned)p.H) & ((unsigned)(a_wi[j] + dx[h]) < (unsigned)p.W);
-      unsigned voff = in ? 2u * (a_base[j] + koff[h]) : OOB;
+      unsigned voff = in ? (unsigned)ES * (a_base[j] + koff[h]) : OOB;
       asm volatile("" : "+v"(voff));  // one select and one load, not two loads under complementary masks
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
+      if constexpr (IN == IN_I8)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
+      else raw[j].load(rsrc_a, voff, chan_bytes);
     }
-    const int step = (first + s) * (KS * 2);
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      unsigned voff = ok[j & 1] ? b_off[j] + (unsigned)step : OOB;
-      voff = b_off[j] == OOB ? OOB : voff;
-      asm volatile("" : "+v"(voff));
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_b, (lds_ptr_t)(my + slot + (NA + j) * 1024), 16, (int)voff, 0, 0, 0);
-    }
+    if constexpr (IN == IN_I8) filters();
   };
 
   // ---- K loop --------------------------------------------------------------------------------------------------------
@@ -234,10 +249,22 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
   double *const row_part = reinterpret_cast<double *>(lds + NW * WAVE_BYTES) + wave * BM;  // [BM]
   if (mine > 0) {
     issue(0);
-    if (mine > 1) issue(1);
+    if (IN == IN_I8 && mine > 1) issue(1);
     for (int s = 0; s < mine; ++s) {
-      if (s + 1 < mine) CATCHQ_WIDE_VMCNT(NI);
-      else CATCHQ_WIDE_VMCNT(0);
+      if constexpr (IN == IN_I8) {
+        if (s + 1 < mine) CATCHQ_WIDE_VMCNT(NI);
+        else CATCHQ_WIDE_VMCNT(0);
+      } else {
+        // the step's activations, quantized into the slot as a transfer would have left them; its filters came before them
+        v4i q[NA];
+#pragma unroll
+        for (int j = 0; j < NA; ++j) q[j] = quantize_piece<IN>(raw[j], p.x_neg_pos);
+        CATCHQ_WIDE_VMCNT(0);
+        const unsigned to = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t *)my + (unsigned)((s & 1) * SLOT_BYTES + lane * 16);
+#pragma unroll
+        for (int j = 0; j < NA; ++j) asm volatile("ds_write_b128 %0, %1" ::"v"(to + (unsigned)(j * 1024)), "v"(q[j]) : "memory");
+        if (s + 1 < mine) issue(s + 1);
+      }
       const unsigned base = row_addr + (unsigned)((s & 1) * SLOT_BYTES);
       Frags f0, f1;
       fetch(f0, base, 0);
@@ -245,7 +272,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
       fetch(f1, base, 1);  // under the first half's arithmetic
       multiply(f0);
       arrived(f1);
-      if (s + 2 < mine) issue(s + 2);  // the slot has been read
+      if (IN == IN_I8 && s + 2 < mine) issue(s + 2);  // the slot has been read
       multiply(f1);
     }
     // a lane holds the digit sums of row (lane & 31) over its half of every K step: add the halves
@@ -329,10 +356,10 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
   }
 }
 
-template <int TM, int TN, int NW, bool DENSE>
+template <int TM, int TN, int NW, bool DENSE, int IN = IN_I8>
 static int launch_wide(WideParams p, const EpiDev &e, hipStream_t s) {
   constexpr int LDS_BYTES = NW * (2 * (TM + TN) * 32 * 128 + TM * 32 * 8);
-  auto kern = wide_i16_kernel<TM, TN, NW, DENSE>;
+  auto kern = wide_i16_kernel<TM, TN, NW, DENSE, IN>;
   if (LDS_BYTES > 64 * 1024) {
     static std::atomic<bool> raised[64];
     if (raise_lds_limit((const void *)kern, LDS_BYTES, raised) != CATCHQ_OK) return CATCHQ_ERR_LAUNCH;
@@ -362,20 +389,25 @@ static int pick_wide(const WideParams &p, const EpiDev &e, hipStream_t s) {
   }
 }
 
-// int16 x int16; -1 when the shape is not eligible (or an int32 accumulator output is asked for: the exact sum has 64 bits)
-int conv2d_mfma_a16w16(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
-                       int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
+// The kernel's constants; false where its arithmetic does not cover the shape.  x_ci channels of x_size bytes in the activations, Ci in
+// the filters; apart: activations in the order [N, channel, H, W].
+static bool wide_params(WideParams *q, const void *x, int x_size, const void *w, int N, int H, int W, int x_ci, bool apart, int Ci, int Co,
+                        int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, bool dense, const EpiDev &e) {
   const int64_t M = (int64_t)N * Ho * Wo, K = (int64_t)kh * kw * Ci;
-  const int64_t a_bytes = (int64_t)N * H * W * Ci * 2, b_bytes = (int64_t)Co * K * 2;
-  if (Ci % 8 != 0 || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31) || a_bytes <= 0 || b_bytes <= 0 || e.acc_out) return -1;
-  if (M >= (1ll << 31) - 64 || K >= (1 << 16) || (int64_t)kh * kw * kw >= (1ll << 31)) return -1;
-  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-  if (!dense && (H >= (1 << 20) || W >= (1 << 20) || (int64_t)dh * kh >= (1 << 20) || (int64_t)dw * kw >= (1 << 20))) return -1;
-  WideParams p = {};
-  p.x = (const int16_t *)x; p.w = (const int16_t *)w;
+  const int64_t a_bytes = ((int64_t)N * H * W * x_ci * x_size + 3) / 4 * 4, b_bytes = (int64_t)Co * K * 2;
+  if (Ci % 8 != 0 || x_ci > Ci || a_bytes >= (1ll << 31) || b_bytes >= (1ll << 31) || a_bytes <= 0 || b_bytes <= 0 || e.acc_out) return false;
+  if (apart && (int64_t)H * W * x_size * (Ci - x_ci + 16) >= (1ll << 30)) return false;  // (no offset wraps)
+  if (M >= (1ll << 31) - 64 || K >= (1 << 16) || (int64_t)kh * kw * kw >= (1ll << 31)) return false;
+  if (!dense && (H >= (1 << 20) || W >= (1 << 20) || (int64_t)dh * kh >= (1 << 20) || (int64_t)dw * kw >= (1 << 20))) return false;
+  WideParams &p = *q;
+  p = {};
+  p.x = x; p.w = (const int16_t *)w;
   p.M = (int)M; p.N = Co; p.K = (int)K;
   p.H = H; p.W = W; p.Ci = Ci; p.Ho = Ho; p.Wo = Wo; p.kw = kw; p.ph = ph; p.pw = pw; p.sh = sh; p.sw = sw; p.dh = dh; p.dw = dw;
-  p.img_stride = (unsigned)((int64_t)H * W * Ci); p.row_stride = (unsigned)((int64_t)W * Ci); p.pix_stride = (unsigned)Ci;
+  p.img_stride = (unsigned)((int64_t)H * W * x_ci);
+  p.row_stride = (unsigned)(apart ? W : (int64_t)W * x_ci);
+  p.pix_stride = apart ? 1u : (unsigned)x_ci;
+  p.chan_stride = apart ? (unsigned)((int64_t)H * W) : 1u;
   auto magic = [](unsigned d, unsigned *m, unsigned *mask) {  // dividends below 2^16: exact for every divisor below 2^16
     *m = d <= 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d);
     *mask = d <= 1 ? ~0u : 0u;
@@ -390,7 +422,47 @@ int conv2d_mfma_a16w16(const void *x, const void *w, int N, int H, int W, int Ci
     if (epi != EPI_SCALAR) { p.epi = epi; p.ragged = 1; }
   }
   p.a_bytes = (unsigned)a_bytes; p.b_bytes = (unsigned)b_bytes;
+  return true;
+}
+
+// int16 x int16; -1 when the shape is not eligible (or an int32 accumulator output is asked for: the exact sum has 64 bits)
+int conv2d_mfma_a16w16(const void *x, const void *w, int N, int H, int W, int Ci, int Co, int kh, int kw, int ph, int pw,
+                       int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
+  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+  WideParams p;
+  if (!wide_params(&p, x, 2, w, N, H, W, Ci, false, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, e)) return -1;
   return dense ? pick_wide<true>(p, e, s) : pick_wide<false>(p, e, s);
+}
+
+template <bool DENSE, int IN>
+static int launch_wide_float(int waves, const WideParams &p, const EpiDev &e, hipStream_t s) {
+  return waves == 4 ? launch_wide<1, 1, 4, DENSE, IN>(p, e, s) : launch_wide<1, 1, 2, DENSE, IN>(p, e, s);
+}
+
+// Floating activations with int16 filters in one launch; -1: another route.  Arguments as contract_small_float's (Ci a multiple of 8).
+//
+// Every block converts its rows again, so the one launch pays while a wave has few K steps of 64 and the device few tiles (a call's time,
+// us, two launches / one): 32 x 32 tiles on four waves, up to one per unit, one step a wave 9.2 / 5.6 (linears), two 9.2 / 5.7, four 9.1 /
+// 7.1, five 10.9 / 9.3 (3 x 3), six 9.7 / 8.4, seven 10.2 / 10.0, eight and more 12 / 14; up to two per unit three 9.5 / 8.0, four 10.6 / 9.7, seven
+// 14.6 / 15.4; on two waves up to four per unit one 9.4 / 6.0, two 9.4 / 7.4, three 10.0 / 9.3, four 11.0 / 10.8; up to eight per unit two 12.4 / 15.7.
+// Channels that lie apart: two steps 10.2 / 7.1, three 10.4 / 9.0, four 10.4 / 10.2, up to two tiles per unit two 10 / 8, three 11 / 15;
+// on two waves one 13 / 9, two 14.4 / 15.
+int contract_wide_float(const void *x, bool half, int position, const void *w, int N, int H, int W, int x_ci, bool apart, int Ci, int Co,
+                        int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, const EpiDev &e, hipStream_t s) {
+  const bool dense = kh == 1 && kw == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0 && !apart;
+  const int64_t M = (int64_t)N * Ho * Wo, tiles = (M + 31) / 32 * ((Co + 31) / 32);
+  const int64_t steps = ((int64_t)kh * kw * Ci + 63) / 64;
+  const int waves = tiles >= 2 * e.cus ? 2 : 4;
+  const int most = apart ? (waves == 2 ? 1 : tiles <= e.cus ? 3 : 2) : (waves == 2 ? 3 : tiles <= e.cus ? 6 : 4);
+  if (tiles > 4 * e.cus || (steps + waves - 1) / waves > most) return -1;
+  WideParams p;
+  if (!wide_params(&p, x, half ? 2 : 4, w, N, H, W, x_ci, apart, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, e)) return -1;
+  p.x_neg_pos = -position;
+  if (apart) return half ? launch_wide_float<false, IN_F16_APART>(waves, p, e, s) : launch_wide_float<false, IN_F32_APART>(waves, p, e, s);
+  if (half && x_ci % 2 != 0)
+    return dense ? launch_wide_float<true, IN_F16_ANY>(waves, p, e, s) : launch_wide_float<false, IN_F16_ANY>(waves, p, e, s);
+  if (half) return dense ? launch_wide_float<true, IN_F16>(waves, p, e, s) : launch_wide_float<false, IN_F16>(waves, p, e, s);
+  return dense ? launch_wide_float<true, IN_F32>(waves, p, e, s) : launch_wide_float<false, IN_F32>(waves, p, e, s);
 }
 
 int gemm_nt_mfma_a16w16(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e, hipStream_t s) {

@@ -257,6 +257,13 @@ int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_position, const v
                              const catchq_epilogue_t *epilogue, void *workspace, size_t workspace_bytes,
                              catchq_stream_t stream);
 
+/* The same in one launch or not at all (CATCHQ_ERR_UNSUPPORTED: quantizing and catchq_conv2d_nhwc serve the call, as they do every
+ * one), and for more operands: filters of w_bits 8 or 16, the activations quantized at as many; activations of fewer channels than the
+ * filters (x_ci of desc->ci, a multiple of 16 resp. 8; the filters hold zeros beyond x_ci); x_nchw: activations [n,x_ci,h,w].  x on 4
+ * bytes. */
+int catchq_float_conv2d_small(const void *x, int x_dtype, int x_position, int x_ci, int x_nchw, const void *w, int w_bits,
+                              const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, catchq_stream_t stream);
+
 /* The same for a linear (a pointwise convolution of unit stride: m pixels) whose int8 filters were laid out once in the order
  * of the matrix instruction: catchq_pack_filters writes catchq_packed_filters_size bytes from w [n,k], k a multiple of 16.
  * x [m,k] fp32/fp16, y [m,n].  CATCHQ_ERR_UNSUPPORTED: catchq_float_conv2d_nhwc on the filters as they are serves the call

@@ -46,3 +46,43 @@ def test_channels_last_input_with_padded_channels(n, ci, h, w, co, k, stride, mo
     other = x.transpose(2, 3).contiguous().transpose(2, 3)     # neither order
     for given in (rows, shifted, other):
         assert torch.equal(torch.ops.torch_mlu.conv2d(given, *args), want)
+
+
+# tiles of 16 and of 32, K over four and eight waves, in one launch and (the last) in two; halfs that start on odd elements
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
+@pytest.mark.parametrize("n,ci,h,w,co,k,stride", [
+    (1, 16, 5, 5, 17, 1, 1), (1, 33, 9, 9, 40, 3, 1), (2, 100, 14, 14, 100, 3, 1), (1, 301, 7, 7, 65, 3, 2), (1, 512, 7, 7, 64, 3, 1),
+    (3, 47, 33, 29, 70, 3, 1), (2, 64, 40, 40, 130, 1, 2), (16, 64, 20, 20, 64, 3, 1), (1, 20, 60, 60, 33, 5, 1),
+])
+def test_layers_of_few_tiles_against_the_oracle(n, ci, h, w, co, k, stride, mode, dtype):
+    from oracle import ops as oops
+    x, wt, b, (scale, qm) = _layer(n, ci, h, w, co, k, dtype, mode)
+    args = ([k // 2, k // 2], [stride, stride], [1, 1], 1)
+    want = torch.from_numpy(oops.conv2d(x.cpu().numpy(), wt.cpu().numpy(), b.cpu().numpy(), *[tuple(a) for a in args[:3]], 1,
+                                        scale.cpu().numpy(), qm.cpu().numpy())["y"]).cuda()
+    for given in (x, x.contiguous(memory_format=torch.channels_last)):
+        got = torch.ops.torch_mlu.conv2d(given, wt, b, *args, scale, qm)
+        assert got.dtype == dtype and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("mode", [1, 2, 3, 4])
+@pytest.mark.parametrize("m,k,n", [
+    (1, 65, 64), (3, 97, 100), (17, 130, 33), (64, 301, 257), (500, 1001, 65), (37, 2303, 500), (129, 64, 4100), (1000, 90, 700),
+    (40, 128, 64), (5, 1536, 30),
+])
+def test_linears_of_few_tiles_against_the_oracle(m, k, n, mode, dtype):
+    from oracle import ops as oops
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    x = torch.randn(m, k, generator=gen, device="cuda").to(dtype)
+    x.view(-1)[-3:] = torch.tensor([math.inf, -math.inf, math.nan], device="cuda")  # at the buffer's very end
+    w = (torch.randn(n, k, generator=gen, device="cuda") / math.sqrt(k)).to(dtype)
+    b = torch.randn(n, generator=gen, device="cuda").to(dtype)
+    scale, qm = _qparams(x, w, mode)
+    want = torch.from_numpy(oops.linear(x.cpu().numpy(), w.cpu().numpy(), b.cpu().numpy(), scale.cpu().numpy(), qm.cpu().numpy())["y"]).cuda()
+    assert torch.equal(torch.ops.torch_mlu.linear(x, w, b, scale, qm), want)
+    whole = torch.zeros(m * k + 3, dtype=dtype, device="cuda")
+    for start in (1, 2):  # on an element's alignment, on a dword's
+        whole[start:start + m * k] = x.reshape(-1)
+        assert torch.equal(torch.ops.torch_mlu.linear(whole[start:start + m * k].view(m, k), w, b, scale, qm), want)
