@@ -102,9 +102,11 @@ def layer_profile(fused, x, iters=20, only=None):
     for pname, (bx, bd) in fused.block_of.items():
         if fused.block_fuses(next(l for l in fused.layers if l.name == pname), *trace[bx.name]["qx"].shape[:3]):
             fused_inner.update((bx.name, bd.name))
+    fused_expansions = set(bx.name for d, bx in fused.expansion_of.items() if d not in fused_inner and fused.expansion_fuses(
+        next(l for l in fused.layers if l.name == d), *trace[bx.name]["qx"].shape[:3]))
     first = fused.first_layers_fuse(*x.shape)  # quantizer, first convolution and pooling in one launch
     for l in fused.layers:
-        if l.kind not in ("conv", "fc") or l.name in fused._fused_away or l.name in fused_heads or l.name in fused_inner \
+        if l.kind not in ("conv", "fc") or l.name in fused._fused_away or l.name in fused_heads or l.name in fused_inner or l.name in fused_expansions \
                 or (only and l.name != only):
             continue
         if first and l is fused.layers[0]:
@@ -167,6 +169,18 @@ def layer_profile(fused, x, iters=20, only=None):
                                        dq.exp2, dq.chan_div, dq.bias, code[bd.act], lq.pos_x, lq.qw, lq.exp2, lq.chan_div,
                                        lq.bias, resid, want_y, y_half, qd[0] if qd else 0, qd[1] if qd else 0, 1.0)
             route = "mfma+block"
+        elif l.kind == "conv" and l.name in fused.expansion_of and fused.expansion_of[l.name].name in fused_expansions:
+            # the expansion runs inside this depthwise layer's launch: its input and filters are read, its output never stored
+            bx = fused.expansion_of[l.name]
+            xq, hx, resid = fused.q[bx.name], trace[bx.name]["qx"], None
+            extra_macs = trace[bx.name]["y"].numel() * xq.qw.shape[-1]
+            extra_bytes = hx.numel() + xq.qw.numel() - qx.numel()
+
+            def run(l=l, lq=lq, xq=xq, hx=hx, bx=bx, qd=qd):
+                code = {"relu": 1, "relu6": 2}
+                return None, ops.qconv2d_expand_dw(hx, xq.qw, xq.exp2, xq.chan_div, xq.bias, code[bx.act], lq.pos_x, lq.qw, l.stride,
+                                                   lq.exp2, lq.chan_div, lq.bias, code[l.act], qd[1])
+            route = "mfma+expansion"
         elif head is not None and head.name in fused_heads:
             # the 1x1 layer in front runs inside this launch: its input and filters are read, its output never stored
             hq = fused.q[head.name]
@@ -281,6 +295,9 @@ def plan_launches(fused, n, h, w):
                 bp = next(m for m in fused.layers if m.name == fused._block_inner[l.name])
                 if fused.block_fuses(bp, n, *shape[fused.block_of[bp.name][0].src]):
                     continue
+            if l.name in fused._expansion_names and fused.expansion_fuses(
+                    next(m for m in fused.layers if fused.expansion_of.get(m.name) is l), n, hi, wi):
+                continue  # inside the launch of the depthwise layer behind it
             lq = fused.q[l.name]
             n_out = n * ho * wo * fused.cdev[l.name]
             ih, iw = shape[("input", "q")] if (fused.stem and l.name == fused.stem["name"]) else (hi, wi)
@@ -294,6 +311,11 @@ def plan_launches(fused, n, h, w):
                 hq = fused.q[head.name]
                 macs += n * hi * wi * fused.cdev[head.name] * hq.qw.shape[-1]
                 b += n * hi * wi * (fused.cdev[head.src] - fused.cdev[l.src]) + hq.qw.numel()
+            expansion = fused.expansion_of.get(l.name)
+            if expansion is not None and fused.expansion_fuses(l, n, hi, wi):
+                xq = fused.q[expansion.name]
+                macs += n * hi * wi * fused.cdev[expansion.name] * xq.qw.shape[-1]
+                b += n * hi * wi * (fused.cdev[expansion.src] - fused.cdev[l.src]) + xq.qw.numel()
             block = fused.block_of.get(l.name)
             if block is not None and fused.block_fuses(l, n, *shape[block[0].src]):
                 bx, bd = block
@@ -616,6 +638,10 @@ def main():
               "fused_blocks": sorted(n for n, (bx, bd) in fused.block_of.items()
                                      if fused.block_fuses(next(l for l in fused.layers if l.name == n), batch // args.streams,
                                                           *head_hw(fused, bx, side))),
+              # depthwise layers whose launch also computes the 1x1 expansion in front of them
+              "fused_expansions": sorted(d for d, bx in fused.expansion_of.items()
+                                         if fused.expansion_fuses(next(l for l in fused.layers if l.name == d), batch // args.streams,
+                                                                  *head_hw(fused, bx, side))),
               # input quantizer, first convolution and max pooling in one launch
               "fused_first_layers": fused.first_layers_fuse(batch // args.streams, fused.chan["input"], side, side),
               # 1x1 convolutions that run inside the launch of the global average pooling behind them

@@ -123,6 +123,10 @@ SIGNATURES = {
                                                      ctypes.POINTER(_SZ)]),
     "catchq_inverted_residual_nhwc": (_I, [_P, _I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(RequantStage),
                                            ctypes.POINTER(RequantStage), _P, ctypes.POINTER(Epilogue), _P, _SZ, _P]),
+    "catchq_expand_depthwise_workspace_size": (_I, [_I, _I, _I, _I, _I, _I, ctypes.POINTER(RequantStage),
+                                                    ctypes.POINTER(RequantStage), _I, ctypes.POINTER(_SZ)]),
+    "catchq_expand_depthwise_nhwc": (_I, [_P, _I, _I, _I, _I, _I, _I, ctypes.POINTER(RequantStage),
+                                          ctypes.POINTER(RequantStage), _P, _I, _P, _SZ, _P]),
     "catchq_first_layers_workspace_size": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(RequantStage), _I, _I, _I,
                                                 _I, ctypes.POINTER(_SZ)]),
     "catchq_first_layers_nchw": (_I, [_P, _I, _I, _I, _I, _I, ctypes.c_float, _I, _I, _I, _I, _I,

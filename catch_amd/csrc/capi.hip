@@ -73,6 +73,9 @@ int conv2d_head_halo_i8(const void *x, int K1, const void *w1, const float *div1
 bool irb_i8_ok(int N, int H, int W, int Cin, int hid, int Co, int S, int cus);
 int irb_i8(const void *x, int N, int H, int W, int Cin, int hid, int Co, int S, const IrbStageDev &s1, const IrbStageDev &s2,
            const void *w3, const EpiDev &e, hipStream_t s);
+bool expand_dw_i8_ok(int N, int H, int W, int Cin, int hid, int S, int cus);
+int expand_dw_i8(const void *x, int N, int H, int W, int Cin, int hid, int S, const IrbStageDev &s1, const IrbStageDev &s2, void *q,
+                 int cus, hipStream_t s);
 bool stem_pool_i8_ok(int N, int C, int H, int W, int Co);
 int stem_pool_i8(const void *x, int N, int C, int H, int W, int x_pos, float x_scale, const IrbStageDev &s, int Co,
                  void *q, hipStream_t st);
@@ -663,14 +666,46 @@ CATCHQ_API int catchq_conv1x1_conv3x3_nhwc(const void *x, const catchq_pointwise
 
 static size_t round256(size_t v) { return (v + 255) / 256 * 256; }
 
+// constants the kernels that keep a hidden tensor on the chip serve
+static bool hidden_stage_ok(const catchq_requant_stage_t *s) {
+  return s->chan_div && s->chan_rcp && s->bias && s->exp2 >= -64 && s->exp2 <= 64;
+}
+static IrbStageDev hidden_stage(const catchq_requant_stage_t *s) {
+  return {(const int8_t *)s->w, s->chan_div, s->chan_rcp, s->bias, s->exp2, -s->q_position, s->act == CATCHQ_ACT_RELU6 ? 1 : 0};
+}
+static bool hidden_stage_aligned(const catchq_requant_stage_t *s) {
+  return aligned16(s->w) && aligned16(s->chan_div) && aligned16(s->chan_rcp) && aligned16(s->bias);
+}
+// such a stage as a launch of its own
+static catchq_epilogue_t hidden_stage_epilogue(const catchq_requant_stage_t *s, void *q, int sharing) {
+  catchq_epilogue_t e;
+  memset(&e, 0, sizeof(e));
+  e.exp2 = s->exp2;
+  e.chan_div = s->chan_div;
+  e.chan_rcp = s->chan_rcp;
+  e.bias = s->bias;
+  e.act = s->act;
+  e.q = q;
+  e.q_bitwidth = 8;
+  e.q_position = s->q_position;
+  e.q_scale = 1.0f;
+  e.sharing = sharing;
+  return e;
+}
+
 // shapes and constants the inverted-residual kernel serves (pointer alignment and the epilogue are checked at the call)
 static bool irb_fusable(int n, int h, int w, int ci, int hid, int co, int stride, const catchq_requant_stage_t *s1,
                         const catchq_requant_stage_t *s2, const catchq_epilogue_t *e) {
-  auto stage_ok = [](const catchq_requant_stage_t *s) {
-    return s->chan_div && s->chan_rcp && s->bias && s->exp2 >= -64 && s->exp2 <= 64;
-  };
-  return stage_ok(s1) && stage_ok(s2) && !e->exp2_dev[0] && !e->exp2_dev[1] && !e->acc_out &&
+  return hidden_stage_ok(s1) && hidden_stage_ok(s2) && !e->exp2_dev[0] && !e->exp2_dev[1] && !e->acc_out &&
          irb_i8_ok(n, h, w, ci, hid, co, stride, planned_cus(e->sharing));
+}
+
+static int check_hidden_stages(const catchq_requant_stage_t *s1, const catchq_requant_stage_t *s2) {
+  for (const catchq_requant_stage_t *s : {s1, s2}) {
+    if (s->act != CATCHQ_ACT_RELU && s->act != CATCHQ_ACT_RELU6) return CATCHQ_ERR_ARG;
+    if (s->exp2 < -126 || s->exp2 > 126 || s->q_position < -126 || s->q_position > 126) return CATCHQ_ERR_ARG;
+  }
+  return CATCHQ_OK;
 }
 
 static int check_irb(int n, int h, int w, int ci, int hid, int co, int stride, const catchq_requant_stage_t *s1,
@@ -678,12 +713,7 @@ static int check_irb(int n, int h, int w, int ci, int hid, int co, int stride, c
   if (!s1 || !s2) return CATCHQ_ERR_ARG;
   if (n < 0 || h <= 0 || w <= 0 || ci <= 0 || hid <= 0 || co <= 0 || stride <= 0) return CATCHQ_ERR_SHAPE;
   const int st = check_epi(e);
-  if (st != CATCHQ_OK) return st;
-  for (const catchq_requant_stage_t *s : {s1, s2}) {
-    if (s->act != CATCHQ_ACT_RELU && s->act != CATCHQ_ACT_RELU6) return CATCHQ_ERR_ARG;
-    if (s->exp2 < -126 || s->exp2 > 126 || s->q_position < -126 || s->q_position > 126) return CATCHQ_ERR_ARG;
-  }
-  return CATCHQ_OK;
+  return st != CATCHQ_OK ? st : check_hidden_stages(s1, s2);
 }
 
 CATCHQ_API int catchq_inverted_residual_workspace_size(int n, int h, int w, int ci, int hid, int co, int stride,
@@ -710,46 +740,75 @@ CATCHQ_API int catchq_inverted_residual_nhwc(const void *x, int n, int h, int w,
   if (ho <= 0 || wo <= 0) return CATCHQ_ERR_SHAPE;
   if (n == 0) return CATCHQ_OK;
   if (!x || !w_project || !expand->w || !depthwise->w) return CATCHQ_ERR_ARG;
-  if (irb_fusable(n, h, w, ci, hid, co, stride, expand, depthwise, epilogue) && aligned16(x) && aligned16(expand->w) &&
-      aligned16(depthwise->w) && aligned16(w_project) && aligned16(expand->chan_div) && aligned16(expand->chan_rcp) &&
-      aligned16(expand->bias) && aligned16(depthwise->chan_div) && aligned16(depthwise->chan_rcp) && aligned16(depthwise->bias)) {
+  if (irb_fusable(n, h, w, ci, hid, co, stride, expand, depthwise, epilogue) && aligned16(x) && aligned16(w_project) &&
+      hidden_stage_aligned(expand) && hidden_stage_aligned(depthwise)) {
     const EpiDev e = make_epi(epilogue, (int64_t)n * ho * wo * co);
-    const IrbStageDev s1 = {(const int8_t *)expand->w, expand->chan_div, expand->chan_rcp, expand->bias, expand->exp2,
-                            -expand->q_position, expand->act == CATCHQ_ACT_RELU6 ? 1 : 0};
-    const IrbStageDev s2 = {(const int8_t *)depthwise->w, depthwise->chan_div, depthwise->chan_rcp, depthwise->bias,
-                            depthwise->exp2, -depthwise->q_position, depthwise->act == CATCHQ_ACT_RELU6 ? 1 : 0};
-    const int st2 = irb_i8(x, n, h, w, ci, hid, co, stride, s1, s2, w_project, e, as_stream(stream));
+    const int st2 = irb_i8(x, n, h, w, ci, hid, co, stride, hidden_stage(expand), hidden_stage(depthwise), w_project, e, as_stream(stream));
     if (st2 >= 0) return st2;
   }
   // three launches: the two hidden tensors go through the workspace
   const size_t b1 = round256((size_t)n * h * w * hid), b2 = round256((size_t)n * ho * wo * hid);
   if (!workspace || workspace_bytes < b1 + b2 || !aligned16(workspace)) return CATCHQ_ERR_ARG;
   void *q1 = workspace, *q2 = (char *)workspace + b1;
-  auto stage_epi = [&](const catchq_requant_stage_t *s, void *q) {
-    catchq_epilogue_t es;
-    memset(&es, 0, sizeof(es));
-    es.exp2 = s->exp2;
-    es.chan_div = s->chan_div;
-    es.chan_rcp = s->chan_rcp;
-    es.bias = s->bias;
-    es.act = s->act;
-    es.q = q;
-    es.q_bitwidth = 8;
-    es.q_position = s->q_position;
-    es.q_scale = 1.0f;
-    es.sharing = epilogue->sharing;
-    return es;
-  };
   const catchq_conv_desc_t d1 = {n, h, w, ci, hid, 1, 1, 0, 0, 1, 1, 1, 1, 1};
-  const catchq_epilogue_t e1 = stage_epi(expand, q1);
+  const catchq_epilogue_t e1 = hidden_stage_epilogue(expand, q1, epilogue->sharing);
   st = catchq_conv2d_nhwc(x, 8, expand->w, 8, &d1, &e1, stream);
   if (st != CATCHQ_OK) return st;
   const catchq_conv_desc_t d2 = {n, h, w, hid, hid, 3, 3, 1, 1, stride, stride, 1, 1, hid};
-  const catchq_epilogue_t e2 = stage_epi(depthwise, q2);
+  const catchq_epilogue_t e2 = hidden_stage_epilogue(depthwise, q2, epilogue->sharing);
   st = catchq_conv2d_nhwc(q1, 8, depthwise->w, 8, &d2, &e2, stream);
   if (st != CATCHQ_OK) return st;
   const catchq_conv_desc_t d3 = {n, ho, wo, hid, co, 1, 1, 0, 0, 1, 1, 1, 1, 1};
   return catchq_conv2d_nhwc(q2, 8, w_project, 8, &d3, epilogue, stream);
+}
+
+// ---- the first two layers of such a block -----------------------------------------------------------------------------
+static int check_expand_dw(int n, int h, int w, int ci, int hid, int stride, const catchq_requant_stage_t *s1,
+                           const catchq_requant_stage_t *s2, int *ho, int *wo) {
+  if (!s1 || !s2) return CATCHQ_ERR_ARG;
+  if (n < 0 || h <= 0 || w <= 0 || ci <= 0 || hid <= 0 || stride <= 0) return CATCHQ_ERR_SHAPE;
+  const int st = check_hidden_stages(s1, s2);
+  if (st != CATCHQ_OK) return st;
+  *ho = catchq_conv_out_size(h, 3, 1, stride, 1);
+  *wo = catchq_conv_out_size(w, 3, 1, stride, 1);
+  return *ho > 0 && *wo > 0 ? CATCHQ_OK : CATCHQ_ERR_SHAPE;
+}
+
+CATCHQ_API int catchq_expand_depthwise_workspace_size(int n, int h, int w, int ci, int hid, int stride,
+                                                      const catchq_requant_stage_t *expand,
+                                                      const catchq_requant_stage_t *depthwise, int sharing, size_t *bytes) {
+  int ho, wo;
+  const int st = check_expand_dw(n, h, w, ci, hid, stride, expand, depthwise, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  if (!bytes) return CATCHQ_ERR_ARG;
+  *bytes = hidden_stage_ok(expand) && hidden_stage_ok(depthwise) && expand_dw_i8_ok(n, h, w, ci, hid, stride, planned_cus(sharing))
+               ? 0 : round256((size_t)n * h * w * hid);
+  return CATCHQ_OK;
+}
+
+CATCHQ_API int catchq_expand_depthwise_nhwc(const void *x, int n, int h, int w, int ci, int hid, int stride,
+                                            const catchq_requant_stage_t *expand, const catchq_requant_stage_t *depthwise, void *q,
+                                            int sharing, void *workspace, size_t workspace_bytes, catchq_stream_t stream) {
+  int ho, wo;
+  int st = check_expand_dw(n, h, w, ci, hid, stride, expand, depthwise, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  if (n == 0) return CATCHQ_OK;
+  if (!x || !q || !expand->w || !depthwise->w) return CATCHQ_ERR_ARG;
+  if (hidden_stage_ok(expand) && hidden_stage_ok(depthwise) && aligned16(x) && aligned16(q) && hidden_stage_aligned(expand) &&
+      hidden_stage_aligned(depthwise)) {
+    st = expand_dw_i8(x, n, h, w, ci, hid, stride, hidden_stage(expand), hidden_stage(depthwise), q, planned_cus(sharing),
+                      as_stream(stream));
+    if (st >= 0) return st;
+  }
+  // two launches: the expanded tensor goes through the workspace
+  if (!workspace || workspace_bytes < round256((size_t)n * h * w * hid) || !aligned16(workspace)) return CATCHQ_ERR_ARG;
+  const catchq_conv_desc_t d1 = {n, h, w, ci, hid, 1, 1, 0, 0, 1, 1, 1, 1, 1};
+  const catchq_epilogue_t e1 = hidden_stage_epilogue(expand, workspace, sharing);
+  st = catchq_conv2d_nhwc(x, 8, expand->w, 8, &d1, &e1, stream);
+  if (st != CATCHQ_OK) return st;
+  const catchq_conv_desc_t d2 = {n, h, w, hid, hid, 3, 3, 1, 1, stride, stride, 1, 1, hid};
+  const catchq_epilogue_t e2 = hidden_stage_epilogue(depthwise, q, sharing);
+  return catchq_conv2d_nhwc(workspace, 8, depthwise->w, 8, &d2, &e2, stream);
 }
 
 // ---- first layers: quantizer + few-channel convolution + max pooling ------------------------------------------------

@@ -7,7 +7,7 @@
 //  * dwconv_i8_kernel: any filter up to 5x5, any stride/dilation.  A block owns a strip of output pixels of one image row and all channels of a
 // 64-channel slab; the input rows the strip needs are staged in LDS once and every tap is read
 // from there, the filter taps of the slab sit in LDS transposed to [tap][channel].
-#include "catchq_common.h"
+#include "dw3x3.h"
 #include "igemm_common.h"
 
 namespace catchq {
@@ -102,15 +102,13 @@ struct Dw3Params {
   int items;  // HG * WG * CQ: work items of one image
 };
 
-constexpr int DW3_PW = 4, DW3_PH = 2;
-
 template <int S, int EPI>
 __global__ __launch_bounds__(256) void dw3x3_kernel(const int8_t *__restrict__ x, const int8_t *__restrict__ w,
                                                    Dw3Params p, EpiDev e) {
   resolve_exp2(e);
   typedef typename EpiOf<EPI>::type Sp;
   constexpr int PW = DW3_PW, PH = DW3_PH;
-  constexpr int NR = (PH - 1) * S + 3;  // input rows of the window
+  constexpr int NR = Dw3Window<S>::NR, NCL = Dw3Window<S>::NCL;
   const int item = blockIdx.x * 256 + threadIdx.x;  // (row group, column group, channel quad), channels fastest
   if (item >= p.items) return;
   const int t0 = item / p.CQ, cq = item - t0 * p.CQ;
@@ -118,34 +116,17 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(const int8_t *__restrict__ x
   const int ho0 = hg * PH, img = blockIdx.y;
   const int c = cq * 4;
 
-  // The multiply-accumulate runs on v_dot4_i32_i8, which sums four byte products: the four bytes of
-  // an operand must be four taps of ONE channel.  A pixel's dword holds four channels, so groups of
-  // four horizontally adjacent pixels are transposed (4x4 bytes, 8 byte permutes, the first stage
-  // shared between overlapping groups) into one dword per channel; a filter row is the byte vector
-  // (w0, w1, w2, 0) or, for the output one pixel to the right within the same group, (0, w0, w1, w2).
-  // 36 filter bytes of the four channels ([channel][tap]):
   int wraw[9];
 #pragma unroll
   for (int i = 0; i < 9; ++i) wraw[i] = *reinterpret_cast<const int *>(w + (int64_t)c * 9 + 4 * i);
-  int wa[4][3], wb[4][3];  // [channel][filter row]
+  int wa[4][3], wb[4][3];
+  dw3_pack(wraw, wa);
 #pragma unroll
   for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      unsigned v = 0;
-#pragma unroll
-      for (int q = 0; q < 3; ++q) {
-        const int b = j * 9 + r * 3 + q;
-        v |= (((unsigned)wraw[b >> 2] >> (8 * (b & 3))) & 0xffu) << (8 * q);
-      }
-      wa[j][r] = (int)v;
-      wb[j][r] = (int)(v << 8);
-    }
+    for (int r = 0; r < 3; ++r) wb[j][r] = (int)((unsigned)wa[j][r] << 8);
 
-  int acc[PH][PW][4];  // every sum starts with filter row 0 (accumulator operand 0), no zeroing pass
-
-  constexpr int NG = (S == 1) ? 2 : 4;  // transposed groups per input row: pixels 0-3, 2-5 [, 4-7, 6-9]
-  constexpr int NCL = 2 * NG + 2;       // input columns loaded (stride 2: one more than the window, weight 0)
+  int acc[PH][PW][4];
   const int hi0 = ho0 * S - p.ph, wi0 = wg * PW * S - p.pw;
   // addresses = a per-image base (the same for the whole block: scalar registers) + a 32-bit offset
   const int8_t *xi = x + (int64_t)img * p.H * p.W * p.C;
@@ -161,36 +142,7 @@ __global__ __launch_bounds__(256) void dw3x3_kernel(const int8_t *__restrict__ x
       if (row_ok && (unsigned)(wi0 + col) < (unsigned)p.W)
         xr[col] = *reinterpret_cast<const unsigned *>(xi + (rowo + (unsigned)(col * p.C)));
     }
-    // first transposition stage on pixel pairs (2m, 2m+1): bytes (a0,b0,a1,b1) and (a2,b2,a3,b3)
-    unsigned lo[NG + 1], hi2[NG + 1];
-#pragma unroll
-    for (int m = 0; m <= NG; ++m) {
-      lo[m] = __builtin_amdgcn_perm(xr[2 * m + 1], xr[2 * m], 0x05010400u);
-      hi2[m] = __builtin_amdgcn_perm(xr[2 * m + 1], xr[2 * m], 0x07030602u);
-    }
-#pragma unroll
-    for (int g = 0; g < NG; ++g) {
-      // second stage: group g = pixels 2g .. 2g+3, one dword per channel
-      int t[4];
-      t[0] = (int)__builtin_amdgcn_perm(lo[g + 1], lo[g], 0x05040100u);
-      t[1] = (int)__builtin_amdgcn_perm(lo[g + 1], lo[g], 0x07060302u);
-      t[2] = (int)__builtin_amdgcn_perm(hi2[g + 1], hi2[g], 0x05040100u);
-      t[3] = (int)__builtin_amdgcn_perm(hi2[g + 1], hi2[g], 0x07060302u);
-#pragma unroll
-      for (int py = 0; py < PH; ++py) {
-        const int r = ri - py * S;
-        if (r < 0 || r > 2) continue;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if constexpr (S == 1) {  // group g serves outputs 2g (taps at bytes 0..2) and 2g+1 (bytes 1..3)
-            acc[py][2 * g][j] = __builtin_amdgcn_sdot4(t[j], wa[j][r], r == 0 ? 0 : acc[py][2 * g][j], false);
-            acc[py][2 * g + 1][j] = __builtin_amdgcn_sdot4(t[j], wb[j][r], r == 0 ? 0 : acc[py][2 * g + 1][j], false);
-          } else {                 // stride 2: group g starts at input pixel 2g = the window of output g
-            acc[py][g][j] = __builtin_amdgcn_sdot4(t[j], wa[j][r], r == 0 ? 0 : acc[py][g][j], false);
-          }
-        }
-      }
-    }
+    dw3_row<S>(ri, xr, wa, wb, acc);
   }
 
   const EpiLane L = epi_lane_setup<Sp>(c, true, e);

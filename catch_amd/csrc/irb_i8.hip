@@ -25,6 +25,7 @@
 // output, 17 per depthwise output) on two waves per SIMD; what it saves is two launch start-ups and the traffic of
 // the hidden tensors.  Measured on MobileNetV2's blocks (64 images) it is the faster route for a lone stream of
 // launches from 14 x 14 outputs on; 7 x 7 images leave it too few blocks.
+#include "dw3x3.h"
 #include "igemm_i8_dma.inc"
 
 namespace catchq {
@@ -52,10 +53,7 @@ __global__ __launch_bounds__(64 * IRB_NW) void irb_kernel(const int8_t *__restri
                                                           const int8_t *__restrict__ W3, IrbParams p, EpiDev e) {
   resolve_exp2(e);
   constexpr int HC = 32 * KS3, NW = IRB_NW, NT = 64 * NW;
-  constexpr int PW = 4, PH = 2;
-  constexpr int NR = (PH - 1) * S + 3;
-  constexpr int NG = (S == 1) ? 2 : 4;
-  constexpr int NCL = 2 * NG + 2;
+  constexpr int PW = DW3_PW, PH = DW3_PH, NR = Dw3Window<S>::NR, NCL = Dw3Window<S>::NCL;
   extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -102,21 +100,14 @@ __global__ __launch_bounds__(64 * IRB_NW) void irb_kernel(const int8_t *__restri
       const int px = i / cpp, k = i - px * cpp;
       *reinterpret_cast<v4i *>(lds + p.off_x + px * p.xs + k * 16) = v;
     };
-    // 36 filter bytes of four channels -> twelve dwords, one per channel and filter row: bytes (w0, w1, w2, 0)
     auto pack_filters = [&](int q, const int (&wraw)[9]) {
+      int wa[4][3];
+      dw3_pack(wraw, wa);
       int *dst = reinterpret_cast<int *>(lds + p.off_wp) + q * 12;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int r = 0; r < 3; ++r) {
-          unsigned v = 0;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) {
-            const int b = j * 9 + r * 3 + k;
-            v |= (((unsigned)wraw[b >> 2] >> (8 * (b & 3))) & 0xffu) << (8 * k);
-          }
-          dst[j * 3 + r] = (int)v;
-        }
+        for (int r = 0; r < 3; ++r) dst[j * 3 + r] = wa[j][r];
     };
     auto fold = [&](int c, const float (&v)[6]) {
       cst[c] = __builtin_ldexpf(v[0], -s1.exp2);
@@ -176,24 +167,7 @@ __global__ __launch_bounds__(64 * IRB_NW) void irb_kernel(const int8_t *__restri
     }
   }
 
-  float q1_hi = __builtin_ldexpf(127.0f, -s1.q_neg_pos), q2_hi = __builtin_ldexpf(127.0f, -s2.q_neg_pos);
-  if (s1.relu6) q1_hi = q1_hi < 6.0f ? q1_hi : 6.0f;
-  if (s2.relu6) q2_hi = q2_hi < 6.0f ? q2_hi : 6.0f;
-  const float q1_sc = __builtin_ldexpf(1.0f, s1.q_neg_pos), q2_sc = __builtin_ldexpf(1.0f, s2.q_neg_pos);
-
-  // requantized ReLU of one lane's four channels: (acc / div + bias) clamped to [0, hi], scaled, rounded to even
-  auto requant4 = [&](const int *a, const v4f dv, const v4f rc, const v4f bs, float hi, float sc) -> unsigned {
-    unsigned b[4];
-#pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      float x = div_by_rcp((float)a[t], dv[t], rc[t]) + bs[t];
-      x = __builtin_amdgcn_fmed3f(x, 0.0f, hi);  // ReLU and the upper clamp; NaN -> 0
-      b[t] = __builtin_bit_cast(unsigned, __builtin_fmaf(x, sc, 12582912.0f));
-    }
-    const unsigned lo = __builtin_amdgcn_perm(b[1], b[0], 0x0c0c0400u);
-    const unsigned hi2 = __builtin_amdgcn_perm(b[3], b[2], 0x04000c0cu);
-    return lo | hi2;
-  };
+  const ReluRequant rq1(s1), rq2(s2);
 
   // the projection: this wave's pixel sub-tile and column tiles
   const int ws = wave % p.nws, wj = wave / p.nws;
@@ -238,8 +212,8 @@ __global__ __launch_bounds__(64 * IRB_NW) void irb_kernel(const int8_t *__restri
       for (int g = 0; g < 4; ++g) {
         const int a[4] = {acc1[4 * g], acc1[4 * g + 1], acc1[4 * g + 2], acc1[4 * g + 3]};
         const float *cb = cbase + 8 * g;
-        const unsigned packed = requant4(a, *reinterpret_cast<const v4f *>(cb), *reinterpret_cast<const v4f *>(cb + p.hid),
-                                         *reinterpret_cast<const v4f *>(cb + 2 * p.hid), q1_hi, q1_sc);
+        const unsigned packed = rq1.four(a, *reinterpret_cast<const v4f *>(cb), *reinterpret_cast<const v4f *>(cb + p.hid),
+                                         *reinterpret_cast<const v4f *>(cb + 2 * p.hid));
         if (in_tile) *reinterpret_cast<unsigned *>(cell + 8 * g) = valid ? packed : 0u;
       }
     }
@@ -286,34 +260,7 @@ __global__ __launch_bounds__(64 * IRB_NW) void irb_kernel(const int8_t *__restri
         unsigned xr[NCL];
 #pragma unroll
         for (int col = 0; col < NCL; ++col) xr[col] = *reinterpret_cast<const unsigned *>(win + (ri * p.PCA + col) * p.hs);
-        unsigned lo[NG + 1], hi2[NG + 1];
-#pragma unroll
-        for (int m = 0; m <= NG; ++m) {
-          lo[m] = __builtin_amdgcn_perm(xr[2 * m + 1], xr[2 * m], 0x05010400u);
-          hi2[m] = __builtin_amdgcn_perm(xr[2 * m + 1], xr[2 * m], 0x07030602u);
-        }
-#pragma unroll
-        for (int g = 0; g < NG; ++g) {
-          int tt[4];
-          tt[0] = (int)__builtin_amdgcn_perm(lo[g + 1], lo[g], 0x05040100u);
-          tt[1] = (int)__builtin_amdgcn_perm(lo[g + 1], lo[g], 0x07060302u);
-          tt[2] = (int)__builtin_amdgcn_perm(hi2[g + 1], hi2[g], 0x05040100u);
-          tt[3] = (int)__builtin_amdgcn_perm(hi2[g + 1], hi2[g], 0x07060302u);
-#pragma unroll
-          for (int py = 0; py < PH; ++py) {
-            const int r = ri - py * S;
-            if (r < 0 || r > 2) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              if constexpr (S == 1) {
-                acc[py][2 * g][j] = __builtin_amdgcn_sdot4(tt[j], wa[j][r], r == 0 ? 0 : acc[py][2 * g][j], false);
-                acc[py][2 * g + 1][j] = __builtin_amdgcn_sdot4(tt[j], wb[j][r], r == 0 ? 0 : acc[py][2 * g + 1][j], false);
-              } else {
-                acc[py][g][j] = __builtin_amdgcn_sdot4(tt[j], wa[j][r], r == 0 ? 0 : acc[py][g][j], false);
-              }
-            }
-          }
-        }
+        dw3_row<S>(ri, xr, wa, wb, acc);
       }
       const float *cb = reinterpret_cast<const float *>(lds + p.off_cst) + 3 * p.hid + c0 + cl;
       const v4f dv = *reinterpret_cast<const v4f *>(cb), rc = *reinterpret_cast<const v4f *>(cb + p.hid);
@@ -324,7 +271,7 @@ __global__ __launch_bounds__(64 * IRB_NW) void irb_kernel(const int8_t *__restri
 #pragma unroll
         for (int px = 0; px < PW; ++px) {
           const int wo = wg * PW + px;
-          const unsigned packed = requant4(acc[py][px], dv, rc, bs, q2_hi, q2_sc);
+          const unsigned packed = rq2.four(acc[py][px], dv, rc, bs);
           if (ho_l < rows && wo < p.Wo) *reinterpret_cast<unsigned *>(lds + p.off_a3 + (ho_l * p.Wo + wo) * p.as + cl) = packed;
         }
       }

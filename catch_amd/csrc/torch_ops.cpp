@@ -263,6 +263,17 @@ bool irb_fuses_op(int64_t n, int64_t h, int64_t w, int64_t ci, int64_t hid, int6
                                                  &bytes) == CATCHQ_OK && bytes == 0;
 }
 
+bool expand_dw_fuses_op(int64_t n, int64_t h, int64_t w, int64_t ci, int64_t hid, int64_t stride) {
+  float one = 1.0f;
+  catchq_requant_stage_t st;
+  std::memset(&st, 0, sizeof(st));
+  st.w = &one; st.chan_div = st.chan_rcp = st.bias = &one;  // presence only: nothing is dereferenced
+  st.act = CATCHQ_ACT_RELU6;
+  size_t bytes = 1;
+  return catchq_expand_depthwise_workspace_size((int)n, (int)h, (int)w, (int)ci, (int)hid, (int)stride, &st, &st, t_launch_sharing,
+                                                &bytes) == CATCHQ_OK && bytes == 0;
+}
+
 bool first_layers_fuse_op(int64_t n, int64_t c, int64_t h, int64_t w, int64_t co, int64_t k, int64_t stride, int64_t pad,
                           int64_t pool_k, int64_t pool_stride, int64_t pool_pad) {
   float one = 1.0f;
@@ -713,6 +724,40 @@ std::tuple<Tensor, Tensor> qconv2d_irb_op(const Tensor &qx, const Tensor &w1, in
                                              &k1.st, &k2.st, w3.data_ptr(), &e, ws.data_ptr(), ws_bytes, current_stream()),
                "torch_mlu::qconv2d_irb");
   return std::make_tuple(o.y, o.q);
+}
+
+// The expansion and the depthwise layer of such a block in one call (catchq_expand_depthwise_nhwc), arguments as above:
+// the depthwise layer's int8 output.
+Tensor qconv2d_expand_dw_op(const Tensor &qx, const Tensor &w1, int64_t exp2_1, const c10::optional<Tensor> &chan_div1,
+                            const c10::optional<Tensor> &bias1, int64_t act1, int64_t q_position1, const Tensor &wd, int64_t stride,
+                            int64_t exp2_2, const c10::optional<Tensor> &chan_div2, const c10::optional<Tensor> &bias2, int64_t act2,
+                            int64_t q_position2) {
+  c10::DeviceGuard guard(qx.device());
+  TORCH_CHECK(qx.dim() == 4 && qx.is_contiguous() && w1.is_contiguous() && wd.is_contiguous(),
+              "qconv2d_expand_dw expects contiguous NHWC activations and contiguous filters");
+  TORCH_CHECK(qx.scalar_type() == at::kChar && w1.scalar_type() == at::kChar && wd.scalar_type() == at::kChar,
+              "qconv2d_expand_dw: int8 operands expected");
+  TORCH_CHECK(w1.device() == qx.device() && wd.device() == qx.device(), "qconv2d_expand_dw: operands on different devices");
+  const int64_t n = qx.size(0), h = qx.size(1), w = qx.size(2), ci = qx.size(3), hid = w1.size(0);
+  TORCH_CHECK(w1.numel() == hid * ci, "qconv2d_expand_dw: the expansion's filters must be [", hid, ", ", ci, "]");
+  TORCH_CHECK(wd.size(0) == hid && wd.numel() == hid * 9, "qconv2d_expand_dw: the depthwise filters must be [", hid, ", 3, 3]");
+  TORCH_CHECK(stride >= 1, "bad stride");
+  const int ho = catchq_conv_out_size((int)h, 3, 1, (int)stride, 1), wo = catchq_conv_out_size((int)w, 3, 1, (int)stride, 1);
+  TORCH_CHECK(ho > 0 && wo > 0, "Calculated output size is too small");
+  StageKeep k1, k2;
+  fill_stage(&k1, w1, exp2_1, chan_div1, bias1, act1, q_position1, hid, "expansion constants");
+  fill_stage(&k2, wd, exp2_2, chan_div2, bias2, act2, q_position2, hid, "depthwise constants");
+  Tensor q = at::empty({n, ho, wo, hid}, qx.options());
+  if (n == 0) return q;
+  size_t ws_bytes = 0;
+  check_status(catchq_expand_depthwise_workspace_size((int)n, (int)h, (int)w, (int)ci, (int)hid, (int)stride, &k1.st, &k2.st,
+                                                      t_launch_sharing, &ws_bytes),
+               "torch_mlu::qconv2d_expand_dw");
+  Tensor ws = at::empty({(int64_t)std::max<size_t>(ws_bytes, 16)}, qx.options());
+  check_status(catchq_expand_depthwise_nhwc(qx.data_ptr(), (int)n, (int)h, (int)w, (int)ci, (int)hid, (int)stride, &k1.st, &k2.st,
+                                            q.data_ptr(), t_launch_sharing, ws.data_ptr(), ws_bytes, current_stream()),
+               "torch_mlu::qconv2d_expand_dw");
+  return q;
 }
 
 // The first layers in one call (catchq_first_layers_nchw): x [N,C,H,W] fp32, w [Co,kh,kw4,4] int8 (filter rows padded
@@ -1702,6 +1747,9 @@ TORCH_LIBRARY(torch_mlu, m) {
         "int exp2, Tensor? chan_div, Tensor? bias, int[] padding, int[] stride, int[] dilation, int act=0, "
         "bool want_y=True, bool y_half=False, int q_bitwidth=0, int q_position=0, float q_scale=1.0, "
         "float act_slope=0.0) -> (Tensor, Tensor)");
+  m.def("qconv2d_expand_dw(Tensor qx, Tensor w1, int exp2_1, Tensor? chan_div1, Tensor? bias1, int act1, int q_position1, "
+        "Tensor wd, int stride, int exp2_2, Tensor? chan_div2, Tensor? bias2, int act2, int q_position2) -> Tensor");
+  m.def("expand_depthwise_fuses(int n, int h, int w, int ci, int hid, int stride) -> bool", &expand_dw_fuses_op);
   m.def("qconv2d_irb(Tensor qx, Tensor w1, int exp2_1, Tensor? chan_div1, Tensor? bias1, int act1, int q_position1, "
         "Tensor wd, int stride, int exp2_2, Tensor? chan_div2, Tensor? bias2, int act2, int q_position2, Tensor w3, "
         "int exp2, Tensor? chan_div, Tensor? bias, Tensor? resid, bool want_y=True, bool y_half=False, "
@@ -1752,6 +1800,7 @@ TORCH_LIBRARY_IMPL(torch_mlu, CUDA, m) {  // ROCm tensors dispatch on the CUDA k
   m.impl("qconv2d_shortcut", &qconv2d_shortcut_op);
   m.impl("qconv2d_head", &qconv2d_head_op);
   m.impl("qconv2d_irb", &qconv2d_irb_op);
+  m.impl("qconv2d_expand_dw", &qconv2d_expand_dw_op);
   m.impl("qconv2d_first_layers", &qconv2d_first_layers_op);
   m.impl("qconv2d_avgpool", &qconv2d_avgpool_op);
   m.impl("qconv2d_chain", &qconv2d_chain_op);

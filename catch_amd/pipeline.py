@@ -170,7 +170,7 @@ def _decode(layer, sd, device, ci_dev, co_dev, fractional=False):
 class FusedNet(object):
     def __init__(self, layers, state_dict, device="cuda", out_half=False, fuse_shortcuts=True,
                  fractional_scale=False, chain_links=None, fuse_heads=True, fuse_blocks=False,
-                 fuse_first_layers=True, fuse_avgpool=True):
+                 fuse_first_layers=True, fuse_avgpool=True, fuse_expansions=True):
         """fractional_scale: quantize activations and weights with position and fractional scale -- the
         general form the reference's fused (graph) mode hands to its backend per tensor / per axis
         (jit/utils/utils.cpp:81-167) -- instead of the eager ops' power-of-two steps.
@@ -193,7 +193,10 @@ class FusedNet(object):
         only reader run as one launch (torch_mlu::qconv2d_first_layers) where the library's kernel serves the shape;
         neither the quantized image nor the convolution's output is then stored.
         fuse_avgpool: a 1x1 convolution whose only reader is the global average pooling runs inside the pooling's launch
-        (torch_mlu::qconv2d_avgpool) where the library's kernel serves the shape; its fp32 output is then never stored."""
+        (torch_mlu::qconv2d_avgpool) where the library's kernel serves the shape; its fp32 output is then never stored.
+        fuse_expansions: a 1x1 convolution behind ReLU / ReLU6 whose only reader is a 3x3 depthwise convolution runs inside
+        that layer's launch (torch_mlu::qconv2d_expand_dw) where the library's kernel serves the shape; its int8 output is
+        then never stored."""
         self.layers = list(layers)
         self._fuse_shortcuts = fuse_shortcuts
         self._chains_by_size = chain_links is None
@@ -263,36 +266,11 @@ class FusedNet(object):
                         and h.name not in self._fused_away and not (self.stem and self.stem["name"] in (l.name, h.name))):
                     self.head_of[l.name] = h
         self._head_names = set(h.name for h in self.head_of.values())
-        # Inverted-residual blocks: block_of[projection layer name] = (expansion layer, depthwise layer).
-        self.block_of = {}
-        if fuse_blocks:
-            by_name = {l.name: l for l in self.layers}
-
-            def only_reader(a, b):
-                readers = [m for m in self.layers
-                           if m.src == a.name or (isinstance(m.src, tuple) and a.name in m.src) or m.add == a.name]
-                return (readers == [b] and a.name not in self.outputs and not self.f_demand[a.name]
-                        and self.q_demand[a.name] == [(8, self.q[b.name].pos_x, 1.0)])
-
-            def inner_ok(a):
-                aq = self.q[a.name]
-                return (a.act in ("relu", "relu6") and not a.add and (aq.bw_x, aq.bw_w) == (8, 8) and aq.scale_x == 1.0
-                        and aq.chan_div is not None and aq.bias is not None and -64 <= aq.exp2 <= 64
-                        and a.name not in self._fused_away and a.name not in self._head_names
-                        and not (self.stem and self.stem["name"] == a.name))
-            for pl in self.layers:
-                d = by_name.get(pl.src) if pl.kind == "conv" and isinstance(pl.src, str) else None
-                x = by_name.get(d.src) if d is not None and d.kind == "conv" and isinstance(d.src, str) else None
-                if x is None or x.kind != "conv" or pl.name in self.chain_of or pl.name in self.shortcut_of:
-                    continue
-                pq = self.q[pl.name]
-                if (pl.k == 1 and pl.pad == 0 and pl.stride == 1 and pl.groups == 1 and pl.act == "none"
-                        and not pl.add_after and (pq.bw_x, pq.bw_w) == (8, 8)
-                        and d.k == 3 and d.pad == 1 and d.stride in (1, 2) and d.groups == d.ci == d.co and d.groups > 1
-                        and x.k == 1 and x.pad == 0 and x.stride == 1 and x.groups == 1
-                        and inner_ok(x) and inner_ok(d) and only_reader(x, d) and only_reader(d, pl)
-                        and self.cdev[x.name] == self.cdev[d.name] == x.co):
-                    self.block_of[pl.name] = (x, d)
+        # Expansions: expansion_of[3x3 depthwise layer name] = the 1x1 layer in front of it.  Inverted-residual blocks:
+        # block_of[projection layer name] = (expansion layer, depthwise layer).
+        self.expansion_of, self.block_of = {}, {}
+        self._plan_blocks(fuse_expansions, fuse_blocks)
+        self._expansion_names = set(x.name for x in self.expansion_of.values())
         # First layers: first_pool = the max-pooling layer behind the few-channel first convolution, when the pooled
         # int8 tensor is all that anything reads of the two.
         self.first_pool = None
@@ -337,6 +315,46 @@ class FusedNet(object):
             self._block_inner[d.name] = pname
 
         self._few = None  # the plan for few pixels (_few_plan), made when first needed
+
+    def _plan_blocks(self, expansions, blocks):
+        by_name = {l.name: l for l in self.layers}
+
+        def only_reader(a, b):
+            readers = [m for m in self.layers
+                       if m.src == a.name or (isinstance(m.src, tuple) and a.name in m.src) or m.add == a.name]
+            return (readers == [b] and a.name not in self.outputs and not self.f_demand[a.name]
+                    and self.q_demand[a.name] == [(8, self.q[b.name].pos_x, 1.0)])
+
+        def inner_ok(a):
+            aq = self.q[a.name]
+            return (a.act in ("relu", "relu6") and not a.add and (aq.bw_x, aq.bw_w) == (8, 8) and aq.scale_x == 1.0
+                    and aq.chan_div is not None and aq.bias is not None and -64 <= aq.exp2 <= 64
+                    and a.name not in self._fused_away and a.name not in self._head_names
+                    and not (self.stem and self.stem["name"] == a.name))
+
+        def conv_in_front(l):
+            c = by_name.get(l.src) if isinstance(l.src, str) else None
+            return c if c is not None and c.kind == "conv" else None
+
+        for d in self.layers:
+            x = conv_in_front(d) if d.kind == "conv" else None
+            if (x is None or d.k != 3 or d.pad != 1 or d.stride not in (1, 2) or not d.groups == d.ci == d.co or d.groups <= 1
+                    or x.k != 1 or x.pad != 0 or x.stride != 1 or x.groups != 1 or not inner_ok(x) or not only_reader(x, d)
+                    or d.act not in ("relu", "relu6")):
+                continue
+            if (expansions and inner_ok(d) and self.cdev[x.name] == self.cdev[d.name] and d.name not in self.outputs
+                    and not self.f_demand[d.name] and len(self.q_demand[d.name]) == 1
+                    and self.q_demand[d.name][0][0] == 8 and self.q_demand[d.name][0][2] == 1.0):
+                self.expansion_of[d.name] = x
+            for pl in self.layers if blocks else ():
+                if pl.kind != "conv" or pl.src != d.name or pl.name in self.chain_of or pl.name in self.shortcut_of:
+                    continue
+                pq = self.q[pl.name]
+                if (pl.k == 1 and pl.pad == 0 and pl.stride == 1 and pl.groups == 1 and pl.act == "none"
+                        and not pl.add_after and (pq.bw_x, pq.bw_w) == (8, 8)
+                        and inner_ok(d) and only_reader(d, pl)
+                        and self.cdev[x.name] == self.cdev[d.name] == x.co):
+                    self.block_of[pl.name] = (x, d)
 
     def _plan_shortcuts(self):
         by_name = {l.name: l for l in self.layers}
@@ -401,6 +419,13 @@ class FusedNet(object):
             return False
         return bool(torch.ops.torch_mlu.inverted_residual_fuses(n, h, w, self.cdev[x.src], self.cdev[x.name],
                                                                 self.cdev[proj.name], d.stride))
+
+    def expansion_fuses(self, dw, n, h, w):
+        """whether the 1x1 layer in front of the depthwise layer `dw` runs inside its launch over n images of h x w"""
+        x = self.expansion_of.get(dw.name)
+        if x is None:
+            return False
+        return bool(torch.ops.torch_mlu.expand_depthwise_fuses(n, h, w, self.cdev[x.src], self.cdev[x.name], dw.stride))
 
     def first_layers_fuse(self, n, c, h, w):
         """whether quantizer, first convolution and pooling run as one launch on a contiguous fp32 batch [n, c, h, w]"""
@@ -580,7 +605,8 @@ class FusedNet(object):
         layer, its quantized input, int32 accumulators and fp32 output (as NHWC tensors).
         keep: optional dict that receives every tensor the plan itself produces, keyed (name, "f") for an
         fp32 (or fp16 output) NHWC tensor and (name, bitwidth, position, scale) for a quantized one -- the
-        untraced plan's own launches, unlike trace, which asks every layer for extra outputs.
+        untraced plan's own launches, unlike trace, which asks every layer for extra outputs -- and what a depthwise
+        layer's launch reads of the expansion inside it (expansion_of), from a launch of the expansion alone.
         timers: optional dict; every conv/fc launch is bracketed by a pair of events recorded on
         the current stream and the pair is appended to timers[layer name] (durations of the
         launches in their real sequence, caches as the previous layer left them)."""
@@ -618,6 +644,7 @@ class FusedNet(object):
                 env[("input",) + d] = ops.quantize_nhwc(x, d[0], d[1], self.cdev["input"], d[2])
         skipped_heads = set()
         skipped_inner = set()
+        skipped_expansions = {}
         pooled_inside = set()
         by_name = {l.name: l for l in self.layers}
         for l in self.layers:
@@ -661,6 +688,26 @@ class FusedNet(object):
                     env[(name,) + qd] = q
                 for dd in self._further_forms(name):
                     env[(name,) + dd] = ops.quantize(y, dd[0], dd[1], dd[2])
+                continue
+            if l.kind == "conv" and not tracing and name in self._expansion_names:
+                d_ = next(m for m in self.layers if self.expansion_of.get(m.name) is l)
+                ex = env[(l.src, 8, self.q[name].pos_x, 1.0)]
+                if self.expansion_fuses(d_, ex.shape[0], ex.shape[1], ex.shape[2]):
+                    skipped_expansions[d_.name] = l  # computed inside the launch of the depthwise layer behind it
+                    if keep is not None:
+                        lq = self.q[name]
+                        env[(name,) + tuple(self.q_demand[name][0])] = ops.qconv2d(
+                            ex, lq.qw, lq.exp2, lq.chan_div, lq.bias, None, [0, 0], [1, 1], [1, 1], 1, _ACT_CODE[l.act], False,
+                            False, False, *self.q_demand[name][0])[1]
+                    continue
+            if name in skipped_expansions:
+                x_, lq, qd = skipped_expansions[name], self.q[name], self.q_demand[name][0]
+                xq = self.q[x_.name]
+                tick(name)
+                env[(name,) + qd] = ops.qconv2d_expand_dw(env[(x_.src, 8, xq.pos_x, 1.0)], xq.qw, xq.exp2, xq.chan_div, xq.bias,
+                                                          _ACT_CODE[x_.act], lq.pos_x, lq.qw, l.stride, lq.exp2, lq.chan_div,
+                                                          lq.bias, _ACT_CODE[l.act], qd[1])
+                tick(name)
                 continue
             if l.kind == "conv" and not tracing and name in self._fused_away:
                 continue
@@ -843,7 +890,7 @@ class FusedNet(object):
         -- has to reach 3.7 us per launch of the graph; the weights are those that put the measured cases on the right side,
         not a forecast of the time (which is 1 to 2 times as long).  Measured, one part / two (us), the smaller a batch that
         is left as one, the larger one that is split:
-          MobileNetV2 224 x 224, 32 images 348 / 353, 48 441 / 426, 64 511 / 490; 192 x 192, 27 277 / 293, 64 434 / 423
+          MobileNetV2 224 x 224, 8 images 186 / 213, 32 269 / 261, 64 387 / 374; 192 x 192, 27 230 / 239, 64 332 / 333
           ResNet-50 224 x 224, 8 images 343 / 365, 20 530 / 528, 64 1066 / 999; 112 x 112, 64 477 / 464 (not split)
           ResNet-18 224 x 224, 16 images 238 / 250, 40 473 / 433; 112 x 112, 64 248 / 261
           Darknet-53 416 x 416, 3 images 841 / 929, 5 1136 / 1106; 320 x 320, 4 806 / 813, 8 1117 / 1061
@@ -863,7 +910,8 @@ class FusedNet(object):
             size[l.name] = hi, wi
             if l.name in self._fused_away or l.name in self._pooled_names or (self.first_pool and l is self.first_pool):
                 continue
-            launches += 1
+            if l.name not in self._expansion_names:  # (their elements are made all the same)
+                launches += 1
             if l.kind in ("conv", "fc"):
                 elems += n * hi * wi * l.co
                 macs += n * hi * wi * l.co * (l.ci // (l.groups or 1)) * (l.k or 1) ** 2 * (2 if self.q[l.name].bw_x == 16 else 1)

@@ -395,6 +395,17 @@ int catchq_inverted_residual_nhwc(const void *x, int n, int h, int w, int ci, in
                                   const void *w_project, const catchq_epilogue_t *epilogue, void *workspace,
                                   size_t workspace_bytes, catchq_stream_t stream);
 
+/* The first two of these layers in one launch (the projection reads all hidden channels of a pixel, the depthwise layer one): q
+ * [n,ho,wo,hid] int8 is the depthwise layer's output, as the block above states it; x, expand and depthwise are its operands.  One
+ * launch for strides 1 and 2, ci a multiple of 16 up to 160, hid a multiple of 16, 2 <= h, 2 <= w <= 256, 16-byte aligned tensors and
+ * constants with chan_div, chan_rcp and bias (-64 <= exp2 <= 64) (the workspace is 0 then); anything else runs as two, with the
+ * expanded tensor in the caller's workspace.  `sharing`: catchq_epilogue_t::sharing. */
+int catchq_expand_depthwise_workspace_size(int n, int h, int w, int ci, int hid, int stride, const catchq_requant_stage_t *expand,
+                                           const catchq_requant_stage_t *depthwise, int sharing, size_t *bytes);
+int catchq_expand_depthwise_nhwc(const void *x, int n, int h, int w, int ci, int hid, int stride, const catchq_requant_stage_t *expand,
+                                 const catchq_requant_stage_t *depthwise, void *q, int sharing, void *workspace,
+                                 size_t workspace_bytes, catchq_stream_t stream);
+
 /* The first layers of an image network in one launch: input quantization, k x k convolution over a few channels,
  * ReLU / ReLU6, requantization, max pooling.  In the reference these are cnnl_quantify_offline on the channels-last
  * input (operators/cnnl/quantify_conv_forward.cpp:62-63,97), torch_mlu::conv2d (cnnl_conv2d,
