@@ -23,7 +23,7 @@ struct SmallSide {
   int K;             // kh * kw * Ci < 2^20
   int H, W, Ci, kw, ph, pw, sh, sw, dh, dw;  // Ci: channels of the filters; where the activations have fewer, those beyond read
                                              // whatever lies there, against zeros
-  unsigned img_stride, row_stride, pix_stride, chan_stride;  // elements
+  unsigned img_stride, row_stride, pix_stride;  // elements
   unsigned magic_ci, magic_kw, mask_ci, mask_kw;  // ceil(2^32 / d), mask 0; for d = 1 magic 0, mask ~0
   unsigned a_bytes, b_bytes;
 };
@@ -150,7 +150,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
   constexpr int RAW = in_loads(IN, 16);     // loads per 16 activations
   FloatPiece<IN, 16> raw[NA];
   (void)raw;
-  const unsigned chan_bytes = in_apart(IN) ? o.chan_stride * (unsigned)ES : 0u;
+  const unsigned chan_stride = in_apart(IN) ? (unsigned)(o.H * o.W) : 1u;
   auto issue = [&](int s) {  // step s of this wave's slice into its slot s & 1 (floating activations: into raw)
     const int slot = (s & 1) * SLOT_BYTES;
     unsigned k[2], koff[2];
@@ -167,7 +167,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
         const unsigned r = div_magic(tap, o.magic_kw, o.mask_kw), q = tap - r * (unsigned)o.kw;
         dy[h] = (int)r * o.dh;
         dx[h] = (int)q * o.dw;
-        koff[h] = (unsigned)dy[h] * o.row_stride + (unsigned)dx[h] * o.pix_stride + (in_apart(IN) ? ci * o.chan_stride : ci);
+        koff[h] = (unsigned)dy[h] * o.row_stride + (unsigned)dx[h] * o.pix_stride + ci * chan_stride;
       }
     }
     // (the filters first: loads complete in order, so a wave that has its activations has its filters)
@@ -190,7 +190,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       if constexpr (IN == IN_I8) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
       } else {
-        raw[j].load(rsrc_a, voff, chan_bytes);
+        raw[j].load(rsrc_a, voff, chan_stride * (unsigned)ES);
       }
     }
   };
@@ -355,7 +355,6 @@ static bool small_side(SmallSide *o, const void *x, int x_size, const void *w, i
   o->img_stride = (unsigned)((int64_t)H * W * x_ci);
   o->row_stride = (unsigned)(apart ? W : (int64_t)W * x_ci);
   o->pix_stride = apart ? 1u : (unsigned)x_ci;
-  o->chan_stride = apart ? (unsigned)((int64_t)H * W) : 1u;
   magic(Ci, &o->magic_ci, &o->mask_ci);
   magic(kw, &o->magic_kw, &o->mask_kw);
   o->a_bytes = (unsigned)a_bytes; o->b_bytes = (unsigned)b_bytes;

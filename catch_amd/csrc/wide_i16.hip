@@ -36,7 +36,7 @@ struct WideParams {
   const int16_t *w;
   int M, N, K;  // K < 2^16
   int H, W, Ci, Ho, Wo, kw, ph, pw, sh, sw, dh, dw;
-  unsigned img_stride, row_stride, pix_stride, chan_stride;  // elements
+  unsigned img_stride, row_stride, pix_stride;  // elements
   int x_neg_pos;      // floating activations: quantized at 2^-x_neg_pos
   unsigned magic_ci, magic_kw, mask_ci, mask_kw;  // ceil(2^32 / d), mask 0; for d = 1 magic 0, mask ~0
   int tiles_m, tiles_n, nblocks;
@@ -119,8 +119,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
   constexpr int ES = IN == IN_I8 ? 2 : in_bytes(IN);  // bytes per activation (IN_I8: integers as they are, of 16 bits)
   FloatPiece<IN, 8> raw[NA];
   (void)raw;
-  const unsigned chan_bytes = in_apart(IN) ? p.chan_stride * (unsigned)ES : 0u;
-  (void)chan_bytes;
+  const unsigned chan_stride = in_apart(IN) ? (unsigned)(p.H * p.W) : 1u;
 
   auto issue = [&](int s) {
     const int slot = (s & 1) * SLOT_BYTES;
@@ -149,7 +148,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
         const unsigned r = wide_div(tap, p.magic_kw, p.mask_kw), q = tap - r * (unsigned)p.kw;
         dy[h] = (int)r * p.dh;
         dx[h] = (int)q * p.dw;
-        koff[h] = (unsigned)dy[h] * p.row_stride + (unsigned)dx[h] * p.pix_stride + (in_apart(IN) ? ci * p.chan_stride : ci);
+        koff[h] = (unsigned)dy[h] * p.row_stride + (unsigned)dx[h] * p.pix_stride + ci * chan_stride;
       }
     }
     const int step = (first + s) * (KS * 2);
@@ -174,7 +173,7 @@ __global__ __launch_bounds__(64 * NW) void wide_i16_kernel(WideParams p, EpiDev 
       asm volatile("" : "+v"(voff));  // one select and one load, not two loads under complementary masks
       if constexpr (IN == IN_I8)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(my + slot + j * 1024), 16, (int)voff, 0, 0, 0);
-      else raw[j].load(rsrc_a, voff, chan_bytes);
+      else raw[j].load(rsrc_a, voff, chan_stride * (unsigned)ES);
     }
     if constexpr (IN == IN_I8) filters();
   };
@@ -407,7 +406,6 @@ static bool wide_params(WideParams *q, const void *x, int x_size, const void *w,
   p.img_stride = (unsigned)((int64_t)H * W * x_ci);
   p.row_stride = (unsigned)(apart ? W : (int64_t)W * x_ci);
   p.pix_stride = apart ? 1u : (unsigned)x_ci;
-  p.chan_stride = apart ? (unsigned)((int64_t)H * W) : 1u;
   auto magic = [](unsigned d, unsigned *m, unsigned *mask) {  // dividends below 2^16: exact for every divisor below 2^16
     *m = d <= 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d);
     *mask = d <= 1 ? ~0u : 0u;
