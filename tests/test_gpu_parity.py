@@ -1437,6 +1437,18 @@ def test_conv1x1_global_avgpool(case):
             assert same_bits(orc.quantize(mean, 16, qp - 8, 0.93), out["q"].cpu().numpy()), (want_mean, q_bw)
 
 
+@pytest.mark.parametrize("case", [
+    (3, 3, 11, 320, 96, True, 1, True),       # 33 pixels, a wave per group: the second has one; half of the last block has no channels
+    (7, 8, 8, 64, 1984, False, 2, True),      # 64 channels a block, 217 of them; 64 pixels
+    (9, 5, 7, 512, 2016, True, 1, True),      # 128 channels a block, the last one short
+    (300, 3, 11, 32, 64, False, 1, True),     # more blocks than units: 64 channels and ...
+    (300, 6, 6, 96, 160, True, 2, True),      # ... with a residual 256, both groups in a wave
+    (257, 4, 8, 64, 32, False, 0, True),      # 32 pixels: one group
+])
+def test_conv1x1_global_avgpool_waves_per_pixel_group(case):
+    test_conv1x1_global_avgpool(case)
+
+
 @pytest.mark.parametrize("seed", range(2))
 def test_first_layers_and_pooled_convolution_random_sweep(seed):
     """random shapes inside the one-launch kernels' domains: 30 convolutions with the average pooling inside (1 to 64
