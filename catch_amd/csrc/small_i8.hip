@@ -61,6 +61,7 @@ __device__ __forceinline__ void small_ds_write(unsigned addr, v4i v) {
 // HALF_BIAS: there is a bias, in half precision (a choice at run time costs every launch 0.05 us).
 template <int T, int NW, bool DENSE, int IN, bool DUAL, bool HALF_BIAS>
 __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev e) {
+  fetch_arguments<sizeof(SmallParams) + sizeof(EpiDev)>();
   resolve_exp2(e);
   constexpr int SLOTS = 2, BKB = 128;
   constexpr int SLOT_BYTES = 2 * T * BKB, WAVE_BYTES = SLOTS * SLOT_BYTES;
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       k[h] = (unsigned)((first + s) * BKB + (chunk0 ^ (4 * h)) * 16);
-      ok[h] = (s < mine) & (k[h] < (unsigned)o.K);
+      ok[h] = k[h] < (unsigned)o.K;
       koff[h] = k[h];
       dy[h] = dx[h] = 0;
       if constexpr (!DENSE) {
@@ -204,10 +205,11 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     const unsigned a_addr = my_addr + (unsigned)(frow * BKB);
     const unsigned sw = (unsigned)((frow >> 1) & 7);
     issue(0);
-    if constexpr (IN == IN_I8) issue(1);  // (past the slice: nothing but zeros, so that the number in flight stays the same)
+    if (IN == IN_I8 && mine > 1) issue(1);
     for (int s = 0; s < mine; ++s) {
       if constexpr (IN == IN_I8) {
-        CATCHQ_SMALL_VMCNT(NI);
+        if (s + 1 < mine) CATCHQ_SMALL_VMCNT(NI);
+        else CATCHQ_SMALL_VMCNT(0);
       } else {
         // the step's activations have arrived, and with them its filters: quantized into the slot, as a transfer
         // would have left them; then the next step's loads
@@ -217,8 +219,12 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
 #pragma unroll
         for (int j = 0; j < NA; ++j)
           small_ds_write(my_addr + (unsigned)((s & 1) * SLOT_BYTES + j * 1024 + lane * 16), q[j]);
-        issue(s + 1);
-        CATCHQ_SMALL_VMCNT(NA + NA * RAW < 63 ? NA + NA * RAW : 63);  // (what the counter holds)
+        if (s + 1 < mine) {
+          issue(s + 1);
+          CATCHQ_SMALL_VMCNT(NA + NA * RAW < 63 ? NA + NA * RAW : 63);  // (what the counter holds)
+        } else {
+          CATCHQ_SMALL_VMCNT(0);
+        }
       }
       const unsigned base = a_addr + (unsigned)((s & 1) * SLOT_BYTES);
       v4i fa[SUB], fb[SUB];
@@ -230,7 +236,7 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       }
 #pragma unroll
       for (int u = 0; u < SUB; ++u) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(fa[u]), "+v"(fb[u])::"memory");
-      if constexpr (IN == IN_I8) issue(s + 2);  // the slot has been read
+      if (IN == IN_I8 && s + 2 < mine) issue(s + 2);  // the slot has been read
       // operands swapped (weights as A): a lane ends up with four consecutive channels of one pixel
 #pragma unroll
       for (int u = 0; u < SUB; ++u) {
@@ -238,7 +244,6 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
         else acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(fb[u], fa[u], acc, 0, 0, 0);
       }
     }
-    CATCHQ_SMALL_VMCNT(0);  // the transfers past the slice have landed: the slots are free
     int *part = reinterpret_cast<int *>(my) + frow * PITCH + fk * 4;
     if constexpr (T == 32) {
 #pragma unroll
@@ -262,14 +267,20 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
     const int px = t / CPR, cg = t % CPR;
     const int m = m0 + px;
     const int *part = reinterpret_cast<const int *>(lds) + px * PITCH + cg * 4;
-    v4i a = *reinterpret_cast<const v4i *>(part);
-    for (int w = 1; w < main_active; ++w) a += *reinterpret_cast<const v4i *>(part + w * (WAVE_BYTES / 4));
+    // every wave's slot at once, also of those without a step (one after the other they cost 100 clocks each)
+    v4i parts[NW], a = {0, 0, 0, 0};
+#pragma unroll
+    for (int w = 0; w < NW; ++w) parts[w] = *reinterpret_cast<const v4i *>(part + w * (WAVE_BYTES / 4));
+#pragma unroll
+    for (int w = 0; w < NW; ++w)
+      if (w < main_active) a += parts[w];
     v4f res = c_res[r];
     if constexpr (DUAL) {
       const int active = min(steps_of(p.side[1].K), NW - main_group);
-      const int *part2 = part + main_group * (WAVE_BYTES / 4);
-      v4i a2 = *reinterpret_cast<const v4i *>(part2);
-      for (int w = 1; w < active; ++w) a2 += *reinterpret_cast<const v4i *>(part2 + w * (WAVE_BYTES / 4));
+      v4i a2 = {0, 0, 0, 0};
+#pragma unroll
+      for (int w = 0; w < NW; ++w)
+        if (w >= main_group && w < main_group + active) a2 += parts[w];
       EpiDev es = {};
       es.exp2 = p.sc.exp2; es.chan_div = p.sc.chan_div; es.chan_rcp = p.sc.chan_rcp; es.bias = p.sc.bias;
       const EpiLane ls = epi_lane_finish<EpiGeneric>(s_div, s_rcp, s_bias, es);
