@@ -253,70 +253,89 @@ __global__ __launch_bounds__(64 * NW) void small_i8_kernel(SmallParams p, EpiDev
       *reinterpret_cast<v4i *>(part) = acc;
     }
   }
-  __syncthreads();
-  if (!epi_wave) return;
+  if (!epi_wave) {
+    __syncthreads();
+    return;
+  }
 
   // ---- partial sums -> outputs ---------------------------------------------------------------------------------------
   auto steps_of = [&](int K) { return (K + BKB - 1) / BKB; };
   const int main_group = DUAL ? p.main_waves : NW;
   const int main_active = min(steps_of(p.side[0].K), main_group);
-#pragma unroll
-  for (int r = 0; r < ROUNDS; ++r) {
-    const int t = threadIdx.x + r * 64 * NW;
-    if (t >= EPI_LANES) break;
-    const int px = t / CPR, cg = t % CPR;
-    const int m = m0 + px;
-    const int *part = reinterpret_cast<const int *>(lds) + px * PITCH + cg * 4;
-    // every wave's slot at once, also of those without a step (one after the other they cost 100 clocks each)
-    v4i parts[NW], a = {0, 0, 0, 0};
+  const int second_active = DUAL ? min(steps_of(p.side[1].K), NW - main_group) : 0;
+  // main and shortcut sums of lane t, four channels of a pixel: every wave's slot at once, also of those without a step (one after
+  // the other they cost 100 clocks each)
+  auto sums_of = [&](int t, v4i &a, v4i &a2) {
+    const int *part = reinterpret_cast<const int *>(lds) + t / CPR * PITCH + t % CPR * 4;
+    v4i parts[NW];
 #pragma unroll
     for (int w = 0; w < NW; ++w) parts[w] = *reinterpret_cast<const v4i *>(part + w * (WAVE_BYTES / 4));
+    a = a2 = v4i{0, 0, 0, 0};
 #pragma unroll
-    for (int w = 0; w < NW; ++w)
+    for (int w = 0; w < NW; ++w) {
       if (w < main_active) a += parts[w];
+      if (DUAL && w >= main_group && w < main_group + second_active) a2 += parts[w];
+    }
+  };
+  EpiLane ls;  // the shortcut's constants
+  if constexpr (DUAL) {
+    EpiDev es = {};
+    es.exp2 = p.sc.exp2; es.chan_div = p.sc.chan_div; es.chan_rcp = p.sc.chan_rcp; es.bias = p.sc.bias;
+    ls = epi_lane_finish<EpiGeneric>(s_div, s_rcp, s_bias, es);
+  }
+  auto residual = [&](int r, const v4i &a2) {
     v4f res = c_res[r];
     if constexpr (DUAL) {
-      const int active = min(steps_of(p.side[1].K), NW - main_group);
-      v4i a2 = {0, 0, 0, 0};
 #pragma unroll
-      for (int w = 0; w < NW; ++w)
-        if (w >= main_group && w < main_group + active) a2 += parts[w];
-      EpiDev es = {};
-      es.exp2 = p.sc.exp2; es.chan_div = p.sc.chan_div; es.chan_rcp = p.sc.chan_rcp; es.bias = p.sc.bias;
-      const EpiLane ls = epi_lane_finish<EpiGeneric>(s_div, s_rcp, s_bias, es);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) res[u] = epi_dequant1((float)a2[u], u, ls, es.exp2);
+      for (int u = 0; u < 4; ++u) res[u] = epi_dequant1((float)a2[u], u, ls, p.sc.exp2);
     }
-    if (m >= p.M || ec >= p.N) continue;
-    const int64_t idx = (int64_t)m * p.N + ec;
-    if (!vec) {
+    return res;
+  };
+  auto run = [&](auto spec) {
+    typedef decltype(spec) S;
+    EpiLane L = epi_lane_finish<S>(c_div, c_rcp, HALF_BIAS ? half4_values(c_bias16) : c_bias, e);  // (in front of the barrier)
+    if constexpr (DUAL) {
+      L.use_res = true;
+      L.res_after = e.resid_after != 0;
+    }
+    __syncthreads();
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        if (ec + u >= p.N) break;
-        if (e.acc_out) e.acc_out[idx + u] = a[u];
-        epi_store(epi_value((float)a[u], idx + u, ec + u, e), idx + u, e);
+    for (int r = 0; r < ROUNDS; ++r) {
+      const int t = threadIdx.x + r * 64 * NW, m = m0 + t / CPR;
+      if (t >= EPI_LANES) break;
+      v4i a, a2;
+      sums_of(t, a, a2);
+      if (m < p.M && ec < p.N) epi_vec4<S>(a, residual(r, a2), L, (int64_t)m * p.N + ec, e);
+    }
+  };
+  switch (p.epi) {
+    case EPI_Q8_RELU: run(EpiOf<EPI_Q8_RELU>::type{}); break;
+    case EPI_RES_Y_Q8: run(EpiOf<EPI_RES_Y_Q8>::type{}); break;
+    case EPI_Y32: run(EpiOf<EPI_Y32>::type{}); break;
+    case EPI_RES_Q8: run(EpiOf<EPI_RES_Q8>::type{}); break;
+    case EPI_Q8_RELU6: run(EpiOf<EPI_Q8_RELU6>::type{}); break;
+    case EPI_Y16: run(EpiOf<EPI_Y16>::type{}); break;
+    case EPI_Y16_STEPS: run(EpiOf<EPI_Y16_STEPS>::type{}); break;
+    case EPI_SCALAR:
+      __syncthreads();
+#pragma unroll
+      for (int r = 0; r < ROUNDS; ++r) {
+        const int t = threadIdx.x + r * 64 * NW, m = m0 + t / CPR;
+        if (t >= EPI_LANES) break;
+        v4i a, a2;
+        sums_of(t, a, a2);
+        const int64_t idx = (int64_t)m * p.N + ec;
+        if (m < p.M) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            if (ec + u >= p.N) break;
+            if (e.acc_out) e.acc_out[idx + u] = a[u];
+            epi_store(epi_value((float)a[u], idx + u, ec + u, e), idx + u, e);
+          }
+        }
       }
-      continue;
-    }
-    auto run = [&](auto spec) {
-      typedef decltype(spec) S;
-      EpiLane L = epi_lane_finish<S>(c_div, c_rcp, HALF_BIAS ? half4_values(c_bias16) : c_bias, e);
-      if constexpr (DUAL) {
-        L.use_res = true;
-        L.res_after = e.resid_after != 0;
-      }
-      epi_vec4<S>(a, res, L, idx, e);
-    };
-    switch (p.epi) {
-      case EPI_Q8_RELU: run(EpiOf<EPI_Q8_RELU>::type{}); break;
-      case EPI_RES_Y_Q8: run(EpiOf<EPI_RES_Y_Q8>::type{}); break;
-      case EPI_Y32: run(EpiOf<EPI_Y32>::type{}); break;
-      case EPI_RES_Q8: run(EpiOf<EPI_RES_Q8>::type{}); break;
-      case EPI_Q8_RELU6: run(EpiOf<EPI_Q8_RELU6>::type{}); break;
-      case EPI_Y16: run(EpiOf<EPI_Y16>::type{}); break;
-      case EPI_Y16_STEPS: run(EpiOf<EPI_Y16_STEPS>::type{}); break;
-      default: run(EpiGeneric{}); break;
-    }
+      break;
+    default: run(EpiGeneric{}); break;
   }
 }
 
