@@ -34,8 +34,12 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
 bool float_rows_takes(bool half, int64_t M, int64_t N, int64_t K, const EpiDev &e);
 int float_rows(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, const EpiDev &e,
                hipStream_t s);
-int64_t packed_digits_bytes(int64_t N, int64_t K);
-int pack_digits(const void *w, int64_t N, int64_t K, int64_t ld, void *packed, hipStream_t s);
+int64_t packed_digits_bytes(int64_t N, int64_t taps, int64_t K);
+int pack_digits(const void *w, int64_t N, int64_t taps, int64_t K, int64_t ld, void *packed, hipStream_t s);
+int64_t conv_digits_bytes(int N, int H, int W, int Ci, int Co, int kh, int kw, int Ho, int Wo, const EpiDev &e);
+int conv_digits(const void *x, bool half, int position, int x_ci, bool apart, const void *packed, int N, int H, int W, int Ci, int Co,
+                int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, void *digits, const EpiDev &e,
+                hipStream_t s);
 int64_t gemm_digits_bytes(int64_t M, int64_t N, int64_t K, const EpiDev &e);
 int gemm_digits(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, void *digits,
                 const EpiDev &e, hipStream_t s);
@@ -521,8 +525,8 @@ CATCHQ_API int catchq_conv3x3_i8_packed(const void *x, const void *packed, int n
 
 CATCHQ_API int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes) {
   if (!bytes || n <= 0 || k <= 0) return CATCHQ_ERR_ARG;
-  if (k > kDigitsMaxK || n >= (1ll << 31) || packed_digits_bytes(n, k) >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
-  *bytes = (size_t)packed_digits_bytes(n, k);
+  if (k > kDigitsMaxK || n >= (1ll << 31) || packed_digits_bytes(n, 1, k) >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
+  *bytes = (size_t)packed_digits_bytes(n, 1, k);
   return CATCHQ_OK;
 }
 
@@ -531,7 +535,54 @@ CATCHQ_API int catchq_pack_digits(const void *w, int64_t n, int64_t k, int64_t l
   const int st = catchq_packed_digits_size(n, k, &bytes);
   if (st != CATCHQ_OK) return st;
   if (!w || !packed || ld < k || !aligned16(packed)) return CATCHQ_ERR_ARG;
-  return pack_digits(w, n, k, ld, packed, as_stream(stream));
+  return pack_digits(w, n, 1, k, ld, packed, as_stream(stream));
+}
+
+CATCHQ_API int catchq_packed_conv_digits_size(int64_t n, int64_t taps, int64_t ci, size_t *bytes) {
+  if (!bytes || n <= 0 || taps <= 0 || ci <= 0) return CATCHQ_ERR_ARG;
+  if (taps < 2 || taps > 25 || ci >= (1 << 14) || n >= (1ll << 31) || packed_digits_bytes(n, taps, ci) >= (1ll << 31))
+    return CATCHQ_ERR_UNSUPPORTED;
+  *bytes = (size_t)packed_digits_bytes(n, taps, ci);
+  return CATCHQ_OK;
+}
+
+CATCHQ_API int catchq_pack_conv_digits(const void *w, int64_t n, int64_t taps, int64_t ci, void *packed, catchq_stream_t stream) {
+  size_t bytes = 0;
+  const int st = catchq_packed_conv_digits_size(n, taps, ci, &bytes);
+  if (st != CATCHQ_OK) return st;
+  if (!w || !packed || !aligned16(packed)) return CATCHQ_ERR_ARG;
+  return pack_digits(w, n, taps, ci, taps * ci, packed, as_stream(stream));
+}
+
+CATCHQ_API int catchq_float_conv2d_digits_workspace_size(const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, size_t *bytes) {
+  int ho, wo;
+  int st = check_conv(desc, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  if (!bytes) return CATCHQ_ERR_ARG;
+  const catchq_conv_desc_t &d = *desc;
+  *bytes = 0;
+  if (d.groups == 1 && d.n > 0)
+    *bytes = (size_t)conv_digits_bytes(d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, ho, wo, make_epi(epilogue, (int64_t)d.n * ho * wo * d.co));
+  return *bytes ? CATCHQ_OK : CATCHQ_ERR_UNSUPPORTED;
+}
+
+CATCHQ_API int catchq_float_conv2d_digits(const void *x, int x_dtype, int x_position, int x_ci, int x_nchw, const void *packed,
+                                          const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, void *workspace,
+                                          size_t workspace_bytes, catchq_stream_t stream) {
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  size_t bytes = 0;
+  const int st = catchq_float_conv2d_digits_workspace_size(desc, epilogue, &bytes);
+  if (st != CATCHQ_OK) return st;
+  const catchq_conv_desc_t &d = *desc;
+  if (x_position < -126 || x_position > 126 || x_ci <= 0 || x_ci > d.ci) return CATCHQ_ERR_ARG;
+  if (!x || !packed || !workspace || workspace_bytes < bytes || !aligned16(packed) || !aligned16(workspace)) return CATCHQ_ERR_ARG;
+  int ho, wo;
+  (void)check_conv(desc, &ho, &wo);
+  return conv_digits(x, x_dtype == CATCHQ_F16, x_position, x_ci, x_nchw != 0, packed, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
+                     d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, workspace,
+                     make_epi(epilogue, (int64_t)d.n * ho * wo * d.co), as_stream(stream));
 }
 
 CATCHQ_API int catchq_float_linear_digits_workspace_size(int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue,

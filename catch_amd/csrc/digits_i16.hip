@@ -1,9 +1,9 @@
-// int16 linears on operands split into digits beforehand: exact in 64 bits.
+// int16 linears and convolutions on operands split into digits beforehand: exact in 64 bits.
 //
 // With  x = 256 xh + xl + 128  and  w = 256 wh + wl + 128  (high byte signed, low byte biased into int8)
 //   sum x w = 65536 S_hh + 256 (S_hl + S_lh) + S_ll + 128 (X + sum w),   X = sum (256 xh + xl)
 // over the K positions walked; positions beyond K and rows beyond M and N hold the value 0.  The four sums are int8 products
-// (|S| <= K 2^14, K <= 2^13), the combination is done in fp64, which holds every value of it, and its one
+// (|S| <= K 2^14, K < 2^14), the combination is done in fp64, which holds every value of it, and its one
 // conversion to fp32 is the int64 sum's.
 //
 // The kernel for int16 operands as they lie splits every fragment in every wave that reads it: 20 vector operations a fragment
@@ -17,7 +17,11 @@
 // and the epilogue (4000).  Tried without gain: floats converted by the blocks themselves (every run of columns converts them
 // again: 67 us), K shared between two groups of waves.
 //
-// Measured: see gemm_digits_bytes below.
+// A convolution's activations lie by pixels instead, [pixel][channel / 32][high, low digits of 32 channels] with a pixel of zeros behind
+// the last one, and a transfer of 32 pixels' digits is 64 lanes' addresses: tap and channels are the wave's, whether the tap is in the
+// image a bit of the lane's.  It lands as the linear's do.
+//
+// Measured: see gemm_digits_bytes and conv_digits_bytes below.
 #include <type_traits>
 
 #include "igemm_common.h"
@@ -45,35 +49,75 @@ __device__ __forceinline__ void digit_wait(v4i (&f)[2][2]) {  // at most N LDS r
   for (int i = 0; i < 2; ++i) asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(f[i][0]), "+v"(f[i][1]) : "n"(N) : "memory");
 }
 
-template <int EPI, bool RAGGED>
+struct DigitConv {
+  int H, W, Ho, Wo, ph, pw, sh, sw, dh, dw, kh, kw;
+  int c32;              // channels / 32, rounded up
+  unsigned pitch;       // bytes of a pixel
+  unsigned zero;        // the pixel of zeros
+  unsigned magic_c32, mask_c32, magic_kw, mask_kw;  // ceil(2^32 / d), mask 0; for d = 1 magic 0, mask ~0
+};
+struct NoConv {};
+__device__ __forceinline__ unsigned digit_div(unsigned n, unsigned magic, unsigned mask) { return __umulhi(n, magic) + (n & mask); }
+
+// WN of the four waves side by side, 32 columns each; SUB: sub-steps of a slab
+template <int EPI, bool RAGGED, int WN, int SUB, class Conv>
 __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__restrict__ A, const int8_t *__restrict__ B,
-                                                                      const int *__restrict__ col_sums, DigitParams p, EpiDev e) {
+                                                                      const int *__restrict__ col_sums, DigitParams p, EpiDev e, Conv c) {
+  constexpr bool CONV = !std::is_same<Conv, NoConv>::value;
   resolve_exp2(e);
-  constexpr int NW = 4, BM = 64, TM = 2, SUB = 8, RING = 8, STAGE = 36;
-  constexpr int PIECES = TM * SUB * 2, SLAB_BYTES = PIECES * 1024;  // of 256 values of K: [row / 32][sub-step][digit]
+  constexpr int NW = 4, BM = 64 * (NW / WN), TM = 2, RING = SUB, STAGE = 36;
+  constexpr int ROW_TILES = BM / 32, PIECES = ROW_TILES * SUB * 2, SLAB_BYTES = PIECES * 1024;  // [row / 32][sub-step][digit]
   extern __shared__ __attribute__((aligned(16))) int8_t lds_dyn[];
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), wn = wave % WN, wm = wave / WN;
   // a die's blocks (every eighth) cover a rectangle of tiles: what its L2 takes in is a part of the rows and a part of the weights
   const int die = blockIdx.x & 7, place = blockIdx.x >> 3;
   const int tile_m = die / p.die_cols * p.rect_m + place / p.rect_n, chunk = die % p.die_cols * p.rect_n + place % p.rect_n;
   if (tile_m >= p.tiles_m || chunk >= p.tiles_n) return;
-  const int64_t m0 = (int64_t)tile_m * BM;
-  const int n32 = (p.N + 31) / 32, m32 = (int)((p.M + 31) / 32), t = chunk * NW + wave;
+  const int64_t m0 = (int64_t)tile_m * BM + wm * 64;  // this wave's rows
+  const int n32 = (p.N + 31) / 32, m32 = (int)((p.M + 31) / 32), t = chunk * WN + wn;
+  const bool columns = t < n32;  // (without: the wave helps with the rows)
   const __amdgpu_buffer_rsrc_t rsrc_a = __builtin_amdgcn_make_buffer_rsrc((void *)A, 0, (int)p.a_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t rsrc_b = __builtin_amdgcn_make_buffer_rsrc((void *)B, 0, (int)p.b_bytes, 0x00020000);
   const unsigned lds_base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) int8_t *)lds_dyn;
   const int my16 = lane * 16;
 
   // rows: piece j of a slab = (row tile j / (2 SUB), sub-step j / 2 % SUB, digit j % 2).  Pieces past the last sub-step or row
-  // tile repeat the last one: their products are not taken, their rows not stored.
+  // tile repeat the last one (a convolution's are zeros): their products are not taken, or met by zeros, their rows not stored.
+  constexpr int MINE = PIECES / NW;  // pieces a wave moves, all of one row tile
+  static_assert(ROW_TILES <= NW);
+  const int row_tile = wave * MINE / (2 * SUB);
+  unsigned px_off = 0, px_zero = 0, px_taps = 0;  // of this lane's pixel: its first tap, a pixel of zeros, bit per tap in the image
+  if constexpr (CONV) {
+    const int64_t m = (int64_t)tile_m * BM + row_tile * 32 + (lane & 31);
+    const unsigned mm = (unsigned)(m < p.M ? m : 0), t = mm / (unsigned)c.Wo, img = t / (unsigned)c.Ho;
+    const int hi = (int)(t - img * (unsigned)c.Ho) * c.sh - c.ph, wi = (int)(mm - t * (unsigned)c.Wo) * c.sw - c.pw;
+    px_off = ((img * (unsigned)c.H + (unsigned)hi) * (unsigned)c.W + (unsigned)wi) * c.pitch + (unsigned)(lane >> 5) * 16u;  // mod 2^32
+    px_zero = c.zero + (unsigned)(lane >> 5) * 16u;
+    unsigned cols = 0;
+    for (int q = 0; q < c.kw; ++q) cols |= ((unsigned)(wi + q * c.dw) < (unsigned)c.W ? 1u : 0u) << q;
+    for (int r = 0; r < c.kh; ++r) px_taps |= (m < p.M && (unsigned)(hi + r * c.dh) < (unsigned)c.H ? cols : 0u) << (r * c.kw);
+  }
   auto issue_a = [&](int slab) {
 #pragma unroll
-    for (int i = 0; i < PIECES / NW; ++i) {
-      const int j = wave * (PIECES / NW) + i;
-      const int run = min(tile_m * TM + j / (2 * SUB), m32 - 1), ks = min(slab * SUB + j / 2 % SUB, p.nk - 1);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(lds_dyn + (slab & 1) * SLAB_BYTES + j * 1024), 16, my16,
-                                               ((run * p.nk + ks) * 2 + j % 2) * 1024, 0, 0);
+    for (int i = 0; i < MINE; i += 2) {
+      const int j = wave * MINE + i, ks = slab * SUB + j / 2 % SUB;
+      lds_ptr_t dst = (lds_ptr_t)(lds_dyn + (slab & 1) * SLAB_BYTES + j * 1024);
+      if constexpr (CONV) {
+        const unsigned tap = digit_div((unsigned)ks, c.magic_c32, c.mask_c32), ch = (unsigned)ks - tap * (unsigned)c.c32;
+        const unsigned r = digit_div(tap, c.magic_kw, c.mask_kw), q = tap - r * (unsigned)c.kw;
+        const unsigned at = (r * (unsigned)(c.dh * c.W) + q * (unsigned)c.dw) * c.pitch;
+        unsigned from = (px_taps >> tap) & 1u ? px_off + at : px_zero;
+        asm volatile("" : "+v"(from));  // one select and one load, not two loads under complementary masks
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, (int)from, (int)(ch * 64u), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(lds_dyn + (slab & 1) * SLAB_BYTES + j * 1024 + 1024), 16, (int)from,
+                                                 (int)(ch * 64u + 32u), 0, 0);
+      } else {
+        const int from = (min(tile_m * ROW_TILES + row_tile, m32 - 1) * p.nk + min(ks, p.nk - 1)) * 2048;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, dst, 16, my16, from, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc_a, (lds_ptr_t)(lds_dyn + (slab & 1) * SLAB_BYTES + j * 1024 + 1024), 16, my16,
+                                                 from + 1024, 0, 0);
+      }
     }
   };
   v4i fb[RING][2];  // this wave's weights of a slab; a slot is refilled for the next slab
@@ -128,7 +172,7 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
     __syncthreads();  // everyone's; and nobody reads the other half of the buffer any more
     if (slab + 1 < slabs) issue_a(slab + 1);
     const int first = slab * SUB, sub = min(SUB, p.nk - first);  // (four or eight)
-    const unsigned at = lds_base + (unsigned)((slab & 1) * SLAB_BYTES + my16);
+    const unsigned at = lds_base + (unsigned)((slab & 1) * SLAB_BYTES + wm * TM * SUB * 2048 + my16);
     v4i fa[2][TM][2];
     auto fetch_a = [&](v4i (&f)[TM][2], int s) {
 #pragma unroll
@@ -143,13 +187,15 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
       for (int r = FROM; r < FROM + 4; ++r) {
         fetch_a(fa[(r + 1) & 1], r + 1 < RING ? r + 1 : r);  // under way before this step's multiplications
         digit_wait<2 * TM>(fa[r & 1]);
-        multiply(fa[r & 1], fb[r]);
+        if (!CONV || columns) multiply(fa[r & 1], fb[r]);  // (the question costs a linear 4 %)
         fetch_b(fb[r], first + RING + r);
-        if (wave == r % NW) add_digits(fa[r & 1]);  // a wave takes the sums of every NW-th step
+        if (wn == r % WN) add_digits(fa[r & 1]);  // a wave takes the sums of every WN-th step
       }
     };
     four(std::integral_constant<int, 0>{});
-    if (sub > 4) four(std::integral_constant<int, 4>{});
+    if constexpr (SUB > 4) {
+      if (sub > 4) four(std::integral_constant<int, 4>{});
+    }
     digit_wait<0>(fa[0]);  // (the spare read)
   }
 
@@ -163,14 +209,14 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
 #pragma unroll
   for (int i = 0; i < TM; ++i) {  // a lane holds the sums of row (lane & 31) over its half of a sub-step
     const int part = 256 * xh_sum[i] + xl_sum[i], both = part + __shfl_xor(part, 32, 64);
-    if (fhalf == 0) rows[wave * BM + i * 32 + frow] = both;
+    if (fhalf == 0) rows[wave * 64 + i * 32 + frow] = both;
   }
-  int *const stage = rows + NW * BM + wave * 3 * 32 * STAGE;
+  int *const stage = rows + NW * 64 + wave * 3 * 32 * STAGE;
   __syncthreads();
-  if (t >= n32) return;
+  if (!columns) return;
   int my_row = 0;  // the digit sum of row `lane`
 #pragma unroll
-  for (int w = 0; w < NW; ++w) my_row += rows[w * BM + lane];
+  for (int w = 0; w < WN; ++w) my_row += rows[(wm * WN + w) * 64 + lane];
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -190,7 +236,7 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
       v4f sums;
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        const int both = 2 * m16[k] + row_sum + col_sum[k];  // (K <= 8192)
+        const int both = 2 * m16[k] + row_sum + col_sum[k];  // (fewer than 2^14 positions of K: each less than 2^17)
         sums[k] = (float)__builtin_fma((double)h16[k], 65536.0, __builtin_fma((double)both, 128.0, (double)l16[k]));
       }
       const int64_t m = m0 + i * 32 + row;
@@ -244,31 +290,32 @@ __global__ __launch_bounds__(256) void quantize_digits_kernel(const TIn *__restr
 }
 
 // w [N, ld] int16, K values of a row used -> digits, zeros beyond N and K, and the rows' sums (once per weight that is
-// read packed).  A block takes 32 rows, its waves every sixteenth sub-step: bound by the latency of the steps that a wave
-// takes one after the other.  1001 x 1000: 5.7 us; a pass that packs (1379 rows, half, on a new weight) 191 us with one wave for
-// a block's rows, 137 with sixteen.
+// read packed).  Rows of `taps` runs of K values: every run starts on a sub-step.  A block takes 32 rows, its waves every sixteenth
+// sub-step: bound by the latency of the steps that a wave takes one after the other.  1001 x 1000: 5.7 us; a pass that packs (1379 rows,
+// half, on a new weight) 191 us with one wave for a block's rows, 137 with sixteen.
 constexpr int kPackWaves = 16;
 __global__ __launch_bounds__(64 * kPackWaves) void pack_digits_kernel(const int16_t *__restrict__ w, int8_t *__restrict__ out,
-                                                                      int *__restrict__ sums, int N, int K, int64_t ld, int nk) {
+                                                                      int *__restrict__ sums, int N, int taps, int K, int64_t ld, int nk) {
   struct __attribute__((aligned(2))) run16 { int16_t v[16]; };
   __shared__ int parts[kPackWaves][32];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = blockIdx.x * 32 + (lane & 31);
   const int16_t *const row = w + (n < N ? n : N - 1) * ld;
   int sum = 0;
   for (int ks = wave; ks < nk; ks += kPackWaves) {
-    const int k = ks * 32 + (lane >> 5) * 16;
+    const int tap = taps > 1 ? ks / ((K + 31) / 32) : 0, k = (ks - tap * ((K + 31) / 32)) * 32 + (lane >> 5) * 16;
+    const int16_t *const run = row + (tap < taps ? tap : 0) * (int64_t)K;
     int q[16];
     if (k + 16 <= K) {
-      const run16 t = *reinterpret_cast<const run16 *>(row + k);
+      const run16 t = *reinterpret_cast<const run16 *>(run + k);
 #pragma unroll
       for (int i = 0; i < 16; ++i) q[i] = t.v[i];
     } else {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) q[i] = k + i < K ? row[k + i] : 0;
+      for (int i = 0; i < 16; ++i) q[i] = k + i < K ? run[k + i] : 0;
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      q[i] = n < N ? q[i] : 0;
+      q[i] = n < N && tap < taps ? q[i] : 0;
       sum += q[i];
     }
     store_digits(out, blockIdx.x, ks, nk, lane, q);
@@ -287,12 +334,18 @@ __global__ __launch_bounds__(64 * kPackWaves) void pack_digits_kernel(const int1
 static int64_t digit_steps(int64_t K) { return (K + 127) / 128 * 4; }
 static int64_t digit_bytes(int64_t rows, int64_t K) { return (rows + 31) / 32 * digit_steps(K) * 2048; }
 
-int64_t packed_digits_bytes(int64_t N, int64_t K) { return digit_bytes(N, K) + (N + 31) / 32 * 32 * 4; }  // (with the sums)
+static int64_t conv_digit_steps(int64_t taps, int64_t Ci) { return (taps * ((Ci + 31) / 32) + 3) / 4 * 4; }
 
-int pack_digits(const void *w, int64_t N, int64_t K, int64_t ld, void *packed, hipStream_t s) {
-  int *sums = reinterpret_cast<int *>(static_cast<int8_t *>(packed) + digit_bytes(N, K));
-  pack_digits_kernel<<<(unsigned)((N + 31) / 32), 64 * kPackWaves, 0, s>>>((const int16_t *)w, (int8_t *)packed, sums, (int)N, (int)K,
-                                                                           ld, (int)digit_steps(K));
+// (with the sums)
+int64_t packed_digits_bytes(int64_t N, int64_t taps, int64_t K) {
+  return (N + 31) / 32 * ((taps > 1 ? conv_digit_steps(taps, K) : digit_steps(K)) * 2048 + 32 * 4);
+}
+
+// rows of `taps` runs of K values each, ld values apart
+int pack_digits(const void *w, int64_t N, int64_t taps, int64_t K, int64_t ld, void *packed, hipStream_t s) {
+  const int64_t nk = taps > 1 ? conv_digit_steps(taps, K) : digit_steps(K), runs = (N + 31) / 32;
+  int *sums = reinterpret_cast<int *>(static_cast<int8_t *>(packed) + runs * nk * 2048);
+  pack_digits_kernel<<<(unsigned)runs, 64 * kPackWaves, 0, s>>>((const int16_t *)w, (int8_t *)packed, sums, (int)N, (int)taps, (int)K, ld, (int)nk);
   return launch_status();
 }
 
@@ -301,6 +354,29 @@ static int digit_epilogue(int N, const EpiDev &e) {
   int epi = pick_epilogue(N, e);
   if (epi != EPI_Y32 && epi != EPI_Y16) epi = ragged_epilogue(N, e);
   return epi == EPI_Y32 || epi == EPI_Y16 ? epi : 0;
+}
+
+template <int WN, int SUB, class Conv>
+static int launch_digits(const int8_t *a, const int8_t *b, const int *sums, DigitParams p, const Conv &c, const EpiDev &e, hipStream_t s) {
+  constexpr int LDS_BYTES = 64 * 1024, BM = 64 * (4 / WN);  // two slabs; behind the loop 4 x (64 + 3 x 32 x 36) sums
+  static_assert(2 * BM / 32 * SUB * 2048 <= LDS_BYTES);
+  p.tiles_m = (int)((p.M + BM - 1) / BM);
+  p.tiles_n = ((p.N + 31) / 32 + WN - 1) / WN;
+  int64_t best = -1;
+  for (int cols = 1; cols <= 8; cols *= 2) {
+    const int64_t rm = (p.tiles_m + 8 / cols - 1) / (8 / cols), rn = (p.tiles_n + cols - 1) / cols;
+    // the tiles of the fullest die, then the rows that its L2 takes in: 4096 x 768 -> 3072 54.6 us with the rows' tiles dealt
+    // out alone, 50.4 in rectangles, 512 x 768 -> 3072 13.4 and 11.4
+    const int64_t cost = rm * rn * 64 + rm * 64 + rn * 128;
+    if (best < 0 || cost < best) best = cost, p.die_cols = cols, p.rect_m = (int)rm, p.rect_n = (int)rn;
+  }
+  const unsigned blocks = (unsigned)(8 * p.rect_m * p.rect_n);
+  const bool whole = pick_epilogue(p.N, e) == EPI_Y32 || pick_epilogue(p.N, e) == EPI_Y16;
+  auto kern = digit_epilogue(p.N, e) == EPI_Y32
+                  ? (whole ? gemm_digits_kernel<EPI_Y32, false, WN, SUB, Conv> : gemm_digits_kernel<EPI_Y32, true, WN, SUB, Conv>)
+                  : (whole ? gemm_digits_kernel<EPI_Y16, false, WN, SUB, Conv> : gemm_digits_kernel<EPI_Y16, true, WN, SUB, Conv>);
+  kern<<<blocks, 256, LDS_BYTES, s>>>(a, b, sums, p, e, c);
+  return launch_status();
 }
 
 // Bytes of the activations' digits where this route serves the product; 0: another one does.
@@ -336,23 +412,115 @@ int gemm_digits(const void *x, bool half, int position, const void *packed, int6
   else quantize_digits_kernel<float><<<quantizers, 256, 0, s>>>((const float *)x, (int8_t *)digits, M, (int)K, p.nk, tasks, -position);
   const int st = launch_status();
   if (st != CATCHQ_OK) return st;
-  constexpr int LDS_BYTES = 64 * 1024;  // two slabs; behind the loop 4 x (64 + 3 x 32 x 36) sums
-  p.tiles_m = (int)((p.M + 63) / 64);
-  p.tiles_n = ((p.N + 31) / 32 + 3) / 4;
-  int64_t best = -1;
-  for (int cols = 1; cols <= 8; cols *= 2) {
-    const int64_t rm = (p.tiles_m + 8 / cols - 1) / (8 / cols), rn = (p.tiles_n + cols - 1) / cols;
-    // the tiles of the fullest die, then the rows that its L2 takes in: 4096 x 768 -> 3072 54.6 us with the rows' tiles dealt
-    // out alone, 50.4 in rectangles, 512 x 768 -> 3072 13.4 and 11.4
-    const int64_t cost = rm * rn * 64 + rm * 64 + rn * 128;
-    if (best < 0 || cost < best) best = cost, p.die_cols = cols, p.rect_m = (int)rm, p.rect_n = (int)rn;
+  return launch_digits<4, 8>(a, b, sums, p, NoConv{}, e, s);
+}
+
+// floats -> digits by pixels, [pixel][channel / 32][high, low digits of 32 channels], and a pixel of zeros behind them.  APART: channels
+// lie HW values apart (NCHW), a lane takes 32 of them and lanes follow the pixels; otherwise two lanes have a pixel's 32 channels.
+template <typename TIn, bool APART>
+__global__ __launch_bounds__(256) void quantize_pixel_digits_kernel(const TIn *__restrict__ x, int8_t *__restrict__ out, int64_t pixels,
+                                                                    int C, int c32, unsigned HW, int64_t tasks, int neg_pos) {
+  struct __attribute__((aligned(sizeof(TIn)))) run16 { TIn v[16]; };
+  const int64_t task = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (task >= tasks) return;
+  constexpr int HALVES = APART ? 2 : 1;  // 16 channels each
+  int64_t px;
+  int ch;
+  if constexpr (APART) {
+    ch = (int)(task / (pixels + 1));
+    px = task - (int64_t)ch * (pixels + 1);
+    ch *= 32;
+  } else {
+    px = task / (2 * c32);
+    ch = (int)(task - px * (2 * c32)) * 16;
   }
-  const unsigned blocks = (unsigned)(8 * p.rect_m * p.rect_n);
-  const bool whole = pick_epilogue((int)N, e) == EPI_Y32 || pick_epilogue((int)N, e) == EPI_Y16;
-  auto kern = digit_epilogue((int)N, e) == EPI_Y32 ? (whole ? gemm_digits_kernel<EPI_Y32, false> : gemm_digits_kernel<EPI_Y32, true>)
-                                                   : (whole ? gemm_digits_kernel<EPI_Y16, false> : gemm_digits_kernel<EPI_Y16, true>);
-  kern<<<blocks, 256, LDS_BYTES, s>>>(a, b, sums, p, e);
-  return launch_status();
+  float v[HALVES][16];
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[h][i] = 0.0f;
+  if (px < pixels) {
+    if constexpr (APART) {
+      const int64_t img = px / HW, at = img * C * HW + (px - img * HW);
+#pragma unroll
+      for (int i = 0; i < 32; ++i)
+        if (ch + i < C) v[i / 16][i % 16] = (float)x[at + (int64_t)(ch + i) * HW];
+    } else {
+      const TIn *const row = x + px * C + ch;
+      if (ch + 16 <= C) {
+        const run16 t = *reinterpret_cast<const run16 *>(row);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[0][i] = (float)t.v[i];
+      } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+          if (ch + i < C) v[0][i] = (float)row[i];
+      }
+    }
+  }
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h) {
+    v4i c[2], hi, lo;
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const int a = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(v[h][g * 8 + d * 2], neg_pos)));
+        const int b = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(v[h][g * 8 + d * 2 + 1], neg_pos)));
+        c[g][d] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pk_i16(a, b));  // (saturates)
+      }
+    split_i16(c[0], c[1], hi, lo);
+    v4i *const dst = reinterpret_cast<v4i *>(out + (px * c32 + ch / 32) * 64 + (ch & 16)) + h;
+    dst[0] = hi;
+    dst[2] = lo;
+  }
+}
+
+// Bytes of the activations' digits where this route serves the convolution; 0: another one does.
+int64_t conv_digits_bytes(int N, int H, int W, int Ci, int Co, int kh, int kw, int Ho, int Wo, const EpiDev &e) {
+  const int64_t M = (int64_t)N * Ho * Wo, pixels = (int64_t)N * H * W, c32 = (Ci + 31) / 32, taps = (int64_t)kh * kw;
+  const int64_t bytes = (pixels + 1) * c32 * 64;
+  if (taps > 25 || conv_digit_steps(taps, Ci) * 32 >= (1 << 14) || M >= (1ll << 31) - 128 || bytes >= (1ll << 31)) return 0;
+  if (packed_digits_bytes(Co, taps, Ci) >= (1ll << 31) || e.resid || e.q || e.acc_out || !digit_epilogue(Co, e)) return 0;
+  return conv_digits_sizes(M, Co, Ci, taps, e.cus) ? bytes : 0;
+}
+
+// x: x_ci channels of the filters' Ci, [N, H, W, x_ci] or (apart) [N, x_ci, H, W] floats or halfs; packed: pack_digits of Co rows of
+// kh * kw runs of Ci
+int conv_digits(const void *x, bool half, int position, int x_ci, bool apart, const void *packed, int N, int H, int W, int Ci, int Co,
+                int kh, int kw, int ph, int pw, int sh, int sw, int dh, int dw, int Ho, int Wo, void *digits, const EpiDev &e,
+                hipStream_t s) {
+  const int64_t pixels = (int64_t)N * H * W;
+  const int c32 = (Ci + 31) / 32;
+  const int64_t tasks = (pixels + 1) * c32 * (apart ? 1 : 2);
+  const unsigned quantizers = (unsigned)((tasks + 255) / 256), hw = (unsigned)((int64_t)H * W);
+  int8_t *const a = static_cast<int8_t *>(digits);
+  auto quantize = [&](auto kern, auto *from) { kern<<<quantizers, 256, 0, s>>>(from, a, pixels, x_ci, c32, hw, tasks, -position); };
+  if (half) {
+    if (apart) quantize(quantize_pixel_digits_kernel<_Float16, true>, (const _Float16 *)x);
+    else quantize(quantize_pixel_digits_kernel<_Float16, false>, (const _Float16 *)x);
+  } else {
+    if (apart) quantize(quantize_pixel_digits_kernel<float, true>, (const float *)x);
+    else quantize(quantize_pixel_digits_kernel<float, false>, (const float *)x);
+  }
+  const int st = launch_status();
+  if (st != CATCHQ_OK) return st;
+  DigitParams p = {};
+  p.M = (int64_t)N * Ho * Wo;
+  p.N = Co;
+  p.nk = (int)conv_digit_steps(kh * kw, Ci);
+  p.a_bytes = (unsigned)((pixels + 1) * c32 * 64);
+  p.b_bytes = (unsigned)((int64_t)(Co + 31) / 32 * p.nk * 2048);
+  DigitConv c = {H, W, Ho, Wo, ph, pw, sh, sw, dh, dw, kh, kw, c32, (unsigned)c32 * 64u, (unsigned)(pixels * c32 * 64), 0, 0, 0, 0};
+  auto magic = [](unsigned d, unsigned *m, unsigned *mask) {  // (dividends and divisors below 2^16)
+    *m = d <= 1 ? 0u : (unsigned)(((1ull << 32) + d - 1) / d);
+    *mask = d <= 1 ? ~0u : 0u;
+  };
+  magic(c32, &c.magic_c32, &c.mask_c32);
+  magic(kw, &c.magic_kw, &c.mask_kw);
+  const int8_t *const b = static_cast<const int8_t *>(packed);
+  const int *const sums = reinterpret_cast<const int *>(b + p.b_bytes);
+  return Co <= 64 ? launch_digits<2, 4>(a, b, sums, p, c, e, s) : launch_digits<4, 8>(a, b, sums, p, c, e, s);
 }
 
 }  // namespace catchq

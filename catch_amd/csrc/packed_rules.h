@@ -23,6 +23,16 @@ inline bool digits_sizes(int64_t m, int64_t n, int64_t k, int cus) {
   return k >= 32 && k <= kDigitsMaxK && (m + 63) / 64 * ((n + 127) / 128) * 8 >= 5 * (int64_t)cus;
 }
 
+// int16 convolutions, conv_digits: five eighths of a tile of 64 x 128 (up to 64 columns 128 x 64) outputs per unit, and 16 sub-steps of
+// 32 values of K for each.  Whole calls, us, operands as they lie / digits: 5 x 59x59, 222 -> 40, 3 x 3 stride 2 55.4 / 21.5, 8 x 76x76,
+// 269 -> 56 163 / 65, 93x93, 326 -> 322, 5 x 5 231 / 127, 2 x 97x97, 192 -> 108 61 / 40, 3 x 91x102, 16 -> 281 half 54 / 36, 3 x 66x77,
+// 90 -> 110 24.1 / 21.4; below the lines 12 x 11x16 -> 8 x 6, 32 -> 476 13.0 / 15.9 (192 tiles of 12 sub-steps), 1 x 51x62, 48 -> 261, 5 x
+// 5 18.4 / 26.5 (150 tiles), 3 x 37x42 -> 18x29, 448 -> 137, 5 x 5 36.5 / 96.8 (50: a lone block waits for its filters).
+inline bool conv_digits_sizes(int64_t m, int64_t n, int64_t ci, int64_t taps, int cus) {
+  const int64_t tiles = n <= 64 ? (m + 127) / 128 : (m + 63) / 64 * ((n + 127) / 128);
+  return taps > 1 && tiles * 8 >= 5 * (int64_t)cus && tiles * ((ci + 31) / 32 * taps) >= 16 * (int64_t)cus;
+}
+
 // int8, conv3x3_i8_packed: the patch-resident kernels (conv3x3_halo_i8.hip) are ahead on the channels they have instances for, the one
 // that walks over tiles (conv3x3_i8_walk.hip) on 32
 inline bool conv3x3_i8_packed_channels(int64_t ci) {

@@ -1153,14 +1153,18 @@ const void *packed_weight(Prepared &p, Takes takes) {
     const int64_t n = p.qw.size(0), k = p.qw.numel() / n;
     size_t bytes = 0;
     const bool digits = p.bw_w == 16;
-    if ((digits ? catchq_packed_digits_size(n, k, &bytes) : catchq_packed_filters_size(n, k, &bytes)) != CATCHQ_OK) return nullptr;
+    const int64_t taps = p.qw.dim() == 4 ? p.qw.size(2) * p.qw.size(3) : 1;
+    if ((digits ? (taps > 1 ? catchq_packed_conv_digits_size(n, taps, k / taps, &bytes) : catchq_packed_digits_size(n, k, &bytes))
+                : catchq_packed_filters_size(n, k, &bytes)) != CATCHQ_OK)
+      return nullptr;
     Tensor packed;
     try {
       packed = device_empty({(int64_t)bytes}, at::kChar, p.qw.device());
     } catch (const c10::OutOfMemoryError &) {
       return nullptr;  // (the other routes need no second copy)
     }
-    check_status(digits ? catchq_pack_digits(p.qw.data_ptr(), n, k, k, packed.data_ptr(), current_stream())
+    check_status(digits ? (taps > 1 ? catchq_pack_conv_digits(p.qw.data_ptr(), n, taps, k / taps, packed.data_ptr(), current_stream())
+                                    : catchq_pack_digits(p.qw.data_ptr(), n, k, k, packed.data_ptr(), current_stream()))
                         : catchq_pack_filters(p.qw.data_ptr(), n, k, packed.data_ptr(), current_stream()),
                  "torch_mlu::quantize");
     p.packed_on = cur.id();
@@ -1331,6 +1335,28 @@ bool conv_small(const Tensor &x, const Prepared &prep, const catchq_conv_desc_t 
   return true;
 }
 
+// The layer at 16 bits through the digits of floating activations, channels-last or contiguous; false: another route serves it.
+bool conv_digits(const Tensor &x, Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e, const Tensor &y) {
+  const int64_t taps = (int64_t)d.kh * d.kw;
+  if (prep.bw_x != 16 || prep.bw_w != 16 || d.groups != 1 ||
+      !catchq::conv_digits_sizes((int64_t)d.n * y.size(2) * y.size(3), d.co, d.ci, taps, catchq::planned_cus(e.sharing)))
+    return false;
+  const bool rows = x.is_contiguous(at::MemoryFormat::ChannelsLast);
+  if (!rows && !x.is_contiguous()) return false;
+  size_t bytes = 0;
+  int st = catchq_float_conv2d_digits_workspace_size(&d, &e, &bytes);
+  if (st == CATCHQ_OK) {
+    const void *packed = packed_weight(prep, [] { return true; });
+    if (!packed) return false;
+    Tensor digits = device_empty({(int64_t)bytes}, at::kChar, x.device());
+    st = catchq_float_conv2d_digits(x.data_ptr(), x.scalar_type() == at::kHalf ? CATCHQ_F16 : CATCHQ_F32, prep.pos_x, (int)x.size(1),
+                                    rows ? 0 : 1, packed, &d, &e, digits.data_ptr(), bytes, current_stream());
+  }
+  if (st == CATCHQ_ERR_UNSUPPORTED) return false;
+  check_status(st, "torch_mlu::conv2d");
+  return true;
+}
+
 // quantized activations [N,H,W,Ci] (or, qx undefined, the floating NHWC activations at x, or those of `input`, whose order and
 // channel count may differ) x prepared weight -> floating output, logical [N,Co,Ho,Wo] over NHWC memory
 Tensor conv_prepared(Tensor qx, const void *x, at::IntArrayRef x_nhwc, Prepared &prep, const Tensor &bias, at::IntArrayRef padding,
@@ -1352,7 +1378,7 @@ Tensor conv_prepared(Tensor qx, const void *x, at::IntArrayRef x_nhwc, Prepared 
   Tensor keep;
   const catchq_epilogue_t e = prepared_epilogue(prep, bias, d.co, y, &keep);
   if (input && !x) {
-    if (conv_small(*input, prep, d, e)) return y;
+    if (conv_small(*input, prep, d, e) || conv_digits(*input, prep, d, e, y)) return y;
     qx = quantize_to_nhwc(*input, prep.bw_x, prep.pos_x, d.ci);
   }
   if (qx.defined()) {

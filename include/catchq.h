@@ -302,6 +302,17 @@ int catchq_float_linear_digits_workspace_size(int64_t m, int64_t n, int64_t k, c
 int catchq_float_linear_digits(const void *x, int x_dtype, int x_position, const void *packed, int64_t m, int64_t n, int64_t k,
                                const catchq_epilogue_t *epilogue, void *workspace, size_t workspace_bytes, catchq_stream_t stream);
 
+/* The same for a convolution of 2 to 25 taps: catchq_pack_conv_digits lays out w [n][taps][ci] int16, the filters that
+ * catchq_conv2d_nhwc reads; x [n,h,w,x_ci] or (x_nchw) [n,x_ci,h,w] of x_ci <= desc->ci channels (zeros in the filters beyond them),
+ * the digits of all channels of all pixels in the caller's workspace.  CATCHQ_ERR_UNSUPPORTED: quantizing and catchq_conv2d_nhwc
+ * serve the call. */
+int catchq_packed_conv_digits_size(int64_t n, int64_t taps, int64_t ci, size_t *bytes);
+int catchq_pack_conv_digits(const void *w, int64_t n, int64_t taps, int64_t ci, void *packed, catchq_stream_t stream);
+int catchq_float_conv2d_digits_workspace_size(const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, size_t *bytes);
+int catchq_float_conv2d_digits(const void *x, int x_dtype, int x_position, int x_ci, int x_nchw, const void *packed,
+                               const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, void *workspace,
+                               size_t workspace_bytes, catchq_stream_t stream);
+
 /* Last convolution of a residual block with the block's projection shortcut evaluated in the same launch.
  * In the reference a block with a projection ends in two torch_mlu::conv2d calls (cnnl_conv2d,
  * operators/cnnl/quantify_conv_forward.cpp:56-147: the 1x1 shortcut and the block's last convolution) and a

@@ -1,0 +1,69 @@
+"""int16 convolutions through the digits of both operands (catchq_float_conv2d_digits).  The weight is laid out at the second call that
+the route takes, so the first call of a layer runs the kernel for operands as they lie and the next ones this one: exact sums, the same
+bits."""
+import ctypes
+import math
+
+import pytest
+import torch
+
+import catch_amd  # noqa: F401
+from catch_amd import _native
+
+pytestmark = pytest.mark.gpu
+
+
+def _served(x, w, k, stride, dil):
+    """whether the route serves the layer"""
+    n, ci, h, wd = x.shape
+    desc = _native.ConvDesc(n, h, wd, (ci + 7) // 8 * 8, w.shape[0], k[0], k[1], dil * (k[0] // 2), dil * (k[1] // 2), stride, stride, dil, dil, 1)
+    e = _native.Epilogue()
+    e.y, e.y_dtype = x.data_ptr(), 1 if x.dtype == torch.float16 else 0
+    bytes_ = ctypes.c_size_t(0)
+    return _native.kernel_lib().catchq_float_conv2d_digits_workspace_size(ctypes.byref(desc), ctypes.byref(e), ctypes.byref(bytes_)) == 0
+
+
+def _calls(x, w, b, k, stride, dil, mode):
+    assert _served(x, w, k, stride, dil)
+    scale_x = 32767.0 / x.float()[torch.isfinite(x)].abs().max().reshape(1)
+    wf = w.float().reshape(w.shape[0], -1).abs()
+    scale = torch.cat([scale_x, torch.zeros_like(scale_x), 32767.0 / wf.amax(1)]) if mode == 4 else torch.cat([scale_x, 32767.0 / wf.max().reshape(1)])
+    qm = torch.tensor([mode], dtype=torch.int32, device="cuda")
+    run = lambda: torch.ops.torch_mlu.conv2d(x, w, b, [dil * (k[0] // 2), dil * (k[1] // 2)], [stride, stride], [dil, dil], 1, scale, qm)
+    first = run()
+    for _ in range(3):
+        again = run()
+        assert again.stride() == first.stride() and torch.equal(first.view(torch.int32 if first.dtype == torch.float32 else torch.int16),
+                                                                again.view(torch.int32 if first.dtype == torch.float32 else torch.int16))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("nhwc", [True, False])
+@pytest.mark.parametrize("n,ci,h,w,co,k,stride,dil", [
+    (37, 32, 40, 41, 64, (3, 3), 1, 1),    # two waves side by side
+    (26, 33, 40, 41, 33, (3, 3), 1, 1),    # one channel of the second block of 32; one column of the second 32
+    (24, 64, 41, 40, 130, (3, 3), 2, 1),   # four waves side by side, two columns in the second run of 128
+    (17, 72, 33, 35, 100, (5, 5), 1, 1),   # 25 taps, a last wave without columns
+    (16, 40, 30, 30, 256, (1, 5), 1, 2),
+    (20, 9, 50, 50, 96, (3, 3), 1, 1),     # nine channels
+    (13, 640, 20, 40, 128, (5, 5), 1, 1),  # 16000 positions of K, close to the most
+])
+def test_same_bits_as_operands_as_they_lie(n, ci, h, w, co, k, stride, dil, nhwc, dtype):
+    gen = torch.Generator(device="cuda").manual_seed(ci)
+    x = torch.randn(n, ci, h, w, generator=gen, device="cuda").to(dtype)
+    x.view(-1)[:3] = torch.tensor([math.inf, -math.inf, math.nan], device="cuda")  # saturate, saturate, 0
+    if nhwc:
+        x = x.contiguous(memory_format=torch.channels_last)
+    wt = (torch.randn(co, ci, *k, generator=gen, device="cuda") / math.sqrt(ci * k[0] * k[1])).to(dtype)
+    b = torch.randn(co, generator=gen, device="cuda").to(dtype)
+    for mode in (2, 4):
+        _calls(x, wt.clone(), b, k, stride, dil, mode)
+
+
+@pytest.mark.parametrize("sx,sw", [(1, 1), (-1, -1), (-1, 1)])
+def test_largest_sums(sx, sw):
+    """every activation and weight at its limit: the sums of the digits and their combination are as large as they get"""
+    x = torch.full((13, 640, 20, 40), float(sx), device="cuda")
+    w = torch.full((128, 640, 5, 5), float(sw), device="cuda")
+    b = torch.zeros(128, device="cuda")
+    _calls(x, w, b, (5, 5), 1, 1, 2)
