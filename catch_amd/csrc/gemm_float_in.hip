@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void gemm_float_kernel(const void *__restrict_
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads();  // the slots are dead: staging area
   int *stage = reinterpret_cast<int *>(lds_dyn) + wave * 32 * EPI_STRIDE;
-  if constexpr (EPI == EPI_SCALAR) igemm_epilogue_columns<1, TN>(acc, stage, m0 + wave_m * 32, n0 + wave_n * WN, lane, p, e);
+  if constexpr (EPI == EPI_SCALAR) igemm_epilogue_any<1, TN>(acc, stage, m0 + wave_m * 32, n0 + wave_n * WN, lane, p, e);
   else igemm_epilogue<1, TN, EPI>(acc, stage, m0 + wave_m * 32, n0 + wave_n * WN, lane, p, e);
 }
 
@@ -135,6 +135,7 @@ static int launch_gemm_float(const void *a, const void *b, IgemmParams p, const 
   const int64_t nb = (p.M + 63) / 64 * p.tiles_n;
   if (nb > 0x7fffffff) return -1;
   p.nblocks = (int)nb;
+  p.ragged = pick_epilogue(p.N, e) == EPI_SCALAR ? ragged_epilogue(p.N, e, true) : EPI_SCALAR;
 #define CATCHQ_FLOAT_CASE(E)                                                                                          \
   case E:                                                                                                             \
     gemm_float_kernel<IN, BN, E><<<p.nblocks, 256, LDS_BYTES, s>>>(a, (const int8_t *)b, p, e, x_neg_pos, (unsigned)a_bytes, \

@@ -29,6 +29,7 @@ struct IgemmParams {
   // groups > 1: per-group offsets -- bytes into the activation tensor (a pixel's channel slice), bytes into the
   // weights (the group's filters) and output channels (columns of the outputs and entries of the per-channel vectors)
   int groups, a_group_bytes, n_group;
+  int ragged;  // EPI_SCALAR: the epilogue that serves the rows all the same (ragged_epilogue), or EPI_SCALAR
   int64_t b_group_bytes;
 };
 
@@ -182,15 +183,16 @@ inline int pick_epilogue(int N, const EpiDev &e) {
 }
 
 // For rows whose length or alignment the vectorised epilogues do not take, a floating output and nothing else: the epilogue
-// (EPI_Y32 or EPI_Y16) that serves them with stores that need no alignment (EpiAtRagged); EPI_SCALAR: neither does.
-inline int ragged_epilogue(int N, const EpiDev &e) {
+// (EPI_Y32, EPI_Y16 or, where the caller has it, EPI_Y16_STEPS) that serves them with stores that need no alignment (EpiAtRagged);
+// EPI_SCALAR: none does.
+inline int ragged_epilogue(int N, const EpiDev &e, bool steps = false) {
   if (N >= (1 << 24)) return EPI_SCALAR;
   EpiDev aligned = e;
   auto stand_in = [](const auto *q) { return reinterpret_cast<decltype(q)>(q ? (uintptr_t)16 : 0); };  // (presence only)
   aligned.chan_div = stand_in(e.chan_div); aligned.chan_rcp = stand_in(e.chan_rcp); aligned.bias = stand_in(e.bias);
   aligned.y = const_cast<void *>((const void *)stand_in((const char *)e.y));
   const int epi = pick_epilogue((N + 3) / 4 * 4, aligned);
-  return epi == EPI_Y32 || epi == EPI_Y16 ? epi : EPI_SCALAR;
+  return epi == EPI_Y32 || epi == EPI_Y16 || (steps && epi == EPI_Y16_STEPS) ? epi : EPI_SCALAR;
 }
 
 // per-channel constants of one lane's four consecutive channels
@@ -253,11 +255,12 @@ __device__ __forceinline__ EpiLane epi_lane_finish(v4f div, v4f rcp, v4f bias, c
 template <class S>
 __device__ __forceinline__ EpiLane epi_lane_setup_ragged(int n, int N, const EpiDev &e) {
   v4f div, rcp, bias;
+  const float *rcps = S::kSteps ? e.half_rcp : e.chan_rcp;
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
     const int c = min(n + t, N - 1);
     div[t] = e.chan_div ? e.chan_div[c] : 1.0f;
-    rcp[t] = e.chan_rcp ? e.chan_rcp[c] : 1.0f;
+    rcp[t] = rcps ? rcps[c] : 1.0f;
     bias[t] = e.bias ? bias_value(e, c) : -0.0f;
   }
   return epi_lane_finish<S>(div, rcp, bias, e);
@@ -673,6 +676,55 @@ __device__ __forceinline__ void igemm_epilogue_columns(v16i (&acc)[TM][TN], int 
         epi_store(epi_value((float)a, idx, k, e), idx, e);
       }
     }
+  }
+}
+
+// Epilogue of one wave for floating rows of any length and alignment (ragged_epilogue) through the wave's staging area, four columns a
+// lane: the vector epilogue's arithmetic on constants read one by one, stores that take any element's alignment.
+template <int TM, int TN, int EPI>
+__device__ __forceinline__ void igemm_epilogue_ragged(v16i (&acc)[TM][TN], int *stage, int64_t m_w, int n_w, int lane,
+                                                      const IgemmParams &p, const EpiDev &e) {
+  typedef typename EpiOf<EPI>::type S;
+  constexpr int WN = TN * 32, EPI_STRIDE = WN + 8, CPR = WN / 4, RPI = 64 / CPR, NIT = 32 / RPI, BATCH = NIT < 4 ? NIT : 4;
+  const int frow = lane & 31, fhalf = lane >> 5, cg = lane % CPR, rsub = lane / CPR;
+  const int n = n_w + cg * 4;
+  const bool n_ok = n < p.N;
+  const EpiLane L = epi_lane_setup_ragged<S>(n_ok ? n : 0, p.N, e);
+  const v4f none = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    // wave-private staging: stores then loads of the same wave, ordered by the LDS counter
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        stage[(8 * (r >> 2) + 4 * fhalf + (r & 3)) * EPI_STRIDE + j * 32 + frow] = acc[i][j][r];
+    const int64_t left = p.M - (m_w + i * 32);
+    const int rows = !n_ok || left < 0 ? 0 : (left > 32 ? 32 : (int)left);
+#pragma unroll 1
+    for (int it = 0; it < NIT; it += BATCH) {
+      v4i av[BATCH];
+#pragma unroll
+      for (int b = 0; b < BATCH; ++b) av[b] = *reinterpret_cast<const v4i *>(stage + ((it + b) * RPI + rsub) * EPI_STRIDE + cg * 4);
+#pragma unroll
+      for (int b = 0; b < BATCH; ++b) {
+        const int row = (it + b) * RPI + rsub;
+        if (row < rows) epi_vec4<S>(av[b], none, L, EpiAtRagged{(m_w + i * 32 + row) * out_ld(p) + n, p.N - n}, e);
+      }
+    }
+  }
+}
+
+// EPI_SCALAR of the tiled kernels: any length and alignment, the rule's choice first.  (Straight from the accumulators, one element at
+// a time, 8127 x 1742 -> 1747 took 110 us where 1748 columns took 34.)
+template <int TM, int TN>
+__device__ __forceinline__ void igemm_epilogue_any(v16i (&acc)[TM][TN], int *stage, int64_t m_w, int n_w, int lane, const IgemmParams &p,
+                                                   const EpiDev &e) {
+  switch (p.ragged) {
+    case EPI_Y32: igemm_epilogue_ragged<TM, TN, EPI_Y32>(acc, stage, m_w, n_w, lane, p, e); break;
+    case EPI_Y16: igemm_epilogue_ragged<TM, TN, EPI_Y16>(acc, stage, m_w, n_w, lane, p, e); break;
+    case EPI_Y16_STEPS: igemm_epilogue_ragged<TM, TN, EPI_Y16_STEPS>(acc, stage, m_w, n_w, lane, p, e); break;
+    default: igemm_epilogue_columns<TM, TN>(acc, stage, m_w, n_w, lane, p, e); break;
   }
 }
 
