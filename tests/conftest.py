@@ -1,3 +1,4 @@
+import gc
 import os
 import sys
 
@@ -10,6 +11,13 @@ if ROOT not in sys.path:
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a real MI355X (run with -m gpu)")
+
+
+@pytest.fixture(scope="module", autouse=True)
+def no_garbage_of_earlier_files():
+    """networks of one file that wait for the collector (modules in cycles, up to 200 MB on the device) are gone before the next file
+    begins: tests that compare what the device holds before and after a call would see them go in between"""
+    gc.collect()
 
 
 @pytest.fixture(scope="session")
