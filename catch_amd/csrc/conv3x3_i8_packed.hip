@@ -103,7 +103,8 @@ __global__ __launch_bounds__(512, 2) void conv3x3_i8_packed_kernel(const int8_t 
   }
   __syncthreads();
   int *const stage = reinterpret_cast<int *>(lds_dyn) + wave * 32 * (32 + 8);
-  igemm_epilogue<TM, 1, EPI>(acc, stage, m0, n0, lane, p.g, e);
+  if constexpr (EPI == EPI_SCALAR) igemm_epilogue_any<TM, 1>(acc, stage, m0, n0, lane, p.g, e);
+  else igemm_epilogue<TM, 1, EPI>(acc, stage, m0, n0, lane, p.g, e);
 }
 
 template <int TM>
@@ -124,6 +125,7 @@ static int launch_packed_i8(const void *x, const void *w, const PackedI8Params &
     CATCHQ_PACKED(EPI_Y16)
     CATCHQ_PACKED(EPI_Y16_STEPS)
     CATCHQ_PACKED(EPI_VECTOR)
+    CATCHQ_PACKED(EPI_SCALAR)
     default: return -1;
   }
 #undef CATCHQ_PACKED
@@ -133,9 +135,10 @@ static int launch_packed_i8(const void *x, const void *w, const PackedI8Params &
 static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e) {
   const int64_t M = N * H * W, groups = ((int64_t)Co + 31) / 32;
   // (the patch-resident kernels: 32 x 28 x 28, 128 channels, 16.4 / 16.8 us with this one, 32 x 14 x 14, 256 14.0 / 15.0)
-  if (!conv3x3_i8_packed_channels(Ci) || W > 512 || H >= (1 << 20) || M * Ci >= (1ll << 31) || groups * Ci * 288 >= (1ll << 31)) return 0;
+  if (!conv3x3_i8_packed_channels(Ci, Co) || W > 512 || H >= (1 << 20) || M * Ci >= (1ll << 31) || groups * Ci * 288 >= (1ll << 31)) return 0;
   const int epi = pick_epilogue(Co, e);
-  if (epi != EPI_Y32 && epi != EPI_Y16 && epi != EPI_Y16_STEPS && epi != EPI_VECTOR) return 0;
+  if (epi != EPI_Y32 && epi != EPI_Y16 && epi != EPI_Y16_STEPS && epi != EPI_VECTOR && !(epi == EPI_SCALAR && ragged_epilogue(Co, e, true)))
+    return 0;
   // Half a block of 32 pixels for a unit (us, tiled / this: 1 x 57 x 75, 96 -> 160, 134 blocks, 9.7 / 9.0, 10 x 14 x 14, 160 -> 512, 124,
   // 11.2 / 11.3, 3 x 30 x 33, 448 -> 224, 93, 14.9 / 16.0, 1 x 28 x 28, 192, 25, 7.9 / 9.8); blocks of 64, which read half the
   // filters, from as many of those on (8 x 25 x 25, 160 -> 320, 158, 13.3 / 12.6 with 64; 8 x 28 x 28, 192, 98, 11.5 / 13.4).
@@ -176,6 +179,7 @@ int conv3x3_i8_packed(const void *x, const void *packed, int64_t N, int H, int W
   const int groups = (Co + 31) / 32;
   PackedI8Params p = {};
   p.g.M = N * H * W;
+  p.g.ragged = pick_epilogue(Co, e) == EPI_SCALAR ? ragged_epilogue(Co, e, true) : EPI_SCALAR;
   p.g.N = Co; p.g.K = 9 * Ci; p.g.H = H; p.g.W = W; p.g.Ci = Ci;
   p.x_bytes = (unsigned)(p.g.M * Ci);
   p.w_bytes = (unsigned)((int64_t)groups * Ci * 288);

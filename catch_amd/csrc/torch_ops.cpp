@@ -1316,7 +1316,7 @@ catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64
 // question: that call answers it.
 const void *conv3x3_packed(Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e) {
   if (prep.bw_x != 8 || prep.bw_w != 8 || d.kh != 3 || d.kw != 3 || d.groups != 1 || d.pad_h != 1 || d.pad_w != 1 || d.stride_h != 1 ||
-      d.stride_w != 1 || d.dil_h != 1 || d.dil_w != 1 || !catchq::conv3x3_i8_packed_channels(d.ci))
+      d.stride_w != 1 || d.dil_h != 1 || d.dil_w != 1 || !catchq::conv3x3_i8_packed_channels(d.ci, d.co))
     return nullptr;
   return packed_weight(prep, [&] { return catchq_conv3x3_i8_packed_takes(d.n, d.h, d.w, d.ci, d.co, &e) == CATCHQ_OK; });
 }

@@ -1,10 +1,13 @@
 """Linears and convolutions whose rows of outputs have a length that no vector divides: the tiled kernels' stores that need no alignment
 (igemm_epilogue_ragged) against the oracle, bit for bit, in every output type."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
 
 import catch_amd  # noqa: F401
+from catch_amd import _native
 from oracle import ops as oops
 
 pytestmark = pytest.mark.gpu
@@ -55,3 +58,27 @@ def test_conv2d(n, ci, h, w, co, k, stride, mode, dtype):
     ref = oops.conv2d(x.numpy(), wt.numpy(), b.numpy(), (k // 2, k // 2), (stride, stride), (1, 1), 1, scale.numpy(), qm.numpy())["y"]
     for xi in (x.cuda(), x.cuda().contiguous(memory_format=torch.channels_last)):
         _same(ref, torch.ops.torch_mlu.conv2d(xi, *args))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("mode", [1, 3])
+@pytest.mark.parametrize("n,ci,h,w,co", [
+    (6, 64, 30, 31, 98), (3, 123, 56, 57, 90), (8, 256, 28, 28, 129), (10, 160, 33, 30, 97), (2, 192, 75, 76, 261), (9, 512, 14, 14, 255),
+])
+def test_conv3x3_on_packed_filters(n, ci, h, w, co, mode, dtype):
+    """filters are packed at the second call of a layer: the calls behind it against the first, and the first against the oracle"""
+    g = torch.Generator().manual_seed(ci + co)
+    x = torch.randn(n, ci, h, w, generator=g).to(dtype)
+    wt, b = (torch.randn(co, ci, 3, 3, generator=g) / (ci * 9) ** 0.5).to(dtype), torch.randn(co, generator=g).to(dtype)
+    scale, qm = _qparams(x, wt, mode)
+    e = _native.Epilogue()
+    e.y = e.chan_div = e.chan_rcp = e.bias = 16  # (presence only: nothing is launched)
+    took = _native.kernel_lib().catchq_conv3x3_i8_packed_takes(n, h, w, (ci + 15) // 16 * 16, co, ctypes.byref(e))
+    assert took == 0 or n * h * w < 2048
+    args = (wt.cuda(), b.cuda(), [1, 1], [1, 1], [1, 1], 1, scale.cuda(), qm.cuda())
+    xd = x.cuda().contiguous(memory_format=torch.channels_last)
+    first = torch.ops.torch_mlu.conv2d(xd, *args)
+    ref = oops.conv2d(x[-1:].numpy(), wt.numpy(), b.numpy(), (1, 1), (1, 1), (1, 1), 1, scale.numpy(), qm.numpy())["y"]
+    _same(ref, first[-1:])
+    for _ in range(3):
+        assert torch.equal(torch.ops.torch_mlu.conv2d(xd, *args), first)
