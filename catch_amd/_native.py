@@ -102,6 +102,7 @@ SIGNATURES = {
     "catchq_pack_digits": (_I, [_P, _I64, _I64, _I64, _P, _P]),
     "catchq_packed_conv_digits_size": (_I, [_I64, _I64, _I64, ctypes.POINTER(_SZ)]),
     "catchq_pack_conv_digits": (_I, [_P, _I64, _I64, _I64, _P, _P]),
+    "catchq_float_depthwise": (_I, [_P, _I, _I, _I, _P, _I, ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue), _P]),
     "catchq_float_conv2d_digits_workspace_size": (_I, [ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue), ctypes.POINTER(_SZ)]),
     "catchq_float_conv2d_digits": (_I, [_P, _I, _I, _I, _I, _P, ctypes.POINTER(ConvDesc), ctypes.POINTER(Epilogue), _P, _SZ, _P]),
     "catchq_float_linear_digits_workspace_size": (_I, [_I64, _I64, _I64, ctypes.POINTER(Epilogue), ctypes.POINTER(_SZ)]),

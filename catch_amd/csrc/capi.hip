@@ -7,6 +7,8 @@ namespace catchq {
 
 int gemm_nt_direct(const void *a, int a_bits, const void *b, int b_bits, int64_t M, int64_t N, int64_t K,
                    const EpiDev &e, hipStream_t s);
+int dw_float(const void *x, bool half, int position, bool nchw, const void *w, int bits, int N, int H, int W, int C, int ph, int pw,
+             int stride, int Ho, int Wo, const EpiDev &e, hipStream_t s);
 int conv2d_direct(const void *x, int x_bits, const void *w, int w_bits, const ConvDev &d, const EpiDev &e,
                   hipStream_t s);
 int gemm_nt_mfma_i8(const void *a, const void *b, int64_t M, int64_t N, int64_t K, const EpiDev &e,
@@ -583,6 +585,26 @@ CATCHQ_API int catchq_float_conv2d_digits(const void *x, int x_dtype, int x_posi
   return conv_digits(x, x_dtype == CATCHQ_F16, x_position, x_ci, x_nchw != 0, packed, d.n, d.h, d.w, d.ci, d.co, d.kh, d.kw, d.pad_h,
                      d.pad_w, d.stride_h, d.stride_w, d.dil_h, d.dil_w, ho, wo, workspace,
                      make_epi(epilogue, (int64_t)d.n * ho * wo * d.co), as_stream(stream));
+}
+
+CATCHQ_API int catchq_float_depthwise(const void *x, int x_dtype, int x_position, int x_nchw, const void *w, int w_bits,
+                                      const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  if (x_dtype != CATCHQ_F32 && x_dtype != CATCHQ_F16) return CATCHQ_ERR_DTYPE;
+  if (w_bits != 8 && w_bits != 16) return CATCHQ_ERR_BITWIDTH;
+  int ho, wo;
+  int st = check_conv(desc, &ho, &wo);
+  if (st != CATCHQ_OK) return st;
+  st = check_epi(epilogue, true);
+  if (st != CATCHQ_OK) return st;
+  const catchq_conv_desc_t &d = *desc;
+  if (x_position < -126 || x_position > 126) return CATCHQ_ERR_ARG;
+  if (d.groups == 1 || d.groups != d.ci || d.co != d.ci || d.kh != 3 || d.kw != 3 || d.dil_h != 1 || d.dil_w != 1 ||
+      d.stride_h != d.stride_w || d.stride_h > 2)
+    return CATCHQ_ERR_UNSUPPORTED;
+  if (d.n == 0) return CATCHQ_OK;
+  if (!x || !w) return CATCHQ_ERR_ARG;
+  return dw_float(x, x_dtype == CATCHQ_F16, x_position, x_nchw != 0, w, w_bits, d.n, d.h, d.w, d.ci, d.pad_h, d.pad_w, d.stride_h, ho, wo,
+                  make_epi(epilogue, (int64_t)d.n * ho * wo * d.co), as_stream(stream));
 }
 
 CATCHQ_API int catchq_float_linear_digits_workspace_size(int64_t m, int64_t n, int64_t k, const catchq_epilogue_t *epilogue,

@@ -1335,6 +1335,18 @@ bool conv_small(const Tensor &x, const Prepared &prep, const catchq_conv_desc_t 
   return true;
 }
 
+// A 3 x 3 depthwise layer on floating activations in one launch, channels-last or contiguous; false: another route serves it.
+bool conv_depthwise(const Tensor &x, const Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e) {
+  if (prep.bw_x != prep.bw_w || d.groups == 1 || x.size(1) != d.ci) return false;
+  const bool rows = x.is_contiguous(at::MemoryFormat::ChannelsLast);
+  if (!rows && !x.is_contiguous()) return false;
+  const int st = catchq_float_depthwise(x.data_ptr(), x.scalar_type() == at::kHalf ? CATCHQ_F16 : CATCHQ_F32, prep.pos_x, rows ? 0 : 1,
+                                        prep.qw.data_ptr(), prep.bw_w, &d, &e, current_stream());
+  if (st == CATCHQ_ERR_UNSUPPORTED) return false;
+  check_status(st, "torch_mlu::conv2d");
+  return true;
+}
+
 // The layer at 16 bits through the digits of floating activations, channels-last or contiguous; false: another route serves it.
 bool conv_digits(const Tensor &x, Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e, const Tensor &y) {
   const int64_t taps = (int64_t)d.kh * d.kw;
@@ -1377,6 +1389,7 @@ Tensor conv_prepared(Tensor qx, const void *x, at::IntArrayRef x_nhwc, Prepared 
   if (d.n == 0 || d.co == 0) return y;  // nothing to compute: the empty output is the result
   Tensor keep;
   const catchq_epilogue_t e = prepared_epilogue(prep, bias, d.co, y, &keep);
+  if (input && conv_depthwise(*input, prep, d, e)) return y;
   if (input && !x) {
     if (conv_small(*input, prep, d, e) || conv_digits(*input, prep, d, e, y)) return y;
     qx = quantize_to_nhwc(*input, prep.bw_x, prep.pos_x, d.ci);
@@ -1465,7 +1478,8 @@ Tensor conv2d_op(const Tensor &input, const Tensor &weight, const Tensor &bias, 
   if (input.is_contiguous(at::MemoryFormat::ChannelsLast)) {
     const bool one_by_one = kw == 1 && weight.size(2) == 1;
     if (prep->bw_x == 8 && prep->bw_w == 8 && ci % 16 == 0)
-      return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), h, w_in, ci}, *prep, bias, padding, stride, dilation, groups, half);
+      return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), h, w_in, ci}, *prep, bias, padding, stride, dilation, groups, half,
+                           &input);
     if (prep->bw_x == 16 && prep->bw_w == 16 && ci % 8 == 0 && dense && one_by_one)
       return conv_prepared(Tensor(), input.data_ptr(), {input.size(0), h, w_in, ci}, *prep, bias, padding, stride, dilation, groups, half,
                            &input);

@@ -264,6 +264,12 @@ int catchq_float_conv2d_nhwc(const void *x, int x_dtype, int x_position, const v
 int catchq_float_conv2d_small(const void *x, int x_dtype, int x_position, int x_ci, int x_nchw, const void *w, int w_bits,
                               const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 
+/* A 3x3 depthwise layer (groups == ci == co, dilation 1, one stride of 1 or 2 in both directions) on floating activations in one launch
+ * or not at all (CATCHQ_ERR_UNSUPPORTED: quantizing and catchq_conv2d_nhwc serve the call): activations [n,h,w,ci] or (x_nchw)
+ * [n,ci,h,w], quantized at w_bits (8 or 16), filters [ci][3][3], a floating output of the activations' type and nothing else. */
+int catchq_float_depthwise(const void *x, int x_dtype, int x_position, int x_nchw, const void *w, int w_bits,
+                           const catchq_conv_desc_t *desc, const catchq_epilogue_t *epilogue, catchq_stream_t stream);
+
 /* The same for a linear (a pointwise convolution of unit stride: m pixels) whose int8 filters were laid out once in the order
  * of the matrix instruction: catchq_pack_filters writes catchq_packed_filters_size bytes from w [n,k], k a multiple of 16.
  * x [m,k] fp32/fp16, y [m,n].  CATCHQ_ERR_UNSUPPORTED: catchq_float_conv2d_nhwc on the filters as they are serves the call
