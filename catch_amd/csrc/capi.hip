@@ -46,8 +46,9 @@ int64_t gemm_digits_bytes(int64_t M, int64_t N, int64_t K, const EpiDev &e);
 int gemm_digits(const void *x, bool half, int position, const void *packed, int64_t M, int64_t N, int64_t K, void *digits,
                 const EpiDev &e, hipStream_t s);
 int pack_filters(const void *w, void *packed, int64_t N, int64_t K, hipStream_t s);
-bool conv3x3_i8_packed_takes(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e);
-int conv3x3_i8_packed(const void *x, const void *packed, int64_t N, int H, int W, int Ci, int Co, const EpiDev &e, hipStream_t s);
+bool conv3x3_i8_packed_takes(int64_t N, int H, int W, int Ci, int Co, bool any_rows, const EpiDev &e);
+int conv3x3_i8_packed(const void *x, const void *packed, int64_t N, int H, int W, int Ci, int Co, bool any_rows, const EpiDev &e,
+                      hipStream_t s);
 int64_t packed3x3_bytes(int64_t Co, int64_t Ci);
 int pack3x3(const void *w, void *packed, int64_t Co, int64_t Ci, hipStream_t s);
 int conv3x3_a16_packed(const void *x, const void *packed, int N, int H, int W, int Ci, int Co, const EpiDev &e, hipStream_t s);
@@ -509,20 +510,39 @@ static int check_conv3x3_i8_packed(int n, int h, int w, int ci, int co, const ca
   return catchq_packed_filters_size(co, 9 * (int64_t)ci, &bytes);
 }
 
-CATCHQ_API int catchq_conv3x3_i8_packed_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {
+static int conv3x3_i8_packed_answer(int n, int h, int w, int ci, int co, bool any_rows, const catchq_epilogue_t *epilogue) {
   const int st = check_conv3x3_i8_packed(n, h, w, ci, co, epilogue);
   if (st != CATCHQ_OK) return st;
-  return n == 0 || conv3x3_i8_packed_takes(n, h, w, ci, co, make_epi(epilogue, (int64_t)n * h * w * co)) ? CATCHQ_OK : CATCHQ_ERR_UNSUPPORTED;
+  return n == 0 || conv3x3_i8_packed_takes(n, h, w, ci, co, any_rows, make_epi(epilogue, (int64_t)n * h * w * co)) ? CATCHQ_OK
+                                                                                                                  : CATCHQ_ERR_UNSUPPORTED;
 }
 
-CATCHQ_API int catchq_conv3x3_i8_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
-                                        const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+static int conv3x3_i8_packed_run(const void *x, const void *packed, int n, int h, int w, int ci, int co, bool any_rows,
+                                 const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
   const int st = check_conv3x3_i8_packed(n, h, w, ci, co, epilogue);
   if (st != CATCHQ_OK || n == 0) return st;
   if (!x || !packed) return CATCHQ_ERR_ARG;
   if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;
-  const int done = conv3x3_i8_packed(x, packed, n, h, w, ci, co, make_epi(epilogue, (int64_t)n * h * w * co), as_stream(stream));
+  const int done = conv3x3_i8_packed(x, packed, n, h, w, ci, co, any_rows, make_epi(epilogue, (int64_t)n * h * w * co), as_stream(stream));
   return done < 0 ? CATCHQ_ERR_UNSUPPORTED : done;
+}
+
+CATCHQ_API int catchq_conv3x3_i8_packed_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {
+  return conv3x3_i8_packed_answer(n, h, w, ci, co, false, epilogue);
+}
+
+CATCHQ_API int catchq_conv3x3_i8_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                                        const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  return conv3x3_i8_packed_run(x, packed, n, h, w, ci, co, false, epilogue, stream);
+}
+
+CATCHQ_API int catchq_conv3x3_i8_packed_any_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {
+  return conv3x3_i8_packed_answer(n, h, w, ci, co, true, epilogue);
+}
+
+CATCHQ_API int catchq_conv3x3_i8_packed_any(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                                            const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  return conv3x3_i8_packed_run(x, packed, n, h, w, ci, co, true, epilogue, stream);
 }
 
 CATCHQ_API int catchq_packed_digits_size(int64_t n, int64_t k, size_t *bytes) {

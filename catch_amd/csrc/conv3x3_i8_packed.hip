@@ -132,12 +132,13 @@ static int launch_packed_i8(const void *x, const void *w, const PackedI8Params &
 }
 
 // The rows of 32 pixels a wave takes, 0: not this kernel's shape
-static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e) {
+static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, bool any_rows, const EpiDev &e) {
+  if (Co % 4 != 0 && !any_rows) return 0;
   const int64_t M = N * H * W, groups = ((int64_t)Co + 31) / 32;
   // (the patch-resident kernels: 32 x 28 x 28, 128 channels, 16.4 / 16.8 us with this one, 32 x 14 x 14, 256 14.0 / 15.0)
   if (!conv3x3_i8_packed_channels(Ci, Co) || W > 512 || H >= (1 << 20) || M * Ci >= (1ll << 31) || groups * Ci * 288 >= (1ll << 31)) return 0;
   const int epi = pick_epilogue(Co, e);
-  if (epi != EPI_Y32 && epi != EPI_Y16 && epi != EPI_Y16_STEPS && epi != EPI_VECTOR && !(epi == EPI_SCALAR && ragged_epilogue(Co, e, true)))
+  if (epi != EPI_Y32 && epi != EPI_Y16 && epi != EPI_Y16_STEPS && epi != EPI_VECTOR && !(any_rows && epi == EPI_SCALAR && ragged_epilogue(Co, e, true)))
     return 0;
   // Half a block of 32 pixels for a unit (us, tiled / this: 1 x 57 x 75, 96 -> 160, 134 blocks, 9.7 / 9.0, 10 x 14 x 14, 160 -> 512, 124,
   // 11.2 / 11.3, 3 x 30 x 33, 448 -> 224, 93, 14.9 / 16.0, 1 x 28 x 28, 192, 25, 7.9 / 9.8); blocks of 64, which read half the
@@ -170,11 +171,15 @@ static int packed_i8_plan(int64_t N, int H, int W, int Ci, int Co, const EpiDev 
   return fits(1) && (groups <= 10 || blocks(1) * 4 <= 13 * (int64_t)e.cus) ? 1 : 0;
 }
 
-bool conv3x3_i8_packed_takes(int64_t N, int H, int W, int Ci, int Co, const EpiDev &e) { return packed_i8_plan(N, H, W, Ci, Co, e) != 0; }
+bool conv3x3_i8_packed_takes(int64_t N, int H, int W, int Ci, int Co, bool any_rows, const EpiDev &e) {
+  return packed_i8_plan(N, H, W, Ci, Co, any_rows, e) != 0;
+}
 
-// x [N, H, W, Ci] int8, packed: pack_filters of w [Co, 9 Ci]; -1: not this kernel's shape
-int conv3x3_i8_packed(const void *x, const void *packed, int64_t N, int H, int W, int Ci, int Co, const EpiDev &e, hipStream_t s) {
-  const int tm = packed_i8_plan(N, H, W, Ci, Co, e);
+// x [N, H, W, Ci] int8, packed: pack_filters of w [Co, 9 Ci]; any_rows: also rows of outputs of any length and alignment; -1: not this
+// kernel's shape
+int conv3x3_i8_packed(const void *x, const void *packed, int64_t N, int H, int W, int Ci, int Co, bool any_rows, const EpiDev &e,
+                      hipStream_t s) {
+  const int tm = packed_i8_plan(N, H, W, Ci, Co, any_rows, e);
   if (!tm) return -1;
   const int groups = (Co + 31) / 32;
   PackedI8Params p = {};

@@ -34,10 +34,9 @@ inline bool conv_digits_sizes(int64_t m, int64_t n, int64_t ci, int64_t taps, in
 }
 
 // int8, conv3x3_i8_packed: the patch-resident kernels (conv3x3_halo_i8.hip) are ahead on the channels they have instances for, the one
-// that walks over tiles (conv3x3_i8_walk.hip) on 32; neither takes rows of outputs that are no multiple of four, which
-// are stored unaligned here, from more than one group of 32 filters on
+// that walks over tiles (conv3x3_i8_walk.hip) on 32; neither takes rows of outputs that are no multiple of four
 inline bool conv3x3_i8_packed_channels(int64_t ci, int64_t co) {
-  return ci >= 64 && ci <= 1024 && ci % 32 == 0 && (co % 4 != 0 ? co > 32 : ci >= 96 && ci != 128 && ci != 256 && ci != 512);
+  return ci >= 64 && ci <= 1024 && ci % 32 == 0 && (co % 4 != 0 || (ci >= 96 && ci != 128 && ci != 256 && ci != 512));
 }
 
 // int16 x int8, conv3x3_a16_packed: what its rule asks of the filters alone.  Blocks have 256 columns; those that do not exist cost as

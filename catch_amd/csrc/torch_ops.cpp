@@ -1135,7 +1135,7 @@ struct RelaxedCapture {
   ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-// The entry's weight as catchq_float_linear_packed and catchq_conv3x3_i8_packed (8 bits) and catchq_float_linear_digits (16) read
+// The entry's weight as catchq_float_linear_packed and catchq_conv3x3_i8_packed_any (8 bits) and catchq_float_linear_digits (16) read
 // it; null: the call goes without.  The weight is laid out at the second call that the route takes.  A caller that rewrites its
 // weight between calls, or uses it once, does not pay for that (6 us of kernel, a launch and an allocation: first pass of 1 x 768 ->
 // 3072 on a new weight 226 us with it, 218 without), and a weight whose calls do not take the route is not held twice.
@@ -1312,13 +1312,13 @@ catchq_epilogue_t prepared_epilogue(const Prepared &p, const Tensor &bias, int64
   return e;
 }
 
-// The filters of a 3 x 3 layer for catchq_conv3x3_i8_packed; null: another route serves it.  Packed ones are handed out without a
+// The filters of a 3 x 3 layer for catchq_conv3x3_i8_packed_any; null: another route serves it.  Packed ones are handed out without a
 // question: that call answers it.
 const void *conv3x3_packed(Prepared &prep, const catchq_conv_desc_t &d, const catchq_epilogue_t &e) {
   if (prep.bw_x != 8 || prep.bw_w != 8 || d.kh != 3 || d.kw != 3 || d.groups != 1 || d.pad_h != 1 || d.pad_w != 1 || d.stride_h != 1 ||
       d.stride_w != 1 || d.dil_h != 1 || d.dil_w != 1 || !catchq::conv3x3_i8_packed_channels(d.ci, d.co))
     return nullptr;
-  return packed_weight(prep, [&] { return catchq_conv3x3_i8_packed_takes(d.n, d.h, d.w, d.ci, d.co, &e) == CATCHQ_OK; });
+  return packed_weight(prep, [&] { return catchq_conv3x3_i8_packed_any_takes(d.n, d.h, d.w, d.ci, d.co, &e) == CATCHQ_OK; });
 }
 
 // The layer on floating activations in one launch, channels-last or contiguous, the channels that only the filters have left out;
@@ -1396,7 +1396,7 @@ Tensor conv_prepared(Tensor qx, const void *x, at::IntArrayRef x_nhwc, Prepared 
   }
   if (qx.defined()) {
     if (const void *packed = conv3x3_packed(prep, d, e)) {
-      const int st = catchq_conv3x3_i8_packed(qx.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
+      const int st = catchq_conv3x3_i8_packed_any(qx.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
       if (st != CATCHQ_ERR_UNSUPPORTED) {
         check_status(st, "torch_mlu::conv2d");
         return y;
@@ -1428,7 +1428,7 @@ Tensor conv_prepared(Tensor qx, const void *x, at::IntArrayRef x_nhwc, Prepared 
     const int64_t elems = (int64_t)d.n * d.h * d.w * d.ci;
     Tensor qn = device_empty({elems}, at::kChar, qw.device());
     check_status(catchq_quantize(x, dt, qn.data_ptr(), 8, elems, prep.pos_x, 1.0f, current_stream()), "torch_mlu::quantize");
-    const int st = catchq_conv3x3_i8_packed(qn.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
+    const int st = catchq_conv3x3_i8_packed_any(qn.data_ptr(), packed, d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
     if (st == CATCHQ_ERR_UNSUPPORTED)
       check_status(catchq_conv2d_nhwc(qn.data_ptr(), 8, qw.data_ptr(), 8, &d, &e, current_stream()), "torch_mlu::conv2d");
     else

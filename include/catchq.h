@@ -296,6 +296,10 @@ int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w
 int catchq_conv3x3_i8_packed_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue);
 int catchq_conv3x3_i8_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
                              const catchq_epilogue_t *epilogue, catchq_stream_t stream);
+/* ... and, for a floating output and nothing else, co that is no multiple of four and tensors of any alignment besides x and packed. */
+int catchq_conv3x3_i8_packed_any_takes(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue);
+int catchq_conv3x3_i8_packed_any(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                                 const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 
 /* A linear on floating activations with int16 weights, both split into the bytes that the matrix cores multiply:
  *   cnnl_quantify_offline_internal (quantify.cpp:69-101) followed by linear.cpp:92-110, 16 bits on either side

@@ -73,7 +73,7 @@ def test_conv3x3_on_packed_filters(n, ci, h, w, co, mode, dtype):
     scale, qm = _qparams(x, wt, mode)
     e = _native.Epilogue()
     e.y = e.chan_div = e.chan_rcp = e.bias = 16  # (presence only: nothing is launched)
-    took = _native.kernel_lib().catchq_conv3x3_i8_packed_takes(n, h, w, (ci + 15) // 16 * 16, co, ctypes.byref(e))
+    took = _native.kernel_lib().catchq_conv3x3_i8_packed_any_takes(n, h, w, (ci + 15) // 16 * 16, co, ctypes.byref(e))
     assert took == 0 or n * h * w < 2048
     args = (wt.cuda(), b.cuda(), [1, 1], [1, 1], [1, 1], 1, scale.cuda(), qm.cuda())
     xd = x.cuda().contiguous(memory_format=torch.channels_last)
