@@ -69,6 +69,11 @@ Tensor device_empty(at::IntArrayRef shape, at::ScalarType type, at::Device devic
   return Tensor(at::detail::empty_cuda(shape, type, device, format));
 }
 
+// at::empty_like (the strides of a dense tensor are kept) likewise
+Tensor device_empty_like(const Tensor &dense, at::ScalarType type) {
+  return Tensor(at::detail::empty_strided_cuda(dense.sizes(), dense.strides(), type, dense.device()));
+}
+
 bool has_bias(const Tensor &b) { return b.defined() && b.numel() != 0 && b.dim() != 0; }
 
 // ------------------------------------------------------------------------------------------------
@@ -80,7 +85,7 @@ Tensor quantize_op(const Tensor &x, int64_t bitwidth, int64_t position, double s
   const int dt = fp_dtype(x, "quantify only support input float/half");
   c10::DeviceGuard guard(x.device());
   Tensor xi = x.is_non_overlapping_and_dense() ? x : x.contiguous();
-  Tensor q = at::empty_like(xi, xi.options().dtype(int_type(bitwidth)));
+  Tensor q = device_empty_like(xi, int_type(bitwidth));
   check_status(catchq_quantize(xi.data_ptr(), dt, q.data_ptr(), (int)bitwidth, xi.numel(), (int)position,
                                (float)scale, current_stream()),
                "torch_mlu::quantize");
@@ -94,7 +99,7 @@ Tensor quantize_dev_op(const Tensor &x, int64_t bitwidth, const Tensor &position
               "position must be a one-element int32 tensor on the input's device");
   c10::DeviceGuard guard(x.device());
   Tensor xi = x.is_non_overlapping_and_dense() ? x : x.contiguous();
-  Tensor q = at::empty_like(xi, xi.options().dtype(int_type(bitwidth)));
+  Tensor q = device_empty_like(xi, int_type(bitwidth));
   check_status(catchq_quantize_devpos(xi.data_ptr(), dt, q.data_ptr(), (int)bitwidth, xi.numel(),
                                       position.data_ptr<int32_t>(), nullptr, current_stream()),
                "torch_mlu::quantize_dev");
@@ -214,7 +219,7 @@ std::tuple<Tensor, Tensor, Tensor> quantize_per_channel_op(const Tensor &w, cons
 Tensor dequantize_op(const Tensor &q, int64_t position, double scale, bool half) {
   c10::DeviceGuard guard(q.device());
   Tensor qi = q.is_non_overlapping_and_dense() ? q : q.contiguous();
-  Tensor y = at::empty_like(qi, qi.options().dtype(half ? at::kHalf : at::kFloat));
+  Tensor y = device_empty_like(qi, half ? at::kHalf : at::kFloat);
   check_status(catchq_dequantize(qi.data_ptr(), bits_of(qi), y.data_ptr(), half ? CATCHQ_F16 : CATCHQ_F32,
                                  qi.numel(), (int)position, (float)scale, current_stream()),
                "torch_mlu::dequantize");
