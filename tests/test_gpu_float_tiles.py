@@ -66,3 +66,13 @@ def test_conv2d(n, ci, h, w, co, k, stride, nhwc, dtype):
         _same(ref, first[i:i + 1])
     for _ in range(2):
         assert torch.equal(torch.ops.torch_mlu.conv2d(xd, *args), first)
+
+
+@pytest.mark.parametrize("n,ci,h,w,co,k", [
+    (5, 362, 30, 30, 503, 5),  # 128x128, eight waves, from half a block a unit on
+    (3, 32, 74, 79, 432, 5), (5, 40, 89, 90, 140, 5),  # 128x64 on taps that a step crosses
+    (9, 129, 52, 53, 131, 5),  # 128x128, four waves, up to 1.8 blocks a unit
+    (14, 288, 60, 60, 173, 5),  # 256x256 on less than 256 columns
+    (4, 64, 92, 92, 378, 5)])  # 128x128 where the last 256 columns are half empty
+def test_conv2d_larger(n, ci, h, w, co, k):
+    test_conv2d(n, ci, h, w, co, k, 1, True, torch.float16)
