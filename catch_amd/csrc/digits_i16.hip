@@ -24,7 +24,7 @@
 // Measured: see gemm_digits_bytes and conv_digits_bytes below.
 #include <type_traits>
 
-#include "igemm_common.h"
+#include "nchw_quantize.h"
 
 namespace catchq {
 
@@ -415,65 +415,44 @@ int gemm_digits(const void *x, bool half, int position, const void *packed, int6
   return launch_digits<4, 8>(a, b, sums, p, NoConv{}, e, s);
 }
 
-// floats -> digits by pixels, [pixel][channel / 32][high, low digits of 32 channels], and a pixel of zeros behind them.  APART: channels
-// lie HW values apart (NCHW), a lane takes 32 of them and lanes follow the pixels; otherwise two lanes have a pixel's 32 channels.
-template <typename TIn, bool APART>
+// channels-last floats -> digits by pixels, [pixel][channel / 32][high, low digits of 32 channels], and a pixel of zeros behind them: two
+// lanes have a pixel's 32 channels (planes: nchw_quantize.h).
+template <typename TIn>
 __global__ __launch_bounds__(256) void quantize_pixel_digits_kernel(const TIn *__restrict__ x, int8_t *__restrict__ out, int64_t pixels,
-                                                                    int C, int c32, unsigned HW, int64_t tasks, int neg_pos) {
+                                                                    int C, int c32, int64_t tasks, int neg_pos) {
   struct __attribute__((aligned(sizeof(TIn)))) run16 { TIn v[16]; };
   const int64_t task = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (task >= tasks) return;
-  constexpr int HALVES = APART ? 2 : 1;  // 16 channels each
-  int64_t px;
-  int ch;
-  if constexpr (APART) {
-    ch = (int)(task / (pixels + 1));
-    px = task - (int64_t)ch * (pixels + 1);
-    ch *= 32;
-  } else {
-    px = task / (2 * c32);
-    ch = (int)(task - px * (2 * c32)) * 16;
-  }
-  float v[HALVES][16];
+  const int64_t px = task / (2 * c32);
+  const int ch = (int)(task - px * (2 * c32)) * 16;
+  float v[16];
 #pragma unroll
-  for (int h = 0; h < HALVES; ++h)
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[h][i] = 0.0f;
+  for (int i = 0; i < 16; ++i) v[i] = 0.0f;
   if (px < pixels) {
-    if constexpr (APART) {
-      const int64_t img = px / HW, at = img * C * HW + (px - img * HW);
+    const TIn *const row = x + px * C + ch;
+    if (ch + 16 <= C) {
+      const run16 t = *reinterpret_cast<const run16 *>(row);
 #pragma unroll
-      for (int i = 0; i < 32; ++i)
-        if (ch + i < C) v[i / 16][i % 16] = (float)x[at + (int64_t)(ch + i) * HW];
+      for (int i = 0; i < 16; ++i) v[i] = (float)t.v[i];
     } else {
-      const TIn *const row = x + px * C + ch;
-      if (ch + 16 <= C) {
-        const run16 t = *reinterpret_cast<const run16 *>(row);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) v[0][i] = (float)t.v[i];
-      } else {
-#pragma unroll
-        for (int i = 0; i < 16; ++i)
-          if (ch + i < C) v[0][i] = (float)row[i];
-      }
+      for (int i = 0; i < 16; ++i)
+        if (ch + i < C) v[i] = (float)row[i];
     }
   }
+  v4i c[2], hi, lo;
 #pragma unroll
-  for (int h = 0; h < HALVES; ++h) {
-    v4i c[2], hi, lo;
+  for (int g = 0; g < 2; ++g)
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
-#pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        const int a = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(v[h][g * 8 + d * 2], neg_pos)));
-        const int b = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(v[h][g * 8 + d * 2 + 1], neg_pos)));
-        c[g][d] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pk_i16(a, b));  // (saturates)
-      }
-    split_i16(c[0], c[1], hi, lo);
-    v4i *const dst = reinterpret_cast<v4i *>(out + (px * c32 + ch / 32) * 64 + (ch & 16)) + h;
-    dst[0] = hi;
-    dst[2] = lo;
-  }
+    for (int d = 0; d < 4; ++d) {
+      const int a = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(v[g * 8 + d * 2], neg_pos)));
+      const int b = cvt_i32_sat(__builtin_rintf(__builtin_ldexpf(v[g * 8 + d * 2 + 1], neg_pos)));
+      c[g][d] = __builtin_bit_cast(int, __builtin_amdgcn_cvt_pk_i16(a, b));  // (saturates)
+    }
+  split_i16(c[0], c[1], hi, lo);
+  v4i *const dst = reinterpret_cast<v4i *>(out + (px * c32 + ch / 32) * 64 + (ch & 16));
+  dst[0] = hi;
+  dst[2] = lo;
 }
 
 // Bytes of the activations' digits where this route serves the convolution; 0: another one does.
@@ -492,16 +471,15 @@ int conv_digits(const void *x, bool half, int position, int x_ci, bool apart, co
                 hipStream_t s) {
   const int64_t pixels = (int64_t)N * H * W;
   const int c32 = (Ci + 31) / 32;
-  const int64_t tasks = (pixels + 1) * c32 * (apart ? 1 : 2);
-  const unsigned quantizers = (unsigned)((tasks + 255) / 256), hw = (unsigned)((int64_t)H * W);
   int8_t *const a = static_cast<int8_t *>(digits);
-  auto quantize = [&](auto kern, auto *from) { kern<<<quantizers, 256, 0, s>>>(from, a, pixels, x_ci, c32, hw, tasks, -position); };
-  if (half) {
-    if (apart) quantize(quantize_pixel_digits_kernel<_Float16, true>, (const _Float16 *)x);
-    else quantize(quantize_pixel_digits_kernel<_Float16, false>, (const _Float16 *)x);
+  if (apart) {
+    auto planes = [&](auto *from) { return pixel_quantize<typename std::remove_cv<typename std::remove_reference<decltype(*from)>::type>::type, PX_DIGITS>(from, a, N, x_ci, (int64_t)H * W, c32 * 64, position, 1.0f, pixels * c32 * 64, s); };
+    if (!(half ? planes(static_cast<const _Float16 *>(x)) : planes(static_cast<const float *>(x)))) return CATCHQ_ERR_UNSUPPORTED;
   } else {
-    if (apart) quantize(quantize_pixel_digits_kernel<float, true>, (const float *)x);
-    else quantize(quantize_pixel_digits_kernel<float, false>, (const float *)x);
+    const int64_t tasks = (pixels + 1) * c32 * 2;
+    const unsigned quantizers = (unsigned)((tasks + 255) / 256);
+    if (half) quantize_pixel_digits_kernel<_Float16><<<quantizers, 256, 0, s>>>((const _Float16 *)x, a, pixels, x_ci, c32, tasks, -position);
+    else quantize_pixel_digits_kernel<float><<<quantizers, 256, 0, s>>>((const float *)x, a, pixels, x_ci, c32, tasks, -position);
   }
   const int st = launch_status();
   if (st != CATCHQ_OK) return st;

@@ -2,7 +2,7 @@
 // lane-contiguous so every wave instruction touches whole cache lines.
 #include <mutex>
 
-#include "catchq_common.h"
+#include "nchw_quantize.h"
 
 namespace catchq {
 
@@ -261,7 +261,8 @@ __global__ __launch_bounds__(kThreads) void quantize_frame_f32_i8c4_kernel(const
   }
 }
 
-// General (any C) transpose-quantize through LDS: tile of 64 pixels x 64 channels, any alignment and pitch of the output.
+// General (any C) transpose-quantize through LDS: tile of 64 pixels x 64 channels, any alignment and pitch of the output
+// (whole aligned 16-byte pieces a pixel: nchw_quantize.h).
 template <typename TIn, int BW>
 __global__ __launch_bounds__(kThreads) void quantize_nchw_nhwc_tile_kernel(const TIn *__restrict__ x,
                                                                           typename QRange<BW>::type *__restrict__ q,
@@ -292,64 +293,6 @@ __global__ __launch_bounds__(kThreads) void quantize_nchw_nhwc_tile_kernel(const
       if (ch < cpad && pix < hw) q[(img * hw + pix) * cpad + ch] = tile[i / 64][i & 63];
     }
     __syncthreads();
-  }
-}
-
-// The same where a pixel of the output is a whole number of aligned 16-byte pieces.  Bound by memory; the kernel above is
-// bound by its instructions (a load, a conversion, a byte store to LDS, one back and a byte store to memory per element:
-// 5 x 96 x 57 x 75 fp32 -> int8 took 10.4 us, this one 4.6).  A lane takes four consecutive pixels of four channels (four
-// 16-byte loads, a wave instruction covering 256 consecutive bytes of four planes), packs a pixel's four channels into a
-// dword (two for int16) in LDS -- the pitch of 16 DW + 1 dwords spreads a wave's stores over all banks -- and leaves with
-// 16-byte stores that cover whole 64-byte runs of a pixel.
-template <typename TIn> struct __attribute__((aligned(sizeof(TIn)))) px4 { TIn v[4]; };
-template <typename TIn, int BW>
-__global__ __launch_bounds__(kThreads) void quantize_nchw_nhwc_vec_kernel(const TIn *__restrict__ x,
-                                                                         typename QRange<BW>::type *__restrict__ q,
-                                                                         int c, int hw, int cpad, int pos, float scale) {
-  constexpr int DW = BW / 8;              // dwords of a pixel's four channels
-  constexpr int PITCH = 16 * DW + 1;
-  __shared__ int tile[64 * PITCH];
-  const int p0 = blockIdx.x * 64, c0 = blockIdx.y * 64;
-  const int64_t img = blockIdx.z;
-  const int pg = threadIdx.x & 15, cq = threadIdx.x >> 4;
-  const int px = p0 + pg * 4, ch = c0 + cq * 4;
-  const TIn *src = x + (img * c + ch) * (int64_t)hw + px;
-  float v[4][4];  // [channel][pixel]
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (ch + j < c && px + 4 <= hw) {
-      const px4<TIn> t = *reinterpret_cast<const px4<TIn> *>(src + (int64_t)j * hw);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[j][i] = ld_f(t.v, i);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) v[j][i] = (ch + j < c && px + i < hw) ? ld_f(src + (int64_t)j * hw, i) : 0.0f;
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int b[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) b[j] = quant1<BW>(v[j][i], scale, -pos);  // 0 -> 0: the padding channels
-    int *dst = tile + (pg * 4 + i) * PITCH + cq * DW;
-    if constexpr (BW == 8) {
-      dst[0] = (int)(__builtin_amdgcn_perm((unsigned)b[1], (unsigned)b[0], 0x0c0c0400u) |
-                     __builtin_amdgcn_perm((unsigned)b[3], (unsigned)b[2], 0x04000c0cu));
-    } else {
-      dst[0] = (b[0] & 0xffff) | (b[1] << 16);
-      dst[1] = (b[2] & 0xffff) | (b[3] << 16);
-    }
-  }
-  __syncthreads();
-  constexpr int PIECES = 4 * DW;  // 16-byte pieces of a pixel's 64 channels
-  const int piece = threadIdx.x % PIECES;
-  const bool c_ok = c0 * DW + piece * 16 < cpad * DW;
-#pragma unroll
-  for (int r = 0; r < DW; ++r) {
-    const int p = threadIdx.x / PIECES + r * (kThreads / PIECES);
-    const int *s = tile + p * PITCH + piece * 4;
-    if (c_ok && p0 + p < hw)
-      reinterpret_cast<v4i *>(q + (img * hw + p0 + p) * (int64_t)cpad + c0)[piece] = v4i{s[0], s[1], s[2], s[3]};
   }
 }
 
@@ -415,9 +358,11 @@ static int launch_nchw_nhwc(const void *x, void *q, int n, int c, int h, int w, 
       launch_rows<TIn, BW, 8>((const TIn *)x, (TQ *)q, n, c, cpad, pos, scale, s);
     else
       launch_rows<TIn, BW, 4>((const TIn *)x, (TQ *)q, n, c, cpad, pos, scale, s);
-  } else if (cpad * sizeof(TQ) % 16 == 0 && aligned16(q) && n < 65536 && cpad < 65536 * 64 && hw < (1ll << 31) - 64) {
-    quantize_nchw_nhwc_vec_kernel<TIn, BW><<<dim3((unsigned)((hw + 63) / 64), (unsigned)((cpad + 63) / 64), (unsigned)n), kThreads, 0, s>>>(
-        (const TIn *)x, (TQ *)q, c, (int)hw, cpad, pos, scale);
+  } else if (cpad * sizeof(TQ) % 16 == 0 && aligned16(q) && cpad < (1 << 30) &&
+             pixel_quantize<typename std::conditional<sizeof(TIn) == 2, _Float16, float>::type, BW>(
+                 reinterpret_cast<const typename std::conditional<sizeof(TIn) == 2, _Float16, float>::type *>(x), (int8_t *)q, n, c, hw,
+                 (int)(cpad * sizeof(TQ)), pos, scale, 0, s)) {
+    // launched
   } else {
     int64_t tiles = (int64_t)n * ((hw + 63) / 64) * ((cpad + 63) / 64);
     quantize_nchw_nhwc_tile_kernel<TIn, BW><<<grid_for(tiles, 1), kThreads, 0, s>>>(
