@@ -274,7 +274,7 @@ int dw_float(const void *x, bool half, int position, bool nchw, const void *w, i
   p.N = N; p.H = H; p.W = W; p.C = C; p.ph = ph; p.pw = pw; p.Ho = Ho; p.Wo = Wo; p.nchw = nchw; p.neg_pos = -position;
   dwf_tile(p, bits, stride, e.cus);
   const int64_t blocks = (int64_t)N * p.bands * p.strips * p.slabs;
-  if (blocks > 0x7ffffff0) return CATCHQ_ERR_UNSUPPORTED;
+  if (blocks >= (1 << 24)) return CATCHQ_ERR_UNSUPPORTED;  // (a launch has less than 2^32 lanes)
   p.blocks = (unsigned)blocks;
 #define CATCHQ_DWF(H_, E_)                                                                                            \
   if (bits == 8) stride == 1 ? dwf_launch<H_, 8, 1, E_>(x, w, p, e, s) : dwf_launch<H_, 8, 2, E_>(x, w, p, e, s);     \

@@ -99,7 +99,7 @@ static bool pixel_quantize(const TIn *x, int8_t *q, int64_t n, int c, int64_t hw
   PixelQuantParams p = {c, (int)hw, (unsigned)((channels + 4 * cq - 1) / (4 * cq)), 0, 0, pitch, -pos, scale, zeros};
   const int groups = 256 / cq;
   auto tiles = [&](int px) { return n * ((hw + px - 1) / px) * p.ctiles; };
-  if (hw >= (1ll << 31) - 1024 || tiles(groups) >= (1ll << 31) - 8) return false;
+  if (hw >= (1ll << 31) - 1024 || tiles(groups) >= (1 << 24)) return false;  // (a launch has less than 2^32 lanes)
   const int pxl = hw < 4 ? 1 : sizeof(TIn) == 2 && hw >= 8 && tiles(groups * 8) >= planned_cus(1) ? 8 : 4;
   p.ptiles = (unsigned)((hw + groups * pxl - 1) / (groups * pxl));
   p.blocks = (unsigned)tiles(groups * pxl);
