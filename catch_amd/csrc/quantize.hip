@@ -26,8 +26,9 @@ __device__ __forceinline__ float ld_f(const float *p, int64_t i) { return p[i]; 
 __device__ __forceinline__ float ld_f(const __half *p, int64_t i) { return __half2float(p[i]); }
 
 // ---- per-tensor quantize -------------------------------------------------------------------------
-// Vector body: each lane converts VEC consecutive elements per step (one 16-byte load).
-template <typename TIn, int BW>
+// Vector body: each lane converts U times VEC consecutive elements per step (16-byte loads, all on their way before the first
+// conversion).
+template <typename TIn, int BW, int U>
 __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(const TIn *__restrict__ x,
                                                                typename QRange<BW>::type *__restrict__ q,
                                                                int64_t n, int pos, float scale,
@@ -40,30 +41,40 @@ __global__ __launch_bounds__(kThreads) void quantize_vec_kernel(const TIn *__res
   const int neg_pos = -pos;
   const int64_t nvec = n / VEC;
   const int64_t stride = (int64_t)gridDim.x * kThreads;
-  for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < nvec; i += stride) {
-    v4i raw = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(x) + i);
-    TQ out[VEC];
-    if constexpr (sizeof(TIn) == 4) {
+  for (int64_t first = (int64_t)blockIdx.x * (kThreads * U) + threadIdx.x; first < nvec; first += stride * U) {
+    v4i loaded[U];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) out[j] = (TQ)quant1<BW>(__int_as_float(raw[j]), scale, neg_pos);
-    } else {
+    for (int u = 0; u < U; ++u)
+      if (u == 0 || first + u * kThreads < nvec)
+        loaded[u] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(x) + first + u * kThreads);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const __half2 h = as_half2(raw[j]);
-        out[2 * j] = (TQ)quant1<BW>(__low2float(h), scale, neg_pos);
-        out[2 * j + 1] = (TQ)quant1<BW>(__high2float(h), scale, neg_pos);
+    for (int u = 0; u < U; ++u) {
+      const int64_t i = first + u * kThreads;
+      if (u != 0 && i >= nvec) break;
+      const v4i raw = loaded[u];
+      TQ out[VEC];
+      if constexpr (sizeof(TIn) == 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[j] = (TQ)quant1<BW>(__int_as_float(raw[j]), scale, neg_pos);
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const __half2 h = as_half2(raw[j]);
+          out[2 * j] = (TQ)quant1<BW>(__low2float(h), scale, neg_pos);
+          out[2 * j + 1] = (TQ)quant1<BW>(__high2float(h), scale, neg_pos);
+        }
       }
-    }
-    constexpr int OUT_BYTES = VEC * sizeof(TQ);
-    if constexpr (OUT_BYTES == 4) {
-      *reinterpret_cast<int *>(q + i * VEC) = *reinterpret_cast<int *>(out);
-    } else if constexpr (OUT_BYTES == 8) {
-      *reinterpret_cast<v2i *>(q + i * VEC) = *reinterpret_cast<v2i *>(out);
-    } else if constexpr (OUT_BYTES == 16) {
-      *reinterpret_cast<v4i *>(q + i * VEC) = *reinterpret_cast<v4i *>(out);
-    } else {
-      reinterpret_cast<v4i *>(q + i * VEC)[0] = reinterpret_cast<v4i *>(out)[0];
-      reinterpret_cast<v4i *>(q + i * VEC)[1] = reinterpret_cast<v4i *>(out)[1];
+      constexpr int OUT_BYTES = VEC * sizeof(TQ);
+      if constexpr (OUT_BYTES == 4) {
+        *reinterpret_cast<int *>(q + i * VEC) = *reinterpret_cast<int *>(out);
+      } else if constexpr (OUT_BYTES == 8) {
+        *reinterpret_cast<v2i *>(q + i * VEC) = *reinterpret_cast<v2i *>(out);
+      } else if constexpr (OUT_BYTES == 16) {
+        *reinterpret_cast<v4i *>(q + i * VEC) = *reinterpret_cast<v4i *>(out);
+      } else {
+        reinterpret_cast<v4i *>(q + i * VEC)[0] = reinterpret_cast<v4i *>(out)[0];
+        reinterpret_cast<v4i *>(q + i * VEC)[1] = reinterpret_cast<v4i *>(out)[1];
+      }
     }
   }
   // tail (< VEC elements) by the first lanes of block 0
@@ -95,9 +106,14 @@ static int launch_quantize(const void *x, void *q, int64_t n, int pos, float sca
   constexpr int VEC = 16 / sizeof(TIn);
   if (aligned16(x) && aligned16(q)) {
     // one vector per lane up to the grid's limit (4.2 M fp32 values), whose lanes walk on from there: a lane's loads follow
-    // each other
-    quantize_vec_kernel<TIn, BW><<<grid_for(n / VEC, kThreads), kThreads, 0, s>>>(
-        (const TIn *)x, (TQ *)q, n, pos, scale, pos_dev, scale_dev);
+    // each other.  From four times that many on two vectors a lane, and no walking (us, 51 M fp32 values to int8 42.8 / 41.0, to int16
+    // 49.3 / 46.4, fp16 27.2 / 25.6; 12 M fp16 8.4 / 8.6; four a lane 43.1).
+    const int64_t nvec = n / VEC, blocks = (nvec + 2 * kThreads - 1) / (2 * kThreads);
+    if (nvec >= 4ll * kMaxBlocks * kThreads && blocks < (1 << 24))
+      quantize_vec_kernel<TIn, BW, 2><<<(unsigned)blocks, kThreads, 0, s>>>((const TIn *)x, (TQ *)q, n, pos, scale, pos_dev, scale_dev);
+    else
+      quantize_vec_kernel<TIn, BW, 1><<<grid_for(nvec, kThreads), kThreads, 0, s>>>((const TIn *)x, (TQ *)q, n, pos, scale, pos_dev,
+                                                                                    scale_dev);
   } else {
     quantize_scalar_kernel<TIn, BW><<<grid_for(n, kThreads * 4), kThreads, 0, s>>>(
         (const TIn *)x, (TQ *)q, n, pos, scale, pos_dev, scale_dev);
