@@ -104,24 +104,21 @@ def layer_profile(fused, x, iters=20, only=None):
             fused_inner.update((bx.name, bd.name))
     fused_expansions = set(bx.name for d, bx in fused.expansion_of.items() if d not in fused_inner and fused.expansion_fuses(
         next(l for l in fused.layers if l.name == d), *trace[bx.name]["qx"].shape[:3]))
-    first = fused.first_layers_fuse(*x.shape)  # quantizer, first convolution and pooling in one launch
+    first = fused.first_layers_run(*x.shape)  # quantizer, first convolution and pooling in one launch
     for l in fused.layers:
         if l.kind not in ("conv", "fc") or l.name in fused._fused_away or l.name in fused_heads or l.name in fused_inner or l.name in fused_expansions \
                 or (only and l.name != only):
             continue
         if first and l is fused.layers[0]:
-            lq, pool, d = fused.q[l.name], fused.first_pool, fused.q_demand["input"][0]
-            qd = fused.q_demand[pool.name][0]
-            code = {"relu": 1, "relu6": 2}[l.act]
+            lq = fused.q[l.name]
 
-            def run(l=l, lq=lq, pool=pool, d=d, qd=qd, code=code):
-                return ops.qconv2d_first_layers(x, d[1], d[2], lq.qw, lq.exp2, lq.chan_div, lq.bias, code, qd[1], l.k, l.stride,
-                                                l.pad, pool.k, pool.stride, pool.pad)
-            pooled = run()
+            def run():
+                return fused.first_layers(x)
+            pooled = run()[1]
             macs = trace[l.name]["y"].numel() * (lq.qw.numel() // lq.qw.shape[0])
             t = event_time(run, iters)
             rows.append(dict(name=l.name, route="mfma+first", t=t, ops=2 * macs,
-                             bytes=x.numel() * 4 + lq.qw.numel() + pooled.numel()))
+                             bytes=x.numel() * 4 + lq.qw.numel() + pooled.numel() * (5 if fused.first_floats else 1)))
             continue
         lq = fused.q[l.name]
         qx = trace[l.name].get("qx_dev", trace[l.name]["qx"])  # the tensor the kernel reads
@@ -256,7 +253,7 @@ def plan_launches(fused, n, h, w):
     rows, shape = [], {}
     pooled_inside = set()  # 1x1 convolutions that run inside the launch of the global average pooling behind them
     cin = fused.cdev["input"]
-    first = fused.first_layers_fuse(n, fused.chan["input"], h, w)  # quantizer, first convolution and pooling in one launch
+    first = fused.first_layers_run(n, fused.chan["input"], h, w)  # quantizer, first convolution and pooling in one launch
     for d in fused.q_demand["input"] if not first else ():
         if fused.stem:
             sp = fused.stem["pad"]
@@ -288,7 +285,7 @@ def plan_launches(fused, n, h, w):
                 lq, pool = fused.q[l.name], fused.first_pool
                 hp, wp = (ho + 2 * pool.pad - pool.k) // pool.stride + 1, (wo + 2 * pool.pad - pool.k) // pool.stride + 1
                 rows.append(dict(name=l.name, kind="conv", ops=2 * n * ho * wo * fused.cdev[l.name] * (lq.qw.numel() // lq.qw.shape[0]),
-                                 bytes=n * fused.chan["input"] * h * w * 4 + lq.qw.numel() + n * hp * wp * fused.cdev[l.name],
+                                 bytes=n * fused.chan["input"] * h * w * 4 + lq.qw.numel() + n * hp * wp * fused.cdev[l.name] * (5 if fused.first_floats else 1),
                                  m=n * ho * wo, n=fused.cdev[l.name], k=lq.qw.numel() // lq.qw.shape[0]))
                 continue
             if l.name in fused._block_inner:
@@ -643,7 +640,7 @@ def main():
                                          if fused.expansion_fuses(next(l for l in fused.layers if l.name == d), batch // args.streams,
                                                                   *head_hw(fused, bx, side))),
               # input quantizer, first convolution and max pooling in one launch
-              "fused_first_layers": fused.first_layers_fuse(batch // args.streams, fused.chan["input"], side, side),
+              "fused_first_layers": fused.first_layers_run(batch // args.streams, fused.chan["input"], side, side),
               # 1x1 convolutions that run inside the launch of the global average pooling behind them
               "fused_avgpool": sorted(c.name for g, c in fused.pooled_conv.items()
                                       if fused.avgpool_fuses(next(l for l in fused.layers if l.name == g), batch // args.streams,

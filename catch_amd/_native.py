@@ -138,6 +138,10 @@ SIGNATURES = {
                                                 _I, ctypes.POINTER(_SZ)]),
     "catchq_first_layers_nchw": (_I, [_P, _I, _I, _I, _I, _I, ctypes.c_float, _I, _I, _I, _I, _I,
                                       ctypes.POINTER(RequantStage), _I, _I, _I, _P, _I, _P, _SZ, _P]),
+    "catchq_first_layers_any_workspace_size": (_I, [_I, _I, _I, _I, _I, _I, _I, _I, _I, ctypes.POINTER(RequantStage), _I, _I, _I,
+                                                    _I, _I, ctypes.POINTER(_SZ)]),
+    "catchq_first_layers_any_nchw": (_I, [_P, _I, _I, _I, _I, _I, ctypes.c_float, _I, _I, _I, _I, _I,
+                                          ctypes.POINTER(RequantStage), _I, _I, _I, _P, _P, _I, _P, _SZ, _P]),
     "catchq_conv1x1_avgpool_workspace_size": (_I, [_I, _I, _I, _I, ctypes.POINTER(Epilogue), ctypes.POINTER(_SZ)]),
     "catchq_conv1x1_avgpool_nhwc": (_I, [_P, _P, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P, _P, _I, _I, ctypes.c_float,
                                          _P, _SZ, _P]),

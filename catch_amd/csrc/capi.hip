@@ -83,9 +83,9 @@ int irb_i8(const void *x, int N, int H, int W, int Cin, int hid, int Co, int S, 
 bool expand_dw_i8_ok(int N, int H, int W, int Cin, int hid, int S, int cus);
 int expand_dw_i8(const void *x, int N, int H, int W, int Cin, int hid, int S, const IrbStageDev &s1, const IrbStageDev &s2, void *q,
                  int cus, hipStream_t s);
-bool stem_pool_i8_ok(int N, int C, int H, int W, int Co);
+bool stem_pool_i8_ok(int N, int C, int H, int W, int Co, bool floats, bool any_width);
 int stem_pool_i8(const void *x, int N, int C, int H, int W, int x_pos, float x_scale, const IrbStageDev &s, int Co,
-                 void *q, hipStream_t st);
+                 float *y, void *q, hipStream_t st);
 struct GapConvDev {
   const float *div, *rcp, *bias, *resid;
   int exp2, act;
@@ -932,46 +932,52 @@ static int check_first_layers(int n, int c, int h, int w, int co, int kh, int kw
 
 static bool first_layers_fusable(int n, int c, int h, int w, int co, int kh, int kw, int stride, int pad,
                                  const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad,
-                                 int sharing) {
+                                 bool floats, bool any_width) {
   return kh == 7 && kw == 7 && stride == 2 && pad == 3 && pool_k == 3 && pool_stride == 2 && pool_pad == 1 &&
          conv->chan_div && conv->chan_rcp && conv->bias && conv->exp2 >= -64 && conv->exp2 <= 64 &&
-         stem_pool_i8_ok(n, c, h, w, co);
+         stem_pool_i8_ok(n, c, h, w, co, floats, any_width);
 }
 
-CATCHQ_API int catchq_first_layers_workspace_size(int n, int c, int h, int w, int co, int kh, int kw, int stride,
-                                                  int pad, const catchq_requant_stage_t *conv, int pool_k,
-                                                  int pool_stride, int pool_pad, int sharing, size_t *bytes) {
+// bytes of the workspace behind each other: the framed int8 image, the convolution's output
+static size_t first_layers_image(int n, const FirstLayersShape &sh) { return round256((size_t)n * sh.fh * sh.fw * 4); }
+static size_t first_layers_conv(int n, int co, bool floats, const FirstLayersShape &sh) {
+  return round256((size_t)n * sh.hc * sh.wc * co * (floats ? 4 : 1));
+}
+
+static int first_layers_bytes(int n, int c, int h, int w, int co, int kh, int kw, int stride, int pad,
+                              const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad, bool floats, bool any_width,
+                              size_t *bytes) {
   FirstLayersShape sh;
   const int st = check_first_layers(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, &sh);
   if (st != CATCHQ_OK) return st;
   if (!bytes) return CATCHQ_ERR_ARG;
-  *bytes = first_layers_fusable(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, sharing)
-               ? 0 : round256((size_t)n * sh.fh * sh.fw * 4) + round256((size_t)n * sh.hc * sh.wc * co);
+  *bytes = first_layers_fusable(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, floats, any_width)
+               ? 0 : first_layers_image(n, sh) + first_layers_conv(n, co, floats, sh);
   return CATCHQ_OK;
 }
 
-CATCHQ_API int catchq_first_layers_nchw(const float *x, int n, int c, int h, int w, int x_position, float x_scale,
-                                        int co, int kh, int kw, int stride, int pad,
-                                        const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad,
-                                        void *q, int sharing, void *workspace, size_t workspace_bytes,
-                                        catchq_stream_t stream) {
+// q, and the pooled floats where there is a y for them
+static int first_layers(const float *x, int n, int c, int h, int w, int x_position, float x_scale, int co, int kh, int kw, int stride, int pad,
+                        const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad, bool any_width, float *y, void *q,
+                        int sharing, void *workspace, size_t workspace_bytes, catchq_stream_t stream) {
   FirstLayersShape sh;
   int st = check_first_layers(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, &sh);
   if (st != CATCHQ_OK) return st;
   if (x_position < -126 || x_position > 126) return CATCHQ_ERR_ARG;
   if (n == 0) return CATCHQ_OK;
   if (!x || !q || !conv->w) return CATCHQ_ERR_ARG;
-  if (first_layers_fusable(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, sharing) &&
-      aligned16(x) && aligned16(conv->w) && aligned16(q)) {
+  const bool floats = y != nullptr;
+  if (first_layers_fusable(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, floats, any_width) &&
+      (w % 4 != 0 || aligned16(x)) && aligned16(conv->w) && aligned16(q) && (!floats || aligned16(y))) {
     const IrbStageDev s = {(const int8_t *)conv->w, conv->chan_div, conv->chan_rcp, conv->bias, conv->exp2,
                            -conv->q_position, conv->act == CATCHQ_ACT_RELU6 ? 1 : 0};
-    const int st2 = stem_pool_i8(x, n, c, h, w, x_position, x_scale, s, co, q, as_stream(stream));
+    const int st2 = stem_pool_i8(x, n, c, h, w, x_position, x_scale, s, co, y, q, as_stream(stream));
     if (st2 >= 0) return st2;
   }
-  // three launches: the framed int8 image and the convolution's output go through the workspace
-  const size_t b1 = round256((size_t)n * sh.fh * sh.fw * 4), b2 = round256((size_t)n * sh.hc * sh.wc * co);
+  // layer by layer: the framed int8 image and the convolution's output go through the workspace
+  const size_t b1 = first_layers_image(n, sh), b2 = first_layers_conv(n, co, floats, sh);
   if (!workspace || workspace_bytes < b1 + b2 || !aligned16(workspace)) return CATCHQ_ERR_ARG;
-  void *qx = workspace, *q1 = (char *)workspace + b1;
+  void *qx = workspace, *out = (char *)workspace + b1;
   st = catchq_quantize_nchw_to_nhwc_frame(x, CATCHQ_F32, qx, 8, n, c, h, w, 4, sh.fh, sh.fw, pad, pad, x_position, x_scale,
                                           stream);
   if (st != CATCHQ_OK) return st;
@@ -982,15 +988,50 @@ CATCHQ_API int catchq_first_layers_nchw(const float *x, int n, int c, int h, int
   es.chan_rcp = conv->chan_rcp;
   es.bias = conv->bias;
   es.act = conv->act;
-  es.q = q1;
-  es.q_bitwidth = 8;
-  es.q_position = conv->q_position;
-  es.q_scale = 1.0f;
   es.sharing = sharing;
+  if (floats) {
+    es.y = out;
+  } else {
+    es.q = out;
+    es.q_bitwidth = 8;
+    es.q_position = conv->q_position;
+    es.q_scale = 1.0f;
+  }
   const catchq_conv_desc_t d = {n, sh.fh, sh.fw, 4, co, kh, sh.kw4, 0, 0, stride, stride, 1, 1, 1};
   st = catchq_conv2d_nhwc(qx, 8, conv->w, 8, &d, &es, stream);
   if (st != CATCHQ_OK) return st;
-  return catchq_maxpool_nhwc(q1, q, 8, n, sh.hc, sh.wc, co, pool_k, pool_stride, pool_pad, stream);
+  st = catchq_maxpool_nhwc(out, floats ? (void *)y : q, floats ? 32 : 8, n, sh.hc, sh.wc, co, pool_k, pool_stride, pool_pad, stream);
+  if (st != CATCHQ_OK || !floats) return st;
+  return catchq_quantize(y, CATCHQ_F32, q, 8, (int64_t)n * sh.hp * sh.wp * co, conv->q_position, 1.0f, stream);
+}
+
+CATCHQ_API int catchq_first_layers_workspace_size(int n, int c, int h, int w, int co, int kh, int kw, int stride,
+                                                  int pad, const catchq_requant_stage_t *conv, int pool_k,
+                                                  int pool_stride, int pool_pad, int sharing, size_t *bytes) {
+  return first_layers_bytes(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, false, false, bytes);
+}
+
+CATCHQ_API int catchq_first_layers_nchw(const float *x, int n, int c, int h, int w, int x_position, float x_scale,
+                                        int co, int kh, int kw, int stride, int pad,
+                                        const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad,
+                                        void *q, int sharing, void *workspace, size_t workspace_bytes,
+                                        catchq_stream_t stream) {
+  return first_layers(x, n, c, h, w, x_position, x_scale, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, false, nullptr, q,
+                      sharing, workspace, workspace_bytes, stream);
+}
+
+CATCHQ_API int catchq_first_layers_any_workspace_size(int n, int c, int h, int w, int co, int kh, int kw, int stride, int pad,
+                                                      const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad,
+                                                      int want_y, int sharing, size_t *bytes) {
+  return first_layers_bytes(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, want_y != 0, true, bytes);
+}
+
+CATCHQ_API int catchq_first_layers_any_nchw(const float *x, int n, int c, int h, int w, int x_position, float x_scale, int co, int kh,
+                                            int kw, int stride, int pad, const catchq_requant_stage_t *conv, int pool_k,
+                                            int pool_stride, int pool_pad, float *y, void *q, int sharing, void *workspace,
+                                            size_t workspace_bytes, catchq_stream_t stream) {
+  return first_layers(x, n, c, h, w, x_position, x_scale, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, true, y, q,
+                      sharing, workspace, workspace_bytes, stream);
 }
 
 // ---- 1x1 convolution + global average pooling ---------------------------------------------------------------------------

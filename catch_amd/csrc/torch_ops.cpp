@@ -292,6 +292,19 @@ bool first_layers_fuse_op(int64_t n, int64_t c, int64_t h, int64_t w, int64_t co
                                             &bytes) == CATCHQ_OK && bytes == 0;
 }
 
+bool first_layers_any_fuse_op(int64_t n, int64_t c, int64_t h, int64_t w, int64_t co, int64_t k, int64_t stride, int64_t pad,
+                          int64_t pool_k, int64_t pool_stride, int64_t pool_pad, bool want_y) {
+  float one = 1.0f;
+  catchq_requant_stage_t st;
+  std::memset(&st, 0, sizeof(st));
+  st.w = &one; st.chan_div = st.chan_rcp = st.bias = &one;  // presence only: nothing is dereferenced
+  st.act = CATCHQ_ACT_RELU;
+  size_t bytes = 1;
+  return catchq_first_layers_any_workspace_size((int)n, (int)c, (int)h, (int)w, (int)co, (int)k, (int)k, (int)stride, (int)pad, &st,
+                                            (int)pool_k, (int)pool_stride, (int)pool_pad, want_y, t_launch_sharing,
+                                            &bytes) == CATCHQ_OK && bytes == 0;
+}
+
 bool conv_avgpool_fuses_op(int64_t n, int64_t hw, int64_t ci, int64_t co) {
   float one = 1.0f;
   catchq_epilogue_t e;
@@ -765,12 +778,13 @@ Tensor qconv2d_expand_dw_op(const Tensor &qx, const Tensor &w1, int64_t exp2_1, 
   return q;
 }
 
-// The first layers in one call (catchq_first_layers_nchw): x [N,C,H,W] fp32, w [Co,kh,kw4,4] int8 (filter rows padded
-// with zero taps to a multiple of 4, and to 4 channels) -> the pooled int8 tensor [N,Hp,Wp,Co].
-Tensor qconv2d_first_layers_op(const Tensor &x, int64_t x_position, double x_scale, const Tensor &w, int64_t exp2,
-                               const c10::optional<Tensor> &chan_div, const c10::optional<Tensor> &bias, int64_t act,
-                               int64_t q_position, int64_t kw, int64_t stride, int64_t pad, int64_t pool_k,
-                               int64_t pool_stride, int64_t pool_pad) {
+// The first layers in one call (catchq_first_layers_nchw or _any_nchw): x [N,C,H,W] fp32, w [Co,kh,kw4,4] int8 (filter rows padded
+// with zero taps to a multiple of 4, and to 4 channels) -> the pooled int8 tensor [N,Hp,Wp,Co]; _any: images of any width, and with
+// want_y the pooled fp32 tensor in front of it.
+std::tuple<Tensor, Tensor> first_layers_call(const Tensor &x, int64_t x_position, double x_scale, const Tensor &w, int64_t exp2,
+                                             const c10::optional<Tensor> &chan_div, const c10::optional<Tensor> &bias, int64_t act,
+                                             int64_t q_position, int64_t kw, int64_t stride, int64_t pad, int64_t pool_k,
+                                             int64_t pool_stride, int64_t pool_pad, bool any, bool want_y) {
   c10::DeviceGuard guard(x.device());
   TORCH_CHECK(x.dim() == 4 && x.is_contiguous() && x.scalar_type() == at::kFloat,
               "qconv2d_first_layers expects a contiguous fp32 NCHW input");
@@ -783,23 +797,47 @@ Tensor qconv2d_first_layers_op(const Tensor &x, int64_t x_position, double x_sca
   StageKeep k;
   fill_stage(&k, w, exp2, chan_div, bias, act, q_position, co, "first-layer constants");
   size_t ws_bytes = 0;
-  check_status(catchq_first_layers_workspace_size((int)n, (int)c, (int)h, (int)wd, (int)co, (int)kh, (int)kw, (int)stride,
-                                                  (int)pad, &k.st, (int)pool_k, (int)pool_stride, (int)pool_pad,
-                                                  t_launch_sharing, &ws_bytes),
+  check_status(any ? catchq_first_layers_any_workspace_size((int)n, (int)c, (int)h, (int)wd, (int)co, (int)kh, (int)kw, (int)stride,
+                                                            (int)pad, &k.st, (int)pool_k, (int)pool_stride, (int)pool_pad, want_y,
+                                                            t_launch_sharing, &ws_bytes)
+                   : catchq_first_layers_workspace_size((int)n, (int)c, (int)h, (int)wd, (int)co, (int)kh, (int)kw, (int)stride,
+                                                        (int)pad, &k.st, (int)pool_k, (int)pool_stride, (int)pool_pad,
+                                                        t_launch_sharing, &ws_bytes),
                "torch_mlu::qconv2d_first_layers");
   const int hc = catchq_conv_out_size((int)h, (int)kh, (int)pad, (int)stride, 1);
   const int wc = catchq_conv_out_size((int)wd, (int)kw, (int)pad, (int)stride, 1);
   const int hp = catchq_conv_out_size(hc, (int)pool_k, (int)pool_pad, (int)pool_stride, 1);
   const int wp = catchq_conv_out_size(wc, (int)pool_k, (int)pool_pad, (int)pool_stride, 1);
-  Tensor q = at::empty({n, hp, wp, co}, x.options().dtype(at::kChar));
-  if (n == 0) return q;
+  Tensor q = at::empty({n, hp, wp, co}, x.options().dtype(at::kChar)), y;
+  if (want_y) y = at::empty({n, hp, wp, co}, x.options());
+  if (n == 0) return std::make_tuple(y, q);
   Tensor ws = at::empty({(int64_t)std::max<size_t>(ws_bytes, 16)}, x.options().dtype(at::kChar));
-  check_status(catchq_first_layers_nchw(x.data_ptr<float>(), (int)n, (int)c, (int)h, (int)wd, (int)x_position, (float)x_scale,
-                                        (int)co, (int)kh, (int)kw, (int)stride, (int)pad, &k.st, (int)pool_k,
-                                        (int)pool_stride, (int)pool_pad, q.data_ptr(), t_launch_sharing, ws.data_ptr(), ws_bytes,
-                                        current_stream()),
+  check_status(any ? catchq_first_layers_any_nchw(x.data_ptr<float>(), (int)n, (int)c, (int)h, (int)wd, (int)x_position, (float)x_scale,
+                                                  (int)co, (int)kh, (int)kw, (int)stride, (int)pad, &k.st, (int)pool_k,
+                                                  (int)pool_stride, (int)pool_pad, want_y ? y.data_ptr<float>() : nullptr,
+                                                  q.data_ptr(), t_launch_sharing, ws.data_ptr(), ws_bytes, current_stream())
+                   : catchq_first_layers_nchw(x.data_ptr<float>(), (int)n, (int)c, (int)h, (int)wd, (int)x_position, (float)x_scale,
+                                              (int)co, (int)kh, (int)kw, (int)stride, (int)pad, &k.st, (int)pool_k, (int)pool_stride,
+                                              (int)pool_pad, q.data_ptr(), t_launch_sharing, ws.data_ptr(), ws_bytes,
+                                              current_stream()),
                "torch_mlu::qconv2d_first_layers");
-  return q;
+  return std::make_tuple(y, q);
+}
+
+Tensor qconv2d_first_layers_op(const Tensor &x, int64_t x_position, double x_scale, const Tensor &w, int64_t exp2,
+                               const c10::optional<Tensor> &chan_div, const c10::optional<Tensor> &bias, int64_t act,
+                               int64_t q_position, int64_t kw, int64_t stride, int64_t pad, int64_t pool_k,
+                               int64_t pool_stride, int64_t pool_pad) {
+  return std::get<1>(first_layers_call(x, x_position, x_scale, w, exp2, chan_div, bias, act, q_position, kw, stride, pad, pool_k,
+                                       pool_stride, pool_pad, false, false));
+}
+
+std::tuple<Tensor, Tensor> qconv2d_first_layers_any_op(const Tensor &x, int64_t x_position, double x_scale, const Tensor &w, int64_t exp2,
+                                                       const c10::optional<Tensor> &chan_div, const c10::optional<Tensor> &bias,
+                                                       int64_t act, int64_t q_position, int64_t kw, int64_t stride, int64_t pad,
+                                                       int64_t pool_k, int64_t pool_stride, int64_t pool_pad, bool want_y) {
+  return first_layers_call(x, x_position, x_scale, w, exp2, chan_div, bias, act, q_position, kw, stride, pad, pool_k, pool_stride,
+                           pool_pad, true, want_y);
 }
 
 // A 1x1 convolution and the global average pooling behind it (catchq_conv1x1_avgpool_nhwc): qx [N,H,W,Ci] int8 NHWC,
@@ -1801,6 +1839,8 @@ TORCH_LIBRARY(torch_mlu, m) {
         "int q_bitwidth=0, int q_position=0, float q_scale=1.0) -> (Tensor, Tensor)");
   m.def("qconv2d_first_layers(Tensor x, int x_position, float x_scale, Tensor w, int exp2, Tensor? chan_div, Tensor? bias, "
         "int act, int q_position, int kw, int stride, int pad, int pool_k, int pool_stride, int pool_pad) -> Tensor");
+  m.def("qconv2d_first_layers_any(Tensor x, int x_position, float x_scale, Tensor w, int exp2, Tensor? chan_div, Tensor? bias, "
+        "int act, int q_position, int kw, int stride, int pad, int pool_k, int pool_stride, int pool_pad, bool want_y) -> (Tensor, Tensor)");
   m.def("qconv2d_avgpool(Tensor qx, Tensor qw, int exp2, Tensor? chan_div, Tensor? bias, Tensor? resid, int act, "
         "bool want_mean=True, int q_bitwidth=0, int q_position=0, float q_scale=1.0) -> (Tensor, Tensor)");
   m.def("qconv2d_chain(Tensor[] xs, Tensor[] ws, int[] strides, int[] exp2s, Tensor[] chan_divs, Tensor[] biases, "
@@ -1818,6 +1858,8 @@ TORCH_LIBRARY(torch_mlu, m) {
   m.def("inverted_residual_fuses(int n, int h, int w, int ci, int hid, int co, int stride) -> bool", &irb_fuses_op);
   m.def("first_layers_fuse(int n, int c, int h, int w, int co, int k, int stride, int pad, int pool_k, int pool_stride, "
         "int pool_pad) -> bool", &first_layers_fuse_op);
+  m.def("first_layers_any_fuse(int n, int c, int h, int w, int co, int k, int stride, int pad, int pool_k, int pool_stride, "
+        "int pool_pad, bool want_y) -> bool", &first_layers_any_fuse_op);
   m.def("conv3x3_packed_serves(int co, int ci) -> bool", &conv3x3_packed_serves_op);
   m.def("conv1x1_avgpool_fuses(int n, int hw, int ci, int co) -> bool", &conv_avgpool_fuses_op);
   m.def("clear_weight_cache() -> ()", &clear_cache_op);
@@ -1847,6 +1889,7 @@ TORCH_LIBRARY_IMPL(torch_mlu, CUDA, m) {  // ROCm tensors dispatch on the CUDA k
   m.impl("qconv2d_irb", &qconv2d_irb_op);
   m.impl("qconv2d_expand_dw", &qconv2d_expand_dw_op);
   m.impl("qconv2d_first_layers", &qconv2d_first_layers_op);
+  m.impl("qconv2d_first_layers_any", &qconv2d_first_layers_any_op);
   m.impl("qconv2d_avgpool", &qconv2d_avgpool_op);
   m.impl("qconv2d_chain", &qconv2d_chain_op);
   m.impl("qlinear", &qlinear_op);

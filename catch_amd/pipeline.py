@@ -272,8 +272,8 @@ class FusedNet(object):
         self._plan_blocks(fuse_expansions, fuse_blocks)
         self._expansion_names = set(x.name for x in self.expansion_of.values())
         # First layers: first_pool = the max-pooling layer behind the few-channel first convolution, when the pooled
-        # int8 tensor is all that anything reads of the two.
-        self.first_pool = None
+        # int8 tensor is all that anything reads of the two, or that and the pooled floats (first_floats).
+        self.first_pool, self.first_floats = None, False
         if fuse_first_layers and self.stem:
             l0 = self.layers[0]
             lq = self.q[l0.name]
@@ -284,10 +284,10 @@ class FusedNet(object):
                     and lq.chan_div is not None and lq.bias is not None and -64 <= lq.exp2 <= 64
                     and self.cdev["input"] == 4 and len(self.q_demand["input"]) == 1
                     and not ({l0.name, pool.name} & set(self.outputs))
-                    and not self.f_demand[l0.name] and not self.f_demand[pool.name]
+                    and self.f_demand[l0.name] == self.f_demand[pool.name]
                     and len(self.q_demand[pool.name]) == 1 and self.q_demand[pool.name][0][0] == 8
                     and self.q_demand[pool.name][0][2] == 1.0 and self.q_demand[l0.name] == self.q_demand[pool.name]):
-                self.first_pool = pool
+                self.first_pool, self.first_floats = pool, bool(self.f_demand[pool.name])
         # Global average pooling: pooled_conv[pooling layer name] = the 1x1 convolution in front of it, when nothing else
         # reads that convolution.
         self.pooled_conv = {}
@@ -428,12 +428,31 @@ class FusedNet(object):
         return bool(torch.ops.torch_mlu.expand_depthwise_fuses(n, h, w, self.cdev[x.src], self.cdev[x.name], dw.stride))
 
     def first_layers_fuse(self, n, c, h, w):
-        """whether quantizer, first convolution and pooling run as one launch on a contiguous fp32 batch [n, c, h, w]"""
-        if self.first_pool is None:
+        """whether quantizer, first convolution and pooling run as one launch of torch_mlu::qconv2d_first_layers on a contiguous
+        fp32 batch [n, c, h, w]"""
+        if self.first_pool is None or self.first_floats:
             return False
         l0, pool = self.layers[0], self.first_pool
         return bool(torch.ops.torch_mlu.first_layers_fuse(n, c, h, w, self.cdev[l0.name], l0.k, l0.stride, l0.pad, pool.k,
                                                           pool.stride, pool.pad))
+
+    def first_layers_run(self, n, c, h, w):
+        """whether they run as one launch at all (first_layers): that one or, for other widths and where the pooled floats are read
+        too, torch_mlu::qconv2d_first_layers_any"""
+        if self.first_pool is None:
+            return False
+        l0, pool = self.layers[0], self.first_pool
+        return bool(torch.ops.torch_mlu.first_layers_any_fuse(n, c, h, w, self.cdev[l0.name], l0.k, l0.stride, l0.pad, pool.k,
+                                                              pool.stride, pool.pad, self.first_floats))
+
+    def first_layers(self, x):
+        """the pooled tensors of a batch for which first_layers_run: (floats or None, int8)"""
+        l0, pool, d = self.layers[0], self.first_pool, self.q_demand["input"][0]
+        lq, ops = self.q[l0.name], torch.ops.torch_mlu
+        y, q = ops.qconv2d_first_layers_any(x, d[1], d[2], lq.qw, lq.exp2, lq.chan_div, lq.bias, _ACT_CODE[l0.act],
+                                            self.q_demand[pool.name][0][1], l0.k, l0.stride, l0.pad, pool.k, pool.stride, pool.pad,
+                                            self.first_floats)
+        return (y if self.first_floats else None), q
 
     def avgpool_fuses(self, gap, n, h, w):
         """whether the 1x1 convolution in front of the pooling layer `gap` runs inside the pooling's launch over n images
@@ -626,14 +645,13 @@ class FusedNet(object):
             timers.setdefault(name, []).append(ev)
             return ev
         first_fused = set()
-        if not tracing and x.dtype == torch.float32 and x.is_contiguous() and self.first_layers_fuse(*x.shape):
-            l0, pool, d = self.layers[0], self.first_pool, self.q_demand["input"][0]
-            lq, qd = self.q[l0.name], self.q_demand[self.first_pool.name][0]
+        if not tracing and x.dtype == torch.float32 and x.is_contiguous() and self.first_layers_run(*x.shape):
+            l0, pool = self.layers[0], self.first_pool
             tick(l0.name)
-            env[(pool.name,) + qd] = ops.qconv2d_first_layers(x, d[1], d[2], lq.qw, lq.exp2, lq.chan_div, lq.bias,
-                                                              _ACT_CODE[l0.act], qd[1], l0.k, l0.stride, l0.pad, pool.k,
-                                                              pool.stride, pool.pad)
+            y, env[(pool.name,) + self.q_demand[pool.name][0]] = self.first_layers(x)
             tick(l0.name)
+            if y is not None:
+                env[(pool.name, "f")] = y
             first_fused = {l0.name, pool.name}
         for d in self.q_demand["input"] if not first_fused else ():
             if self.stem:

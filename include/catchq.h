@@ -452,6 +452,16 @@ int catchq_first_layers_nchw(const float *x, int n, int c, int h, int w, int x_p
                              int pool_stride, int pool_pad, void *q, int sharing, void *workspace,
                              size_t workspace_bytes, catchq_stream_t stream);
 
+/* The same for images of any width (in one launch from 8 pixels on), and, where y is not NULL, with the pooled floats y [n, hp, wp, co]
+ * as well: the maximum of the convolution's floating output over each window, the shortcut of a residual block that reads the pooled
+ * tensor (q is their quantization, the same values as above).  want_y: whether there will be a y. */
+int catchq_first_layers_any_workspace_size(int n, int c, int h, int w, int co, int kh, int kw, int stride, int pad,
+                                           const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad, int want_y,
+                                           int sharing, size_t *bytes);
+int catchq_first_layers_any_nchw(const float *x, int n, int c, int h, int w, int x_position, float x_scale, int co, int kh, int kw,
+                                 int stride, int pad, const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad,
+                                 float *y, void *q, int sharing, void *workspace, size_t workspace_bytes, catchq_stream_t stream);
+
 /* A 1x1 convolution and the global average pooling behind it in one launch (the end of a classifier's feature
  * extractor).  In the reference: torch_mlu::conv2d (cnnl_conv2d, operators/cnnl/quantify_conv_forward.cpp:56-147), the
  * block's float add (cnnl_add, operators/cnnl/add.cpp) and ReLU (operators/cnnl/activation.cpp) where it has them,
