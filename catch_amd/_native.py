@@ -95,6 +95,7 @@ SIGNATURES = {
     "catchq_packed_conv3x3_size": (_I, [_I64, _I64, ctypes.POINTER(_SZ)]),
     "catchq_pack_conv3x3": (_I, [_P, _I64, _I64, _P, _P]),
     "catchq_conv3x3_packed": (_I, [_P, _P, _I, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P]),
+    "catchq_conv3x3_packed_s2": (_I, [_P, _P, _I, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P]),
     "catchq_conv3x3_i8_packed_takes": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(Epilogue)]),
     "catchq_conv3x3_i8_packed_any_takes": (_I, [_I, _I, _I, _I, _I, ctypes.POINTER(Epilogue)]),
     "catchq_conv3x3_i8_packed": (_I, [_P, _P, _I, _I, _I, _I, _I, ctypes.POINTER(Epilogue), _P]),

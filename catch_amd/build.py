@@ -19,7 +19,7 @@ INCLUDE = os.path.join(ROOT, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 
-KERNEL_SOURCES = ["conv3x3_halo_c512.hip", "conv3x3_halo_c512_s2.hip", "conv3x3_halo_c256.hip", "quantize.hip", "contract_direct.hip", "igemm_i8.hip", "small_i8.hip", "gemm_float_in.hip", "wide_i16.hip", "igemm_i8_dma_gemm.hip", "igemm_i8_dma_conv.hip", "igemm_i8_dual.hip", "igemm_i8_chain.hip", "conv3x3_halo_c64.hip", "conv3x3_halo_c128.hip", "conv3x3_halo_i8.hip", "igemm_a16_dma.hip", "pw_i8.hip", "dwconv_i8.hip", "dw_float.hip", "irb_i8.hip", "expand_dw_i8.hip", "stem_pool_i8.hip", "conv1x1_gap_i8.hip", "pool.hip", "diag.hip", "capi.hip", "ksplit.hip", "float_rows.hip", "digits_i16.hip", "concat.hip", "conv3x3_a16_packed.hip", "conv3x3_a16_walk.hip", "conv3x3_i8_walk.hip", "pw_a16_short.hip", "conv3x3_i8_packed.hip",
+KERNEL_SOURCES = ["conv3x3_halo_c512.hip", "conv3x3_halo_c512_s2.hip", "conv3x3_halo_c256.hip", "quantize.hip", "contract_direct.hip", "igemm_i8.hip", "small_i8.hip", "gemm_float_in.hip", "wide_i16.hip", "igemm_i8_dma_gemm.hip", "igemm_i8_dma_conv.hip", "igemm_i8_dual.hip", "igemm_i8_chain.hip", "conv3x3_halo_c64.hip", "conv3x3_halo_c128.hip", "conv3x3_halo_i8.hip", "igemm_a16_dma.hip", "pw_i8.hip", "dwconv_i8.hip", "dw_float.hip", "irb_i8.hip", "expand_dw_i8.hip", "stem_pool_i8.hip", "conv1x1_gap_i8.hip", "pool.hip", "diag.hip", "capi.hip", "ksplit.hip", "float_rows.hip", "digits_i16.hip", "concat.hip", "conv3x3_a16_packed.hip", "conv3x3_a16_packed_s2.hip", "conv3x3_a16_walk.hip", "conv3x3_i8_walk.hip", "pw_a16_short.hip", "conv3x3_i8_packed.hip",
                   "host_math.cpp"]
 
 # -packed-fp32-ops off: hipcc must not form v_pk_*_f32 from the fp32 epilogue math.

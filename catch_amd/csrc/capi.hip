@@ -52,6 +52,7 @@ int conv3x3_i8_packed(const void *x, const void *packed, int64_t N, int H, int W
 int64_t packed3x3_bytes(int64_t Co, int64_t Ci);
 int pack3x3(const void *w, void *packed, int64_t Co, int64_t Ci, hipStream_t s);
 int conv3x3_a16_packed(const void *x, const void *packed, int N, int H, int W, int Ci, int Co, const EpiDev &e, hipStream_t s);
+int conv3x3_a16_packed_s2(const void *x, const void *packed, int N, int H, int W, int Ci, int Co, const EpiDev &e, hipStream_t s);
 bool gemm_float_ok(int64_t in_pixels, int64_t M, int64_t N, int64_t K, int elem_bytes, int cus);
 int gemm_float(const void *x, bool half, int position, const void *w, int N_img, int H, int W, int Ci, int Co, int sh, int sw, int Ho,
                int Wo, const EpiDev &e, hipStream_t s);
@@ -485,8 +486,8 @@ CATCHQ_API int catchq_pack_conv3x3(const void *w, int64_t co, int64_t ci, void *
   return pack3x3(w, packed, co, ci, as_stream(stream));
 }
 
-CATCHQ_API int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
-                                     const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+static int conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co, bool stride_2,
+                          const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
   int st = check_epi(epilogue, true);
   if (st != CATCHQ_OK) return st;
   if (n < 0 || h <= 0 || w <= 0) return CATCHQ_ERR_ARG;
@@ -497,8 +498,20 @@ CATCHQ_API int catchq_conv3x3_packed(const void *x, const void *packed, int n, i
   if (!x || !packed) return CATCHQ_ERR_ARG;
   if (!aligned16(x) || !aligned16(packed)) return CATCHQ_ERR_UNSUPPORTED;
   if ((int64_t)h * w >= (1ll << 31) || (int64_t)n * h * w >= (1ll << 31)) return CATCHQ_ERR_UNSUPPORTED;
-  st = conv3x3_a16_packed(x, packed, n, h, w, ci, co, make_epi(epilogue, (int64_t)n * h * w * co), as_stream(stream));
+  const int64_t pixels = (int64_t)n * (stride_2 ? (int64_t)((h + 1) / 2) * ((w + 1) / 2) : (int64_t)h * w);
+  st = (stride_2 ? conv3x3_a16_packed_s2 : conv3x3_a16_packed)(x, packed, n, h, w, ci, co, make_epi(epilogue, pixels * co),
+                                                               as_stream(stream));
   return st < 0 ? CATCHQ_ERR_UNSUPPORTED : st;
+}
+
+CATCHQ_API int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                                     const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  return conv3x3_packed(x, packed, n, h, w, ci, co, false, epilogue, stream);
+}
+
+CATCHQ_API int catchq_conv3x3_packed_s2(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                                        const catchq_epilogue_t *epilogue, catchq_stream_t stream) {
+  return conv3x3_packed(x, packed, n, h, w, ci, co, true, epilogue, stream);
 }
 
 static int check_conv3x3_i8_packed(int n, int h, int w, int ci, int co, const catchq_epilogue_t *epilogue) {

@@ -45,4 +45,9 @@ inline bool conv3x3_a16_packed_filters(int64_t co, int64_t ci) {
   return ci % 64 == 0 && co % 4 == 0 && co * 4 >= (co + 255) / 256 * 256 * 3;
 }
 
+// ... at stride 2 (conv3x3_a16_packed_s2.hip, where both sides are measured): not a quarter of one column of blocks, nor 64 channels, whose
+// four steps do not repay the longer way to the first (108 x 114, 64 -> 768 14.0 us on the tiled kernel / 17.5, 4 x 64 x 58, 64 -> 1024
+// 17.1 / 18.4, two launches at a time)
+inline bool conv3x3_a16_packed_s2_filters(int64_t co, int64_t ci) { return conv3x3_a16_packed_filters(co, ci) && ci >= 128 && co >= 224; }
+
 }  // namespace catchq

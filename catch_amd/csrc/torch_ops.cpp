@@ -470,9 +470,10 @@ EpiOut qconv2d_impl(const Tensor &qx, const Tensor &qw, at::IntArrayRef padding,
                     catchq_packed_conv3x3_size(d.co, d.ci, &bytes) == CATCHQ_OK && packed->scalar_type() == at::kChar &&
                     packed->is_contiguous() && packed->numel() == (int64_t)bytes && packed->device() == qx.device(),
                 "qconv2d: the packed filters are not those of the weight");
-    if (qx.scalar_type() == at::kShort && d.pad_h == 1 && d.pad_w == 1 && d.stride_h == 1 && d.stride_w == 1 && d.dil_h == 1 &&
-        d.dil_w == 1) {
-      const int st = catchq_conv3x3_packed(qx.data_ptr(), packed->data_ptr(), d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
+    if (qx.scalar_type() == at::kShort && d.pad_h == 1 && d.pad_w == 1 && d.stride_h == d.stride_w && d.stride_h <= 2 &&
+        d.dil_h == 1 && d.dil_w == 1) {
+      const int st = (d.stride_h == 1 ? catchq_conv3x3_packed : catchq_conv3x3_packed_s2)(
+          qx.data_ptr(), packed->data_ptr(), d.n, d.h, d.w, d.ci, d.co, &e, current_stream());
       if (st != CATCHQ_ERR_UNSUPPORTED) {
         check_status(st, "torch_mlu::conv2d");
         return o;
@@ -579,10 +580,12 @@ std::tuple<Tensor, Tensor, Tensor> qconv2d_op(const Tensor &qx, const Tensor &qw
                                     q_position, q_scale, act_slope, resid_after_act), packed));
 }
 
-// Whether catchq_conv3x3_packed serves any call of such filters (by their channels: the rest of its rule is the image's)
-bool conv3x3_packed_serves_op(int64_t co, int64_t ci) {
+// Whether catchq_conv3x3_packed, or at stride 2 catchq_conv3x3_packed_s2, serves any call of such filters (by their channels: the rest
+// of the rules is the image's)
+bool conv3x3_packed_serves_op(int64_t co, int64_t ci, int64_t stride) {
   size_t bytes = 0;
-  return catchq_packed_conv3x3_size(co, ci, &bytes) == CATCHQ_OK && catchq::conv3x3_a16_packed_filters(co, ci);
+  if (catchq_packed_conv3x3_size(co, ci, &bytes) != CATCHQ_OK) return false;
+  return stride == 1 ? catchq::conv3x3_a16_packed_filters(co, ci) : stride == 2 && catchq::conv3x3_a16_packed_s2_filters(co, ci);
 }
 
 // qw [Co,3,3,Ci] int8 in the order that catchq_conv3x3_packed reads
@@ -1860,7 +1863,7 @@ TORCH_LIBRARY(torch_mlu, m) {
         "int pool_pad) -> bool", &first_layers_fuse_op);
   m.def("first_layers_any_fuse(int n, int c, int h, int w, int co, int k, int stride, int pad, int pool_k, int pool_stride, "
         "int pool_pad, bool want_y) -> bool", &first_layers_any_fuse_op);
-  m.def("conv3x3_packed_serves(int co, int ci) -> bool", &conv3x3_packed_serves_op);
+  m.def("conv3x3_packed_serves(int co, int ci, int stride=1) -> bool", &conv3x3_packed_serves_op);
   m.def("conv1x1_avgpool_fuses(int n, int hw, int ci, int co) -> bool", &conv_avgpool_fuses_op);
   m.def("clear_weight_cache() -> ()", &clear_cache_op);
   m.def("weight_cache_size() -> int", &cache_size_op);

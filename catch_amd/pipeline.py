@@ -161,8 +161,8 @@ def _decode(layer, sd, device, ci_dev, co_dev, fractional=False):
             q.chan_div = pad(q.chan_div, (0, co_dev - co), value=1.0)
     q.qw = qw.contiguous()
     q.packed = None
-    if ((layer.kind, layer.k, layer.stride, layer.pad, q.groups, q.bw_x, q.bw_w) == ("conv", 3, 1, 1, 1, 16, 8)
-            and torch.ops.torch_mlu.conv3x3_packed_serves(q.qw.shape[0], ci_dev)):
+    if ((layer.kind, layer.k, layer.pad, q.groups, q.bw_x, q.bw_w) == ("conv", 3, 1, 1, 16, 8)
+            and torch.ops.torch_mlu.conv3x3_packed_serves(q.qw.shape[0], ci_dev, layer.stride)):
         q.packed = torch.ops.torch_mlu.pack_conv3x3(q.qw)  # (the calls of a few blocks, or wide images, read the filters as they are)
     return q
 

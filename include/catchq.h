@@ -290,6 +290,10 @@ int catchq_packed_conv3x3_size(int64_t co, int64_t ci, size_t *bytes);
 int catchq_pack_conv3x3(const void *w, int64_t co, int64_t ci, void *packed, catchq_stream_t stream);
 int catchq_conv3x3_packed(const void *x, const void *packed, int n, int h, int w, int ci, int co,
                           const catchq_epilogue_t *epilogue, catchq_stream_t stream);
+/* at stride 2 (padding 1, images of even height and width; others CATCHQ_ERR_UNSUPPORTED), outputs [n, h / 2, w / 2, co], on the same
+ * filters */
+int catchq_conv3x3_packed_s2(const void *x, const void *packed, int n, int h, int w, int ci, int co,
+                             const catchq_epilogue_t *epilogue, catchq_stream_t stream);
 
 /* The same for int8 activations, ci a multiple of 32, and filters that catchq_pack_filters laid out from w [co, 9 * ci] (taps first).
  * *_takes answers CATCHQ_ERR_UNSUPPORTED without a launch where catchq_conv2d_nhwc serves the call better, or alone. */

@@ -77,6 +77,48 @@ def test_packed_conv3x3(n, h, w, ci, co, sharing, taken):
     assert torch.equal(acc.cpu().double(), want.permute(0, 2, 3, 1))  # integers below 2^53: exact
 
 
+# stride 2: the last widths of each number of passes over a block's four runs (63 and 127 output columns), images of one and of many
+# blocks, odd extents, which are not taken, and either side of the rule (channels, blocks for the units, long K)
+@pytest.mark.parametrize("n,h,w,ci,co,sharing,taken", [
+    (1, 2, 2, 128, 256, 256, True), (2, 6, 126, 128, 256, 256, True), (1, 4, 128, 128, 252, 256, True), (1, 4, 254, 128, 448, 256, True),
+    (1, 4, 256, 128, 256, 256, False), (5, 14, 10, 192, 512, 256, True), (3, 7, 8, 128, 256, 256, False), (1, 8, 9, 128, 256, 256, False),
+    (9, 2, 6, 128, 388, 256, True), (9, 2, 6, 128, 380, 256, False), (1, 8, 16, 128, 224, 256, True), (1, 8, 16, 128, 220, 256, False), (1, 8, 16, 128, 384, 256, True),
+    (1, 8, 16, 64, 256, 256, False),
+    # blocks of 32 pixels
+    (1, 20, 30, 128, 256, 40, True), (1, 4, 126, 128, 256, 40, True), (1, 4, 128, 192, 256, 40, True), (1, 2, 254, 128, 256, 40, True),
+    (7, 6, 6, 128, 512, 40, True), (1, 10, 10, 128, 256, 40, False), (1, 20, 30, 576, 256, 40, False), (1, 16, 48, 576, 256, 40, True),
+    (1, 26, 26, 128, 256, 1, False),
+])
+def test_packed_conv3x3_stride_2(n, h, w, ci, co, sharing, taken):
+    ops = torch.ops.torch_mlu
+    x, qw = _case(n, h, w, ci, co)
+    gen = torch.Generator().manual_seed(11)
+    other = qw[torch.randperm(co, generator=gen)].contiguous()  # which of the two were read shows in the outputs
+    x, qw, other = x.cuda(), qw.cuda(), other.cuda()
+    bias = torch.randn(co, generator=gen).cuda()
+    resid = torch.randn(n, (h + 1) // 2, (w + 1) // 2, co, generator=gen).cuda()
+    div = (torch.rand(co, generator=gen) + 0.5).cuda()
+    geometry = ([1, 1], [2, 2], [1, 1], 1)
+    calls = [  # chan_div, resid, act, want_y, y_half, want_acc, q_bitwidth, q_position, q_scale, slope, resid_after
+        (None, None, 3, False, False, False, 16, -8, 1.0, 0.1, False), (None, None, 3, True, False, False, 16, -8, 1.0, 0.1, False),
+        (None, None, 0, True, True, False, 0, 0, 1.0, 0.0, False), (None, resid, 3, True, False, False, 16, -8, 1.0, 0.1, True),
+        (div, resid, 1, True, False, True, 8, -2, 1.3, 0.0, False)]
+    packed, read = ops.pack_conv3x3(other), other if taken else qw
+    ops.set_launch_sharing(sharing)
+    try:
+        for d, r, act, *rest in calls:
+            got = ops.qconv2d(x, qw, -12, d, bias, r, *geometry, act, *rest, packed)
+            want = ops.qconv2d(x, read, -12, d, bias, r, *geometry, act, *rest)
+            assert len(_outputs(got)) == len(_outputs(want)) > 0
+            for a, b in zip(_outputs(got), _outputs(want)):
+                assert torch.equal(a, b)
+        acc = ops.qconv2d(x, qw, 0, None, None, None, *geometry, 0, False, False, True, 0, 0, 1.0, 0.0, False, packed)[2]
+    finally:
+        ops.set_launch_sharing(1)
+    want = torch.nn.functional.conv2d(x.cpu().double().permute(0, 3, 1, 2), read.cpu().double().permute(0, 3, 1, 2), stride=2, padding=1)
+    assert torch.equal(acc.cpu().double(), want.permute(0, 2, 3, 1))  # integers below 2^53: exact
+
+
 def test_packed_conv3x3_large_grid():
     """more than one round of blocks in either order of the grid"""
     ops = torch.ops.torch_mlu
@@ -87,6 +129,17 @@ def test_packed_conv3x3_large_grid():
         want = ops.qconv2d(x, qw, *args)[2]
         got = ops.qconv2d(x, qw, *args, 0, 0, 1.0, 0.0, False, ops.pack_conv3x3(qw))[2]
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("n,h,w,ci,co", [(16, 104, 104, 128, 256), (16, 26, 26, 512, 1024)])
+def test_packed_conv3x3_stride_2_large_grid(n, h, w, ci, co):
+    """likewise"""
+    ops = torch.ops.torch_mlu
+    x, qw = _case(n, h, w, ci, co)
+    x, qw = x.cuda(), qw.cuda()
+    args = (-12, None, None, None, [1, 1], [2, 2], [1, 1], 1, 0, False, False, True)
+    want = ops.qconv2d(x, qw, *args)[2]
+    assert torch.equal(ops.qconv2d(x, qw, *args, 0, 0, 1.0, 0.0, False, ops.pack_conv3x3(qw))[2], want)
 
 
 def test_packed_conv3x3_other_calls():

@@ -513,6 +513,13 @@ def test_plans_pack_filters_that_a_launch_can_read():
     assert serves(256, 64 * 14500) and not serves(256, 64 * 14600) and not serves(8, 1 << 23)
 
 
+def test_plans_pack_filters_of_stride_2_that_a_launch_can_read():
+    """... and from 128 channels in and 224 out on"""
+    serves = torch.ops.torch_mlu.conv3x3_packed_serves
+    assert serves(256, 128, 2) and serves(224, 128, 2) and not serves(220, 128, 2) and not serves(256, 64, 2) and not serves(256, 128, 3)
+    assert not serves(380, 128, 2) and serves(384, 128, 2) and serves(256, 128) == serves(256, 128, 1)
+
+
 def test_int16_layers_of_64_channels_at_stride_2(lib):
     """128 columns ask for two tiles of 8 x 4 outputs a unit; up to 96, and stride 1, for three quarters of one"""
     from catch_amd import _native
