@@ -47,6 +47,7 @@ constexpr int GC_YP = 36;  // dwords per pixel row of a wave's output tile
 template <int NW, int PG, bool RES>
 __global__ __launch_bounds__(64 * NW) void conv1x1_gap_kernel(const int8_t *__restrict__ X, const int8_t *__restrict__ Wt,
                                                              GapConvDev e, GapConvParams p) {
+  fetch_arguments<16 + sizeof(GapConvDev) + sizeof(GapConvParams)>();
   extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);

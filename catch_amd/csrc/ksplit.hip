@@ -40,6 +40,7 @@ enum { KW_DENSE = 0, KW_TAP = 1, KW_PIECE = 2 };
 // A16: int16 activations.  SLOTS: K steps a wave has in LDS or on the way there.
 template <int TM, int TN, int NW, int SLOTS, int WALK, bool A16>
 __global__ __launch_bounds__(64 * NW, TM * TN == 4 ? 2 : 0) void ksplit_kernel(KsplitParams p, EpiDev e) {
+  fetch_arguments<sizeof(KsplitParams) + sizeof(EpiDev)>();  // plans, us: six 208 x 208 ResNet-18 133.1 / 128.0, four 320 x 320 Darknet-53 773 / 765
   resolve_exp2(e);
   constexpr int BM = TM * 32, BN = TN * 32, KS = 64;  // values of K per step
   constexpr int ES = A16 ? 2 : 1, AROW = KS * ES;     // bytes per activation, of a tile row of them per step
