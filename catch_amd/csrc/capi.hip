@@ -981,7 +981,7 @@ static int first_layers(const float *x, int n, int c, int h, int w, int x_positi
   if (!x || !q || !conv->w) return CATCHQ_ERR_ARG;
   const bool floats = y != nullptr;
   if (first_layers_fusable(n, c, h, w, co, kh, kw, stride, pad, conv, pool_k, pool_stride, pool_pad, floats, any_width) &&
-      (w % 4 != 0 || aligned16(x)) && aligned16(conv->w) && aligned16(q) && (!floats || aligned16(y))) {
+      aligned16(conv->w) && aligned16(q) && (!floats || aligned16(y))) {  // (x on any float)
     const IrbStageDev s = {(const int8_t *)conv->w, conv->chan_div, conv->chan_rcp, conv->bias, conv->exp2,
                            -conv->q_position, conv->act == CATCHQ_ACT_RELU6 ? 1 : 0};
     const int st2 = stem_pool_i8(x, n, c, h, w, x_position, x_scale, s, co, y, q, as_stream(stream));

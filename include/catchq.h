@@ -445,9 +445,9 @@ int catchq_expand_depthwise_nhwc(const void *x, int n, int h, int w, int ci, int
  *   q  = max of q1 over windows pool_k x pool_k, stride pool_stride, padding pool_pad       int8 [n, hp, wp, co]
  * The values are those of catchq_quantize_nchw_to_nhwc_frame, catchq_conv2d_nhwc and catchq_maxpool_nhwc called one
  * after the other, bit for bit.  The fused kernel serves 7x7 / 2 / 3 convolutions of c <= 3 channels into 32, 64 or
- * 128 channels followed by 3x3 / 2 / 1 pooling, w % 4 == 0, x 16-byte aligned, the stage with chan_div, chan_rcp and
- * bias (-64 <= exp2 <= 64) (catchq_first_layers_workspace_size reports 0 then); anything else runs as the three
- * launches with qx and q1 in the caller's workspace.  `sharing` is the planning hint of catchq_epilogue_t::sharing. */
+ * 128 channels followed by 3x3 / 2 / 1 pooling, w % 4 == 0, the stage with chan_div, chan_rcp and bias
+ * (-64 <= exp2 <= 64) (catchq_first_layers_workspace_size reports 0 then; x on any float, the filters and q on 16
+ * bytes); anything else runs as the three launches with qx and q1 in the caller's workspace.  `sharing` is the planning hint of catchq_epilogue_t::sharing. */
 int catchq_first_layers_workspace_size(int n, int c, int h, int w, int co, int kh, int kw, int stride, int pad,
                                        const catchq_requant_stage_t *conv, int pool_k, int pool_stride, int pool_pad,
                                        int sharing, size_t *bytes);

@@ -61,3 +61,24 @@ def test_network_whose_first_block_adds_the_pooled_tensor(batch, h, w):
         assert torch.equal(replay(), want)
     static_in.copy_(x.flip(0))
     assert torch.equal(replay(), apart.forward(x.flip(0)))
+
+
+@pytest.mark.parametrize("name", ["resnet18", "resnet50"])  # with and without the pooled floats
+@pytest.mark.parametrize("w", [64, 66])
+def test_batches_that_start_on_any_element(name, w):
+    """a contiguous batch inside a larger buffer, on 4 bytes and no more"""
+    layers = nets.NETS[name]()
+    sd = pipeline.calibrate(nets.FloatNet(layers, seed=0, weight_std="he").eval(), torch.randn(2, 3, 64, 64), "int8", True)
+    fused = pipeline.FusedNet(layers, sd)
+    flat = torch.randn(2 * 3 * 64 * w + 4, device="cuda")
+    for first in (1, 2, 3):
+        x = flat[first:first + 2 * 3 * 64 * w].view(2, 3, 64, w)
+        assert x.is_contiguous() and x.data_ptr() % 16 and fused.first_layers_run(*x.shape)
+        assert torch.equal(fused.forward(x), fused.forward(x.clone()))
+    if w % 4 == 0:  # the op for these widths alone
+        r = np.random.default_rng(w)
+        wt = r.integers(-127, 128, (64, 7, 8, 4)).astype(np.int8)
+        wt[:, :, 7], wt[..., 3] = 0, 0
+        rest = (-5, 1.0, torch.from_numpy(wt).cuda(), -11, torch.ones(64, device="cuda"), torch.zeros(64, device="cuda"), 1, -3, 7, 2, 3, 3, 2, 1)
+        op = torch.ops.torch_mlu.qconv2d_first_layers
+        assert torch.equal(op(x, *rest), op(x.clone(), *rest))
