@@ -13,7 +13,8 @@
 //               row, two pixels of four planes each), quantized and stored as [pixel][channel] in LDS, the padding as zeros.  The pixel's stride
 //               is odd in units of four channels, so that a wave's stores and reads go over all banks.
 //   2  stencil  a lane owns four channels of PH x PW outputs.  8 bits: dw3x3.h.  16 bits: nine products of up to 2^30 do not fit 32 bits,
-//               and 64-bit integer products are a quarter of the rate of doubles, which hold the sum exactly.
+//               and 64-bit integer products are a quarter of the rate of doubles, which hold the sum exactly.  It starts at +0.0: a sum
+//               of zeros under negative filters is the integer's +0.0.
 // Channels beyond the last group of four: the group is read from where it lies whole and shifted, outputs are stored one by one.
 #include "dw3x3.h"
 #include "igemm_common.h"
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(256) void dw_float_kernel(const void *__restrict__ 
               if (r < 0 || r > 2 || q < 0 || q > 2) continue;
 #pragma unroll
               for (int j = 0; j < 4; ++j)
-                acc[py][px][j] = r == 0 && q == 0 ? xv[j] * wd[0][j] : __builtin_fma(xv[j], wd[r * 3 + q][j], acc[py][px][j]);
+                acc[py][px][j] = __builtin_fma(xv[j], wd[r * 3 + q][j], r == 0 && q == 0 ? 0.0 : acc[py][px][j]);  // (0 x -1 + 0: +0)
             }
         }
 #pragma unroll

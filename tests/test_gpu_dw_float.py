@@ -1,4 +1,6 @@
 """3x3 depthwise convolutions called one by one on floating activations (one launch, dw_float.hip) against the oracle, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -67,3 +69,34 @@ def test_any_element_of_a_buffer(c, dtype):
     for xd in (flat.view(2, 10, 9, c).permute(0, 3, 1, 2), flat.view(2, c, 10, 9)):
         ref = torch.ops.torch_mlu.conv2d(xd.clone(memory_format=torch.preserve_format), *rest)
         assert torch.equal(torch.ops.torch_mlu.conv2d(xd, *rest), ref)
+
+
+@pytest.mark.parametrize("bits", [8, 16])
+@pytest.mark.parametrize("half,steps", [(False, 0), (True, 0), (True, 1)])  # (rounded step by step: the epilogue that keeps a sum's sign)
+@pytest.mark.parametrize("nchw", [0, 1])
+def test_sums_of_nothing_are_positive_zeros(nchw, half, steps, bits):
+    """windows of zeros under filters that are all negative, no bias: the integer sum is 0, which converts to +0.0, so the bits are those
+    of the quantizer and the convolution on its integers"""
+    from catch_amd import _native
+    lib, p, check = _native.kernel_lib(), lambda t: t.data_ptr(), _native.check
+    stream = torch.cuda.current_stream().cuda_stream
+    n, h, w, c = 2, 9, 10, 36
+    x = torch.zeros(n, h, w, c, dtype=torch.float16 if half else torch.float32, device="cuda")
+    x[1, 4, 4] = 1.0
+    wt = torch.full((c, 3, 3, 1), -100, dtype=torch.int8 if bits == 8 else torch.int16, device="cuda")
+    div = torch.full((c,), 1.5, device="cuda")
+    rcp = 1.0 / div
+    desc = _native.ConvDesc(n, h, w, c, c, 3, 3, 1, 1, 1, 1, 1, 1, c)
+    y = [torch.full_like(x, 7.0) for _ in range(2)]
+    e = _native.Epilogue()
+    e.exp2, e.chan_div, e.chan_rcp, e.y_dtype, e.half_steps = -9, p(div), p(rcp), int(half), steps
+    e.y = p(y[0])
+    qx = torch.empty(x.shape, dtype=wt.dtype, device="cuda")
+    check(lib.catchq_quantize(p(x), int(half), p(qx), bits, x.numel(), -4, 1.0, stream))
+    check(lib.catchq_conv2d_nhwc(p(qx), bits, p(wt), bits, ctypes.byref(desc), ctypes.byref(e), stream))
+    e.y = p(y[1])
+    xd = x.permute(0, 3, 1, 2).contiguous() if nchw else x
+    check(lib.catchq_float_depthwise(p(xd), int(half), -4, nchw, p(wt), bits, ctypes.byref(desc), ctypes.byref(e), stream))
+    assert (y[0][1, 3:6, 3:6] < 0).all() and not torch.signbit(y[0][0]).any()
+    ints = torch.int16 if half else torch.int32
+    assert torch.equal(y[1].view(ints), y[0].view(ints))
