@@ -166,8 +166,9 @@ __global__ __launch_bounds__(256, 2) void gemm_digits_kernel(const int8_t *__res
   else L = epi_lane_setup<S>(n, n < p.N, e);
   const v4i col_sum = *reinterpret_cast<const v4i *>(col_sums + n0 + cg * 4);
   for (int slab = 0; slab < slabs; ++slab) {
-    // this wave's pieces of the slab have landed: what was sent for behind them are weights of this wave
-    if (slab == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // this wave's pieces of the slab have landed: what was sent for behind them are weights of this wave.  (Of a wave without columns
+    // nothing uses those: whether they were sent for at all is the compiler's choice, so it waits for everything.)
+    if (slab == 0 || (CONV && !columns)) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * 4) : "memory");
     __syncthreads();  // everyone's; and nobody reads the other half of the buffer any more
     if (slab + 1 < slabs) issue_a(slab + 1);

@@ -67,3 +67,46 @@ def test_largest_sums(sx, sw):
     w = torch.full((128, 640, 5, 5), float(sw), device="cuda")
     b = torch.zeros(128, device="cuda")
     _calls(x, w, b, (5, 5), 1, 1, 2)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("nchw", [0, 1])
+@pytest.mark.parametrize("n,ci,h,w,co,k,stride", [
+    (40, 70, 40, 41, 20, 3, 1),    # the second of two waves side by side has no columns
+    (17, 72, 33, 35, 96, 5, 1),    # the fourth of four
+    (24, 64, 41, 40, 130, 3, 2),   # three of the second run's four
+    (8, 200, 60, 60, 257, 3, 1),   # three of the third run's, blocks of many slabs
+])
+def test_waves_without_columns(n, ci, h, w, co, k, stride, nchw, half):
+    """the entry points called by themselves, against the quantizer and the convolution on its integers, bit for bit"""
+    lib, p, check = _native.kernel_lib(), lambda t: t.data_ptr(), _native.check
+    stream = torch.cuda.current_stream().cuda_stream
+    gen = torch.Generator(device="cuda").manual_seed(co)
+    cd, ho, wo = (ci + 7) // 8 * 8, (h - 1) // stride + 1, (w - 1) // stride + 1
+    x = torch.randn(n, h, w, ci, generator=gen, device="cuda").to(torch.float16 if half else torch.float32)
+    wt = torch.randint(-32768, 32768, (co, k, k, cd), generator=gen, device="cuda", dtype=torch.int16)
+    wt[..., ci:] = 0
+    bias = torch.randn(co, generator=gen, device="cuda")
+    desc = _native.ConvDesc(n, h, w, cd, co, k, k, k // 2, k // 2, stride, stride, 1, 1, 1)
+    e = _native.Epilogue()
+    e.exp2, e.bias, e.y_dtype = -28, p(bias), int(half)
+    y = [torch.empty(n, ho, wo, co, dtype=x.dtype, device="cuda") for _ in range(2)]
+    qx = torch.empty(n, h, w, cd, dtype=torch.int16, device="cuda")
+    xn = x.permute(0, 3, 1, 2).contiguous()
+    check(lib.catchq_quantize_nchw_to_nhwc(p(xn), int(half), p(qx), 16, n, ci, h, w, cd, -13, 1.0, stream))
+    e.y = p(y[0])
+    check(lib.catchq_conv2d_nhwc(p(qx), 16, p(wt), 16, ctypes.byref(desc), ctypes.byref(e), stream))
+    size = ctypes.c_size_t(0)
+    check(lib.catchq_packed_conv_digits_size(co, k * k, cd, ctypes.byref(size)))
+    packed = torch.empty(size.value, dtype=torch.int8, device="cuda")
+    check(lib.catchq_pack_conv_digits(p(wt), co, k * k, cd, p(packed), stream))
+    check(lib.catchq_float_conv2d_digits_workspace_size(ctypes.byref(desc), ctypes.byref(e), ctypes.byref(size)))
+    ws = torch.empty(size.value, dtype=torch.int8, device="cuda")
+    e.y = p(y[1])
+    ints = torch.int16 if half else torch.int32
+    for _ in range(3):
+        y[1].fill_(7.0)
+        check(lib.catchq_float_conv2d_digits(p(xn if nchw else x), int(half), -13, ci, nchw, p(packed), ctypes.byref(desc), ctypes.byref(e),
+                                             p(ws), ws.numel(), stream))
+        assert torch.equal(y[1].view(ints), y[0].view(ints))
+    assert y[0].float().std() > 0.5
