@@ -357,10 +357,9 @@ static int digit_epilogue(int N, const EpiDev &e) {
   return epi == EPI_Y32 || epi == EPI_Y16 ? epi : 0;
 }
 
-template <int WN, int SUB, class Conv>
-static int launch_digits(const int8_t *a, const int8_t *b, const int *sums, DigitParams p, const Conv &c, const EpiDev &e, hipStream_t s) {
-  constexpr int LDS_BYTES = 64 * 1024, BM = 64 * (4 / WN);  // two slabs; behind the loop 4 x (64 + 3 x 32 x 36) sums
-  static_assert(2 * BM / 32 * SUB * 2048 <= LDS_BYTES);
+// The tiles of blocks of WN waves side by side, and the dies' share of them; the blocks of the launch.
+static int64_t digit_tiles(DigitParams &p, int WN) {
+  const int BM = 64 * (4 / WN);
   p.tiles_m = (int)((p.M + BM - 1) / BM);
   p.tiles_n = ((p.N + 31) / 32 + WN - 1) / WN;
   int64_t best = -1;
@@ -371,7 +370,15 @@ static int launch_digits(const int8_t *a, const int8_t *b, const int *sums, Digi
     const int64_t cost = rm * rn * 64 + rm * 64 + rn * 128;
     if (best < 0 || cost < best) best = cost, p.die_cols = cols, p.rect_m = (int)rm, p.rect_n = (int)rn;
   }
-  const unsigned blocks = (unsigned)(8 * p.rect_m * p.rect_n);
+  return 8ll * p.rect_m * p.rect_n;
+}
+static int conv_digits_side(int Co) { return Co <= 64 ? 2 : 4; }  // waves side by side
+
+template <int WN, int SUB, class Conv>
+static int launch_digits(const int8_t *a, const int8_t *b, const int *sums, DigitParams p, const Conv &c, const EpiDev &e, hipStream_t s) {
+  constexpr int LDS_BYTES = 64 * 1024;  // two slabs; behind the loop 4 x (64 + 3 x 32 x 36) sums
+  static_assert(2 * 64 * (4 / WN) / 32 * SUB * 2048 <= LDS_BYTES);
+  const unsigned blocks = (unsigned)digit_tiles(p, WN);
   const bool whole = pick_epilogue(p.N, e) == EPI_Y32 || pick_epilogue(p.N, e) == EPI_Y16;
   auto kern = digit_epilogue(p.N, e) == EPI_Y32
                   ? (whole ? gemm_digits_kernel<EPI_Y32, false, WN, SUB, Conv> : gemm_digits_kernel<EPI_Y32, true, WN, SUB, Conv>)
@@ -462,6 +469,10 @@ int64_t conv_digits_bytes(int N, int H, int W, int Ci, int Co, int kh, int kw, i
   const int64_t bytes = (pixels + 1) * c32 * 64;
   if (taps > 25 || conv_digit_steps(taps, Ci) * 32 >= (1 << 14) || M >= (1ll << 31) - 128 || bytes >= (1ll << 31)) return 0;
   if (packed_digits_bytes(Co, taps, Ci) >= (1ll << 31) || e.resid || e.q || e.acc_out || !digit_epilogue(Co, e)) return 0;
+  DigitParams tiles = {};
+  tiles.M = M;
+  tiles.N = Co;
+  if (digit_tiles(tiles, conv_digits_side(Co)) >= (1 << 24)) return 0;  // (a launch has less than 2^32 lanes)
   return conv_digits_sizes(M, Co, Ci, taps, e.cus) ? bytes : 0;
 }
 
@@ -499,7 +510,7 @@ int conv_digits(const void *x, bool half, int position, int x_ci, bool apart, co
   magic(kw, &c.magic_kw, &c.mask_kw);
   const int8_t *const b = static_cast<const int8_t *>(packed);
   const int *const sums = reinterpret_cast<const int *>(b + p.b_bytes);
-  return Co <= 64 ? launch_digits<2, 4>(a, b, sums, p, c, e, s) : launch_digits<4, 8>(a, b, sums, p, c, e, s);
+  return conv_digits_side(Co) == 2 ? launch_digits<2, 4>(a, b, sums, p, c, e, s) : launch_digits<4, 8>(a, b, sums, p, c, e, s);
 }
 
 }  // namespace catchq

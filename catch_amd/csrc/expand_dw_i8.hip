@@ -195,7 +195,7 @@ static bool expand_dw_tile(int N, int H, int W, int Cin, int hid, int S, int cus
   const int pca = cols < W + 2 ? W + 2 : cols;
   const int64_t lds = (int64_t)(rows < in_rows ? in_rows : rows) * pca * (kc * 32 + 4);
   const int64_t blocks = (int64_t)N * bands * chunks;
-  if (lds > 64 * 1024 || blocks > 0x7fffffff) return false;
+  if (lds > 64 * 1024 || blocks >= (1 << 24)) return false;  // (a launch has less than 2^32 lanes)
   // Both phases are vector arithmetic: a 32 x 32 piece of the expansion counts as 250 instructions of a wave, 64 lanes' stencils as
   // 600, and a block as 400 more.  The cost is what the busiest unit's SIMDs have to do and, once for every generation of co-resident
   // blocks, a block's start (400) and its own chain.  On 56 shapes (MobileNetV2's at 192 x 192 and 224 x 224, 1 to 64 images) the tile it

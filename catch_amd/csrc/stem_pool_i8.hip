@@ -395,13 +395,12 @@ static bool stem_pool_plan(int N, int C, int H, int W, int Co, bool floats, bool
   if (!best) return false;
   p.PR = best;
   p.bands = (p.Hp + best - 1) / best;
-  if ((int64_t)N * p.bands > 0x7fffffff) return false;
   p.off_in = up(Co * 12);
   p.off_tile = p.off_in + up((4 * best + SP_KH) * p.in_pitch);
   lds_bytes = lds_of(best);
   waves = lds_bytes > 80 * 1024 ? 16 : 8;
   if (const char *t = tuning_env("CATCHQ_STEM_NW")) waves = atoi(t) == 16 ? 16 : 8;
-  return true;
+  return (int64_t)N * p.bands * 64 * waves < (1ll << 32);  // (lanes of a launch)
 }
 
 bool stem_pool_i8_ok(int N, int C, int H, int W, int Co, bool floats, bool any_width) {

@@ -520,6 +520,33 @@ def test_plans_pack_filters_of_stride_2_that_a_launch_can_read():
     assert not serves(380, 128, 2) and serves(384, 128, 2) and serves(256, 128) == serves(256, 128, 1)
 
 
+def test_launches_of_2_32_lanes_are_left_to_other_routes(lib):
+    """a launch has less than 2^32 lanes: kernels of a block for each part of an image answer for smaller batches alone"""
+    from catch_amd import _native
+    one = ctypes.pointer(ctypes.c_float(1.0))
+    stage = _native.RequantStage()
+    stage.w = stage.chan_div = stage.chan_rcp = stage.bias = ctypes.cast(one, ctypes.c_void_p)  # (presence only)
+    stage.act = 1
+    size = ctypes.c_size_t(1)
+
+    def expansion(n):  # a block of 256 lanes an image
+        assert lib.catchq_expand_depthwise_workspace_size(n, 2, 2, 16, 16, 1, ctypes.byref(stage), ctypes.byref(stage), 1, ctypes.byref(size)) == 0
+        return size.value
+    assert expansion((1 << 24) - 1) == 0 and expansion(1 << 24) == (1 << 24) * 2 * 2 * 16
+
+    def first_layers(n, want_y):  # 512 lanes an image
+        assert lib.catchq_first_layers_any_workspace_size(n, 1, 7, 8, 32, 7, 7, 2, 3, ctypes.byref(stage), 3, 2, 1, want_y, 1, ctypes.byref(size)) == 0
+        return size.value
+    for want_y in (0, 1):
+        assert first_layers((1 << 23) - 1, want_y) == 0 and first_layers(1 << 23, want_y) > 0
+
+    def digits(n):  # images of one pixel, each 61 x 61 outputs behind the padding: a block of 256 lanes for 64 of them
+        d = _native.ConvDesc(n, 1, 1, 32, 128, 3, 3, 31, 31, 1, 1, 1, 1, 1)
+        return lib.catchq_float_conv2d_digits_workspace_size(ctypes.byref(d), ctypes.byref(_native.Epilogue(y=16)), ctypes.byref(size))
+    most = ((1 << 24) - 8) * 64 // 3721  # (the dies share tiles in eights)
+    assert digits(most) == 0 and digits(most + 1) == 6  # CATCHQ_ERR_UNSUPPORTED
+
+
 def test_int16_layers_of_64_channels_at_stride_2(lib):
     """128 columns ask for two tiles of 8 x 4 outputs a unit; up to 96, and stride 1, for three quarters of one"""
     from catch_amd import _native
