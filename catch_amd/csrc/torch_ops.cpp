@@ -74,6 +74,15 @@ Tensor device_empty_like(const Tensor &dense, at::ScalarType type) {
   return Tensor(at::detail::empty_strided_cuda(dense.sizes(), dense.strides(), type, dense.device()));
 }
 
+// Scratch memory of a route that another one, of less of it, can stand in for; undefined: there is not that much.
+Tensor device_scratch(int64_t bytes, at::Device device) {
+  try {
+    return device_empty({bytes}, at::kChar, device);
+  } catch (const c10::OutOfMemoryError &) {
+    return Tensor();
+  }
+}
+
 bool has_bias(const Tensor &b) { return b.defined() && b.numel() != 0 && b.dim() != 0; }
 
 // ------------------------------------------------------------------------------------------------
@@ -1203,12 +1212,8 @@ const void *packed_weight(Prepared &p, Takes takes) {
     if ((digits ? (taps > 1 ? catchq_packed_conv_digits_size(n, taps, k / taps, &bytes) : catchq_packed_digits_size(n, k, &bytes))
                 : catchq_packed_filters_size(n, k, &bytes)) != CATCHQ_OK)
       return nullptr;
-    Tensor packed;
-    try {
-      packed = device_empty({(int64_t)bytes}, at::kChar, p.qw.device());
-    } catch (const c10::OutOfMemoryError &) {
-      return nullptr;  // (the other routes need no second copy)
-    }
+    Tensor packed = device_scratch((int64_t)bytes, p.qw.device());
+    if (!packed.defined()) return nullptr;  // (the other routes need no second copy)
     check_status(digits ? (taps > 1 ? catchq_pack_conv_digits(p.qw.data_ptr(), n, taps, k / taps, packed.data_ptr(), current_stream())
                                     : catchq_pack_digits(p.qw.data_ptr(), n, k, k, packed.data_ptr(), current_stream()))
                         : catchq_pack_filters(p.qw.data_ptr(), n, k, packed.data_ptr(), current_stream()),
@@ -1258,7 +1263,8 @@ bool linear_digits(const void *x, int dt, Prepared &prep, int64_t m, int64_t n, 
   if (st == CATCHQ_OK) {
     const void *packed = packed_weight(prep, [] { return true; });
     if (!packed) return false;
-    Tensor digits = device_empty({(int64_t)bytes}, at::kChar, device);
+    Tensor digits = device_scratch((int64_t)bytes, device);
+    if (!digits.defined()) return false;  // (rows padded to 128 values: up to four times the other route's)
     st = catchq_float_linear_digits(x, dt, prep.pos_x, packed, m, n, k, &e, digits.data_ptr(), bytes, current_stream());
   }
   if (st == CATCHQ_ERR_UNSUPPORTED) return false;
@@ -1406,7 +1412,8 @@ bool conv_digits(const Tensor &x, Prepared &prep, const catchq_conv_desc_t &d, c
   if (st == CATCHQ_OK) {
     const void *packed = packed_weight(prep, [] { return true; });
     if (!packed) return false;
-    Tensor digits = device_empty({(int64_t)bytes}, at::kChar, x.device());
+    Tensor digits = device_scratch((int64_t)bytes, x.device());
+    if (!digits.defined()) return false;  // (pixels padded to 32 channels: up to four times the other route's)
     st = catchq_float_conv2d_digits(x.data_ptr(), x.scalar_type() == at::kHalf ? CATCHQ_F16 : CATCHQ_F32, prep.pos_x, (int)x.size(1),
                                     rows ? 0 : 1, packed, &d, &e, digits.data_ptr(), bytes, current_stream());
   }

@@ -110,3 +110,32 @@ def test_waves_without_columns(n, ci, h, w, co, k, stride, nchw, half):
                                              p(ws), ws.numel(), stream))
         assert torch.equal(y[1].view(ints), y[0].view(ints))
     assert y[0].float().std() > 0.5
+
+
+@pytest.mark.parametrize("linear", [False, True])
+def test_scratch_that_does_not_fit(linear):
+    """digits are up to four times the integers as they lie: where only those fit, the route without digits serves the call"""
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    if linear:
+        x, w = torch.randn(1 << 20, 32, generator=gen, device="cuda").half(), torch.randn(32, 32, generator=gen, device="cuda").half()
+    else:
+        x, w = torch.randn(64, 8, 256, 256, generator=gen, device="cuda"), torch.randn(16, 8, 3, 3, generator=gen, device="cuda")
+    b = torch.randn(w.shape[0], generator=gen, device="cuda").to(x.dtype)
+    scale = torch.cat([32767.0 / t.float().abs().max().reshape(1) for t in (x, w)])
+    mode = torch.tensor([2], dtype=torch.int32, device="cuda")
+    ops = torch.ops.torch_mlu
+    run = lambda: ops.linear(x, w, b, scale, mode) if linear else ops.conv2d(x, w, b, [1, 1], [1, 1], [1, 1], 1, scale, mode)
+    want = run()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    run()  # (its digits, if it is the one that lays the weight out, and what it leaves in the cache)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.mem_get_info()[1]
+    room = want.numel() * want.element_size() + x.numel() * 2 + (32 << 20)  # an output, the integers (64 MiB) and some; digits are 256 MiB
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + room) / total)
+        for _ in range(3):
+            assert torch.equal(run(), want)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
