@@ -2,6 +2,7 @@
 the route takes, so the first call of a layer runs the kernel for operands as they lie and the next ones this one: exact sums, the same
 bits."""
 import ctypes
+import gc
 import math
 
 import pytest
@@ -23,18 +24,35 @@ def _served(x, w, k, stride, dil):
     return _native.kernel_lib().catchq_float_conv2d_digits_workspace_size(ctypes.byref(desc), ctypes.byref(e), ctypes.byref(bytes_)) == 0
 
 
-def _calls(x, w, b, k, stride, dil, mode):
+def _held():
+    torch.cuda.synchronize()
+    return torch.cuda.memory_allocated()
+
+
+def _calls(x, w, b, k, stride, dil, mode, scale=None):
+    """the first call's output; the next ones ran through the digits: they laid the weight out and keep that"""
     assert _served(x, w, k, stride, dil)
-    scale_x = 32767.0 / x.float()[torch.isfinite(x)].abs().max().reshape(1)
-    wf = w.float().reshape(w.shape[0], -1).abs()
-    scale = torch.cat([scale_x, torch.zeros_like(scale_x), 32767.0 / wf.amax(1)]) if mode == 4 else torch.cat([scale_x, 32767.0 / wf.max().reshape(1)])
+    if scale is None:
+        scale_x = 32767.0 / x.float()[torch.isfinite(x)].abs().max().reshape(1)
+        wf = w.float().reshape(w.shape[0], -1).abs()
+        scale = torch.cat([scale_x, torch.zeros_like(scale_x), 32767.0 / wf.amax(1)]) if mode == 4 else torch.cat([scale_x, 32767.0 / wf.max().reshape(1)])
+        del scale_x, wf
     qm = torch.tensor([mode], dtype=torch.int32, device="cuda")
     run = lambda: torch.ops.torch_mlu.conv2d(x, w, b, [dil * (k[0] // 2), dil * (k[1] // 2)], [stride, stride], [dil, dil], 1, scale, qm)
+    size = ctypes.c_size_t(0)
+    _native.check(_native.kernel_lib().catchq_packed_conv_digits_size(w.shape[0], k[0] * k[1], (x.shape[1] + 7) // 8 * 8, ctypes.byref(size)))
+    gc.collect()
+    torch.ops.torch_mlu.clear_weight_cache()
     first = run()
+    held = [_held()]
     for _ in range(3):
         again = run()
         assert again.stride() == first.stride() and torch.equal(first.view(torch.int32 if first.dtype == torch.float32 else torch.int16),
                                                                 again.view(torch.int32 if first.dtype == torch.float32 else torch.int16))
+        del again
+        held.append(_held())
+    assert size.value <= held[1] - held[0] < size.value + (1 << 21) and held[3] == held[2] == held[1]
+    return first
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
@@ -66,7 +84,12 @@ def test_largest_sums(sx, sw):
     x = torch.full((13, 640, 20, 40), float(sx), device="cuda")
     w = torch.full((128, 640, 5, 5), float(sw), device="cuda")
     b = torch.zeros(128, device="cuda")
-    _calls(x, w, b, (5, 5), 1, 1, 2)
+    y = _calls(x, w, b, (5, 5), 1, 1, 2, torch.full((2,), 32767.0 / 0.999, device="cuda"))  # (steps of 2^-15: one saturates)
+    qx, qw = 32767 if sx > 0 else -32768, 32767 if sw > 0 else -32768
+    taps = lambda n: torch.tensor([min(i + 2, n - 1) - max(i - 2, 0) + 1 for i in range(n)])
+    sums = (taps(20)[:, None] * taps(40)) * (640 * qx * qw)
+    assert sums.abs().max() == 16000 * abs(qx * qw)
+    assert torch.equal(y.cpu(), (sums.float() * 2.0 ** -30).expand(y.shape))
 
 
 @pytest.mark.parametrize("half", [False, True])
