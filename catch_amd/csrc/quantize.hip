@@ -106,10 +106,14 @@ static int launch_quantize(const void *x, void *q, int64_t n, int pos, float sca
   constexpr int VEC = 16 / sizeof(TIn);
   if (aligned16(x) && aligned16(q)) {
     // one vector per lane up to the grid's limit (4.2 M fp32 values), whose lanes walk on from there: a lane's loads follow
-    // each other.  From four times that many on two vectors a lane, and no walking (us, 51 M fp32 values to int8 42.8 / 41.0, to int16
-    // 49.3 / 46.4, fp16 27.2 / 25.6; 12 M fp16 8.4 / 8.6; four a lane 43.1).
+    // each other.  On large tensors two vectors a lane, and no walking (us, 51 M fp32 values to int8 42.8 / 41.0, to int16
+    // 49.3 / 46.4, fp16 27.2 / 25.6; 12 M fp16 8.4 / 8.6; four a lane 43.1).  Floats that the launch in front has just read, part of
+    // which the Infinity Cache still holds, come faster to lanes that walk: range, quantization on the device and dequantization of
+    // fp32, walking / two a lane, to int8 18 M 44.0 / 46.7, 30 M 69.5 / 71.1, 42 M 94.1 / 94.4, 48 M 107.4 / 106.8, to int16 47 M 124.3 /
+    // 125.7, 56 M 147.2 / 154.4, 60 M 164.2 / 165.0, 70 M 197.1 / 191.4; of halfs 0.97 to 1.00 times as long from 34 M on.
     const int64_t nvec = n / VEC, blocks = (nvec + 2 * kThreads - 1) / (2 * kThreads);
-    if (nvec >= 4ll * kMaxBlocks * kThreads && blocks < (1 << 24))
+    const int64_t two = sizeof(TIn) == 2 ? 4ll * kMaxBlocks * kThreads : BW == 8 ? 11 << 20 : 1 << 24;
+    if (nvec >= two && blocks < (1 << 24))
       quantize_vec_kernel<TIn, BW, 2><<<(unsigned)blocks, kThreads, 0, s>>>((const TIn *)x, (TQ *)q, n, pos, scale, pos_dev, scale_dev);
     else
       quantize_vec_kernel<TIn, BW, 1><<<grid_for(nvec, kThreads), kThreads, 0, s>>>((const TIn *)x, (TQ *)q, n, pos, scale, pos_dev,

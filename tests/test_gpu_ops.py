@@ -1219,3 +1219,21 @@ def test_strided_pointwise_layer_on_more_than_2_gib_of_activations():
     got = torch.ops.torch_mlu.conv2d(x.permute(0, 3, 1, 2), w.cuda(), b.cuda(), [0, 0], [stride, stride], [1, 1], 1, scale.cuda(),
                                      mode.cuda())
     assert same_bits(want, got.cpu().contiguous().numpy())
+
+
+@pytest.mark.parametrize("dtype,bits,vectors", [(torch.float32, 8, 11 << 20), (torch.float32, 16, 1 << 24), (torch.float16, 8, 1 << 22),
+                                                (torch.float16, 16, 1 << 22)])
+def test_quantize_large_tensors(dtype, bits, vectors):
+    """two vectors of 16 bytes a lane from `vectors` on: the last size below, a block's last lanes without a second vector or any, and
+    values behind the last vector, with the position from the host and from the device"""
+    per, lo, hi = 16 // dtype.itemsize, -(1 << bits - 1), (1 << bits - 1) - 1
+    pos = -5 if bits == 8 else -12
+    x = torch.randn(vectors * per + 3000 * per, generator=torch.Generator(device="cuda").manual_seed(bits), device="cuda").to(dtype)
+    x[::5] *= 40.0  # beyond the range
+    x[torch.tensor([0, 511 * per, vectors * per - 1])] = torch.tensor([math.inf, math.nan, -math.inf], device="cuda").to(dtype)
+    want = torch.round(x.float() * 2.0 ** -pos).nan_to_num(0.0, hi, lo).clamp(lo, hi).to(torch.int8 if bits == 8 else torch.int16)
+    at = torch.tensor([pos], dtype=torch.int32, device="cuda")
+    for n in (vectors * per - 1, vectors * per, (vectors + 1) * per + 1, (vectors + 256) * per, (vectors + 257) * per + per - 1,
+              (vectors + 511) * per + 2, x.numel()):
+        assert torch.equal(torch.ops.torch_mlu.quantize(x[:n], bits, pos, 1.0), want[:n]), n
+        assert torch.equal(torch.ops.torch_mlu.quantize_dev(x[:n], bits, at), want[:n]), n
