@@ -492,7 +492,10 @@ int contract_small_dual_i8(const void *x, const void *w, int N_img, int H, int W
 // two launches / one, 3 x 3 and 1 x 1 layers of 16 to 512 channels): 16 x 16 tiles on four waves, one step a wave 10.5 / 7.0, two 10.6 /
 // 7.1, three and four 10.6 / 7.8 to 10.0 with up to a tile per unit and 11 / 13 to 17 with two; on eight waves two 11.9 / 10.3, three
 // 11 / 12; 32 x 32 tiles one 10.5 / 6.8, two 11.8 / 9.1 up to a tile per unit, three 10.6 / 13.9.  Rows of any length in halfs, read in
-// whole dwords, lie within 1 us of aligned ones: linears of an unaligned K 9.2 / 5.6, pixels of padded channels 10 / 7.
+// whole dwords, lie within 1 us of aligned ones: linears of an unaligned K 9.2 / 5.6, pixels of padded channels 10 / 7.  But rows that
+// start off their pieces cost a wave more, and with more than a tile per unit a step less is what pays: 32 x 32 tiles on three steps, 310,
+// 364 and 448 of them 8.5 / 11.9, 8.3 / 10.7 and 9.0 / 11.7, up to 256 8.3 / 7.9; 16 x 16 tiles on six, 306 to 498 of them 8.3 to 9.0 /
+// 8.7 to 10.1, up to 256 8.5 / 7.1, on five 8.2 to 9.4 / 8.0 to 8.6.
 //
 // The plan (as small_plan) and the kernel's constants; 0: not the one launch.  The question and the launch ask it both.
 static int small_float_plan(SmallSide *o, const void *x, bool half, const void *w, int N_img, int H, int W, int Ci, int Co, int kh,
@@ -503,11 +506,13 @@ static int small_float_plan(SmallSide *o, const void *x, bool half, const void *
   if (!plan) return 0;
   const int waves = plan % 100;
   const int64_t per_wave = ((K + 127) / 128 + waves - 1) / waves;
-  int most = plan / 100 == 32 ? 3 : 6;
+  const int64_t M = (int64_t)N_img * Ho * Wo, T = plan / 100, tiles = ((M + T - 1) / T) * ((Co + T - 1) / T);
+  int most = T == 32 ? 3 : 6;
   if (apart) {
-    const int64_t M = (int64_t)N_img * Ho * Wo;
-    if (plan / 100 == 32) most = waves == 4 ? (((M + 31) / 32) * ((Co + 31) / 32) <= cus ? 2 : 1) : 0;
-    else most = waves == 4 && ((M + 15) / 16) * ((Co + 15) / 16) <= cus ? 4 : 2;
+    if (T == 32) most = waves == 4 ? (tiles <= cus ? 2 : 1) : 0;
+    else most = waves == 4 && tiles <= cus ? 4 : 2;
+  } else if (x_ci != Ci && tiles > cus) {
+    most -= 1;
   }
   if (per_wave > most) return 0;
   return small_side(o, x, half ? 2 : 4, w, N_img, H, W, Ci, Co, kh, kw, ph, pw, sh, sw, dh, dw, Ho, Wo, dense, x_ci, apart) ? plan : 0;

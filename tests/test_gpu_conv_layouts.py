@@ -86,3 +86,32 @@ def test_linears_of_few_tiles_against_the_oracle(m, k, n, mode, dtype):
     for start in (1, 2):  # on an element's alignment, on a dword's
         whole[start:start + m * k] = x.reshape(-1)
         assert torch.equal(torch.ops.torch_mlu.linear(whole[start:start + m * k].view(m, k), w, b, scale, qm), want)
+
+
+@pytest.mark.parametrize("half", [False, True])
+@pytest.mark.parametrize("m,k,n,served", [
+    (310, 1300, 990, False), (255, 1300, 1020, True),    # 32 x 32 tiles on three steps a wave: 310 of them, 256
+    (300, 1010, 990, True),                              # 310 on two
+    (139, 2897, 739, False), (139, 2401, 739, True),     # 423 of 16 x 16 on six, on five
+    (139, 2897, 400, True), (310, 1312, 992, True),      # 225 on six; whole pieces a row
+])
+def test_rows_that_start_off_their_pieces_in_one_launch(m, k, n, served, half):
+    """which linears catchq_float_conv2d_small takes: with more than a tile per unit, a step a wave less of those rows"""
+    import ctypes
+    from catch_amd import _native
+    kd = (k + 15) // 16 * 16
+    x = torch.randn(m, k, generator=torch.Generator(device="cuda").manual_seed(k), device="cuda").to(torch.float16 if half else torch.float32)
+    w = torch.randint(-127, 128, (n, kd), generator=torch.Generator(device="cuda").manual_seed(n), dtype=torch.int8, device="cuda")
+    w[:, k:] = 0
+    y, want = (torch.zeros(m, n, device="cuda") for _ in range(2))
+    desc, e = _native.ConvDesc(m, 1, 1, kd, n, 1, 1, 0, 0, 1, 1, 1, 1, 1), _native.Epilogue()
+    e.exp2, e.y = -12, y.data_ptr()
+    lib, stream = _native.kernel_lib(), torch.cuda.current_stream().cuda_stream
+    status = lib.catchq_float_conv2d_small(x.data_ptr(), int(half), -5, k, 0, w.data_ptr(), 8, ctypes.byref(desc), ctypes.byref(e), stream)
+    assert status == (0 if served else 6)  # CATCHQ_ERR_UNSUPPORTED
+    if served:
+        q = torch.zeros(m, kd, dtype=torch.int8, device="cuda")
+        q[:, :k] = torch.ops.torch_mlu.quantize(x, 8, -5, 1.0)
+        e.y = want.data_ptr()
+        _native.check(lib.catchq_gemm_nt(q.data_ptr(), 8, w.data_ptr(), 8, m, n, kd, ctypes.byref(e), stream))
+        assert torch.equal(y, want) and want.std() > 0.1
