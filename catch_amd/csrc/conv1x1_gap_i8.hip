@@ -207,7 +207,9 @@ static bool gap_plan(int N, int HW, int K, int Co, bool resid, int &nw, int &pg,
   // while every block has a unit to itself and 128 while those do; beyond, 64 channels and, with a residual (and the longer K that
   // such layers have: fewer reads of the pixels), 256 with both groups in a wave.  us, 49 pixels, images of 320 -> 1280 / of 512 -> 2048
   // with a residual, four waves of 32 channels each (eight from 256 blocks on), as it was, / now: one image 9.0 / 5.0 and 11.8 / 5.9,
-  // 16 8.9 / 5.5 and 12.6 / 6.3, 27 9.4 / 6.4 and 10.3 / 9.1, 64 10.8 / 8.2 and 15.8 / 15.1.
+  // 16 8.9 / 5.5 and 12.6 / 6.3, 27 9.4 / 6.4 and 10.3 / 9.1, 64 10.8 / 8.2 and 15.8 / 15.1.  Images of one group: 256 channels, also where
+  // that leaves units without a block (16 pixels, 128 channels there, as it was, / 256: one image 6.0 / 5.3 and 8.0 / 6.7, 16 6.3 / 5.5 and
+  // 8.5 / 7.0, 31 7.0 / 5.6 and 9.6 / 7.2; 25 pixels, one 6.5 / 5.8 and 8.8 / 7.1; this kernel's other changes among them).
   p = GapConvParams{};
   p.N = N; p.HW = HW; p.K = K; p.Co = Co;
   p.groups = (HW + 31) / 32;

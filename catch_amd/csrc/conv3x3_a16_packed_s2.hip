@@ -7,9 +7,10 @@
 // the plane of its parities at q, q - 1, q - Wo or q - Wo - 1.  So a block stages four runs, BM, BM + 1, BM + Wo and BM + Wo + 1 pixels,
 // already split, and the nine taps are constant shifts in LDS as they are at stride 1.  The patch is four times as large as there:
 // 32 channels a step instead of 64, so that two buffers leave room for two blocks a unit.
-// What bounds it now: as at stride 1 the matrix pipes while a block has its unit to itself and the last round of blocks; and where
-// channels are few (128) the input, of which every block reads whole cache lines in two steps.  Two blocks a unit (237 registers with
-// 64 pixels), three of 32 pixels (145 to 158).
+// What bounds it now: no unit by itself.  Counters of the three layers below (676, 338 and 340 blocks): matrix pipes 28 % of all SIMD
+// cycles, vector instructions 14 to 27 %, LDS 15 to 17 %; waves wait a fifth to a third of their lives, and the blocks are no whole
+// number of rounds (two a unit, 237 registers with 64 pixels; three of 32 pixels, 145 to 158).  Where channels are few (128) every block
+// reads whole cache lines of the input in two steps.
 // us, tiled kernel / this, fp32 and int16 outputs, repeated in a graph: 16 images of 104 x 104, 128 -> 256 43.6 / 37.3, 52 x 52, 256 ->
 // 512 37.1 / 33.8, 26 x 26, 512 -> 1024 44.4 / 34.3; 12 images 33.7 / 26.7, 34.3 / 25.4, 33.1 / 26.3; 4 x 80 x 80, 128 -> 256 13.5 /
 // 10.1; one of 110 x 104, 192 -> 1024 20.2 / 15.7; 8 x 102 x 96, 384 -> 512 118 / 81.

@@ -55,7 +55,7 @@ __device__ __forceinline__ void small_ds_write(unsigned addr, v4i v) {
   asm volatile("ds_write_b128 %0, %1" ::"v"(addr), "v"(v) : "memory");
 }
 
-// DENSE: a plain GEMM -- row m starts at m * K, no taps.  IN: type of the activations.  DUAL: a residual block's last
+// DENSE: a plain GEMM -- row m starts at m * pix_stride (the channels of the activations, which may be fewer than K), no taps.  IN: type of the activations.  DUAL: a residual block's last
 // convolution and its projection shortcut over the same output tile; the block's waves are shared out between the two
 // in proportion to their K steps, and the shortcut's sums, dequantized with its own constants, are the residual.
 // HALF_BIAS: there is a bias, in half precision (a choice at run time costs every launch 0.05 us).

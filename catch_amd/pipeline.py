@@ -190,8 +190,8 @@ class FusedNet(object):
         parallel streams, where one part's launches already fill the other's start-up gaps, MobileNetV2 at batch 128
         measured 2 % slower with it (one stream: 1.5 % faster).
         fuse_first_layers: the input quantizer, a few-channel first convolution + ReLU and the max pooling that is its
-        only reader run as one launch (torch_mlu::qconv2d_first_layers) where the library's kernel serves the shape;
-        neither the quantized image nor the convolution's output is then stored.
+        only reader run as one launch (torch_mlu::qconv2d_first_layers_any, first_layers_run) where the library's kernel serves
+        the shape; neither the quantized image nor the convolution's output is then stored.
         fuse_avgpool: a 1x1 convolution whose only reader is the global average pooling runs inside the pooling's launch
         (torch_mlu::qconv2d_avgpool) where the library's kernel serves the shape; its fp32 output is then never stored.
         fuse_expansions: a 1x1 convolution behind ReLU / ReLU6 whose only reader is a 3x3 depthwise convolution runs inside
@@ -428,8 +428,8 @@ class FusedNet(object):
         return bool(torch.ops.torch_mlu.expand_depthwise_fuses(n, h, w, self.cdev[x.src], self.cdev[x.name], dw.stride))
 
     def first_layers_fuse(self, n, c, h, w):
-        """whether quantizer, first convolution and pooling run as one launch of torch_mlu::qconv2d_first_layers on a contiguous
-        fp32 batch [n, c, h, w]"""
+        """whether the op torch_mlu::qconv2d_first_layers serves the plan's first layers on a contiguous fp32 batch [n, c, h, w]
+        in one launch: widths that are a multiple of four, the pooled floats not read.  (A pass asks first_layers_run.)"""
         if self.first_pool is None or self.first_floats:
             return False
         l0, pool = self.layers[0], self.first_pool
@@ -437,8 +437,8 @@ class FusedNet(object):
                                                           pool.stride, pool.pad))
 
     def first_layers_run(self, n, c, h, w):
-        """whether they run as one launch at all (first_layers): that one or, for other widths and where the pooled floats are read
-        too, torch_mlu::qconv2d_first_layers_any"""
+        """whether a pass over a contiguous fp32 batch [n, c, h, w] runs quantizer, first convolution and pooling as one launch
+        (first_layers): images of any width, also where the pooled floats are read"""
         if self.first_pool is None:
             return False
         l0, pool = self.layers[0], self.first_pool
